@@ -105,6 +105,12 @@ typedef struct {
 /* Rows of A per tile for `rows` rows (experts: the mean number) with each of `matrices` matrices of N rows. */
 int dlm_gemm_tile_rows(int dtype, int rows, int N, int matrices);
 int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream);
+/* Not grouped, with the tile (tile_rows is not read) and the number of slices along K chosen by shape: dlm_gemm_slices gives the
+ * number, 1 .. 64 and at most K / 64 (a caller may take another one; more than one: bf16 only).  More than one slice: parts holds
+ * slices * M * N floats, one matrix [M, N] after the other, that a second launch adds up into out; with out NULL (epilogue 1) they
+ * are left to the caller, as dlm_add_norm_parts and dlm_residual_norm_parts take them. */
+int dlm_gemm_slices(int dtype, int M, int N, int K, int epilogue);
+int dlm_gemm_sliced(int dtype, const dlm_gemm_args *g, int slices, float *parts, void *stream);
 
 int dlm_embed_rows(int dtype, const int32_t *tokens, const void *embed, float scale, float *res, void *h, int M, int width, void *stream);
 /* res += y / rms(y) * norm_w; h (optional) = res in the element type.  weights NULL: y fp32 [M, width]; otherwise y in the
@@ -114,6 +120,11 @@ int dlm_residual_norm_rows(int dtype, float *res, const void *y, const float *we
 /* v = embed[tokens] * scale (tokens given), res + y (y given) or res; res = v, h (optional) = v / rms(v) * norm_w in the element type */
 int dlm_add_norm_rows(int dtype, float *res, const float *y, const int32_t *tokens, const void *embed, float scale, const float *norm_w, float eps,
                       int true_width, void *h, int M, int width, void *stream);
+/* The two with y the sum of `parts` fp32 matrices [M, width]. */
+int dlm_residual_norm_parts(int dtype, float *res, const float *y, int parts, const float *norm_w, float eps, int true_width, void *h, int M, int width,
+                            void *stream);
+int dlm_add_norm_parts(int dtype, float *res, const float *y, int parts, const float *norm_w, float eps, int true_width, void *h, int M, int width,
+                       void *stream);
 /* out[i] = res[rows[i]] / rms * norm_w in the element type (rows NULL: i) */
 int dlm_norm_rows(int dtype, const float *res, const int32_t *rows, const float *norm_w, float eps, int true_width, void *out, int n,
                   int width, void *stream);

@@ -152,6 +152,10 @@ DENSE_SYMBOLS = {
     "dlm_moe_plan": (_ci, [_vp] + [_ci] * 3 + [_vp] * 3),
     "dlm_gemm_tile_rows": (_ci, [_ci] * 4),
     "dlm_gemm": (_ci, [_ci, _vp, _vp]),
+    "dlm_gemm_slices": (_ci, [_ci] * 5),
+    "dlm_gemm_sliced": (_ci, [_ci, _vp, _ci, _vp, _vp]),
+    "dlm_residual_norm_parts": (_ci, [_ci, _vp, _vp, _ci, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),
+    "dlm_add_norm_parts": (_ci, [_ci, _vp, _vp, _ci, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),
     "dlm_embed_rows": (_ci, [_ci, _vp, _vp, _cf, _vp, _vp, _ci, _ci, _vp]),
     "dlm_residual_norm_rows": (_ci, [_ci, _vp, _vp, _vp, _ci, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),
     "dlm_norm_rows": (_ci, [_ci, _vp, _vp, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),

@@ -172,8 +172,10 @@ def argmax(keys, token=None, position=None, history=None):
     _lib.check_dense(lib.dlm_argmax(_ptr(keys), keys.numel(), _opt(token), _opt(position), _opt(history), _stream()))
 
 
-def gemm(a, w, out_f32=False, lda=None, rows=None, out=None, silu=None, gate=GATE_NONE):
-    """out[M, N] = A[M, K] W[N, K]^T; a: [M, >= K] with row stride `lda` (default: its width).  `silu`, `gate` as in gemv_normed."""
+def gemm(a, w, out_f32=False, lda=None, rows=None, out=None, silu=None, gate=GATE_NONE, parts=False):
+    """out[M, N] = A[M, K] W[N, K]^T; a: [M, >= K] with row stride `lda` (default: its width).  `silu`, `gate` as in gemv_normed.
+    Products that leave most of the GPU idle run in slices along K that a second launch adds up; `parts` (with out_f32): the caller
+    takes their results one by one, [slices, M, N], as residual_norm_rows and add_norm_rows do."""
     lib = _lib.load_dense_library()
     _need_cuda(w)
     _same("gemm", w, a)
@@ -183,14 +185,17 @@ def gemm(a, w, out_f32=False, lda=None, rows=None, out=None, silu=None, gate=GAT
     if not a.is_cuda or a.stride(-1) != 1 or a.shape[1] < K or M > a.shape[0]:
         raise ValueError(f"gemm: A must be a GPU matrix with at least {K} columns and {M} rows")
     width = N // 2 if gate else N
-    if out is None:
-        out = torch.empty((M, width), dtype=torch.float32 if out_f32 else w.dtype, device=w.device)
     begin, end = silu or (0, 0)
     epilogue = OUT_F32 if out_f32 else {GATE_NONE: OUT_ELEM, GATE_SILU: OUT_SWIGLU, GATE_GELU: OUT_GEGLU}[gate]
-    g = _lib.GemmArgs(a=a.data_ptr(), w=_ptr(w), out=_ptr(out), lda=lda, ldo=width, M=M, N=N, K=K, epilogue=epilogue, silu_begin=begin, silu_end=end,
-                      tile_rows=lib.dlm_gemm_tile_rows(dtype_code(w), M, N, 1))
-    _lib.check_dense(lib.dlm_gemm(dtype_code(w), ctypes.byref(g), _stream()))
-    return out
+    dt = dtype_code(w)
+    slices = lib.dlm_gemm_slices(dt, M, N, K, epilogue)
+    keep = parts and out_f32 and out is None
+    if out is None and not (keep and slices > 1):
+        out = torch.empty((M, width), dtype=torch.float32 if out_f32 else w.dtype, device=w.device)
+    pieces = torch.empty((slices, M, N), dtype=torch.float32, device=w.device) if slices > 1 else None
+    g = _lib.GemmArgs(a=a.data_ptr(), w=_ptr(w), out=_opt(out), lda=lda, ldo=width, M=M, N=N, K=K, epilogue=epilogue, silu_begin=begin, silu_end=end)
+    _lib.check_dense(lib.dlm_gemm_sliced(dt, ctypes.byref(g), slices, _opt(pieces), _stream()))
+    return out if out is not None and not keep else pieces if out is None else out.unsqueeze(0)
 
 
 def embed_rows(tokens, embed, scale):
@@ -208,32 +213,40 @@ def embed_rows(tokens, embed, scale):
 
 def residual_norm_rows(res, y, norm_w, eps, width, dtype, weights=None):
     """res += norm(y) in place; returns res in the element type.  With router weights [M, top], y [M * top, K] holds the
-    chosen experts' outputs in the element type; otherwise y is fp32 [M, K]."""
+    chosen experts' outputs in the element type; otherwise y is fp32 [M, K], or parts [n, M, K] of it."""
     lib = _lib.load_dense_library()
     _need_cuda(res, y, norm_w)
     _need_f32(res, norm_w, weights)
     M, K = res.shape
     top = 0 if weights is None else weights.shape[1]
-    if tuple(y.shape) != (M * max(top, 1), K) or norm_w.numel() != K or y.dtype != (dtype if top else torch.float32):
+    parts = y.shape[0] if y.dim() == 3 and not top else 0
+    if tuple(y.shape) != ((parts, M, K) if parts else (M * max(top, 1), K)) or norm_w.numel() != K or y.dtype != (dtype if top else torch.float32):
         raise ValueError("residual_norm_rows: shapes or types of y and the norm weight do not match")
     h = torch.empty((M, K), dtype=dtype, device=res.device)
+    if parts:
+        _lib.check_dense(lib.dlm_residual_norm_parts(dtype_code(dtype), _ptr(res), _ptr(y), parts, _ptr(norm_w), eps, width, _ptr(h), M, K, _stream()))
+        return h
     _lib.check_dense(lib.dlm_residual_norm_rows(dtype_code(dtype), _ptr(res), _ptr(y), _opt(weights), top, _ptr(norm_w), eps, width, _ptr(h), M, K,
                                                 _stream()))
     return h
 
 
 def add_norm_rows(res, y, norm_w, eps, width, dtype, tokens=None, embed=None, scale=1.0):
-    """The residual rows brought up to date in place - res + y (y fp32 [M, K] or None), or with `tokens` the embedding rows times
+    """The residual rows brought up to date in place - res + y (y fp32 [M, K], parts [n, M, K] of it, or None), or with `tokens` the embedding rows times
     `scale` - and their norm in the element type (None without norm_w)."""
     lib = _lib.load_dense_library()
     _need_cuda(res)
     _need_f32(res, y, norm_w)
     M, K = res.shape
-    if (y is not None and tuple(y.shape) != (M, K)) or (norm_w is not None and norm_w.numel() != K):
+    parts = y.shape[0] if y is not None and y.dim() == 3 else 0
+    if (y is not None and tuple(y.shape[-2:]) != (M, K)) or (y is not None and y.dim() > 3) or (norm_w is not None and norm_w.numel() != K):
         raise ValueError("add_norm_rows: shapes of the residual, y and the norm weight do not match")
     if tokens is not None and (tokens.dtype != torch.int32 or tokens.numel() != M or embed.shape[1] != K or embed.dtype != dtype or y is not None):
         raise ValueError("add_norm_rows: int32 tokens, one per row, and an embedding of the rows' width")
     h = None if norm_w is None else torch.empty((M, K), dtype=dtype, device=res.device)
+    if parts:
+        _lib.check_dense(lib.dlm_add_norm_parts(dtype_code(dtype), _ptr(res), _ptr(y), parts, _opt(norm_w), eps, width, _opt(h), M, K, _stream()))
+        return h
     _lib.check_dense(lib.dlm_add_norm_rows(dtype_code(dtype), _ptr(res), _opt(y), _opt(tokens), _opt(embed), scale, _opt(norm_w), eps, width, _opt(h), M, K,
                                            _stream()))
     return h

@@ -269,7 +269,7 @@ class KuvonexModel(DenseModel):
         res, h = dense.embed_rows(tokens, self.embed, c.embed_scale)
         for l in self.layers:
             attn = self._attend(l, dense.gemm(h, l.w_in), cache, pos)
-            y = dense.gemm(attn, l.w_o, out_f32=True)
+            y = dense.gemm(attn, l.w_o, out_f32=True, parts=True)
             h = dense.residual_norm_rows(res, y, l.norm1, c.eps, c.width, self.dtype)
             if l.router is not None:
                 logits = dense.gemm(h, l.w_router, out_f32=True)

@@ -405,12 +405,12 @@ class SitiraxModel(DenseModel):
             h = dense.add_norm_rows(res, y, l.norm1, c.eps, c.width, self.dtype, **embedding)
             embedding = {}
             out = self._mix(i, dense.gemm(h, l.mixer.w_in, silu=l.mixer.silu), cache, pos)
-            y = dense.gemm(out, l.mixer.w_o, out_f32=True)
+            y = dense.gemm(out, l.mixer.w_o, out_f32=True, parts=True)
             if l.norm2 is not None:
                 h = dense.add_norm_rows(res, y, l.norm2, c.eps, c.width, self.dtype)
-                y = dense.gemm(dense.gemm(h, l.w_gate_up, gate=dense.GATE_GELU), l.w_down, out_f32=True)
+                y = dense.gemm(dense.gemm(h, l.w_gate_up, gate=dense.GATE_GELU), l.w_down, out_f32=True, parts=True)
             if trace is not None:
-                trace.append(res + y)
+                trace.append(res + y.sum(0))
         dense.add_norm_rows(res, y, None, c.eps, c.width, self.dtype, **embedding)
         return res
 

@@ -169,7 +169,18 @@ __device__ __forceinline__ float sigmoid_of(float z) {
     if constexpr (sizeof(T) == 2) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
     return sigmoid_f32(z);
 }
-__device__ __forceinline__ float gelu_tanh_f32(float z) { return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * fmaf(0.044715f * z * z, z, z))); }
+template <class T>
+__device__ __forceinline__ float silu_of(float z) {
+    if constexpr (sizeof(T) == 2) return z * sigmoid_of<T>(z);
+    return silu_f32(z);
+}
+// 0.5 z (1 + tanh u) = z sigmoid(2 u), u = sqrt(2 / pi) (z + 0.044715 z^3): no cancellation, one exponential
+template <class T>
+__device__ __forceinline__ float gelu_tanh_of(float z) {
+    const float v = 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
+    if constexpr (sizeof(T) == 2) return z * sigmoid_of<T>(v);
+    return z / (1.0f + expf(-v));
+}
 // log(1 + e^z) = max(z, 0) + log(1 + t), t = e^-|z|; log(1 + t) = log(u) t / (u - 1) with u the rounded 1 + t, whose error the
 // quotient takes back (Goldberg, "What Every Computer Scientist Should Know About Floating-Point Arithmetic", 1991)
 __device__ __forceinline__ float softplus_f32(float z) {

@@ -239,10 +239,9 @@ int dlm_moe_plan(const int32_t *ids, int entries, int experts, int tile_rows, in
 
 int dlm_gemm_tile_rows(int dtype, int rows, int N, int matrices) { return dense_gemm_tile_rows(dtype, rows, N, matrices); }
 
-int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
-    if (!g || !g->a || !g->w || !g->out) return DLM_ERR_NULL;
+static int gemm_args(int dtype, const dlm_gemm_args *g, GemmArgs &a) {
+    if (!g || !g->a || !g->w) return DLM_ERR_NULL;
     if (bad_type(dtype) || g->M <= 0 || g->N <= 0 || g->N % 16 || g->K <= 0 || g->K % 64 || g->lda < g->K || g->lda % 8 || g->ldo % 8) return DLM_ERR_SHAPE;
-    if (g->tile_rows != 32 && g->tile_rows != 128 && g->tile_rows != 256) return DLM_ERR_SHAPE;
     if (g->tiles) {
         if (!g->order) return DLM_ERR_NULL;
         if (g->n_tiles <= 0 || g->gather < 0 || g->epilogue == kOutF32 || g->epilogue == kOutGeglu || g->silu_begin < g->silu_end || g->w_stride < (int64_t)g->N * g->K) return DLM_ERR_SHAPE;
@@ -252,7 +251,6 @@ int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
     if (g->silu_begin < g->silu_end && (g->epilogue != kOutElem || g->silu_begin % 16 || g->silu_end % 16)) return DLM_ERR_SHAPE;
     if (g->epilogue < 0 || g->epilogue > kOutGeglu || g->ldo < (paired ? g->N / 2 : g->N)) return DLM_ERR_SHAPE;
     if (odd(g->a) || odd(g->w) || odd(g->out)) return DLM_ERR_ALIGN;
-    GemmArgs a;
     a.a = g->a;
     a.w = g->w;
     a.out = g->out;
@@ -269,8 +267,30 @@ int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
     a.w_stride = g->w_stride;
     a.silu_begin = g->silu_begin;
     a.silu_end = g->silu_end;
+    return DLM_OK;
+}
+
+int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
+    GemmArgs a;
+    if (g && !g->out) return DLM_ERR_NULL;
+    if (const int e = gemm_args(dtype, g, a)) return e;
+    if (g->tile_rows != 32 && g->tile_rows != 128 && g->tile_rows != 256) return DLM_ERR_SHAPE;
     return done(launch_dense_gemm(dtype, a, g->tile_rows, hs(stream)));
 }
+
+int dlm_gemm_slices(int dtype, int M, int N, int K, int epilogue) {
+    return bad_type(dtype) || M <= 0 || N <= 0 || K <= 0 ? 0 : dense_gemm_slices(dtype, M, N, K, epilogue);
+}
+
+int dlm_gemm_sliced(int dtype, const dlm_gemm_args *g, int slices, float *parts, void *stream) {
+    GemmArgs a;
+    if (const int e = gemm_args(dtype, g, a)) return e;
+    if (g->tiles || slices < 1 || slices > g->K / 64 || slices > 64 || (slices > 1 && dtype != kBf16)) return DLM_ERR_SHAPE;
+    if (slices == 1 ? !g->out : (!parts || (!g->out && g->epilogue != kOutF32))) return DLM_ERR_NULL;
+    if (slices > 1 && odd(parts)) return DLM_ERR_ALIGN;
+    return done(launch_dense_gemm_sliced(dtype, a, slices, parts, hs(stream)));
+}
+
 
 int dlm_embed_rows(int dtype, const int32_t *tokens, const void *embed, float scale, float *res, void *h, int M, int width, void *stream) {
     if (!tokens || !embed || !res || !h) return DLM_ERR_NULL;
@@ -286,7 +306,7 @@ int dlm_residual_norm_rows(int dtype, float *res, const void *y, const float *we
         (weights && top <= 0))
         return DLM_ERR_SHAPE;
     if (odd(res) || odd(y) || odd(norm_w) || odd(h)) return DLM_ERR_ALIGN;
-    return done(launch_residual_norm_rows(dtype, res, y, weights, top, norm_w, eps, true_width, h, M, width, hs(stream)));
+    return done(launch_residual_norm_rows(dtype, res, y, 1, weights, top, norm_w, eps, true_width, h, M, width, hs(stream)));
 }
 
 int dlm_norm_rows(int dtype, const float *res, const int32_t *rows, const float *norm_w, float eps, int true_width, void *out, int n, int width,
@@ -297,13 +317,31 @@ int dlm_norm_rows(int dtype, const float *res, const int32_t *rows, const float 
     return done(launch_norm_rows(dtype, res, rows, norm_w, eps, true_width, out, n, width, hs(stream)));
 }
 
+int dlm_residual_norm_parts(int dtype, float *res, const float *y, int parts, const float *norm_w, float eps, int true_width, void *h, int M, int width,
+                            void *stream) {
+    if (!res || !y || !norm_w) return DLM_ERR_NULL;
+    if (bad_type(dtype) || M <= 0 || width <= 0 || width % 64 || width > kMaxWidth || parts < 1 || true_width <= 0 || true_width > width || !(eps >= 0.f))
+        return DLM_ERR_SHAPE;
+    if (odd(res) || odd(y) || odd(norm_w) || odd(h)) return DLM_ERR_ALIGN;
+    return done(launch_residual_norm_rows(dtype, res, y, parts, nullptr, 0, norm_w, eps, true_width, h, M, width, hs(stream)));
+}
+
+int dlm_add_norm_parts(int dtype, float *res, const float *y, int parts, const float *norm_w, float eps, int true_width, void *h, int M, int width,
+                       void *stream) {
+    if (!res || !y || (h && !norm_w)) return DLM_ERR_NULL;
+    if (bad_type(dtype) || M <= 0 || width <= 0 || width % 64 || width > kMaxWidth || parts < 1 || true_width <= 0 || true_width > width || !(eps >= 0.f))
+        return DLM_ERR_SHAPE;
+    if (odd(res) || odd(y) || odd(norm_w) || odd(h)) return DLM_ERR_ALIGN;
+    return done(launch_add_norm_rows(dtype, res, y, parts, nullptr, nullptr, 1.f, norm_w, eps, true_width, h, M, width, hs(stream)));
+}
+
 int dlm_add_norm_rows(int dtype, float *res, const float *y, const int32_t *tokens, const void *embed, float scale, const float *norm_w, float eps,
                       int true_width, void *h, int M, int width, void *stream) {
     if (!res || (tokens && !embed) || (h && !norm_w)) return DLM_ERR_NULL;
     if (bad_type(dtype) || M <= 0 || width <= 0 || width % 64 || width > kMaxWidth || true_width <= 0 || true_width > width || !(eps >= 0.f) || (tokens && y))
         return DLM_ERR_SHAPE;
     if (odd(res) || odd(y) || odd(embed) || odd(norm_w) || odd(h)) return DLM_ERR_ALIGN;
-    return done(launch_add_norm_rows(dtype, res, y, tokens, embed, scale, norm_w, eps, true_width, h, M, width, hs(stream)));
+    return done(launch_add_norm_rows(dtype, res, y, 1, tokens, embed, scale, norm_w, eps, true_width, h, M, width, hs(stream)));
 }
 
 int dlm_head_decode_supported(int dtype, const dlm_head_shape *s) {

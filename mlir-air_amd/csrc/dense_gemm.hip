@@ -2,11 +2,16 @@
 // type, fp32 accumulation; plain, or grouped over the experts of a mixture (row tiles from moe_plan_kernel).
 //
 // Both operands have k contiguous, so a tile of either is a set of rows of 128 bytes per K-step (64 bf16 or 32 floats) and
-// goes global -> LDS without passing through registers (global_load_lds_dwordx4) into a ring of STAGES buffers, STAGES - 1
-// K-steps ahead (two where the tile is large; the small tile has little to multiply per step): one wave instruction
-// fills 1 KiB, 8 rows, lane l writing 16-byte slot l % 8 of row l / 8 and fetching chunk slot ^ row % 8, so that the operand
-// reads of 16 consecutive rows are spread over the banks without padding.  One barrier per K-step.  W is the first MFMA
-// operand: a lane then holds four consecutive n of one row m and stores them as one word.
+// goes global -> LDS without passing through registers (global_load_lds_dwordx4): one wave instruction fills 1 KiB, 8 rows, lane l
+// writing 16-byte slot l % 8 of row l / 8 and fetching chunk slot ^ row % 8, so that the operand reads of 16 consecutive rows are
+// spread over the banks without padding.  W is the first MFMA operand: a lane then holds four consecutive n of one row m.
+//
+//   dense_gemm_kernel        fp32, few rows, experts with few rows: a ring of STAGES buffers, STAGES - 1 K-steps ahead, one barrier
+//                            per K-step, the compiler's own order of reads and products
+//   dense_gemm_wide_kernel   bf16 from 128 rows on: one wave per SIMD with 128 x 128 results in AGPRs, every read and copy at its
+//                            place between the products
+//
+// Products with too few tiles for the GPU run in slices along K (blockIdx.y) whose fp32 parts are added afterwards.
 //
 // Row gathers cost nothing here: every lane of a copy has its own source row.  The waves of a SIMD differ in their rows, so
 // that a wave whose rows lie behind the end of an expert's run can leave the matrix pipe to the other.
@@ -33,7 +38,58 @@ struct GemmKernelArgs {
     long w_stride;
     int tiles_m, tiles_n;
     int silu_begin, silu_end;
+    long slice_stride;   // elements between the parts of two slices along K (blockIdx.y); one slice: anything
 };
+
+// The K-steps of this workgroup's slice.
+struct KSlice {
+    int first, steps;
+};
+__device__ __forceinline__ KSlice k_slice(int steps) {
+    const int first = (int)((long)steps * blockIdx.y / gridDim.y);
+    return {first, (int)((long)steps * (blockIdx.y + 1) / gridDim.y) - first};
+}
+
+// A wave's block of the result, NT x MT tiles of 16 x 16: a lane holds row ql of every tile and its columns 4 g .. + 3.
+template <class T, int MT, int NT, int EPI, bool GROUPED>
+__device__ __forceinline__ void store_tile(const GemmKernelArgs<T> &p, floatx4 (&acc)[NT][MT], int m_first, int m_end, int n_first) {
+    const int lane = threadIdx.x & 63, ql = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = m_first + 16 * i + ql;
+        if (m >= m_end) continue;
+        size_t row = m;
+        if constexpr (GROUPED)
+            if (p.gather == 0) row = p.order[m];
+        if constexpr (EPI == kOutSwiglu || EPI == kOutGeglu) {
+#pragma unroll
+            for (int j = 0; j < NT; j += 2) {
+                const int n = n_first + 16 * j;
+                if (n >= p.N) continue;
+                float v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = (EPI == kOutGeglu ? gelu_tanh_of<T>(acc[j][i][r]) : silu_of<T>(acc[j][i][r])) * acc[j + 1][i][r];
+                store4(static_cast<T *>(p.out) + row * p.ldo + n / 2 + 4 * g, v[0], v[1], v[2], v[3]);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int n = n_first + 16 * j + 4 * g;
+                if (n >= p.N) continue;
+                if constexpr (EPI == kOutElem && !GROUPED) {
+                    if (n >= p.silu_begin && n < p.silu_end) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[j][i][r] = silu_of<T>(acc[j][i][r]);
+                    }
+                }
+                if constexpr (EPI == kOutF32)
+                    store4(static_cast<float *>(p.out) + blockIdx.y * p.slice_stride + row * p.ldo + n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
+                else
+                    store4(static_cast<T *>(p.out) + row * p.ldo + n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
+            }
+        }
+    }
+}
 
 // BM x BN tile, WM x WN waves (m x n); GROUPED: expert row tiles
 template <class T, int BM, int BN, int WM, int WN, int STAGES, int EPI, bool GROUPED>
@@ -112,7 +168,10 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_gemm_kernel(const GemmKern
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    const int steps = p.K / KE;
+    const KSlice slice = k_slice(p.K / KE);
+    const int steps = slice.steps;
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) src[i] += (size_t)slice.first * kRowBytes;
     const bool idle = GROUPED && m0 + wm * (BM / WM) >= m_end;
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i)
@@ -145,46 +204,293 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_gemm_kernel(const GemmKern
         }
     }
 
-    // lane: row m = ... + ql, columns 4 g .. + 3 of each 16-column block
+    store_tile<T, MT, NT, EPI, GROUPED>(p, acc, m0 + wm * (BM / WM), m_end, n0 + wn * (BN / WN));
+}
+
+// ---- wide tiles, bf16 ------------------------------------------------------------------------------------------------------
+// 128 WM rows x 16 NT (4 / WM) columns, four waves WM x 4 / WM, a wave 128 rows x 16 NT columns.
+//
+// What bounds it: the matrix pipe at the clock that the power limit leaves (1.9 GHz), if nothing else holds the one wave of a SIMD
+// up, which issues in order.  A K-step of 256 x 256 is 128 products of 16 cycles a wave, in four quarters: (columns 0 .. 63 | 64 .. 127 of the
+// wave) x (k 0 .. 31 | 32 .. 63).  Each quarter's operands are read during the one before it, two products apart; the last quarter
+// reads the next K-step's, so the one wait and barrier of a K-step stands in front of it, with the matrix pipe full and the operands of
+// 32 products in registers.  Copies: A of K-step t + 2 in the last quarter of t and the first of t + 1, W of t + 3 (three buffers; A has two)
+// in the middle ones, evenly: LDS is filled at 64 bytes a cycle, so the 64 KiB of a K-step take half of its 2048 cycles, and copies in
+// bursts stopped the products (215 -> 197 us below).
+// Two waves per SIMD with 128 x 64 each (the kernel before) read half as much again from LDS: 1536 + 512 cycles of reads and copies for
+// 2048 of products.  2048 x 8192 x 8192 236 -> 197 us = 1.39 PFLOP/s, 4096^3 122 -> 100 us = 1.38, 2048 x 16384 x 2048 with gelu 135 -> 106.
+constexpr int kWideThreads = 256, kWideStagesW = 3;
+constexpr size_t wide_lds(int wm, int nt) { return (2 * (size_t)(128 * wm) + kWideStagesW * (size_t)(4 / wm * 16 * nt)) * kRowBytes; }
+
+// acc += w a.  Volatile asm: the accumulators stay in their AGPRs and the order of the source is kept.
+__device__ __forceinline__ void mfma_in_place(floatx4 &acc, const bf16x8 &w, const bf16x8 &a) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
+}
+// COLS x 8 products, `behind(n)` issued behind the n-th of them
+template <int COLS, int W, class F>
+__device__ __forceinline__ void quarter(floatx4 (*acc)[8], const bf16x8 (&w)[W], const bf16x8 (&a)[8], F behind) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int m = m0 + wm * (BM / WM) + 16 * i + ql;
-        if (m >= m_end) continue;
-        size_t row = m;
-        if constexpr (GROUPED)
-            if (p.gather == 0) row = p.order[m];
-        if constexpr (EPI == kOutSwiglu || EPI == kOutGeglu) {
+    for (int n = 0; n < 8 * COLS; ++n) {
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_in_place(acc[n / 8][n % 8], w[n / 8], a[n % 8]);
+        __builtin_amdgcn_sched_barrier(0);
+        behind(n);
+    }
+}
+// Which of `items` LDS reads goes behind product n of `products`: every second product has one, or every one where that would run
+// into their last quarter.  Which of `items` copies: spread evenly, because the four waves' copies fill LDS at 64 bytes a cycle, 16
+// cycles each, and one that finds the path taken holds up its wave's products.  -1: none.
+__device__ constexpr int read_behind(int n, int products, int items) {
+    const int stride = items * 8 <= products * 3 ? 2 : 1;
+    return n % stride == 0 && n / stride < items ? n / stride : -1;
+}
+__device__ constexpr int copy_behind(int n, int products, int items) {
+    const int stride = products / items;
+    return n % stride == stride - 1 && n / stride < items ? n / stride : -1;
+}
+// A wave-uniform pointer that stays in scalar registers: a copy's address is then this plus a 32-bit offset per lane.
+typedef const __attribute__((address_space(1))) char *gptr;
+__device__ __forceinline__ gptr scalar_ptr(const void *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return reinterpret_cast<gptr>(((uint64_t)hi << 32) | lo);
+}
+
+// A wave's NT x 8 tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
+// has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
+constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
+template <int NT, int EPI, bool GROUPED>
+__device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][8], char *lds, int m_first, int m_end, int n_first) {
+    typedef typename std::conditional<EPI == kOutF32, float, bf16>::type Out;
+    constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
+    constexpr int kCols = 16 * NT / (kPair ? 2 : 1), kPiece = 16 / (int)sizeof(Out), kPitch = kCols + kPiece;
+    constexpr int kPieces = 16 * kCols / kPiece;   // of 16 rows
+    static_assert(16 * kPitch * sizeof(Out) <= kWideStore, "fits the wave's part");
+    const int lane = threadIdx.x & 63, ql = lane & 15, g = lane >> 4;
+    Out *rows = reinterpret_cast<Out *>(lds);
+    const int n_out = kPair ? n_first / 2 : n_first, n_end = kPair ? p.N / 2 : p.N;
 #pragma unroll
-            for (int j = 0; j < NT; j += 2) {
-                const int n = n0 + wn * (BN / WN) + 16 * j;
-                if (n >= p.N) continue;
-                float v[4];
+    for (int i = 0; i < 8; ++i) {
+        if (m_first + 16 * i >= m_end) break;   // uniform
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = (EPI == kOutGeglu ? gelu_tanh_f32(acc[j][i][r]) : silu_f32(acc[j][i][r])) * acc[j + 1][i][r];
-                store4(static_cast<T *>(p.out) + row * p.ldo + n / 2 + 4 * g, v[0], v[1], v[2], v[3]);
+        for (int j = 0; j < NT; j += kPair ? 2 : 1) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] = acc[j][i][r];
+                if constexpr (kPair) v[r] = (EPI == kOutGeglu ? gelu_tanh_of<bf16>(v[r]) : silu_of<bf16>(v[r])) * acc[j + 1][i][r];
             }
-        } else {
+            if constexpr (EPI == kOutElem && !GROUPED) {
+                const int n = n_first + 16 * j;   // (the range is in whole tiles)
+                if (n >= p.silu_begin && n < p.silu_end) {
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int n = n0 + wn * (BN / WN) + 16 * j + 4 * g;
-                if (n >= p.N) continue;
-                if constexpr (EPI == kOutElem && !GROUPED) {
-                    if (n >= p.silu_begin && n < p.silu_end) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[j][i][r] = silu_f32(acc[j][i][r]);
-                    }
+                    for (int r = 0; r < 4; ++r) v[r] = silu_of<bf16>(v[r]);
                 }
-                if constexpr (EPI == kOutF32)
-                    store4(static_cast<float *>(p.out) + row * p.ldo + n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
-                else
-                    store4(static_cast<T *>(p.out) + row * p.ldo + n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
             }
+            store4(rows + ql * kPitch + 16 * (kPair ? j / 2 : j) + 4 * g, v[0], v[1], v[2], v[3]);
         }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = lane; t < kPieces; t += 64) {
+            const int row = t / (kCols / kPiece), col = t % (kCols / kPiece) * kPiece, m = m_first + 16 * i + row;
+            if (m >= m_end || n_out + col >= n_end) continue;
+            size_t to = m;
+            if constexpr (GROUPED)
+                if (p.gather == 0) to = p.order[m];
+            const long part = EPI == kOutF32 ? blockIdx.y * p.slice_stride : 0;
+            *reinterpret_cast<u32x4 *>(static_cast<Out *>(p.out) + part + to * p.ldo + n_out + col) = *reinterpret_cast<const u32x4 *>(rows + row * kPitch + col);
+        }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
-template <class T, int BM, int BN, int WM, int WN, int STAGES>
-hipError_t launch_tile(const GemmArgs &g, hipStream_t stream) {
+template <int WM, int NT, int EPI, bool GROUPED>
+__device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, KSlice slice) {
+    constexpr int WN = 4 / WM, BM = 128 * WM, BN = 16 * NT * WN;
+    constexpr int H0 = (NT + 1) / 2, H1 = NT - H0;        // column tiles of the two halves of a wave's columns
+    static_assert(H1 >= 2, "room for a quarter's LDS reads");
+    constexpr int CA = BM / 32, CW = BN / 32;             // copies of a wave and K-step
+    constexpr int CA0 = CA / 2, CW0 = (CW + 1) / 2;
+    constexpr int kSideA = BM * kRowBytes, kSideW = BN * kRowBytes;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int ql = lane & 15, g = lane >> 4;
+
+    // Copy i of a wave fills KiB i of the wave's part of a stage: eight rows, lane's chunk (lane % 8) ^ row % 8.  Four copies share
+    // their LDS base (M0) and differ in the instruction's offset, which the hardware adds to both addresses: the source takes it back.
+    // (Offsets from the wave's first row, 64 rows at most; gathered rows lie anywhere: their addresses are per lane.)
+    uint32_t off_a[CA], off_w[CW];
+    const char *row_a[CA];
+    const int m_wave = m0 + 8 * CA * wave < m_end ? m0 + 8 * CA * wave : m_end - 1, n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
+#pragma unroll
+    for (int i = 0; i < CA; ++i) {
+        const int row = 8 * (CA * wave + i) + (lane >> 3);
+        const uint32_t chunk = 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+        int m = m0 + row < m_end ? m0 + row : m_end - 1;
+        if constexpr (GROUPED) {
+            if (p.gather > 0) m = p.order[m] / p.gather;
+            row_a[i] = reinterpret_cast<const char *>(p.a + (size_t)m * p.lda) + chunk;
+        } else {
+            off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + chunk;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+        const int row = 8 * (CW * wave + i) + (lane >> 3);
+        const int n = n0 + row < p.N ? n0 + row : p.N - 1;
+        off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+    }
+    const size_t from = (size_t)slice.first * kRowBytes;
+    gptr base_a = scalar_ptr((GROUPED ? nullptr : reinterpret_cast<const char *>(p.a + (size_t)m_wave * p.lda)) + from - 4096);
+    gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from - 4096);
+    auto copy = [&](gptr from, int at, int i) {
+        const auto *src = (const __attribute__((address_space(1))) void *)from;
+        auto *dst = (__attribute__((address_space(3))) void *)(lds + at + 1024 * (i & ~3));
+        switch (i & 3) {
+            case 0: __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0); break;
+            case 1: __builtin_amdgcn_global_load_lds(src, dst, 16, 1024, 0); break;
+            case 2: __builtin_amdgcn_global_load_lds(src, dst, 16, 2048, 0); break;
+            default: __builtin_amdgcn_global_load_lds(src, dst, 16, 3072, 0); break;
+        }
+    };
+    auto copy_a = [&](int side, int i) {
+        if constexpr (GROUPED) copy((gptr)(row_a[i] + (ptrdiff_t)base_a), side + 1024 * CA * wave, i);
+        else copy(base_a + off_a[i], side + 1024 * CA * wave, i);
+    };
+    auto copy_w = [&](int side, int i) { copy(base_w + off_w[i], 2 * kSideA + side + 1024 * CW * wave, i); };
+
+    const int steps = slice.steps;
+    // operand addresses of the two halves (32 k) of a K-step; tile i is the instruction's offset
+    uint32_t at_a[2], at_w[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        const uint32_t o = ql * kRowBytes + 16 * ((4 * ks + g) ^ (ql & 7));
+        at_a[ks] = o + wm * 128 * kRowBytes;
+        at_w[ks] = o + 2 * kSideA + wn * 16 * NT * kRowBytes;
+    }
+    auto read = [&](uint32_t at, int i) { return *reinterpret_cast<const bf16x8 *>(lds + at + i * 16 * kRowBytes); };
+
+    floatx4 acc[NT][8];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    // A of K-steps 0 and 1, W of 0, 1 and 2 are on their way when the loop begins (past the end: the last K-step's once more, into
+    // a buffer that nobody reads)
+    int next_a = 0, next_w = 0;   // K-steps that the sources stand at
+    auto step_a = [&]() { return next_a + 1 < steps ? (++next_a, kRowBytes) : 0; };
+    auto step_w = [&]() { return next_w + 1 < steps ? (++next_w, kRowBytes) : 0; };
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+        for (int i = 0; i < CW; ++i) copy_w(s * kSideW, i);
+        base_w += step_w();
+#pragma unroll
+        for (int i = 0; i < (s == 0 ? CA : CA0); ++i) copy_a(s * kSideA, i);
+        if (s == 0) base_a += step_a();
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CW + CA0) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    bf16x8 a0[8], a1[8], w0[H0], w1[H0];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a0[i] = read(at_a[0], i);
+#pragma unroll
+    for (int j = 0; j < H0; ++j) w0[j] = read(at_w[0], j);
+
+    int side_a = 0, side_w = 0, fill_w = 2 * kSideW;   // of the K-step that is multiplied; of the one that W is copied for
+#pragma unroll 1
+    for (int kt = 0; kt < steps; ++kt) {
+        // (opaque in this block: the offsets' zero extension folds into the copies only if it is not taken out of the loop)
+#pragma unroll
+        for (int i = 0; i < CA && !GROUPED; ++i) asm volatile("" : "+v"(off_a[i]));
+#pragma unroll
+        for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
+        // first columns, first half of the K-step; the other half of A's copies for the next K-step
+        quarter<H0>(acc, w0, a0, [&](int n) {
+            if (const int r = read_behind(n, 8 * H0, H0 + 8); r >= 0) {
+                if (r < H0) w1[r] = read(at_w[1], r);
+                else a1[r - H0] = read(at_a[1], r - H0);
+            }
+            if (const int i = copy_behind(n, 8 * H0, CA - CA0); i >= 0) copy_a(side_a ^ kSideA, CA0 + i);
+        });
+        base_a += step_a();
+        // second half; W two K-steps on
+        quarter<H0>(acc, w1, a1, [&](int n) {
+            if (const int r = read_behind(n, 8 * H0, H1); r >= 0) w0[r] = read(at_w[0], H0 + r);
+            if (const int i = copy_behind(n, 8 * H0, CW0); i >= 0) copy_w(fill_w, i);
+        });
+        // the other columns, first half
+        quarter<H1>(acc + H0, w0, a0, [&](int n) {
+            if (const int r = read_behind(n, 8 * H1, H1); r >= 0) w1[r] = read(at_w[1], H0 + r);
+            if (const int i = copy_behind(n, 8 * H1, CW - CW0); i >= 0) copy_w(fill_w, CW0 + i);
+        });
+        base_w += step_w();
+        __builtin_amdgcn_sched_barrier(0);
+        // everything of the next K-step has landed (W of the one after it need not have), everybody has read all of this one
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(CW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int filled = side_a;
+        side_a ^= kSideA;
+        const int ahead = side_w == 2 * kSideW ? -2 * kSideW : kSideW;
+        side_w += ahead;
+        fill_w = fill_w == 2 * kSideW ? 0 : fill_w + kSideW;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            at_a[ks] ^= kSideA;
+            at_w[ks] += ahead;
+        }
+        // second half; A two K-steps on
+        quarter<H1>(acc + H0, w1, a1, [&](int n) {
+            if (const int r = read_behind(n, 8 * H1, H0 + 8); r >= 0) {
+                if (r < H0) w0[r] = read(at_w[0], r);
+                else a0[r - H0] = read(at_a[0], r - H0);
+            }
+            if (const int i = copy_behind(n, 8 * H1, CA0); i >= 0) copy_a(filled, i);
+        });
+    }
+    // no copy, of any wave, is on its way to LDS any more; the products have left the matrix pipe
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+        asm volatile("" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
+
+    store_rows<NT, EPI, GROUPED>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
+}
+
+// GROUPED: an expert's last tile may have 128 rows or less; the waves then lie side by side and it takes half as long.
+template <int WM, int NT, int EPI, bool GROUPED>
+__global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const GemmKernelArgs<bf16> p) {
+    extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
+    constexpr int BM = 128 * WM, BN = 16 * NT * (4 / WM);
+    const int tiles_m = GROUPED ? p.tiles[4 * p.tiles_m] : p.tiles_m;
+    const int total = tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= total) return;
+    const int band = tile / (4 * p.tiles_n), in_band = tile % (4 * p.tiles_n);
+    const int rows_in_band = tiles_m - 4 * band < 4 ? tiles_m - 4 * band : 4;
+    const int tm = 4 * band + in_band % rows_in_band, tn = in_band / rows_in_band;
+    const KSlice slice = k_slice(p.K / 64);
+    if constexpr (GROUPED) {
+        const int32_t *t = p.tiles + 4 * tm;
+        const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
+        if (t[2] <= 128) wide_tile<1, NT / 2, EPI, true>(p, gemm_lds, w, t[1], t[1] + t[2], tn * BN, slice);
+        else wide_tile<WM, NT, EPI, true>(p, gemm_lds, w, t[1], t[1] + t[2], tn * BN, slice);
+    } else {
+        wide_tile<WM, NT, EPI, false>(p, gemm_lds, p.w, tm * BM, p.M, tn * BN, slice);
+    }
+}
+
+
+template <class T>
+GemmKernelArgs<T> kernel_args(const GemmArgs &g, int bm, int bn) {
     GemmKernelArgs<T> p;
     p.a = static_cast<const T *>(g.a);
     p.w = static_cast<const T *>(g.w);
@@ -200,18 +506,28 @@ hipError_t launch_tile(const GemmArgs &g, hipStream_t stream) {
     p.w_stride = g.w_stride;
     p.silu_begin = g.silu_begin;
     p.silu_end = g.silu_end;
-    p.tiles_m = g.tiles ? g.n_tiles : (g.M + BM - 1) / BM;
-    p.tiles_n = (g.N + BN - 1) / BN;
-    const int total = p.tiles_m * p.tiles_n, grid = (total + 7) / 8 * 8;
+    p.slice_stride = (long)g.M * g.ldo;
+    p.tiles_m = g.tiles ? g.n_tiles : (g.M + bm - 1) / bm;
+    p.tiles_n = (g.N + bn - 1) / bn;
+    return p;
+}
+
+template <class P>
+hipError_t run_tiles(void (*kernel)(P), const P &p, int threads, size_t lds, int slices, hipStream_t stream) {
+    if (lds > 48 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const int total = p.tiles_m * p.tiles_n;
+    hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8, slices), dim3(threads), lds, stream, p);
+    return hipGetLastError();
+}
+
+template <class T, int BM, int BN, int WM, int WN, int STAGES>
+hipError_t launch_tile(const GemmArgs &g, int slices, hipStream_t stream) {
+    const GemmKernelArgs<T> p = kernel_args<T>(g, BM, BN);
     constexpr size_t lds = STAGES * (size_t)(BM + BN) * kRowBytes;
-    auto run = [&](auto kernel) {
-        if (lds > 48 * 1024) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WM * WN), lds, stream, p);
-        return hipGetLastError();
-    };
+    auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<T>>(kernel, p, 64 * WM * WN, lds, slices, stream); };
     if (g.tiles)
         return g.epilogue == kOutSwiglu ? run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutSwiglu, true>)
                                         : run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutElem, true>);
@@ -223,27 +539,150 @@ hipError_t launch_tile(const GemmArgs &g, hipStream_t stream) {
     }
 }
 
+template <int WM, int NT>
+hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
+    const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, 128 * WM, 16 * NT * (4 / WM));
+    auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, wide_lds(WM, NT), slices, stream); };
+    if constexpr (WM == 2 && NT == 8)
+        if (g.tiles) return g.epilogue == kOutSwiglu ? run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu, true>) : run(&dense_gemm_wide_kernel<WM, NT, kOutElem, true>);
+    switch (g.epilogue) {
+        case kOutF32: return run(&dense_gemm_wide_kernel<WM, NT, kOutF32, false>);
+        case kOutSwiglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu, false>);
+        case kOutGeglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutGeglu, false>);
+        default: return run(&dense_gemm_wide_kernel<WM, NT, kOutElem, false>);
+    }
+}
+
+// out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_sum_kernel(const float *parts, int slices, int M, int N, void *out, long ldo, int silu_begin, int silu_end) {
+    constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
+    const int quads = (kPair ? N / 2 : N) / 4;
+    const long t = (long)blockIdx.x * 256 + threadIdx.x, size = (long)M * N;
+    if (t >= (long)M * quads) return;
+    const long m = t / quads;
+    const int col = (int)(t % quads) * 4;
+    const float *p = parts + m * N + (kPair ? col / 16 * 32 + col % 16 : col);
+    auto sum = [&](const float *q) {
+        floatx4 v = *reinterpret_cast<const floatx4 *>(q);
+        for (int s = 1; s < slices; ++s) v += *reinterpret_cast<const floatx4 *>(q + s * size);
+        return v;
+    };
+    floatx4 v = sum(p);
+    if constexpr (kPair) {
+        const floatx4 up = sum(p + 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (EPI == kOutGeglu ? gelu_tanh_of<bf16>(v[r]) : silu_of<bf16>(v[r])) * up[r];
+    } else if (EPI == kOutElem && col >= silu_begin && col < silu_end) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = silu_of<bf16>(v[r]);
+    }
+    if constexpr (EPI == kOutF32) store4(static_cast<float *>(out) + m * ldo + col, v[0], v[1], v[2], v[3]);
+    else store4(static_cast<bf16 *>(out) + m * ldo + col, v[0], v[1], v[2], v[3]);
+}
+
+// ---- choice of tile and slices ---------------------------------------------------------------------------------------------------
+// A kernel's time: full rounds of its workgroups on 256 CUs (`together` of them to a CU), then a last one whose K-steps are the
+// faster the emptier it is; in us.  Fitted to 18 products of 16 .. 2048 rows, K = 2048 .. 8192, in 1, 2, 4 and 8 slices, each alone
+// on the GPU with cold weights (rms error of the time 4 to 10 %; the choice it leads to is within 8 % of the best kernel's time at 17 of
+// the 18).  M x N x K with the parts added up, before there were slices / now: 64 x 2048 x 8192 130 / 16 us, 300 x 2048 x 8192 79 / 28,
+// 2048 x 2048 x 8192 90 / 71; 64 x 16384 x 2048 with gelu 50 / 13 (64-row tiles).
+// Narrow tiles read W from L2 once per 32 or 64 rows, which costs more in a model, where other kernels have been there, than alone:
+// up to eight of them (2048 x 2048 x 2048 behind an attention: 32 us with 64-row tiles, 25 with wide ones alone).
+struct GemmKind {
+    int rows, cols, together;
+    float tile_us, step_us, step_full_us, store_tbs;   // per tile; per K-step alone and in a full round; fp32 results
+};
+enum : int { kTile32, kTile64, kWide128, kWide192, kWide256, kKinds };
+constexpr GemmKind kGemmKinds[kKinds] = {
+    {32, 128, 2, 1.0f, 0.215f, 0.43f, 6.8f}, {64, 128, 2, 0.f, 0.364f, 0.541f, 3.7f},    {128, 256, 1, 2.6f, 0.566f, 0.696f, 5.8f},
+    {256, 192, 1, 5.8f, 0.728f, 0.947f, 10.3f}, {256, 256, 1, 7.5f, 0.953f, 1.201f, 11.f}};
+float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int slices) {
+    const long tiles = (long)((M + k.rows - 1) / k.rows) * ((N + k.cols - 1) / k.cols) * slices, cap = 256 * k.together;
+    const long full = tiles / cap, rest = tiles % cap;
+    const int per = (steps + slices - 1) / slices;
+    const float mb = 4e-6f * M * N;   // of one part
+    float t = 4.f + full * (k.tile_us + per * k.step_full_us);
+    if (rest) t += k.tile_us + per * (k.step_us + (k.step_full_us - k.step_us) * rest / cap);
+    if (epilogue == kOutF32 || slices > 1) t += slices * mb / k.store_tbs;
+    if (slices > 1) t += epilogue == kOutF32 ? (slices - 1) * mb / 5.f : 3.5f + (slices + 0.5f) * mb / 4.f;   // whoever adds them up
+    return t;
+}
+
+struct GemmChoice {
+    int kind, slices;
+};
+// slices 0: any number
+GemmChoice choose_gemm(int M, int N, int K, int epilogue, int slices) {
+    GemmChoice best{kWide256, 1};
+    float least = 1e30f;
+    const int steps = K / 64, first = slices ? slices : 1, last = slices ? slices : steps >= 8 ? (steps / 4 < 8 ? steps / 4 : 8) : 1;
+    for (int kind = M > 512 ? kWide128 : M > 256 ? kTile64 : kTile32; kind < kKinds; ++kind)
+        for (int n = first; n <= last; n *= 2) {
+            const float t = gemm_time(kGemmKinds[kind], M, N, steps, epilogue, n);
+            if (t < least) {
+                least = t;
+                best = {kind, n};
+            }
+        }
+    return best;
+}
+
+// Rows as long as this do not fit the wide tiles' 32-bit offsets (64 rows of them).
+bool long_rows(const GemmArgs &g) { return g.K >= 1 << 25 || (!g.tiles && g.lda >= 1 << 25); }
+
+hipError_t launch_kind(const GemmArgs &g, int kind, int slices, hipStream_t stream) {
+    if (long_rows(g) && kind > kTile64) kind = kTile64;
+    switch (kind) {
+        case kTile32: return launch_tile<bf16, 32, 128, 1, 4, 4>(g, slices, stream);
+        case kTile64: return launch_tile<bf16, 64, 128, 1, 4, 3>(g, slices, stream);
+        case kWide128: return launch_wide<1, 4>(g, slices, stream);
+        case kWide192: return launch_wide<2, 6>(g, slices, stream);
+        default: return launch_wide<2, 8>(g, slices, stream);
+    }
+}
+
 }  // namespace
 
-// Rows of A per tile for a product of `rows` rows with each of `matrices` matrices.  Measured: full of work, the 256 x 256
-// kernel runs at 1.22 PFLOP/s with one workgroup per CU, the 128 x 128 one at 0.9 to 1.0 with two; each loses what its last
-// round of workgroups leaves idle.  Experts with enough rows take the large tile (their tiles are rarely full in either case).
+// Rows of A per tile for a product of `rows` rows with each of `matrices` matrices.
 int dense_gemm_tile_rows(int dtype, int rows, int N, int matrices) {
     if (rows <= 48 || N < 96) return 32;
     if (dtype != kBf16) return 128;
     if (matrices > 1) return rows >= 160 && N >= 256 ? 256 : 128;
-    const int t256 = ((rows + 255) / 256) * ((N + 255) / 256), t128 = ((rows + 127) / 128) * ((N + 127) / 128);
-    const float e256 = 1.22f * t256 / ((t256 + 255) / 256 * 256);
-    const float e128 = t128 < 512 ? 1.1f * t128 / 512 : 0.88f * t128 / ((t128 + 255) / 256 * 256);
-    return e256 > e128 ? 256 : 128;
+    return rows > 128 ? 256 : 128;
 }
 
 hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStream_t stream) {
-    if (dtype == kF32) return tile_rows == 32 ? launch_tile<float, 32, 128, 1, 4, 4>(g, stream) : launch_tile<float, 128, 128, 2, 2, 2>(g, stream);
-    switch (tile_rows) {
-        case 32: return launch_tile<bf16, 32, 128, 1, 4, 4>(g, stream);
-        case 128: return launch_tile<bf16, 128, 128, 2, 2, 2>(g, stream);
-        default: return launch_tile<bf16, 256, 256, 2, 4, 2>(g, stream);
+    if (dtype == kF32) return tile_rows == 32 ? launch_tile<float, 32, 128, 1, 4, 4>(g, 1, stream) : launch_tile<float, 128, 128, 2, 2, 2>(g, 1, stream);
+    if (tile_rows == 32) return launch_tile<bf16, 32, 128, 1, 4, 4>(g, 1, stream);
+    if (g.tiles) return tile_rows == 128 ? launch_tile<bf16, 128, 128, 2, 2, 2>(g, 1, stream) : long_rows(g) ? hipErrorInvalidValue : launch_wide<2, 8>(g, 1, stream);
+    return launch_kind(g, tile_rows == 256 ? kWide256 : kWide128, 1, stream);
+}
+
+int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue) { return dtype == kBf16 ? choose_gemm(M, N, K, epilogue, 0).slices : 1; }
+
+hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream) {
+    if (dtype != kBf16 || g.tiles) return launch_dense_gemm(dtype, g, dense_gemm_tile_rows(dtype, g.M, g.N, 1), stream);
+    const int kind = choose_gemm(g.M, g.N, g.K, g.epilogue, slices).kind;
+    if (slices == 1) return launch_kind(g, kind, 1, stream);
+    GemmArgs p = g;
+    p.out = parts;
+    p.ldo = g.N;
+    p.epilogue = kOutF32;
+    p.silu_begin = p.silu_end = 0;
+    const hipError_t e = launch_kind(p, kind, slices, stream);
+    if (e != hipSuccess || !g.out) return e;
+    const bool pair = g.epilogue == kOutSwiglu || g.epilogue == kOutGeglu;
+    const long threads = (long)g.M * (pair ? g.N / 2 : g.N) / 4;
+    auto add = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, parts, slices, g.M, g.N, g.out, g.ldo, g.silu_begin, g.silu_end);
+        return hipGetLastError();
+    };
+    switch (g.epilogue) {
+        case kOutF32: return add(&gemm_sum_kernel<kOutF32>);
+        case kOutSwiglu: return add(&gemm_sum_kernel<kOutSwiglu>);
+        case kOutGeglu: return add(&gemm_sum_kernel<kOutGeglu>);
+        default: return add(&gemm_sum_kernel<kOutElem>);
     }
 }
 

@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
 #pragma unroll
             for (int r = 0; r < R; r += 2) {
                 const float a = wave_reduce<false>(acc[r]), b = wave_reduce<false>(acc[r + 1]);
-                mine = lane == r / 2 ? (p.ro.gate == kGateGelu ? gelu_tanh_f32(a) : silu_f32(a)) * b : mine;
+                mine = lane == r / 2 ? (p.ro.gate == kGateGelu ? gelu_tanh_of<float>(a) : silu_f32(a)) * b : mine;
             }
             const int o = g * (R / 2) + lane;
             if (lane < R / 2 && 2 * o < p.N) p.out[o] = from_float<T>(mine);

@@ -84,15 +84,20 @@ struct GemmArgs {
 };
 int dense_gemm_tile_rows(int dtype, int rows, int N, int matrices);   // rows of a tile (what launch_moe_plan gets as bm)
 hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStream_t stream);
+// The same, not grouped, with tile and slices along K by shape.  More than one slice: parts holds slices * M * N floats, part after
+// part, that a second launch adds up; g.out == NULL (kOutF32): they are left to the caller.
+int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue);
+hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream);
 
-// v = embed[tokens] * scale, or res + y, or res; res = v; h (optional) = the norm norm_w of v in the element type
-hipError_t launch_add_norm_rows(int dtype, float *res, const float *y, const int32_t *tokens, const void *embed, float scale, const float *norm_w,
+// v = embed[tokens] * scale, or res + y, or res; y: the sum of `parts` matrices [M, width]; res = v; h (optional) = the norm norm_w of v in the element type
+hipError_t launch_add_norm_rows(int dtype, float *res, const float *y, int parts, const int32_t *tokens, const void *embed, float scale, const float *norm_w,
                                 float eps, int true_width, void *h, int M, int width, hipStream_t stream);
 hipError_t launch_embed_rows(int dtype, const int32_t *tokens, const void *embed, float scale, float *res, void *h, int M, int width,
                              hipStream_t stream);
 // res += y / rms(y) * norm_w per row; h = res in the element type.  With weights (experts): y is [M * top, width] in the
-// element type and the row is sum_s weights[m, s] y[m * top + s]; otherwise y is fp32 [M, width].
-hipError_t launch_residual_norm_rows(int dtype, float *res, const void *y, const float *weights, int top, const float *norm_w, float eps,
+// element type and the row is sum_s weights[m, s] y[m * top + s]; otherwise y is the sum of
+// `parts` fp32 matrices [M, width].
+hipError_t launch_residual_norm_rows(int dtype, float *res, const void *y, int parts, const float *weights, int top, const float *norm_w, float eps,
                                      int true_width, void *h, int M, int width, hipStream_t stream);
 // out[i] = norm of res[rows[i]] (rows nullptr: i)
 hipError_t launch_norm_rows(int dtype, const float *res, const int32_t *rows, const float *norm_w, float eps, int true_width, void *out, int n,

@@ -31,10 +31,21 @@ __global__ void __launch_bounds__(kRowThreads) embed_rows_kernel(const int32_t *
     }
 }
 
+// y[m] of a row's four elements: the sum of `parts` matrices [M][width] (a product's slices along K)
+__device__ __forceinline__ void load_parts(const float *y, int parts, size_t size, float (&v)[4]) {
+    load4(y, v);
+    for (int s = 1; s < parts; ++s) {
+        float u[4];
+        load4(y + s * size, u);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += u[j];
+    }
+}
+
 // Y: type of y; top > 0: y holds `top` rows per token, summed with the router's weights (kept in LDS between the passes)
 template <class T, class Y>
-__global__ void __launch_bounds__(kRowThreads) residual_norm_kernel(float *res, const Y *y, const float *weights, int top, const float *norm_w, float eps,
-                                                                    int true_width, T *h, int width) {
+__global__ void __launch_bounds__(kRowThreads) residual_norm_kernel(float *res, const Y *y, int parts, const float *weights, int top, const float *norm_w,
+                                                                    float eps, int true_width, T *h, int width) {
     extern __shared__ float sum_lds[];
     __shared__ float red[4];
     const size_t m = blockIdx.x;
@@ -51,8 +62,8 @@ __global__ void __launch_bounds__(kRowThreads) residual_norm_kernel(float *res, 
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = fmaf(wt, u[j], v[j]);
             }
-        } else {
-            load4(y + m * width + i, v);
+        } else if constexpr (sizeof(Y) == 4) {
+            load_parts(y + m * width + i, parts, (size_t)gridDim.x * width, v);
         }
         store4(sum_lds + i, v[0], v[1], v[2], v[3]);   // read back by the same thread
 #pragma unroll
@@ -94,8 +105,8 @@ __global__ void __launch_bounds__(kRowThreads) norm_rows_kernel(const float *res
 
 // the residual brought up to date and its norm: what the sublayers of a model with norms on their inputs read
 template <class T>
-__global__ void __launch_bounds__(kRowThreads) add_norm_rows_kernel(float *res, const float *y, const int32_t *tokens, const T *embed, float scale,
-                                                                    const float *norm_w, float eps, int true_width, T *h, int width) {
+__global__ void __launch_bounds__(kRowThreads) add_norm_rows_kernel(float *res, const float *y, int parts, const int32_t *tokens, const T *embed,
+                                                                    float scale, const float *norm_w, float eps, int true_width, T *h, int width) {
     extern __shared__ float sum_lds[];
     __shared__ float red[4];
     const size_t m = blockIdx.x;
@@ -111,7 +122,7 @@ __global__ void __launch_bounds__(kRowThreads) add_norm_rows_kernel(float *res, 
             load4(res + m * width + i, v);
             if (y) {
                 float u[4];
-                load4(y + m * width + i, u);
+                load_parts(y + m * width + i, parts, (size_t)gridDim.x * width, u);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] += u[j];
             }
@@ -133,14 +144,14 @@ __global__ void __launch_bounds__(kRowThreads) add_norm_rows_kernel(float *res, 
 
 }  // namespace
 
-hipError_t launch_add_norm_rows(int dtype, float *res, const float *y, const int32_t *tokens, const void *embed, float scale, const float *norm_w,
+hipError_t launch_add_norm_rows(int dtype, float *res, const float *y, int parts, const int32_t *tokens, const void *embed, float scale, const float *norm_w,
                                 float eps, int true_width, void *h, int M, int width, hipStream_t stream) {
     const size_t lds = (size_t)width * sizeof(float);   // (the C ABI keeps width within 64 KiB)
     if (dtype == kF32)
-        hipLaunchKernelGGL(add_norm_rows_kernel<float>, dim3(M), dim3(kRowThreads), lds, stream, res, y, tokens, static_cast<const float *>(embed), scale,
+        hipLaunchKernelGGL(add_norm_rows_kernel<float>, dim3(M), dim3(kRowThreads), lds, stream, res, y, parts, tokens, static_cast<const float *>(embed), scale,
                            norm_w, eps, true_width, static_cast<float *>(h), width);
     else
-        hipLaunchKernelGGL(add_norm_rows_kernel<bf16>, dim3(M), dim3(kRowThreads), lds, stream, res, y, tokens, static_cast<const bf16 *>(embed), scale, norm_w,
+        hipLaunchKernelGGL(add_norm_rows_kernel<bf16>, dim3(M), dim3(kRowThreads), lds, stream, res, y, parts, tokens, static_cast<const bf16 *>(embed), scale, norm_w,
                            eps, true_width, static_cast<bf16 *>(h), width);
     return hipGetLastError();
 }
@@ -156,18 +167,18 @@ hipError_t launch_embed_rows(int dtype, const int32_t *tokens, const void *embed
     return hipGetLastError();
 }
 
-hipError_t launch_residual_norm_rows(int dtype, float *res, const void *y, const float *weights, int top, const float *norm_w, float eps,
+hipError_t launch_residual_norm_rows(int dtype, float *res, const void *y, int parts, const float *weights, int top, const float *norm_w, float eps,
                                      int true_width, void *h, int M, int width, hipStream_t stream) {
     const size_t lds = (size_t)width * sizeof(float);   // (the C ABI keeps width within 64 KiB)
     if (!weights) top = 0;
     if (dtype == kF32)
-        hipLaunchKernelGGL((residual_norm_kernel<float, float>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const float *>(y), weights, top,
+        hipLaunchKernelGGL((residual_norm_kernel<float, float>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const float *>(y), parts, weights, top,
                            norm_w, eps, true_width, static_cast<float *>(h), width);
     else if (top > 0)
-        hipLaunchKernelGGL((residual_norm_kernel<bf16, bf16>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const bf16 *>(y), weights, top,
+        hipLaunchKernelGGL((residual_norm_kernel<bf16, bf16>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const bf16 *>(y), parts, weights, top,
                            norm_w, eps, true_width, static_cast<bf16 *>(h), width);
     else
-        hipLaunchKernelGGL((residual_norm_kernel<bf16, float>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const float *>(y), weights, top,
+        hipLaunchKernelGGL((residual_norm_kernel<bf16, float>), dim3(M), dim3(kRowThreads), lds, stream, res, static_cast<const float *>(y), parts, weights, top,
                            norm_w, eps, true_width, static_cast<bf16 *>(h), width);
     return hipGetLastError();
 }

@@ -1,0 +1,131 @@
+"""Products over many rows at the edges of their tiles and slices, against float64 products of the same bf16 numbers.
+
+fp32 results: sums of K products of 16 significant bits in fp32, any order, stay within K 2^-24 of the sum of magnitudes, which for
+random signs is about K^1/2 times the result's rms; 2^-24 K^3/2 is 4e-5 at K = 8192, and what is seen is 30 times less.  bf16 results add
+half an ulp of the value, 2^-8 with the rounding to either neighbour."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dense():
+    from air_hip import dense as d
+    return d
+
+
+def rand(seed, *shape):
+    return torch.randn(shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed))
+
+
+def close(got, want, bf16, what):
+    rms = want.square().mean().sqrt()
+    bound = 4e-5 * rms + (2.0 ** -8 * want.abs() if bf16 else 0.0)
+    bad = (got.double() - want).abs() > bound
+    assert not bad.any(), (what, int(bad.sum()), bad.nonzero()[0].tolist())
+
+
+def interleaved(g, u):
+    n, K = g.shape
+    return torch.stack([g.reshape(n // 16, 16, K), u.reshape(n // 16, 16, K)], 1).reshape(2 * n, K).contiguous()
+
+
+SHAPES = [(1, 16, 64, 1), (17, 144, 192, 3), (31, 96, 1024, 8), (33, 272, 128, 2), (64, 400, 512, 4), (127, 256, 576, 5), (128, 528, 64, 1), (129, 784, 320, 2),
+          (255, 240, 704, 4), (256, 512, 128, 2), (257, 1040, 448, 7), (300, 2048, 8192, 8), (513, 208, 640, 1), (700, 1104, 1216, 2), (1025, 3088, 192, 1)]
+
+
+@pytest.mark.parametrize("M,N,K,slices", SHAPES)
+def test_sliced_products(dense, M, N, K, slices):
+    print("sliced", M, N, K, slices, flush=True)
+    from air_hip import _lib
+    lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
+    a, w = rand(M, M, K + 64).bfloat16()[:, 8:K + 8], (rand(N + 1, N, K) * K ** -0.5).bfloat16()
+    want = a.double() @ w.double().t()
+    pair = N // 32 * 32
+    silu, gelu = torch.nn.functional.silu, lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    for n in {1, slices, lib.dlm_gemm_slices(0, M, N, K, dense.OUT_F32)}:
+        for epilogue in (dense.OUT_F32, dense.OUT_ELEM, dense.OUT_SWIGLU, dense.OUT_GEGLU):
+            cols, width = (N, N) if epilogue < 2 else (pair, pair // 2)
+            if not cols:
+                continue
+            out = torch.full((M, width + 8), 7.0, device="cuda", dtype=torch.float32 if epilogue == dense.OUT_F32 else torch.bfloat16)
+            parts = torch.empty((n, M, cols), device="cuda")
+            begin, end = (16, N // 32 * 16) if epilogue == dense.OUT_ELEM else (0, 0)
+            g = _lib.GemmArgs(a=a.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), lda=a.stride(0), ldo=width + 8, M=M, N=cols, K=K, epilogue=epilogue,
+                              silu_begin=begin, silu_end=end)
+            _lib.check_dense(lib.dlm_gemm_sliced(0, ctypes.byref(g), n, parts.data_ptr(), stream))
+            ref = want[:, :cols].clone()
+            if epilogue >= 2:
+                q = ref.reshape(M, -1, 2, 16)
+                ref = ((silu if epilogue == dense.OUT_SWIGLU else gelu)(q[:, :, 0]) * q[:, :, 1]).reshape(M, width)
+            elif begin < end:
+                ref[:, begin:end] = silu(ref[:, begin:end])
+            close(out[:, :width], ref, epilogue != dense.OUT_F32, (n, epilogue))
+            assert (out[:, width:] == 7.0).all(), "columns past the width were written"
+
+
+@pytest.mark.parametrize("M,K", [(3, 64), (300, 2048)])
+def test_parts_meet_in_the_row_kernels(dense, M, K):
+    a, w = rand(1, M, 512).bfloat16(), (rand(2, K, 512) * 512 ** -0.5).bfloat16()
+    res, nw = rand(3, M, K), 1.0 + 0.1 * rand(4, K)
+    y = a.double() @ w.double().t()
+    parts = torch.stack([dense.gemm(a[:, i:i + 64].contiguous(), w[:, i:i + 64].contiguous(), out_f32=True) for i in range(0, 512, 64)])
+    norm = lambda v: v / torch.sqrt(v.square().mean(-1, keepdim=True) + 1e-5) * nw.double()
+    for dtype in (torch.float32, torch.bfloat16):
+        r = res.clone()
+        h = dense.residual_norm_rows(r, parts, nw, 1e-5, K, dtype)
+        close(r, res.double() + norm(y), False, "residual")
+        close(h, res.double() + norm(y), dtype == torch.bfloat16, "residual, element type")
+        r = res.clone()
+        h = dense.add_norm_rows(r, parts, nw, 1e-5, K, dtype)
+        close(r, res.double() + y, False, "sum")
+        close(h, norm(res.double() + y), dtype == torch.bfloat16, "norm of the sum")
+    assert dense.gemm(a, w, out_f32=True, parts=True).shape[1:] == (M, K)
+
+
+COUNTS = [(0, 1, 15, 128, 129, 255, 256, 257), (512, 0, 0, 300, 64, 127, 383, 385), (16, 16, 16, 16, 16, 16, 16, 16), (0, 0, 0, 700, 0, 0, 0, 0)]
+
+
+@pytest.mark.parametrize("tile_rows", [32, 128, 256])
+@pytest.mark.parametrize("counts", COUNTS)
+def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows):
+    print("experts", counts, tile_rows, flush=True)
+    from air_hip import _lib
+    lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
+    E, K, ff, N, top = len(counts), 192, 144, 272, 2
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    if len(ids) % top:
+        ids = torch.cat([ids, ids[-1:]])
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(5))].to(torch.int32).cuda()
+    entries = len(ids)
+    h = rand(6, entries // top, K).bfloat16()
+    gate, up = ((rand(7 + i, E, ff, K) * K ** -0.5).bfloat16() for i in range(2))
+    w1, w2 = torch.stack([interleaved(g, u) for g, u in zip(gate, up)]), (rand(9, E, N, 192) * ff ** -0.5).bfloat16()
+    order = torch.empty((entries,), dtype=torch.int32, device="cuda")
+    n_tiles = lib.dlm_moe_max_tiles(entries, E, tile_rows)
+    tiles = torch.empty((n_tiles + 1, 4), dtype=torch.int32, device="cuda")
+    _lib.check_dense(lib.dlm_moe_plan(ids.data_ptr(), entries, E, tile_rows, order.data_ptr(), tiles.data_ptr(), stream))
+    act = torch.zeros((entries, 192), dtype=torch.bfloat16, device="cuda")
+    out = torch.full((entries, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    common = dict(tiles=tiles.data_ptr(), order=order.data_ptr(), M=entries, n_tiles=n_tiles, tile_rows=tile_rows)
+    g = _lib.GemmArgs(a=h.data_ptr(), w=w1.data_ptr(), out=act.data_ptr(), lda=K, ldo=192, w_stride=2 * ff * K, N=2 * ff, K=K, epilogue=dense.OUT_SWIGLU,
+                      gather=top, **common)
+    _lib.check_dense(lib.dlm_gemm(0, ctypes.byref(g), stream))
+    g = _lib.GemmArgs(a=act.data_ptr(), w=w2.data_ptr(), out=out.data_ptr(), lda=192, ldo=N, w_stride=N * 192, N=N, K=192, epilogue=dense.OUT_ELEM, gather=0,
+                      **common)
+    _lib.check_dense(lib.dlm_gemm(0, ctypes.byref(g), stream))
+    e, token = ids.long(), torch.arange(entries, device="cuda") // top
+    for i in range(E):
+        at = (e == i).nonzero()[:, 0]
+        if not len(at):
+            continue
+        x = h[token[at]].double()
+        a = torch.nn.functional.silu(x @ gate[i].double().t()) * (x @ up[i].double().t())
+        place = torch.empty((entries,), dtype=torch.long, device="cuda")
+        place[order.long()] = torch.arange(entries, device="cuda")
+        got = act[place[at]]
+        close(got[:, :ff], a, True, ("gate / up", i))
+        close(out[at], got.double() @ w2[i].double().t(), True, ("down", i))
