@@ -37,7 +37,7 @@ CONFIGS = {
     # the same product on the AutoAWQ checkpoint layout (split-K kernel with a workspace)
     "gemv_awq": dict(M=1, K=4096, N=11008, cfg=None, desc="decode GEMV W4A16 M=1 K=4096 N=11008 g128, checkpoint-layout weights"),
     "gemm16": dict(M=16, K=4096, N=14336, cfg=2, desc="batched decode GEMM W4A16 M=16 K=4096 N=14336 g128, stream-order weights"),
-    # the same product for a batch of 64 (split along K, a launch of four row tiles plus the launch that adds the slices;
+    # the same product for a batch of 64 (tiles of rows and columns, the second one in slices of K plus the launch that adds them;
     # no BASELINE config)
     "gemm64": dict(M=64, K=4096, N=14336, cfg=None, desc="batched decode GEMM W4A16 M=64 K=4096 N=14336 g128, stream-order weights"),
     "gemm64_down": dict(M=64, K=14336, N=4096, cfg=None, desc="batched decode GEMM W4A16 M=64 K=14336 N=4096 g128 (down projection), stream-order weights, split along K"),
@@ -294,7 +294,7 @@ def run_workload(name, steps, warmup, with_cpu_baseline):
         elif name == "probe":
             rc = lib.w4a16_probe_stream_read(w[0].data_ptr(), probe_out.data_ptr(), K, N, st)
         elif name in ("gemm16", "gemm64", "gemm64_down", "prefill"):
-            # (17 .. 128 rows: split along K with plain scratch; other row counts take no scratch)
+            # (exact products of 17 rows and more: slices of K with plain scratch; others take no scratch)
             rc = lib.w4a16_gemm_stream_scratch_bf16(x.data_ptr(), w[0].data_ptr(), outs[0].data_ptr(), M, K, N, 128,
                                                     gemm_scratch.data_ptr(), gemm_scratch.numel(), st)
         elif name == "q4nx_gemv":
@@ -1067,7 +1067,7 @@ def main():
     if t:
         roof["traffic_measured_at"] = {"commit": t["commit"], "profile": t["profile"]}
     roof["kernel"] = {"dequant": "dequant_kernel", "prefill": "gemm_wsp_kernel", "q4nx_prefill": "gemm_wsp_kernel", "q4nx_gemv": "gemv_ws_kernel", "q4nx_gemm16": "gemm_ws_kernel", "prefill_awq": "gemm_kernel", "lm_head": "lm_head_kernel",
-                      "gemv": "gemv_ws_kernel", "probe": "probe_ws_kernel", "gemm16": "gemm_ws_kernel", "gemm64": "gemm_ws_rows_kernel", "gemm64_down": "gemm_wsk_kernel", "ffn": "gemv_ws_kernel", "block": "gemv_ws_kernel", "layer": "gemv_ws_kernel"}.get(name, "stream_kernel")
+                      "gemv": "gemv_ws_kernel", "probe": "probe_ws_kernel", "gemm16": "gemm_ws_kernel", "gemm64": "gemm_wsm_kernel", "gemm64_down": "gemm_wsm_kernel", "ffn": "gemv_ws_kernel", "block": "gemv_ws_kernel", "layer": "gemv_ws_kernel"}.get(name, "stream_kernel")
     roof["algorithmic_per_launch"] = main_res["flops"] if name in ("prefill", "prefill_awq", "q4nx_prefill") else main_res["bytes"]
     roof["avg_launch_us"] = main_res["cold_us"]
 

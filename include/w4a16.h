@@ -223,30 +223,27 @@ int w4a16_gemv_add_stream_bf16(const uint16_t *x, const void *wstream, const uin
 int w4a16_probe_stream_read(const void *wstream, uint32_t *out_words, int K, int N, void *stream);
 /* Batched decode on a stream-order matrix: y[M, N] = bf16(x[M, K] . W), unrounded weights, fp32 accumulation
  * (matmul_int4_packed.cpu_reference, programming_examples/matrix_multiplication/int4_awq/matmul_int4_packed.py:89-105;
- * device kernel matmul_int4_bf16_packed_f32, mv_int4_bf16.cc:430-448).  Up to 64 rows per launch stream the weights
- * once (M <= 128: launches of 64 rows and a rest, the second over cache-resident weights); stateless like the GEMV.  From
- * M = 129 on,
- * with K % 256 == 0 and N % 64 == 0 (N / 64 = 3, 4 or >= 6), the tiled prefill kernel runs instead: it dequantises the
- * weights to bf16 in registers (W = bf16_rne((q - z) * s), the dense dequant's values) and feeds bf16 MFMA with fp32
- * accumulation; other shapes stay with the launches of 64 rows.  So the numerics change between M = 128 and M = 129:
+ * device kernel matmul_int4_bf16_packed_f32, mv_int4_bf16.cc:430-448).  16 rows a launch, or more rows in one launch of
+ * row and column tiles, by their expected times; stateless like the GEMV.  From M = 129 on, with K % 256 == 0 and
+ * N % 64 == 0, the weights are dequantised to bf16 in registers (W = bf16_rne((q - z) * s), the dense dequant's values)
+ * and multiplied by bf16 MFMA with fp32 accumulation.  So the numerics change between M = 128 and M = 129:
  * below, y is one rounding of the fp32 sum over exact weights (q - z) s, as the reference's cpu_reference computes it;
  * above, the weights carry one more bf16 rounding each (relative 2^-9), which moves y by at most 2^-9 sum |x w| and
- * stays inside the reference's gate (rtol 0.1, atol 0.05, 0.05 % budget, r >= 0.999); a caller that needs the same
- * bits for every M keeps M <= 128 per call.  K % 128 == 0, N % 16 == 0. */
+ * stays inside the reference's gate (rtol 0.1, atol 0.05, 0.05 % budget, r >= 0.999); a caller that needs exact
+ * weights for every M keeps M <= 128 per call.  K % 128 == 0, N % 16 == 0. */
 int w4a16_gemm_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group,
                            void *stream);
-/* w4a16_gemm_stream_bf16 with plain scratch for the shapes where 17 .. 128 rows run faster split along K (same
+/* w4a16_gemm_stream_bf16 with plain scratch, for exact products of 17 rows and more (same
  * reference, matmul_int4_packed.py:89-105; the reference's own kernel also walks K in slices, one L1 K-chunk at a
- * time, and adds them in an fp32 accumulator, matmul_int4_packed.py:179-181, 293-345).  A workgroup takes 256 columns and a slice of K, shares
- * the x rows of its slice through LDS and writes fp32 partial sums to `scratch`; a second launch adds the slices in
- * slice order and rounds once.  That pays where the whole-K launches re-read the x rows most: K >= 4096, rows * K / 128
- * >= 1536 and N < 12800 (K = 14336, N = 4096, 64 rows: 27.9 us against 59.0 us; K = 4096, N = 6144: 18.1 against 34.2);
- * for every other shape and row count the call is w4a16_gemm_stream_bf16 itself and `scratch` is not touched.
- * w4a16_gemm_stream_scratch_bytes(M, K, N) is the scratch the call needs (0 where it takes none): no initialisation,
+ * time, and adds them in an fp32 accumulator, matmul_int4_packed.py:179-181, 293-345).  A workgroup takes a tile of rows and
+ * columns and a slice of K and writes fp32 partial sums to `scratch`; a second launch adds the slices in slice order and
+ * rounds once.  As many slices are taken as pay and fit (64 rows of K = 14336, N = 4096: 18 us with four, 32 us without).
+ * w4a16_gemm_stream_scratch_bytes(M, K, N) is the scratch the call insists on (0: any, also none), and
+ * w4a16_gemm_stream_best_scratch_bytes what the fastest plan takes (0: none): no initialisation,
  * nothing kept between calls, 16-byte aligned; calls that overlap on one GPU need a buffer each.  Same numerics as
- * w4a16_gemm_stream_bf16 below 129 rows (exact weights, fp32 sums, one rounding); the two differ by the order of the
- * fp32 additions only. */
+ * w4a16_gemm_stream_bf16; the two differ by the order of the fp32 additions only. */
 size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N);
+size_t w4a16_gemm_stream_best_scratch_bytes(int M, int K, int N);
 int w4a16_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group,
                                    void *scratch, size_t scratch_bytes, void *stream);
 int w4a16_gemv_swiglu_stream_bf16(const uint16_t *x, const void *gate_wstream, const void *up_wstream,
@@ -552,14 +549,19 @@ int w4a16_q4nx_repack_stream(const int32_t *qweight, const uint16_t *scales, con
                              void *stream);
 int w4a16_q4nx_gemv_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int K, int N,
                                 void *stream);
-/* y[M, N] = bf16(x[M, K] . W + residual [M, N]): the GEMV at M = 1, the batched whole-K kernel in launches of 16 rows
- * above (exact weights s q + min', fp32 sums, one rounding).  From M = 65 on, without a residual and with K % 256 == 0,
- * N % 64 == 0, the tiled MFMA kernel of w4a16_gemm_stream_bf16 runs on the Q4NX order: it dequantises each K-step of a
+/* y[M, N] = bf16(x[M, K] . W + residual [M, N]): the GEMV at M = 1, launches of 16 rows or of row and column tiles above
+ * (weights s q + min' to 16 significant bits or more, fp32 sums, one rounding).  From M = 65 on, without a residual and with K % 256 == 0,
+ * N % 64 == 0, the tiled MFMA kernels of w4a16_gemm_stream_bf16 run on the Q4NX order: they dequantise each K-step of a
  * cell with its own (scale, min') word to W = bf16_rne(s q + min'), the dense dequant's values (q4nx_dequant_bf16,
- * bit for bit), and multiplies those, which is what the reference's prompt pass of these models computes with its
- * dense bf16 GEMMs on dequantised weights (programming_examples/llms/llama31_8b_q4nx/README.md:11-15). */
+ * bit for bit), and multiply those, which is what the reference's prompt pass of these models computes with its
+ * dense bf16 GEMMs on dequantised weights (programming_examples/llms/llama31_8b_q4nx/README.md:11-15).
+ * With scratch (may be NULL; w4a16_q4nx_gemm_stream_best_scratch_bytes is what the fastest plan takes, 0: none) as
+ * w4a16_gemm_stream_scratch_bf16. */
 int w4a16_q4nx_gemm_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,
                                 void *stream);
+size_t w4a16_q4nx_gemm_stream_best_scratch_bytes(int M, int K, int N, int has_residual);
+int w4a16_q4nx_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,
+                                        void *scratch, size_t scratch_bytes, void *stream);
 /* The two prompt-pass blocks (w4a16_prefill_rms_qkv_rope_stream_bf16, w4a16_prefill_o_ffn_stream_bf16: same arguments
  * without `group`, same stages, rounding points and workspaces) on matrices in Q4NX order: the reference runs these
  * stages op by op as bf16 GEMM / RMSNorm / RoPE / SwiGLU on the dequantised weights
@@ -587,7 +589,7 @@ int w4a16_q4nx_o_gemv_ffn_stream_bf16(const uint16_t *attn_out, const uint16_t *
  * "gemv_spin_limit" (reducer poll bound), "gemv_skip_publish" (fault injection for the
  * timeout test: split-K producers do not publish), "gemv_ws_ct", "gemv_ws_waves",
  * "gemm_ws_cb", "gemm_ws_rows" (stream-order GEMV / small-batch shapes; rows: most rows per batched launch, 16, 32 or 64), "prefill_tile" (one tile width only, 1: 256 columns, 2: 192, 3: 128,
- * 4: 64; 5: 256 mixed with 128 in the launches that take that mix; 0: by shape), "prefill_min_m" (smallest M given to the tiled prefill kernel), "prefill_band" (row panels per band of its tile order), "gemm_splitk" (w4a16_gemm_stream_scratch_bf16 at 17 .. 128 rows: 0 split along K by shape, 1 always, 2 never) and "prefill_swiglu_split" (1: the
+ * 4: 64; 5: 256 mixed with 128 in the launches that take that mix; 0: by shape), "prefill_min_m" (smallest M given to the tiled prefill kernel), "prefill_band" (row panels per band of its tile order), "gemm_splitk" (exact products of 17 rows and more: 0 by shape, 1 always tiles and slices, 2 always whole-K launches) and "prefill_swiglu_split" (1: the
  * stream-order prompt-pass FFN runs its gate and up projections as two launches instead of one; same bits).  Process-wide.
  */
 int w4a16_tune(const char *key, int value);

@@ -57,6 +57,8 @@ SYMBOLS = {
     "w4a16_q4nx_repack_stream": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _vp]),
     "w4a16_q4nx_gemv_stream_bf16": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _vp]),
     "w4a16_q4nx_gemm_stream_bf16": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp]),
+    "w4a16_q4nx_gemm_stream_best_scratch_bytes": (_sz, [_ci, _ci, _ci, _ci]),
+    "w4a16_q4nx_gemm_stream_scratch_bf16": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp, _sz, _vp]),
     "w4a16_q4nx_rms_gemv_stream_bf16": (_ci, [_vp, _vp, _ci, _vp, _cf, _vp, _vp, _ci, _ci, _vp]),
     "w4a16_q4nx_o_gemv_ffn_stream_bf16": (_ci, [_vp, _vp, _vp, _cf] + [_vp] * 8 + [_ci, _ci, _vp, _sz, _vp]),
     "w4a16_stream_bytes": (_sz, [_ci, _ci]),
@@ -65,6 +67,7 @@ SYMBOLS = {
     "w4a16_probe_stream_read": (_ci, [_vp, _vp, _ci, _ci, _vp]),
     "w4a16_gemm_stream_bf16": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp]),
     "w4a16_gemm_stream_scratch_bytes": (_sz, [_ci, _ci, _ci]),
+    "w4a16_gemm_stream_best_scratch_bytes": (_sz, [_ci, _ci, _ci]),
     "w4a16_gemm_stream_scratch_bf16": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _sz, _vp]),
     "w4a16_gemv_add_stream_bf16": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp]),
     "w4a16_gemv_swiglu_stream_bf16": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp]),

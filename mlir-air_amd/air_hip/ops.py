@@ -265,13 +265,14 @@ def w4a16_gemv_stream(x, w, residual=None, group=GROUP, out=None):
     return out
 
 
-_gemm_scratch = {}
+def _gemm_scratch(nbytes, device):
+    """Plain scratch of one call (or None, 0): of the caller's stream and, in a capture, of its graph."""
+    return (torch.empty(int(nbytes), dtype=torch.uint8, device=device), int(nbytes)) if nbytes else (None, 0)
 
 
 def w4a16_gemm_stream(x, w, group=GROUP, out=None):
-    """y[M, N] = bf16(x[M, K] . W) on a StreamWeight; x may be a vector [K].  Batches of 17 to 128 rows run split along
-    K with their partial sums in a scratch buffer of this module (plain scratch per device and stream, grown on
-    demand, nothing kept in it between calls)."""
+    """y[M, N] = bf16(x[M, K] . W) on a StreamWeight; x may be a vector [K].  Batches of 17 rows and more run in slices of
+    K where that is the faster way, their partial sums in plain scratch of the call."""
     lib = _lib.load_library()
     _need_cuda(x, w.buf)
     _need_order("awq", w)
@@ -282,16 +283,9 @@ def w4a16_gemm_stream(x, w, group=GROUP, out=None):
         raise ValueError(f"x has K={K} but the matrix has {w.K} rows")
     if out is None:
         out = torch.empty((M, w.N), dtype=torch.bfloat16, device=x.device)
-    need = lib.w4a16_gemm_stream_scratch_bytes(M, K, w.N)
-    if need:
-        key = (x.device.index, _stream())
-        scratch = _gemm_scratch.get(key)
-        if scratch is None or scratch.numel() < need:
-            scratch = _gemm_scratch[key] = torch.empty(int(need), dtype=torch.uint8, device=x.device)
-        _lib.check(lib.w4a16_gemm_stream_scratch_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group, _ptr(scratch),
-                                                      scratch.numel(), _stream()))
-    else:
-        _lib.check(lib.w4a16_gemm_stream_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group, _stream()))
+    scratch, nbytes = _gemm_scratch(lib.w4a16_gemm_stream_best_scratch_bytes(M, K, w.N) if M > 16 else 0, x.device)
+    _lib.check(lib.w4a16_gemm_stream_scratch_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group,
+                                                  _ptr(scratch) if nbytes else None, nbytes, _stream()))
     return out.squeeze(0) if vec else out
 
 
@@ -850,8 +844,9 @@ def q4nx_gemm_stream(x, w, residual=None, out=None):
         raise ValueError("q4nx_gemm_stream: x must be [M, K], residual [M, N]")
     if out is None:
         out = torch.empty((M, w.N), dtype=torch.bfloat16, device=x.device)
-    _lib.check(lib.w4a16_q4nx_gemm_stream_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(_bits(residual)) if residual is not None else None,
-                                               _ptr(out), M, K, w.N, _stream()))
+    scratch, nbytes = _gemm_scratch(lib.w4a16_q4nx_gemm_stream_best_scratch_bytes(M, K, w.N, residual is not None) if M > 16 else 0, x.device)
+    _lib.check(lib.w4a16_q4nx_gemm_stream_scratch_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(_bits(residual)) if residual is not None else None,
+                                                       _ptr(out), M, K, w.N, _ptr(scratch) if nbytes else None, nbytes, _stream()))
     return out.squeeze(0) if vec else out
 
 

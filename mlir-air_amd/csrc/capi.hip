@@ -542,42 +542,78 @@ int w4a16_gemv_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, 
     return gemv_stream_call(x, wstream, nullptr, y, K, N, group, stream, GemvWsExtras());
 }
 
-int w4a16_gemm_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group, void *stream) {
+// Products of 2 rows and more, whose arguments have been checked.  By precision: bf16-rounded weights from 129 rows on (Q4NX: 65, and
+// not with a residual, which is added in fp32 before the one rounding) where the tiled kernel takes the shape, else exact ones.  Between
+// the kernels of each kind by their estimated times (us, 64 and 300 rows of K = 14336, N = 4096: whole-K launches 55, tiled 150;
+// gemm_wsm 18 with slices and 32 without, 73; 2048 rows of K = 4096, N = 14336: tiled 172, gemm_wsm 275).
+static bool gemm_stream_rounded(int M, int K, int N, bool q4, bool residual) {
+    const int least = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : q4 ? 65 : kGemmWsMaxM + 1;
+    return M >= least && !(q4 && residual) && gemm_prefill_ws_supported(M, K, N);
+}
+
+// The plan of gemm_wsm.hip with at most `scratch_bytes` of scratch; us < 0: another kernel takes the product
+static WsmPlan gemm_stream_plan(int M, int K, int N, bool q4, bool residual, size_t scratch_bytes) {
+    const auto &tune = g_gemv_ws_tune;
+    const bool rounded = gemm_stream_rounded(M, K, N, q4, residual);
+    WsmPlan p;
+    p.us = -1;
+    if (!gemm_wsm_supported(M, K, N) || (rounded ? tune.prefill_tile != 0 : tune.gemm_rows || tune.cb || tune.splitk == 2)) return p;
+    p = plan_gemm_wsm(M, K, N, q4, rounded, scratch_bytes);
+    const bool always = !rounded && tune.splitk == 1;
+    if (!always && p.us > 0.95 * (rounded ? gemm_prefill_ws_us(M, K, N, q4) : gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
+    return p;
+}
+
+static int gemm_stream_run(const uint16_t *x, const void *w, const uint16_t *residual, uint16_t *y, int M, int K, int N, bool q4, void *scratch,
+                           size_t scratch_bytes, void *stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool rounded = gemm_stream_rounded(M, K, N, q4, residual != nullptr);
+    const WsmPlan plan = gemm_stream_plan(M, K, N, q4, residual != nullptr, scratch ? scratch_bytes : 0);
+    hipError_t e = plan.us >= 0 ? launch_gemm_wsm(plan, x, w, y, residual, static_cast<float *>(scratch), M, K, N, q4, rounded, st)
+                   : rounded    ? launch_gemm_prefill_ws(x, w, y, M, K, N, st, kEpiNone, nullptr, nullptr, q4)
+                                : launch_gemm_ws(x, w, y, residual, M, K, N, st, q4);
+    return e == hipSuccess ? W4A16_OK : hip_fail(e);
+}
+
+// Slices of at least four groups, 256 workgroups of 256 columns, 64 rows: what the call insists on where whole-K launches are slowest
+size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N) {
+    if (M <= 16 || M > kGemmWsMaxM || K <= 0 || N <= 0 || K % kGroup != 0 || N % kWsTileCols != 0 || g_gemv_ws_tune.splitk == 2) return 0;
+    const int G = K / kGroup, tiles = N / kWsTileCols, rows = M < 64 ? M : 64, sets = (tiles + 15) / 16;
+    if (g_gemv_ws_tune.splitk == 0 && (G < 32 || rows * G < 1536 || (tiles % 4 == 0 && tiles / 4 >= 200))) return 0;
+    const int want = std::min((256 + sets - 1) / sets, 16), groups = std::max(((G + want - 1) / want + 3) & ~3, 4), slices = (G + groups - 1) / groups;
+    return slices > 1 ? (size_t)slices * rows * N * sizeof(float) : 0;
+}
+
+constexpr size_t kGemmScratchMost = (size_t)256 << 20;
+
+size_t w4a16_gemm_stream_best_scratch_bytes(int M, int K, int N) {
+    const size_t least = w4a16_gemm_stream_scratch_bytes(M, K, N);
+    if (!gemm_wsm_supported(M, K, N)) return least;
+    const WsmPlan p = gemm_stream_plan(M, K, N, false, false, kGemmScratchMost);
+    return p.us >= 0 ? std::max(gemm_wsm_scratch_bytes(p, M, N), least) : least;
+}
+
+static int gemm_stream_call(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group, void *scratch, size_t scratch_bytes,
+                            bool insist, void *stream) {
     if (M == 1) return gemv_stream_call(x, wstream, nullptr, y, K, N, group, stream, GemvWsExtras());
     if (!x || !wstream || !y) return W4A16_ERR_NULL;
     if (group != kGroup) return W4A16_ERR_GROUP;
     if (M <= 0 || K <= 0 || N <= 0 || K % kGroup != 0 || N % kWsTileCols != 0) return W4A16_ERR_SHAPE;
     if (misaligned(x) || misaligned(wstream) || misaligned(y)) return W4A16_ERR_ALIGN;
-    // up to here the weights are streamed once per 64 rows (exact weights); from here on the tiled kernel that
-    // multiplies bf16-rounded weights.  The tiled kernel takes the same time for any M <= 256 (K = 4096, N = 14336:
-    // 51 us; N = 4096: 49 us; K = 2048, N = 8192: 27 us), two launches of 64 rows 46, 38 and 24 us, three 67, 56 and 36 us.
-    const int prefill_min_m = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : kGemmWsMaxM + 1;
-    hipError_t e = M >= prefill_min_m && gemm_prefill_ws_supported(M, K, N)
-                       ? launch_gemm_prefill_ws(x, wstream, y, M, K, N, static_cast<hipStream_t>(stream))
-                       : launch_gemm_ws(x, wstream, y, nullptr, M, K, N, static_cast<hipStream_t>(stream));
-    return e == hipSuccess ? W4A16_OK : hip_fail(e);
+    const size_t need = insist && !gemm_stream_rounded(M, K, N, false, false) ? w4a16_gemm_stream_scratch_bytes(M, K, N) : 0;
+    if (need && misaligned(scratch)) return W4A16_ERR_ALIGN;
+    if (need && (!scratch || scratch_bytes < need)) return W4A16_ERR_WORKSPACE;
+    if (misaligned(scratch)) scratch = nullptr;
+    return gemm_stream_run(x, wstream, nullptr, y, M, K, N, false, scratch, scratch_bytes, stream);
 }
 
-size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N) {
-    if (M <= 16 || M > kGemmWsMaxM || K <= 0 || N <= 0 || K % kGroup != 0 || N % kWsTileCols != 0) return 0;
-    return gemm_wsk_pays(M, K, N) ? gemm_wsk_scratch_bytes(M, K, N) : 0;
+int w4a16_gemm_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group, void *stream) {
+    return gemm_stream_call(x, wstream, y, M, K, N, group, nullptr, 0, false, stream);
 }
 
 int w4a16_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group, void *scratch,
                                    size_t scratch_bytes, void *stream) {
-    // 17 .. 128 rows of a shape where the split along K is the faster one: the split-K kernel; everything else is
-    // w4a16_gemm_stream_bf16
-    const int prefill_min_m = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : kGemmWsMaxM + 1;
-    const bool shape_ok = K > 0 && N > 0 && K % kGroup == 0 && N % kWsTileCols == 0;
-    if (M <= 16 || M >= prefill_min_m || !shape_ok || !gemm_wsk_pays(M, K, N))
-        return w4a16_gemm_stream_bf16(x, wstream, y, M, K, N, group, stream);
-    if (!x || !wstream || !y) return W4A16_ERR_NULL;
-    if (group != kGroup) return W4A16_ERR_GROUP;
-    if (misaligned(x) || misaligned(wstream) || misaligned(y) || misaligned(scratch)) return W4A16_ERR_ALIGN;
-    const size_t need = gemm_wsk_scratch_bytes(M, K, N);
-    if (need && (!scratch || scratch_bytes < need)) return W4A16_ERR_WORKSPACE;
-    hipError_t e = launch_gemm_wsk(x, wstream, y, nullptr, static_cast<float *>(scratch), M, K, N, static_cast<hipStream_t>(stream));
-    return e == hipSuccess ? W4A16_OK : hip_fail(e);
+    return gemm_stream_call(x, wstream, y, M, K, N, group, scratch, scratch_bytes, true, stream);
 }
 
 int w4a16_gemv_add_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int K, int N,
@@ -968,18 +1004,21 @@ int w4a16_q4nx_gemv_stream_bf16(const uint16_t *x, const void *wstream, const ui
 
 int w4a16_q4nx_gemm_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,
                                 void *stream) {
+    return w4a16_q4nx_gemm_stream_scratch_bf16(x, wstream, residual, y, M, K, N, nullptr, 0, stream);
+}
+
+size_t w4a16_q4nx_gemm_stream_best_scratch_bytes(int M, int K, int N, int has_residual) {
+    const WsmPlan p = gemm_stream_plan(M, K, N, true, has_residual != 0, kGemmScratchMost);
+    return p.us >= 0 ? gemm_wsm_scratch_bytes(p, M, N) : 0;
+}
+
+int w4a16_q4nx_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,
+                                        void *scratch, size_t scratch_bytes, void *stream) {
     if (M == 1) return w4a16_q4nx_gemv_stream_bf16(x, wstream, residual, y, K, N, stream);
     if (!x || !wstream || !y) return W4A16_ERR_NULL;
     if (M <= 0 || K <= 0 || N <= 0 || K % kGroup != 0 || N % kWsTileCols != 0) return W4A16_ERR_SHAPE;
-    if (misaligned(x) || misaligned(wstream) || misaligned(y) || (residual && misaligned(residual))) return W4A16_ERR_ALIGN;
-    // launches of 16 rows take 13 us each at K = 4096, N = 14336, the tiled kernel ~55 us for up to 256 rows: from 65 rows on
-    // the tiled kernel (bf16-rounded weights, as the dense dequant gives them); a residual stays with the launches of 16
-    // rows, which add it in fp32 before the one rounding
-    const int tiled_min_m = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : 65;
-    hipError_t e = M >= tiled_min_m && !residual && gemm_prefill_ws_supported(M, K, N)
-                       ? launch_gemm_prefill_ws(x, wstream, y, M, K, N, static_cast<hipStream_t>(stream), kEpiNone, nullptr, nullptr, true)
-                       : launch_gemm_ws(x, wstream, y, residual, M, K, N, static_cast<hipStream_t>(stream), true);
-    return e == hipSuccess ? W4A16_OK : hip_fail(e);
+    if (misaligned(x) || misaligned(wstream) || misaligned(y) || (residual && misaligned(residual)) || misaligned(scratch)) return W4A16_ERR_ALIGN;
+    return gemm_stream_run(x, wstream, residual, y, M, K, N, true, scratch, scratch_bytes, stream);
 }
 
 int w4a16_q4nx_rms_gemv_stream_bf16(const uint16_t *x, const float *x_sumsq, int n_pieces, const uint16_t *norm_weight, float eps,

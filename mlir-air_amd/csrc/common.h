@@ -117,4 +117,16 @@ __device__ __forceinline__ float load_agent(const float *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A wave-uniform pointer pinned to scalar registers: loads and copies through it take the form "scalar base + 32-bit lane offset", and
+// the per-lane part stays one VGPR (left alone the compiler folds the lane offset into a 64-bit VGPR base per stream and spends two
+// VGPRs and a 64-bit add on every request).  The offset's zero extension has to be in the same basic block as its request to fold
+// into the instruction: a loop makes its offsets opaque once per turn.
+typedef const __attribute__((address_space(1))) char *gptr;
+__device__ __forceinline__ gptr scalar_ptr(const void *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return reinterpret_cast<gptr>(((uint64_t)hi << 32) | lo);
+}
+
 }  // namespace w4a16

@@ -248,15 +248,6 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
     const int stride = products / items;
     return n % stride == stride - 1 && n / stride < items ? n / stride : -1;
 }
-// A wave-uniform pointer that stays in scalar registers: a copy's address is then this plus a 32-bit offset per lane.
-typedef const __attribute__((address_space(1))) char *gptr;
-__device__ __forceinline__ gptr scalar_ptr(const void *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    asm volatile("" : "+s"(lo), "+s"(hi));
-    return reinterpret_cast<gptr>(((uint64_t)hi << 32) | lo);
-}
-
 // A wave's NT x 8 tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding

@@ -56,6 +56,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "wsdequant.h"
 #include "wstream.h"
 
 namespace w4a16 {
@@ -66,21 +67,6 @@ constexpr int kPfThreads = 256;
 constexpr int kPfRowTiles = 16;              // row tiles of 16 per wave
 constexpr int kPfRows = 16 * kPfRowTiles;    // rows per workgroup tile
 constexpr double kPfSlowdown128 = 1.4, kPfSlowdown64 = 2.0;   // time per column of 128- and 64-column tiles against 256
-
-// eight weights of one dword (rows 8 lg .. 8 lg + 7 of the lane's column) as the four registers of a B operand
-__device__ __forceinline__ bf16x8 dequant_operand(uint32_t w, float sf, float c0) {
-    uint32_t e = w & 0x0F0F0F0Fu;          // nibbles 0, 2, 4, 6 -> rows 0, 4, 1, 5
-    uint32_t o = (w >> 4) & 0x0F0F0F0Fu;   // nibbles 1, 3, 5, 7 -> rows 2, 6, 3, 7
-    // kept opaque: the compiler would otherwise fold the masks into one v_bfe_u32 per nibble in front of every
-    // convert (two instructions per weight) instead of the byte-select converts v_cvt_f32_ubyte0..3 (one)
-    asm volatile("" : "+v"(e), "+v"(o));
-    const float k0 = fmaf(static_cast<float>(e & 0xFFu), sf, c0), k4 = fmaf(static_cast<float>((e >> 8) & 0xFFu), sf, c0);
-    const float k1 = fmaf(static_cast<float>((e >> 16) & 0xFFu), sf, c0), k5 = fmaf(static_cast<float>(e >> 24), sf, c0);
-    const float k2 = fmaf(static_cast<float>(o & 0xFFu), sf, c0), k6 = fmaf(static_cast<float>((o >> 8) & 0xFFu), sf, c0);
-    const float k3 = fmaf(static_cast<float>((o >> 16) & 0xFFu), sf, c0), k7 = fmaf(static_cast<float>(o >> 24), sf, c0);
-    const u32x4 b = {pack_bf16x2(k0, k1), pack_bf16x2(k2, k3), pack_bf16x2(k4, k5), pack_bf16x2(k6, k7)};
-    return __builtin_bit_cast(bf16x8, b);
-}
 
 // Four MFMAs of one B operand (row tiles 4 Q .. 4 Q + 3) with, behind each of them, one slot of the NEXT operand's
 // dequant: dequant_operand cut into 12 slots of two instructions that do not depend on each other (quarters 0..2;
@@ -137,36 +123,12 @@ __device__ __forceinline__ void mfma_one(floatx4 &acc, const bf16x8 &a, const bf
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
-// Q4NX order: scale word -> scale s and min' (two bf16 halves)
-__device__ __forceinline__ void decode_md_q4(uint32_t md, float &sf, float &c0) {
-    sf = __builtin_bit_cast(float, md << 16);
-    c0 = __builtin_bit_cast(float, md & 0xFFFF0000u);
-}
-
-// A wave-uniform pointer pinned to scalar registers: the loads below then take the form "scalar base + 32-bit lane
-// offset" and the per-lane part stays one loop-invariant VGPR (left alone the compiler folds the lane offset into
-// a 64-bit VGPR base per stream and spends two VGPRs and a 64-bit add on every request).
-using gptr = const __attribute__((address_space(1))) char *;
-__device__ __forceinline__ gptr scalar_ptr(const char *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    asm volatile("" : "+s"(lo), "+s"(hi));
-    return reinterpret_cast<gptr>(((uint64_t)hi << 32) | lo);
-}
-
 // p - bytes, kept in scalar registers (and not re-associated into the lane offsets)
 __device__ __forceinline__ gptr scalar_sub(gptr p, uint32_t bytes) {
     const uint64_t v = reinterpret_cast<uint64_t>(p) - bytes;
     uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
     asm volatile("" : "+s"(lo), "+s"(hi));
     return reinterpret_cast<gptr>(((uint64_t)hi << 32) | lo);
-}
-
-// scale word -> scale s and -z * s (exact: (128 + z) - 128 and an 8 x 8 bit product)
-__device__ __forceinline__ void decode_md(uint32_t md, float &sf, float &c0) {
-    sf = __builtin_bit_cast(float, md << 16);
-    const float nz = __builtin_bit_cast(float, md & 0xFFFF0000u);   // -(128 + z)
-    c0 = (nz + 128.0f) * sf;
 }
 
 // Gate and up projection in one tile (launch_gemm_prefill_ws_swiglu): a tile of 64 NCB columns holds 32 NCB columns of
@@ -676,6 +638,15 @@ hipError_t launch_wsp(const PfArgs &p, hipStream_t stream) {
 }  // namespace
 
 bool gemm_prefill_ws_supported(int M, int K, int N) { return M > 0 && K > 0 && K % (2 * kGroup) == 0 && N > 0 && N % 64 == 0; }
+
+// Rounds of tiles over the chip, each K steps of a cost linear in the tile's width (fitted to 300 .. 2048 rows of twelve matrices,
+// within 20 %: K = 4096, N = 4096, 300 rows 45 estimated / 43 measured; N = 14336, 700 rows 83 / 79; K = 14336, N = 4096, 2048 rows 186 / 214 us)
+double gemm_prefill_ws_us(int M, int K, int N, bool q4) {
+    const int tiles_m = (M + kPfRows - 1) / kPfRows;
+    const Widths wd = pick_widths(tiles_m, N / 64, 256, false);
+    const long rounds = ((long)tiles_m * (wd.wide + wd.narrow) + 255) / 256;
+    return 2.5 + 1e-3 * K * rounds * (q4 ? 8.0 + 3.5 * wd.ncb : 6.8 + 3.0 * wd.ncb);
+}
 
 hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, hipStream_t stream, int epi,
                                   const uint16_t *aux, const GemmRope *rope, bool q4) {

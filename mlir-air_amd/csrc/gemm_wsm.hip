@@ -1,0 +1,471 @@
+// Products of 17 rows and more on stream-order weights (wstream.h), both codecs, any K % 128 == 0 and N % 16 == 0:
+// y[M, N] = bf16(x[M, K] . W (+ residual)) with the exact weights, fp32 accumulation.
+//
+// A wave goes through a group of 128 k in about 1900 cycles, of which the matrix pipe works a third: LDS reads, 145 vector and 60
+// scalar instructions and the barrier are a chain.  So a workgroup puts KW waves on every SIMD, each set of four on a group of its own
+// (their sums meet in LDS at the end), and K is cut into slices besides where there are few columns.  64 rows, K = 14336, N = 4096: one
+// wave per SIMD 22.9 us, two 18.2 us, the launches of 64 whole-K rows that ran before 27.3 us (split along K) and 54.9 us; 300 rows of
+// K = 4096, N = 11008 43 us (tiled kernel: 54 us); Q4NX, 2048 rows of the ragged K = 2176, N = 5744 101 us (16 rows a launch: 972 us).
+//
+//   workgroup  = 16 RT rows x 64 NT columns; wave (part kq < KW of K, wq < 4): row tiles all, stream tiles NT wq .. of the column set
+//   step       = KW groups; x goes global -> LDS once per workgroup (global_load_lds_dwordx4) and so do a wave's cells and scale words
+//                (a cell is the B operand of four K-steps), R - 1 steps ahead, in a ring of R.  (Cells in registers instead: the
+//                compiler waits for every request in flight once per turn of a loop that carries loads from one turn to the next.)
+//   AWQ        : operands are (128 + q) exactly, flushed per group: y += s (sum (128 + q) x - (128 + z) sum x); the sums of x of the
+//                next step are taken by one wave per row tile with an MFMA against ones and handed round through LDS, with R = 2 by
+//                every wave for itself
+//   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: w = s q + min in fp32, cut into two bf16
+//                (16 significant bits, the product of each with x is exact), two MFMAs per K-step
+//   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits
+//   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
+#include <algorithm>
+
+#include "common.h"
+#include "kernels.h"
+#include "wsdequant.h"
+#include "wstream.h"
+
+namespace w4a16 {
+
+namespace {
+
+constexpr int kSmLds = 160 * 1024;
+enum : int { kSmAwq, kSmQ4, kSmAwqRounded, kSmQ4Rounded };
+
+struct SmArgs {
+    const uint16_t *x;
+    const char *w;
+    float *partial;
+    uint16_t *y;
+    const uint16_t *residual;
+    int M, K, N, G, NB;
+    int sets, slices, blocks;      // column sets, slices of K, blocks of rows
+};
+
+// A step in LDS: the x tiles of its groups, then per wave its cells and its scale words ([64]: tile lane / 16, column lane % 16; Q4NX:
+// [NT][64], K-step lane / 16)
+constexpr int sm_wave_bytes(int nt, bool q4) { return nt * (int)kWsCellBytes + (q4 ? nt : 1) * 256; }
+constexpr int sm_stage(int rt, int nt, int kw, bool q4) { return kw * (16 * rt * 256 + 4 * sm_wave_bytes(nt, q4)); }
+constexpr int sm_ring(int rt, int nt, int kw, bool q4) {
+    const int n = ((kw == 1 ? kSmLds / 2 : kSmLds) - (q4 || rt > 4 ? 0 : 2 * kw * 16 * rt * 4)) / sm_stage(rt, nt, kw, q4);
+    return n < 4 ? n : 4;
+}
+
+template <int RT, int NT, int KW, int MODE>
+__global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(const SmArgs p) {
+    constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded, kExact = MODE == kSmAwq;
+    constexpr int ROWS = 16 * RT, XT = ROWS * 256;                     // rows and bytes of an x tile (a group: 128 bf16 a row)
+    constexpr int MC = Q4 ? NT : 1;                                    // copies (256 bytes) of a wave's scale words
+    constexpr int V = RT + NT + MC;                                    // requests of a wave and step: x, cells, scale words
+    constexpr int kWave = sm_wave_bytes(NT, Q4), kStage = sm_stage(RT, NT, KW, Q4), R = sm_ring(RT, NT, KW, Q4);
+    constexpr bool kSums = kExact && R > 2 && RT <= 4;                 // sums of x handed round; else a wave takes its own
+    constexpr int CW = 64 * NT, kThreads = 256 * KW;
+    static_assert(R >= 2, "two steps fit LDS");
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    float *xs_lds = reinterpret_cast<float *>(lds + R * kStage);       // [2][KW][ROWS]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kq = wave >> 2, wq = wave & 3;
+    const int lg = lane >> 4, ln = lane & 15;
+
+    // An XCD takes a contiguous range of (slice, column set, row block), row blocks first: those that run together on it share the
+    // weights of a set and the x of a slice in its L2.
+    const int total = p.sets * p.slices * p.blocks, per_xcd = (total + 7) / 8;
+    const int id = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || id >= total) return;
+    const int block = id % p.blocks, set = id / p.blocks % p.sets, slice = id / (p.blocks * p.sets);
+    const int g_lo = (int)((long)p.G * slice / p.slices), g_hi = (int)((long)p.G * (slice + 1) / p.slices);
+    const int m0 = block * ROWS, rows = min(ROWS, p.M - m0);
+
+    // tiles past the matrix (ragged last set) read the last tile and are not stored
+    const int ntiles = p.N / kWsTileCols;
+    constexpr int kMd = Q4 ? kWsQ4MdKiB : 1;   // KiB of scale words in front of a block's cells
+    const size_t tile_bytes = (size_t)(kMd * p.NB + p.G) * kWsCellBytes;
+    const int first = min((set * 4 + wq) * NT, ntiles - 1);
+    gptr tb[NT];
+#pragma unroll
+    for (int c = 0; c < NT; ++c) tb[c] = scalar_ptr(p.w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
+    // this lane's cell and scale words: 32-bit offsets from a tile's start (from the first tile's for the AWQ words, one copy of which
+    // serves all the wave's tiles)
+    const uint32_t lane16 = 16 * lane;
+    const uint32_t word_off = 16 * ln + (Q4 ? lg * (uint32_t)kWsCellBytes : (uint32_t)(min(first + lg % NT, ntiles - 1) - first) * (uint32_t)tile_bytes);
+
+    // copy j of the wave: rows 4 q .. + 3 of its group's x, q = 4 j + wq; lane l fetches chunk (l % 16) ^ row % 16 of row l / 16
+    const gptr xbase = scalar_ptr(p.x + (size_t)m0 * p.K);
+    uint32_t xoff[RT];   // (at most 111 rows: the host keeps K below 2^24)
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+        const int row = 4 * (4 * j + wq) + lg;
+        xoff[j] = (uint32_t)min(row, rows - 1) * (uint32_t)(p.K * 2) + 16 * (ln ^ (row & 15));
+    }
+    const int x_lds = kq * XT, wave_lds = KW * XT + wave * kWave;
+    auto copy16 = [&](gptr src, int dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)(lds + dst), 16, 0, 0);
+    };
+    auto copy4 = [&](gptr src, int dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)(lds + dst), 4, 0, 0);
+    };
+    auto request = [&](int g, int stage) {
+        const gptr xs = xbase + (size_t)g * 256;
+#pragma unroll
+        for (int j = 0; j < RT; ++j) copy16(xs + xoff[j], stage + x_lds + 1024 * (4 * j + wq));
+        const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
+        uint32_t cell = lane16 + (blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes), word = word_off + (blk + 64 * (g & 12) + 4 * (g & 3));
+        asm volatile("" : "+v"(cell), "+v"(word));   // (a 32-bit sum: folds into the copies as their offset)
+#pragma unroll
+        for (int c = 0; c < NT; ++c) copy16(tb[c] + cell, stage + wave_lds + c * (int)kWsCellBytes);
+#pragma unroll
+        for (int c = 0; c < MC; ++c) copy4(tb[c] + word, stage + wave_lds + NT * (int)kWsCellBytes + 256 * c);
+    };
+    auto cell_at = [&](int stage, int c) { return *reinterpret_cast<const u32x4 *>(lds + stage + wave_lds + c * (int)kWsCellBytes + 16 * lane); };
+    auto word_at = [&](int stage, int c, int t) {   // (AWQ: t = 0)
+        return *reinterpret_cast<const uint32_t *>(lds + stage + wave_lds + NT * (int)kWsCellBytes + (Q4 ? 256 * c + 64 * t : 64 * c) + 4 * ln);
+    };
+
+    uint32_t nib_mask = 0x000F000Fu, magic = 0x43004300u;
+    asm volatile("" : "+s"(nib_mask));
+    asm volatile("" : "+v"(magic));
+    auto exact_operand = [&](uint32_t w) {   // rows (2 v, 2 v + 1) as bf16 (128 + q)
+        u32x4 b;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b[v] = ((w >> (4 * v)) & nib_mask) | magic;
+        return __builtin_bit_cast(bf16x8, b);
+    };
+    // eight weights s q + low as the sum of two bf16
+    auto two_operands = [&](uint32_t w, uint32_t md, bf16x8 &high, bf16x8 &rest) {
+        const float s = __builtin_bit_cast(float, md << 16), low = __builtin_bit_cast(float, md & 0xFFFF0000u);
+        uint32_t e = w & 0x0F0F0F0Fu, o = (w >> 4) & 0x0F0F0F0Fu;   // rows 0, 4, 1, 5 and 2, 6, 3, 7
+        asm volatile("" : "+v"(e), "+v"(o));
+        const uint32_t src[4] = {e, o, e, o};
+        u32x4 h, l;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const uint32_t n = src[v] >> (v < 2 ? 0 : 8);
+            const float w0 = fmaf(static_cast<float>(n & 0xFFu), s, low), w1 = fmaf(static_cast<float>((n >> 16) & 0xFFu), s, low);
+            const uint32_t p2 = pack_bf16x2(w0, w1);
+            h[v] = p2;
+            l[v] = pack_bf16x2(w0 - __builtin_bit_cast(float, p2 << 16), w1 - __builtin_bit_cast(float, p2 & 0xFFFF0000u));
+        }
+        high = __builtin_bit_cast(bf16x8, h);
+        rest = __builtin_bit_cast(bf16x8, l);
+    };
+    auto operand_a = [&](int stage, int t, int rt) {
+        return *reinterpret_cast<const bf16x8 *>(lds + stage + x_lds + (16 * rt + ln) * 256 + (((4 * t + lg) ^ ln) << 4));
+    };
+    // the sums of x of row tile `wave` of a stage, left for its flush
+    auto sum_rows = [&](const bf16x8 (&a)[4], int half) {
+        const uint32_t one = 0x3F803F80u;
+        const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
+        floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], ones, s, 0, 0, 0);
+        if (ln == 0) *reinterpret_cast<floatx4 *>(xs_lds + (half * KW + kq) * ROWS + 16 * wq + 4 * lg) = s;
+    };
+    auto read_sum_operands = [&](int stage, bf16x8 (&a)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) a[t] = operand_a(stage, t, wq);
+    };
+    const bool sums = kSums && wq < RT;
+
+    floatx4 Y[RT][NT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int c = 0; c < NT; ++c) Y[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    // One group.  A wave's LDS reads are in flight long before their products: everything at the head of the group where there are
+    // registers for it (four row tiles or less), else the operands of a K-step while the one before it multiplies.
+    constexpr int AHEAD = RT <= 4 ? 4 : 2;
+    auto multiply = [&](int half, int stage, int next) {
+        u32x4 cell[NT];
+        uint32_t word[NT][Q4 ? 4 : 1];
+        bf16x8 a[AHEAD][RT], as[4];
+#pragma unroll
+        for (int c = 0; c < NT; ++c) cell[c] = cell_at(stage, c);
+#pragma unroll
+        for (int t = 0; t < (AHEAD == 4 ? 4 : 1); ++t)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) a[t][rt] = operand_a(stage, t, rt);
+#pragma unroll
+        for (int c = 0; c < NT; ++c)
+#pragma unroll
+            for (int t = 0; t < (Q4 ? 4 : 1); ++t) word[c][t] = word_at(stage, c, t);
+        __builtin_amdgcn_sched_barrier(0);
+        floatx4 acc[RT][NT], own[RT];
+        if constexpr (kExact && !kSums) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) own[rt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        if constexpr (MODE == kSmAwq) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int c = 0; c < NT; ++c) acc[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        float s[NT], low[NT];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if constexpr (AHEAD == 2) {
+                if (t < 3) {
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) a[(t + 1) & 1][rt] = operand_a(stage, t + 1, rt);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (t == 2 && sums) read_sum_operands(next, as);
+            if constexpr (kExact && !kSums) {
+                const uint32_t one = 0x3F803F80u;
+                const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) own[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t % AHEAD][rt], ones, own[rt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < NT; ++c) {
+                const bf16x8(&at)[RT] = a[t % AHEAD];
+                if constexpr (MODE == kSmAwq) {
+                    const bf16x8 b = exact_operand(cell[c][t]);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, acc[rt][c], 0, 0, 0);
+                } else if constexpr (MODE == kSmQ4) {
+                    bf16x8 high, rest;
+                    two_operands(cell[c][t], word[c][t], high, rest);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], high, Y[rt][c], 0, 0, 0);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], rest, Y[rt][c], 0, 0, 0);
+                } else {
+                    if (Q4) decode_md_q4(word[c][Q4 ? t : 0], s[c], low[c]);
+                    else if (t == 0) decode_md(word[c][0], s[c], low[c]);
+                    const bf16x8 b = dequant_operand(cell[c][t], s[c], low[c]);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, Y[rt][c], 0, 0, 0);
+                }
+            }
+            if (AHEAD == 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (sums) sum_rows(as, half ^ 1);
+        if constexpr (MODE == kSmAwq) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {   // register i of lane group lg is row 16 rt + 4 lg + i
+                const floatx4 xs = kSums ? *reinterpret_cast<const floatx4 *>(xs_lds + (half * KW + kq) * ROWS + 16 * rt + 4 * lg) : own[rt];
+#pragma unroll
+                for (int c = 0; c < NT; ++c) {
+                    const float sc = __builtin_bit_cast(float, word[c][0] << 16), nz = __builtin_bit_cast(float, word[c][0] & 0xFFFF0000u);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) Y[rt][c][i] = fmaf(sc, fmaf(nz, xs[i], acc[rt][c][i]), Y[rt][c][i]);
+                }
+            }
+        }
+    };
+
+    // The first R - 1 steps are requested; past the slice's end its last group once more (into a stage that nobody reads again).
+    const int g_wave = g_lo + kq, g_last = g_hi - 1;
+#pragma unroll
+    for (int i = 0; i < R - 1; ++i) request(min(g_wave + i * KW, g_last), i * kStage);
+    if (kSums) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * V - RT) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        bf16x8 as[4];
+        if (sums) {
+            read_sum_operands(0, as);
+            sum_rows(as, 0);
+        }
+    }
+
+    int stage = 0, half = 0;
+    for (int g0 = g_lo; g0 < g_hi; g0 += KW) {
+        // This step's requests and, for the sums, the next step's x have landed (younger ones: R - 2 steps, less that x); this wave is done
+        // with the step before, and behind the barrier so is everybody.
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kSums ? (R - 2) * V - RT : (R - 2) * V) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
+        const int fill = stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
+        request(min(g0 + kq + (R - 1) * KW, g_last), fill);
+        __builtin_amdgcn_sched_barrier(0);
+        if (KW == 1 || g0 + kq < g_hi) multiply(half, stage, next);
+        stage = next;
+        half ^= 1;
+    }
+
+    // The parts of K meet, then the sums leave through LDS, so that a store is whole rows of the workgroup's columns.  (No copy of
+    // any wave may still be on its way into it.)
+    constexpr int LDP = CW + 4;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if constexpr (KW > 1) {
+        floatx4 *parts = reinterpret_cast<floatx4 *>(lds);
+        if (kq > 0) {
+#pragma unroll
+            for (int i = 0; i < RT * NT; ++i) parts[((wave - 4) * RT * NT + i) * 64 + lane] = Y[i / NT][i % NT];
+        }
+        __syncthreads();
+        if (kq == 0) {
+#pragma unroll
+            for (int k = 1; k < KW; ++k)
+#pragma unroll
+                for (int i = 0; i < RT * NT; ++i) Y[i / NT][i % NT] += parts[((4 * (k - 1) + wq) * RT * NT + i) * 64 + lane];
+        }
+        __syncthreads();
+    }
+    float *yt = reinterpret_cast<float *>(lds);
+    if (kq == 0) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) yt[(16 * rt + 4 * lg + i) * LDP + (NT * wq + c) * kWsTileCols + ln] = Y[rt][c][i];
+    }
+    __syncthreads();
+    const int col0 = set * CW, ncols = min(CW, p.N - col0);   // a multiple of 16
+    for (int i = tid; i < rows * (CW / 4); i += kThreads) {
+        const int row = i / (CW / 4), col = i % (CW / 4) * 4;
+        if (col >= ncols) continue;
+        floatx4 v = *reinterpret_cast<const floatx4 *>(yt + row * LDP + col);
+        const size_t at = (size_t)(m0 + row) * p.N + col0 + col;
+        if (p.slices > 1) {
+            *reinterpret_cast<floatx4 *>(p.partial + (size_t)slice * p.M * p.N + at) = v;
+            continue;
+        }
+        if (p.residual) {
+            const uint2 q = *reinterpret_cast<const uint2 *>(p.residual + at);
+            v[0] += bf16_bits_to_float(q.x & 0xFFFFu), v[1] += bf16_bits_to_float(q.x >> 16);
+            v[2] += bf16_bits_to_float(q.y & 0xFFFFu), v[3] += bf16_bits_to_float(q.y >> 16);
+        }
+        *reinterpret_cast<uint2 *>(p.y + at) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+}
+
+// y = bf16(sum over the slices, in slice order (+ residual)); four columns per thread
+__global__ void __launch_bounds__(256) gemm_wsm_sum_kernel(const float *__restrict__ partial, const uint16_t *__restrict__ residual,
+                                                           uint16_t *__restrict__ y, size_t mn, int slices) {
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (at >= mn) return;
+    floatx4 s = *reinterpret_cast<const floatx4 *>(partial + at);
+    for (int k = 1; k < slices; ++k) s += *reinterpret_cast<const floatx4 *>(partial + (size_t)k * mn + at);
+    if (residual) {
+        const uint2 r = *reinterpret_cast<const uint2 *>(residual + at);
+        s[0] += bf16_bits_to_float(r.x & 0xFFFFu), s[1] += bf16_bits_to_float(r.x >> 16);
+        s[2] += bf16_bits_to_float(r.y & 0xFFFFu), s[3] += bf16_bits_to_float(r.y >> 16);
+    }
+    *reinterpret_cast<uint2 *>(y + at) = uint2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+}
+
+template <int RT, int NT, int KW, int MODE>
+hipError_t launch_wsm(const SmArgs &p, hipStream_t stream) {
+    constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded;
+    constexpr size_t ring = (size_t)sm_ring(RT, NT, KW, Q4) * sm_stage(RT, NT, KW, Q4) + (Q4 || RT > 4 ? 0 : 2 * KW * 16 * RT * sizeof(float));
+    constexpr size_t out = (size_t)16 * RT * (64 * NT + 4) * sizeof(float), parts = (size_t)(KW - 1) * 4 * RT * NT * 1024;
+    constexpr size_t lds = ring > out ? (ring > parts ? ring : parts) : out > parts ? out : parts;
+    static_assert(lds <= kSmLds, "fits LDS");
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wsm_kernel<RT, NT, KW, MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    if ((p.blocks - 1) * 16 * RT >= p.M || p.blocks * 16 * RT < p.M) return hipErrorInvalidValue;   // every block has rows, every row a block
+    const int total = p.sets * p.slices * p.blocks;
+    hipLaunchKernelGGL((gemm_wsm_kernel<RT, NT, KW, MODE>), dim3((total + 7) / 8 * 8), dim3(256 * KW), lds, stream, p);
+    return hipGetLastError();
+}
+
+// Four groups to a step for the smallest row tiles, whose waves have least to do in one.
+template <int NT, int MODE>
+hipError_t launch_wsm_rt(int rt, const SmArgs &p, hipStream_t stream) {
+    constexpr int KW = MODE >= kSmAwqRounded ? 1 : 2;   // (rounded: the sums in one order)
+    switch (rt) {
+        case 1:
+        case 2: return launch_wsm<2, NT, KW == 1 ? 1 : 4, MODE>(p, stream);
+        case 3: return launch_wsm<3, NT, KW, MODE>(p, stream);
+        case 4: return launch_wsm<4, NT, KW, MODE>(p, stream);
+        case 5: return launch_wsm<5, NT, KW, MODE>(p, stream);
+        case 6: return launch_wsm<6, NT, KW, MODE>(p, stream);
+        default: return launch_wsm<7, NT, KW, MODE>(p, stream);
+    }
+}
+
+template <int MODE>
+hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t stream) {
+    if constexpr (MODE >= kSmAwqRounded)
+        if (plan.nt == 3) return plan.rt == 3 ? launch_wsm<3, 3, 1, MODE>(p, stream) : plan.rt == 4 ? launch_wsm<4, 3, 1, MODE>(p, stream) : launch_wsm<5, 3, 1, MODE>(p, stream);
+    return plan.nt == 1 ? launch_wsm_rt<1, MODE>(plan.rt, p, stream) : launch_wsm_rt<2, MODE>(plan.rt, p, stream);
+}
+
+// The time of a launch, fitted to 10800 timings (13 matrices from 512 x 1024 to 13056 x 5744, 17 .. 3500 rows, every tile, 1 .. 16
+// slices; rms error 7 % exact, 10 % rounded; the plan it picks takes 1 % more than the best of them on average, 24 % at worst):
+// microseconds of start, of a workgroup, and of a step alone on the chip (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with
+// every CU busy; a step of four groups costs 1 + four of one of two.
+struct SmCost {
+    double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, tb_s;
+};
+constexpr SmCost kSmCost[3] = {{2.6, 2.1, 0.06, 0.084, 0.075, 0.076, 0.16, 0.017, 0, 0, 0.69, 2.0, 5.9},
+                               {3.0, 1.6, 0, 0.042, 0.535, 0.100, 0.11, 0.021, 0.028, 0, 0.88, 1.9, 5.2},
+                               {1.8, 2.5, 0, 0.030, 0.150, 0.035, 0.07, 0.018, 0.09, 0.03, 0, 0, 1}};
+
+double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
+    const SmCost &c = kSmCost[rounded ? 2 : q4];
+    const bool four = !rounded && p.rt <= 2;
+    const int kw = rounded ? 1 : four ? 4 : 2, chip = rounded ? 512 : 256;   // (two workgroups a CU where one has a wave per SIMD)
+    const int groups = (K / kGroup + p.slices - 1) / p.slices, steps = (groups + kw - 1) / kw;
+    const double alone = c.a0 + c.a1 * p.rt + c.a2 * p.nt + c.a3 * p.rt * p.nt, more = c.b0 + c.b1 * p.rt + c.b2 * p.nt + c.b3 * p.rt * p.nt;
+    const long wgs = (long)((N + 64 * p.nt - 1) / (64 * p.nt)) * p.blocks * p.slices, full = wgs / chip;
+    const double rest = (double)(wgs % chip) / chip, step = steps * (four ? 1 + c.four : 1.0);
+    double us = c.start + full * (c.group + step * (alone + more));
+    if (rest > 0) us += c.group + step * (alone + more * rest);
+    if (p.slices > 1) us += c.sum + p.slices * ((double)M * N * 8e-6 / c.tb_s);
+    return us;
+}
+
+}  // namespace
+
+WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch_bytes) {
+    const int tiles = (M + 15) / 16, G = K / kGroup;
+    WsmPlan best;
+    best.us = -1;
+    for (int nt = 1; nt <= (rounded ? 3 : 2); ++nt) {
+        const int most = nt == 3 ? 5 : 7, least = nt == 3 ? 3 : 2, few = (tiles + most - 1) / most;
+        const int options[3] = {few, few + 1, (tiles + 3) / 4};   // blocks of rows
+        for (int blocks : options) {
+            WsmPlan p;
+            p.nt = nt;
+            p.rt = std::max((tiles + blocks - 1) / blocks, least);
+            p.blocks = (tiles + p.rt - 1) / p.rt;
+            for (int slices : {1, 2, 3, 4, 6, 8, 12, 16}) {
+                p.slices = slices;
+                if (slices > 1 && (rounded || G / slices < 2 || gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes)) break;
+                p.us = wsm_us(p, M, K, N, q4, rounded);
+                if (best.us < 0 || p.us < best.us) best = p;
+            }
+        }
+    }
+    return best;
+}
+
+bool gemm_wsm_supported(int M, int K, int N) { return M > 16 && K > 0 && K % kGroup == 0 && K < 1 << 24 && N > 0 && N % kWsTileCols == 0; }
+
+size_t gemm_wsm_scratch_bytes(const WsmPlan &p, int M, int N) { return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0; }
+
+hipError_t launch_gemm_wsm(const WsmPlan &plan, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *residual, float *scratch, int M, int K, int N,
+                           bool q4, bool rounded, hipStream_t stream) {
+    SmArgs p;
+    p.x = x;
+    p.w = static_cast<const char *>(w);
+    p.partial = scratch;
+    p.y = y;
+    p.residual = residual;
+    p.M = M, p.K = K, p.N = N, p.G = K / kGroup, p.NB = ws_blocks(K);
+    if (!gemm_wsm_supported(M, K, N)) return hipErrorInvalidValue;
+    p.sets = (N + 64 * plan.nt - 1) / (64 * plan.nt);
+    p.slices = plan.slices, p.blocks = plan.blocks;
+    if (plan.slices > 1 && !scratch) return hipErrorInvalidValue;
+    const hipError_t e = q4 ? (rounded ? launch_wsm_mode<kSmQ4Rounded>(plan, p, stream) : launch_wsm_mode<kSmQ4>(plan, p, stream))
+                            : (rounded ? launch_wsm_mode<kSmAwqRounded>(plan, p, stream) : launch_wsm_mode<kSmAwq>(plan, p, stream));
+    if (e != hipSuccess || plan.slices == 1) return e;
+    const size_t mn = (size_t)M * N;   // N % 16 == 0: whole groups of four columns
+    hipLaunchKernelGGL(gemm_wsm_sum_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, residual, y, mn, plan.slices);
+    return hipGetLastError();
+}
+
+}  // namespace w4a16

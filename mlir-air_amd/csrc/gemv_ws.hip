@@ -490,7 +490,7 @@ hipError_t launch_repack_ws(const int32_t *qweight, const int32_t *qzeros, const
 
 }  // namespace w4a16
 
-// ---- batched decode, 2 <= M <= 16 (gemm_ws_kernel) and up to 64 rows (gemm_ws_rows_kernel), on the same layout ----
+// ---- batched decode, 2 <= M <= 16 (gemm_ws_kernel) and up to 64 rows (gemm_ws_rows_kernel, where gemm_wsm.hip is not the faster), on the same layout ----
 //
 // The 16 rows of the A operand are the rows of x (row m <-> lane ln = m), so a cell's product is the whole
 // [16 x 16] block of y for its 16 columns and the group flush applies to all four accumulator registers.  A workgroup
@@ -815,14 +815,28 @@ hipError_t launch_gemm_ws_cb(const uint16_t *x, const void *w, uint16_t *y, cons
 
 }  // namespace
 
+// Columns of tiles per workgroup of a batched launch
+static int gemm_ws_cb(int tiles) {
+    int cb = g_gemv_ws_tune.cb;
+    if (!cb) cb = tiles % 4 == 0 && tiles / 4 >= 200 ? 4 : (tiles % 2 == 0 && tiles / 2 >= 200 ? 2 : 1);
+    return tiles % cb ? 1 : cb;
+}
+
+// Each launch rounds of workgroups over the chip, a group of K a cost by rows and tile columns (fitted to 13 matrices at 8 .. 128 rows;
+// AWQ, 17 / 64 rows: K = 4096, N = 4096 7.3 estimated / 7.5 measured and 18.6 / 19.1 us, K = 14336, N = 4096 20.0 / 22.1 and 58.9 / 54.9;
+// Q4NX, 32 rows: K = 4096, N = 14336 26.1 / 24.1)
+double gemm_ws_us(int M, int K, int N, bool q4, bool residual) {
+    const int tiles = N / kWsTileCols, cb = gemm_ws_cb(tiles), most = q4 || residual ? 16 : 64, G = K / kGroup;
+    const double rounds = (tiles / cb + 255) / 256, wide = cb == 4 ? 0.14 : cb == 2 ? 0.06 : 0.03, step16 = cb == 4 ? 0.33 : cb == 2 ? 0.20 : 0.15;
+    auto launch = [&](int rows) { return 2.5 + G * rounds * (most == 16 ? step16 * (0.5 + rows / 32.0) : wide + 0.0074 * rows); };
+    return (M / most) * launch(most) + (M % most ? launch(M % most) : 0);
+}
+
 // y[M, N] = bf16(x[M, K] . W (+ residual)): up to 64 rows per launch (Q4NX order, or with a residual: 16), more rows as
 // further launches.
 hipError_t launch_gemm_ws(const uint16_t *x, const void *w, uint16_t *y, const uint16_t *residual, int M, int K, int N,
                           hipStream_t stream, bool q4) {
-    const int tiles = N / kWsTileCols;
-    int cb = g_gemv_ws_tune.cb;
-    if (!cb) cb = tiles % 4 == 0 && tiles / 4 >= 200 ? 4 : (tiles % 2 == 0 && tiles / 2 >= 200 ? 2 : 1);
-    if (tiles % cb) cb = 1;
+    const int cb = gemm_ws_cb(N / kWsTileCols);
     hipError_t e = hipSuccess;
     // (the launches of several row tiles take the AWQ order and no residual)
     const int max_rows = q4 || residual || g_gemv_ws_tune.gemm_rows == 16 ? 16 : (g_gemv_ws_tune.gemm_rows == 32 ? 32 : 64);

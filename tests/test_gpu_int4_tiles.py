@@ -1,0 +1,66 @@
+"""Int4 products of 17 rows and more at the edges of their row blocks, column sets, steps and slices, both codecs: exact weights against the
+float64 product (one bf16 rounding of an fp32 sum: 1 ulp and 2e-3, as for the other exact products), with no scratch and with scratch for
+any number of slices; rounded weights against the tiled kernel, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_bf16_close, dense_f64, make_awq, make_x
+from oracle import awq as oawq
+from oracle.bf16 import bf16_bits_to_f32
+from test_gpu_q4nx import make
+from test_gpu_stream_order import bits, dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 128, 16), (32, 384, 48), (33, 128 * 19, 272), (64, 4096, 64), (65, 1024, 528), (96, 512, 128), (112, 2176, 144),
+                                   (113, 512, 1040), (129, 640, 320), (129, 256, 64), (257, 1024, 192), (300, 2048, 1088)])
+@pytest.mark.parametrize("q4", [False, True])
+def test_int4_tiles(q4, M, K, N):
+    from air_hip import _lib, ops
+    print("int4 tiles", "q4nx" if q4 else "awq", M, K, N, flush=True)
+    lib, stream = _lib.load_library(), torch.cuda.current_stream().cuda_stream
+    x = make_x((M, K), seed=M + K)
+    res = make_x((M, N), seed=N) if q4 else None
+    if q4:
+        q, s, m = make(N, K, seed=M + N)   # [N, K] and [N, K / 32]
+        w = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+        dense = (q.astype(np.float64).reshape(N, K // 32, 32) * bf16_bits_to_f32(s).astype(np.float64)[:, :, None]
+                 + bf16_bits_to_f32(m).astype(np.float64)[:, :, None]).reshape(N, K).T
+    else:
+        tri = make_awq(K, N, seed=M + N)
+        w, dense = ops.repack_stream(*map(dev, tri)), dense_f64(*tri)
+    want = bf16_bits_to_f32(x).astype(np.float64) @ dense
+    xd, rd = dev(x), dev(res) if q4 else None
+    scratch = torch.full((1 << 26,), 0xFF, dtype=torch.uint8, device="cuda")
+
+    def call(nbytes, residual):
+        y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        at = scratch.data_ptr() if nbytes else None
+        if q4:
+            _lib.check(lib.w4a16_q4nx_gemm_stream_scratch_bf16(xd.data_ptr(), w.buf.data_ptr(), residual, y.data_ptr(), M, K, N, at, nbytes, stream))
+        elif nbytes:
+            _lib.check(lib.w4a16_gemm_stream_scratch_bf16(xd.data_ptr(), w.buf.data_ptr(), y.data_ptr(), M, K, N, 128, at, nbytes, stream))
+        else:
+            _lib.check(lib.w4a16_gemm_stream_bf16(xd.data_ptr(), w.buf.data_ptr(), y.data_ptr(), M, K, N, 128, stream))
+        return bits(y)
+
+    rounded = M >= (65 if q4 else 129) and K % 256 == 0 and N % 64 == 0
+    ops.tune("gemm_splitk", 1)
+    try:
+        for nbytes in (0, 1 << 26):
+            got = call(nbytes, None)
+            if rounded:
+                ops.tune("prefill_tile", 4)
+                assert np.array_equal(got, call(0, None))
+                ops.tune("prefill_tile", 0)
+            else:
+                assert_bf16_close(got, want, ulps=1.0, atol=2e-3, what=f"int4 tiles, {nbytes} bytes of scratch")
+            if q4:
+                assert_bf16_close(call(nbytes, rd.data_ptr()), want + bf16_bits_to_f32(res).astype(np.float64), ulps=1.0, atol=2e-3,
+                                  what=f"int4 tiles with a residual, {nbytes} bytes of scratch")
+    finally:
+        ops.tune("gemm_splitk", 0)
+        ops.tune("prefill_tile", 0)
+
