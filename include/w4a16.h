@@ -583,6 +583,29 @@ int w4a16_q4nx_o_gemv_ffn_stream_bf16(const uint16_t *attn_out, const uint16_t *
                                       int E, int H, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * Decode steps of a whole model on stream-order matrices, every launch of n_tokens tokens from one call: per layer the RMSNorm +
+ * Q|K|V GEMV, the attention and the O / FFN block of the entry points above (the same launches, the same bits), then the lm_head
+ * with its argmax, which also fetches the next token's embedding row (run_npu_decode_step and the greedy loop around it,
+ * programming_examples/llms/llama32_1b_int4/llama32_1b_int4_inference.py:429-560; nothing returns to the host in between).
+ * `first_x`: the embedding row of the token at start_pos; ids[i] receives the argmax of step i and logits [vocab] the last
+ * step's.  `workspace`: w4a16_decode_run_workspace_bytes bytes of plain scratch.  Everything is checked before the first launch.
+ */
+typedef struct {
+    const void *wqkv, *wo, *gate, *up, *down;      /* stream order; wqkv [emb, (n_heads + 2 n_kv_heads) head_dim] */
+    const uint16_t *attn_norm, *ffn_norm;
+    uint16_t *k_cache, *v_cache;                   /* [n_kv_heads, max_seq, head_dim] */
+} w4a16_decode_layer_t;
+typedef struct {
+    const w4a16_decode_layer_t *layers;
+    const uint16_t *embed, *final_norm, *lm_head, *rope_lut;   /* [embed_rows, emb], [emb], [vocab, emb], [lut_rows, head_dim] */
+    int32_t n_layers, emb, hidden, n_heads, n_kv_heads, head_dim, vocab, embed_rows, lut_rows, max_seq, q4nx;
+    float eps;
+} w4a16_decode_model_t;
+size_t w4a16_decode_run_workspace_bytes(const w4a16_decode_model_t *model);
+int w4a16_decode_run_bf16(const w4a16_decode_model_t *model, const uint16_t *first_x, int n_tokens, int start_pos, int32_t *ids,
+                          uint16_t *logits, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Launch-shape override for benchmarking sweeps (not needed for normal use).  Keys:
  * "gemv_lw", "gemv_ksteps", "gemv_waves", "gemv_units", "gemv_ksplit" (0 = built-in heuristic),
  * "gemm_stream_max_m" (largest M given to the streaming kernel, 0 = default 96, otherwise >= 16) and

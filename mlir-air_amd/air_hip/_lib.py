@@ -65,6 +65,8 @@ SYMBOLS = {
     "w4a16_repack_stream": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp]),
     "w4a16_gemv_stream_bf16": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _vp]),
     "w4a16_probe_stream_read": (_ci, [_vp, _vp, _ci, _ci, _vp]),
+    "w4a16_decode_run_workspace_bytes": (_sz, [_vp]),
+    "w4a16_decode_run_bf16": (_ci, [_vp, _vp, _ci, _ci, _vp, _vp, _vp, _sz, _vp]),
     "w4a16_gemm_stream_bf16": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp]),
     "w4a16_gemm_stream_scratch_bytes": (_sz, [_ci, _ci, _ci]),
     "w4a16_gemm_stream_best_scratch_bytes": (_sz, [_ci, _ci, _ci]),
@@ -90,6 +92,16 @@ _i32, _i64 = ctypes.c_int32, ctypes.c_int64
 class Intake(ctypes.Structure):
     _fields_ = [("mode", _i32), ("width", _i32), ("eps", _cf), ("scale", _cf), ("x", _vp), ("res", _vp), ("y", _vp), ("norm_w", _vp),
                 ("final_w", _vp), ("res_out", _vp), ("h_out", _vp), ("embed", _vp), ("token", _vp)]
+
+
+class DecodeLayer(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("wqkv", "wo", "gate", "up", "down", "attn_norm", "ffn_norm", "k_cache", "v_cache")]
+
+
+class DecodeModel(ctypes.Structure):
+    _fields_ = ([("layers", ctypes.POINTER(DecodeLayer))] + [(n, _vp) for n in ("embed", "final_norm", "lm_head", "rope_lut")]
+                + [(n, _i32) for n in ("n_layers", "emb", "hidden", "n_heads", "n_kv_heads", "head_dim", "vocab", "embed_rows", "lut_rows", "max_seq",
+                                       "q4nx")] + [("eps", _cf)])
 
 
 class Router(ctypes.Structure):

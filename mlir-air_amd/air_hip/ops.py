@@ -5,6 +5,8 @@ the current torch stream of the tensors' device and returns without
 synchronising.  There is no CPU path: tensors must live on the GPU.
 """
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -739,6 +741,50 @@ def lm_head(x, lm_head_weight, norm_weight=None, eps=1e-5, return_argmax=True, a
                                      float(eps), _ptr(_bits(lm_head_weight)), _ptr(logits),
                                      _ptr(best) if return_argmax else None, V, E, _ptr(ws), ws.numel(), _stream()))
     return (logits, best) if return_argmax else logits
+
+
+def decode_run(first_x, layers, embed_table, final_norm, lm_head_weight, rope_lut, config, kv_cache, start_pos, n_tokens, ids):
+    """All launches of n_tokens decode steps from one native call: `layers` with stream-order matrices of one codec, first_x the embedding
+    row at start_pos, `ids` int32 [n_tokens] the argmaxes.  Returns the last step's logits bf16 [V], or None, with nothing launched, where
+    the tensors are not of the form that the call takes (the ops of a single layer say what is wrong with them)."""
+    lib = _lib.load_library()
+    pairs = list(zip(layers, kv_cache))
+    names = ("wqkv", "wo", "w_gate", "w_up", "w_down")
+    if not pairs or any(l.stream is None for l, _ in pairs) or not (isinstance(start_pos, int) and n_tokens > 0 and start_pos >= 0):
+        return None
+    first, (k0, _) = pairs[0]
+    if k0.dim() != 3 or embed_table.dim() != 2 or lm_head_weight.dim() != 2 or rope_lut.dim() != 2:
+        return None
+    n_kv, max_seq, hd = k0.shape
+    E, H, codec, n_heads = first_x.numel(), first.stream["w_gate"].N, first.codec, config.n_heads
+    want = {"wqkv": (E, (n_heads + 2 * n_kv) * hd), "wo": (E, E), "w_gate": (E, H), "w_up": (E, H), "w_down": (H, E)}
+    plain = [first_x, embed_table, final_norm, lm_head_weight, rope_lut]
+    rows = (_lib.DecodeLayer * len(pairs))()
+    for r, (l, (kc, vc)) in zip(rows, pairs):
+        w = [l.stream[n] for n in names]
+        if (l.codec != codec or any(m.order != codec or (m.K, m.N) != want[n] for m, n in zip(w, names)) or kc.shape != k0.shape
+                or vc.shape != k0.shape or l.attn_norm.numel() != E or l.ffn_norm.numel() != E):
+            return None
+        tensors = [l.attn_norm, l.ffn_norm, kc, vc]
+        plain += tensors
+        bufs = [m.buf for m in w]
+        if not all(b.is_cuda and b.is_contiguous() for b in bufs):
+            return None
+        (r.wqkv, r.wo, r.gate, r.up, r.down), (r.attn_norm, r.ffn_norm, r.k_cache, r.v_cache) = [b.data_ptr() for b in bufs], [t.data_ptr() for t in tensors]
+    if (not all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() for t in plain) or final_norm.numel() != E
+            or embed_table.shape[1] != E or lm_head_weight.shape[1] != E or rope_lut.shape[1] != hd):
+        return None
+    V = lm_head_weight.shape[0]
+    m = _lib.DecodeModel(layers=rows, embed=_ptr(embed_table), final_norm=_ptr(final_norm), lm_head=_ptr(lm_head_weight), rope_lut=_ptr(rope_lut),
+                         n_layers=len(pairs), emb=E, hidden=H, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd, vocab=V,
+                         embed_rows=embed_table.shape[0], lut_rows=rope_lut.shape[0], max_seq=max_seq, q4nx=codec == "q4nx", eps=config.rms_eps)
+    nbytes = lib.w4a16_decode_run_workspace_bytes(ctypes.byref(m))
+    if not nbytes or start_pos + n_tokens > min(max_seq, rope_lut.shape[0]) or any(t.data_ptr() % 16 for t in plain):
+        return None
+    scratch = torch.empty(int(nbytes), dtype=torch.uint8, device=first_x.device)
+    logits = torch.empty((V,), dtype=torch.bfloat16, device=first_x.device)
+    _lib.check(lib.w4a16_decode_run_bf16(ctypes.byref(m), _ptr(first_x), n_tokens, start_pos, _ptr(ids), _ptr(logits), _ptr(scratch), int(nbytes), _stream()))
+    return logits
 
 
 def q4nx_dequant(blocks, M, K, mode=0, out=None):

@@ -955,6 +955,92 @@ int lm_head_gemv_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps,
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
 
+// [x E][qkv][attention output E][sums of squares E / 16][attention][block][lm_head]
+struct DecodeRunScratch {
+    uint16_t *x[2], *qkv, *attn;
+    float *sumsq;
+    void *attn_ws, *block_ws, *head_ws;
+    size_t attn_bytes, block_bytes, head_bytes, bytes;
+};
+static DecodeRunScratch decode_run_scratch(const w4a16_decode_model_t &m, void *workspace) {
+    DecodeRunScratch s;
+    char *p = static_cast<char *>(workspace);
+    size_t at = 0;
+    auto take = [&](size_t n) {
+        char *q = p ? p + at : nullptr;
+        at += round256(n);
+        return q;
+    };
+    const size_t E = m.emb;
+    for (auto &x : s.x) x = reinterpret_cast<uint16_t *>(take(E * 2));
+    s.qkv = reinterpret_cast<uint16_t *>(take((size_t)(m.n_heads + 2 * m.n_kv_heads) * m.head_dim * 2));
+    s.attn = reinterpret_cast<uint16_t *>(take(E * 2));
+    s.sumsq = reinterpret_cast<float *>(take((E / kWsTileCols + 1) * sizeof(float)));
+    s.attn_ws = take(s.attn_bytes = w4a16_attention_workspace_bytes(m.n_heads, m.head_dim));
+    s.block_ws = take(s.block_bytes = w4a16_block_stream_workspace_bytes(m.emb, m.hidden));
+    s.head_ws = take(s.head_bytes = lm_head_workspace_bytes(m.vocab));
+    s.bytes = at;
+    return s;
+}
+
+static bool decode_run_shapes_ok(const w4a16_decode_model_t &m) {
+    if (m.n_layers <= 0 || m.n_layers > 4096 || m.emb <= 0 || m.hidden <= 0 || m.emb % kGroup || m.hidden % kGroup || m.emb > 1 << 16) return false;
+    if ((m.head_dim != 64 && m.head_dim != 128) || m.n_heads <= 0 || m.n_kv_heads <= 0 || m.n_heads % m.n_kv_heads || m.n_heads * m.head_dim != m.emb) return false;
+    const int g = m.n_heads / m.n_kv_heads;
+    return (g == 1 || g == 2 || g == 4 || g == 8) && m.max_seq > 0 && lm_head_supported(m.vocab, m.emb) && m.embed_rows >= m.vocab && m.eps >= 0.f;
+}
+
+size_t w4a16_decode_run_workspace_bytes(const w4a16_decode_model_t *m) { return m && decode_run_shapes_ok(*m) ? decode_run_scratch(*m, nullptr).bytes : 0; }
+
+int w4a16_decode_run_bf16(const w4a16_decode_model_t *model, const uint16_t *first_x, int n_tokens, int start_pos, int32_t *ids,
+                          uint16_t *logits, void *workspace, size_t workspace_bytes, void *stream) {
+    if (!model || !first_x || !ids || !logits || !workspace) return W4A16_ERR_NULL;
+    const w4a16_decode_model_t &m = *model;
+    if (!m.layers || !m.embed || !m.final_norm || !m.lm_head || !m.rope_lut) return W4A16_ERR_NULL;
+    if (!decode_run_shapes_ok(m) || n_tokens <= 0 || start_pos < 0 || start_pos > m.max_seq - n_tokens || start_pos > m.lut_rows - n_tokens) return W4A16_ERR_SHAPE;
+    if (misaligned(first_x) || misaligned(m.embed) || misaligned(m.final_norm) || misaligned(m.lm_head) || misaligned(m.rope_lut) || misaligned(logits) ||
+        misaligned(workspace) || (reinterpret_cast<uintptr_t>(ids) & 3))
+        return W4A16_ERR_ALIGN;
+    const DecodeRunScratch s = decode_run_scratch(m, workspace);
+    if (workspace_bytes < s.bytes) return W4A16_ERR_WORKSPACE;
+    for (int i = 0; i < m.n_layers; ++i) {
+        const w4a16_decode_layer_t &l = m.layers[i];
+        const void *all[] = {l.wqkv, l.wo, l.gate, l.up, l.down, l.attn_norm, l.ffn_norm, l.k_cache, l.v_cache};
+        for (const void *p : all) {
+            if (!p) return W4A16_ERR_NULL;
+            if (misaligned(p)) return W4A16_ERR_ALIGN;
+        }
+    }
+    const int E = m.emb, nqkv = (m.n_heads + 2 * m.n_kv_heads) * m.head_dim;
+    const bool q4 = m.q4nx != 0;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    for (int t = 0; t < n_tokens; ++t) {
+        const int pos = start_pos + t;
+        const uint16_t *x = t == 0 ? first_x : s.x[1];
+        for (int i = 0; i < m.n_layers; ++i) {
+            const w4a16_decode_layer_t &l = m.layers[i];
+            GemvWsExtras ex;
+            ex.q4 = q4;
+            ex.norm_w = l.attn_norm;
+            ex.eps = m.eps;
+            if (i) ex.sumsq_in = s.sumsq, ex.sumsq_n = E / kWsTileCols;
+            int rc = gemv_stream_call(x, l.wqkv, nullptr, s.qkv, E, nqkv, kGroup, stream, ex);
+            if (rc) return rc;
+            const hipError_t e = launch_decode_attention(s.qkv, m.rope_lut + (size_t)pos * m.head_dim, l.k_cache, l.v_cache, s.attn, pos, m.max_seq, m.n_heads,
+                                                         m.n_kv_heads, m.head_dim, s.attn_ws, st);
+            if (e != hipSuccess) return hip_fail(e);
+            uint16_t *y = s.x[x == s.x[0] ? 1 : 0];
+            rc = o_gemv_ffn_stream_impl(s.attn, x, l.ffn_norm, m.eps, l.wo, l.gate, l.up, l.down, y, nullptr, nullptr, s.sumsq, E, m.hidden, kGroup,
+                                        s.block_ws, s.block_bytes, stream, false, q4);
+            if (rc) return rc;
+            x = y;
+        }
+        const hipError_t e = launch_lm_head(x, m.final_norm, m.eps, m.lm_head, logits, ids + t, m.vocab, E, s.head_ws, st, t + 1 < n_tokens ? m.embed : nullptr, s.x[1]);
+        if (e != hipSuccess) return hip_fail(e);
+    }
+    return W4A16_OK;
+}
+
 int q4nx_dequant_bf16(const void *blocks, uint16_t *out_bf16, int M, int K, int mode, void *stream) {
     if (!blocks || !out_bf16) return W4A16_ERR_NULL;
     if (M <= 0 || K <= 0 || M % 32 != 0 || K % 256 != 0 || mode < 0 || mode > 2) return W4A16_ERR_SHAPE;

@@ -199,7 +199,7 @@ hipError_t launch_q4nx_blocks_to_stream(const void *blocks, void *out, int M, in
 bool lm_head_supported(int V, int E);
 size_t lm_head_scratch_bytes(int V);
 hipError_t launch_lm_head(const uint16_t *x, const uint16_t *norm_w, float eps, const uint16_t *w, uint16_t *logits,
-                          int32_t *argmax_out, int V, int E, void *workspace, hipStream_t stream);
+                          int32_t *argmax_out, int V, int E, void *workspace, hipStream_t stream, const uint16_t *embed = nullptr, uint16_t *row = nullptr);   // embed: row [E] receives embed[argmax]
 
 // Decode attention (attention.hip).  The scratch buffer holds per-chunk softmax partials and
 // needs no initialisation.

@@ -153,8 +153,10 @@ __global__ void __launch_bounds__(kWaves * 64) lm_head_kernel(const LmHeadParams
     if (lane == 0) p.keys[gw] = key;
 }
 
-__global__ void __launch_bounds__(1024) lm_head_argmax_kernel(const unsigned long long *keys, int n, int32_t *out) {
+__global__ void __launch_bounds__(1024) lm_head_argmax_kernel(const unsigned long long *keys, int n, int32_t *out, const uint16_t *embed,
+                                                              uint16_t *row, int E) {
     __shared__ unsigned long long part[16];
+    __shared__ uint32_t id;
     unsigned long long best = 0;
     // eight independent loads per thread and round trip (one round for up to 131072 rows)
     for (int base = 0; base < n; base += 8 * 1024) {
@@ -173,8 +175,13 @@ __global__ void __launch_bounds__(1024) lm_head_argmax_kernel(const unsigned lon
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int i = 1; i < 16; ++i) best = part[i] > best ? part[i] : best;
-        out[0] = (int32_t)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull));
+        id = 0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull);
+        out[0] = (int32_t)id;
     }
+    if (!embed) return;
+    __syncthreads();
+    for (int e = 8 * threadIdx.x; e < E; e += 8 * 1024)
+        *reinterpret_cast<u32x4 *>(row + e) = *reinterpret_cast<const u32x4 *>(embed + (size_t)id * E + e);
 }
 
 template <int NCH, int RG>
@@ -203,7 +210,7 @@ size_t lm_head_scratch_bytes(int V) {
 }
 
 hipError_t launch_lm_head(const uint16_t *x, const uint16_t *norm_w, float eps, const uint16_t *w, uint16_t *logits,
-                          int32_t *argmax_out, int V, int E, void *workspace, hipStream_t stream) {
+                          int32_t *argmax_out, int V, int E, void *workspace, hipStream_t stream, const uint16_t *embed, uint16_t *row) {
     LmHeadParams p;
     p.x = x;
     p.norm_w = norm_w;
@@ -229,7 +236,7 @@ hipError_t launch_lm_head(const uint16_t *x, const uint16_t *norm_w, float eps, 
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !argmax_out) return e;
-    hipLaunchKernelGGL(lm_head_argmax_kernel, dim3(1), dim3(1024), 0, stream, p.keys, waves, argmax_out);
+    hipLaunchKernelGGL(lm_head_argmax_kernel, dim3(1), dim3(1024), 0, stream, p.keys, waves, argmax_out, embed, row, E);
     return hipGetLastError();
 }
 
