@@ -579,14 +579,16 @@ __global__ void __launch_bounds__(256) gemm_sum_kernel(const float *parts, int s
 // the 18).  M x N x K with the parts added up, before there were slices / now: 64 x 2048 x 8192 130 / 16 us, 300 x 2048 x 8192 79 / 28,
 // 2048 x 2048 x 8192 90 / 71; 64 x 16384 x 2048 with gelu 50 / 13 (64-row tiles).
 // Narrow tiles read W from L2 once per 32 or 64 rows, which costs more in a model, where other kernels have been there, than alone:
-// up to eight of them (2048 x 2048 x 2048 behind an attention: 32 us with 64-row tiles, 25 with wide ones alone).
+// up to eight of them (2048 x 2048 x 2048 behind an attention: 32 us with 64-row tiles, 25 with wide ones alone).  128 x 128 tiles stay
+// for what fills less than a round (808 x 1472 x 1664 with gelu: 23.6 us, 24.4 in wide tiles; 808 x 640 x 1664 5.7 / 7.6).
 struct GemmKind {
     int rows, cols, together;
     float tile_us, step_us, step_full_us, store_tbs;   // per tile; per K-step alone and in a full round; fp32 results
 };
-enum : int { kTile32, kTile64, kWide128, kWide192, kWide256, kKinds };
+enum : int { kTile32, kTile64, kTile128, kWide128, kWide192, kWide256, kKinds };
 constexpr GemmKind kGemmKinds[kKinds] = {
-    {32, 128, 2, 1.0f, 0.215f, 0.43f, 6.8f}, {64, 128, 2, 0.f, 0.364f, 0.541f, 3.7f},    {128, 256, 1, 2.6f, 0.566f, 0.696f, 5.8f},
+    {32, 128, 2, 1.0f, 0.215f, 0.43f, 6.8f}, {64, 128, 2, 0.f, 0.364f, 0.541f, 3.7f},  {128, 128, 2, 0.f, 0.547f, 0.866f, 4.4f},
+    {128, 256, 1, 2.6f, 0.566f, 0.696f, 5.8f},
     {256, 192, 1, 5.8f, 0.728f, 0.947f, 10.3f}, {256, 256, 1, 7.5f, 0.953f, 1.201f, 11.f}};
 float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int slices) {
     const long tiles = (long)((M + k.rows - 1) / k.rows) * ((N + k.cols - 1) / k.cols) * slices, cap = 256 * k.together;
@@ -596,7 +598,8 @@ float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int sl
     float t = 4.f + full * (k.tile_us + per * k.step_full_us);
     if (rest) t += k.tile_us + per * (k.step_us + (k.step_full_us - k.step_us) * rest / cap);
     if (epilogue == kOutF32 || slices > 1) t += slices * mb / k.store_tbs;
-    if (slices > 1) t += epilogue == kOutF32 ? (slices - 1) * mb / 5.f : 3.5f + (slices + 0.5f) * mb / 4.f;   // whoever adds them up
+    // whoever adds them up: the next kernel, or a launch (3.5 us on the GPU, 6 with its allocation on the host, which short prompts wait for)
+    if (slices > 1) t += epilogue == kOutF32 ? (slices - 1) * mb / 5.f : 6.f + (slices + 0.5f) * mb / 4.f;
     return t;
 }
 
@@ -608,7 +611,7 @@ GemmChoice choose_gemm(int M, int N, int K, int epilogue, int slices) {
     GemmChoice best{kWide256, 1};
     float least = 1e30f;
     const int steps = K / 64, first = slices ? slices : 1, last = slices ? slices : steps >= 8 ? (steps / 4 < 8 ? steps / 4 : 8) : 1;
-    for (int kind = M > 512 ? kWide128 : M > 256 ? kTile64 : kTile32; kind < kKinds; ++kind)
+    for (int kind = M > 1024 ? kWide128 : M > 512 ? kTile128 : M > 256 ? kTile64 : kTile32; kind < kKinds; ++kind)
         for (int n = first; n <= last; n *= 2) {
             const float t = gemm_time(kGemmKinds[kind], M, N, steps, epilogue, n);
             if (t < least) {
@@ -627,6 +630,7 @@ hipError_t launch_kind(const GemmArgs &g, int kind, int slices, hipStream_t stre
     switch (kind) {
         case kTile32: return launch_tile<bf16, 32, 128, 1, 4, 4>(g, slices, stream);
         case kTile64: return launch_tile<bf16, 64, 128, 1, 4, 3>(g, slices, stream);
+        case kTile128: return launch_tile<bf16, 128, 128, 2, 2, 2>(g, slices, stream);
         case kWide128: return launch_wide<1, 4>(g, slices, stream);
         case kWide192: return launch_wide<2, 6>(g, slices, stream);
         default: return launch_wide<2, 8>(g, slices, stream);
