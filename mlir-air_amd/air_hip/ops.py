@@ -21,7 +21,8 @@ def _ptr(t):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream, as torch.cuda.current_stream().cuda_stream (which takes 1 us longer to build its object)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need_cuda(*tensors):
