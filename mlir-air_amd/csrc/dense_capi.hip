@@ -274,7 +274,7 @@ int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
     GemmArgs a;
     if (g && !g->out) return DLM_ERR_NULL;
     if (const int e = gemm_args(dtype, g, a)) return e;
-    if (g->tile_rows != 32 && g->tile_rows != 128 && g->tile_rows != 256) return DLM_ERR_SHAPE;
+    if (g->tile_rows != 32 && g->tile_rows != 128 && g->tile_rows != 256 && !(g->tiles && g->tile_rows == 384 && dtype == kBf16)) return DLM_ERR_SHAPE;
     return done(launch_dense_gemm(dtype, a, g->tile_rows, hs(stream)));
 }
 

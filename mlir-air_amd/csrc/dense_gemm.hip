@@ -248,11 +248,11 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
     const int stride = products / items;
     return n % stride == stride - 1 && n / stride < items ? n / stride : -1;
 }
-// A wave's NT x 8 tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
+// A wave's NT x MT tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
-template <int NT, int EPI, bool GROUPED>
-__device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][8], char *lds, int m_first, int m_end, int n_first) {
+template <int NT, int MT, int EPI, bool GROUPED>
+__device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first) {
     typedef typename std::conditional<EPI == kOutF32, float, bf16>::type Out;
     constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
     constexpr int kCols = 16 * NT / (kPair ? 2 : 1), kPiece = 16 / (int)sizeof(Out), kPitch = kCols + kPiece;
@@ -262,7 +262,7 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
     Out *rows = reinterpret_cast<Out *>(lds);
     const int n_out = kPair ? n_first / 2 : n_first, n_end = kPair ? p.N / 2 : p.N;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MT; ++i) {
         if (m_first + 16 * i >= m_end) break;   // uniform
 #pragma unroll
         for (int j = 0; j < NT; j += kPair ? 2 : 1) {
@@ -296,7 +296,7 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
     }
 }
 
-template <int WM, int NT, int EPI, bool GROUPED>
+template <int WM, int NT, int EPI>
 __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, KSlice slice) {
     constexpr int WN = 4 / WM, BM = 128 * WM, BN = 16 * NT * WN;
     constexpr int H0 = (NT + 1) / 2, H1 = NT - H0;        // column tiles of the two halves of a wave's columns
@@ -311,21 +311,15 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
 
     // Copy i of a wave fills KiB i of the wave's part of a stage: eight rows, lane's chunk (lane % 8) ^ row % 8.  Four copies share
     // their LDS base (M0) and differ in the instruction's offset, which the hardware adds to both addresses: the source takes it back.
-    // (Offsets from the wave's first row, 64 rows at most; gathered rows lie anywhere: their addresses are per lane.)
+    // (Offsets from the wave's first row, 64 rows at most.)
     uint32_t off_a[CA], off_w[CW];
-    const char *row_a[CA];
     const int m_wave = m0 + 8 * CA * wave < m_end ? m0 + 8 * CA * wave : m_end - 1, n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
         const int row = 8 * (CA * wave + i) + (lane >> 3);
         const uint32_t chunk = 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
-        int m = m0 + row < m_end ? m0 + row : m_end - 1;
-        if constexpr (GROUPED) {
-            if (p.gather > 0) m = p.order[m] / p.gather;
-            row_a[i] = reinterpret_cast<const char *>(p.a + (size_t)m * p.lda) + chunk;
-        } else {
-            off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + chunk;
-        }
+        const int m = m0 + row < m_end ? m0 + row : m_end - 1;
+        off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + chunk;
     }
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
@@ -334,7 +328,7 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
         off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
     }
     const size_t from = (size_t)slice.first * kRowBytes;
-    gptr base_a = scalar_ptr((GROUPED ? nullptr : reinterpret_cast<const char *>(p.a + (size_t)m_wave * p.lda)) + from - 4096);
+    gptr base_a = scalar_ptr(reinterpret_cast<const char *>(p.a + (size_t)m_wave * p.lda) + from - 4096);
     gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from - 4096);
     auto copy = [&](gptr from, int at, int i) {
         const auto *src = (const __attribute__((address_space(1))) void *)from;
@@ -346,10 +340,7 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
             default: __builtin_amdgcn_global_load_lds(src, dst, 16, 3072, 0); break;
         }
     };
-    auto copy_a = [&](int side, int i) {
-        if constexpr (GROUPED) copy((gptr)(row_a[i] + (ptrdiff_t)base_a), side + 1024 * CA * wave, i);
-        else copy(base_a + off_a[i], side + 1024 * CA * wave, i);
-    };
+    auto copy_a = [&](int side, int i) { copy(base_a + off_a[i], side + 1024 * CA * wave, i); };
     auto copy_w = [&](int side, int i) { copy(base_w + off_w[i], 2 * kSideA + side + 1024 * CW * wave, i); };
 
     const int steps = slice.steps;
@@ -398,7 +389,7 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
     for (int kt = 0; kt < steps; ++kt) {
         // (opaque in this block: the offsets' zero extension folds into the copies only if it is not taken out of the loop)
 #pragma unroll
-        for (int i = 0; i < CA && !GROUPED; ++i) asm volatile("" : "+v"(off_a[i]));
+        for (int i = 0; i < CA; ++i) asm volatile("" : "+v"(off_a[i]));
 #pragma unroll
         for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
         // first columns, first half of the K-step; the other half of A's copies for the next K-step
@@ -453,32 +444,201 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
     for (int j = 0; j < NT; ++j)
         asm volatile("" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
 
-    store_rows<NT, EPI, GROUPED>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
+    store_rows<NT, 8, EPI, false>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
 }
 
-// GROUPED: an expert's last tile may have 128 rows or less; the waves then lie side by side and it takes half as long.
-template <int WM, int NT, int EPI, bool GROUPED>
+template <int WM, int NT, int EPI>
 __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const GemmKernelArgs<bf16> p) {
     extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
     constexpr int BM = 128 * WM, BN = 16 * NT * (4 / WM);
-    const int tiles_m = GROUPED ? p.tiles[4 * p.tiles_m] : p.tiles_m;
+    const int tiles_m = p.tiles_m;
     const int total = tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
     const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= total) return;
     const int band = tile / (4 * p.tiles_n), in_band = tile % (4 * p.tiles_n);
     const int rows_in_band = tiles_m - 4 * band < 4 ? tiles_m - 4 * band : 4;
     const int tm = 4 * band + in_band % rows_in_band, tn = in_band / rows_in_band;
-    const KSlice slice = k_slice(p.K / 64);
-    if constexpr (GROUPED) {
-        const int32_t *t = p.tiles + 4 * tm;
-        const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
-        if (t[2] <= 128) wide_tile<1, NT / 2, EPI, true>(p, gemm_lds, w, t[1], t[1] + t[2], tn * BN, slice);
-        else wide_tile<WM, NT, EPI, true>(p, gemm_lds, w, t[1], t[1] + t[2], tn * BN, slice);
-    } else {
-        wide_tile<WM, NT, EPI, false>(p, gemm_lds, p.w, tm * BM, p.M, tn * BN, slice);
-    }
+    wide_tile<WM, NT, EPI>(p, gemm_lds, p.w, tm * BM, p.M, tn * BN, k_slice(p.K / 64));
 }
 
+
+// ---- experts, bf16 -----------------------------------------------------------------------------------------------------------
+// 64 MT rows of an expert (MT <= 6) x 128 columns, four waves one below the other, a wave 16 MT rows x 128 columns.
+//
+// What bounds it: an expert's W is read for its few hundred rows alone, so HBM (W once: 64 experts of 2048 x 2048 take 100 us) as well as the
+// matrix pipe.  A workgroup has all of an expert's rows where they are 384 or less (else even parts of them), so W leaves HBM once, in
+// 128 columns, so that there are many workgroups of even work, and does whole 64-row tiles' products only.
+// A K-step is two halves of 8 MT products of 16 cycles; each half's operands are read during the one before it.  One wait and barrier
+// stand between the halves: all of the next K-step has landed, everybody has read all of this one, and the copies of a K-step two or three
+// on (buffers: W three, A three up to 256 rows, else two; more of them for few rows were no faster) go out behind the products after it.
+constexpr int kExpertCols = 128, kExpertRows = 384;
+constexpr int kExpertStagesW = 3;
+constexpr int expert_stages_a(int mt) { return mt <= 4 ? 3 : 2; }
+constexpr size_t expert_lds(int mt) { return (size_t)(expert_stages_a(mt) * 64 * mt + kExpertStagesW * kExpertCols) * kRowBytes; }
+// of `items` that are to be spread over the products [0, upto): the first one that goes behind product n or later
+__device__ constexpr int items_before(int n, int upto, int items) { return n >= upto ? items : n * items / upto; }
+
+template <int MT, int EPI>
+__device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, int first) {
+    constexpr int kSideA = 64 * MT * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(MT), RW = kExpertStagesW;
+    constexpr int kBehind = RA == RW ? (RA - 2) * (2 * MT + 4) : 4;   // copies that may be on their way at the wait
+    constexpr int CA = 2 * MT, CW = 4, V = CA + CW, kEarly = V / 2;   // copies of a wave and K-step; those right behind the barrier
+    constexpr int kProducts = 8 * MT, kReads = 8 + MT, kReadsUpto = MT == 1 ? 4 : kProducts * 3 / 4;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ql = lane & 15, g = lane >> 4;
+
+    // copies as in wide_tile: KiB i of the wave's part of a stage, eight rows, lane's chunk (lane % 8) ^ row % 8
+    const char *row_a[CA];
+    uint32_t off_w[CW];
+    const int n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
+#pragma unroll
+    for (int i = 0; i < CA; ++i) {
+        const int row = 8 * (CA * wave + i) + (lane >> 3);
+        int m = m0 + row < m_end ? m0 + row : m_end - 1;
+        if (p.gather > 0) m = p.order[m] / p.gather;
+        row_a[i] = reinterpret_cast<const char *>(p.a + (size_t)m * p.lda) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+    }
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+        const int row = 8 * (CW * wave + i) + (lane >> 3);
+        const int n = n0 + row < p.N ? n0 + row : p.N - 1;
+        off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+    }
+    const int steps = p.K / 64;
+    ptrdiff_t from_a = (ptrdiff_t)first * kRowBytes - 4096;
+    gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from_a);
+    auto copy = [&](gptr from, int at, int i) {
+        const auto *src = (const __attribute__((address_space(1))) void *)from;
+        auto *dst = (__attribute__((address_space(3))) void *)(lds + at + 1024 * (i & ~3));
+        switch (i & 3) {
+            case 0: __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0); break;
+            case 1: __builtin_amdgcn_global_load_lds(src, dst, 16, 1024, 0); break;
+            case 2: __builtin_amdgcn_global_load_lds(src, dst, 16, 2048, 0); break;
+            default: __builtin_amdgcn_global_load_lds(src, dst, 16, 3072, 0); break;
+        }
+    };
+    int fill_a = 0, fill_w = 0;   // stages that the next K-step's copies go to
+    // copy i of a K-step, A's first; behind the last one of each the source moves on (at the end it stays)
+    int next_a = first, next_w = first;
+    auto step_copy = [&](int i) {
+        if (i < CA) {
+            copy((gptr)(row_a[i < CA ? i : 0] + from_a), fill_a + 1024 * CA * wave, i);
+            if (i == CA - 1) {
+                const bool wrap = next_a + 1 == steps;
+                next_a = wrap ? 0 : next_a + 1;
+                from_a += wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
+                fill_a = fill_a == (RA - 1) * kSideA ? 0 : fill_a + kSideA;
+            }
+        } else {
+            copy(base_w + off_w[i < CA ? 0 : i - CA], RA * kSideA + fill_w + 1024 * CW * wave, i - CA);
+            if (i == V - 1) {
+                const bool wrap = next_w + 1 == steps;
+                next_w = wrap ? 0 : next_w + 1;
+                base_w += wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
+                fill_w = fill_w == (RW - 1) * kSideW ? 0 : fill_w + kSideW;
+            }
+        }
+    };
+
+    // operand addresses of the two halves (32 k) of a K-step; tile i is the instruction's offset
+    uint32_t at_a[2], at_w[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        const uint32_t o = ql * kRowBytes + 16 * ((4 * ks + g) ^ (ql & 7));
+        at_a[ks] = o + wave * 16 * MT * kRowBytes;
+        at_w[ks] = o + RA * kSideA;
+    }
+    auto read = [&](uint32_t at, int i) { return *reinterpret_cast<const bf16x8 *>(lds + at + i * 16 * kRowBytes); };
+
+    floatx4 acc[8][MT];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 a0[MT], a1[MT], w0[8], w1[8];
+    // 8 MT products with the reads of the next half and copies [c0, c1) of a K-step behind them
+    auto half = [&](const bf16x8 (&wh)[8], const bf16x8 (&ah)[MT], bf16x8 (&wn)[8], bf16x8 (&an)[MT], uint32_t from_wn, uint32_t from_an, auto c0, auto c1) {
+#pragma unroll
+        for (int n = 0; n < kProducts; ++n) {
+            __builtin_amdgcn_sched_barrier(0);
+            mfma_in_place(acc[n % 8][n / 8], wh[n % 8], ah[n / 8]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < kReads; ++r)
+                if (r >= items_before(n, kReadsUpto, kReads) && r < items_before(n + 1, kReadsUpto, kReads)) {
+                    if (r < 8) wn[r < 8 ? r : 0] = read(from_wn, r);
+                    else an[r < 8 ? 0 : r - 8] = read(from_an, r - 8);
+                }
+#pragma unroll
+            for (int c = 0; c < V; ++c)
+                if (c >= c0 + items_before(n, kProducts, c1 - c0) && c < c0 + items_before(n + 1, kProducts, c1 - c0)) step_copy(c);
+        }
+    };
+
+    // All buffers but one each, and the first copies of the next K-step (with two buffers for A and three for W, A of K-step t + 2 goes with
+    // W of t + 3)
+#pragma unroll
+    for (int s = 0; s < RW - 1; ++s)
+#pragma unroll
+        for (int i = s == 1 && RA == 2 ? CA : 0; i < V; ++i) step_copy(i);
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) step_copy(i);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + kEarly) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w0[j] = read(at_w[0], j);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a0[i] = read(at_a[0], i);
+
+    int side_a = 0, side_w = 0;   // of the K-step that is multiplied
+#pragma unroll 1
+    for (int kt = 0; kt < steps; ++kt) {
+#pragma unroll
+        for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
+        half(w0, a0, w1, a1, at_w[1], at_a[1], std::integral_constant<int, kEarly>(), std::integral_constant<int, V>());
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int by_a = side_a == (RA - 1) * kSideA ? -side_a : kSideA, by_w = side_w == (RW - 1) * kSideW ? -side_w : kSideW;
+        side_a += by_a;
+        side_w += by_w;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) at_a[ks] += by_a, at_w[ks] += by_w;
+        half(w1, a1, w0, a0, at_w[0], at_a[0], std::integral_constant<int, 0>(), std::integral_constant<int, kEarly>());
+    }
+    // no copy, of any wave, is on its way to LDS any more; the products have left the matrix pipe
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+        asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]), "+a"(acc[4][i]), "+a"(acc[5][i]), "+a"(acc[6][i]), "+a"(acc[7][i]));
+    store_rows<8, MT, EPI, true>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0);
+}
+
+template <int EPI>
+__global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_expert_kernel(const GemmKernelArgs<bf16> p) {
+    extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
+    const int tiles_m = p.tiles[4 * p.tiles_m];
+    const int total = tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= total) return;
+    const int32_t *t = p.tiles + 4 * (tile / p.tiles_n);   // columns first: an XCD's workgroups share the rows of two experts or so in its L2
+    const int n0 = tile % p.tiles_n * kExpertCols, m0 = t[1], m_end = m0 + t[2];
+    const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
+    const int first = (5 * t[0] + 3 * (tile % p.tiles_n)) % (p.K / 64);
+    switch ((t[2] + 63) / 64) {
+        case 1: return expert_tile<1, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+        case 2: return expert_tile<2, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+        case 3: return expert_tile<3, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+        case 4: return expert_tile<4, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+        case 5: return expert_tile<5, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+        default: return expert_tile<6, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+    }
+}
 
 template <class T>
 GemmKernelArgs<T> kernel_args(const GemmArgs &g, int bm, int bn) {
@@ -519,9 +679,10 @@ hipError_t launch_tile(const GemmArgs &g, int slices, hipStream_t stream) {
     const GemmKernelArgs<T> p = kernel_args<T>(g, BM, BN);
     constexpr size_t lds = STAGES * (size_t)(BM + BN) * kRowBytes;
     auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<T>>(kernel, p, 64 * WM * WN, lds, slices, stream); };
-    if (g.tiles)
-        return g.epilogue == kOutSwiglu ? run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutSwiglu, true>)
-                                        : run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutElem, true>);
+    if constexpr (std::is_same<T, float>::value)
+        if (g.tiles)
+            return g.epilogue == kOutSwiglu ? run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutSwiglu, true>)
+                                            : run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutElem, true>);
     switch (g.epilogue) {
         case kOutF32: return run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutF32, false>);
         case kOutSwiglu: return run(&dense_gemm_kernel<T, BM, BN, WM, WN, STAGES, kOutSwiglu, false>);
@@ -534,14 +695,20 @@ template <int WM, int NT>
 hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
     const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, 128 * WM, 16 * NT * (4 / WM));
     auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, wide_lds(WM, NT), slices, stream); };
-    if constexpr (WM == 2 && NT == 8)
-        if (g.tiles) return g.epilogue == kOutSwiglu ? run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu, true>) : run(&dense_gemm_wide_kernel<WM, NT, kOutElem, true>);
     switch (g.epilogue) {
-        case kOutF32: return run(&dense_gemm_wide_kernel<WM, NT, kOutF32, false>);
-        case kOutSwiglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu, false>);
-        case kOutGeglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutGeglu, false>);
-        default: return run(&dense_gemm_wide_kernel<WM, NT, kOutElem, false>);
+        case kOutF32: return run(&dense_gemm_wide_kernel<WM, NT, kOutF32>);
+        case kOutSwiglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu>);
+        case kOutGeglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutGeglu>);
+        default: return run(&dense_gemm_wide_kernel<WM, NT, kOutElem>);
     }
+}
+
+hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
+    const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, kExpertRows, kExpertCols);
+    constexpr size_t lds = expert_lds(6);
+    static_assert(lds <= 160 * 1024 && expert_lds(4) <= lds && expert_lds(5) <= lds && 4 * kWideStore <= lds, "fits LDS");
+    return g.epilogue == kOutSwiglu ? run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutSwiglu>, p, kWideThreads, lds, 1, stream)
+                                    : run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutElem>, p, kWideThreads, lds, 1, stream);
 }
 
 // out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
@@ -641,16 +808,15 @@ hipError_t launch_kind(const GemmArgs &g, int kind, int slices, hipStream_t stre
 
 // Rows of A per tile for a product of `rows` rows with each of `matrices` matrices.
 int dense_gemm_tile_rows(int dtype, int rows, int N, int matrices) {
+    if (dtype == kBf16 && matrices > 1) return kExpertRows;
     if (rows <= 48 || N < 96) return 32;
-    if (dtype != kBf16) return 128;
-    if (matrices > 1) return rows >= 160 && N >= 256 ? 256 : 128;
-    return rows > 128 ? 256 : 128;
+    return dtype == kBf16 && rows > 128 ? 256 : 128;
 }
 
 hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStream_t stream) {
     if (dtype == kF32) return tile_rows == 32 ? launch_tile<float, 32, 128, 1, 4, 4>(g, 1, stream) : launch_tile<float, 128, 128, 2, 2, 2>(g, 1, stream);
+    if (g.tiles) return g.K < 1 << 26 ? launch_experts(g, stream) : hipErrorInvalidValue;   // (any plan: its tiles are 384 rows or less)
     if (tile_rows == 32) return launch_tile<bf16, 32, 128, 1, 4, 4>(g, 1, stream);
-    if (g.tiles) return tile_rows == 128 ? launch_tile<bf16, 128, 128, 2, 2, 2>(g, 1, stream) : long_rows(g) ? hipErrorInvalidValue : launch_wide<2, 8>(g, 1, stream);
     return launch_kind(g, tile_rows == 256 ? kWide256 : kWide128, 1, stream);
 }
 

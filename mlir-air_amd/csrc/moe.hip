@@ -132,14 +132,17 @@ __global__ void __launch_bounds__(1024) moe_plan_kernel(const int32_t *ids, int 
         }
         __syncthreads();
     }
-    if (t < experts)
-        for (int i = 0; i * bm < n; ++i) {
+    if (t < experts && n) {   // as few tiles as there have to be, even ones where they are tall (in 64 rows)
+        const int parts = (n + bm - 1) / bm, each = bm > 256 && bm % 64 == 0 ? ((n + parts - 1) / parts + 63) / 64 * 64 : bm;
+        for (int i = 0; i < parts; ++i) {
             int32_t *row = tiles + 4 * (tile0[t] + i);
+            const int left = n - i * each;
             row[0] = t;
-            row[1] = first[t] + i * bm;
-            row[2] = n - i * bm < bm ? n - i * bm : bm;
+            row[1] = first[t] + i * each;
+            row[2] = left < each ? left : each;
             row[3] = 0;
         }
+    }
     if (t == 0) tiles[4 * max_tiles] = tile0[1024];
     count[t] = 0;
     __syncthreads();

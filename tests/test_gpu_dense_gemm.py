@@ -86,10 +86,10 @@ def test_parts_meet_in_the_row_kernels(dense, M, K):
     assert dense.gemm(a, w, out_f32=True, parts=True).shape[1:] == (M, K)
 
 
-COUNTS = [(0, 1, 15, 128, 129, 255, 256, 257), (512, 0, 0, 300, 64, 127, 383, 385), (16, 16, 16, 16, 16, 16, 16, 16), (0, 0, 0, 700, 0, 0, 0, 0)]
+COUNTS = [(0, 1, 15, 128, 129, 255, 256, 257), (512, 0, 0, 300, 64, 127, 383, 385), (16, 16, 16, 16, 16, 16, 16, 16), (0, 0, 0, 700, 0, 0, 0, 0), [384, 385, 320, 770, 192, 321]]
 
 
-@pytest.mark.parametrize("tile_rows", [32, 128, 256])
+@pytest.mark.parametrize("tile_rows", [32, 128, 256, 384])
 @pytest.mark.parametrize("counts", COUNTS)
 def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows):
     print("experts", counts, tile_rows, flush=True)
