@@ -560,7 +560,7 @@ static WsmPlan gemm_stream_plan(int M, int K, int N, bool q4, bool residual, siz
     if (!gemm_wsm_supported(M, K, N) || (rounded ? tune.prefill_tile != 0 : tune.gemm_rows || tune.cb || tune.splitk == 2)) return p;
     p = plan_gemm_wsm(M, K, N, q4, rounded, scratch_bytes);
     const bool always = !rounded && tune.splitk == 1;
-    if (!always && p.us > 0.95 * (rounded ? gemm_prefill_ws_us(M, K, N, q4) : gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
+    if (!always && p.us > 0.95 * (rounded ? gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
     return p;
 }
 
@@ -570,7 +570,7 @@ static int gemm_stream_run(const uint16_t *x, const void *w, const uint16_t *res
     const bool rounded = gemm_stream_rounded(M, K, N, q4, residual != nullptr);
     const WsmPlan plan = gemm_stream_plan(M, K, N, q4, residual != nullptr, scratch ? scratch_bytes : 0);
     hipError_t e = plan.us >= 0 ? launch_gemm_wsm(plan, x, w, y, residual, static_cast<float *>(scratch), M, K, N, q4, rounded, st)
-                   : rounded    ? launch_gemm_prefill_ws(x, w, y, M, K, N, st, kEpiNone, nullptr, nullptr, q4)
+                   : rounded    ? launch_gemm_prefill_ws(x, w, y, M, K, N, st, kEpiNone, nullptr, nullptr, q4, static_cast<float *>(scratch), scratch_bytes)
                                 : launch_gemm_ws(x, w, y, residual, M, K, N, st, q4);
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
@@ -584,13 +584,14 @@ size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N) {
     return slices > 1 ? (size_t)slices * rows * N * sizeof(float) : 0;
 }
 
-constexpr size_t kGemmScratchMost = (size_t)256 << 20;
+static size_t gemm_stream_best_scratch(int M, int K, int N, bool q4, bool residual) {
+    constexpr size_t kMost = (size_t)1 << 30;
+    const WsmPlan p = gemm_stream_plan(M, K, N, q4, residual, kMost);
+    return p.us >= 0 ? gemm_wsm_scratch_bytes(p, M, N) : gemm_stream_rounded(M, K, N, q4, residual) ? gemm_prefill_ws_scratch_bytes(M, K, N, q4, kMost) : 0;
+}
 
 size_t w4a16_gemm_stream_best_scratch_bytes(int M, int K, int N) {
-    const size_t least = w4a16_gemm_stream_scratch_bytes(M, K, N);
-    if (!gemm_wsm_supported(M, K, N)) return least;
-    const WsmPlan p = gemm_stream_plan(M, K, N, false, false, kGemmScratchMost);
-    return p.us >= 0 ? std::max(gemm_wsm_scratch_bytes(p, M, N), least) : least;
+    return std::max(gemm_stream_best_scratch(M, K, N, false, false), w4a16_gemm_stream_scratch_bytes(M, K, N));
 }
 
 static int gemm_stream_call(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group, void *scratch, size_t scratch_bytes,
@@ -1094,8 +1095,7 @@ int w4a16_q4nx_gemm_stream_bf16(const uint16_t *x, const void *wstream, const ui
 }
 
 size_t w4a16_q4nx_gemm_stream_best_scratch_bytes(int M, int K, int N, int has_residual) {
-    const WsmPlan p = gemm_stream_plan(M, K, N, true, has_residual != 0, kGemmScratchMost);
-    return p.us >= 0 ? gemm_wsm_scratch_bytes(p, M, N) : 0;
+    return gemm_stream_best_scratch(M, K, N, true, has_residual != 0);
 }
 
 int w4a16_q4nx_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,

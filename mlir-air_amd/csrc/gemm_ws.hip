@@ -149,6 +149,7 @@ struct PfArgs {
     int rope_cols, rope_hd, rope_pos0;
     int band;               // row panels per band of the tile order (pf_tile_of)
     bool q4;                // the matrices are in Q4NX order
+    float *parts;           // slices of K (the grid's y): fp32 sums [slice][M, N] instead of y
 };
 
 // One output tile: rows m0 .., columns col0 .. col0 + 64 NCB - 1.
@@ -157,8 +158,8 @@ struct PfArgs {
 // and the operand of K-step t is dequantised with its own word.  Same loop otherwise: four scale-word requests per
 // tile and group instead of one, two more instructions per operand (the word's halves to two fp32 registers) instead
 // of three per group.
-template <int NCB, bool Q4>
-__device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int m0, int col0) {
+template <int NCB, bool Q4, bool PARTS>
+__device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int m0, int col0, int g_lo, int g_hi) {
     constexpr int RT = kPfRowTiles, TM = kPfRows, WN = 16 * NCB, TN = 4 * WN;
     constexpr int kStageBytes = TM * 256;
 
@@ -304,7 +305,7 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     // and in a second copy of the loop body the register allocator moves them, through VGPRs, right behind MFMAs it
     // does not know of.
     auto group_step = [&](int g, int stage, int set) {
-        const int gn = g + 1 < G ? g + 1 : g;
+        const int gn = g + 1 < g_hi ? g + 1 : g;
         const XSrc xs = x_src(gn);
         // The zero extension of a lane offset must sit in the same basic block as its request to fold into the
         // instruction's 32-bit offset; taken opaque here, once per group, not next to the request (the compiler puts an
@@ -391,9 +392,9 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     };
 
 #pragma unroll
-    for (int i = 0; i < RT; ++i) copy_x_part(0, x_src(0), i);   // (64-bit addresses here: once per tile)
+    for (int i = 0; i < RT; ++i) copy_x_part(0, x_src(g_lo), i);   // (64-bit addresses here: once per tile)
 #pragma unroll
-    for (int c = 0; c < NCB; ++c) load_w_tile(0, w_offsets(0), c);
+    for (int c = 0; c < NCB; ++c) load_w_tile(0, w_offsets(g_lo), c);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the x tile copy writes LDS behind the compiler's back
     __syncthreads();
     take_w(0);
@@ -407,8 +408,8 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     for (int r = 0; r < RT; ++r) a[0][r] = read_a(0, 0, r);
     b_cur = dequant_operand(cell[0][0][0], sf[0], c0[0]);
 
-    // two groups per trip (G is even): stage / register set 0, then 1
-    for (int g = 0; g < G; g += 2) {
+    // two groups per trip (an even number of them): stage / register set 0, then 1
+    for (int g = g_lo; g < g_hi; g += 2) {
         group_step(g, 0, 0);
         group_step(g + 1, 1, 1);
     }
@@ -423,6 +424,26 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
 #pragma unroll
         for (int c = 0; c < NCB; ++c) asm volatile("" : "+a"(acc[r][c]));   // and no read of them moves above that wait
     __syncthreads();                                      // every wave is done reading the last x tile
+    if constexpr (PARTS) {   // whole rows of the tile's columns, 128 rows at a time
+        constexpr int LDF = TN + 4;
+        float *cf = reinterpret_cast<float *>(lds), *part = p.parts + (size_t)blockIdx.y * M * N;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (half) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < RT / 2; ++r)
+#pragma unroll
+                for (int c = 0; c < NCB; ++c)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) cf[(16 * r + 4 * lg + i) * LDF + wave * WN + 16 * c + ln] = acc[half * (RT / 2) + r][c][i];
+            __syncthreads();
+            for (int chunk = threadIdx.x; chunk < TM / 2 * (TN / 4); chunk += kPfThreads) {
+                const int row = chunk / (TN / 4), col = chunk % (TN / 4) * 4, m = m0 + half * (TM / 2) + row;
+                if (m < M) *reinterpret_cast<floatx4 *>(part + (size_t)m * N + col0 + col) = *reinterpret_cast<const floatx4 *>(cf + row * LDF + col);
+            }
+        }
+        return;
+    }
     uint16_t *ct = reinterpret_cast<uint16_t *>(lds);
 #pragma unroll
     for (int r = 0; r < RT; ++r)
@@ -516,10 +537,11 @@ __device__ __forceinline__ void pf_tile_of(int idx, int tiles_m, int n_cols, int
 
 // blockIdx -> tile.  The wide tiles come first in dispatch order, so that the narrow ones fill in behind them.  Each
 // XCD (blockIdx % 8) takes a contiguous range of the tiles of either width in the order of pf_tile_of.
-template <int NW, int NN, bool Q4>
+template <int NW, int NN, bool Q4, bool PARTS>
 __global__ void __launch_bounds__(kPfThreads, 1) gemm_wsp_kernel(const PfArgs p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int pairs = p.G / 2, g_lo = PARTS ? (int)((long)pairs * blockIdx.y / gridDim.y) * 2 : 0, g_hi = PARTS ? (int)((long)pairs * (blockIdx.y + 1) / gridDim.y) * 2 : p.G;
     const int wide_total = p.tiles_m * p.n_wide, narrow_total = p.tiles_m * p.n_narrow;
     const int wide_per_xcd = (wide_total + 7) / 8, narrow_per_xcd = (narrow_total + 7) / 8;
     if (slot < wide_per_xcd) {
@@ -527,13 +549,13 @@ __global__ void __launch_bounds__(kPfThreads, 1) gemm_wsp_kernel(const PfArgs p)
         if (tile >= wide_total) return;
         int row, col;
         pf_tile_of(tile, p.tiles_m, p.n_wide, p.band, row, col);
-        pf_tile<NW, Q4>(p, lds, row * kPfRows, col * 64 * NW);
+        pf_tile<NW, Q4, PARTS>(p, lds, row * kPfRows, col * 64 * NW, g_lo, g_hi);
     } else if constexpr (NN > 0) {
         const int tile = xcd * narrow_per_xcd + (slot - wide_per_xcd);
         if (tile >= narrow_total) return;
         int row, col;
         pf_tile_of(tile, p.tiles_m, p.n_narrow, p.band, row, col);
-        pf_tile<NN, Q4>(p, lds, row * kPfRows, p.n_wide * 64 * NW + col * 64 * NN);
+        pf_tile<NN, Q4, PARTS>(p, lds, row * kPfRows, p.n_wide * 64 * NW + col * 64 * NN, g_lo, g_hi);
     }
 }
 
@@ -616,40 +638,83 @@ int pf_band(int tiles_m) {
     return want < tiles_m ? want : tiles_m;
 }
 
-template <int NW, int NN, bool Q4>
-hipError_t launch_wsp_q(const PfArgs &p, hipStream_t stream) {
+template <int NW, int NN, bool Q4, bool PARTS>
+hipError_t launch_wsp_q(const PfArgs &p, hipStream_t stream, int slices) {
     constexpr size_t kStages = 2 * (size_t)kPfRows * 256, kOut = (size_t)kPfRows * (64 * NW + 8) * sizeof(uint16_t);
     constexpr size_t kLds = kStages > kOut ? kStages : kOut;
-    static_assert(kLds <= 160 * 1024, "tile does not fit LDS");
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wsp_kernel<NW, NN, Q4>),
+    static_assert(kLds <= 160 * 1024 && (size_t)kPfRows / 2 * (64 * NW + 4) * sizeof(float) <= kLds, "tile does not fit LDS");
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wsp_kernel<NW, NN, Q4, PARTS>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
     if (e != hipSuccess) return e;
     const int wide_per_xcd = (p.tiles_m * p.n_wide + 7) / 8, narrow_per_xcd = (p.tiles_m * p.n_narrow + 7) / 8;
     const int grid = 8 * (wide_per_xcd + narrow_per_xcd);
-    hipLaunchKernelGGL((gemm_wsp_kernel<NW, NN, Q4>), dim3(grid), dim3(kPfThreads), kLds, stream, p);
+    hipLaunchKernelGGL((gemm_wsp_kernel<NW, NN, Q4, PARTS>), dim3(grid, slices), dim3(kPfThreads), kLds, stream, p);
     return hipGetLastError();
 }
 
-template <int NW, int NN>
-hipError_t launch_wsp(const PfArgs &p, hipStream_t stream) {
-    return p.q4 ? launch_wsp_q<NW, NN, true>(p, stream) : launch_wsp_q<NW, NN, false>(p, stream);
+template <int NW, int NN, bool PARTS = false>
+hipError_t launch_wsp(const PfArgs &p, hipStream_t stream, int slices = 1) {
+    return p.q4 ? launch_wsp_q<NW, NN, true, PARTS>(p, stream, slices) : launch_wsp_q<NW, NN, false, PARTS>(p, stream, slices);
+}
+
+// y = bf16(the sum over the slices, in their order), or that added to aux and rounded again; four columns per thread
+__global__ void __launch_bounds__(256) gemm_wsp_sum_kernel(const float *__restrict__ parts, const uint16_t *__restrict__ aux, uint16_t *__restrict__ y,
+                                                           size_t mn, int slices) {
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (at >= mn) return;
+    floatx4 v = *reinterpret_cast<const floatx4 *>(parts + at);
+    for (int k = 1; k < slices; ++k) v += *reinterpret_cast<const floatx4 *>(parts + (size_t)k * mn + at);
+    uint2 o = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    if (aux) {
+        const uint2 a = *reinterpret_cast<const uint2 *>(aux + at);
+        auto add = [](uint32_t p, uint32_t q) {
+            return pack_bf16x2(bf16_bits_to_float(p & 0xFFFFu) + bf16_bits_to_float(q & 0xFFFFu), bf16_bits_to_float(p >> 16) + bf16_bits_to_float(q >> 16));
+        };
+        o = uint2{add(o.x, a.x), add(o.y, a.y)};
+    }
+    *reinterpret_cast<uint2 *>(y + at) = o;
 }
 
 }  // namespace
 
 bool gemm_prefill_ws_supported(int M, int K, int N) { return M > 0 && K > 0 && K % (2 * kGroup) == 0 && N > 0 && N % 64 == 0; }
 
-// Rounds of tiles over the chip, each K steps of a cost linear in the tile's width (fitted to 300 .. 2048 rows of twelve matrices,
-// within 20 %: K = 4096, N = 4096, 300 rows 45 estimated / 43 measured; N = 14336, 700 rows 83 / 79; K = 14336, N = 4096, 2048 rows 186 / 214 us)
-double gemm_prefill_ws_us(int M, int K, int N, bool q4) {
+// Rounds of tiles over the chip, each K steps of a cost linear in the tile's width and growing with the share of the CUs that are busy
+// (fitted to 300 .. 2048 rows of twelve matrices, within 20 %: estimated / measured us at K = 4096, N = 4096, 300 rows 43 / 43; N = 11008,
+// 300 rows 58 / 54; K = 14336, N = 4096, 1024 rows 174 / 189, 2048 rows 221 / 218)
+static double wsp_us(int K, long tiles, int ncb, bool q4) {
+    const long rounds = (tiles + 255) / 256;
+    return 2.5 + 1e-3 * K * rounds * (0.8 + 0.4 * tiles / (256.0 * rounds)) * (q4 ? 8.3 + 3.1 * ncb : 7.3 + 2.7 * ncb);
+}
+
+// Slices of K (1: none) in tiles of 256 columns for products of many rows that have too few of them for the chip, where the whole-K
+// launch takes narrow ones: they cost 1.4 to 2 times as much per column.  The fp32 sums are written and read once, at 5 TB/s.
+// (No more of them than x and y have bytes: a prompt pass has that much of its workspace free behind an FFN, and so it and the plain
+// product run the same slices.)  K = 14336, N = 4096, whole K / two slices: 1500 rows 202 / 166 us, 2048 rows 218 / 187 us, Q4NX 225 / 201.
+struct WspSlices {
+    int slices;
+    double us;
+};
+static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
     const Widths wd = pick_widths(tiles_m, N / 64, 256, false);
-    const long rounds = ((long)tiles_m * (wd.wide + wd.narrow) + 255) / 256;
-    return 2.5 + 1e-3 * K * rounds * (q4 ? 8.0 + 3.5 * wd.ncb : 6.8 + 3.0 * wd.ncb);
+    WspSlices best{1, wsp_us(K, (long)tiles_m * (wd.wide + wd.narrow), wd.ncb, q4)};
+    if (M < 512 || N % 256 || g_gemv_ws_tune.prefill_tile) return best;
+    const double whole = best.us;
+    for (int s = 2; s <= 8 && s <= K / (4 * kGroup) && 2L * s * N <= (long)K + N && (size_t)s * M * N * sizeof(float) <= scratch_bytes; ++s) {
+        const double us = wsp_us((K + s - 1) / s, (long)tiles_m * (N / 256) * s, 4, q4) + 3.0 + s * ((double)M * N * 8e-6 / 5.0);
+        if (us < 0.92 * whole && us < best.us) best = {s, us};
+    }
+    return best;
+}
+double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes) { return wsp_slices(M, K, N, q4, scratch_bytes).us; }
+size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most) {
+    const int s = wsp_slices(M, K, N, q4, most).slices;
+    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
 hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, hipStream_t stream, int epi,
-                                  const uint16_t *aux, const GemmRope *rope, bool q4) {
+                                  const uint16_t *aux, const GemmRope *rope, bool q4, float *scratch, size_t scratch_bytes) {
     if (!gemm_prefill_ws_supported(M, K, N)) return hipErrorInvalidValue;
     if ((epi != kEpiNone && !aux) || (epi == kEpiRope && (!rope || (rope->head_dim != 64 && rope->head_dim != 128) ||
                                                           rope->cols % rope->head_dim || N % rope->head_dim)))
@@ -667,6 +732,16 @@ hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y,
     p.tiles_m = (M + kPfRows - 1) / kPfRows;
     p.band = pf_band(p.tiles_m);
     const int U = N / 64;
+    const int slices = scratch && (epi == kEpiNone || epi == kEpiAddRounded) ? wsp_slices(M, K, N, q4, scratch_bytes).slices : 1;
+    if (slices > 1) {
+        p.parts = scratch;
+        p.n_wide = U / 4;
+        const hipError_t e = launch_wsp<4, 0, true>(p, stream, slices);
+        if (e != hipSuccess) return e;
+        const size_t mn = (size_t)M * N;
+        hipLaunchKernelGGL(gemm_wsp_sum_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, aux, y, mn, slices);
+        return hipGetLastError();
+    }
     Widths wd = pick_widths(p.tiles_m, U, 256, heads128);
     // tuning: one tile width only (1: 256 columns, 2: 192, 3: 128, 4: 64) where it divides N; 5: 256 mixed with 128
     // where the launch takes that mix (RoPE heads of 128, gate and up in one tile)

@@ -16,7 +16,8 @@
 //                every wave for itself
 //   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: w = s q + min in fp32, cut into two bf16
 //                (16 significant bits, the product of each with x is exact), two MFMAs per K-step
-//   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits
+//   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits, and a residual is
+//                added to the rounded product as its epilogue does
 //   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
 #include <algorithm>
 
@@ -334,6 +335,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         }
         if (p.residual) {
             const uint2 q = *reinterpret_cast<const uint2 *>(p.residual + at);
+            if constexpr (MODE >= kSmAwqRounded) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = bf16_bits_to_float(float_to_bf16_bits(v[i]));
+            }
             v[0] += bf16_bits_to_float(q.x & 0xFFFFu), v[1] += bf16_bits_to_float(q.x >> 16);
             v[2] += bf16_bits_to_float(q.y & 0xFFFFu), v[3] += bf16_bits_to_float(q.y >> 16);
         }

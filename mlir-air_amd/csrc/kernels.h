@@ -128,7 +128,7 @@ hipError_t launch_gemm_ws(const uint16_t *x, const void *w, uint16_t *y, const u
 double gemm_ws_us(int M, int K, int N, bool q4, bool residual);   // its time, an estimate for choosing between the kernels
 // The same for 17 rows and more in one launch (gemm_wsm.hip), both codecs: `rt` row tiles of 16 in each of `blocks` blocks of rows,
 // 64 nt columns a workgroup, `slices` of K (more than one: gemm_wsm_scratch_bytes of plain scratch and a launch that adds them up).
-// `rounded`: bf16-rounded weights, the bits of launch_gemm_prefill_ws.
+// `rounded`: bf16-rounded weights, the bits of launch_gemm_prefill_ws; a residual is added to the rounded product.
 struct WsmPlan {
     int rt, blocks, nt, slices;
     double us;   // the estimate by which it was chosen
@@ -140,11 +140,12 @@ hipError_t launch_gemm_wsm(const WsmPlan &p, const uint16_t *x, const void *w, u
                            bool q4, bool rounded, hipStream_t stream);
 // Prefill GEMM on stream-order weights (gemm_ws.hip): bf16-rounded weights dequantised in registers, x through LDS.
 bool gemm_prefill_ws_supported(int M, int K, int N);   // K % 256 == 0, N % 64 == 0
-double gemm_prefill_ws_us(int M, int K, int N, bool q4);   // its time without an epilogue, an estimate for choosing between the kernels
+double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes);   // its time without an epilogue, an estimate for choosing between the kernels
+size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most);   // plain scratch that makes it faster (0: none)
 // Epilogues as for launch_gemm_prefill (kEpi*); kEpiRope with heads of 128 needs N % 128 == 0.
 // `q4`: the matrix is in Q4NX order (launch_repack_ws_q4), W = bf16_rne(q s + min').
 hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, hipStream_t stream,
-                                  int epi = kEpiNone, const uint16_t *aux = nullptr, const GemmRope *rope = nullptr, bool q4 = false);
+                                  int epi = kEpiNone, const uint16_t *aux = nullptr, const GemmRope *rope = nullptr, bool q4 = false, float *scratch = nullptr, size_t scratch_bytes = 0);
 // h[M, H] = bf16(silu(bf16(x . W_gate)) * bf16(x . W_up)) in one launch (H % 64 == 0): bit for bit the gate launch followed
 // by the up launch with kEpiSiluGateMul.
 hipError_t launch_gemm_prefill_ws_swiglu(const uint16_t *x, const void *w_gate, const void *w_up, uint16_t *h, int M, int K, int H,

@@ -153,6 +153,17 @@ hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t 
     return launch_gemm_prefill_ws(normed, wqkv, qkv_out, M, E, (n_heads + 2 * n_kv) * head_dim, stream, kEpiRope, rope_lut, &rope, q4);
 }
 
+// y = bf16(bf16(x . W) + aux): the kernel for a few hundred rows where it is the faster one (same bits), else the tiled one, with slices of
+// K where they pay and fit `scratch`
+static hipError_t product_add(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, const uint16_t *aux, void *scratch, size_t scratch_bytes,
+                              hipStream_t stream, bool q4) {
+    if (gemm_wsm_supported(M, K, N) && !g_gemv_ws_tune.prefill_tile) {
+        const WsmPlan plan = plan_gemm_wsm(M, K, N, q4, true, 0);
+        if (plan.us < 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes)) return launch_gemm_wsm(plan, x, w, y, aux, nullptr, M, K, N, q4, true, stream);
+    }
+    return launch_gemm_prefill_ws(x, w, y, M, K, N, stream, kEpiAddRounded, aux, nullptr, q4, static_cast<float *>(scratch), scratch_bytes);
+}
+
 hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t *x_residual, const uint16_t *ffn_norm_w, float eps,
                                        const void *wo, const void *wg, const void *wu, const void *wd, uint16_t *y,
                                        uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace,
@@ -165,9 +176,11 @@ hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t 
     uint16_t *gate = reinterpret_cast<uint16_t *>(base);
     base += round256((size_t)M * H * sizeof(uint16_t));
     uint16_t *h = reinterpret_cast<uint16_t *>(base);
+    // scratch of the two products with a residual: what is not in use yet (gate, h) or any more (normed, gate)
+    const size_t own_h = round256((size_t)M * H * sizeof(uint16_t)), own_e = round256((size_t)M * E * sizeof(uint16_t));
     if (res1_out) res1 = res1_out;
     if (h_out) h = h_out;
-    hipError_t e = launch_gemm_prefill_ws(attn_out, wo, res1, M, E, E, stream, kEpiAddRounded, x_residual, nullptr, q4);
+    hipError_t e = product_add(attn_out, wo, res1, M, E, E, x_residual, gate, 2 * own_h, stream, q4);
     if (e != hipSuccess) return e;
     e = launch_rmsnorm_rows(res1, ffn_norm_w, normed, M, E, eps, stream);
     if (e != hipSuccess) return e;
@@ -179,7 +192,7 @@ hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t 
         e = launch_gemm_prefill_ws_swiglu(normed, wg, wu, h, M, E, H, stream, q4);
     }
     if (e != hipSuccess) return e;
-    return launch_gemm_prefill_ws(h, wd, y, M, H, E, stream, kEpiAddRounded, res1, nullptr, q4);
+    return product_add(h, wd, y, M, H, E, res1, normed, own_e + own_h, stream, q4);
 }
 
 }  // namespace w4a16

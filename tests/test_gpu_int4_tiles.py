@@ -7,7 +7,7 @@ import torch
 
 from helpers import assert_bf16_close, dense_f64, make_awq, make_x
 from oracle import awq as oawq
-from oracle.bf16 import bf16_bits_to_f32
+from oracle.bf16 import bf16_bits_to_f32, f32_to_bf16_bits
 from test_gpu_q4nx import make
 from test_gpu_stream_order import bits, dev
 
@@ -64,3 +64,35 @@ def test_int4_tiles(q4, M, K, N):
         ops.tune("gemm_splitk", 0)
         ops.tune("prefill_tile", 0)
 
+
+
+@pytest.mark.parametrize("q4", [False, True])
+def test_tiled_products_in_slices(q4):
+    """Many rows of a long K with few columns: the tiled kernel in slices of K, alone and behind an FFN's down projection (bit for bit)."""
+    from air_hip import _lib, ops
+    M, K, N = 1030, 14336, 1024
+    print("tiled slices", "q4nx" if q4 else "awq", M, K, N, flush=True)
+    lib = _lib.load_library()
+    x, aux = make_x((M, K), seed=3), make_x((M, N), seed=4)
+    if q4:
+        q, s, m = make(N, K, seed=5)
+        w = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+        exact = (q.astype(np.float32).reshape(N, K // 32, 32) * bf16_bits_to_f32(s)[:, :, None] + bf16_bits_to_f32(m)[:, :, None]).reshape(N, K).T
+        dense = bf16_bits_to_f32(f32_to_bf16_bits(np.ascontiguousarray(exact))).astype(np.float64)
+    else:
+        tri = make_awq(K, N, seed=5)
+        w, dense = ops.repack_stream(*map(dev, tri)), dense_f64(*tri, rounded=True)
+    need = lib.w4a16_q4nx_gemm_stream_best_scratch_bytes(M, K, N, 0) if q4 else lib.w4a16_gemm_stream_best_scratch_bytes(M, K, N)
+    assert need >= 2 * M * N * 4
+    y = (ops.q4nx_gemm_stream if q4 else ops.w4a16_gemm_stream)(dev(x), w)
+    want = (torch.from_numpy(bf16_bits_to_f32(x)).double().cuda() @ torch.from_numpy(dense).cuda()).cpu().numpy()
+    assert_bf16_close(bits(y), want, ulps=1.0, atol=2e-3, what="tiled slices")
+    if not q4:
+        H, E = K, N
+        mats = [ops.repack_stream(*map(dev, make_awq(E, n, seed=6 + i))) for i, n in enumerate((E, H, H))]
+        nw = dev(make_x((E,), seed=9))
+        out, res1, h = ops.prefill_o_ffn_stream(dev(make_x((M, E), seed=10)), dev(aux), nw, *mats, w, return_intermediates=True)
+        torch.cuda.synchronize()
+        prod = ops.w4a16_gemm_stream(h, w)
+        both = (prod.float() + res1.float()).bfloat16()
+        assert torch.equal(out.view(torch.int16), both.view(torch.int16))
