@@ -89,12 +89,38 @@ __device__ __forceinline__ void rope8(const uint16_t *src, const uint16_t *lut, 
     }
 }
 
+// Two lane halves (SWAP 32) or neighbouring rows of 16 lanes (SWAP 16): first + second of the values that each pair of lanes holds of `a`
+// in the one lane, of `b` in the other.
+template <int SWAP, bool MAX>
+__device__ __forceinline__ float swap_reduce(float a, float b) {
+    const auto r = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false)
+                              : __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned first = r[0], second = r[1];   // (a bit cast of an element itself reads the vector's first one)
+    const float x = __builtin_bit_cast(float, first), y = __builtin_bit_cast(float, second);
+    return MAX ? fmaxf(x, y) : x + y;
+}
+// Over the lanes with equal `sub` (one per position), every one of them receiving the result.
+template <int LPP, bool MAX>
+__device__ __forceinline__ float slots_reduce(float v) {
+    if constexpr (LPP == 8) {
+        const float o = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));   // row_ror:8
+        v = MAX ? fmaxf(v, o) : v + o;
+    }
+    v = swap_reduce<16, MAX>(v, v);
+    return swap_reduce<32, MAX>(v, v);
+}
+
+// What bounds it: latencies in a row, at 64 positions a workgroup: the fresh qkv and the cache (requested together: the new token's K and V
+// are taken from registers, not read back), the scores' sums, one maximum per wave and head, and the sums over positions.  Those halve
+// what a lane holds with every exchange (v_permlane*_swap: half the values go each way), 28 exchanges for a head group of 4, where full
+// butterflies of (m, l, acc) took 120 shuffles through LDS.   32 heads of 64 over 8, 1000 positions: 7.3 -> 4.9 us.
 template <int HD, int G>
 __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     constexpr int LPP = HD / 8;        // lanes per position
     constexpr int PPW = 64 / LPP;      // positions per wave and load
-    constexpr int STATE = 2 + HD;      // m, l, acc[HD] per head
-    __shared__ float sh[4 * G * STATE];
+    constexpr int STATE = 4 + HD;      // m, l, -, -, acc[HD] per head
+    constexpr int UN = 2, STEP = UN * 4 * PPW;   // positions per lane and trip, per workgroup and trip
+    __shared__ __attribute__((aligned(16))) float sh[4 * G * STATE];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPP, slot = lane / LPP;
@@ -104,22 +130,35 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     const int t1 = min(seq_len, t0 + p.chunk);
     const int nq = p.n_heads * HD, nkv = p.n_kv * HD;
 
-    uint16_t *kc = p.k_cache + (size_t)kvh * p.max_seq * HD;
-    uint16_t *vc = p.v_cache + (size_t)kvh * p.max_seq * HD;
+    uint16_t *kc = p.k_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
+    uint16_t *vc = p.v_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
+
+    u32x4 kraw[UN], vraw[UN];
+    auto request = [&](int tb) {
+#pragma unroll
+        for (int i = 0; i < UN; ++i) {
+            const int t = tb + i * 4 * PPW;
+            const size_t at = (size_t)min(t, t1 - 1) * HD;   // in range (t1 >= 1, also where the chunk is empty); a clamped slot's result is discarded
+            kraw[i] = *reinterpret_cast<const u32x4 *>(kc + at);
+            vraw[i] = *reinterpret_cast<const u32x4 *>(vc + at);
+        }
+    };
+    int tb = t0 + wave * PPW + slot;
+    request(tb);
 
     // the chunk that owns `pos` appends the new token's K (rotated) and V
-    if (t0 <= p.pos && p.pos < t1) {
-        if (threadIdx.x < LPP) {
-            float kr[8];
-            rope8<HD>(p.qkv + nq + kvh * HD, p.lut, 8 * sub, kr);
-            u32x4 o;
+    u32x4 knew, vnew;
+    const bool owner = t0 <= p.pos && p.pos < t1;
+    if (owner) {
+        float kr[8];
+        rope8<HD>(p.qkv + nq + kvh * HD, p.lut, 8 * sub, kr);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(kr[2 * j], kr[2 * j + 1]);
-            *reinterpret_cast<u32x4 *>(kc + (size_t)p.pos * HD + 8 * sub) = o;
-            *reinterpret_cast<u32x4 *>(vc + (size_t)p.pos * HD + 8 * sub) =
-                *reinterpret_cast<const u32x4 *>(p.qkv + nq + nkv + kvh * HD + 8 * sub);
+        for (int j = 0; j < 4; ++j) knew[j] = pack_bf16x2(kr[2 * j], kr[2 * j + 1]);
+        vnew = *reinterpret_cast<const u32x4 *>(p.qkv + nq + nkv + kvh * HD + 8 * sub);
+        if (threadIdx.x < LPP) {
+            *reinterpret_cast<u32x4 *>(kc + (size_t)p.pos * HD) = knew;
+            *reinterpret_cast<u32x4 *>(vc + (size_t)p.pos * HD) = vnew;
         }
-        __syncthreads();
     }
 
     // rotated, bf16-rounded query slices of the G heads, pre-scaled for exp2
@@ -131,74 +170,75 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
         for (int j = 0; j < 8; ++j) q[h][j] *= p.scale * kLog2e;
     }
 
-    float m[G], l[G], acc[G][8];
+    float m[G], l[G], acc[G * 8];   // m of the wave; l and acc of the lane's positions
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-        m[h] = kNegBig;
-        l[h] = 0.f;
+    for (int h = 0; h < G; ++h) m[h] = kNegBig, l[h] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[h][j] = 0.f;
-    }
+    for (int n = 0; n < G * 8; ++n) acc[n] = 0.f;
 
-    // UN positions per lane are requested together, so that a chunk costs one or two memory
-    // round trips instead of one per position
-    constexpr int UN = G == 8 ? 2 : 4;
-    for (int tb = t0 + wave * PPW + slot; tb < t1; tb += UN * 4 * PPW) {
-        u32x4 kraw[UN], vraw[UN];
+    for (int base = t0; base < t1; base += STEP, tb += STEP) {   // (the same number of trips for every lane)
+        float s[UN][G], v[UN][8];
+        bool live[UN];
 #pragma unroll
         for (int i = 0; i < UN; ++i) {
             const int t = tb + i * 4 * PPW;
-            const int tc = t < t1 ? t : t0;   // in range; the result of a clamped slot is discarded
-            kraw[i] = *reinterpret_cast<const u32x4 *>(kc + (size_t)tc * HD + 8 * sub);
-            vraw[i] = *reinterpret_cast<const u32x4 *>(vc + (size_t)tc * HD + 8 * sub);
-        }
-#pragma unroll
-        for (int i = 0; i < UN; ++i) {
-            if (tb + i * 4 * PPW >= t1) break;   // uniform within a lane group
-            float k[8], v[8];
-            unpack8(kraw[i], k);
-            unpack8(vraw[i], v);
+            live[i] = t < t1;
+            float k[8];
+            const bool fresh = owner && t == p.pos;
+            unpack8(fresh ? knew : kraw[i], k);
+            unpack8(fresh ? vnew : vraw[i], v[i]);
 #pragma unroll
             for (int h = 0; h < G; ++h) {
-                float s = 0.f;
+                float d = 0.f;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) s = fmaf(q[h][j], k[j], s);
-                s = group_sum<LPP>(s);
-                const float mn = fmaxf(m[h], s);
-                const float corr = exp2_nonpos(m[h] - mn);
-                const float pr = exp2_nonpos(s - mn);
-                m[h] = mn;
-                l[h] = l[h] * corr + pr;
+                for (int j = 0; j < 8; ++j) d = fmaf(q[h][j], k[j], d);
+                s[i][h] = group_sum<LPP>(d);
+            }
+        }
+        if (base + STEP < t1) request(tb + STEP);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(pr, v[j], acc[h][j] * corr);
+        for (int h = 0; h < G; ++h) {
+            float mn = m[h];
+#pragma unroll
+            for (int i = 0; i < UN; ++i) mn = fmaxf(mn, live[i] ? s[i][h] : kNegBig);
+            mn = slots_reduce<LPP, true>(mn);
+            const float corr = exp2_nonpos(m[h] - mn);
+            m[h] = mn;
+            l[h] *= corr;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[8 * h + j] *= corr;
+#pragma unroll
+            for (int i = 0; i < UN; ++i) {
+                const float pr = live[i] ? exp2_nonpos(s[i][h] - mn) : 0.f;
+                l[h] += pr;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[8 * h + j] = fmaf(pr, live[i] ? v[i][j] : 0.f, acc[8 * h + j]);
             }
         }
     }
 
-    // merge the lane groups of the wave (lanes with equal `sub`)
+    // sums over the wave's positions: lanes 32 .. 63 go on with the upper half of the values, odd rows of lanes with the upper half of theirs
+    constexpr int NV = G * 8, QV = NV / 4;
 #pragma unroll
-    for (int off = LPP; off < 64; off <<= 1) {
+    for (int n = 0; n < NV / 2; ++n) acc[n] = swap_reduce<32, false>(acc[n], acc[n + NV / 2]);
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
-            const float m2 = __shfl_xor(m[h], off), l2 = __shfl_xor(l[h], off);
-            const float mn = fmaxf(m[h], m2);
-            const float c1 = exp2_nonpos(m[h] - mn), c2 = exp2_nonpos(m2 - mn);
-            m[h] = mn;
-            l[h] = l[h] * c1 + l2 * c2;
+    for (int n = 0; n < QV; ++n) acc[n] = swap_reduce<16, false>(acc[n], acc[n + QV]);
+    if constexpr (LPP == 8) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[h][j] = acc[h][j] * c1 + __shfl_xor(acc[h][j], off) * c2;
-        }
+        for (int n = 0; n < QV; ++n) acc[n] = dpp_add<0x128>(acc[n]);
     }
-    if (slot == 0) {
+#pragma unroll
+    for (int h = 0; h < G; ++h) l[h] = slots_reduce<LPP, false>(l[h]);
+    if (LPP == 16 || !(lane & 8)) {
+        const int first = (lane & 32 ? NV / 2 : 0) + (lane & 16 ? QV : 0);
+#pragma unroll
+        for (int n = 0; n < QV; ++n) sh[(wave * G + (first + n) / 8) * STATE + 4 + 8 * sub + (first + n) % 8] = acc[n];
+    }
+    if (lane == 0) {
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-            float *dst = sh + (wave * G + h) * STATE;
-            if (sub == 0) {
-                dst[0] = m[h];
-                dst[1] = l[h];
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) dst[2 + 8 * sub + j] = acc[h][j];
+            sh[(wave * G + h) * STATE] = m[h];
+            sh[(wave * G + h) * STATE + 1] = l[h];
         }
     }
     __syncthreads();
@@ -215,7 +255,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
             const float *src = sh + (w * G + h) * STATE;
             const float c = exp2f(src[0] - mn);
             ls += src[1] * c;
-            as += src[2 + e] * c;
+            as += src[4 + e] * c;
         }
         const int head = kvh * G + h;
         if (p.nsplit == 1) {
