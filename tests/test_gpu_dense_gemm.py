@@ -129,3 +129,26 @@ def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows):
         got = act[place[at]]
         close(got[:, :ff], a, True, ("gate / up", i))
         close(out[at], got.double() @ w2[i].double().t(), True, ("down", i))
+
+
+@pytest.mark.parametrize("entries,experts", [(1, 1), (1000, 7), (16384, 64), (16385, 1024), (50000, 3)])
+def test_expert_plan(dense, entries, experts):
+    print("plan", entries, experts, flush=True)
+    from air_hip import _lib
+    lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
+    ids = torch.randint(0, experts, (entries,), dtype=torch.int32, device="cuda", generator=torch.Generator(device="cuda").manual_seed(entries))
+    for bm in (32, 384):
+        most = lib.dlm_moe_max_tiles(entries, experts, bm)
+        order, tiles = torch.full((entries,), -1, dtype=torch.int32, device="cuda"), torch.empty((most + 1, 4), dtype=torch.int32, device="cuda")
+        _lib.check_dense(lib.dlm_moe_plan(ids.data_ptr(), entries, experts, bm, order.data_ptr(), tiles.data_ptr(), stream))
+        n = int(tiles[most, 0])
+        assert torch.equal(order.sort()[0], torch.arange(entries, dtype=torch.int32, device="cuda"))
+        assert torch.equal(ids[order.long()], ids.sort()[0])
+        rows = tiles[:n].tolist()
+        assert n <= most and all(0 < r[2] <= bm for r in rows)
+        at = 0
+        for e, first, height, _ in rows:   # the tiles follow each other and stay within their expert
+            assert first == at
+            at += height
+            assert bool((ids[order[first:at].long()] == e).all()) if n <= 200 else True
+        assert at == entries
