@@ -47,3 +47,11 @@ def test_native_decode_steps(monkeypatch, codec, n_layers, n_heads, n_kv, hd, hi
     logits2, best2 = decode.decode_token(int(first), layers, embed, final, head, cfg, copies, start, lut, return_argmax=True)
     assert torch.equal(got, want) and torch.equal(best, best2) and torch.equal(logits, logits2)
     assert all(torch.equal(a, b) and torch.equal(c, d) for (a, c), (b, d) in zip(caches, copies))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,positions", [(8, 2, 64, 3000, [2048, 2976, 2999]), (4, 4, 64, 2200, [2100]), (16, 2, 64, 2600, [64, 2500])])
+def test_decode_attention_past_a_trip(n_heads, n_kv, hd, max_seq, positions):
+    """More than 32 chunks of 64: several trips of a workgroup, and workgroups without a position."""
+    import test_gpu_decode
+    from air_hip import ops
+    test_gpu_decode.test_decode_attention(ops, n_heads, n_kv, hd, max_seq, positions)
