@@ -159,6 +159,7 @@ def decode_token(token_id, layers, embed_table, final_norm, lm_head, config, kv_
     fp32 [vocab], like the reference, and with return_argmax also the greedy token as a device
     int32 tensor [1] (no host synchronisation here)."""
     x = embed_table[token_id].contiguous()
+    layers, kv_cache = list(layers), list(kv_cache)   # (walked twice where the native steps do not take them)
     best = torch.empty((1,), dtype=torch.int32, device=x.device)
     logits = ops.decode_run(x, layers, embed_table, final_norm, lm_head, rope_lut, config, kv_cache, current_pos, 1, best)
     if logits is not None:

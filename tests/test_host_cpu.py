@@ -367,3 +367,18 @@ def test_fake_quantize_matches_the_oracle_loop():
     assert got[0].shape == (12, 256) and got[1].shape == (4, 12) and got[2].dtype == np.uint8
     with pytest.raises(ValueError):
         awq.fake_quantize_awq_int4(w[:, :100], 128)
+
+
+def test_decode_token_takes_its_layers_once(monkeypatch):
+    """Layers and caches that can be walked only once: looking whether the native steps take them leaves them to the steps op by op."""
+    import types
+
+    import torch
+    from air_hip import decode, ops
+
+    ran = []
+    monkeypatch.setattr(decode, "run_decode_block", lambda x, layer, *a, **k: (ran.append(layer), (x, None))[1])
+    monkeypatch.setattr(ops, "lm_head", lambda x, head, **k: (x, torch.zeros(1)))
+    layers = [types.SimpleNamespace(stream=None, name=i) for i in range(3)]
+    decode.decode_token(0, iter(layers), torch.zeros((2, 8)), None, None, types.SimpleNamespace(rms_eps=1e-5), iter([(0, 0)] * 3), 0, None)
+    assert ran == layers
