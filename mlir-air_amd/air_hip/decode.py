@@ -179,6 +179,7 @@ def decode_greedy(token, n_tokens, layers, embed_table, final_norm, lm_head, con
     afterwards (the reference stops at it, so later entries are to be dropped)."""
     out = torch.empty((n_tokens,), dtype=torch.int32, device=embed_table.device)
     tok = token.to(torch.int32).reshape(1)
+    layers, kv_cache = list(layers), list(kv_cache)   # (walked twice where the native steps do not take them)
     # all launches from one native call (eager, a step of 16 small layers takes 770 us of Python for 570 us of kernels)
     if n_tokens > 0 and ops.decode_run(embed_table.index_select(0, tok).reshape(-1), layers, embed_table, final_norm, lm_head, rope_lut, config,
                                        kv_cache, start_pos, n_tokens, out) is not None:

@@ -382,3 +382,5 @@ def test_decode_token_takes_its_layers_once(monkeypatch):
     layers = [types.SimpleNamespace(stream=None, name=i) for i in range(3)]
     decode.decode_token(0, iter(layers), torch.zeros((2, 8)), None, None, types.SimpleNamespace(rms_eps=1e-5), iter([(0, 0)] * 3), 0, None)
     assert ran == layers
+    decode.decode_greedy(torch.zeros(1), 1, iter(layers), torch.zeros((2, 8)), None, None, types.SimpleNamespace(rms_eps=1e-5), iter([(0, 0)] * 3), 0, None)
+    assert ran == layers + layers
