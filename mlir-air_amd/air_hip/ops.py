@@ -751,7 +751,7 @@ def decode_run(first_x, layers, embed_table, final_norm, lm_head_weight, rope_lu
     lib = _lib.load_library()
     pairs = list(zip(layers, kv_cache))
     names = ("wqkv", "wo", "w_gate", "w_up", "w_down")
-    if not pairs or any(l.stream is None for l, _ in pairs) or not (isinstance(start_pos, int) and n_tokens > 0 and start_pos >= 0):
+    if final_norm is None or not pairs or any(l.stream is None for l, _ in pairs) or not (isinstance(start_pos, int) and n_tokens > 0 and start_pos >= 0):
         return None
     first, (k0, _) = pairs[0]
     if k0.dim() != 3 or embed_table.dim() != 2 or lm_head_weight.dim() != 2 or rope_lut.dim() != 2:

@@ -384,3 +384,21 @@ def test_decode_token_takes_its_layers_once(monkeypatch):
     assert ran == layers
     decode.decode_greedy(torch.zeros(1), 1, iter(layers), torch.zeros((2, 8)), None, None, types.SimpleNamespace(rms_eps=1e-5), iter([(0, 0)] * 3), 0, None)
     assert ran == layers + layers
+
+
+def test_decode_run_leaves_a_model_without_a_final_norm_to_the_ops():
+    import types
+
+    import torch
+    from air_hip import ops
+
+    buf = types.SimpleNamespace(is_cuda=True, is_contiguous=lambda: True, data_ptr=lambda: 256)
+    matrix = lambda K, N: types.SimpleNamespace(order="awq", K=K, N=N, buf=buf)
+    E, H, V = 256, 512, 8
+    layer = types.SimpleNamespace(codec="awq", attn_norm=torch.ones(E), ffn_norm=torch.ones(E),
+                                  stream={"wqkv": matrix(E, 3 * E), "wo": matrix(E, E), "w_gate": matrix(E, H), "w_up": matrix(E, H), "w_down": matrix(H, E)})
+    cache = (torch.zeros((4, 16, 64)), torch.zeros((4, 16, 64)))
+    args = (torch.zeros(E), [layer], torch.zeros((V, E)))
+    rest = (torch.zeros((V, E)), torch.zeros((16, 64)), types.SimpleNamespace(n_heads=4, rms_eps=1e-5), [cache], 0, 1, torch.zeros(1, dtype=torch.int32))
+    assert ops.decode_run(*args, torch.ones(E), *rest) is None   # (not on a GPU)
+    assert ops.decode_run(*args, None, *rest) is None
