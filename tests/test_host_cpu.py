@@ -398,7 +398,9 @@ def test_decode_run_leaves_a_model_without_a_final_norm_to_the_ops():
     layer = types.SimpleNamespace(codec="awq", attn_norm=torch.ones(E), ffn_norm=torch.ones(E),
                                   stream={"wqkv": matrix(E, 3 * E), "wo": matrix(E, E), "w_gate": matrix(E, H), "w_up": matrix(E, H), "w_down": matrix(H, E)})
     cache = (torch.zeros((4, 16, 64)), torch.zeros((4, 16, 64)))
-    args = (torch.zeros(E), [layer], torch.zeros((V, E)))
+    on_gpu = lambda *shape: types.SimpleNamespace(shape=shape, is_cuda=True, dtype=torch.bfloat16, is_contiguous=lambda: True, data_ptr=lambda: 256,
+                                                  dim=lambda: len(shape), numel=lambda: shape[-1])
+    args = (on_gpu(E), [layer], on_gpu(V, E))
     rest = (torch.zeros((V, E)), torch.zeros((16, 64)), types.SimpleNamespace(n_heads=4, rms_eps=1e-5), [cache], 0, 1, torch.zeros(1, dtype=torch.int32))
-    assert ops.decode_run(*args, torch.ones(E), *rest) is None   # (not on a GPU)
+    assert ops.decode_run(*args, torch.ones(E), *rest) is None   # (a norm that is not on the GPU)
     assert ops.decode_run(*args, None, *rest) is None
