@@ -550,7 +550,7 @@ int w4a16_q4nx_repack_stream(const int32_t *qweight, const uint16_t *scales, con
 int w4a16_q4nx_gemv_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int K, int N,
                                 void *stream);
 /* y[M, N] = bf16(x[M, K] . W + residual [M, N]): the GEMV at M = 1, launches of 16 rows or of row and column tiles above
- * (weights s q + min' to 16 significant bits or more, fp32 sums, one rounding).  From M = 65 on, without a residual and with K % 256 == 0,
+ * (exact weights s q + min', fp32 sums, one rounding).  From M = 65 on, without a residual and with K % 256 == 0,
  * N % 64 == 0, the tiled MFMA kernels of w4a16_gemm_stream_bf16 run on the Q4NX order: they dequantise each K-step of a
  * cell with its own (scale, min') word to W = bf16_rne(s q + min'), the dense dequant's values (q4nx_dequant_bf16,
  * bit for bit), and multiply those, which is what the reference's prompt pass of these models computes with its

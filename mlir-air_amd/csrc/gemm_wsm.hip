@@ -14,8 +14,9 @@
 //   AWQ        : operands are (128 + q) exactly, flushed per group: y += s (sum (128 + q) x - (128 + z) sum x); the sums of x of the
 //                next step are taken by one wave per row tile with an MFMA against ones and handed round through LDS, with R = 2 by
 //                every wave for itself
-//   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: w = s q + min in fp32, cut into two bf16
-//                (16 significant bits, the product of each with x is exact), two MFMAs per K-step
+//   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: s q, which has 12 significant bits, is cut
+//                into two bf16, and the minimum is an operand of its own: three MFMAs per K-step with every product exact, as s sum q x +
+//                min sum x has them.  (s q + min in two operands keeps 16 bits of it, which loses minima small against the scale.)
 //   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits, and a residual is
 //                added to the rounded product as its epilogue does
 //   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
@@ -133,9 +134,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         for (int v = 0; v < 4; ++v) b[v] = ((w >> (4 * v)) & nib_mask) | magic;
         return __builtin_bit_cast(bf16x8, b);
     };
-    // eight weights s q + low as the sum of two bf16
-    auto two_operands = [&](uint32_t w, uint32_t md, bf16x8 &high, bf16x8 &rest) {
-        const float s = __builtin_bit_cast(float, md << 16), low = __builtin_bit_cast(float, md & 0xFFFF0000u);
+    // eight products s q as the sum of two bf16: 8 + 4 bits, exact (the cuts do not round, so nothing carries into the first one)
+    auto two_operands = [&](uint32_t w, float s, bf16x8 &high, bf16x8 &rest) {
         uint32_t e = w & 0x0F0F0F0Fu, o = (w >> 4) & 0x0F0F0F0Fu;   // rows 0, 4, 1, 5 and 2, 6, 3, 7
         asm volatile("" : "+v"(e), "+v"(o));
         const uint32_t src[4] = {e, o, e, o};
@@ -143,10 +143,11 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint32_t n = src[v] >> (v < 2 ? 0 : 8);
-            const float w0 = fmaf(static_cast<float>(n & 0xFFu), s, low), w1 = fmaf(static_cast<float>((n >> 16) & 0xFFu), s, low);
-            const uint32_t p2 = pack_bf16x2(w0, w1);
-            h[v] = p2;
-            l[v] = pack_bf16x2(w0 - __builtin_bit_cast(float, p2 << 16), w1 - __builtin_bit_cast(float, p2 & 0xFFFF0000u));
+            const float w0 = static_cast<float>(n & 0xFFu) * s, w1 = static_cast<float>((n >> 16) & 0xFFu) * s;
+            const uint32_t b0 = __builtin_bit_cast(uint32_t, w0), b1 = __builtin_bit_cast(uint32_t, w1);
+            const float r0 = w0 - __builtin_bit_cast(float, b0 & 0xFFFF0000u), r1 = w1 - __builtin_bit_cast(float, b1 & 0xFFFF0000u);
+            h[v] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+            l[v] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, r1), __builtin_bit_cast(uint32_t, r0), 0x07060302u);
         }
         high = __builtin_bit_cast(bf16x8, h);
         rest = __builtin_bit_cast(bf16x8, l);
@@ -230,11 +231,15 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
                     for (int rt = 0; rt < RT; ++rt) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, acc[rt][c], 0, 0, 0);
                 } else if constexpr (MODE == kSmQ4) {
                     bf16x8 high, rest;
-                    two_operands(cell[c][t], word[c][t], high, rest);
+                    two_operands(cell[c][t], __builtin_bit_cast(float, word[c][t] << 16), high, rest);
+                    const uint32_t min2 = __builtin_amdgcn_perm(word[c][t], word[c][t], 0x03020302u);
+                    const bf16x8 low8 = __builtin_bit_cast(bf16x8, u32x4{min2, min2, min2, min2});
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], high, Y[rt][c], 0, 0, 0);
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], rest, Y[rt][c], 0, 0, 0);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], low8, Y[rt][c], 0, 0, 0);
                 } else {
                     if (Q4) decode_md_q4(word[c][Q4 ? t : 0], s[c], low[c]);
                     else if (t == 0) decode_md(word[c][0], s[c], low[c]);
@@ -399,14 +404,14 @@ hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t str
 }
 
 // The time of a launch, fitted to 10800 timings (13 matrices from 512 x 1024 to 13056 x 5744, 17 .. 3500 rows, every tile, 1 .. 16
-// slices; rms error 7 % exact, 10 % rounded; the plan it picks takes 1 % more than the best of them on average, 24 % at worst):
+// slices; rms error 7 % exact, 10 % rounded; the plan it picks takes 1 % more than the best of them on average, 24 % at worst; Q4NX: a3 and b3 raised by what the third product took at 14 of them):
 // microseconds of start, of a workgroup, and of a step alone on the chip (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with
 // every CU busy; a step of four groups costs 1 + four of one of two.
 struct SmCost {
     double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, tb_s;
 };
 constexpr SmCost kSmCost[3] = {{2.6, 2.1, 0.06, 0.084, 0.075, 0.076, 0.16, 0.017, 0, 0, 0.69, 2.0, 5.9},
-                               {3.0, 1.6, 0, 0.042, 0.535, 0.100, 0.11, 0.021, 0.028, 0, 0.88, 1.9, 5.2},
+                               {3.0, 1.6, 0, 0.042, 0.535, 0.123, 0.11, 0.021, 0.028, 0.023, 0.88, 1.9, 5.2},
                                {1.8, 2.5, 0, 0.030, 0.150, 0.035, 0.07, 0.018, 0.09, 0.03, 0, 0, 1}};
 
 double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {

@@ -65,6 +65,42 @@ def test_int4_tiles(q4, M, K, N):
         ops.tune("prefill_tile", 0)
 
 
+@pytest.mark.parametrize("M,K,N", [(17, 128, 48), (40, 640, 272), (64, 2048, 528), (100, 384, 1040)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_q4nx_minima_of_any_size(residual, M, K, N):
+    """Row m adds 32 rows of one scale block and takes away 32 of the next; a column has one q and one scale everywhere, so what is left is
+    32 times the difference of two minima, from 2^-12 to 2^4 scales.  Exact products in fp32: three matrix instructions a block, each at most two
+    roundings of 2^-24 of the sum of magnitudes, then a bf16 rounding.  Weights kept in 16 bits miss it by up to 2^-17 of that sum."""
+    from air_hip import _lib, ops
+    print("q4nx minima", residual, M, K, N, flush=True)
+    rng = np.random.default_rng(M + K + N)
+    B = K // 32
+    q = np.repeat(rng.integers(1, 16, (N, 1), dtype=np.uint8), K, axis=1)
+    s = np.repeat(f32_to_bf16_bits(rng.uniform(0.5, 2.0, (N, 1)).astype(np.float32)), B, axis=1)
+    m = f32_to_bf16_bits((bf16_bits_to_f32(s) * 2.0 ** rng.uniform(-12, 4, (N, B)) * rng.choice([-1.0, 1.0], (N, B))).astype(np.float32))
+    x = np.zeros((M, K), np.float32)
+    for i in range(M):
+        x[i, 32 * (i % B):32 * (i % B) + 32], x[i, 32 * ((i + 1) % B):32 * ((i + 1) % B) + 32] = 1.0, -1.0
+    w = (q.astype(np.float64).reshape(N, B, 32) * bf16_bits_to_f32(s).astype(np.float64)[:, :, None] + bf16_bits_to_f32(m).astype(np.float64)[:, :, None]).reshape(N, K).T
+    parts = (q.astype(np.float64).reshape(N, B, 32) * bf16_bits_to_f32(s).astype(np.float64)[:, :, None]
+             + np.abs(bf16_bits_to_f32(m)).astype(np.float64)[:, :, None]).reshape(N, K).T
+    res = make_x((M, N), seed=N) if residual else None
+    want = x.astype(np.float64) @ w + (bf16_bits_to_f32(res) if residual else 0.0)
+    sums = np.abs(x).astype(np.float64) @ parts
+    stream = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(np.ascontiguousarray(s.T)), dev(np.ascontiguousarray(m.T)))
+    lib = _lib.load_library()
+    xd, y = dev(f32_to_bf16_bits(x)), torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    rd = dev(res) if residual else None
+    ops.tune("gemm_splitk", 1)
+    try:
+        _lib.check(lib.w4a16_q4nx_gemm_stream_bf16(xd.data_ptr(), stream.buf.data_ptr(), rd.data_ptr() if residual else None, y.data_ptr(), M, K, N,
+                                                   torch.cuda.current_stream().cuda_stream))
+    finally:
+        ops.tune("gemm_splitk", 0)
+    got = bf16_bits_to_f32(bits(y)).astype(np.float64)
+    bad = np.abs(got - want) > 2.0 ** -8 * np.abs(want) + 2.0 ** -24 * 12 * sums
+    assert not bad.any(), (int(bad.sum()), bad.size, float((np.abs(got - want) / sums).max()))
+
 
 @pytest.mark.parametrize("q4", [False, True])
 def test_tiled_products_in_slices(q4):
