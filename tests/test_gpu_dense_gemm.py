@@ -67,6 +67,40 @@ def test_sliced_products(dense, M, N, K, slices):
             assert (out[:, width:] == 7.0).all(), "columns past the width were written"
 
 
+@pytest.mark.parametrize("M,N,K,slices", [(64, 4096, 64, 1), (260, 2048, 128, 2), (1040, 512, 64, 1)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_silu_behind_a_product_is_an_fp32_one(dense, gated, M, N, K, slices):
+    """Two products of bf16 numbers make the argument, exact in fp32 (multiples of 2^-16), from -80 to -47.  silu in fp32 is off by one unit of
+    2^-24 on average at most, which changes one bf16 rounding (2^-8 apart at least) in 2^16; an exponent rounded after log2 e is off by
+    2^-19 ln 2 on average."""
+    from air_hip import _lib
+    print("silu", gated, M, N, K, slices, flush=True)
+    lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
+    a, w = torch.zeros((M, K), device="cuda").bfloat16(), torch.zeros((N, K), device="cuda").bfloat16()
+    g = torch.Generator(device="cuda").manual_seed(M)
+    uniform = lambda n, lo, hi: (lo + (hi - lo) * torch.rand(n, device="cuda", generator=g)).bfloat16()
+    a[:, 0], a[:, 1], a[:, 2] = -8.0, uniform(M, 0.5, 1.0), 1.0
+    width = N // 2 if gated else N
+    z = torch.stack([uniform(width, 6.0, 10.0), uniform(width, 0.5, 1.0)], 1)
+    if gated:   # 16 gate rows, 16 rows that give 1
+        v = w.view(N // 32, 2, 16, K)
+        v[:, 0, :, :2], v[:, 1, :, 2] = z.view(-1, 16, 2), 1.0
+    else:
+        w[:, :2] = z
+    out, parts = torch.empty((M, width), device="cuda", dtype=torch.bfloat16), torch.empty((slices, M, N), device="cuda")
+    args = _lib.GemmArgs(a=a.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), lda=K, ldo=width, M=M, N=N, K=K, silu_begin=0, silu_end=0 if gated else N,
+                         epilogue=dense.OUT_SWIGLU if gated else dense.OUT_ELEM)
+    _lib.check_dense(lib.dlm_gemm_sliced(0, ctypes.byref(args), slices, parts.data_ptr(), stream))
+    want = torch.nn.functional.silu(a[:, :2].double() @ z.double().t())
+    down = want.float().bfloat16().double()   # (fp32 first: a double rounding shows as rarely)
+    wrong = int((out.double() != down).sum())
+    assert wrong <= out.numel() * 2.0 ** -16 + 4 * (out.numel() * 2.0 ** -16) ** 0.5, (wrong, out.numel())
+    if not gated:
+        a[:3, 0] = torch.tensor([float("inf"), float("-inf"), float("nan")])   # inf, -inf / inf, NaN
+        _lib.check_dense(lib.dlm_gemm_sliced(0, ctypes.byref(args), slices, parts.data_ptr(), stream))
+        assert bool((out[0] == float("inf")).all()) and bool(out[1:3].isnan().all()) and bool(out[3:].isfinite().all())
+
+
 @pytest.mark.parametrize("M,K", [(3, 64), (300, 2048)])
 def test_parts_meet_in_the_row_kernels(dense, M, K):
     a, w = rand(1, M, 512).bfloat16(), (rand(2, K, 512) * 512 ** -0.5).bfloat16()
