@@ -99,7 +99,7 @@ typedef struct {
     void *out;
     int64_t lda, ldo, w_stride;
     const int32_t *tiles, *order;
-    int32_t M, N, K, epilogue, n_tiles, gather, tile_rows;   /* tile_rows: dlm_gemm_tile_rows, or 32, 128, 256, grouped bf16 also 384 */
+    int32_t M, N, K, epilogue, n_tiles, gather, tile_rows;   /* tile_rows: dlm_gemm_tile_rows, or 32, 128, 256, grouped bf16 also 384; grouped: the plan's */
     int32_t silu_begin, silu_end;
 } dlm_gemm_args;
 /* Rows of A per tile for `rows` rows (experts: the mean number) with each of `matrices` matrices of N rows. */

@@ -471,16 +471,20 @@ __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const 
 // A K-step is two halves of 8 MT products of 16 cycles; each half's operands are read during the one before it.  One wait and barrier
 // stand between the halves: all of the next K-step has landed, everybody has read all of this one, and the copies of a K-step two or three
 // on (buffers: W three, A three up to 256 rows, else two; more of them for few rows were no faster) go out behind the products after it.
-constexpr int kExpertCols = 128, kExpertRows = 384;
+// Few rows (plans of 128 to a tile): two workgroups to a CU, whose starts and stores then stand beside each other's products; 80 KiB of LDS and
+// 192 registers each.  64 experts of 2 x 1024 x 2048 and 1024 x 2048, one / two to a CU, gate and up, then down: 16 tokens of 8 92 / 84 + 50 / 44 us,
+// 128 tokens 100 / 97 + 57 / 53, 512 tokens 108 / 107 + 69 / 62 (32- and 128-row tiles before: 96 + 42, 118 + 54, 137 + 64); 768 tokens, 96 rows an
+// expert on average and up to 188, 117 / 138 + 77 / 80, which is where the second reading of W costs more: up to 64 on average.
+constexpr int kExpertCols = 128, kExpertRows = 384, kFewRows = 128, kFewMean = 64;
 constexpr int kExpertStagesW = 3;
-constexpr int expert_stages_a(int mt) { return mt <= 4 ? 3 : 2; }
-constexpr size_t expert_lds(int mt) { return (size_t)(expert_stages_a(mt) * 64 * mt + kExpertStagesW * kExpertCols) * kRowBytes; }
+constexpr int expert_stages_a(int mt, bool few) { return mt <= (few ? 1 : 4) ? 3 : 2; }
+constexpr size_t expert_lds(int mt, bool few) { return (size_t)(expert_stages_a(mt, few) * 64 * mt + kExpertStagesW * kExpertCols) * kRowBytes; }
 // of `items` that are to be spread over the products [0, upto): the first one that goes behind product n or later
 __device__ constexpr int items_before(int n, int upto, int items) { return n >= upto ? items : n * items / upto; }
 
-template <int MT, int EPI>
+template <int MT, int EPI, bool FEW>
 __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, int first) {
-    constexpr int kSideA = 64 * MT * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(MT), RW = kExpertStagesW;
+    constexpr int kSideA = 64 * MT * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(MT, FEW), RW = kExpertStagesW;
     constexpr int kBehind = RA == RW ? (RA - 2) * (2 * MT + 4) : 4;   // copies that may be on their way at the wait
     constexpr int CA = 2 * MT, CW = 4, V = CA + CW, kEarly = V / 2;   // copies of a wave and K-step; those right behind the barrier
     constexpr int kProducts = 8 * MT, kReads = 8 + MT, kReadsUpto = MT == 1 ? 4 : kProducts * 3 / 4;
@@ -619,8 +623,8 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     store_rows<8, MT, EPI, true>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0);
 }
 
-template <int EPI>
-__global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_expert_kernel(const GemmKernelArgs<bf16> p) {
+template <int EPI, bool FEW>
+__global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_kernel(const GemmKernelArgs<bf16> p) {
     extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
     const int tiles_m = p.tiles[4 * p.tiles_m];
     const int total = tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
@@ -630,13 +634,21 @@ __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_expert_kernel(cons
     const int n0 = tile % p.tiles_n * kExpertCols, m0 = t[1], m_end = m0 + t[2];
     const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
     const int first = (5 * t[0] + 3 * (tile % p.tiles_n)) % (p.K / 64);
-    switch ((t[2] + 63) / 64) {
-        case 1: return expert_tile<1, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
-        case 2: return expert_tile<2, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
-        case 3: return expert_tile<3, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
-        case 4: return expert_tile<4, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
-        case 5: return expert_tile<5, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
-        default: return expert_tile<6, EPI>(p, gemm_lds, w, m0, m_end, n0, first);
+    if constexpr (FEW) {
+        if (t[2] <= 64) return expert_tile<1, EPI, true>(p, gemm_lds, w, m0, m_end, n0, first);
+        for (int m = m0; m < m_end; m += kFewRows) {   // (once, for a plan of the tile_rows that the launch was given)
+            if (m > m0) __syncthreads();
+            expert_tile<2, EPI, true>(p, gemm_lds, w, m, m_end - m < kFewRows ? m_end : m + kFewRows, n0, first);
+        }
+    } else {
+        switch ((t[2] + 63) / 64) {
+            case 1: return expert_tile<1, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 2: return expert_tile<2, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 3: return expert_tile<3, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 4: return expert_tile<4, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 5: return expert_tile<5, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            default: return expert_tile<6, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+        }
     }
 }
 
@@ -703,12 +715,14 @@ hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
     }
 }
 
+template <bool FEW>
 hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
     const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, kExpertRows, kExpertCols);
-    constexpr size_t lds = expert_lds(6);
-    static_assert(lds <= 160 * 1024 && expert_lds(4) <= lds && expert_lds(5) <= lds && 4 * kWideStore <= lds, "fits LDS");
-    return g.epilogue == kOutSwiglu ? run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutSwiglu>, p, kWideThreads, lds, 1, stream)
-                                    : run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutElem>, p, kWideThreads, lds, 1, stream);
+    constexpr size_t lds = FEW ? expert_lds(2, true) : expert_lds(6, false);
+    static_assert(lds <= (FEW ? 80 : 160) * 1024 && 4 * kWideStore <= lds, "fits LDS, twice for few rows");
+    static_assert(FEW ? expert_lds(1, true) <= lds : expert_lds(4, false) <= lds && expert_lds(5, false) <= lds, "the other heights too");
+    return g.epilogue == kOutSwiglu ? run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutSwiglu, FEW>, p, kWideThreads, lds, 1, stream)
+                                    : run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutElem, FEW>, p, kWideThreads, lds, 1, stream);
 }
 
 // out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
@@ -808,14 +822,17 @@ hipError_t launch_kind(const GemmArgs &g, int kind, int slices, hipStream_t stre
 
 // Rows of A per tile for a product of `rows` rows with each of `matrices` matrices.
 int dense_gemm_tile_rows(int dtype, int rows, int N, int matrices) {
-    if (dtype == kBf16 && matrices > 1) return kExpertRows;
+    if (dtype == kBf16 && matrices > 1) return rows <= kFewMean ? kFewRows : kExpertRows;
     if (rows <= 48 || N < 96) return 32;
     return dtype == kBf16 && rows > 128 ? 256 : 128;
 }
 
 hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStream_t stream) {
     if (dtype == kF32) return tile_rows == 32 ? launch_tile<float, 32, 128, 1, 4, 4>(g, 1, stream) : launch_tile<float, 128, 128, 2, 2, 2>(g, 1, stream);
-    if (g.tiles) return g.K < 1 << 26 ? launch_experts(g, stream) : hipErrorInvalidValue;   // (any plan: its tiles are 384 rows or less)
+    if (g.tiles) {   // (any plan: its tiles are 384 rows or less)
+        if (g.K >= 1 << 26) return hipErrorInvalidValue;
+        return tile_rows <= kFewRows ? launch_experts<true>(g, stream) : launch_experts<false>(g, stream);
+    }
     if (tile_rows == 32) return launch_tile<bf16, 32, 128, 1, 4, 4>(g, 1, stream);
     return launch_kind(g, tile_rows == 256 ? kWide256 : kWide128, 1, stream);
 }

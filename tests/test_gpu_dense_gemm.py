@@ -123,10 +123,10 @@ def test_parts_meet_in_the_row_kernels(dense, M, K):
 COUNTS = [(0, 1, 15, 128, 129, 255, 256, 257), (512, 0, 0, 300, 64, 127, 383, 385), (16, 16, 16, 16, 16, 16, 16, 16), (0, 0, 0, 700, 0, 0, 0, 0), [384, 385, 320, 770, 192, 321]]
 
 
-@pytest.mark.parametrize("tile_rows", [32, 128, 256, 384])
+@pytest.mark.parametrize("tile_rows,launched", [(32, 32), (128, 128), (256, 256), (384, 384), (384, 128), (64, 384)])   # of the plan, of the launch
 @pytest.mark.parametrize("counts", COUNTS)
-def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows):
-    print("experts", counts, tile_rows, flush=True)
+def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows, launched):
+    print("experts", counts, tile_rows, launched, flush=True)
     from air_hip import _lib
     lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
     E, K, ff, N, top = len(counts), 192, 144, 272, 2
@@ -144,7 +144,7 @@ def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows):
     _lib.check_dense(lib.dlm_moe_plan(ids.data_ptr(), entries, E, tile_rows, order.data_ptr(), tiles.data_ptr(), stream))
     act = torch.zeros((entries, 192), dtype=torch.bfloat16, device="cuda")
     out = torch.full((entries, N), 7.0, dtype=torch.bfloat16, device="cuda")
-    common = dict(tiles=tiles.data_ptr(), order=order.data_ptr(), M=entries, n_tiles=n_tiles, tile_rows=tile_rows)
+    common = dict(tiles=tiles.data_ptr(), order=order.data_ptr(), M=entries, n_tiles=n_tiles, tile_rows=launched)
     g = _lib.GemmArgs(a=h.data_ptr(), w=w1.data_ptr(), out=act.data_ptr(), lda=K, ldo=192, w_stride=2 * ff * K, N=2 * ff, K=K, epilogue=dense.OUT_SWIGLU,
                       gather=top, **common)
     _lib.check_dense(lib.dlm_gemm(0, ctypes.byref(g), stream))

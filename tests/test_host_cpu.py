@@ -404,3 +404,10 @@ def test_decode_run_leaves_a_model_without_a_final_norm_to_the_ops():
     rest = (torch.zeros((V, E)), torch.zeros((16, 64)), types.SimpleNamespace(n_heads=4, rms_eps=1e-5), [cache], 0, 1, torch.zeros(1, dtype=torch.int32))
     assert ops.decode_run(*args, torch.ones(E), *rest) is None   # (a norm that is not on the GPU)
     assert ops.decode_run(*args, None, *rest) is None
+
+
+def test_experts_with_few_rows_get_their_own_tiles():
+    """64 rows an expert on average or less: plans of 128-row tiles, two workgroups to a CU."""
+    lib = _lib.load_dense_library()
+    assert [lib.dlm_gemm_tile_rows(0, rows, 2048, 64) for rows in (0, 1, 16, 64, 65, 256, 4096)] == [128, 128, 128, 128, 384, 384, 384]
+    assert [lib.dlm_gemm_tile_rows(1, rows, 2048, 64) for rows in (16, 48, 49, 256)] == [32, 32, 128, 128]   # fp32
