@@ -108,8 +108,9 @@ int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream);
 /* Not grouped, with the tile (tile_rows is not read) and the number of slices along K chosen by shape: dlm_gemm_slices gives the
  * number, 1 .. 64 and at most K / 64 (a caller may take another one; more than one: bf16 only).  More than one slice: parts holds
  * slices * M * N floats, one matrix [M, N] after the other, that a second launch adds up into out; with out NULL (epilogue 1) they
- * are left to the caller, as dlm_add_norm_parts and dlm_residual_norm_parts take them. */
+ * are left to the caller, as dlm_add_norm_parts and dlm_residual_norm_parts take them: dlm_gemm_parts gives their number for that. */
 int dlm_gemm_slices(int dtype, int M, int N, int K, int epilogue);
+int dlm_gemm_parts(int dtype, int M, int N, int K);
 int dlm_gemm_sliced(int dtype, const dlm_gemm_args *g, int slices, float *parts, void *stream);
 
 int dlm_embed_rows(int dtype, const int32_t *tokens, const void *embed, float scale, float *res, void *h, int M, int width, void *stream);

@@ -168,6 +168,7 @@ DENSE_SYMBOLS = {
     "dlm_gemm_tile_rows": (_ci, [_ci] * 4),
     "dlm_gemm": (_ci, [_ci, _vp, _vp]),
     "dlm_gemm_slices": (_ci, [_ci] * 5),
+    "dlm_gemm_parts": (_ci, [_ci] * 4),
     "dlm_gemm_sliced": (_ci, [_ci, _vp, _ci, _vp, _vp]),
     "dlm_residual_norm_parts": (_ci, [_ci, _vp, _vp, _ci, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),
     "dlm_add_norm_parts": (_ci, [_ci, _vp, _vp, _ci, _vp, _cf, _ci, _vp, _ci, _ci, _vp]),

@@ -188,8 +188,8 @@ def gemm(a, w, out_f32=False, lda=None, rows=None, out=None, silu=None, gate=GAT
     begin, end = silu or (0, 0)
     epilogue = OUT_F32 if out_f32 else {GATE_NONE: OUT_ELEM, GATE_SILU: OUT_SWIGLU, GATE_GELU: OUT_GEGLU}[gate]
     dt = dtype_code(w)
-    slices = lib.dlm_gemm_slices(dt, M, N, K, epilogue)
     keep = parts and out_f32 and out is None
+    slices = lib.dlm_gemm_parts(dt, M, N, K) if keep else lib.dlm_gemm_slices(dt, M, N, K, epilogue)
     if out is None and not (keep and slices > 1):
         out = torch.empty((M, width), dtype=torch.float32 if out_f32 else w.dtype, device=w.device)
     pieces = torch.empty((slices, M, N), dtype=torch.float32, device=w.device) if slices > 1 else None

@@ -279,7 +279,11 @@ int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream) {
 }
 
 int dlm_gemm_slices(int dtype, int M, int N, int K, int epilogue) {
-    return bad_type(dtype) || M <= 0 || N <= 0 || K <= 0 ? 0 : dense_gemm_slices(dtype, M, N, K, epilogue);
+    return bad_type(dtype) || M <= 0 || N <= 0 || K <= 0 ? 0 : dense_gemm_slices(dtype, M, N, K, epilogue, false);
+}
+
+int dlm_gemm_parts(int dtype, int M, int N, int K) {
+    return bad_type(dtype) || M <= 0 || N <= 0 || K <= 0 ? 0 : dense_gemm_slices(dtype, M, N, K, kOutF32, true);
 }
 
 int dlm_gemm_sliced(int dtype, const dlm_gemm_args *g, int slices, float *parts, void *stream) {

@@ -771,7 +771,7 @@ constexpr GemmKind kGemmKinds[kKinds] = {
     {32, 128, 2, 1.0f, 0.215f, 0.43f, 6.8f}, {64, 128, 2, 0.f, 0.364f, 0.541f, 3.7f},  {128, 128, 2, 0.f, 0.547f, 0.866f, 4.4f},
     {128, 256, 1, 2.6f, 0.566f, 0.696f, 5.8f},
     {256, 192, 1, 5.8f, 0.728f, 0.947f, 10.3f}, {256, 256, 1, 7.5f, 0.953f, 1.201f, 11.f}};
-float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int slices) {
+float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int slices, bool kept) {
     const long tiles = (long)((M + k.rows - 1) / k.rows) * ((N + k.cols - 1) / k.cols) * slices, cap = 256 * k.together;
     const long full = tiles / cap, rest = tiles % cap;
     const int per = (steps + slices - 1) / slices;
@@ -779,22 +779,24 @@ float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int sl
     float t = 4.f + full * (k.tile_us + per * k.step_full_us);
     if (rest) t += k.tile_us + per * (k.step_us + (k.step_full_us - k.step_us) * rest / cap);
     if (epilogue == kOutF32 || slices > 1) t += slices * mb / k.store_tbs;
-    // whoever adds them up: the next kernel, or a launch (3.5 us on the GPU, 6 with its allocation on the host, which short prompts wait for)
-    if (slices > 1) t += epilogue == kOutF32 ? (slices - 1) * mb / 5.f : 6.f + (slices + 0.5f) * mb / 4.f;
+    // whoever adds them up: the next kernel where the parts are kept, else a launch (3.5 us on the GPU, 6 with its allocation on the host, which
+    // short prompts wait for)
+    if (slices > 1) t += kept ? (slices - 1) * mb / 5.f : 6.f + (slices + 0.5f) * mb / 4.f;
     return t;
 }
 
 struct GemmChoice {
     int kind, slices;
 };
-// slices 0: any number
-GemmChoice choose_gemm(int M, int N, int K, int epilogue, int slices) {
+// slices 0: any number; kept: the caller takes the parts.  Up to 128 columns are one tile's in any kind, so narrow tiles read nothing but their
+// little W again: a router, 2048 x 64 x 2048, takes 11 us in one launch of 32-row tiles, 17 in eight slices of 128-row ones and their sum.
+GemmChoice choose_gemm(int M, int N, int K, int epilogue, int slices, bool kept) {
     GemmChoice best{kWide256, 1};
     float least = 1e30f;
     const int steps = K / 64, first = slices ? slices : 1, last = slices ? slices : steps >= 8 ? (steps / 4 < 8 ? steps / 4 : 8) : 1;
-    for (int kind = M > 1024 ? kWide128 : M > 512 ? kTile128 : M > 256 ? kTile64 : kTile32; kind < kKinds; ++kind)
+    for (int kind = N <= 128 ? kTile32 : M > 1024 ? kWide128 : M > 512 ? kTile128 : M > 256 ? kTile64 : kTile32; kind < kKinds; ++kind)
         for (int n = first; n <= last; n *= 2) {
-            const float t = gemm_time(kGemmKinds[kind], M, N, steps, epilogue, n);
+            const float t = gemm_time(kGemmKinds[kind], M, N, steps, epilogue, n, kept);
             if (t < least) {
                 least = t;
                 best = {kind, n};
@@ -837,11 +839,11 @@ hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStr
     return launch_kind(g, tile_rows == 256 ? kWide256 : kWide128, 1, stream);
 }
 
-int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue) { return dtype == kBf16 ? choose_gemm(M, N, K, epilogue, 0).slices : 1; }
+int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue, bool kept) { return dtype == kBf16 ? choose_gemm(M, N, K, epilogue, 0, kept).slices : 1; }
 
 hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream) {
     if (dtype != kBf16 || g.tiles) return launch_dense_gemm(dtype, g, dense_gemm_tile_rows(dtype, g.M, g.N, 1), stream);
-    const int kind = choose_gemm(g.M, g.N, g.K, g.epilogue, slices).kind;
+    const int kind = choose_gemm(g.M, g.N, g.K, g.epilogue, slices, !g.out).kind;
     if (slices == 1) return launch_kind(g, kind, 1, stream);
     GemmArgs p = g;
     p.out = parts;

@@ -86,7 +86,7 @@ int dense_gemm_tile_rows(int dtype, int rows, int N, int matrices);   // rows of
 hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStream_t stream);
 // The same, not grouped, with tile and slices along K by shape.  More than one slice: parts holds slices * M * N floats, part after
 // part, that a second launch adds up; g.out == NULL (kOutF32): they are left to the caller.
-int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue);
+int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue, bool kept);   // kept: the caller takes the parts
 hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream);
 
 // v = embed[tokens] * scale, or res + y, or res; y: the sum of `parts` matrices [M, width]; res = v; h (optional) = the norm norm_w of v in the element type

@@ -411,3 +411,12 @@ def test_experts_with_few_rows_get_their_own_tiles():
     lib = _lib.load_dense_library()
     assert [lib.dlm_gemm_tile_rows(0, rows, 2048, 64) for rows in (0, 1, 16, 64, 65, 256, 4096)] == [128, 128, 128, 128, 384, 384, 384]
     assert [lib.dlm_gemm_tile_rows(1, rows, 2048, 64) for rows in (16, 48, 49, 256)] == [32, 32, 128, 128]   # fp32
+
+
+def test_slices_that_a_launch_adds_up_are_charged_for_it():
+    """fp32 products whose parts nobody takes: a router's narrow one runs whole; one whose caller takes the parts is cut."""
+    lib = _lib.load_dense_library()
+    assert [lib.dlm_gemm_slices(0, M, 64, 2048, 1) for M in (2048, 4096, 8192)] == [1] * 3
+    assert lib.dlm_gemm_parts(0, 2048, 2048, 8192) > 1 and lib.dlm_gemm_parts(0, 64, 2048, 8192) > 1
+    assert lib.dlm_gemm_slices(0, 64, 2048, 8192, 1) > 1                                     # worth its launch
+    assert lib.dlm_gemm_parts(1, 64, 2048, 8192) == 1 and lib.dlm_gemm_parts(0, 0, 64, 64) == 0   # fp32 weights, no rows
