@@ -239,9 +239,11 @@ int w4a16_gemm_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, 
  * columns and a slice of K and writes fp32 partial sums to `scratch`; a second launch adds the slices in slice order and
  * rounds once.  As many slices are taken as pay and fit (64 rows of K = 14336, N = 4096: 18 us with four, 32 us without).
  * w4a16_gemm_stream_scratch_bytes(M, K, N) is the scratch the call insists on (0: any, also none), and
- * w4a16_gemm_stream_best_scratch_bytes what the fastest plan takes (0: none): no initialisation,
- * nothing kept between calls, 16-byte aligned; calls that overlap on one GPU need a buffer each.  Same numerics as
- * w4a16_gemm_stream_bf16; the two differ by the order of the fp32 additions only. */
+ * w4a16_gemm_stream_best_scratch_bytes what is worth giving it (up to 1 GiB; 0: w4a16_gemm_stream_bf16 is as fast, a second launch and the
+ * buffer counted as 12 us of a host that issues calls back to back, which a captured graph does not pay): no initialisation,
+ * nothing kept between calls, 16-byte aligned; calls that overlap on one GPU need a buffer each.  Any row count may write to it, and
+ * the number of slices, so the order of the fp32 additions, depends on how much is given: the same call with a smaller buffer may differ in
+ * the last bit.  Same numerics as w4a16_gemm_stream_bf16 otherwise. */
 size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N);
 size_t w4a16_gemm_stream_best_scratch_bytes(int M, int K, int N);
 int w4a16_gemm_stream_scratch_bf16(const uint16_t *x, const void *wstream, uint16_t *y, int M, int K, int N, int group,
@@ -555,7 +557,7 @@ int w4a16_q4nx_gemv_stream_bf16(const uint16_t *x, const void *wstream, const ui
  * cell with its own (scale, min') word to W = bf16_rne(s q + min'), the dense dequant's values (q4nx_dequant_bf16,
  * bit for bit), and multiply those, which is what the reference's prompt pass of these models computes with its
  * dense bf16 GEMMs on dequantised weights (programming_examples/llms/llama31_8b_q4nx/README.md:11-15).
- * With scratch (may be NULL; w4a16_q4nx_gemm_stream_best_scratch_bytes is what the fastest plan takes, 0: none) as
+ * With scratch (may be NULL; w4a16_q4nx_gemm_stream_best_scratch_bytes is what is worth giving) as
  * w4a16_gemm_stream_scratch_bf16. */
 int w4a16_q4nx_gemm_stream_bf16(const uint16_t *x, const void *wstream, const uint16_t *residual, uint16_t *y, int M, int K, int N,
                                 void *stream);

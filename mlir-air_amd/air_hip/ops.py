@@ -287,8 +287,10 @@ def w4a16_gemm_stream(x, w, group=GROUP, out=None):
     if out is None:
         out = torch.empty((M, w.N), dtype=torch.bfloat16, device=x.device)
     scratch, nbytes = _gemm_scratch(lib.w4a16_gemm_stream_best_scratch_bytes(M, K, w.N) if M > 16 else 0, x.device)
-    _lib.check(lib.w4a16_gemm_stream_scratch_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group,
-                                                  _ptr(scratch) if nbytes else None, nbytes, _stream()))
+    if nbytes:
+        _lib.check(lib.w4a16_gemm_stream_scratch_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group, _ptr(scratch), nbytes, _stream()))
+    else:
+        _lib.check(lib.w4a16_gemm_stream_bf16(_ptr(_bits(x2)), _ptr(w.buf), _ptr(out), M, K, w.N, group, _stream()))
     return out.squeeze(0) if vec else out
 
 

@@ -425,9 +425,7 @@ double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
     double us = c.start + full * (c.group + step * (alone + more));
     if (rest > 0) us += c.group + step * (alone + more * rest);
     if (p.slices > 1) us += c.sum + p.slices * ((double)M * N * 8e-6 / c.tb_s);
-    // a second launch and its scratch take the host 12 us a call with the first (30 rows of K = 3328, N = 1472: 12.4 us back to back in slices
-    // that the GPU does in 8.5, 9.8 in one whole-K launch)
-    return p.slices > 1 && us < 12.0 ? 12.0 : us;
+    return us;
 }
 
 }  // namespace
