@@ -105,7 +105,8 @@ typedef struct {
 /* Rows of A per tile for `rows` rows (experts: the mean number) with each of `matrices` matrices of N rows. */
 int dlm_gemm_tile_rows(int dtype, int rows, int N, int matrices);
 int dlm_gemm(int dtype, const dlm_gemm_args *g, void *stream);
-/* Not grouped, with the tile (tile_rows is not read) and the number of slices along K chosen by shape: dlm_gemm_slices gives the
+/* Not grouped, with the tile (tile_rows -1 .. -6, for tests and measurements: 32 x 128, 64 x 128, 128 x 128, 128 x 256, 256 x 192, 256 x 256 of
+ * the bf16 kernels; not read otherwise) and the number of slices along K chosen by shape: dlm_gemm_slices gives the
  * number, 1 .. 64 and at most K / 64 (a caller may take another one; more than one: bf16 only).  More than one slice: parts holds
  * slices * M * N floats, one matrix [M, N] after the other, that a second launch adds up into out; with out NULL (epilogue 1) they
  * are left to the caller, as dlm_add_norm_parts and dlm_residual_norm_parts take them: dlm_gemm_parts gives their number for that. */

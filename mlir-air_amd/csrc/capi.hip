@@ -557,9 +557,9 @@ static WsmPlan gemm_stream_plan(int M, int K, int N, bool q4, bool residual, siz
     const bool rounded = gemm_stream_rounded(M, K, N, q4, residual);
     WsmPlan p;
     p.us = -1;
-    if (!gemm_wsm_supported(M, K, N) || (rounded ? tune.prefill_tile != 0 : tune.gemm_rows || tune.cb || tune.splitk == 2)) return p;
+    if (!gemm_wsm_supported(M, K, N) || (rounded ? tune.prefill_tile || tune.prefill_wsm == 2 : tune.gemm_rows || tune.cb || tune.splitk == 2)) return p;
     p = plan_gemm_wsm(M, K, N, q4, rounded, scratch_bytes);
-    const bool always = !rounded && tune.splitk == 1;
+    const bool always = rounded ? tune.prefill_wsm == 1 : tune.splitk == 1;
     if (!always && p.us > 0.95 * (rounded ? gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
     return p;
 }
@@ -1169,6 +1169,18 @@ int w4a16_tune(const char *key, int value) {
     } else if (!strcmp(key, "gemm_splitk")) {
         if (value < 0 || value > 2) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.splitk = value;
+    } else if (!strcmp(key, "gemm_wsm_rt")) {
+        if (value == 1 || value > 7) return W4A16_ERR_TUNE;
+        g_gemv_ws_tune.wsm_rt = value;
+    } else if (!strcmp(key, "gemm_wsm_nt")) {
+        if (value > 3) return W4A16_ERR_TUNE;
+        g_gemv_ws_tune.wsm_nt = value;
+    } else if (!strcmp(key, "gemm_wsm_slices")) {
+        if (value > 16) return W4A16_ERR_TUNE;
+        g_gemv_ws_tune.wsm_slices = value;
+    } else if (!strcmp(key, "prefill_wsm")) {
+        if (value > 2) return W4A16_ERR_TUNE;
+        g_gemv_ws_tune.prefill_wsm = value;
     } else if (!strcmp(key, "prefill_band")) {
         if (value > 64) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.prefill_band = value;

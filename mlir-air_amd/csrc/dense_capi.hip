@@ -292,9 +292,8 @@ int dlm_gemm_sliced(int dtype, const dlm_gemm_args *g, int slices, float *parts,
     if (g->tiles || slices < 1 || slices > g->K / 64 || slices > 64 || (slices > 1 && dtype != kBf16)) return DLM_ERR_SHAPE;
     if (slices == 1 ? !g->out : (!parts || (!g->out && g->epilogue != kOutF32))) return DLM_ERR_NULL;
     if (slices > 1 && odd(parts)) return DLM_ERR_ALIGN;
-    return done(launch_dense_gemm_sliced(dtype, a, slices, parts, hs(stream)));
+    return done(launch_dense_gemm_sliced(dtype, a, slices, parts, hs(stream), g->tile_rows < 0 && g->tile_rows >= -kGemmTiles ? -1 - g->tile_rows : -1));
 }
-
 
 int dlm_embed_rows(int dtype, const int32_t *tokens, const void *embed, float scale, float *res, void *h, int M, int width, void *stream) {
     if (!tokens || !embed || !res || !h) return DLM_ERR_NULL;

@@ -774,6 +774,7 @@ struct GemmKind {
     float tile_us, step_us, step_full_us, store_tbs;   // per tile; per K-step alone and in a full round; fp32 results
 };
 enum : int { kTile32, kTile64, kTile128, kWide128, kWide192, kWide256, kKinds };
+static_assert(kKinds == kGemmTiles, "");
 constexpr GemmKind kGemmKinds[kKinds] = {
     {32, 128, 2, 1.0f, 0.215f, 0.43f, 6.8f}, {64, 128, 2, 0.f, 0.364f, 0.541f, 3.7f},  {128, 128, 2, 0.f, 0.547f, 0.866f, 4.4f},
     {128, 256, 1, 2.6f, 0.566f, 0.696f, 5.8f},
@@ -848,9 +849,9 @@ hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStr
 
 int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue, bool kept) { return dtype == kBf16 ? choose_gemm(M, N, K, epilogue, 0, kept).slices : 1; }
 
-hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream) {
+hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream, int tile) {
     if (dtype != kBf16 || g.tiles) return launch_dense_gemm(dtype, g, dense_gemm_tile_rows(dtype, g.M, g.N, 1), stream);
-    const int kind = choose_gemm(g.M, g.N, g.K, g.epilogue, slices, !g.out).kind;
+    const int kind = tile >= 0 && tile < kKinds ? tile : choose_gemm(g.M, g.N, g.K, g.epilogue, slices, !g.out).kind;
     if (slices == 1) return launch_kind(g, kind, 1, stream);
     GemmArgs p = g;
     p.out = parts;

@@ -87,7 +87,8 @@ hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStr
 // The same, not grouped, with tile and slices along K by shape.  More than one slice: parts holds slices * M * N floats, part after
 // part, that a second launch adds up; g.out == NULL (kOutF32): they are left to the caller.
 int dense_gemm_slices(int dtype, int M, int N, int K, int epilogue, bool kept);   // kept: the caller takes the parts
-hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream);
+constexpr int kGemmTiles = 6;   // 32 x 128, 64 x 128, 128 x 128, 128 x 256, 256 x 192, 256 x 256
+hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, float *parts, hipStream_t stream, int tile = -1);   // tile: -1 by shape
 
 // v = embed[tokens] * scale, or res + y, or res; y: the sum of `parts` matrices [M, width]; res = v; h (optional) = the norm norm_w of v in the element type
 hipError_t launch_add_norm_rows(int dtype, float *res, const float *y, int parts, const int32_t *tokens, const void *embed, float scale, const float *norm_w,

@@ -431,23 +431,31 @@ double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
 }  // namespace
 
 WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch_bytes) {
-    const int tiles = (M + 15) / 16, G = K / kGroup;
+    const auto &tune = g_gemv_ws_tune;
+    const int tiles = (M + 15) / 16, G = K / kGroup, most_nt = rounded ? 3 : 2;
+    const int only_nt = tune.wsm_nt <= most_nt ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
     WsmPlan best;
     best.us = -1;
-    for (int nt = 1; nt <= (rounded ? 3 : 2); ++nt) {
+    for (int nt = 1; nt <= most_nt; ++nt) {
+        if (only_nt && nt != only_nt) continue;
         const int most = nt == 3 ? 5 : 7, least = nt == 3 ? 3 : 2, few = (tiles + most - 1) / most;
         const int options[3] = {few, few + 1, (tiles + 3) / 4};   // blocks of rows
         for (int blocks : options) {
             WsmPlan p;
             p.nt = nt;
             p.rt = std::max((tiles + blocks - 1) / blocks, least);
+            if (tune.wsm_rt) p.rt = std::min(std::max(tune.wsm_rt, least), most);
             p.blocks = (tiles + p.rt - 1) / p.rt;
-            for (int slices : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            auto try_slices = [&](int slices) {   // false: no room for so many
                 p.slices = slices;
-                if (slices > 1 && (rounded || G / slices < 2 || gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes)) break;
+                if (slices > 1 && (rounded || gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes)) return false;
                 p.us = wsm_us(p, M, K, N, q4, rounded);
                 if (best.us < 0 || p.us < best.us) best = p;
-            }
+                return true;
+            };
+            if (only_slices > 1 && try_slices(only_slices)) continue;
+            for (int slices : {1, 2, 3, 4, 6, 8, 12, 16})
+                if ((slices > 1 && (only_slices || G / slices < 2)) || !try_slices(slices)) break;
         }
     }
     return best;

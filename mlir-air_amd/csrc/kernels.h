@@ -108,7 +108,9 @@ struct GemvWsTune {
     int gemm_rows = 0;       // batched kernel: most rows per launch, 16, 32 or 64 (0 = 64)
     int prefill_min_m = 0;   // smallest M that w4a16_gemm_stream_bf16 gives to the prefill kernel (0 = default)
     int prefill_band = 0;    // prefill kernel: row panels per band of the tile order (0 = default)
-    int splitk = 0;          // exact products of 17 rows and more: 0 by shape, 1 always slices of K that fit the scratch, 2 always whole-K launches
+    int splitk = 0;          // exact products of 17 rows and more: 0 by shape, 1 always gemm_wsm.hip, in two slices of K where the scratch holds them, 2 always whole-K launches
+    int wsm_rt = 0, wsm_nt = 0, wsm_slices = 0;   // gemm_wsm.hip: row tiles, 64-column sets and slices where a kernel has them (0: by time)
+    int prefill_wsm = 0;     // products of rounded weights: 0 by time, 1 always gemm_wsm.hip, 2 never
     int prefill_swiglu_split = 0;   // 1: the prompt-pass FFN runs gate and up as two launches instead of one
 };
 extern GemvWsTune g_gemv_ws_tune;

@@ -157,9 +157,10 @@ hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t 
 // K where they pay and fit `scratch`
 static hipError_t product_add(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, const uint16_t *aux, void *scratch, size_t scratch_bytes,
                               hipStream_t stream, bool q4) {
-    if (gemm_wsm_supported(M, K, N) && !g_gemv_ws_tune.prefill_tile) {
+    const auto &tune = g_gemv_ws_tune;
+    if (gemm_wsm_supported(M, K, N) && !tune.prefill_tile && tune.prefill_wsm != 2) {
         const WsmPlan plan = plan_gemm_wsm(M, K, N, q4, true, 0);
-        if (plan.us < 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes)) return launch_gemm_wsm(plan, x, w, y, aux, nullptr, M, K, N, q4, true, stream);
+        if (tune.prefill_wsm == 1 || plan.us < 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes)) return launch_gemm_wsm(plan, x, w, y, aux, nullptr, M, K, N, q4, true, stream);
     }
     return launch_gemm_prefill_ws(x, w, y, M, K, N, stream, kEpiAddRounded, aux, nullptr, q4, static_cast<float *>(scratch), scratch_bytes);
 }

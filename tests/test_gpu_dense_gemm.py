@@ -1,4 +1,5 @@
-"""Products over many rows at the edges of their tiles and slices, against float64 products of the same bf16 numbers.
+"""Products over many rows at the edges of their tiles and slices, each tile set by hand and as the rule picks them, against float64 products of the
+same bf16 numbers.
 
 fp32 results: sums of K products of 16 significant bits in fp32, any order, stay within K 2^-24 of the sum of magnitudes, which for
 random signs is about K^1/2 times the result's rms; 2^-24 K^3/2 is 4e-5 at K = 8192, and what is seen is 30 times less.  bf16 results add
@@ -37,25 +38,24 @@ SHAPES = [(1, 16, 64, 1), (17, 144, 192, 3), (31, 96, 1024, 8), (33, 272, 128, 2
           (255, 240, 704, 4), (256, 512, 128, 2), (257, 1040, 448, 7), (300, 2048, 8192, 8), (513, 208, 640, 1), (700, 1104, 1216, 2), (1025, 3088, 192, 1)]
 
 
-@pytest.mark.parametrize("M,N,K,slices", SHAPES)
-def test_sliced_products(dense, M, N, K, slices):
-    print("sliced", M, N, K, slices, flush=True)
+def products(dense, M, N, K, counts, tile=0):
+    """Every epilogue in each number of slices, against float64; rows of A and out are longer than what is used of them."""
     from air_hip import _lib
     lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
     a, w = rand(M, M, K + 64).bfloat16()[:, 8:K + 8], (rand(N + 1, N, K) * K ** -0.5).bfloat16()
     want = a.double() @ w.double().t()
     pair = N // 32 * 32
     silu, gelu = torch.nn.functional.silu, lambda t: torch.nn.functional.gelu(t, approximate="tanh")
-    for n in {1, slices, lib.dlm_gemm_slices(0, M, N, K, dense.OUT_F32)}:
+    for n in counts:
         for epilogue in (dense.OUT_F32, dense.OUT_ELEM, dense.OUT_SWIGLU, dense.OUT_GEGLU):
             cols, width = (N, N) if epilogue < 2 else (pair, pair // 2)
             if not cols:
                 continue
             out = torch.full((M, width + 8), 7.0, device="cuda", dtype=torch.float32 if epilogue == dense.OUT_F32 else torch.bfloat16)
-            parts = torch.empty((n, M, cols), device="cuda")
+            parts = torch.full((n, M, cols), float("nan"), device="cuda")
             begin, end = (16, N // 32 * 16) if epilogue == dense.OUT_ELEM else (0, 0)
             g = _lib.GemmArgs(a=a.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), lda=a.stride(0), ldo=width + 8, M=M, N=cols, K=K, epilogue=epilogue,
-                              silu_begin=begin, silu_end=end)
+                              silu_begin=begin, silu_end=end, tile_rows=tile)
             _lib.check_dense(lib.dlm_gemm_sliced(0, ctypes.byref(g), n, parts.data_ptr(), stream))
             ref = want[:, :cols].clone()
             if epilogue >= 2:
@@ -65,6 +65,24 @@ def test_sliced_products(dense, M, N, K, slices):
                 ref[:, begin:end] = silu(ref[:, begin:end])
             close(out[:, :width], ref, epilogue != dense.OUT_F32, (n, epilogue))
             assert (out[:, width:] == 7.0).all(), "columns past the width were written"
+            assert bool(parts.isnan().all()) if n == 1 else bool(parts.isfinite().all()), "as many parts as slices"
+
+
+@pytest.mark.parametrize("M,N,K,slices", SHAPES)
+def test_sliced_products(dense, M, N, K, slices):
+    """The tiles that the rule picks."""
+    print("sliced", M, N, K, slices, flush=True)
+    from air_hip import _lib
+    products(dense, M, N, K, {1, slices, _lib.load_dense_library().dlm_gemm_slices(0, M, N, K, dense.OUT_F32)})
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("M,N,K", [(255, 208, 64), (257, 272, 128), (129, 144, 192), (513, 544, 256), (33, 400, 320)])
+def test_every_tile(dense, tile, M, N, K):
+    """Each of the six tiles at one row less and more than its blocks, one 16-column tile past its columns, one to five K-steps, in one slice and
+    in uneven ones (three, of one or two K-steps)."""
+    print("tile", tile, M, N, K, flush=True)
+    products(dense, M, N, K, {1, min(3, K // 64)}, -tile)
 
 
 @pytest.mark.parametrize("M,N,K,slices", [(64, 4096, 64, 1), (260, 2048, 128, 2), (1040, 512, 64, 1)])
@@ -178,11 +196,9 @@ def test_expert_plan(dense, entries, experts):
         n = int(tiles[most, 0])
         assert torch.equal(order.sort()[0], torch.arange(entries, dtype=torch.int32, device="cuda"))
         assert torch.equal(ids[order.long()], ids.sort()[0])
-        rows = tiles[:n].tolist()
-        assert n <= most and all(0 < r[2] <= bm for r in rows)
-        at = 0
-        for e, first, height, _ in rows:   # the tiles follow each other and stay within their expert
-            assert first == at
-            at += height
-            assert bool((ids[order[first:at].long()] == e).all()) if n <= 200 else True
-        assert at == entries
+        rows = tiles[:n].long()
+        assert n <= most and bool(((rows[:, 2] > 0) & (rows[:, 2] <= bm)).all())
+        # the tiles follow each other and stay within their expert
+        ends = rows[:, 2].cumsum(0)
+        assert torch.equal(rows[:, 1], ends - rows[:, 2]) and int(ends[-1]) == entries
+        assert torch.equal(ids[order.long()].long(), torch.repeat_interleave(rows[:, 0], rows[:, 2]))

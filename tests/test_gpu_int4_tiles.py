@@ -1,6 +1,7 @@
 """Int4 products of 17 rows and more at the edges of their row blocks, column sets, steps and slices, both codecs: exact weights against the
-float64 product (one bf16 rounding of an fp32 sum: 1 ulp and 2e-3, as for the other exact products), with no scratch and with scratch for
-any number of slices; rounded weights against the tiled kernel, bit for bit."""
+float64 product (one bf16 rounding of an fp32 sum: 1 ulp and 2e-3, as for the other exact products); rounded weights against the tiled kernel,
+bit for bit.  What the rule picks and two slices at a range of shapes, then every kernel that there is, set by hand, with slices of uneven length;
+the scratch says how many there were."""
 import numpy as np
 import pytest
 import torch
@@ -48,6 +49,7 @@ def test_int4_tiles(q4, M, K, N):
 
     rounded = M >= (65 if q4 else 129) and K % 256 == 0 and N % 64 == 0
     ops.tune("gemm_splitk", 1)
+    ops.tune("prefill_wsm", 1)
     try:
         for nbytes in (0, 1 << 26):
             got = call(nbytes, None)
@@ -62,7 +64,68 @@ def test_int4_tiles(q4, M, K, N):
                                   what=f"int4 tiles with a residual, {nbytes} bytes of scratch")
     finally:
         ops.tune("gemm_splitk", 0)
+        ops.tune("prefill_wsm", 0)
         ops.tune("prefill_tile", 0)
+
+
+@pytest.mark.parametrize("rt", [2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("mode", ["awq", "q4nx", "awq rounded", "q4nx rounded"])
+def test_every_int4_tile(mode, rt):
+    """Two blocks of rows or more, the last one ragged; two sets of columns and a ragged third; an odd number of groups in one slice, two and three."""
+    from air_hip import _lib, ops
+    q4, rounded = mode.startswith("q4nx"), mode.endswith("rounded")
+    lib, stream = _lib.load_library(), torch.cuda.current_stream().cuda_stream
+    M = 16 * rt * (max(129 // (16 * rt), 1) + 1) - 5
+    K = 256 * 3 if rounded else 128 * 11
+    for nt in (1, 2, 3) if rounded and 3 <= rt <= 5 else (1, 2):
+        N = 64 * nt * 2 + (64 if rounded else 48)
+        if rounded and nt == 1:
+            N = 128
+        print("int4 tile", mode, rt, nt, M, K, N, flush=True)
+        x = make_x((M, K), seed=M)
+        if q4:
+            q, s, m = make(N, K, seed=rt)
+            w = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+            dense = (q.astype(np.float64).reshape(N, K // 32, 32) * bf16_bits_to_f32(s).astype(np.float64)[:, :, None]
+                     + bf16_bits_to_f32(m).astype(np.float64)[:, :, None]).reshape(N, K).T
+        else:
+            tri = make_awq(K, N, seed=rt)
+            w, dense = ops.repack_stream(*map(dev, tri)), dense_f64(*tri)
+        want = bf16_bits_to_f32(x).astype(np.float64) @ dense
+        xd = dev(x)
+        fill = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+
+        def call(scratch):
+            y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+            at, nbytes = (None, 0) if scratch is None else (scratch.data_ptr(), scratch.numel() * 4)
+            if q4:
+                _lib.check(lib.w4a16_q4nx_gemm_stream_scratch_bf16(xd.data_ptr(), w.buf.data_ptr(), None, y.data_ptr(), M, K, N, at, nbytes, stream))
+            elif scratch is not None:
+                _lib.check(lib.w4a16_gemm_stream_scratch_bf16(xd.data_ptr(), w.buf.data_ptr(), y.data_ptr(), M, K, N, 128, at, nbytes, stream))
+            else:
+                _lib.check(lib.w4a16_gemm_stream_bf16(xd.data_ptr(), w.buf.data_ptr(), y.data_ptr(), M, K, N, 128, stream))
+            return bits(y)
+
+        keys = {"gemm_splitk": 1, "prefill_wsm": 1, "prefill_min_m": M if rounded else M + 1, "gemm_wsm_rt": rt, "gemm_wsm_nt": nt}
+        try:
+            for key, value in keys.items():
+                ops.tune(key, value)
+            if rounded:
+                got = call(None)
+                ops.tune("prefill_tile", 4)
+                assert np.array_equal(got, call(None)), (mode, rt, nt)
+                dense_r = bf16_bits_to_f32(f32_to_bf16_bits(np.ascontiguousarray(dense.astype(np.float32)))).astype(np.float64)
+                assert_bf16_close(got, bf16_bits_to_f32(x).astype(np.float64) @ dense_r, ulps=1.0, atol=2e-3, what=f"{mode} {rt} {nt}")
+                continue
+            for slices in (1, 2, 3):
+                ops.tune("gemm_wsm_slices", slices)
+                scratch = fill.repeat(4 * M * N)   # NaNs: a part is written whole, and nothing behind the parts
+                assert_bf16_close(call(scratch), want, ulps=1.0, atol=2e-3, what=f"{mode} {rt} {nt}, {slices} slices")
+                parts = slices * M * N if slices > 1 else 0
+                assert bool((scratch[:parts] != -1).all()) and bool((scratch[parts:] == -1).all()), "parts in the scratch"
+        finally:
+            for key in [*keys, "gemm_wsm_slices", "prefill_tile"]:
+                ops.tune(key, 0)
 
 
 @pytest.mark.parametrize("M,K,N", [(17, 128, 48), (40, 640, 272), (64, 2048, 528), (100, 384, 1040)])

@@ -197,11 +197,11 @@ def test_gemm_stream_more_than_sixteen_rows(ops, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(17, 256, 64), (32, 1024, 544), (48, 128 * 19, 48), (64, 4096, 6400), (65, 1024, 512),
                                    (128, 2048, 2048), (30, 128 * 19, 528), (64, 4096, 14336), (20, 14336, 4096), (33, 128, 272)])
 def test_gemm_stream_split_k_against_whole_k(ops, M, K, N):
-    """17 .. 128 rows through ops.w4a16_gemm_stream run split along K where that is the faster way (256-column
-    workgroups, x through LDS, the slices added by a second launch), else as the whole-K launches of
-    w4a16_gemm_stream_bf16; here each way is forced in turn.  Both are within one ulp of the float64 product (checked
+    """17 .. 128 rows through ops.w4a16_gemm_stream run in tiles of rows and columns, split along K where that is the faster
+    way (the slices added by a second launch), else as the whole-K launches of 16 to 64 rows; here tiles in two slices
+    and whole-K launches are forced in turn.  Both are within one ulp of the float64 product (checked
     by _gemm_case) and differ from each other by summation order only.  Shapes: one slice (K = 128), ragged column sets
-    (N = 48, 272, 528, 544), a short last quad of groups (19), two launches of rows (65, 128), both row-tile counts."""
+    (N = 48, 272, 528, 544), slices of uneven length (19 groups), two launches of rows (65, 128)."""
     try:
         ops.tune("gemm_splitk", 1)
         split = bf16_bits_to_f32(_gemm_case(ops, M, K, N, seed=M + K + N)).astype(np.float64)
@@ -214,13 +214,14 @@ def test_gemm_stream_split_k_against_whole_k(ops, M, K, N):
 
 
 def test_gemm_stream_split_k_scratch_contract(ops):
-    """The split-K entry point: scratch size by shape (none below 17 rows, above 128, or for a single slice), a short or
-    missing scratch buffer is refused before any launch, and the result does not depend on what the scratch held."""
+    """The split-K entry point: the scratch that it insists on by shape (none below 17 rows, above 128, or for a single slice), a
+    short or missing scratch buffer is refused before any launch, and the result (here in two slices) does not depend on what the
+    scratch held."""
     from air_hip import _lib
     lib = _lib.load_library()
     K, N, M = 1024, 512, 40
-    # by shape: long K, enough rows, and not where the whole-K workgroups are 64 columns wide already
-    assert lib.w4a16_gemm_stream_scratch_bytes(64, 14336, 4096) == 14 * 64 * 4096 * 4       # 112 groups in slices of 8
+    # by shape, whatever number of slices runs: long K, enough rows, and not where the whole-K workgroups are 64 columns wide already
+    assert lib.w4a16_gemm_stream_scratch_bytes(64, 14336, 4096) == 14 * 64 * 4096 * 4
     assert lib.w4a16_gemm_stream_scratch_bytes(64, 4096, 4096) > 0 and lib.w4a16_gemm_stream_scratch_bytes(32, 4096, 4096) == 0
     assert lib.w4a16_gemm_stream_scratch_bytes(64, 2048, 8192) == 0 and lib.w4a16_gemm_stream_scratch_bytes(64, 4096, 14336) == 0
     assert lib.w4a16_gemm_stream_scratch_bytes(M, K, N) == 0
@@ -236,8 +237,8 @@ def _split_k_scratch_contract(ops, lib, M, K, N):
     assert lib.w4a16_gemm_stream_scratch_bytes(16, K, N) == 0 and lib.w4a16_gemm_stream_scratch_bytes(129, K, N) == 0
     assert lib.w4a16_gemm_stream_scratch_bytes(M, 128, N) == 0                 # one group: one slice
     need = lib.w4a16_gemm_stream_scratch_bytes(M, K, N)
-    assert need == 2 * M * N * 4                                              # 8 groups in slices of 4
-    assert lib.w4a16_gemm_stream_scratch_bytes(128, K, N) == 2 * 64 * N * 4   # launches of 64 rows share it
+    assert need == 2 * M * N * 4
+    assert lib.w4a16_gemm_stream_scratch_bytes(128, K, N) == 2 * 64 * N * 4
     qw, qz, s = make_awq(K, N, seed=91)
     w = _stream_weight(ops, qw, qz, s)
     x = dev(make_x((M, K), seed=92))
@@ -253,6 +254,7 @@ def _split_k_scratch_contract(ops, lib, M, K, N):
     _lib.check(lib.w4a16_gemm_stream_scratch_bf16(p(x), p(w.buf), p(y), M, K, N, 128, p(scratch), need, st))
     y2 = ops.w4a16_gemm_stream(x, w)
     torch.cuda.synchronize()
+    assert not scratch.view(torch.int32).eq(-1).any(), "two slices fill the scratch"
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16)) and torch.isfinite(y.float()).all()
     # rows outside the split range go to the same launches as w4a16_gemm_stream_bf16, scratch or not
     x16 = x[:16].contiguous()
@@ -304,18 +306,20 @@ def test_gemm_stream_rows_equal_the_gemv_up_to_summation_order(ops):
 
 
 def _prefill_case(ops, M, K, N, seed):
-    """The tiled prefill kernel multiplies bf16-rounded weights W = bf16_rne((q - z) * s): within 1 bf16 ulp of the
+    """The tiled prefill kernel (gemm_wsm_kernel, which takes some of these shapes by itself, kept out) multiplies bf16-rounded weights W = bf16_rne((q - z) * s): within 1 bf16 ulp of the
     float64 product on those weights, and inside the reference's gate against the unrounded product
     (matmul_int4_packed.cpu_reference, matmul_int4_packed.py:89-105: rtol 0.1, atol 0.05, 0.05 % budget, r >= 0.999)."""
     print(f"prefill stream M={M} K={K} N={N} seed={seed}", flush=True)
     qw, qz, s = make_awq(K, N, seed=seed)
     x = make_x((M, K), seed=seed + 1)
     ops.tune("prefill_min_m", 17)   # (by itself the tiled kernel runs from M = 129 on)
+    ops.tune("prefill_wsm", 2)
     try:
         y = ops.w4a16_gemm_stream(dev(x), _stream_weight(ops, qw, qz, s))
         torch.cuda.synchronize()
     finally:
         ops.tune("prefill_min_m", 0)
+        ops.tune("prefill_wsm", 0)
     got = bits(y)
     xf = bf16_bits_to_f32(x).astype(np.float64)
     assert_bf16_close(got, xf @ dense_f64(qw, qz, s, rounded=True), ulps=1.0, atol=2e-3, what=f"prefill stream M={M} K={K} N={N}")
@@ -362,8 +366,8 @@ def test_prefill_stream_small_m_through_the_tiled_kernel(ops):
 
 
 def test_gemm_stream_hands_over_to_the_tiled_kernel_above_128_rows(ops):
-    """M = 128 is two launches of the batched kernel (unrounded weights), M = 129 the tiled kernel (bf16-rounded
-    weights): row 0 of x gives the batched kernel's bits in the first case and the tiled kernel's in the second."""
+    """M = 128 multiplies unrounded weights, M = 129 bf16-rounded ones: its first 128 rows have the tiled kernel's bits, whichever kernel
+    runs by itself."""
     K, N = 1024, 512
     qw, qz, s = make_awq(K, N, seed=55)
     w = _stream_weight(ops, qw, qz, s)
@@ -371,10 +375,12 @@ def test_gemm_stream_hands_over_to_the_tiled_kernel_above_128_rows(ops):
     y128 = bits(ops.w4a16_gemm_stream(dev(x[:128]), w))
     y129 = bits(ops.w4a16_gemm_stream(dev(x), w))
     ops.tune("prefill_min_m", 17)
+    ops.tune("prefill_wsm", 2)
     try:
         tiled = bits(ops.w4a16_gemm_stream(dev(x[:128]), w))
     finally:
         ops.tune("prefill_min_m", 0)
+        ops.tune("prefill_wsm", 0)
     batched = bits(ops.w4a16_gemm_stream(dev(x[:16]), w))
     torch.cuda.synchronize()
     assert np.array_equal(y129[:128], tiled) and not np.array_equal(y128, tiled)
