@@ -223,7 +223,7 @@ int w4a16_gemv_add_stream_bf16(const uint16_t *x, const void *wstream, const uin
 int w4a16_probe_stream_read(const void *wstream, uint32_t *out_words, int K, int N, void *stream);
 /* Batched decode on a stream-order matrix: y[M, N] = bf16(x[M, K] . W), unrounded weights, fp32 accumulation
  * (matmul_int4_packed.cpu_reference, programming_examples/matrix_multiplication/int4_awq/matmul_int4_packed.py:89-105;
- * device kernel matmul_int4_bf16_packed_f32, mv_int4_bf16.cc:430-448).  16 rows a launch, or more rows in one launch of
+ * device kernel matmul_int4_bf16_packed_f32, mv_int4_bf16.cc:430-448).  Up to 64 rows a launch, or any in one launch of
  * row and column tiles, by their expected times; stateless like the GEMV.  From M = 129 on, with K % 256 == 0 and
  * N % 64 == 0, the weights are dequantised to bf16 in registers (W = bf16_rne((q - z) * s), the dense dequant's values)
  * and multiplied by bf16 MFMA with fp32 accumulation.  So the numerics change between M = 128 and M = 129:

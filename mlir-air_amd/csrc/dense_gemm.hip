@@ -530,7 +530,7 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
         }
     };
     int fill_a = 0, fill_w = 0;   // stages that the next K-step's copies go to
-    // copy i of a K-step, A's first; behind the last one of each the source moves on (at the end it stays)
+    // copy i of a K-step, A's first; behind the last one of each the source moves on (from the last K-step to the first)
     int next_a = first, next_w = first;
     auto step_copy = [&](int i) {
         if (i < CA) {

@@ -137,8 +137,8 @@ hipError_t launch_prefill_o_ffn(const uint16_t *attn_out, const uint16_t *x_resi
     return launch_gemm_prefill(h, wd.qw, wd.qz, wd.sc, y, M, H, E, stream, kEpiAddRounded, res1, sk, cus);
 }
 
-// The same two blocks on stream-order weights (gemm_ws.hip): no split-K scratch, the narrow-tile choice of that kernel
-// covers the projections with few tiles.
+// The same two blocks on stream-order weights (gemm_ws.hip, gemm_wsm.hip).  The products with a residual may run in slices of K, whose
+// parts lie in what the workspace has free then (product_add); narrow tiles cover the other projections with few tiles.
 bool prefill_block_stream_supported(int M, int E, int H) {
     return prefill_block_supported(M, E, H) && gemm_prefill_ws_supported(M, E, E) && gemm_prefill_ws_supported(M, E, H) &&
            gemm_prefill_ws_supported(M, H, E);

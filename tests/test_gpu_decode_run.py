@@ -55,3 +55,37 @@ def test_decode_attention_past_a_trip(n_heads, n_kv, hd, max_seq, positions):
     import test_gpu_decode
     from air_hip import ops
     test_gpu_decode.test_decode_attention(ops, n_heads, n_kv, hd, max_seq, positions)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(8, 2, 64), (4, 4, 128), (16, 2, 128)])
+def test_decode_attention_with_infinities(n_heads, n_kv, hd):
+    """Keys that no head looks at (scores of minus infinity: one, a wave's positions, a whole chunk), an infinite value, a NaN key, and NaN
+    behind the last position; against float64 with the same rows."""
+    from air_hip import ops
+    print("attention infinities", n_heads, n_kv, hd, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(hd + n_heads)
+    randn = lambda *shape: torch.randn(shape, device="cuda", generator=g).bfloat16()
+    inf, pos, max_seq = float("inf"), 299, 320
+    lut = torch.cat([torch.ones(hd // 2), torch.zeros(hd // 2)]).bfloat16().cuda()   # no rotation
+    for rows, value, nan in ([77], None, None), (list(range(8)) + list(range(64, 136)), None, None), ([298], (150, -inf), None), ([0], (299, inf), 1):
+        qkv, k, v = randn((n_heads + 2 * n_kv) * hd), randn(n_kv, max_seq, hd), randn(n_kv, max_seq, hd)
+        q, k_new, v_new = (t.view(-1, hd) for t in qkv.split([n_heads * hd, n_kv * hd, n_kv * hd]))
+        q[:, 5] = q[:, 5].abs() + 1.0
+        k[:, rows, 5] = -inf
+        k[:, pos + 1:], v[:, pos + 1:] = float("nan"), float("nan")
+        if value:
+            (v_new if value[0] == pos else v[:, value[0]])[:, 3] = value[1]
+        if nan is not None:
+            k[0, nan, 9] = float("nan")
+        keys, values = k[:, :pos + 1].double(), v[:, :pos + 1].double()
+        keys[:, pos], values[:, pos] = k_new.double(), v_new.double()
+        out = ops.decode_attention(qkv, lut, k, v, pos, n_heads).view(n_heads, hd)
+        for h in range(n_heads):
+            kv = h // (n_heads // n_kv)
+            w = torch.softmax((keys[kv] * q[h].double()).sum(-1) * hd ** -0.5, 0)
+            want = (w[:, None] * values[kv]).sum(0)
+            assert torch.equal(out[h].isnan(), want.isnan()) and torch.equal(out[h].isinf(), want.isinf()), (h, rows, value, nan)
+            at = want.isfinite()
+            assert torch.equal(out[h][want.isinf()].double(), want[want.isinf()])
+            # as the other attention tests: 1 bf16 ulp (2^-7 of the value) and 2e-3
+            assert bool(((out[h].double() - want)[at].abs() <= 2.0 ** -7 * want[at].abs() + 2e-3).all())
