@@ -240,7 +240,7 @@ int w4a16_gemm_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, 
  * rounds once.  As many slices are taken as pay and fit (64 rows of K = 14336, N = 4096: 18 us with four, 32 us without).
  * w4a16_gemm_stream_scratch_bytes(M, K, N) is the scratch the call insists on (0: any, also none), and
  * w4a16_gemm_stream_best_scratch_bytes what is worth giving it (up to 1 GiB; 0: w4a16_gemm_stream_bf16 is as fast, a second launch and the
- * buffer counted as 12 us of a host that issues calls back to back, which a captured graph does not pay): no initialisation,
+ * buffer counted as 12.5 us of a host that issues calls back to back, which a captured graph does not pay): no initialisation,
  * nothing kept between calls, 16-byte aligned; calls that overlap on one GPU need a buffer each.  Any row count may write to it, and
  * the number of slices, so the order of the fp32 additions, depends on how much is given: the same call with a smaller buffer may differ in
  * the last bit.  Same numerics as w4a16_gemm_stream_bf16 otherwise. */

@@ -403,16 +403,17 @@ hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t str
     return plan.nt == 1 ? launch_wsm_rt<1, MODE>(plan.rt, p, stream) : launch_wsm_rt<2, MODE>(plan.rt, p, stream);
 }
 
-// The time of a launch, fitted to 10800 timings (13 matrices from 512 x 1024 to 13056 x 5744, 17 .. 3500 rows, every tile, 1 .. 16
-// slices; rms error 7 % exact, 10 % rounded; the plan it picks takes 1 % more than the best of them on average, 24 % at worst; Q4NX: a3 and b3 raised by what the third product took at 14 of them):
-// microseconds of start, of a workgroup, and of a step alone on the chip (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with
-// every CU busy; a step of four groups costs 1 + four of one of two.
+// The time of a launch on the GPU.  Exact modes: fitted to 3900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows,
+// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 1 % more than the best of them on average, 14 % at worst); rounded: to
+// 2500 (13 matrices, 65 .. 3500 rows; rms error 10 %, 24 % at worst).  Microseconds of start, of a workgroup, and of a step alone on the chip
+// (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of one of two.  The launch that
+// adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
 struct SmCost {
-    double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, tb_s;
+    double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, part, tb_s;
 };
-constexpr SmCost kSmCost[3] = {{2.6, 2.1, 0.06, 0.084, 0.075, 0.076, 0.16, 0.017, 0, 0, 0.69, 2.0, 5.9},
-                               {3.0, 1.6, 0, 0.042, 0.535, 0.123, 0.11, 0.021, 0.028, 0.023, 0.88, 1.9, 5.2},
-                               {1.8, 2.5, 0, 0.030, 0.150, 0.035, 0.07, 0.018, 0.09, 0.03, 0, 0, 1}};
+constexpr SmCost kSmCost[3] = {{2.94, 1.70, 0.184, 0.065, 0.055, 0.083, 0.154, 0, 0, 0, 0.65, 0.91, 0.23, 5.0},
+                               {3.79, 1.28, 0, 0.018, 0.422, 0.165, 0.138, 0.019, 0.089, 0, 0.83, 0.60, 0.21, 5.6},
+                               {1.8, 2.5, 0, 0.030, 0.150, 0.035, 0.07, 0.018, 0.09, 0.03, 0, 0, 0, 1}};
 
 double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
     const SmCost &c = kSmCost[rounded ? 2 : q4];
@@ -424,7 +425,7 @@ double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
     const double rest = (double)(wgs % chip) / chip, step = steps * (four ? 1 + c.four : 1.0);
     double us = c.start + full * (c.group + step * (alone + more));
     if (rest > 0) us += c.group + step * (alone + more * rest);
-    if (p.slices > 1) us += c.sum + p.slices * ((double)M * N * 8e-6 / c.tb_s);
+    if (p.slices > 1) us += c.sum + p.slices * (c.part + (double)M * N * 8e-6 / c.tb_s);
     return us;
 }
 

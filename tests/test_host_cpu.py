@@ -423,10 +423,10 @@ def test_slices_that_a_launch_adds_up_are_charged_for_it():
 
 
 def test_int4_slices_are_ranked_by_time_and_advised_past_what_their_launch_costs():
-    """Products under the 12 us that two launches and a buffer take a host: among sliced plans the fastest, not the first; and none where
+    """Products under the 12.5 us that two launches and a buffer take a host: among sliced plans the fastest, not the first; and none where
     the call without scratch is done by then."""
     lib = _lib.load_library()
     slices = lambda M, K, N: lib.w4a16_q4nx_gemm_stream_best_scratch_bytes(M, K, N, 0) / (4 * M * N)
-    assert slices(33, 128 * 19, 272) > 2 and slices(20, 5120, 1280) > 4   # (two and four were the first below 12 us)
+    assert slices(64, 4096, 1024) > 4 and slices(20, 5120, 1280) > 4 and slices(33, 128 * 19, 272) == 0   # (four were the first below 12 us)
     assert lib.w4a16_gemm_stream_best_scratch_bytes(30, 3328, 1472) == 0 and lib.w4a16_gemm_stream_best_scratch_bytes(20, 5120, 1280) == 0
     assert lib.w4a16_gemm_stream_best_scratch_bytes(64, 14336, 4096) >= lib.w4a16_gemm_stream_scratch_bytes(64, 14336, 4096)
