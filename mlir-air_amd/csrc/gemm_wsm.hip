@@ -404,7 +404,7 @@ hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t str
 }
 
 // The time of a launch on the GPU.  Exact modes: fitted to 3900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows,
-// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 1 % more than the best of them on average, 14 % at worst); rounded: to
+// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 0.5 % more than the best of them on average, 10 % at worst); rounded: to
 // 2500 (13 matrices, 65 .. 3500 rows; rms error 10 %, 24 % at worst).  Microseconds of start, of a workgroup, and of a step alone on the chip
 // (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of one of two.  The launch that
 // adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
@@ -437,6 +437,7 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
     const int only_nt = tune.wsm_nt <= most_nt ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
     WsmPlan best;
     best.us = -1;
+    double best_rank = 0;   // slices have to be 4 % faster: the estimate is no better than that
     for (int nt = 1; nt <= most_nt; ++nt) {
         if (only_nt && nt != only_nt) continue;
         const int most = nt == 3 ? 5 : 7, least = nt == 3 ? 3 : 2, few = (tiles + most - 1) / most;
@@ -451,7 +452,8 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
                 p.slices = slices;
                 if (slices > 1 && (rounded || gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes)) return false;
                 p.us = wsm_us(p, M, K, N, q4, rounded);
-                if (best.us < 0 || p.us < best.us) best = p;
+                const double rank = slices > 1 ? 1.04 * p.us : p.us;
+                if (best.us < 0 || rank < best_rank) best = p, best_rank = rank;
                 return true;
             };
             if (only_slices > 1 && try_slices(only_slices)) continue;
