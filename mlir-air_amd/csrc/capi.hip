@@ -575,7 +575,8 @@ static int gemm_stream_run(const uint16_t *x, const void *w, const uint16_t *res
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
 
-// Slices of at least four groups, 256 workgroups of 256 columns, 64 rows: what the call insists on where whole-K launches are slowest
+// What the call insists on where whole-K launches are slowest: slices of at least four groups, 256 workgroups of 256 columns, 64 rows.  The number
+// and the refusal of less are the entry point's contract; how many slices run, the plan says.
 size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N) {
     if (M <= 16 || M > kGemmWsMaxM || K <= 0 || N <= 0 || K % kGroup != 0 || N % kWsTileCols != 0 || g_gemv_ws_tune.splitk == 2) return 0;
     const int G = K / kGroup, tiles = N / kWsTileCols, rows = M < 64 ? M : 64, sets = (tiles + 15) / 16;
