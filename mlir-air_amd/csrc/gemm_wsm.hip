@@ -5,7 +5,7 @@
 // scalar instructions and the barrier are a chain.  So a workgroup puts KW waves on every SIMD, each set of four on a group of its own
 // (their sums meet in LDS at the end), and K is cut into slices besides where there are few columns.  64 rows, K = 14336, N = 4096: one
 // wave per SIMD 22.9 us, two 18.2 us, the launches of 64 whole-K rows that ran before 27.3 us (split along K) and 54.9 us; 300 rows of
-// K = 4096, N = 11008 43 us (tiled kernel: 54 us); Q4NX, 2048 rows of the ragged K = 2176, N = 5744 101 us (16 rows a launch: 972 us).
+// K = 4096, N = 11008 43 us (tiled kernel: 54 us); Q4NX, 2000 rows of the ragged K = 2176, N = 5744 151 us (16 rows a launch: 949 us).
 //
 //   workgroup  = 16 RT rows x 64 NT columns; wave (part kq < KW of K, wq < 4): row tiles all, stream tiles NT wq .. of the column set
 //   step       = KW groups; x goes global -> LDS once per workgroup (global_load_lds_dwordx4) and so do a wave's cells and scale words
