@@ -60,7 +60,9 @@ __device__ __forceinline__ void unpack8_f32(uint32_t w, float (&q)[8]) {
 
 // Maximum / sum over the 64 lanes of a wavefront, every lane receiving the result: the four steps inside a row of
 // 16 lanes on DPP moves (quad permutes for distances 1 and 2, half-row and row mirrors for 4 and 8: once the
-// quads agree, mirroring meets the partner quad), the two steps across rows by shuffle.
+// quads agree, mirroring meets the partner quad), the two steps across rows by exchanging rows and halves of two copies, which then hold a
+// lane's own value and its partner's (a shuffle goes through LDS; the same sums,
+// bit for bit.  The choice of 8 experts by one wave, eight maxima one after the other: 14.5 -> 14.0 us for the launch that makes it).
 template <bool MAX>
 __device__ __forceinline__ float wave_reduce(float v) {
     auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
@@ -73,8 +75,12 @@ __device__ __forceinline__ float wave_reduce(float v) {
     dpp(std::integral_constant<int, 0x4E>());    // quad_perm [2, 3, 0, 1]
     dpp(std::integral_constant<int, 0x141>());   // row_half_mirror
     dpp(std::integral_constant<int, 0x140>());   // row_mirror
-    v = op(v, __shfl_xor(v, 16));
-    return op(v, __shfl_xor(v, 32));
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);   // rows (0, 1) and (2, 3) exchanged
+    v = op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    const uint32_t w = __builtin_bit_cast(uint32_t, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(w, w, false, false);   // halves exchanged
+    return op(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1]));
 }
 
 // Maximum / sum over the 16 lanes of a DPP row, every lane of the row receiving it (the four in-row steps of wave_reduce).
