@@ -241,53 +241,88 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gate_up_gemv_kernel(const Moe
     }
 }
 
-// y[n] = sum_s weight_s (down_s h_s)[n]; a wave owns R rows, the pieces of all slots run through one loop
-template <class T, int R, int U>
-__global__ void __launch_bounds__(kMoeThreads) moe_down_gemv_kernel(const MoeGemv<T> p) {
+// y[n] = sum_s weight_s (down_s h_s)[n]; a wave owns a row, the pieces of all slots run through one loop, U of them in flight.  What bounds it:
+// HBM, behind two round trips, the choice's and the weights'.  So h is asked for first, a wave's pieces at once, then
+// the choice, a slot to a lane, and the weights before h is stored to LDS, all of a row where it is U pieces.  (No branch and no wait between
+// the requests: addresses past the end are clamped.)  8 experts of 2048 x 1024 (33.5 MB): 10.1 -> 8.9 us (a round trip per slot
+// for h and two rounds of 8 pieces before).
+template <class T, int U>
+__global__ void __launch_bounds__(kMoeThreads, 2) moe_down_gemv_kernel(const MoeGemv<T> p) {
     extern __shared__ __attribute__((aligned(16))) char moe_lds[];
     T *hs = reinterpret_cast<T *>(moe_lds);
-    const int kl = (p.ff + kMoePiece - 1) / kMoePiece * kMoePiece;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int s = 0; s < p.top; ++s) {
-        for (int i = 8 * tid; i < p.ff; i += 8 * kMoeThreads) store8(hs + s * kl + i, load8(p.h + (size_t)s * p.ff + i));
-        for (int i = p.ff + 8 * tid; i < kl; i += 8 * kMoeThreads) store8(hs + s * kl + i, zero8<T>());
+    constexpr int H = 4;   // pieces of h that a wave has in flight
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int pieces = (p.ff + kMoePiece - 1) / kMoePiece, items = p.top * pieces, stride = gridDim.x * kMoeWaves;
+    const int last = p.ff - 8;   // (ff is a multiple of 64)
+    // element offset of this lane's chunk in piece i: slot i / pieces, and whether the piece has that much
+    auto chunk = [&](int i, int &slot, bool &in) {
+        slot = i / pieces;
+        const int k = (i - slot * pieces) * kMoePiece + 8 * lane;
+        in = k <= last;
+        return in ? k : last;
+    };
+    Vec8<T> hv[H];
+    auto request_h = [&](int i0) {
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+            int slot;
+            bool in;
+            const int k = chunk(min(i0 + kMoeWaves * j, items - 1), slot, in);
+            hv[j] = load8(p.h + (size_t)slot * p.ff + k);
+            if (!in) hv[j] = zero8<T>();
+        }
+    };
+    request_h(wave);
+    const int id = p.ids[lane < p.top ? lane : 0];   // (top <= 32)
+    const float weight = p.weights[lane < p.top ? lane : 0];
+    int n = blockIdx.x * kMoeWaves + wave;
+    Vec8<T> w[U];
+    float wt[U];
+    auto request = [&](int row, int i0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int slot;
+            bool in;
+            const int k = chunk(min(i0 + u, items - 1), slot, in);
+            const int expert = __builtin_amdgcn_readlane(id, slot);
+            const float x = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), slot));
+            wt[u] = i0 + u < items ? x : 0.f;
+            w[u] = stream8(p.w + ((size_t)expert * p.N + row) * p.ff + k);
+        }
+    };
+    request(min(n, p.N - 1), 0);
+    for (int i0 = wave;;) {
+#pragma unroll
+        for (int j = 0; j < H; ++j)
+            if (i0 + kMoeWaves * j < items) store8(hs + (i0 + kMoeWaves * j) * kMoePiece + 8 * lane, hv[j]);   // (slot s, piece c) lies at s * kl + c * 512
+        i0 += kMoeWaves * H;
+        if (i0 >= items) break;
+        request_h(i0);
     }
     __syncthreads();
-    const int pieces = kl / kMoePiece, items = p.top * pieces;
-    for (int n0 = (blockIdx.x * kMoeWaves + wave) * R; n0 < p.N; n0 += gridDim.x * kMoeWaves * R) {
-        float acc[R];
+    float acc = 0.f;
+    for (int i0 = 0; n < p.N;) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = 0.f;
-        for (int i0 = 0; i0 < items; i0 += U) {
-            Vec8<T> w[R][U];
-            float wt[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = i0 + u < items ? i0 + u : items - 1;
-                const int s = i / pieces, k = (i % pieces) * kMoePiece + 8 * lane;
-                wt[u] = i0 + u < items ? p.weights[s] : 0.f;
-                const T *base = p.w + (size_t)p.ids[s] * p.N * p.ff + k;
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int row = n0 + r < p.N ? n0 + r : p.N - 1;
-                    w[r][u] = k < p.ff ? stream8(base + (size_t)row * p.ff) : zero8<T>();
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = i0 + u < items ? i0 + u : items - 1;
-                const Vec8<T> hv = load8(hs + i * kMoePiece + 8 * lane);   // (slot s, piece c) lies at s * kl + c * 512
-#pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] = fmaf(wt[u], dot8(w[r][u], hv, 0.f), acc[r]);
-            }
+        for (int u = 0; u < U; ++u) {
+            int slot;
+            bool in;
+            const int i = min(i0 + u, items - 1);
+            chunk(i, slot, in);
+            const Vec8<T> row = in ? w[u] : zero8<T>();
+            acc = fmaf(wt[u], dot8(row, load8(hs + i * kMoePiece + 8 * lane), 0.f), acc);
         }
-        float mine = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float s = wave_reduce<false>(acc[r]);
-            mine = lane == r ? s : mine;
+        __builtin_amdgcn_sched_barrier(0);   // (the next weights go into the same registers)
+        i0 += U;
+        if (i0 >= items) {
+            const float sum = wave_reduce<false>(acc);
+            if (lane == 0) p.y[n] = sum;
+            acc = 0.f;
+            i0 = 0;
+            n += stride;
+            if (n >= p.N) break;
         }
-        if (lane < R && n0 + lane < p.N) p.y[n0 + lane] = mine;
+        request(n, i0);
     }
 }
 
@@ -337,7 +372,7 @@ hipError_t down(const void *h, const void *w, const int32_t *ids, const float *w
     p.N = N;
     p.top = top;
     const size_t lds = (size_t)top * ((ff + kMoePiece - 1) / kMoePiece) * kMoePiece * sizeof(T);
-    auto kernel = &moe_down_gemv_kernel<T, 1, 8>;
+    auto kernel = &moe_down_gemv_kernel<T, sizeof(T) == 2 ? 16 : 8>;
     const hipError_t e = with_lds(kernel, lds);
     if (e != hipSuccess) return e;
     const int need = (N + kMoeWaves - 1) / kMoeWaves;
