@@ -8,7 +8,7 @@
 // The intake computes x where another kernel would otherwise be launched for it: the embedding row, or the residual
 // stream with the normed output of the previous sublayer added (every workgroup redoes this small sum from L2; one of
 // them stores it), or the final norm of that, or the norm of the stream with the previous sublayer's output added.  The first
-// weights are requested before it.  The row sums can be combined in pairs: activation of a gate row times an up row.
+// weights are requested before it is waited for.  The row sums can be combined in pairs: activation of a gate row times an up row.
 #include "dense.h"
 #include "dense_kernels.h"
 
@@ -19,6 +19,7 @@ namespace {
 constexpr int kGemvWaves = 4, kGemvThreads = 64 * kGemvWaves;
 constexpr int kMaxBlocks = 1024;
 constexpr int kPiece = 512;   // elements of a row that a wave reads at once
+constexpr int kIntakeNormedEmbed = 8;   // kIntakeNormed of an embedding row
 
 template <class T>
 struct GemvParams {
@@ -51,122 +52,141 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
     return s;
 }
 
-// x into LDS (K elements, zeros up to the next piece)
+// x into LDS (K elements, zeros up to the next piece).  What it is made of is asked for in front of the first weights (a wave's loads return in
+// order) and all at once, up to 2048 elements of it (as they are: 8192) kept in registers from one pass over x to the next.  (Behind the weights, a
+// round trip per 1024 elements and pass: gate and up of 2 x 8192 x 2048 behind a norm 14.1 -> 12.8 us = 5.3 TB/s, a router of 64 x 2048 behind a residual 4.5 -> 3.3 us.)
 template <class T, int MODE>
-__device__ __forceinline__ void take_in(const GemvParams<T> &p, T *xs, float *red) {
-    const int tid = threadIdx.x;
-    const int kl = (p.K + kPiece - 1) / kPiece * kPiece;
-    for (int i = p.K + 8 * tid; i < kl; i += 8 * kGemvThreads) store8(xs + i, zero8<T>());
-    if constexpr (MODE == kIntakePlain) {
-        for (int i = 8 * tid; i < p.K; i += 8 * kGemvThreads) store8(xs + i, load8(p.x + i));
-    } else if constexpr (MODE == kIntakeEmbed) {
-        const T *row = p.embed + (size_t)p.token[0] * p.K;
-        for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-            float e[4];
-            load4(row + i, e);
+struct Intake {
+    static constexpr int NB = MODE == kIntakePlain ? 8 : 2, kStep = 4 * kGemvThreads;   // quads of a thread in a batch; elements between them
+    static constexpr bool kRow = MODE == kIntakeEmbed || MODE == kIntakeNormedEmbed, kNormed = MODE == kIntakeNormed || MODE == kIntakeNormedEmbed;
+    const GemvParams<T> &p;
+    T *xs;
+    float *red;
+    Vec8<T> x[NB / 2];
+    floatx4 res[NB], y[NB], norm[NB], last[NB];
+
+    __device__ __forceinline__ int quad(int q, int b) const { return 4 * (int)threadIdx.x + (q * NB + b) * kStep; }
+    __device__ __forceinline__ static floatx4 quad_of(const float *v) { return *reinterpret_cast<const floatx4 *>(v); }
+    // batch q of the operands; past the end the last ones
+    __device__ __forceinline__ void load(int q) {
+        if constexpr (MODE == kIntakePlain) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) e[j] *= p.scale;
-            store4(xs + i, e[0], e[1], e[2], e[3]);
-            if (blockIdx.x == 0) {
-                store4(p.res_out + i, e[0], e[1], e[2], e[3]);
-                if (p.h_out) store4(p.h_out + i, e[0], e[1], e[2], e[3]);
+            for (int b = 0; b < NB / 2; ++b) {
+                const int i = 2 * (4 * (int)threadIdx.x + (q * NB / 2 + b) * kStep);
+                x[b] = load8(p.x + (i < p.K ? i : p.K - 8));
             }
+            return;
         }
-    } else if constexpr (MODE == kIntakeNormed) {
-        const T *row = p.embed ? p.embed + (size_t)p.token[0] * p.K : nullptr;
-        auto value = [&](int i, float (&v)[4]) {
-            if (row) {
-                load4(row + i, v);
+        const T *row = kRow ? p.embed + (size_t)p.token[0] * p.K : nullptr;
+        const float *ys = p.y ? p.y : p.res, *norms = p.y ? p.norm_w : p.res;   // (without y: read all the same, and not used)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] *= p.scale;
-                return;
+        for (int b = 0; b < NB; ++b) {
+            const int i = quad(q, b) < p.K ? quad(q, b) : p.K - 4;
+            if constexpr (kRow) {
+                float e[4];
+                load4(row + i, e);
+                res[b] = floatx4{e[0], e[1], e[2], e[3]} * p.scale;
+            } else {
+                res[b] = quad_of(p.res + i);
+                y[b] = quad_of(ys + i);
             }
-            load4(p.res + i, v);
-            if (p.y) {
-                float u[4];
-                load4(p.y + i, u);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] += u[j];
-            }
-        };
-        float ss = 0.f;
-        for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-            float v[4];
-            value(i, v);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
-            if (blockIdx.x == 0 && p.res_out) store4(p.res_out + i, v[0], v[1], v[2], v[3]);
-        }
-        const float rstd = 1.0f / sqrtf(block_sum(ss, red) / (float)p.width + p.eps);
-        for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-            float v[4], w[4];
-            value(i, v);
-            load4(p.final_w + i, w);
-            store4(xs + i, v[0] * rstd * w[0], v[1] * rstd * w[1], v[2] * rstd * w[2], v[3] * rstd * w[3]);
-        }
-    } else {
-        float rstd = 0.f;
-        if (p.y) {
-            float ss = 0.f;
-            for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-                float v[4];
-                load4(p.y + i, v);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
-            }
-            rstd = 1.0f / sqrtf(block_sum(ss, red) / (float)p.width + p.eps);
-        }
-        auto value = [&](int i, float (&v)[4]) {
-            load4(p.res + i, v);
-            if (p.y) {
-                float u[4], w[4];
-                load4(p.y + i, u);
-                load4(p.norm_w + i, w);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = fmaf(u[j] * rstd, w[j], v[j]);
-            }
-        };
-        if constexpr (MODE == kIntakeResidual) {
-            for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-                float v[4];
-                value(i, v);
-                store4(xs + i, v[0], v[1], v[2], v[3]);
-                if (blockIdx.x == 0) {
-                    if (p.res_out) store4(p.res_out + i, v[0], v[1], v[2], v[3]);
-                    if (p.h_out) store4(p.h_out + i, v[0], v[1], v[2], v[3]);
-                }
-            }
-        } else {
-            float ss = 0.f;
-            for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-                float v[4];
-                value(i, v);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
-            }
-            const float r2 = 1.0f / sqrtf(block_sum(ss, red) / (float)p.width + p.eps);
-            for (int i = 4 * tid; i < p.K; i += 4 * kGemvThreads) {
-                float v[4], w[4];
-                value(i, v);
-                load4(p.final_w + i, w);
-                store4(xs + i, v[0] * r2 * w[0], v[1] * r2 * w[1], v[2] * r2 * w[2], v[3] * r2 * w[3]);
-            }
+            if constexpr (MODE == kIntakeResidual || MODE == kIntakeFinal) norm[b] = quad_of(norms + i);
+            if constexpr (MODE == kIntakeFinal || kNormed) last[b] = quad_of(p.final_w + i);
         }
     }
-}
+    __device__ __forceinline__ static float squares(floatx4 v, float ss) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
+        return ss;
+    }
+    __device__ __forceinline__ float rstd_of(float ss) const { return 1.0f / sqrtf(block_sum(ss, red) / (float)p.width + p.eps); }
+    // f(batch's index b, first element) over all of x; `again`: the operands of the batch are to be loaded (if they are not the only one's)
+    template <class F>
+    __device__ __forceinline__ void pass(bool again, F f) {
+        const int batches = (p.K + NB * kStep - 1) / (NB * kStep);
+        for (int q = 0; q < batches; ++q) {
+            if (q > 0 || (again && batches > 1)) load(q);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                if (quad(q, b) < p.K) f(b, quad(q, b));
+        }
+    }
+    __device__ __forceinline__ void finish() {
+        const int kl = (p.K + kPiece - 1) / kPiece * kPiece;
+        for (int i = p.K + 8 * (int)threadIdx.x; i < kl; i += 8 * kGemvThreads) store8(xs + i, zero8<T>());
+        if constexpr (MODE == kIntakePlain) {
+            for (int q = 0; q * NB * kStep < p.K; ++q) {
+                if (q > 0) load(q);
+#pragma unroll
+                for (int b = 0; b < NB / 2; ++b) {
+                    const int i = 2 * (4 * (int)threadIdx.x + (q * NB / 2 + b) * kStep);
+                    if (i < p.K) store8(xs + i, x[b]);
+                }
+            }
+            return;
+        }
+        // the new residual, kept in `res`
+        float rstd = 0.f;
+        bool again = false;   // behind a first pass over several batches
+        if constexpr (MODE == kIntakeResidual || MODE == kIntakeFinal) {
+            if (p.y) {
+                float ss = 0.f;
+                pass(false, [&](int b, int) { ss = squares(y[b], ss); });
+                rstd = rstd_of(ss);
+                again = true;
+            }
+        }
+        auto value = [&](int b) {
+            if constexpr (kRow) return res[b];
+            if constexpr (MODE == kIntakeNormed) return p.y ? res[b] + y[b] : res[b];
+            floatx4 v = res[b];
+            if (p.y) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = fmaf(y[b][j] * rstd, norm[b][j], v[j]);
+            }
+            return v;
+        };
+        auto keep = [&](int i, floatx4 v) {
+            if (blockIdx.x != 0) return;
+            if (p.res_out) store4(p.res_out + i, v[0], v[1], v[2], v[3]);
+            if constexpr (!kNormed)
+                if (p.h_out) store4(p.h_out + i, v[0], v[1], v[2], v[3]);
+        };
+        if constexpr (MODE == kIntakeEmbed || MODE == kIntakeResidual) {
+            pass(again, [&](int b, int i) {
+                const floatx4 v = value(b);
+                store4(xs + i, v[0], v[1], v[2], v[3]);
+                keep(i, v);
+            });
+        } else {
+            float ss = 0.f;
+            pass(again, [&](int b, int i) {
+                const floatx4 v = value(b);
+                ss = squares(v, ss);
+                if constexpr (kNormed) keep(i, v);
+            });
+            const float r2 = rstd_of(ss);
+            pass(true, [&](int b, int i) {
+                const floatx4 v = value(b), w = last[b];
+                store4(xs + i, v[0] * r2 * w[0], v[1] * r2 * w[1], v[2] * r2 * w[2], v[3] * r2 * w[3]);
+            });
+        }
+    }
+};
 
-// (PAIR: rows 2 o and 2 o + 1 of the walk are the gate and the up row of output o)
+// (PAIR: rows 2 o and 2 o + 1 of the walk are the gate and the up row of output o.)  Past the end: read in range, left out of the
+// sum or never stored; no branch, behind which nobody could count the requests that are on their way.
 template <class T, int R, int U, bool PAIR>
 __device__ __forceinline__ void request(Vec8<T> (&w)[R][U], const T *base, int K, int N, int row0, int c0) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        int row = row0 + r < N ? row0 + r : N - 1;   // past the end: read in range, never stored
+        int row = row0 + r < N ? row0 + r : N - 1;
         if constexpr (PAIR) row = (row >> 5) * 32 + ((row & 31) >> 1) + 16 * (row & 1);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = (c0 + u) * kPiece + 8 * lane;
-            w[r][u] = k < K ? stream8(base + (size_t)row * K + k) : zero8<T>();
+            w[r][u] = stream8(base + (size_t)row * K + (k < K ? k : K - 8));
         }
     }
 }
@@ -181,8 +201,12 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
     const int pieces = (p.K + kPiece - 1) / kPiece;
     int g = blockIdx.x * kGemvWaves + wave;
     Vec8<T> w[R][U];
-    if (g < p.groups) request<T, R, U, PAIR>(w, p.w, p.K, p.N, g * R, 0);
-    take_in<T, MODE>(p, xs, red);
+    Intake<T, MODE> in{p, xs, red};
+    in.load(0);
+    __builtin_amdgcn_sched_barrier(0);
+    request<T, R, U, PAIR>(w, p.w, p.K, p.N, g * R, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    in.finish();
     __syncthreads();
     unsigned long long best = 0;
     for (; g < p.groups; g += stride) {
@@ -192,10 +216,11 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
         for (int c0 = 0; c0 < pieces; c0 += U) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int c = c0 + u < pieces ? c0 + u : pieces - 1;   // (weights past the last piece are zeros)
-                const Vec8<T> xv = load8(xs + c * kPiece + 8 * lane);
+                if (c0 + u >= pieces) break;   // uniform
+                const Vec8<T> xv = load8(xs + (c0 + u) * kPiece + 8 * lane);
+                const bool in = (c0 + u) * kPiece + 8 * lane < p.K;
 #pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] = dot8(w[r][u], xv, acc[r]);
+                for (int r = 0; r < R; ++r) acc[r] = dot8(in ? w[r][u] : zero8<T>(), xv, acc[r]);
             }
             if (c0 + U < pieces) request<T, R, U, PAIR>(w, p.w, p.K, p.N, g * R, c0 + U);
         }
@@ -266,14 +291,17 @@ hipError_t launch_mode(const GemvParams<T> &p, int mode, int grid, size_t lds, h
     };
     if (p.ro.gate) {
         if constexpr (R >= 2)
-            return mode == kIntakeNormed ? run(&dense_gemv_kernel<T, R, U, kIntakeNormed, true>) : run(&dense_gemv_kernel<T, R, U, kIntakePlain, true>);
+            return mode != kIntakeNormed ? run(&dense_gemv_kernel<T, R, U, kIntakePlain, true>)
+                   : p.embed             ? run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, true>)
+                                         : run(&dense_gemv_kernel<T, R, U, kIntakeNormed, true>);
         return hipErrorInvalidValue;
     }
-    switch (mode) {
+    switch (mode == kIntakeNormed && p.embed ? (int)kIntakeNormedEmbed : mode) {
         case kIntakePlain: return run(&dense_gemv_kernel<T, R, U, kIntakePlain, false>);
         case kIntakeResidual: return run(&dense_gemv_kernel<T, R, U, kIntakeResidual, false>);
         case kIntakeEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeEmbed, false>);
         case kIntakeNormed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormed, false>);
+        case kIntakeNormedEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, false>);
         default: return run(&dense_gemv_kernel<T, R, U, kIntakeFinal, false>);
     }
 }
