@@ -261,8 +261,15 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
 __global__ void __launch_bounds__(1024) argmax_keys_kernel(const unsigned long long *keys, int n, int32_t *token, int32_t *position,
                                                            int32_t *history) {
     __shared__ unsigned long long part[16];
+    const int32_t here = position ? position[0] : 0;   // (every thread: asked for with the keys)
     unsigned long long best = 0;
-    for (int i = threadIdx.x; i < n; i += 1024) best = keys[i] > best ? keys[i] : best;
+    for (int i0 = threadIdx.x; i0 < n; i0 += 4 * 1024) {   // four at a time: a round trip for up to 4096 of them
+        unsigned long long k[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k[j] = keys[i0 + 1024 * j < n ? i0 + 1024 * j : i0];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) best = k[j] > best ? k[j] : best;
+    }
     best = wave_max_u64(best);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
     __syncthreads();
@@ -272,7 +279,7 @@ __global__ void __launch_bounds__(1024) argmax_keys_kernel(const unsigned long l
         const int32_t id = (int32_t)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull));
         if (token) token[0] = id;
         if (position) {
-            const int32_t next = position[0] + 1;   // the position of the chosen token
+            const int32_t next = here + 1;   // the position of the chosen token
             position[0] = next;
             if (history) history[next] = id;
         }

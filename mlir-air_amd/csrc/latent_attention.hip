@@ -48,26 +48,41 @@ __device__ __forceinline__ void rotate_pair(const T *src, T *dst, const float *l
     dst[1] = from_float<T>(v * c + u * s);
 }
 
-// The cache row of token m: by one workgroup.  Padding columns of the projections are zeros and stay zeros.
+// The cache row of token m: by one workgroup.  Padding columns of the projections are zeros and stay zeros.  (Up to 1024 columns are read
+// once, with the norm's weights, before the position is there.)
 template <class T>
 __device__ __forceinline__ void append_row(const LatentArgs<T> &p, int m, int position, float *red) {
+    constexpr int NB = 4;
     const T *src = p.proj + (size_t)m * p.ld + p.kv_off;
     T *dst = p.cache + (size_t)position * (p.s.rank + p.s.rot);
+    float x[NB], w[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int at = (int)threadIdx.x + kLatThreads * b, i = at < p.s.rank ? at : p.s.rank - 1;
+        x[b] = to_float(src[i]);
+        w[b] = p.kv_norm[i];
+    }
     float ss = 0.f;
-    for (int i = threadIdx.x; i < p.s.rank; i += kLatThreads) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if ((int)threadIdx.x + kLatThreads * b < p.s.rank) ss = fmaf(x[b], x[b], ss);
+    for (int i = threadIdx.x + kLatThreads * NB; i < p.s.rank; i += kLatThreads) {
         const float v = to_float(src[i]);
         ss = fmaf(v, v, ss);
     }
     ss = wave_reduce<false>(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.s.true_rank + p.eps);
-    for (int i = threadIdx.x; i < p.s.rank; i += kLatThreads) dst[i] = from_float<T>(to_float(src[i]) * rstd * p.kv_norm[i]);
     for (int i = threadIdx.x; i < p.s.rot / 2; i += kLatThreads) {
         T *d = dst + p.s.rank + 2 * i;
         if (i < p.s.rot_pairs) rotate_pair(src + p.s.rank + 2 * i, d, p.lut + ((size_t)position * p.s.rot_pairs + i) * 2);
         else d[0] = d[1] = from_float<T>(0.f);
     }
+    __syncthreads();
+    const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.s.true_rank + p.eps);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if (const int i = (int)threadIdx.x + kLatThreads * b; i < p.s.rank) dst[i] = from_float<T>(x[b] * rstd * w[b]);
+    for (int i = threadIdx.x + kLatThreads * NB; i < p.s.rank; i += kLatThreads) dst[i] = from_float<T>(to_float(src[i]) * rstd * p.kv_norm[i]);
 }
 
 // one workgroup per token
@@ -102,22 +117,30 @@ __global__ void __launch_bounds__(kLatThreads) latent_absorb_kernel(const Latent
     T *out = qa + ((size_t)m * p.s.heads + h) * lq;
     const int col = r0 + 8 * (tid & 15), dg = tid >> 4;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // eight rows of W at a time, the first of them asked for with the query (past the end: the last row and column, not added)
+    constexpr int kRows = 8;
+    const T *w = w_uk + (size_t)h * p.s.dim * p.s.rank + (col < p.s.rank ? col : p.s.rank - 8);
+    Vec8<T> v[kRows];
+    auto request = [&](int d0) {
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) {
+            const int d = d0 + dg + 16 * j;
+            v[j] = load8(w + (size_t)(d < p.s.dim ? d : p.s.dim - 1) * p.s.rank);
+        }
+    };
+    request(0);
     for (int i = tid; i < p.s.dim; i += kLatThreads) qs[i] = to_float(q[i]);
     __syncthreads();
-    if (col < p.s.rank) {
-        const T *w = w_uk + ((size_t)h * p.s.dim + dg) * p.s.rank + col;
-        for (int d = dg; d < p.s.dim; d += 64) {       // dim is a multiple of 32: two or four rows at a time
-            Vec8<T> v[4];
+    for (int d0 = 0; d0 < p.s.dim; d0 += 16 * kRows) {
+        if (d0 > 0) request(d0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = d + 16 * j < p.s.dim ? load8(w + (size_t)(d - dg + 16 * j) * p.s.rank) : zero8<T>();
+        for (int j = 0; j < kRows; ++j) {
+            const int d = d0 + dg + 16 * j;
+            if (d >= p.s.dim) continue;
+            float f[8];
+            unpack8(v[j], f);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float f[8];
-                unpack8(v[j], f);
-                const float x = d + 16 * j < p.s.dim ? qs[d + 16 * j] : 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] = fmaf(x, f[e], acc[e]);
-            }
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(qs[d], f[e], acc[e]);
         }
     }
 #pragma unroll
@@ -331,8 +354,6 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = blockIdx.x / value_blocks, v0 = (blockIdx.x % value_blocks) * kValueRows, m = blockIdx.y;
     const size_t row = (size_t)m * p.s.heads + h;
-    const int total = first_position(p) + p.M, per = keys_per_split(total, nsplit, kb);
-    const int active = (total + per - 1) / per;
     const int rank = p.s.rank;
 
     // the first 512 columns of this wave's value rows are requested before anything is waited for
@@ -340,14 +361,25 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
     Vec8<T> w_first[kRowsPerWave];
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) w_first[i] = 8 * lane < rank ? load8(w_row + (size_t)i * rank + 8 * lane) : zero8<T>();
+    // ... and so are the gate, every split's maximum and sum and the first 512 columns of up to 64 splits, whether the position uses them or not
+    const int quarter = tid >> 7, col = 4 * (tid & 127);
+    constexpr int BATCH = 16;
+    floatx4 ahead[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+        const int i = quarter + 4 * j;
+        ahead[j] = *reinterpret_cast<const floatx4 *>(part_o + (row * nsplit + (i < nsplit ? i : 0)) * rank + (col < rank ? col : 0));
+    }
+    const float *ml = part_ml + (row * nsplit + (tid < nsplit ? tid : 0)) * 2;
+    const float ml_m = ml[0], ml_l = ml[1];
+    const int value = h * p.s.vdim + v0 + kRowsPerWave * wave + (lane < kRowsPerWave ? lane : 0);
+    const float gate = to_float(p.proj[(size_t)m * p.ld + p.gate_off + value]);
     // factors of the splits in the log2 domain; the sink is one more term of the denominator
     const float snk = sink[h] * 1.4426950408889634f;
+    const int total = first_position(p) + p.M, per = keys_per_split(total, nsplit, kb);
+    const int active = (total + per - 1) / per;
     float ms = kAttnNegBig, ls = 0.f;
-    if (tid < active) {
-        const float *ml = part_ml + (row * nsplit + tid) * 2;
-        ms = ml[0];
-        ls = ml[1];
-    }
+    if (tid < active) ms = ml_m, ls = ml_l;
     float top = wave_reduce<true>(ms);
     if (lane == 0) red[wave] = top;
     __syncthreads();
@@ -364,15 +396,18 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
     if (tid < kMaxSplits) f[tid] = fac / den;
     __syncthreads();
     // merged latent: a thread adds every fourth split of four columns, the quarters meet in LDS
-    const int quarter = tid >> 7, col = 4 * (tid & 127);
     float *piece = merged + (rank + 511) / 512 * 512;
-    constexpr int BATCH = 16;
     for (int r0 = 0; r0 < rank; r0 += 512) {
         const int r = r0 + col;
         floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
         if (r < rank) {
             const float *src = part_o + row * nsplit * rank + r;
-            for (int i = quarter; i < active; i += 4 * BATCH) {
+            if (r0 == 0) {
+#pragma unroll
+                for (int j = 0; j < BATCH; ++j)
+                    if (quarter + 4 * j < active) s += ahead[j] * f[quarter + 4 * j];
+            }
+            for (int i = quarter + (r0 == 0 ? 4 * BATCH : 0); i < active; i += 4 * BATCH) {
                 floatx4 v[BATCH];
 #pragma unroll
                 for (int j = 0; j < BATCH; ++j) v[j] = *reinterpret_cast<const floatx4 *>(src + (size_t)(i + 4 * j < active ? i + 4 * j : i) * rank);
@@ -402,11 +437,7 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
         acc = wave_reduce<false>(acc);
         mine = lane == i ? acc : mine;
     }
-    if (lane < kRowsPerWave) {
-        const int v = h * p.s.vdim + v0 + kRowsPerWave * wave + lane;
-        const float gate = to_float(p.proj[(size_t)m * p.ld + p.gate_off + v]);
-        out[(size_t)m * ldo + v] = from_float<T>(mine * sigmoid_f32(gate));
-    }
+    if (lane < kRowsPerWave) out[(size_t)m * ldo + value] = from_float<T>(mine * sigmoid_f32(gate));
 }
 
 template <class T>

@@ -1,6 +1,9 @@
 // The steps around attention and recurrences as device functions of one workgroup each, so that steps of one token that do not
 // wait for each other can share a launch (mixer_steps.hip), besides having launches of their own (head_attention.hip,
 // linear_attention.hip).
+//
+// What bounds them at one token: launch and round trips to memory, one after the other.  So everything is asked for before the first
+// wait, also where the position (on the device) will say that it does not count, and kept in registers from the sum of a norm to its use.
 #pragma once
 
 #include "dense.h"
@@ -32,27 +35,32 @@ __device__ __forceinline__ void head_prepare_step(const HeadShape &s, const Head
     const int g = is_q ? unit / group : is_v ? unit - H - G : unit - H;
     T *row = cache + ((size_t)g * s.ring + position % s.ring) * row_len;
     T *dst = is_q ? q + (((size_t)g * M + m) * group + unit % group) * s.dim : is_v ? row + s.dim : row;
+    const float *w = is_q ? rows.q_norm : rows.k_norm;
+    // (a vector of up to 512 elements is one turn; the first turn's operands serve both passes)
+    const int i0 = 8 * lane < n ? 8 * lane : n - 8;
+    const Vec8<T> x0 = load8(src + i0);
+    const Vec8<float> w0 = load8(w + (is_v ? 0 : i0));
     float rstd = 1.f;
     if (!is_v) {
         float ss = 0.f;
         for (int i = 8 * lane; i < n; i += 8 * lanes) {
             float v[8];
-            unpack8(load8(src + i), v);
+            unpack8(i == 8 * lane ? x0 : load8(src + i), v);
 #pragma unroll
             for (int j = 0; j < 8; ++j) ss = fmaf(v[j], v[j], ss);
         }
         rstd = 1.0f / sqrtf(group_sum(ss, lanes) / (float)s.true_dim + rows.eps);
     }
-    const float *w = is_q ? rows.q_norm : rows.k_norm;
     for (int i = 8 * lane; i < n; i += 8 * lanes) {
-        const Vec8<T> x = load8(src + i);
+        const bool first = i == 8 * lane;
+        const Vec8<T> x = first ? x0 : load8(src + i);
         if (is_v) {
             store8(dst + i, x);
             continue;
         }
         float v[8], f[8];
         unpack8(x, v);
-        unpack8(load8(w + i), f);
+        unpack8(first ? w0 : load8(w + i), f);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] *= rstd * f[j];
         store8(dst + i, pack8<T>(v));
@@ -68,13 +76,21 @@ __device__ __forceinline__ void head_merge_step(const HeadShape &s, int M, const
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int group = s.heads / s.kv_heads;
     const size_t row = ((size_t)(h / group) * M + m) * group + h % group;
+    // The first splits of the first columns and every split's maximum and sum, also of splits that the position leaves unused.
+    constexpr int kAhead = 4;
+    const int width0 = s.vdim / 4 < kStepThreads ? s.vdim / 4 : kStepThreads, ways0 = kStepThreads / width0;
+    floatx4 ahead[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+        const int i = tid / width0 + j * ways0;
+        ahead[j] = *reinterpret_cast<const floatx4 *>(part_o + (row * nsplit + (i < nsplit ? i : 0)) * s.vdim + 4 * (tid % width0));
+    }
+    const float *ml = part_ml + (row * nsplit + (tid < nsplit ? tid : 0)) * 2;
+    const float ml_m = ml[0], ml_l = ml[1];
     const int pos0 = pos_dev ? pos_dev[0] : pos, n = pos0 + M - first_block_key(pos0, s.window, kb);
     const int per = keys_per_split(n, nsplit, kb), active = (n + per - 1) / per;
     float ms = kAttnNegBig, ls = 0.f;
-    if (tid < active) {
-        ms = part_ml[(row * nsplit + tid) * 2];
-        ls = part_ml[(row * nsplit + tid) * 2 + 1];
-    }
+    if (tid < active) ms = ml_m, ls = ml_l;
     float top = wave_reduce<true>(ms);
     if (lane == 0) red[wave] = top;
     __syncthreads();
@@ -90,8 +106,15 @@ __device__ __forceinline__ void head_merge_step(const HeadShape &s, int M, const
         const int width = (s.vdim - c0) / 4 < kStepThreads ? (s.vdim - c0) / 4 : kStepThreads;   // four-column pieces of this pass
         const int ways = kStepThreads / width, way = tid / width, col = c0 + 4 * (tid % width);
         floatx4 a = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (way < ways)
-            for (int i = way; i < active; i += ways) a += *reinterpret_cast<const floatx4 *>(part_o + (row * nsplit + i) * s.vdim + col) * f[i];
+        if (way < ways) {
+            int i = way;
+            if (c0 == 0) {
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j, i += ways)
+                    if (i < active) a += ahead[j] * f[i];
+            }
+            for (; i < active; i += ways) a += *reinterpret_cast<const floatx4 *>(part_o + (row * nsplit + i) * s.vdim + col) * f[i];
+        }
         part[tid] = a;
         __syncthreads();
         if (way == 0) {
@@ -104,6 +127,34 @@ __device__ __forceinline__ void head_merge_step(const HeadShape &s, int M, const
 }
 
 constexpr int kConvTokens = 4;   // tokens per thread
+
+// The convolution of one token at eight channels: up to four taps at a time.
+template <class T>
+__device__ __forceinline__ void one_token_conv(const ConvArgs &c, const T *proj, T *history, int ch, int C, int pos0, float (&acc)[8]) {
+    constexpr int kTaps = 4;
+    const Vec8<T> mine = load8(proj + ch);
+    for (int j0 = 0; j0 < c.taps; j0 += kTaps) {
+        Vec8<float> w[kTaps];
+        Vec8<T> x[kTaps];
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t) {
+            const int j = j0 + t < c.taps ? j0 + t : c.taps - 1, at = pos0 + j - (c.taps - 1);   // the tap's position; the last tap's is this token's
+            w[t] = load8(c.w + (size_t)j * C + ch);
+            x[t] = load8(history + (size_t)(at >= 0 ? at % c.taps : 0) * C + ch);
+        }
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t) {
+            const int j = j0 + t;
+            if (j >= c.taps || pos0 + j - (c.taps - 1) < 0) continue;
+            float f[8], v[8];
+            unpack8(w[t], f);
+            unpack8(j == c.taps - 1 ? mine : x[t], v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(f[e], v[e], acc[e]);
+        }
+    }
+    store8(history + (size_t)(pos0 % c.taps) * C + ch, mine);   // (nobody else reads these channels; the slot's old row is one too old for any tap)
+}
 
 // Vectors (q and k heads, then v heads) by groups of `lanes` lanes, eight channels per lane at a time; tokens m0 .. m0 + kConvTokens - 1.
 // Rows in front of the portion come from the history, a ring of `taps` rows by position.
@@ -124,7 +175,9 @@ __device__ __forceinline__ void short_conv_step(const ConvArgs &c, const T *proj
         for (int t = 0; t < kConvTokens; ++t)
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[t][e] = 0.f;
-        if (inside) {
+        if (c.M == 1) {
+            one_token_conv<T>(c, proj, history, ch, C, pos0, acc[0]);
+        } else if (inside) {
             for (int j = 0; j < c.taps; ++j) {
                 const T *row = proj + (size_t)(m0 + j - (c.taps - 1)) * c.ld + ch;
                 float w[8];
@@ -166,7 +219,6 @@ __device__ __forceinline__ void short_conv_step(const ConvArgs &c, const T *proj
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss[t] = fmaf(acc[t][e], acc[t][e], ss[t]);
         }
-        if (c.M == 1) store8(history + (size_t)(pos0 % c.taps) * C + ch, load8(proj + ch));   // (nobody else reads these channels, nor this slot)
     }
     if (is_v) return;
 #pragma unroll
@@ -188,7 +240,7 @@ __device__ __forceinline__ void recurrence_step(const LinearArgs &a, float *o, i
     float *st = a.state + ((size_t)h * a.vdim + col) * a.dim + l4;
     floatx4 s[ND];
 #pragma unroll
-    for (int c = 0; c < ND; ++c) s[c] = pos0 > 0 ? *reinterpret_cast<const floatx4 *>(st + 64 * c) : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < ND; ++c) s[c] = *reinterpret_cast<const floatx4 *>(st + 64 * c);
 
     float ea = 0.f, g1 = 1.f;
     floatx4 bias[ND];
@@ -220,6 +272,10 @@ __device__ __forceinline__ void recurrence_step(const LinearArgs &a, float *o, i
     };
     Row cur;
     fetch(0, cur);
+    if (pos0 == 0) {   // what was read does not count: a sequence begins
+#pragma unroll
+        for (int c = 0; c < ND; ++c) s[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
     for (int m = 0; m < a.M; ++m) {
         Row next;
         fetch(m + 1 < a.M ? m + 1 : m, next);
@@ -253,27 +309,48 @@ __device__ __forceinline__ void recurrence_step(const LinearArgs &a, float *o, i
     for (int c = 0; c < ND; ++c) *reinterpret_cast<floatx4 *>(st + 64 * c) = s[c];
 }
 
-// One long group, token m.  red: 4 floats of LDS.
+// One long group, token m; up to 2048 columns stay in registers.  red: 4 floats of LDS.
 template <class T>
 __device__ __forceinline__ void gated_norm_row_step(const GatedNorm &g, const T *gate, T *out, size_t m, float *red) {
+    constexpr int NB = 2, kStep = 4 * kStepThreads;
     const float *o = g.o + m * g.cols;
-    float ss = 0.f;
-    for (int i = 4 * threadIdx.x; i < g.cols; i += 4 * kStepThreads) {
-        const floatx4 v = *reinterpret_cast<const floatx4 *>(o + i);
+    floatx4 v[NB], w[NB];
+    float z[NB][4];
+    auto load = [&](int q) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
+        for (int b = 0; b < NB; ++b) {
+            const int at = 4 * (int)threadIdx.x + (q * NB + b) * kStep, i = at < g.cols ? at : g.cols - 4;
+            v[b] = *reinterpret_cast<const floatx4 *>(o + i);
+            w[b] = *reinterpret_cast<const floatx4 *>(g.w + i);
+            load4(gate + m * g.ld_gate + i, z[b]);
+        }
+    };
+    const int batches = (g.cols + NB * kStep - 1) / (NB * kStep);
+    load(0);
+    float ss = 0.f;
+    for (int q = 0; q < batches; ++q) {
+        if (q > 0) load(q);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            if (4 * (int)threadIdx.x + (q * NB + b) * kStep < g.cols) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ss = fmaf(v[b][j], v[b][j], ss);
+            }
     }
     ss = wave_reduce<false>(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)g.true_cols + g.eps);
-    for (int i = 4 * threadIdx.x; i < g.cols; i += 4 * kStepThreads) {
-        const floatx4 v = *reinterpret_cast<const floatx4 *>(o + i), w = *reinterpret_cast<const floatx4 *>(g.w + i);
-        float z[4];
-        load4(gate + m * g.ld_gate + i, z);
+    for (int q = 0; q < batches; ++q) {
+        if (batches > 1) load(q);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) z[j] = v[j] * rstd * w[j] * sigmoid_of<T>(z[j]);
-        store4(out + m * g.ld_out + i, z[0], z[1], z[2], z[3]);
+        for (int b = 0; b < NB; ++b) {
+            const int i = 4 * (int)threadIdx.x + (q * NB + b) * kStep;
+            if (i >= g.cols) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) z[b][j] = v[b][j] * rstd * w[b][j] * sigmoid_of<T>(z[b][j]);
+            store4(out + m * g.ld_out + i, z[b][0], z[b][1], z[b][2], z[b][3]);
+        }
     }
 }
 
