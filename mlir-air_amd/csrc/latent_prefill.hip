@@ -11,8 +11,9 @@
 // The D layout gives a lane keys 4 g .. + 3 of each 16-key block; the k slots of the second product are defined as exactly
 // those keys, so P never moves between lanes.  Four waves of QB blocks of 16 queries each share the K and V rows going through
 // LDS; the next block of keys travels global -> registers while one is multiplied.  With SETS = 2 a second set of four waves
-// takes the odd key blocks for the same queries, and the two partial results are merged through LDS at the end: the longest
-// rows take half as long, and two waves share a SIMD.  The grid puts the longest rows first.  The running maximum may lag the true one by 2^8 (as in prefill_attention.hip), so
+// takes the odd key blocks for the same queries, and the two partial results are merged through LDS at the end, a block of queries by
+// each set: the longest rows take half as long, and two waves share a SIMD.  (2048 tokens, 16 heads of 128 + 64 / 128: merge, gates and stores by one
+// set 7.8 of 65 us, gates by an exponential and a division each and asked for one by one; now 3.7 of 62.)  The grid puts the longest rows first.  The running maximum may lag the true one by 2^8 (as in prefill_attention.hip), so
 // rescaling is rare; the row sum is a product with a row of ones.
 //
 // Head sizes that are common have kernels of their own (EXACT: everything unrolled); any other size runs on the next
@@ -44,6 +45,12 @@ struct PrefillArgs {
     int group, window, ring;                // query heads per key / value head
     float out_scale;
 };
+
+// v sigmoid(z); a z that is not a number stays one (told by its bits: this file is compiled without NaNs)
+__device__ __forceinline__ float gated(float v, float z) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, z);
+    return __builtin_bit_cast(float, (bits & 0x7FFFFFFFu) > 0x7F800000u ? bits : __builtin_bit_cast(uint32_t, gated_f32(v, z)));
+}
 
 template <class T>
 __device__ __forceinline__ Vec8<T> ones8();
@@ -236,25 +243,23 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
         __syncthreads();
     }
 
-    if constexpr (SETS == 2) {   // the same wave and lane of the other set holds the same queries and output elements
-        constexpr int NREG = QB * (4 * NV + 2);
-        float *xch = reinterpret_cast<float *>(pf_lds) + wave * NREG * 64 + lane;
-        if (set == 1) {
+    // The same wave and lane of the other set holds the same queries and output elements.  With two blocks of queries each set finishes one
+    // of them, so that both work on the gates.
+    constexpr bool kShare = SETS == 2 && QB == 2;
+    if constexpr (SETS == 2) {
+        constexpr int NREG = (kShare ? 1 : QB) * (4 * NV + 2);
+        float *mine = reinterpret_cast<float *>(pf_lds) + (wave + (kShare ? 4 * set : 0)) * NREG * 64 + lane;   // what this wave takes
+        float *other = reinterpret_cast<float *>(pf_lds) + (wave + (kShare ? 4 * (set ^ 1) : 0)) * NREG * 64 + lane;
+        auto give = [&](int b, float *to) {
 #pragma unroll
-            for (int b = 0; b < QB; ++b) {
+            for (int d = 0; d < NV; ++d)
 #pragma unroll
-                for (int d = 0; d < NV; ++d)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) xch[((b * NV + d) * 4 + r) * 64] = o[b][d][r];
-                xch[(4 * QB * NV + 2 * b) * 64] = m[b];
-                xch[(4 * QB * NV + 2 * b + 1) * 64] = l[b][0];
-            }
-        }
-        __syncthreads();
-        if (set == 1) return;
-#pragma unroll
-        for (int b = 0; b < QB; ++b) {
-            const float m1 = xch[(4 * QB * NV + 2 * b) * 64], l1 = xch[(4 * QB * NV + 2 * b + 1) * 64];
+                for (int r = 0; r < 4; ++r) to[(d * 4 + r) * 64] = o[b][d][r];
+            to[4 * NV * 64] = m[b];
+            to[(4 * NV + 1) * 64] = l[b][0];
+        };
+        auto take = [&](int b, const float *from) {
+            const float m1 = from[4 * NV * 64], l1 = from[(4 * NV + 1) * 64];
             const float mm = fmaxf(m[b], m1);
             const float f0 = __builtin_amdgcn_exp2f((m[b] - mm) * p.scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mm) * p.scale_log2);
             m[b] = mm;
@@ -262,28 +267,58 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
 #pragma unroll
             for (int d = 0; d < NV; ++d)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) o[b][d][r] = o[b][d][r] * f0 + xch[((b * NV + d) * 4 + r) * 64] * f1;
+                for (int r = 0; r < 4; ++r) o[b][d][r] = o[b][d][r] * f0 + from[(d * 4 + r) * 64] * f1;
+        };
+        if constexpr (kShare) {
+            if (set == 0) give(1, other);
+            else give(0, other);
+            __syncthreads();
+            if (set == 0) take(0, mine);
+            else take(1, mine);
+        } else {
+            if (set == 1) {
+#pragma unroll
+                for (int b = 0; b < QB; ++b) give(b, other + b * (4 * NV + 2) * 64);
+            }
+            __syncthreads();
+            if (set == 1) return;
+#pragma unroll
+            for (int b = 0; b < QB; ++b) take(b, mine + b * (4 * NV + 2) * 64);
         }
     }
 
     const float snk = WINDOW ? 0.f : p.sink[head] * 1.4426950408889634f;
-#pragma unroll
-    for (int b = 0; b < QB; ++b) {
+    auto finish = [&](int b) {
         const int qi = q0 + 16 * b + ql;
-        if (qi >= p.M) continue;
+        if (qi >= p.M) return;
         const float inv = WINDOW ? p.out_scale / l[b][0] : 1.0f / (l[b][0] + exp2f(snk - m[b] * p.scale_log2));
         const int col = head * p.vdim + vcol0 + 4 * g;
         const T *gate = p.q + (size_t)qi * p.ldq + p.gate_off + col;
         T *dst = p.out + (size_t)qi * p.ldo + col;
+        float z[WINDOW ? 1 : NV][4];
+        if constexpr (!WINDOW) {   // all of them on their way before the first is used
+#pragma unroll
+            for (int d = 0; d < NV; ++d)
+                if (EXACT || d < nv) load4(gate + 16 * d, z[d]);
+        }
 #pragma unroll
         for (int d = 0; d < NV; ++d)
             if (EXACT || d < nv) {
-                float z[4];
-                if (!WINDOW) load4(gate + 16 * d, z);
+                float v[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) z[r] = o[b][d][r] * inv * (WINDOW ? 1.0f : sigmoid_f32(z[r]));
-                store4(dst + 16 * d, z[0], z[1], z[2], z[3]);
+                for (int r = 0; r < 4; ++r) {
+                    v[r] = o[b][d][r] * inv;
+                    if constexpr (!WINDOW) v[r] = sizeof(T) == 2 ? gated(v[r], z[d][r]) : v[r] * sigmoid_f32(z[d][r]);
+                }
+                store4(dst + 16 * d, v[0], v[1], v[2], v[3]);
             }
+    };
+    if constexpr (kShare) {
+        if (set == 0) finish(0);
+        else finish(1);
+    } else {
+#pragma unroll
+        for (int b = 0; b < QB; ++b) finish(b);
     }
 }
 
