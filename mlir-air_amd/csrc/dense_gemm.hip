@@ -264,8 +264,10 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
 // A wave's NT x MT tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
+// GROUPED, second product: out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
 template <int NT, int MT, int EPI, bool GROUPED>
-__device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first) {
+__device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first,
+                                           const int (&out_rows)[2] = {0, 0}) {
     typedef typename std::conditional<EPI == kOutF32, float, bf16>::type Out;
     constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
     constexpr int kCols = 16 * NT / (kPair ? 2 : 1), kPiece = 16 / (int)sizeof(Out), kPitch = kCols + kPiece;
@@ -292,10 +294,10 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
 #pragma unroll
         for (int t = lane; t < kPieces; t += 64) {
             const int row = t / (kCols / kPiece), col = t % (kCols / kPiece) * kPiece, m = m_first + 16 * i + row;
-            if (m >= m_end || n_out + col >= n_end) continue;
             size_t to = m;
-            if constexpr (GROUPED)
-                if (p.gather == 0) to = p.order[m];
+            if constexpr (GROUPED && !kPair)
+                if (p.gather == 0) to = __shfl(out_rows[i / 4], 16 * (i % 4) + row);
+            if (m >= m_end || n_out + col >= n_end) continue;
             const long part = EPI == kOutF32 ? blockIdx.y * p.slice_stride : 0;
             *reinterpret_cast<u32x4 *>(static_cast<Out *>(p.out) + part + to * p.ldo + n_out + col) = *reinterpret_cast<const u32x4 *>(rows + row * kPitch + col);
         }
@@ -530,23 +532,24 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
         }
     };
     int fill_a = 0, fill_w = 0;   // stages that the next K-step's copies go to
-    // copy i of a K-step, A's first; behind the last one of each the source moves on (from the last K-step to the first)
-    int next_a = first, next_w = first;
+    // copy i of a K-step, A's first; behind the last one of each the source moves on, from the last K-step to the first, but not past all of
+    // them (what is copied then, into buffers that nobody reads, comes from L2)
+    int next_a = first, next_w = first, left_a = steps - 1, left_w = steps - 1;
     auto step_copy = [&](int i) {
         if (i < CA) {
             copy((gptr)(row_a[i < CA ? i : 0] + from_a), fill_a + 1024 * CA * wave, i);
             if (i == CA - 1) {
-                const bool wrap = next_a + 1 == steps;
+                const bool more = left_a-- > 0, wrap = next_a + 1 == steps;
                 next_a = wrap ? 0 : next_a + 1;
-                from_a += wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
+                from_a += !more ? 0 : wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
                 fill_a = fill_a == (RA - 1) * kSideA ? 0 : fill_a + kSideA;
             }
         } else {
             copy(base_w + off_w[i < CA ? 0 : i - CA], RA * kSideA + fill_w + 1024 * CW * wave, i - CA);
             if (i == V - 1) {
-                const bool wrap = next_w + 1 == steps;
+                const bool more = left_w-- > 0, wrap = next_w + 1 == steps;
                 next_w = wrap ? 0 : next_w + 1;
-                base_w += wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
+                base_w += !more ? 0 : wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
                 fill_w = fill_w == (RW - 1) * kSideW ? 0 : fill_w + kSideW;
             }
         }
@@ -561,6 +564,15 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
         at_w[ks] = o + RA * kSideA;
     }
     auto read = [&](uint32_t at, int i) { return *reinterpret_cast<const bf16x8 *>(lds + at + i * 16 * kRowBytes); };
+
+    // where the second product's rows go: asked for here, because a store that has to ask waits once per 16 rows (down of 64 experts of
+    // 1024 x 2048, 16384 entries: 109 -> 101 us, with nothing read past the last K-step)
+    int out_rows[2] = {0, 0};
+    if (EPI == kOutElem && p.gather == 0) {
+        const int own = m0 + wave * 16 * MT;
+        out_rows[0] = p.order[own + lane < m_end ? own + lane : m_end - 1];
+        if (MT > 4) out_rows[1] = p.order[own + 64 + lane < m_end ? own + 64 + lane : m_end - 1];
+    }
 
     floatx4 acc[8][MT];
 #pragma unroll
@@ -627,7 +639,7 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
 #pragma unroll
     for (int i = 0; i < MT; ++i)
         asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]), "+a"(acc[4][i]), "+a"(acc[5][i]), "+a"(acc[6][i]), "+a"(acc[7][i]));
-    store_rows<8, MT, EPI, true>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0);
+    store_rows<8, MT, EPI, true>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0, out_rows);
 }
 
 template <int EPI, bool FEW>
