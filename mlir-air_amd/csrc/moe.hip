@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(kMoeThreads, 2) moe_down_gemv_kernel(const Moe
             const int k = chunk(min(i0 + u, items - 1), slot, in);
             const int expert = __builtin_amdgcn_readlane(id, slot);
             const float x = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), slot));
-            wt[u] = i0 + u < items ? x : 0.f;
+            wt[u] = x;
             w[u] = stream8(p.w + ((size_t)expert * p.N + row) * p.ff + k);
         }
     };
@@ -305,9 +305,10 @@ __global__ void __launch_bounds__(kMoeThreads, 2) moe_down_gemv_kernel(const Moe
     for (int i0 = 0; n < p.N;) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            if (i0 + u >= items) break;   // uniform; nothing is added for what is not there, not even 0 times an infinity
             int slot;
             bool in;
-            const int i = min(i0 + u, items - 1);
+            const int i = i0 + u;
             chunk(i, slot, in);
             const Vec8<T> row = in ? w[u] : zero8<T>();
             acc = fmaf(wt[u], dot8(row, load8(hs + i * kMoePiece + 8 * lane), 0.f), acc);

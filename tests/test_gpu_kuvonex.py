@@ -202,6 +202,20 @@ def test_mixture(dense, dtype, M, experts, top, groups, keep, K, ff, N):
     close(got, want, dtype, bf16=3e-2)
 
 
+@pytest.mark.parametrize("ff", [64, 512, 576])
+def test_one_token_mixture_that_overflows(dense, ff):
+    """An expert's activation beyond the element type stays an infinity: pieces that a row does not have add nothing, not 0 times it."""
+    say("overflow", ff)
+    experts, top, K, N = 4, 3, 64, 64
+    h = torch.full((K,), 1.0, dtype=BF16, device="cuda")
+    gu = torch.zeros((experts, 2 * ff, K), dtype=BF16, device="cuda")
+    gu[:, -1], gu[:, -17] = 1e20, 1e20                          # gate and up row of the last column of ff: 6e21 each
+    down = torch.full((experts, N, ff), 0.5, dtype=BF16, device="cuda")
+    logits = torch.zeros((16,), device="cuda")
+    y = dense.moe_gemv(h, logits, dense.RouterSpec(torch.zeros((experts,), device="cuda"), experts, top, 1, 1), gu, down)
+    assert bool((y == float("inf")).all())
+
+
 # ---- latent attention -----------------------------------------------------------------------------------------------------
 LATENT_SIZES = [   # heads, dim, rot, vdim, rank
     (3, 24, 8, 40, 56), (6, 64, 32, 64, 192), (5, 16, 6, 24, 40), (16, 128, 64, 128, 512), (2, 192, 64, 256, 320), (1, 300, 20, 288, 1000), (17, 32, 32, 32, 64),
