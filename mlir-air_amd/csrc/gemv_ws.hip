@@ -119,8 +119,8 @@ __global__ void __launch_bounds__(kMaxWaves * 64) gemv_ws_kernel(const uint16_t 
     for (int m = 0; m < NMAT; ++m) yv[m] = 0.f;
 
     // The residual is added last and asked for first: behind the sums it is a round trip of its own (O product of 2048 x 2048, 4.0 -> 3.8 us, down of 8192 x 2048 5.0 -> 4.7).
-    // Without one the output's old value is read, and not used.
-    const uint32_t add = (residual ? residual : y)[tile * kWsTileCols + (threadIdx.x & (kWsTileCols - 1))];
+    // Without one some x is read, and not used.
+    const uint32_t add = (residual ? residual + tile * kWsTileCols : x)[threadIdx.x & (kWsTileCols - 1)];
 
     // RMS: the partial sums are requested first and consumed only after the first task's loads have been requested
     // (below), so that their round trip overlaps with the weights' instead of standing in front of them (gate / up
