@@ -7,12 +7,22 @@
 //   (1 + diag(beta) A) U = diag(beta) (V - (k e^G) S)       u of the delta rule; U = V without it
 //   O = (q e^G) S + B U,    S' = e^(G_last) S + (k e^(G_last - G))^T U
 //
-// so that everything but the products with S can be done for all chunks at once:
+// With U = V (one decay per head) S' needs nothing but a product of the chunk's own and a multiple of S:
 //
-//   linear_chunk / delta_chunk   one workgroup per head and chunk: q e^G, (k e^(G_last - G))^T, B, e^(G_last), and U as
-//                                U0 - W S: U0 = V, or U0 = (1 + diag(beta) A)^-1 diag(beta) V and W the same of k e^G
-//   chunk_scan                   one workgroup per head and 16 value columns goes through the chunks: S stays in registers (and
-//                                in LDS as an operand)
+//   linear_state    one workgroup per head and chunk: (k e^(G_last - G))^T V
+//   linear_scan     every element of S on its own: the S in front of every chunk in place of its product
+//   linear_output   one workgroup per head and chunk: O
+//
+// With the delta rule everything but the products with S can be done for all chunks at once:
+//
+//   delta_chunk     one workgroup per head and chunk: q e^G, (k e^(G_last - G))^T, B, e^(G_last), and U as U0 - W S:
+//                   U0 = (1 + diag(beta) A)^-1 diag(beta) V and W the same of k e^G
+//   delta_scan      one workgroup per head and 16 value columns goes through the chunks: S stays in registers (and in LDS as an operand)
+//
+// What bounds them: fp32 products (a CU does 256 flops a clock), S and the chunks' operands on their way through memory, and the chain of a scan over the
+// chunks.  2048 tokens, 16 heads of 128 / 128: one decay per head 17 + 14 + 25 us (89 with the scan of the delta rule, whose 128 workgroups do all
+// of the products one chunk after the other), the delta rule 40 + 89 (its outputs in a launch of their own, S and U left in memory for it: 61 + 25 us instead of the
+// 89, and at 300 tokens 12 + 11 instead of 16: not taken).
 //
 // All of it is 32-bit, products included (fp32 MFMA).  No exponent is ever positive: the 16 x 16 blocks on the diagonal of A
 // and B weigh every pair of tokens on its own, the blocks under it go through the decay up to the border of the row block,
@@ -27,19 +37,21 @@ namespace {
 constexpr int kC = 64, kThreads = 256;
 constexpr float kLog2E = 1.4426950408889634f;
 
-// Work of one head and chunk, in floats.  The matrices lie in the order in which the scan's waves read them as first operands, a
-// kilobyte of neighbouring lanes per load: [16 rows][32 columns][half of 8 columns][lane][4]; u as it is added to a product:
+// Work of one head and chunk of the delta rule, in floats (without it: S alone).  The matrices lie in the order in which waves read them as operands,
+// a kilobyte of neighbouring lanes per load: [16 rows][32 columns][half of 8 columns][lane][4]; u as it is added to a product:
 // [16 columns][16 tokens][lane][4 tokens].
 struct ChunkLayout {
-    int dim, vdim, delta;
+    int dim, vdim;
     __host__ __device__ size_t q() const { return 0; }                                   // [kC][dim]
     __host__ __device__ size_t k() const { return (size_t)kC * dim; }                    // [dim][kC]
     __host__ __device__ size_t b() const { return k() + (size_t)kC * dim; }              // [kC][kC]
     __host__ __device__ size_t u() const { return b() + kC * kC; }                       // [kC][vdim]
     __host__ __device__ size_t e() const { return u() + (size_t)kC * vdim; }             // [dim]
     __host__ __device__ size_t w() const { return e() + dim; }                           // [kC][dim]
-    __host__ __device__ size_t size() const { return w() + (delta ? (size_t)kC * dim : 0); }
+    __host__ __device__ size_t size() const { return w() + (size_t)kC * dim; }
 };
+// floats of work of a head and chunk
+size_t chunk_work(const LinearArgs &a) { return a.z ? ChunkLayout{a.dim, a.vdim}.size() : (size_t)a.vdim * a.dim; }
 
 // Place of elements (row, column .. column + 3) of a matrix with `steps` times 32 columns.
 __device__ __forceinline__ int place_of(int row, int col, int steps) {
@@ -60,68 +72,218 @@ __device__ __forceinline__ void clear_upper(float *b, int lane) {
     *reinterpret_cast<floatx4 *>(b + place_of(32 + row, 48 + c, 2)) = zero;
 }
 
-// blockIdx.x = chunk, blockIdx.y = head.  One decay per head, u = v.
-template <class T, int ND>
-__global__ void __launch_bounds__(kThreads) linear_chunk_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work) {
-    constexpr int D = 64 * ND, P = D + 4;
+// First operand of a product, in the order of ChunkLayout: 16 rows and 32 columns
+__device__ __forceinline__ Vec8<float> operand(const float *m, int piece, int lane) {
+    const float *x = m + piece * 512 + lane * 4;
+    return Vec8<float>{*reinterpret_cast<const floatx4 *>(x), *reinterpret_cast<const floatx4 *>(x + 256)};
+}
+
+// What a workgroup of the form with one decay per head works on: blockIdx.x = chunk, blockIdx.y = head.
+template <class T>
+struct LinearChunk {
+    const T *q, *k, *v;
+    float ld;
+    int n;   // tokens
+    __device__ __forceinline__ LinearChunk(const LinearArgs &a, const T *q0, const T *k0, const T *v0) {
+        const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC;
+        const int D = a.dim;
+        n = a.M - m0 < kC ? a.M - m0 : kC;
+        ld = a.log2_decay[h];
+        q = q0 + (size_t)m0 * a.ld + (size_t)kh * D;
+        k = k0 + (size_t)m0 * a.ld + (size_t)kh * D;
+        v = v0 + (size_t)m0 * a.ld + (size_t)h * a.vdim;
+    }
+    __device__ __forceinline__ float power(int e) const { return __builtin_amdgcn_exp2f(ld * (float)e); }
+    // second operand: tokens 32 t .. + 31 of 16 columns, zeros behind the end
+    __device__ __forceinline__ Vec8<float> values(const LinearArgs &a, int vt, int t) const {
+        const int lane = threadIdx.x & 63, row = 32 * t + 8 * (lane >> 4);
+        const T *x = v + 16 * vt + (lane & 15);
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = to_float(x[(size_t)(row + e < n ? row + e : n - 1) * a.ld]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = row + e < n ? f[e] : 0.f;
+        return pack8<float>(f);
+    }
+};
+
+// A wave has NV times 16 value columns of all channels; keys, already decayed, through LDS.
+template <class T, int ND, int NV>
+__global__ void __launch_bounds__(kThreads) linear_state_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work) {
+    constexpr int D = 64 * ND, P = D + 4, KS = 2 * ND;
     __shared__ __attribute__((aligned(16))) float ks[kC][P];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ql = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC, n = a.M - m0 < kC ? a.M - m0 : kC;
-    const ChunkLayout lay{D, a.vdim, 0};
-    float *out = work + ((size_t)h * gridDim.x + blockIdx.x) * lay.size();
-    const float ld = a.log2_decay[h];
-    auto power = [&](int e) { return __builtin_amdgcn_exp2f(ld * (float)e); };
-    q += (size_t)m0 * a.ld + (size_t)kh * D;
-    k += (size_t)m0 * a.ld + (size_t)kh * D;
-    v += (size_t)m0 * a.ld + (size_t)h * a.vdim;
-    for (int i = tid; i < kC * D / 8; i += kThreads) {
-        const int r = i / (D / 8), c = 8 * (i % (D / 8));
-        float y[8];
-        unpack8(r < n ? load8(k + (size_t)r * a.ld + c) : zero8<T>(), y);
-        store8(&ks[r][c], pack8<float>(y));
-    }
-    for (int i = tid; i < kC * D / 4; i += kThreads) {
-        int r, c;
-        at_place(i, 2 * ND, r, c);
-        float x[4] = {0.f, 0.f, 0.f, 0.f};
-        if (r < n) load4(q + (size_t)r * a.ld + c, x);
-        const float f = power(r + 1);
-        store4(out + lay.q() + 4 * i, x[0] * f, x[1] * f, x[2] * f, x[3] * f);
-    }
-    for (int i = tid; i < kC * a.vdim / 4; i += kThreads) {
-        const int t = 16 * ((i >> 6) & 3) + 4 * ((i & 63) >> 4), c = 16 * (i >> 8) + (i & 15);
-        float x[4];
+    const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tiles = a.vdim / 16;
+    const LinearChunk<T> c(a, q, k, v);
+    work += ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * a.vdim * D;
+    constexpr int kRows = kC * D / 8 / kThreads;   // pieces of keys of a thread
+    Vec8<T> kr[kRows];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = t + e < n ? to_float(v[(size_t)(t + e) * a.ld + c]) : 0.f;
-        store4(out + lay.u() + 4 * i, x[0], x[1], x[2], x[3]);
+    for (int i = 0; i < kRows; ++i) {
+        const int at = tid + kThreads * i, r = at / (D / 8);
+        kr[i] = load8(c.k + (size_t)(r < c.n ? r : c.n - 1) * a.ld + 8 * (at % (D / 8)));
     }
-    if (tid < D) out[lay.e() + tid] = power(n);
-    // scores: rows of one wave against the blocks up to the diagonal (first operand: k, so that a lane owns one query)
+    Vec8<float> u[NV][2];
+    auto fetch = [&](int vt0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) u[i][t] = c.values(a, vt0 + i < tiles ? vt0 + i : tiles - 1, t);
+    };
+    fetch(wave * NV);
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int at = tid + kThreads * i, r = at / (D / 8);
+        const float f = c.power(c.n - 1 - r);
+        float x[8];
+        unpack8(kr[i], x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = r < c.n ? x[e] * f : 0.f;
+        store8(&ks[r][8 * (at % (D / 8))], pack8<float>(x));
+    }
+    __syncthreads();
+    for (int vt0 = wave * NV; vt0 < tiles;) {
+#pragma unroll 2
+        for (int ct = 0; ct < 4 * ND; ++ct) {
+            Vec8<float> m[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = ks[32 * t + 8 * g + e][16 * ct + ql];
+                m[t] = pack8<float>(x);
+            }
+            floatx4 s[NV];
+#pragma unroll
+            for (int i = 0; i < NV; ++i) s[i] = mma32(m[0], u[i][0], floatx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int i = 0; i < NV; ++i) s[i] = mma32(m[1], u[i][1], s[i]);
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                if (vt0 + i < tiles) *reinterpret_cast<floatx4 *>(work + (vt0 + i) * 16 * D + place_of(ql, 16 * ct + 4 * g, KS)) = s[i];
+        }
+        vt0 += 4 * NV;
+        if (vt0 < tiles) fetch(vt0);
+    }
+}
+
+// Four elements of S to a thread, the products of kAhead chunks on their way.
+constexpr int kAhead = 8;
+template <int ND>
+__global__ void __launch_bounds__(kThreads) linear_scan_kernel(const LinearArgs a, float *work, int chunks, bool first) {
+    constexpr int D = 64 * ND, KS = 2 * ND;
+    const int h = blockIdx.y, i = blockIdx.x * kThreads + threadIdx.x;   // (vdim dim / 4 is a multiple of kThreads)
+    const size_t size = (size_t)a.vdim * D;
+    work += (size_t)h * chunks * size + 4 * i;
+    floatx4 x[kAhead];
+    auto fetch = [&](int slot, int chunk) { x[slot] = *reinterpret_cast<const floatx4 *>(work + (chunk < chunks ? chunk : chunks - 1) * size); };
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) fetch(j, j);
+    int row, col;
+    at_place(i, KS, row, col);
+    float *st = a.state + (size_t)h * size + (size_t)row * D + col;
+    floatx4 s = *reinterpret_cast<const floatx4 *>(st);
+    if (first && (a.pos_dev ? a.pos_dev[0] : a.pos) == 0) s = floatx4{0.f, 0.f, 0.f, 0.f};
+    const float ld = a.log2_decay[h], e = __builtin_amdgcn_exp2f(ld * (float)kC);
+    const float e_last = __builtin_amdgcn_exp2f(ld * (float)(a.M - (chunks - 1) * kC));
+    for (int c0 = 0; c0 < chunks; c0 += kAhead) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            if (c0 + j >= chunks) break;
+            *reinterpret_cast<floatx4 *>(work + (c0 + j) * size) = s;
+            s = s * (c0 + j + 1 < chunks ? e : e_last) + x[j];
+            if (c0 + j + kAhead < chunks) fetch(j, c0 + j + kAhead);
+        }
+    }
+    *reinterpret_cast<floatx4 *>(st) = s;
+}
+
+// q e^G by all, the scores of 16 tokens by each wave, then the outputs.
+template <class T, int ND>
+__global__ void __launch_bounds__(kThreads, 2) linear_output_kernel(const LinearArgs a, const T *q, const T *k, const T *v, const float *work, float *o) {
+    constexpr int D = 64 * ND, KS = 2 * ND;
+    __shared__ __attribute__((aligned(16))) float qf[kC * D], bs[kC * kC];   // q e^G and B, in the order of ChunkLayout
+    const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tiles = a.vdim / 16;
+    const LinearChunk<T> c(a, q, k, v);
+    work += ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * a.vdim * D;
+    o += ((size_t)blockIdx.x * kC * a.heads + blockIdx.y) * a.vdim;
+    auto row_of = [&](const T *x, int r) { return x + (size_t)(r < c.n ? r : c.n - 1) * a.ld; };
+    constexpr int kRows = kC * D / 8 / kThreads;   // pieces of queries of a thread
+    Vec8<T> qr[kRows], qs[KS], ks[KS];
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int at = tid + kThreads * i;
+        qr[i] = load8(row_of(c.q, at / (D / 8)) + 8 * (at % (D / 8)));
+    }
     const int qi = 16 * wave + ql;
-    const T *qr = q + (size_t)(qi < n ? qi : n - 1) * a.ld + 8 * g;
-    for (int bj = 0; bj <= wave; ++bj) {
-        const int kj = 16 * bj + ql;
-        const T *kr = k + (size_t)(kj < n ? kj : n - 1) * a.ld + 8 * g;
-        floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 2 * ND; ++t) s = mma32(load8(kr + 32 * t), load8(qr + 32 * t), s);
+    for (int t = 0; t < KS; ++t) qs[t] = load8(row_of(c.q, qi) + 8 * g + 32 * t);
+    auto fetch_keys = [&](int bj) {
+#pragma unroll
+        for (int t = 0; t < KS; ++t) ks[t] = load8(row_of(c.k, 16 * bj + ql) + 8 * g + 32 * t);
+    };
+    fetch_keys(0);
+    Vec8<float> s[KS], u[2];
+    auto fetch = [&](int vt, Vec8<float> (&s)[KS], Vec8<float> (&u)[2]) {
+#pragma unroll
+        for (int t = 0; t < KS; ++t) s[t] = operand(work, vt * KS + t, lane);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) u[t] = c.values(a, vt, t);
+    };
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int at = tid + kThreads * i, r = at / (D / 8), col = 8 * (at % (D / 8));
+        const float f = c.power(r + 1);
+        float x[8];
+        unpack8(qr[i], x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] *= f;
+        store4(qf + place_of(r, col, KS), x[0], x[1], x[2], x[3]);
+        store4(qf + place_of(r, col + 4, KS), x[4], x[5], x[6], x[7]);
+    }
+    // scores: the blocks up to the diagonal (first operand: k, so that a lane owns one query)
+    for (int bj = 0; bj <= wave; ++bj) {
+        floatx4 x = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < KS; ++t) x = mma32(ks[t], qs[t], x);
+        fetch_keys(bj < wave ? bj + 1 : bj);
         float w[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int j = 16 * bj + 4 * g + r;
-            w[r] = j <= qi && j < n && qi < n ? s[r] * power(qi - j) : 0.f;
+            w[r] = j <= qi && j < c.n && qi < c.n ? x[r] * c.power(qi - j) : 0.f;
         }
-        store4(out + lay.b() + place_of(qi, 16 * bj + 4 * g, 2), w[0], w[1], w[2], w[3]);
+        store4(bs + place_of(qi, 16 * bj + 4 * g, 2), w[0], w[1], w[2], w[3]);
     }
-    if (wave == 0) clear_upper(out + lay.b(), lane);
+    if (wave == 0) clear_upper(bs, lane);
+    fetch(wave < tiles ? wave : tiles - 1, s, u);
     __syncthreads();
-    for (int i = tid; i < D * kC / 4; i += kThreads) {
-        int r, c;
-        at_place(i, 2, c, r);
-        float x[4];
+    for (int vt = wave; vt < tiles; vt += 4) {   // every fourth 16 value columns, the next ones' operands ahead
+        Vec8<float> s1[KS], u1[2];
+        fetch(vt + 4 < tiles ? vt + 4 : vt, s1, u1);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = r + e < n ? ks[r + e][c] * power(n - 1 - r - e) : 0.f;
-        store4(out + lay.k() + 4 * i, x[0], x[1], x[2], x[3]);
+        for (int b = 0; b < 4; ++b) {
+            floatx4 x = floatx4{0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll
+            for (int t = 0; t < KS; t += 2) {
+                x = mma32(operand(qf, b * KS + t, lane), s[t], x);
+                y = mma32(operand(qf, b * KS + t + 1, lane), s[t + 1], y);
+            }
+            x = mma32(operand(bs, b * 2, lane), u[0], x);
+            if (b >= 2) y = mma32(operand(bs, b * 2 + 1, lane), u[1], y);
+            x += y;
+            const int row = 16 * b + 4 * g;
+            float *dst = o + (size_t)row * a.heads * a.vdim + 16 * vt + ql;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (row + r < c.n) dst[(size_t)r * a.heads * a.vdim] = x[r];
+            __builtin_amdgcn_sched_barrier(0);   // (all four turns' operands at once do not fit the registers of half a SIMD)
+        }
+#pragma unroll
+        for (int t = 0; t < KS; ++t) s[t] = s1[t];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) u[t] = u1[t];
     }
 }
 
@@ -154,7 +316,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) delta_chunk_
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC, n = a.M - m0 < kC ? a.M - m0 : kC;
-    const ChunkLayout lay{D, a.vdim, 1};
+    const ChunkLayout lay{D, a.vdim};
     float *out = work + ((size_t)h * gridDim.x + blockIdx.x) * lay.size();
     const float ea = -expf(a.a_log[h]) * kLog2E;
     q += (size_t)m0 * a.ld + (size_t)kh * D;
@@ -385,8 +547,8 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) delta_chunk_
 // A wave requests the operands of the next chunk as soon as it has multiplied those of this one, products with S while those with U
 // are made and the other way round.  (Behind the last chunk that one is fetched again rather than nothing, so that the number of loads
 // in flight is known at every wait.)
-template <int ND, bool DELTA>
-__global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const LinearArgs a, const float *work, int chunks, bool first, float *o) {
+template <int ND>
+__global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const LinearArgs a, const float *work, int chunks, bool first, float *o) {
     constexpr int D = 64 * ND, KS = 2 * ND;
     __shared__ __attribute__((aligned(16))) float ss[2][16][D + 4], us[2][16][kC + 4];
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
@@ -394,12 +556,8 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
     const int tiles = a.vdim / 16, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
     const int h = 8 * (at / tiles) + xcd, v0 = 16 * (at % tiles), tok = 16 * wave;
     if (h >= a.heads) return;
-    const ChunkLayout lay{D, a.vdim, DELTA};
+    const ChunkLayout lay{D, a.vdim};
     work += (size_t)h * chunks * lay.size();
-    auto operand = [&](const float *m, int piece) {
-        const float *x = m + piece * 512 + lane * 4;
-        return Vec8<float>{*reinterpret_cast<const floatx4 *>(x), *reinterpret_cast<const floatx4 *>(x + 256)};
-    };
     const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
     // m S (two chains), and the operands from LDS in registers before the first product: the compiler would fetch them two by two
     auto times_state = [&](const Vec8<float> (&m)[KS], const float (*rows)[D + 4], floatx4 &x, floatx4 &y) {
@@ -423,13 +581,11 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
             s[c] = from_zero ? zero : *reinterpret_cast<const floatx4 *>(st + 16 * (wave + 4 * c));
             *reinterpret_cast<floatx4 *>(&ss[0][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
         }
-        Vec8<float> w[KS], k[ND][2];   // (w: the delta rule only)
+        Vec8<float> w[KS], k[ND][2];
         floatx4 u, e[ND];
         auto fetch_w = [&](const float *p) {
-            if constexpr (DELTA) {
 #pragma unroll
-                for (int t = 0; t < KS; ++t) w[t] = operand(p + lay.w(), wave * KS + t);
-            }
+            for (int t = 0; t < KS; ++t) w[t] = operand(p + lay.w(), wave * KS + t, lane);
             u = *reinterpret_cast<const floatx4 *>(p + lay.u() + ((v0 / 16 * 4 + wave) * 64 + lane) * 4);
 #pragma unroll
             for (int c = 0; c < ND; ++c) e[c] = *reinterpret_cast<const floatx4 *>(p + lay.e() + 16 * (wave + 4 * c) + 4 * g);
@@ -438,26 +594,21 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
 #pragma unroll
             for (int c = 0; c < ND; ++c)
 #pragma unroll
-                for (int t = 0; t < 2; ++t) k[c][t] = operand(p + lay.k(), (wave + 4 * c) * 2 + t);
+                for (int t = 0; t < 2; ++t) k[c][t] = operand(p + lay.k(), (wave + 4 * c) * 2 + t, lane);
         };
         fetch_w(work);
         fetch_k(work);
-        if constexpr (!DELTA) *reinterpret_cast<floatx4 *>(&us[0][ql][tok + 4 * g]) = u;
         __syncthreads();
         for (int chunk = 0; chunk < chunks; ++chunk) {
             const int b = chunk & 1;
             work += chunk + 1 < chunks ? lay.size() : 0;
 #pragma unroll
             for (int c = 0; c < ND; ++c) s[c] *= e[c];
-            if constexpr (DELTA) {
-                floatx4 x = zero, y = zero;
-                times_state(w, ss[b], x, y);
-                *reinterpret_cast<floatx4 *>(&us[b][ql][tok + 4 * g]) = u - (x + y);
-                fetch_w(work);
-                __syncthreads();   // U is there
-            } else {
-                fetch_w(work);
-            }
+            floatx4 x = zero, y = zero;
+            times_state(w, ss[b], x, y);
+            *reinterpret_cast<floatx4 *>(&us[b][ql][tok + 4 * g]) = u - (x + y);
+            fetch_w(work);
+            __syncthreads();   // U is there
             const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -468,8 +619,7 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
                 *reinterpret_cast<floatx4 *>(&ss[b ^ 1][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
             }
             fetch_k(work);
-            if constexpr (!DELTA) *reinterpret_cast<floatx4 *>(&us[b ^ 1][ql][tok + 4 * g]) = u;
-            __syncthreads();       // the next S (and, without the delta rule, U) is there, this one has been read
+            __syncthreads();       // the next S is there, this one has been read
         }
 #pragma unroll
         for (int c = 0; c < ND; ++c) *reinterpret_cast<floatx4 *>(st + 16 * (wave + 4 * c)) = s[c];
@@ -477,11 +627,11 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
         Vec8<float> q[KS], m[2];
         auto fetch_q = [&](const float *p) {
 #pragma unroll
-            for (int t = 0; t < KS; ++t) q[t] = operand(p + lay.q(), wave * KS + t);
+            for (int t = 0; t < KS; ++t) q[t] = operand(p + lay.q(), wave * KS + t, lane);
         };
         auto fetch_b = [&](const float *p) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) m[t] = operand(p + lay.b(), wave * 2 + t);   // (the first two waves use one)
+            for (int t = 0; t < 2; ++t) m[t] = operand(p + lay.b(), wave * 2 + t, lane);   // (the first two waves use one)
         };
         fetch_q(work);
         fetch_b(work);
@@ -493,7 +643,7 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
             floatx4 x = zero, y = zero;
             times_state(q, ss[b], x, y);
             fetch_q(work);
-            if constexpr (DELTA) __syncthreads();
+            __syncthreads();
             const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
             x = mma32(m[0], ua, x);
             if (wave >= 2) y = mma32(m[1], ub, y);
@@ -510,8 +660,7 @@ __global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const Linea
 
 // Chunks that are worked on at once: their operands stay within reach of the last-level cache.
 int segment_chunks(const LinearArgs &a) {
-    const ChunkLayout lay{a.dim, a.vdim, a.z != nullptr};
-    const size_t per = lay.size() * sizeof(float) * a.heads;
+    const size_t per = chunk_work(a) * sizeof(float) * a.heads;
     const int all = (a.M + kC - 1) / kC, fit = (int)((size_t)160 * 1024 * 1024 / per);
     return all < fit ? all : fit < 8 ? (all < 8 ? all : 8) : fit;
 }
@@ -528,18 +677,21 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
     for (int m0 = 0; m0 < M; m0 += seg * kC) {
         a.M = M - m0 < seg * kC ? M - m0 : seg * kC;
         const int n = (a.M + kC - 1) / kC;
-        const dim3 grid(n, a.heads), scan(8 * ((a.heads + 7) / 8) * (a.vdim / 16));
+        const dim3 grid(n, a.heads);
+        const bool wide = a.vdim > 64;   // two 16-column tiles to a wave: past that all four waves have some
         const T *q = qkv + (size_t)m0 * a.ld + a.q_off, *k = qkv + (size_t)m0 * a.ld + a.k_off, *v = qkv + (size_t)m0 * a.ld + a.v_off;
         float *om = o + (size_t)m0 * a.heads * a.vdim;
+        auto run = [&](auto kernel, auto... args) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, args...); };
         if (a.z) {
             LinearArgs b = a;
             b.z += (size_t)m0 * a.heads * a.dim;
             b.factors += (size_t)m0 * 2 * a.k_heads;
             hipLaunchKernelGGL((delta_chunk_kernel<T, ND>), grid, dim3(kThreads), lds, stream, b, q, k, v, beta + (size_t)m0 * a.ld_beta, work);
-            hipLaunchKernelGGL((chunk_scan_kernel<ND, true>), scan, dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
+            hipLaunchKernelGGL((delta_scan_kernel<ND>), dim3(8 * ((a.heads + 7) / 8) * (a.vdim / 16)), dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
         } else {
-            hipLaunchKernelGGL((linear_chunk_kernel<T, ND>), grid, dim3(kThreads), 0, stream, a, q, k, v, work);
-            hipLaunchKernelGGL((chunk_scan_kernel<ND, false>), scan, dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
+            run(wide ? &linear_state_kernel<T, ND, 2> : &linear_state_kernel<T, ND, 1>, a, q, k, v, work);
+            hipLaunchKernelGGL((linear_scan_kernel<ND>), dim3(a.vdim * a.dim / (4 * kThreads), a.heads), dim3(kThreads), 0, stream, a, work, n, m0 == 0);
+            run(&linear_output_kernel<T, ND>, a, q, k, v, work, om);
         }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -552,8 +704,7 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
 bool linear_chunks_supported(const LinearArgs &a) { return a.dim <= 128; }
 
 size_t linear_chunk_bytes(const LinearArgs &a) {
-    const ChunkLayout lay{a.dim, a.vdim, a.z != nullptr};
-    return lay.size() * sizeof(float) * a.heads * segment_chunks(a);
+    return chunk_work(a) * sizeof(float) * a.heads * segment_chunks(a);
 }
 
 hipError_t launch_linear_chunks(int dtype, const LinearArgs &a, void *work, float *o, hipStream_t stream) {

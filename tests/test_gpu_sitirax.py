@@ -419,6 +419,27 @@ def test_many_chunks_and_several_segments(dense):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("heads,dim,vdim", [(9, 64, 16), (2, 64, 96), (1, 64, 320), (2, 128, 64), (1, 128, 160), (3, 128, 272)])
+def test_one_decay_per_head_in_chunks(dense, dtype, heads, dim, vdim):
+    """Value columns that fewer than four waves have, one or two 16-column tiles to a wave, several turns and an odd last one; ends of a portion."""
+    say("one decay per head", dtype, heads, dim, vdim)
+    x = Recurrence(dense, "lightning", heads, heads, dim, vdim, 209, dtype, seed=vdim, far=[(200, 1), (64, 63), (65, 64)])
+    want, state = x.want()
+    for cuts in ((0, 209), (0, 64, 65, 209), (0, 2, 130, 209)):
+        x.state.fill_(float("nan"))
+        close(torch.cat([x.run(a, b, True) for a, b in zip(cuts, cuts[1:])]), want, dtype, cuts, **STATE_TOL)
+        close(x.final(), state, dtype, "state", **STATE_TOL)
+
+
+def test_one_decay_per_head_in_two_segments(dense):
+    say("segments, one decay per head")
+    x = Recurrence(dense, "lightning", 1024, 1024, 64, 64, 650, F32, seed=10)      # ten chunks to a segment
+    want, state = x.want()
+    close(x.run(0, 650, True), want, F32, "lightning", f32=2e-4)
+    close(x.final(), state, F32, "state", f32=2e-4)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("groups,cols,true", [(1, 96, 70), (1, 1536, 1500), (5, 32, 24), (3, 128, 128), (2, 320, 300)])
 def test_gated_norm(dense, dtype, groups, cols, true):
     rng = np.random.default_rng(cols)
