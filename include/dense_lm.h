@@ -88,6 +88,8 @@ int dlm_moe_down_gemv(int dtype, const void *h, const void *w_down, const int32_
 /* Many tokens: ids, weights [tokens, top]; then the entries token * top + slot sorted by expert (order[tokens * top]) and
  * their row tiles (int32 [dlm_moe_max_tiles(..) + 1, 4]; the last row holds the number of tiles in use). */
 int dlm_moe_select(const dlm_router *r, int tokens, int32_t *ids, float *weights, void *stream);
+/* The same on logits [parts, tokens, ld] whose sum counts, as dlm_gemm_sliced leaves them. */
+int dlm_moe_select_parts(const dlm_router *r, int parts, int tokens, int32_t *ids, float *weights, void *stream);
 int dlm_moe_max_tiles(int entries, int experts, int tile_rows);
 int dlm_moe_plan(const int32_t *ids, int entries, int experts, int tile_rows, int32_t *order, int32_t *tiles, void *stream);
 

@@ -163,6 +163,7 @@ DENSE_SYMBOLS = {
     "dlm_moe_gate_up_gemv": (_ci, [_ci] + [_vp] * 6 + [_ci, _ci, _vp]),
     "dlm_moe_down_gemv": (_ci, [_ci] + [_vp] * 5 + [_ci] * 4 + [_vp]),
     "dlm_moe_select": (_ci, [_vp, _ci, _vp, _vp, _vp]),
+    "dlm_moe_select_parts": (_ci, [_vp, _ci, _ci, _vp, _vp, _vp]),
     "dlm_moe_max_tiles": (_ci, [_ci] * 3),
     "dlm_moe_plan": (_ci, [_vp] + [_ci] * 3 + [_vp] * 3),
     "dlm_gemm_tile_rows": (_ci, [_ci] * 4),

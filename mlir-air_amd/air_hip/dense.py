@@ -303,13 +303,13 @@ def moe_gemv(x, logits, router, w_gate_up, w_down):
 
 
 def moe_select(logits, router):
-    """(ids int32 [M, top], weights fp32 [M, top]) for router logits [M, ld]."""
+    """(ids int32 [M, top], weights fp32 [M, top]) for router logits [M, ld], or parts [n, M, ld] of them."""
     lib = _lib.load_dense_library()
-    M = logits.shape[0]
+    parts, M = (logits.shape[0], logits.shape[1]) if logits.dim() == 3 else (1, logits.shape[0])
     ids = torch.empty((M, router.top), dtype=torch.int32, device=logits.device)
     wts = torch.empty((M, router.top), dtype=torch.float32, device=logits.device)
     r = router.bind(logits)
-    _lib.check_dense(lib.dlm_moe_select(ctypes.byref(r), M, _ptr(ids), _ptr(wts), _stream()))
+    _lib.check_dense(lib.dlm_moe_select_parts(ctypes.byref(r), parts, M, _ptr(ids), _ptr(wts), _stream()))
     return ids, wts
 
 
@@ -320,7 +320,7 @@ def moe_rows(h, logits, router, w_gate_up, w_down):
     _same("moe_rows", w_gate_up, h, w_down)
     E, ff2, K = w_gate_up.shape
     ff, N, top = ff2 // 2, w_down.shape[1], router.top
-    if h.shape[1] != K or tuple(w_down.shape) != (E, N, ff) or E != router.experts or logits.shape[0] != h.shape[0]:
+    if h.shape[1] != K or tuple(w_down.shape) != (E, N, ff) or E != router.experts or logits.shape[-2] != h.shape[0]:
         raise ValueError("moe_rows: shapes of the rows and the experts do not match")
     M, dev, dt = h.shape[0], h.device, dtype_code(h)
     ids, wts = moe_select(logits, router)

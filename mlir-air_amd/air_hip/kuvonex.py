@@ -272,7 +272,7 @@ class KuvonexModel(DenseModel):
             y = dense.gemm(attn, l.w_o, out_f32=True, parts=True)
             h = dense.residual_norm_rows(res, y, l.norm1, c.eps, c.width, self.dtype)
             if l.router is not None:
-                logits = dense.gemm(h, l.w_router, out_f32=True)
+                logits = dense.gemm(h, l.w_router, out_f32=True, parts=True)
                 y, wts = dense.moe_rows(h, logits, l.router, l.w_gate_up, l.w_down)
                 h = dense.residual_norm_rows(res, y, l.norm2, c.eps, c.width, self.dtype, weights=wts)
             if trace is not None:

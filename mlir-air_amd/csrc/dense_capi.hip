@@ -220,11 +220,15 @@ int dlm_moe_down_gemv(int dtype, const void *h, const void *w_down, const int32_
 }
 
 int dlm_moe_select(const dlm_router *r, int tokens, int32_t *ids, float *weights, void *stream) {
+    return dlm_moe_select_parts(r, 1, tokens, ids, weights, stream);
+}
+
+int dlm_moe_select_parts(const dlm_router *r, int parts, int tokens, int32_t *ids, float *weights, void *stream) {
     const int c = check_router(r);
     if (c) return c;
     if (!ids || !weights) return DLM_ERR_NULL;
-    if (tokens <= 0) return DLM_ERR_SHAPE;
-    return done(launch_moe_select(router_of(r), tokens, ids, weights, hs(stream)));
+    if (tokens <= 0 || parts < 1) return DLM_ERR_SHAPE;
+    return done(launch_moe_select(router_of(r), parts, tokens, ids, weights, hs(stream)));
 }
 
 int dlm_moe_max_tiles(int entries, int experts, int tile_rows) {

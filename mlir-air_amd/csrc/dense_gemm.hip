@@ -809,7 +809,8 @@ struct GemmChoice {
     int kind, slices;
 };
 // slices 0: any number; kept: the caller takes the parts.  Up to 128 columns are one tile's in any kind, so narrow tiles read nothing but their
-// little W again: a router, 2048 x 64 x 2048, takes 11 us in one launch of 32-row tiles, 17 in eight slices of 128-row ones and their sum.
+// little W again: a router, 2048 x 64 x 2048, takes 13.7 us in one launch of 32-row tiles (its 32 K-steps on 64 CUs are all latency), 7.4 in eight
+// slices of 64-row ones whose sum is left to the choice of the experts (5.0 -> 5.3 us), 17 in slices of 128-row ones and their sum.
 GemmChoice choose_gemm(int M, int N, int K, int epilogue, int slices, bool kept) {
     GemmChoice best{kWide256, 1};
     float least = 1e30f;

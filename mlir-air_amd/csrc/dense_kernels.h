@@ -60,7 +60,8 @@ hipError_t launch_moe_gate_up_gemv(int dtype, const Router &r, const void *x, co
 hipError_t launch_moe_down_gemv(int dtype, const void *h, const void *w_down, const int32_t *ids, const float *weights, float *y, int top,
                                 int ff, int N, hipStream_t stream);
 // many tokens
-hipError_t launch_moe_select(const Router &r, int tokens, int32_t *ids, float *weights, hipStream_t stream);
+// (logits [parts][tokens][ld] are added up)
+hipError_t launch_moe_select(const Router &r, int parts, int tokens, int32_t *ids, float *weights, hipStream_t stream);
 // entries (token * top + slot) sorted by expert, and the row tiles of `bm` entries that the grouped product runs over:
 // tiles[i] = {expert, first sorted entry, entries, 0}, and behind the most tiles that there can be {number of tiles}
 int moe_max_tiles(int entries, int experts, int bm);

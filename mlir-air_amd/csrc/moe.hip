@@ -96,12 +96,29 @@ auto with_lanes(int experts, F f) {
 }
 
 template <int PL>
-__global__ void __launch_bounds__(kMoeThreads) moe_select_kernel(const Router r, int tokens, int32_t *ids, float *weights) {
+__global__ void __launch_bounds__(kMoeThreads) moe_select_kernel(const Router r, int parts, int tokens, int32_t *ids, float *weights) {
     extern __shared__ float select_lds[];
-    const int wave = threadIdx.x >> 6, t = blockIdx.x * kMoeWaves + wave;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x * kMoeWaves + wave;
     if (t >= tokens) return;   // whole waves leave; no workgroup barrier below
     float *mine = select_lds + wave * (r.experts + r.groups);
-    choose_experts<PL>(r, r.logits + (size_t)t * r.ld, mine, mine + r.experts, ids + (size_t)t * r.top, weights + (size_t)t * r.top);
+    const float *logits = r.logits + (size_t)t * r.ld;
+    if (parts > 1) {   // the router's product in slices along K, up to eight of them on their way; a lane reads back what it wrote
+        float *sum = select_lds + kMoeWaves * (r.experts + r.groups) + wave * r.experts;
+        const size_t size = (size_t)tokens * r.ld;
+        for (int e = lane; e < r.experts; e += 64) {
+            float z = 0.f;
+            for (int s0 = 0; s0 < parts; s0 += 8) {
+                float x[8];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) x[s] = logits[(s0 + s < parts ? s0 + s : s0) * size + e];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) z = s0 + s < parts ? z + x[s] : z;
+            }
+            sum[e] = z;
+        }
+        logits = sum;
+    }
+    choose_experts<PL>(r, logits, mine, mine + r.experts, ids + (size_t)t * r.top, weights + (size_t)t * r.top);
 }
 
 // One workgroup: sort the entries by expert (counting sort) and cut every expert's run into tiles of bm entries, or even ones where they
@@ -394,11 +411,11 @@ hipError_t launch_moe_down_gemv(int dtype, const void *h, const void *w_down, co
     return dtype == kF32 ? down<float>(h, w_down, ids, weights, y, top, ff, N, stream) : down<bf16>(h, w_down, ids, weights, y, top, ff, N, stream);
 }
 
-hipError_t launch_moe_select(const Router &r, int tokens, int32_t *ids, float *weights, hipStream_t stream) {
-    const size_t lds = (size_t)kMoeWaves * (r.experts + r.groups) * sizeof(float);
+hipError_t launch_moe_select(const Router &r, int parts, int tokens, int32_t *ids, float *weights, hipStream_t stream) {
+    const size_t lds = (size_t)kMoeWaves * (r.experts * (parts > 1 ? 2 : 1) + r.groups) * sizeof(float);   // (48 KiB at most)
     return with_lanes(r.experts, [&](auto pl) {
-        hipLaunchKernelGGL(moe_select_kernel<decltype(pl)::value>, dim3((tokens + kMoeWaves - 1) / kMoeWaves), dim3(kMoeThreads), lds, stream, r, tokens,
-                           ids, weights);
+        hipLaunchKernelGGL(moe_select_kernel<decltype(pl)::value>, dim3((tokens + kMoeWaves - 1) / kMoeWaves), dim3(kMoeThreads), lds, stream, r, parts,
+                           tokens, ids, weights);
         return hipGetLastError();
     });
 }

@@ -173,6 +173,22 @@ def test_router_choice(dense, experts, top, groups, keep, shift):
         assert np.allclose(wts[m].cpu().numpy(), wt, rtol=1e-5)
 
 
+@pytest.mark.parametrize("parts", [1, 2, 8, 9])
+@pytest.mark.parametrize("experts", [6, 64, 72, 320])
+def test_routing_of_logits_in_parts(dense, experts, parts):
+    """Logits that a product left in slices: the same choice as of their sum, to the bit."""
+    say("routing of parts", experts, parts)
+    g = torch.Generator().manual_seed(experts + parts)
+    z = torch.randn((parts, 11, (experts + 15) // 16 * 16), generator=g).cuda()
+    z[:, :, experts:] = 50.0
+    spec = dense.RouterSpec(torch.randn((experts,), generator=g).cuda() * 0.1, experts, 3, 2, 1)
+    total = z[0].clone()
+    for p in z[1:]:
+        total += p
+    got, want = dense.moe_select(z, spec), dense.moe_select(total, spec)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("M,experts,top,groups,keep,K,ff,N", [(1, 10, 2, 2, 1, 64, 128, 128), (1, 16, 5, 4, 2, 1152, 576, 320), (2, 9, 2, 3, 1, 128, 64, 64),
                                                                (61, 6, 3, 6, 4, 192, 128, 192), (700, 5, 2, 1, 1, 64, 192, 64)])
