@@ -70,17 +70,11 @@ __device__ __forceinline__ float group_sum(float s) {
     return s;
 }
 
-// Half-split RoPE of elements [e0, e0 + 8) of one head: x at src, rounded to bf16 (returned as floats).
-template <int HD>
-__device__ __forceinline__ void rope8(const uint16_t *src, const uint16_t *lut, int e0, float (&out)[8]) {
-    constexpr int HALF = HD / 2;
-    const bool low = e0 < HALF;
-    const int i0 = low ? e0 : e0 - HALF;
-    float x[8], y[8], c[8], s[8];
-    unpack8(*reinterpret_cast<const u32x4 *>(src + e0), x);
-    unpack8(*reinterpret_cast<const u32x4 *>(src + (low ? e0 + HALF : e0 - HALF)), y);
-    unpack8(*reinterpret_cast<const u32x4 *>(lut + i0), c);
-    unpack8(*reinterpret_cast<const u32x4 *>(lut + HALF + i0), s);
+// Half-split RoPE of the eight elements x of one head's half, y the same places of the other half, rounded to bf16 (returned as floats).
+__device__ __forceinline__ void rope8(const u32x4 xr, const u32x4 yr, const float (&c)[8], const float (&s)[8], bool low, float (&out)[8]) {
+    float x[8], y[8];
+    unpack8(xr, x);
+    unpack8(yr, y);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         // low half: x1 cos - x2 sin; high half: x2 cos + x1 sin (x is the lane's own element)
@@ -110,10 +104,11 @@ __device__ __forceinline__ float slots_reduce(float v) {
     return swap_reduce<32, MAX>(v, v);
 }
 
-// What bounds it: latencies in a row, at 64 positions a workgroup: the fresh qkv and the cache (requested together: the new token's K and V
-// are taken from registers, not read back), the scores' sums, one maximum per wave and head, and the sums over positions.  Those halve
+// What bounds it: latencies in a row, at 64 positions a workgroup: the fresh qkv and the cache (requested together and without a branch between
+// them, qkv first, so that it is rotated while the cache is on its way; the new token's K and V are taken from registers, not read back), the scores' sums, one maximum per wave and head, and the sums over positions.  Those halve
 // what a lane holds with every exchange (v_permlane*_swap: half the values go each way), 28 exchanges for a head group of 4, where full
-// butterflies of (m, l, acc) took 120 shuffles through LDS.   32 heads of 64 over 8, 1000 positions: 7.3 -> 4.9 us.
+// butterflies of (m, l, acc) took 120 shuffles through LDS.   32 heads of 64 over 8, 1000 positions: 7.3 -> 4.9 us; -> 4.5 a layer of
+// the model since the new token's row and the queries are no longer asked for one after the other behind the cache.
 template <int HD, int G>
 __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     constexpr int LPP = HD / 8;        // lanes per position
@@ -133,6 +128,21 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     uint16_t *kc = p.k_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
     uint16_t *vc = p.v_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
 
+    // rotation and this lane's slices of qkv, the new K and V also where the chunk does not own them
+    const bool low = 8 * sub < HD / 2;
+    const int other = low ? 8 * sub + HD / 2 : 8 * sub - HD / 2, turn = low ? 8 * sub : other;
+    auto raw = [](const uint16_t *at) { return *reinterpret_cast<const u32x4 *>(at); };
+    const u32x4 cos_raw = raw(p.lut + turn), sin_raw = raw(p.lut + HD / 2 + turn);
+    u32x4 qx[G], qy[G];
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+        const uint16_t *src = p.qkv + (size_t)(kvh * G + h) * HD;
+        qx[h] = raw(src + 8 * sub);
+        qy[h] = raw(src + other);
+    }
+    const uint16_t *k_row = p.qkv + nq + kvh * HD;
+    const u32x4 kx = raw(k_row + 8 * sub), ky = raw(k_row + other), vnew = raw(k_row + nkv + 8 * sub);
+
     u32x4 kraw[UN], vraw[UN];
     auto request = [&](int tb) {
 #pragma unroll
@@ -146,26 +156,24 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     int tb = t0 + wave * PPW + slot;
     request(tb);
 
+    __builtin_amdgcn_sched_barrier(0);
+    float cos[8], sin[8];
+    unpack8(cos_raw, cos);
+    unpack8(sin_raw, sin);
     // the chunk that owns `pos` appends the new token's K (rotated) and V
-    u32x4 knew, vnew;
     const bool owner = t0 <= p.pos && p.pos < t1;
-    if (owner) {
+    u32x4 knew;
+    {
         float kr[8];
-        rope8<HD>(p.qkv + nq + kvh * HD, p.lut, 8 * sub, kr);
+        rope8(kx, ky, cos, sin, low, kr);
 #pragma unroll
         for (int j = 0; j < 4; ++j) knew[j] = pack_bf16x2(kr[2 * j], kr[2 * j + 1]);
-        vnew = *reinterpret_cast<const u32x4 *>(p.qkv + nq + nkv + kvh * HD + 8 * sub);
-        if (threadIdx.x < LPP) {
-            *reinterpret_cast<u32x4 *>(kc + (size_t)p.pos * HD) = knew;
-            *reinterpret_cast<u32x4 *>(vc + (size_t)p.pos * HD) = vnew;
-        }
     }
-
     // rotated, bf16-rounded query slices of the G heads, pre-scaled for exp2
     float q[G][8];
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-        rope8<HD>(p.qkv + (size_t)(kvh * G + h) * HD, p.lut, 8 * sub, q[h]);
+        rope8(qx[h], qy[h], cos, sin, low, q[h]);
 #pragma unroll
         for (int j = 0; j < 8; ++j) q[h][j] *= p.scale * kLog2e;
     }
@@ -215,6 +223,11 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
                 for (int j = 0; j < 8; ++j) acc[8 * h + j] = fmaf(pr, live[i] ? v[i][j] : 0.f, acc[8 * h + j]);
             }
         }
+    }
+
+    if (owner && threadIdx.x < LPP) {   // (behind the loop: no wait in it counts stores)
+        *reinterpret_cast<u32x4 *>(kc + (size_t)p.pos * HD) = knew;
+        *reinterpret_cast<u32x4 *>(vc + (size_t)p.pos * HD) = vnew;
     }
 
     // sums over the wave's positions: lanes 32 .. 63 go on with the upper half of the values, odd rows of lanes with the upper half of theirs
