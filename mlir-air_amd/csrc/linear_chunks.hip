@@ -11,6 +11,7 @@
 //
 //   linear_state    one workgroup per head and chunk: (k e^(G_last - G))^T V
 //   linear_scan     every element of S on its own: the S in front of every chunk in place of its product
+//   linear_steps    instead of the two, for a few chunks: a workgroup's value columns of a head through all of them
 //   linear_output   one workgroup per head and chunk: O
 //
 // With the delta rule everything but the products with S can be done for all chunks at once:
@@ -78,14 +79,14 @@ __device__ __forceinline__ Vec8<float> operand(const float *m, int piece, int la
     return Vec8<float>{*reinterpret_cast<const floatx4 *>(x), *reinterpret_cast<const floatx4 *>(x + 256)};
 }
 
-// What a workgroup of the form with one decay per head works on: blockIdx.x = chunk, blockIdx.y = head.
+// What a workgroup of the form with one decay per head works on: a chunk of head blockIdx.y.
 template <class T>
 struct LinearChunk {
     const T *q, *k, *v;
     float ld;
     int n;   // tokens
-    __device__ __forceinline__ LinearChunk(const LinearArgs &a, const T *q0, const T *k0, const T *v0) {
-        const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC;
+    __device__ __forceinline__ LinearChunk(const LinearArgs &a, const T *q0, const T *k0, const T *v0, int chunk) {
+        const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = chunk * kC;
         const int D = a.dim;
         n = a.M - m0 < kC ? a.M - m0 : kC;
         ld = a.log2_decay[h];
@@ -107,22 +108,51 @@ struct LinearChunk {
     }
 };
 
-// A wave has NV times 16 value columns of all channels; keys, already decayed, through LDS.
+// A chunk's keys, already decayed, on their way to LDS
+template <class T, int ND>
+struct DecayedKeys {
+    static constexpr int D = 64 * ND, P = D + 4, kRows = kC * D / 8 / kThreads;   // kRows: pieces of a thread
+    Vec8<T> x[kRows];
+    __device__ __forceinline__ void request(const LinearArgs &a, const LinearChunk<T> &c) {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const int at = threadIdx.x + kThreads * i, r = at / (D / 8);
+            x[i] = load8(c.k + (size_t)(r < c.n ? r : c.n - 1) * a.ld + 8 * (at % (D / 8)));
+        }
+    }
+    __device__ __forceinline__ void store(const LinearChunk<T> &c, float (*ks)[P]) const {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const int at = threadIdx.x + kThreads * i, r = at / (D / 8);
+            const float f = c.power(c.n - 1 - r);
+            float y[8];
+            unpack8(x[i], y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = r < c.n ? y[e] * f : 0.f;
+            store8(&ks[r][8 * (at % (D / 8))], pack8<float>(y));
+        }
+    }
+    // first operand: tokens 32 t .. + 31 of 16 channels
+    __device__ __forceinline__ static Vec8<float> channels(const float (*ks)[P], int ct, int t) {
+        const int lane = threadIdx.x & 63;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = ks[32 * t + 8 * (lane >> 4) + e][16 * ct + (lane & 15)];
+        return pack8<float>(y);
+    }
+};
+
+// A wave has NV times 16 value columns of all channels.
 template <class T, int ND, int NV>
 __global__ void __launch_bounds__(kThreads) linear_state_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work) {
     constexpr int D = 64 * ND, P = D + 4, KS = 2 * ND;
     __shared__ __attribute__((aligned(16))) float ks[kC][P];
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tiles = a.vdim / 16;
-    const LinearChunk<T> c(a, q, k, v);
+    const LinearChunk<T> c(a, q, k, v, blockIdx.x);
     work += ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * a.vdim * D;
-    constexpr int kRows = kC * D / 8 / kThreads;   // pieces of keys of a thread
-    Vec8<T> kr[kRows];
-#pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-        const int at = tid + kThreads * i, r = at / (D / 8);
-        kr[i] = load8(c.k + (size_t)(r < c.n ? r : c.n - 1) * a.ld + 8 * (at % (D / 8)));
-    }
+    DecayedKeys<T, ND> keys;
+    keys.request(a, c);
     Vec8<float> u[NV][2];
     auto fetch = [&](int vt0) {
 #pragma unroll
@@ -131,28 +161,12 @@ __global__ void __launch_bounds__(kThreads) linear_state_kernel(const LinearArgs
             for (int t = 0; t < 2; ++t) u[i][t] = c.values(a, vt0 + i < tiles ? vt0 + i : tiles - 1, t);
     };
     fetch(wave * NV);
-#pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-        const int at = tid + kThreads * i, r = at / (D / 8);
-        const float f = c.power(c.n - 1 - r);
-        float x[8];
-        unpack8(kr[i], x);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = r < c.n ? x[e] * f : 0.f;
-        store8(&ks[r][8 * (at % (D / 8))], pack8<float>(x));
-    }
+    keys.store(c, ks);
     __syncthreads();
     for (int vt0 = wave * NV; vt0 < tiles;) {
 #pragma unroll 2
         for (int ct = 0; ct < 4 * ND; ++ct) {
-            Vec8<float> m[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = ks[32 * t + 8 * g + e][16 * ct + ql];
-                m[t] = pack8<float>(x);
-            }
+            const Vec8<float> m[2] = {keys.channels(ks, ct, 0), keys.channels(ks, ct, 1)};
             floatx4 s[NV];
 #pragma unroll
             for (int i = 0; i < NV; ++i) s[i] = mma32(m[0], u[i][0], floatx4{0.f, 0.f, 0.f, 0.f});
@@ -165,6 +179,46 @@ __global__ void __launch_bounds__(kThreads) linear_state_kernel(const LinearArgs
         vt0 += 4 * NV;
         if (vt0 < tiles) fetch(vt0);
     }
+}
+
+// The state kernel and the scan in one, for one or two chunks: four times 16 value columns of a head, the chunks one after the other.  A prompt through
+// four layers of width 2048, 16 heads of 128 / 128 in two of them: 128 tokens 558 us (557 before outputs were a launch of their own), 256 tokens 690 with
+// it and 673 with the two launches (677 before); the host, which narrow models' short portions wait for, is spared a launch.
+constexpr int kFewChunks = 2;
+template <class T, int ND>
+__global__ void __launch_bounds__(kThreads) linear_steps_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work, int chunks, bool first) {
+    constexpr int D = 64 * ND, P = D + 4, KS = 2 * ND, NC = 4 * ND;
+    __shared__ __attribute__((aligned(16))) float ks[kC][P];
+    const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
+    const int tiles = a.vdim / 16, mine = 4 * blockIdx.x + __builtin_amdgcn_readfirstlane(tid >> 6), vt = mine < tiles ? mine : tiles - 1;
+    work += (size_t)blockIdx.y * chunks * a.vdim * D + vt * 16 * D + place_of(ql, 4 * g, KS);
+    float *st = a.state + ((size_t)blockIdx.y * a.vdim + 16 * vt + ql) * D + 4 * g;
+    floatx4 s[NC];
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) s[ct] = *reinterpret_cast<const floatx4 *>(st + 16 * ct);
+    if (first && (a.pos_dev ? a.pos_dev[0] : a.pos) == 0) {
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) s[ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    DecayedKeys<T, ND> keys;
+    for (int chunk = 0; chunk < chunks; ++chunk) {
+        const LinearChunk<T> c(a, q, k, v, chunk);
+        keys.request(a, c);
+        const Vec8<float> u[2] = {c.values(a, vt, 0), c.values(a, vt, 1)};
+        if (chunk > 0) __syncthreads();
+        keys.store(c, ks);
+        __syncthreads();
+        const float e = c.power(c.n);
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) {
+            if (mine < tiles) *reinterpret_cast<floatx4 *>(work + (size_t)chunk * a.vdim * D + place_of(0, 16 * ct, KS)) = s[ct];
+            const floatx4 x = mma32(keys.channels(ks, ct, 0), u[0], floatx4{0.f, 0.f, 0.f, 0.f});
+            s[ct] = s[ct] * e + mma32(keys.channels(ks, ct, 1), u[1], x);
+        }
+    }
+    if (mine >= tiles) return;
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) *reinterpret_cast<floatx4 *>(st + 16 * ct) = s[ct];
 }
 
 // Four elements of S to a thread, the products of kAhead chunks on their way.
@@ -205,7 +259,7 @@ __global__ void __launch_bounds__(kThreads, 2) linear_output_kernel(const Linear
     __shared__ __attribute__((aligned(16))) float qf[kC * D], bs[kC * kC];   // q e^G and B, in the order of ChunkLayout
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tiles = a.vdim / 16;
-    const LinearChunk<T> c(a, q, k, v);
+    const LinearChunk<T> c(a, q, k, v, blockIdx.x);
     work += ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * a.vdim * D;
     o += ((size_t)blockIdx.x * kC * a.heads + blockIdx.y) * a.vdim;
     auto row_of = [&](const T *x, int r) { return x + (size_t)(r < c.n ? r : c.n - 1) * a.ld; };
@@ -689,8 +743,12 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
             hipLaunchKernelGGL((delta_chunk_kernel<T, ND>), grid, dim3(kThreads), lds, stream, b, q, k, v, beta + (size_t)m0 * a.ld_beta, work);
             hipLaunchKernelGGL((delta_scan_kernel<ND>), dim3(8 * ((a.heads + 7) / 8) * (a.vdim / 16)), dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
         } else {
-            run(wide ? &linear_state_kernel<T, ND, 2> : &linear_state_kernel<T, ND, 1>, a, q, k, v, work);
-            hipLaunchKernelGGL((linear_scan_kernel<ND>), dim3(a.vdim * a.dim / (4 * kThreads), a.heads), dim3(kThreads), 0, stream, a, work, n, m0 == 0);
+            if (n <= kFewChunks) {
+                hipLaunchKernelGGL((linear_steps_kernel<T, ND>), dim3((a.vdim + 63) / 64, a.heads), dim3(kThreads), 0, stream, a, q, k, v, work, n, m0 == 0);
+            } else {
+                run(wide ? &linear_state_kernel<T, ND, 2> : &linear_state_kernel<T, ND, 1>, a, q, k, v, work);
+                hipLaunchKernelGGL((linear_scan_kernel<ND>), dim3(a.vdim * a.dim / (4 * kThreads), a.heads), dim3(kThreads), 0, stream, a, work, n, m0 == 0);
+            }
             run(&linear_output_kernel<T, ND>, a, q, k, v, work, om);
         }
         const hipError_t e = hipGetLastError();

@@ -421,11 +421,12 @@ def test_many_chunks_and_several_segments(dense):
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("heads,dim,vdim", [(9, 64, 16), (2, 64, 96), (1, 64, 320), (2, 128, 64), (1, 128, 160), (3, 128, 272)])
 def test_one_decay_per_head_in_chunks(dense, dtype, heads, dim, vdim):
-    """Value columns that fewer than four waves have, one or two 16-column tiles to a wave, several turns and an odd last one; ends of a portion."""
+    """Value columns that fewer than four waves have, one or two 16-column tiles to a wave, several turns and an odd last one; one and two
+    chunks (in one launch) and more; ends of a portion."""
     say("one decay per head", dtype, heads, dim, vdim)
-    x = Recurrence(dense, "lightning", heads, heads, dim, vdim, 209, dtype, seed=vdim, far=[(200, 1), (64, 63), (65, 64)])
+    x = Recurrence(dense, "lightning", heads, heads, dim, vdim, 385, dtype, seed=vdim, far=[(380, 1), (64, 63), (65, 64), (258, 250)])
     want, state = x.want()
-    for cuts in ((0, 209), (0, 64, 65, 209), (0, 2, 130, 209)):
+    for cuts in ((0, 385), (0, 64, 65, 385), (0, 128, 257, 385), (0, 129, 385), (0, 2, 130, 321, 385)):
         x.state.fill_(float("nan"))
         close(torch.cat([x.run(a, b, True) for a, b in zip(cuts, cuts[1:])]), want, dtype, cuts, **STATE_TOL)
         close(x.final(), state, dtype, "state", **STATE_TOL)
