@@ -346,6 +346,20 @@ def test_latent_attention_forms_agree_token_by_token_and_with_the_position_on_th
             close(got, want[i], dtype, (i, nsplit), f32=5e-5, bf16=6e-2)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("sizes", [(2, 24, 8, 40, 56), (2, 24, 8, 32, 600)])
+def test_latent_attention_of_one_token_in_many_splits(dense, dtype, sizes):
+    """One to many blocks of keys to a split (two of them ahead of the products), and more splits in use than the merge reads ahead (64)."""
+    say("many splits", dtype, sizes)
+    T = 2200                                                 # 69 blocks
+    x = Latents(dense, sizes, T, dtype, seed=11, own=False, far=[(2199, 0), (2198, 2100)])
+    x.fill()
+    want = x.want()
+    for nsplit in (1, 23, 35, 64, 69, 128, 256):
+        for i in (2198, 2199):
+            close(x.run("absorbed", i, i + 1, nsplit=nsplit)[0], want[i], dtype, (i, nsplit), f32=5e-5, bf16=6e-2)
+
+
 @pytest.mark.parametrize("form", ["rows", "absorbed"])
 def test_latent_attention_over_another_layers_rows(dense, form):
     say("shared latents", form)
