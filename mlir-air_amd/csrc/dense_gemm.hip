@@ -264,7 +264,7 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
 // A wave's NT x MT tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
-// GROUPED, second product: out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
+// GROUPED without a pair, entries as rows of the result: out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
 template <int NT, int MT, int EPI, bool GROUPED>
 __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first,
                                            const int (&out_rows)[2] = {0, 0}) {
@@ -298,6 +298,8 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
             if constexpr (GROUPED && !kPair)
                 if (p.gather == 0) to = __shfl(out_rows[i / 4], 16 * (i % 4) + row);
             if (m >= m_end || n_out + col >= n_end) continue;
+            if constexpr (GROUPED && kPair)
+                if (p.gather == 0) to = p.order[m];   // (no product of the mixture: asked for here, the registers of out_rows are worth more)
             const long part = EPI == kOutF32 ? blockIdx.y * p.slice_stride : 0;
             *reinterpret_cast<u32x4 *>(static_cast<Out *>(p.out) + part + to * p.ldo + n_out + col) = *reinterpret_cast<const u32x4 *>(rows + row * kPitch + col);
         }

@@ -183,6 +183,34 @@ def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows, launched):
         close(out[at], got.double() @ w2[i].double().t(), True, ("down", i))
 
 
+@pytest.mark.parametrize("dtype,tile_rows", [(torch.bfloat16, 32), (torch.bfloat16, 128), (torch.bfloat16, 384), (torch.float32, 32), (torch.float32, 128)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_grouped_products_with_rows_in_either_order(dense, dtype, tile_rows, pair):
+    """Both sides of `gather` with both epilogues: rows of A by entry and results at sorted places, or the other way round."""
+    print("grouped rows", dtype, tile_rows, pair, flush=True)
+    from air_hip import _lib
+    lib, stream, dt = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream, int(dtype == torch.float32)
+    counts, K, N, top = (1, 130, 0, 400, 65), 128, 160, 4
+    E, entries, width = len(counts), sum(counts), 80 if pair else 160
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(entries, generator=torch.Generator().manual_seed(1))].to(torch.int32).cuda()
+    order = torch.empty((entries,), dtype=torch.int32, device="cuda")
+    n_tiles = lib.dlm_moe_max_tiles(entries, E, tile_rows)
+    tiles = torch.empty((n_tiles + 1, 4), dtype=torch.int32, device="cuda")
+    _lib.check_dense(lib.dlm_moe_plan(ids.data_ptr(), entries, E, tile_rows, order.data_ptr(), tiles.data_ptr(), stream))
+    a, w = rand(2, entries, K).bfloat16().to(dtype), (rand(3, E, N, K) * K ** -0.5).bfloat16().to(dtype)
+    w1 = torch.stack([interleaved(m[:N // 2], m[N // 2:]) for m in w]) if pair else w
+    e, at = ids.long(), order.long()
+    for gather in (0, top):
+        out = torch.full((entries, width), 7.0, dtype=dtype, device="cuda")
+        g = _lib.GemmArgs(a=a.data_ptr(), w=w1.data_ptr(), out=out.data_ptr(), lda=K, ldo=width, w_stride=N * K, N=N, K=K, gather=gather, tiles=tiles.data_ptr(),
+                          epilogue=dense.OUT_SWIGLU if pair else dense.OUT_ELEM, order=order.data_ptr(), M=entries, n_tiles=n_tiles, tile_rows=tile_rows)
+        _lib.check_dense(lib.dlm_gemm(dt, ctypes.byref(g), stream))
+        rows = a[at // top] if gather else a                      # by sorted place
+        y = torch.bmm(w[e[at]].float(), rows.float()[:, :, None]).squeeze(2).double()   # (fp32 products of 128 bf16 numbers: 2^-24 of their sum)
+        y = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:] if pair else y
+        close(out if gather else out[at], y, not dt, (gather, pair))
+
+
 @pytest.mark.parametrize("entries,experts", [(1, 1), (1000, 7), (16384, 64), (16385, 1024), (50000, 3)])
 def test_expert_plan(dense, entries, experts):
     print("plan", entries, experts, flush=True)
