@@ -303,9 +303,13 @@ def moe_gemv(x, logits, router, w_gate_up, w_down):
 
 
 def moe_select(logits, router):
-    """(ids int32 [M, top], weights fp32 [M, top]) for router logits [M, ld], or parts [n, M, ld] of them."""
+    """(ids int32 [M, top], weights fp32 [M, top]) for router logits [M, ld] (or [M, 1, ld]), or parts [n, M, ld] of several tokens' logits."""
+    in_parts = logits.dim() == 3 and logits.shape[1] != 1
+    return _moe_select(logits, router, *(logits.shape[:2] if in_parts else (1, logits.shape[0])))
+
+
+def _moe_select(logits, router, parts, M):
     lib = _lib.load_dense_library()
-    parts, M = (logits.shape[0], logits.shape[1]) if logits.dim() == 3 else (1, logits.shape[0])
     ids = torch.empty((M, router.top), dtype=torch.int32, device=logits.device)
     wts = torch.empty((M, router.top), dtype=torch.float32, device=logits.device)
     r = router.bind(logits)
@@ -314,16 +318,18 @@ def moe_select(logits, router):
 
 
 def moe_rows(h, logits, router, w_gate_up, w_down):
-    """Chosen experts' outputs in the element type [M * top, N] (row token * top + slot) and the router weights [M, top]."""
+    """Chosen experts' outputs in the element type [M * top, N] (row token * top + slot) and the router weights [M, top].  logits [M, ld]
+    or parts [n, M, ld] of them."""
     lib = _lib.load_dense_library()
     _need_cuda(h, w_gate_up, w_down)
     _same("moe_rows", w_gate_up, h, w_down)
     E, ff2, K = w_gate_up.shape
     ff, N, top = ff2 // 2, w_down.shape[1], router.top
-    if h.shape[1] != K or tuple(w_down.shape) != (E, N, ff) or E != router.experts or logits.shape[-2] != h.shape[0]:
-        raise ValueError("moe_rows: shapes of the rows and the experts do not match")
     M, dev, dt = h.shape[0], h.device, dtype_code(h)
-    ids, wts = moe_select(logits, router)
+    in_parts = logits.dim() == 3 and logits.shape[1] == M        # ([M, 1, ld], which is not, are rows)
+    if h.shape[1] != K or tuple(w_down.shape) != (E, N, ff) or E != router.experts or logits.shape[int(in_parts)] != M:
+        raise ValueError("moe_rows: shapes of the rows and the experts do not match")
+    ids, wts = _moe_select(logits, router, logits.shape[0] if in_parts else 1, M)
     entries = M * top
     tile_rows = lib.dlm_gemm_tile_rows(dt, entries // E, max(ff2, N), E)
     n_tiles = lib.dlm_moe_max_tiles(entries, E, tile_rows)

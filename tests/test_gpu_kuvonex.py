@@ -189,6 +189,23 @@ def test_routing_of_logits_in_parts(dense, experts, parts):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("M", [1, 2, 5])
+def test_logits_of_a_row_each_are_not_parts(dense, M):
+    """[M, 1, ld] are M tokens; [n, M, ld] parts of M, also beside the rows of one token."""
+    say("logits", M)
+    E, top, K, ff, N = 6, 2, 64, 64, 64
+    z = torch.randn((3, M, 16), generator=torch.Generator().manual_seed(M)).cuda()
+    spec = dense.RouterSpec(torch.zeros((E,), device="cuda"), E, top, 1, 1)
+    h, gu, down = rnd((M, K), 1), rnd((E, 2 * ff, K), 2, K ** -0.5), rnd((E, N, ff), 3, ff ** -0.5)
+    total = z[0] + z[1] + z[2]
+    want, rows = dense.moe_select(total, spec), dense.moe_rows(h, total, spec, gu, down)
+    for got in (dense.moe_select(total[:, None], spec), dense.moe_rows(h, total[:, None], spec, gu, down)[1:], dense.moe_rows(h, z, spec, gu, down)[1:]):
+        assert all(torch.equal(a, b) for a, b in zip(got, want[2 - len(got):])) and got[-1].shape == (M, top)
+    assert torch.equal(dense.moe_rows(h, total[:, None], spec, gu, down)[0], rows[0]) and torch.equal(dense.moe_rows(h, z, spec, gu, down)[0], rows[0])
+    with pytest.raises(ValueError):
+        dense.moe_rows(h, z.reshape(3 * M, 16), spec, gu, down)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("M,experts,top,groups,keep,K,ff,N", [(1, 10, 2, 2, 1, 64, 128, 128), (1, 16, 5, 4, 2, 1152, 576, 320), (2, 9, 2, 3, 1, 128, 64, 64),
                                                                (61, 6, 3, 6, 4, 192, 128, 192), (700, 5, 2, 1, 1, 64, 192, 64)])
