@@ -7,21 +7,25 @@
 //   (1 + diag(beta) A) U = diag(beta) (V - (k e^G) S)       u of the delta rule; U = V without it
 //   O = (q e^G) S + B U,    S' = e^(G_last) S + (k e^(G_last - G))^T U
 //
-// With U = V (one decay per head) S' needs nothing but a product of the chunk's own and a multiple of S:
+// so that everything but the products with S can be done for all chunks at once:
+//
+//   linear_chunk / delta_chunk   one workgroup per head and chunk: q e^G, (k e^(G_last - G))^T, B, e^(G_last), and U as
+//                                U0 - W S: U0 = V, or U0 = (1 + diag(beta) A)^-1 diag(beta) V and W the same of k e^G
+//   chunk_scan                   one workgroup per head and 16 value columns goes through the chunks: S stays in registers (and
+//                                in LDS as an operand)
+//
+// With U = V (one decay per head) S' needs nothing but a product of the chunk's own and a multiple of S, so a long portion's outputs need
+// not wait for a scan that makes products (in_parallel below says how long):
 //
 //   linear_state    one workgroup per head and chunk: (k e^(G_last - G))^T V
 //   linear_scan     every element of S on its own: the S in front of every chunk in place of its product
-//   linear_steps    instead of the two, for a few chunks: a workgroup's value columns of a head through all of them
+//   linear_steps    instead of the two, for one or two chunks of many heads: a workgroup's value columns of a head through all of them
 //   linear_output   one workgroup per head and chunk: O
 //
-// With the delta rule everything but the products with S can be done for all chunks at once:
-//
-//   delta_chunk     one workgroup per head and chunk: q e^G, (k e^(G_last - G))^T, B, e^(G_last), and U as U0 - W S:
-//                   U0 = (1 + diag(beta) A)^-1 diag(beta) V and W the same of k e^G
-//   delta_scan      one workgroup per head and 16 value columns goes through the chunks: S stays in registers (and in LDS as an operand)
+// Either way products and sums are the same ones in the same order, bit for bit.
 //
 // What bounds them: fp32 products (a CU does 256 flops a clock), S and the chunks' operands on their way through memory, and the chain of a scan over the
-// chunks.  2048 tokens, 16 heads of 128 / 128: one decay per head 17 + 14 + 25 us (89 with the scan of the delta rule, whose 128 workgroups do all
+// chunks.  2048 tokens, 16 heads of 128 / 128: one decay per head 17 + 14 + 25 us (the other form 82, whose 128 workgroups do all
 // of the products one chunk after the other), the delta rule 40 + 89 (its outputs in a launch of their own, S and U left in memory for it: 61 + 25 us instead of the
 // 89, and at 300 tokens 12 + 11 instead of 16: not taken).
 //
@@ -38,22 +42,18 @@ namespace {
 constexpr int kC = 64, kThreads = 256;
 constexpr float kLog2E = 1.4426950408889634f;
 
-// Work of one head and chunk of the delta rule, in floats (without it: S alone).  The matrices lie in the order in which waves read them as operands,
-// a kilobyte of neighbouring lanes per load: [16 rows][32 columns][half of 8 columns][lane][4]; u as it is added to a product:
-// [16 columns][16 tokens][lane][4 tokens].
+// Work of one head and chunk, in floats.  The matrices lie in the order in which waves read them as operands, a kilobyte of neighbouring
+// lanes per load: [16 rows][32 columns][half of 8 columns][lane][4]; u as it is added to a product: [16 columns][16 tokens][lane][4 tokens].
 struct ChunkLayout {
-    int dim, vdim;
+    int dim, vdim, delta;
     __host__ __device__ size_t q() const { return 0; }                                   // [kC][dim]
     __host__ __device__ size_t k() const { return (size_t)kC * dim; }                    // [dim][kC]
     __host__ __device__ size_t b() const { return k() + (size_t)kC * dim; }              // [kC][kC]
     __host__ __device__ size_t u() const { return b() + kC * kC; }                       // [kC][vdim]
     __host__ __device__ size_t e() const { return u() + (size_t)kC * vdim; }             // [dim]
     __host__ __device__ size_t w() const { return e() + dim; }                           // [kC][dim]
-    __host__ __device__ size_t size() const { return w() + (size_t)kC * dim; }
+    __host__ __device__ size_t size() const { return w() + (delta ? (size_t)kC * dim : 0); }
 };
-// floats of work of a head and chunk
-size_t chunk_work(const LinearArgs &a) { return a.z ? ChunkLayout{a.dim, a.vdim}.size() : (size_t)a.vdim * a.dim; }
-
 // Place of elements (row, column .. column + 3) of a matrix with `steps` times 32 columns.
 __device__ __forceinline__ int place_of(int row, int col, int steps) {
     return (((row >> 4) * steps + (col >> 5)) * 2 + ((col >> 2) & 1)) * 256 + (((col & 31) >> 3) * 16 + (row & 15)) * 4;
@@ -65,12 +65,77 @@ __device__ __forceinline__ void at_place(int slot, int steps, int &row, int &col
     col = 32 * step + 8 * (lane >> 4) + 4 * half;
 }
 
-// zeros of the blocks above the diagonal that the scan reads (columns 16 .. 31 of rows 0 .. 15, 48 .. 63 of rows 32 .. 47)
+// zeros of the blocks above the diagonal that products read all the same (columns 16 .. 31 of rows 0 .. 15, 48 .. 63 of rows 32 .. 47)
 __device__ __forceinline__ void clear_upper(float *b, int lane) {
     const int row = lane >> 2, c = 4 * (lane & 3);
     const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
     *reinterpret_cast<floatx4 *>(b + place_of(row, 16 + c, 2)) = zero;
     *reinterpret_cast<floatx4 *>(b + place_of(32 + row, 48 + c, 2)) = zero;
+}
+
+// blockIdx.x = chunk, blockIdx.y = head.  One decay per head, u = v.
+template <class T, int ND>
+__global__ void __launch_bounds__(kThreads) linear_chunk_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work) {
+    constexpr int D = 64 * ND, P = D + 4;
+    __shared__ __attribute__((aligned(16))) float ks[kC][P];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ql = lane & 15, g = lane >> 4;
+    const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC, n = a.M - m0 < kC ? a.M - m0 : kC;
+    const ChunkLayout lay{D, a.vdim, 0};
+    float *out = work + ((size_t)h * gridDim.x + blockIdx.x) * lay.size();
+    const float ld = a.log2_decay[h];
+    auto power = [&](int e) { return __builtin_amdgcn_exp2f(ld * (float)e); };
+    q += (size_t)m0 * a.ld + (size_t)kh * D;
+    k += (size_t)m0 * a.ld + (size_t)kh * D;
+    v += (size_t)m0 * a.ld + (size_t)h * a.vdim;
+    for (int i = tid; i < kC * D / 8; i += kThreads) {
+        const int r = i / (D / 8), c = 8 * (i % (D / 8));
+        float y[8];
+        unpack8(r < n ? load8(k + (size_t)r * a.ld + c) : zero8<T>(), y);
+        store8(&ks[r][c], pack8<float>(y));
+    }
+    for (int i = tid; i < kC * D / 4; i += kThreads) {
+        int r, c;
+        at_place(i, 2 * ND, r, c);
+        float x[4] = {0.f, 0.f, 0.f, 0.f};
+        if (r < n) load4(q + (size_t)r * a.ld + c, x);
+        const float f = power(r + 1);
+        store4(out + lay.q() + 4 * i, x[0] * f, x[1] * f, x[2] * f, x[3] * f);
+    }
+    for (int i = tid; i < kC * a.vdim / 4; i += kThreads) {
+        const int t = 16 * ((i >> 6) & 3) + 4 * ((i & 63) >> 4), c = 16 * (i >> 8) + (i & 15);
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = t + e < n ? to_float(v[(size_t)(t + e) * a.ld + c]) : 0.f;
+        store4(out + lay.u() + 4 * i, x[0], x[1], x[2], x[3]);
+    }
+    if (tid < D) out[lay.e() + tid] = power(n);
+    // scores: rows of one wave against the blocks up to the diagonal (first operand: k, so that a lane owns one query)
+    const int qi = 16 * wave + ql;
+    const T *qr = q + (size_t)(qi < n ? qi : n - 1) * a.ld + 8 * g;
+    for (int bj = 0; bj <= wave; ++bj) {
+        const int kj = 16 * bj + ql;
+        const T *kr = k + (size_t)(kj < n ? kj : n - 1) * a.ld + 8 * g;
+        floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 2 * ND; ++t) s = mma32(load8(kr + 32 * t), load8(qr + 32 * t), s);
+        float w[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * bj + 4 * g + r;
+            w[r] = j <= qi && j < n && qi < n ? s[r] * power(qi - j) : 0.f;
+        }
+        store4(out + lay.b() + place_of(qi, 16 * bj + 4 * g, 2), w[0], w[1], w[2], w[3]);
+    }
+    if (wave == 0) clear_upper(out + lay.b(), lane);
+    __syncthreads();
+    for (int i = tid; i < D * kC / 4; i += kThreads) {
+        int r, c;
+        at_place(i, 2, c, r);
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = r + e < n ? ks[r + e][c] * power(n - 1 - r - e) : 0.f;
+        store4(out + lay.k() + 4 * i, x[0], x[1], x[2], x[3]);
+    }
 }
 
 // First operand of a product, in the order of ChunkLayout: 16 rows and 32 columns
@@ -181,10 +246,7 @@ __global__ void __launch_bounds__(kThreads) linear_state_kernel(const LinearArgs
     }
 }
 
-// The state kernel and the scan in one, for one or two chunks: four times 16 value columns of a head, the chunks one after the other.  A prompt through
-// four layers of width 2048, 16 heads of 128 / 128 in two of them: 128 tokens 558 us (557 before outputs were a launch of their own), 256 tokens 690 with
-// it and 673 with the two launches (677 before); the host, which narrow models' short portions wait for, is spared a launch.
-constexpr int kFewChunks = 2;
+// The state kernel and the scan in one, for one or two chunks of many heads: four times 16 value columns of a head, the chunks one after the other.
 template <class T, int ND>
 __global__ void __launch_bounds__(kThreads) linear_steps_kernel(const LinearArgs a, const T *q, const T *k, const T *v, float *work, int chunks, bool first) {
     constexpr int D = 64 * ND, P = D + 4, KS = 2 * ND, NC = 4 * ND;
@@ -370,7 +432,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) delta_chunk_
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, kh = h / (a.heads / a.k_heads), m0 = blockIdx.x * kC, n = a.M - m0 < kC ? a.M - m0 : kC;
-    const ChunkLayout lay{D, a.vdim};
+    const ChunkLayout lay{D, a.vdim, 1};
     float *out = work + ((size_t)h * gridDim.x + blockIdx.x) * lay.size();
     const float ea = -expf(a.a_log[h]) * kLog2E;
     q += (size_t)m0 * a.ld + (size_t)kh * D;
@@ -601,8 +663,8 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) delta_chunk_
 // A wave requests the operands of the next chunk as soon as it has multiplied those of this one, products with S while those with U
 // are made and the other way round.  (Behind the last chunk that one is fetched again rather than nothing, so that the number of loads
 // in flight is known at every wait.)
-template <int ND>
-__global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const LinearArgs a, const float *work, int chunks, bool first, float *o) {
+template <int ND, bool DELTA>
+__global__ void __launch_bounds__(2 * kThreads, 1) chunk_scan_kernel(const LinearArgs a, const float *work, int chunks, bool first, float *o) {
     constexpr int D = 64 * ND, KS = 2 * ND;
     __shared__ __attribute__((aligned(16))) float ss[2][16][D + 4], us[2][16][kC + 4];
     const int tid = threadIdx.x, lane = tid & 63, ql = lane & 15, g = lane >> 4;
@@ -610,7 +672,7 @@ __global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const Linea
     const int tiles = a.vdim / 16, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
     const int h = 8 * (at / tiles) + xcd, v0 = 16 * (at % tiles), tok = 16 * wave;
     if (h >= a.heads) return;
-    const ChunkLayout lay{D, a.vdim};
+    const ChunkLayout lay{D, a.vdim, DELTA};
     work += (size_t)h * chunks * lay.size();
     const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
     // m S (two chains), and the operands from LDS in registers before the first product: the compiler would fetch them two by two
@@ -635,11 +697,13 @@ __global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const Linea
             s[c] = from_zero ? zero : *reinterpret_cast<const floatx4 *>(st + 16 * (wave + 4 * c));
             *reinterpret_cast<floatx4 *>(&ss[0][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
         }
-        Vec8<float> w[KS], k[ND][2];
+        Vec8<float> w[KS], k[ND][2];   // (w: the delta rule only)
         floatx4 u, e[ND];
         auto fetch_w = [&](const float *p) {
+            if constexpr (DELTA) {
 #pragma unroll
-            for (int t = 0; t < KS; ++t) w[t] = operand(p + lay.w(), wave * KS + t, lane);
+                for (int t = 0; t < KS; ++t) w[t] = operand(p + lay.w(), wave * KS + t, lane);
+            }
             u = *reinterpret_cast<const floatx4 *>(p + lay.u() + ((v0 / 16 * 4 + wave) * 64 + lane) * 4);
 #pragma unroll
             for (int c = 0; c < ND; ++c) e[c] = *reinterpret_cast<const floatx4 *>(p + lay.e() + 16 * (wave + 4 * c) + 4 * g);
@@ -652,28 +716,46 @@ __global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const Linea
         };
         fetch_w(work);
         fetch_k(work);
+        if constexpr (!DELTA) *reinterpret_cast<floatx4 *>(&us[0][ql][tok + 4 * g]) = u;
         __syncthreads();
         for (int chunk = 0; chunk < chunks; ++chunk) {
             const int b = chunk & 1;
             work += chunk + 1 < chunks ? lay.size() : 0;
+            if constexpr (DELTA) {
 #pragma unroll
-            for (int c = 0; c < ND; ++c) s[c] *= e[c];
-            floatx4 x = zero, y = zero;
-            times_state(w, ss[b], x, y);
-            *reinterpret_cast<floatx4 *>(&us[b][ql][tok + 4 * g]) = u - (x + y);
-            fetch_w(work);
-            __syncthreads();   // U is there
-            const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
-            __builtin_amdgcn_sched_barrier(0);
+                for (int c = 0; c < ND; ++c) s[c] *= e[c];
+                floatx4 x = zero, y = zero;
+                times_state(w, ss[b], x, y);
+                *reinterpret_cast<floatx4 *>(&us[b][ql][tok + 4 * g]) = u - (x + y);
+                fetch_w(work);
+                __syncthreads();   // U is there
+                const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < ND; ++c) s[c] = mma32(k[c][0], ua, s[c]);
+                for (int c = 0; c < ND; ++c) s[c] = mma32(k[c][0], ua, s[c]);
 #pragma unroll
-            for (int c = 0; c < ND; ++c) {
-                s[c] = mma32(k[c][1], ub, s[c]);
-                *reinterpret_cast<floatx4 *>(&ss[b ^ 1][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
+                for (int c = 0; c < ND; ++c) {
+                    s[c] = mma32(k[c][1], ub, s[c]);
+                    *reinterpret_cast<floatx4 *>(&ss[b ^ 1][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
+                }
+            } else {               // (the products do not wait for S, and are added to it as linear_scan does)
+                floatx4 x[ND], now[ND];
+#pragma unroll
+                for (int c = 0; c < ND; ++c) now[c] = e[c];
+                fetch_w(work);
+                const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < ND; ++c) x[c] = mma32(k[c][0], ua, zero);
+#pragma unroll
+                for (int c = 0; c < ND; ++c) {
+                    s[c] = s[c] * now[c] + mma32(k[c][1], ub, x[c]);
+                    *reinterpret_cast<floatx4 *>(&ss[b ^ 1][ql][16 * (wave + 4 * c) + 4 * g]) = s[c];
+                }
             }
             fetch_k(work);
-            __syncthreads();       // the next S is there, this one has been read
+            if constexpr (!DELTA) *reinterpret_cast<floatx4 *>(&us[b ^ 1][ql][tok + 4 * g]) = u;
+            __syncthreads();       // the next S (and, without the delta rule, U) is there, this one has been read
         }
 #pragma unroll
         for (int c = 0; c < ND; ++c) *reinterpret_cast<floatx4 *>(st + 16 * (wave + 4 * c)) = s[c];
@@ -697,7 +779,7 @@ __global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const Linea
             floatx4 x = zero, y = zero;
             times_state(q, ss[b], x, y);
             fetch_q(work);
-            __syncthreads();
+            if constexpr (DELTA) __syncthreads();
             const Vec8<float> ua = load8(&us[b][ql][8 * g]), ub = load8(&us[b][ql][32 + 8 * g]);
             x = mma32(m[0], ua, x);
             if (wave >= 2) y = mma32(m[1], ub, y);
@@ -712,16 +794,40 @@ __global__ void __launch_bounds__(2 * kThreads, 1) delta_scan_kernel(const Linea
     }
 }
 
+// With one decay per head, how a portion goes through: in_steps linear_steps and linear_output, in_parallel linear_state, linear_scan and
+// linear_output, else linear_chunk and chunk_scan.  A chunk costs the scan 1.3 us (64 channels) or 1.9 (128), more where there are more workgroups than
+// CUs.  The products of all chunks in launches of their own cost much the same up to 8 chunks of 16 heads, but their workgroups grow with
+// the value columns, whose S then costs as much memory as what the scan reads.  us, parallel / scan, 8 heads: 64 / 64 3 chunks 13 / 14, 128 / 128 3 chunks
+// 23 / 22, 5 chunks 24 / 26, 32 chunks 34 / 75, 128 / 256 5 chunks 38 / 31, 12 chunks 43 / 45, 128 / 512 16 chunks 72 / 70, 32 chunks 85 / 96, 16 heads
+// of it in fp32 24 chunks 142 / 118; 64 heads of 128 / 128 5 chunks 44 / 44, 32 chunks 172 / 224.  In steps / scan, 2 chunks: 16 heads of 128 / 128 23 / 21, 64 heads
+// 25 / 32, 128 heads 28 / 40; 1 chunk of 64 heads 21 / 22, 128 heads 24 / 32.
+int chunks_of(const LinearArgs &a) { return (a.M + kC - 1) / kC; }
+bool in_steps(const LinearArgs &a) { return chunks_of(a) <= 2 && (long)a.heads * chunks_of(a) >= 128; }
+// the first number of chunks that takes the parallel form
+int parallel_from(const LinearArgs &a) {
+    const int tiles = a.vdim / 16, rounds = ((long)a.heads * tiles + 255) / 256 < 3 ? (int)(((long)a.heads * tiles + 255) / 256) : 3;
+    if (tiles > 16) return tiles;
+    const int least = (5 * tiles + 7) / 8 < 3 ? 3 : (5 * tiles + 7) / 8;
+    return (least + rounds - 1) / rounds;
+}
+bool in_parallel(const LinearArgs &a) { return chunks_of(a) >= parallel_from(a); }
+
+// floats of work of a head and chunk
+size_t chunk_work(const LinearArgs &a) {
+    return !a.z && (in_steps(a) || in_parallel(a)) ? (size_t)a.vdim * a.dim : ChunkLayout{a.dim, a.vdim, a.z != nullptr}.size();
+}
+
 // Chunks that are worked on at once: their operands stay within reach of the last-level cache.
 int segment_chunks(const LinearArgs &a) {
     const size_t per = chunk_work(a) * sizeof(float) * a.heads;
-    const int all = (a.M + kC - 1) / kC, fit = (int)((size_t)160 * 1024 * 1024 / per);
+    const int all = chunks_of(a), fit = (int)((size_t)160 * 1024 * 1024 / per);
     return all < fit ? all : fit < 8 ? (all < 8 ? all : 8) : fit;
 }
 
 template <class T, int ND>
 hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
     const int seg = segment_chunks(a), M = a.M;
+    const bool steps = in_steps(a), parallel = in_parallel(a);
     const T *qkv = static_cast<const T *>(a.qkv), *beta = static_cast<const T *>(a.beta);
     constexpr size_t lds = sizeof(DeltaLds<T, ND>);
     if (a.z && lds > 48 * 1024) {
@@ -731,7 +837,7 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
     for (int m0 = 0; m0 < M; m0 += seg * kC) {
         a.M = M - m0 < seg * kC ? M - m0 : seg * kC;
         const int n = (a.M + kC - 1) / kC;
-        const dim3 grid(n, a.heads);
+        const dim3 grid(n, a.heads), scan(8 * ((a.heads + 7) / 8) * (a.vdim / 16));
         const bool wide = a.vdim > 64;   // two 16-column tiles to a wave: past that all four waves have some
         const T *q = qkv + (size_t)m0 * a.ld + a.q_off, *k = qkv + (size_t)m0 * a.ld + a.k_off, *v = qkv + (size_t)m0 * a.ld + a.v_off;
         float *om = o + (size_t)m0 * a.heads * a.vdim;
@@ -741,15 +847,17 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
             b.z += (size_t)m0 * a.heads * a.dim;
             b.factors += (size_t)m0 * 2 * a.k_heads;
             hipLaunchKernelGGL((delta_chunk_kernel<T, ND>), grid, dim3(kThreads), lds, stream, b, q, k, v, beta + (size_t)m0 * a.ld_beta, work);
-            hipLaunchKernelGGL((delta_scan_kernel<ND>), dim3(8 * ((a.heads + 7) / 8) * (a.vdim / 16)), dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
-        } else {
-            if (n <= kFewChunks) {
-                hipLaunchKernelGGL((linear_steps_kernel<T, ND>), dim3((a.vdim + 63) / 64, a.heads), dim3(kThreads), 0, stream, a, q, k, v, work, n, m0 == 0);
-            } else {
-                run(wide ? &linear_state_kernel<T, ND, 2> : &linear_state_kernel<T, ND, 1>, a, q, k, v, work);
-                hipLaunchKernelGGL((linear_scan_kernel<ND>), dim3(a.vdim * a.dim / (4 * kThreads), a.heads), dim3(kThreads), 0, stream, a, work, n, m0 == 0);
-            }
+            hipLaunchKernelGGL((chunk_scan_kernel<ND, true>), scan, dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
+        } else if (steps) {
+            hipLaunchKernelGGL((linear_steps_kernel<T, ND>), dim3((a.vdim + 63) / 64, a.heads), dim3(kThreads), 0, stream, a, q, k, v, work, n, m0 == 0);
             run(&linear_output_kernel<T, ND>, a, q, k, v, work, om);
+        } else if (parallel) {
+            run(wide ? &linear_state_kernel<T, ND, 2> : &linear_state_kernel<T, ND, 1>, a, q, k, v, work);
+            hipLaunchKernelGGL((linear_scan_kernel<ND>), dim3(a.vdim * a.dim / (4 * kThreads), a.heads), dim3(kThreads), 0, stream, a, work, n, m0 == 0);
+            run(&linear_output_kernel<T, ND>, a, q, k, v, work, om);
+        } else {
+            run(&linear_chunk_kernel<T, ND>, a, q, k, v, work);
+            hipLaunchKernelGGL((chunk_scan_kernel<ND, false>), scan, dim3(2 * kThreads), 0, stream, a, work, n, m0 == 0, om);
         }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -761,8 +869,16 @@ hipError_t chunks(LinearArgs a, float *work, float *o, hipStream_t stream) {
 
 bool linear_chunks_supported(const LinearArgs &a) { return a.dim <= 128; }
 
+// (no less for a longer portion, whatever its form: work that is enough for the longest one is enough for all)
 size_t linear_chunk_bytes(const LinearArgs &a) {
-    return chunk_work(a) * sizeof(float) * a.heads * segment_chunks(a);
+    size_t most = 0;
+    for (const int chunks : {1, parallel_from(a) - 1, chunks_of(a)}) {
+        LinearArgs b = a;
+        b.M = kC * chunks < a.M ? kC * chunks : a.M;
+        const size_t bytes = b.M > 0 ? chunk_work(b) * sizeof(float) * b.heads * segment_chunks(b) : 0;
+        most = bytes > most ? bytes : most;
+    }
+    return most;
 }
 
 hipError_t launch_linear_chunks(int dtype, const LinearArgs &a, void *work, float *o, hipStream_t stream) {

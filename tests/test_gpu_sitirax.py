@@ -432,6 +432,24 @@ def test_one_decay_per_head_in_chunks(dense, dtype, heads, dim, vdim):
         close(x.final(), state, dtype, "state", **STATE_TOL)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("heads,dim,vdim,least", [(2, 64, 32, 3), (3, 128, 128, 5), (17, 64, 256, 5), (1, 128, 272, 17), (1, 64, 320, 20), (64, 64, 32, 2)])
+def test_one_decay_per_head_in_either_form(dense, dtype, heads, dim, vdim, least):
+    """From `least` chunks on a portion goes another way (its products on all CUs; two chunks of 64 heads in steps) than its parts, one
+    chunk after the other: the same numbers, to the bit."""
+    say("either form", dtype, heads, dim, vdim)
+    T = 64 * least - 1
+    x = Recurrence(dense, "lightning", heads, heads, dim, vdim, T, dtype, seed=least, far=[(T - 1, 0), (T - 2, 63), (65, 64)])
+    want, state = x.want()
+    x.state.fill_(float("nan"))
+    whole, left = x.run(0, T, True), x.state.clone()
+    close(whole, want, dtype, "whole", **STATE_TOL)
+    close(x.final(), state, dtype, "state", **STATE_TOL)
+    for cuts in [(0, 64 * (least - 1), T)] + [(0, 64, 64 * (least - 1), T)] * (least > 2):
+        x.state.fill_(float("nan"))
+        assert torch.equal(torch.cat([x.run(a, b, True) for a, b in zip(cuts, cuts[1:])]), whole) and torch.equal(x.state, left), cuts
+
+
 def test_one_decay_per_head_in_two_segments(dense):
     say("segments, one decay per head")
     x = Recurrence(dense, "lightning", 1024, 1024, 64, 64, 650, F32, seed=10)      # ten chunks to a segment

@@ -208,6 +208,18 @@ def test_sizes_without_a_kernel_are_refused_when_the_model_is_made():
             sitirax.SitiraxModel(cfg, lambda n, s: torch.from_numpy(w[n]), torch.float32, "cpu")
 
 
+@pytest.mark.parametrize("heads", [1, 16, 64, 128, 1024])
+def test_work_of_a_recurrence_is_no_less_for_a_longer_portion(heads):
+    """Portions of other lengths take other forms; whoever allocates for the longest one has enough for all."""
+    from air_hip import _lib
+
+    lib = _lib.load_dense_library()
+    for dim, vdim, z in ((64, 32, None), (64, 256, None), (128, 128, None), (128, 272, None), (128, 128, 16)):
+        sizes = [lib.dlm_recurrence_chunk_bytes(ctypes.byref(_lib.RecurrenceArgs(heads=heads, k_heads=heads, dim=dim, vdim=vdim, M=M, z=z)))
+                 for M in [*range(1, 2400, 21), 30000]]
+        assert sizes == sorted(sizes) and sizes[0] > 0, (dim, vdim)
+
+
 def test_abi_rejects_bad_arguments_before_touching_the_gpu():
     from air_hip import _lib
 
