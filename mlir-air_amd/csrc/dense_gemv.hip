@@ -52,46 +52,62 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
     return s;
 }
 
-// x into LDS (K elements, zeros up to the next piece).  What it is made of is asked for in front of the first weights (a wave's loads return in
-// order) and all at once, up to 2048 elements of it (as they are: 8192) kept in registers from one pass over x to the next.  (Behind the weights, a
+// x into LDS (K elements, zeros up to the next piece).  QUADS > 0: for up to 1024 QUADS elements.  What x is made of is asked for in front of the
+// first weights (a wave's loads return in order) and all at once, and kept in registers from one pass over x to the next.  (Behind the weights, a
 // round trip per 1024 elements and pass: gate and up of 2 x 8192 x 2048 behind a norm 14.1 -> 12.8 us = 5.3 TB/s, a router of 64 x 2048 behind a residual 4.5 -> 3.3 us.)
-template <class T, int MODE>
+// QUADS 0, any length: every pass asks for what it uses, behind the weights.  (Registers in batches, every pass all operands of them anew,
+// took 13.5 us instead of 10.5 for 2112 x 5120 behind a final norm.)  An x that is there already comes as it is, 8192 elements at a time.
+template <class T, int MODE, int QUADS>
 struct Intake {
-    static constexpr int NB = MODE == kIntakePlain ? 8 : 2, kStep = 4 * kGemvThreads;   // quads of a thread in a batch; elements between them
+    static constexpr int kKept = QUADS > 0 ? QUADS : 1, kStep = 4 * kGemvThreads;   // quads of a thread; elements between them
     static constexpr bool kRow = MODE == kIntakeEmbed || MODE == kIntakeNormedEmbed, kNormed = MODE == kIntakeNormed || MODE == kIntakeNormedEmbed;
+    static constexpr bool kPlain = MODE == kIntakePlain, kAhead = kPlain || QUADS > 0;
+    static constexpr int kY = 1, kRest = 2, kLast = 4, kAll = 7;   // operands: y; what else makes the value; final_w
+    struct Operands {
+        floatx4 res, y, norm, last;
+    };
     const GemvParams<T> &p;
     T *xs;
     float *red;
-    Vec8<T> x[NB / 2];
-    floatx4 res[NB], y[NB], norm[NB], last[NB];
+    const T *row = nullptr;   // of the embedding
+    Vec8<T> x[4];
+    Operands kept[kKept];
 
-    __device__ __forceinline__ int quad(int q, int b) const { return 4 * (int)threadIdx.x + (q * NB + b) * kStep; }
     __device__ __forceinline__ static floatx4 quad_of(const float *v) { return *reinterpret_cast<const floatx4 *>(v); }
-    // batch q of the operands; past the end the last ones
-    __device__ __forceinline__ void load(int q) {
-        if constexpr (MODE == kIntakePlain) {
-#pragma unroll
-            for (int b = 0; b < NB / 2; ++b) {
-                const int i = 2 * (4 * (int)threadIdx.x + (q * NB / 2 + b) * kStep);
-                x[b] = load8(p.x + (i < p.K ? i : p.K - 8));
-            }
-            return;
+    template <int WHAT>
+    __device__ __forceinline__ Operands load(int i) const {
+        Operands o;
+        if constexpr (kRow) {
+            float e[4];
+            load4(row + i, e);
+            o.res = floatx4{e[0], e[1], e[2], e[3]} * p.scale;
+        } else {
+            // (without y: read all the same where operands are kept, and not used)
+            if constexpr (WHAT & kRest) o.res = quad_of(p.res + i);
+            if (WHAT & kY)
+                if (kAhead || p.y) o.y = quad_of((kAhead && !p.y ? p.res : p.y) + i);
+            if ((MODE == kIntakeResidual || MODE == kIntakeFinal) && (WHAT & kRest))
+                if (kAhead || p.y) o.norm = quad_of((kAhead && !p.y ? p.res : p.norm_w) + i);
         }
-        const T *row = kRow ? p.embed + (size_t)p.token[0] * p.K : nullptr;
-        const float *ys = p.y ? p.y : p.res, *norms = p.y ? p.norm_w : p.res;   // (without y: read all the same, and not used)
+        if constexpr ((MODE == kIntakeFinal || kNormed) && (WHAT & kLast)) o.last = quad_of(p.final_w + i);
+        return o;
+    }
+    __device__ __forceinline__ void load_plain(int q) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int i = quad(q, b) < p.K ? quad(q, b) : p.K - 4;
-            if constexpr (kRow) {
-                float e[4];
-                load4(row + i, e);
-                res[b] = floatx4{e[0], e[1], e[2], e[3]} * p.scale;
-            } else {
-                res[b] = quad_of(p.res + i);
-                y[b] = quad_of(ys + i);
+        for (int b = 0; b < 4; ++b) {
+            const int i = 8 * ((int)threadIdx.x + (4 * q + b) * kGemvThreads);
+            x[b] = load8(p.x + (i < p.K ? i : p.K - 8));
+        }
+    }
+    __device__ __forceinline__ void begin() {
+        if constexpr (kRow) row = p.embed + (size_t)p.token[0] * p.K;
+        if constexpr (kPlain) load_plain(0);
+        else if constexpr (kAhead) {
+#pragma unroll
+            for (int b = 0; b < kKept; ++b) {
+                const int i = 4 * (int)threadIdx.x + b * kStep;
+                kept[b] = load<kAll>(i < p.K ? i : p.K - 4);   // (past the end the last ones)
             }
-            if constexpr (MODE == kIntakeResidual || MODE == kIntakeFinal) norm[b] = quad_of(norms + i);
-            if constexpr (MODE == kIntakeFinal || kNormed) last[b] = quad_of(p.final_w + i);
         }
     }
     __device__ __forceinline__ static float squares(floatx4 v, float ss) {
@@ -100,49 +116,46 @@ struct Intake {
         return ss;
     }
     __device__ __forceinline__ float rstd_of(float ss) const { return 1.0f / sqrtf(block_sum(ss, red) / (float)p.width + p.eps); }
-    // f(batch's index b, first element) over all of x; `again`: the operands of the batch are to be loaded (if they are not the only one's)
-    template <class F>
-    __device__ __forceinline__ void pass(bool again, F f) {
-        const int batches = (p.K + NB * kStep - 1) / (NB * kStep);
-        for (int q = 0; q < batches; ++q) {
-            if (q > 0 || (again && batches > 1)) load(q);
+    // f(operands, first element) over all of x
+    template <int WHAT, class F>
+    __device__ __forceinline__ void pass(F f) const {
+        if constexpr (kAhead) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-                if (quad(q, b) < p.K) f(b, quad(q, b));
+            for (int b = 0; b < kKept; ++b)
+                if (const int i = 4 * (int)threadIdx.x + b * kStep; i < p.K) f(kept[b], i);
+        } else {
+            for (int i = 4 * (int)threadIdx.x; i < p.K; i += kStep) f(load<WHAT>(i), i);
         }
     }
     __device__ __forceinline__ void finish() {
         const int kl = (p.K + kPiece - 1) / kPiece * kPiece;
         for (int i = p.K + 8 * (int)threadIdx.x; i < kl; i += 8 * kGemvThreads) store8(xs + i, zero8<T>());
-        if constexpr (MODE == kIntakePlain) {
-            for (int q = 0; q * NB * kStep < p.K; ++q) {
-                if (q > 0) load(q);
+        if constexpr (kPlain) {
+            for (int q = 0; q * 4 * 8 * kGemvThreads < p.K; ++q) {
+                if (q > 0) load_plain(q);
 #pragma unroll
-                for (int b = 0; b < NB / 2; ++b) {
-                    const int i = 2 * (4 * (int)threadIdx.x + (q * NB / 2 + b) * kStep);
+                for (int b = 0; b < 4; ++b) {
+                    const int i = 8 * ((int)threadIdx.x + (4 * q + b) * kGemvThreads);
                     if (i < p.K) store8(xs + i, x[b]);
                 }
             }
             return;
         }
-        // the new residual, kept in `res`
         float rstd = 0.f;
-        bool again = false;   // behind a first pass over several batches
         if constexpr (MODE == kIntakeResidual || MODE == kIntakeFinal) {
             if (p.y) {
                 float ss = 0.f;
-                pass(false, [&](int b, int) { ss = squares(y[b], ss); });
+                pass<kY>([&](const Operands &o, int) { ss = squares(o.y, ss); });
                 rstd = rstd_of(ss);
-                again = true;
             }
         }
-        auto value = [&](int b) {
-            if constexpr (kRow) return res[b];
-            if constexpr (MODE == kIntakeNormed) return p.y ? res[b] + y[b] : res[b];
-            floatx4 v = res[b];
+        auto value = [&](const Operands &o) {   // the new residual
+            if constexpr (kRow) return o.res;
+            if constexpr (MODE == kIntakeNormed) return p.y ? o.res + o.y : o.res;
+            floatx4 v = o.res;
             if (p.y) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = fmaf(y[b][j] * rstd, norm[b][j], v[j]);
+                for (int j = 0; j < 4; ++j) v[j] = fmaf(o.y[j] * rstd, o.norm[j], v[j]);
             }
             return v;
         };
@@ -153,22 +166,22 @@ struct Intake {
                 if (p.h_out) store4(p.h_out + i, v[0], v[1], v[2], v[3]);
         };
         if constexpr (MODE == kIntakeEmbed || MODE == kIntakeResidual) {
-            pass(again, [&](int b, int i) {
-                const floatx4 v = value(b);
+            pass<kY | kRest>([&](const Operands &o, int i) {
+                const floatx4 v = value(o);
                 store4(xs + i, v[0], v[1], v[2], v[3]);
                 keep(i, v);
             });
         } else {
             float ss = 0.f;
-            pass(again, [&](int b, int i) {
-                const floatx4 v = value(b);
+            pass<kY | kRest>([&](const Operands &o, int i) {
+                const floatx4 v = value(o);
                 ss = squares(v, ss);
                 if constexpr (kNormed) keep(i, v);
             });
             const float r2 = rstd_of(ss);
-            pass(true, [&](int b, int i) {
-                const floatx4 v = value(b), w = last[b];
-                store4(xs + i, v[0] * r2 * w[0], v[1] * r2 * w[1], v[2] * r2 * w[2], v[3] * r2 * w[3]);
+            pass<kAll>([&](const Operands &o, int i) {
+                const floatx4 v = value(o);
+                store4(xs + i, v[0] * r2 * o.last[0], v[1] * r2 * o.last[1], v[2] * r2 * o.last[2], v[3] * r2 * o.last[3]);
             });
         }
     }
@@ -191,7 +204,7 @@ __device__ __forceinline__ void request(Vec8<T> (&w)[R][U], const T *base, int K
     }
 }
 
-template <class T, int R, int U, int MODE, bool PAIR>
+template <class T, int R, int U, int MODE, bool PAIR, int QUADS>
 __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvParams<T> p) {
     extern __shared__ __attribute__((aligned(16))) char gemv_lds[];
     __shared__ float red[kGemvWaves];
@@ -201,8 +214,8 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
     const int pieces = (p.K + kPiece - 1) / kPiece;
     int g = blockIdx.x * kGemvWaves + wave;
     Vec8<T> w[R][U];
-    Intake<T, MODE> in{p, xs, red};
-    in.load(0);
+    Intake<T, MODE, QUADS> in{p, xs, red};
+    in.begin();
     __builtin_amdgcn_sched_barrier(0);
     request<T, R, U, PAIR>(w, p.w, p.K, p.N, g * R, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -286,7 +299,7 @@ __global__ void __launch_bounds__(1024) argmax_keys_kernel(const unsigned long l
     }
 }
 
-template <class T, int R, int U>
+template <class T, int R, int U, int QUADS>
 hipError_t launch_mode(const GemvParams<T> &p, int mode, int grid, size_t lds, hipStream_t stream) {
     auto run = [&](auto kernel) {
         if (lds > 48 * 1024) {
@@ -298,19 +311,31 @@ hipError_t launch_mode(const GemvParams<T> &p, int mode, int grid, size_t lds, h
     };
     if (p.ro.gate) {
         if constexpr (R >= 2)
-            return mode != kIntakeNormed ? run(&dense_gemv_kernel<T, R, U, kIntakePlain, true>)
-                   : p.embed             ? run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, true>)
-                                         : run(&dense_gemv_kernel<T, R, U, kIntakeNormed, true>);
+            return mode != kIntakeNormed ? run(&dense_gemv_kernel<T, R, U, kIntakePlain, true, 2>)
+                   : p.embed             ? run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, true, QUADS>)
+                                         : run(&dense_gemv_kernel<T, R, U, kIntakeNormed, true, QUADS>);
         return hipErrorInvalidValue;
     }
-    switch (mode == kIntakeNormed && p.embed ? (int)kIntakeNormedEmbed : mode) {
-        case kIntakePlain: return run(&dense_gemv_kernel<T, R, U, kIntakePlain, false>);
-        case kIntakeResidual: return run(&dense_gemv_kernel<T, R, U, kIntakeResidual, false>);
-        case kIntakeEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeEmbed, false>);
-        case kIntakeNormed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormed, false>);
-        case kIntakeNormedEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, false>);
-        default: return run(&dense_gemv_kernel<T, R, U, kIntakeFinal, false>);
-    }
+    if constexpr (R > 1 && QUADS != 2) return hipErrorInvalidValue;   // (without a gate rows past 2048 come one to a wave)
+    else
+        switch (mode == kIntakeNormed && p.embed ? (int)kIntakeNormedEmbed : mode) {
+            case kIntakePlain: return run(&dense_gemv_kernel<T, R, U, kIntakePlain, false, 2>);
+            case kIntakeResidual: return run(&dense_gemv_kernel<T, R, U, kIntakeResidual, false, QUADS>);
+            case kIntakeEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeEmbed, false, QUADS>);
+            case kIntakeNormed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormed, false, QUADS>);
+            case kIntakeNormedEmbed: return run(&dense_gemv_kernel<T, R, U, kIntakeNormedEmbed, false, QUADS>);
+            default: return run(&dense_gemv_kernel<T, R, U, kIntakeFinal, false, QUADS>);
+        }
+}
+
+// By the length of x: two or four quads of its operands in a thread's registers (four: up to 150, three waves to a SIMD in fp32), which is faster wherever they
+// fit, or passes that ask for them.  4096 x 4096 behind a final norm, four quads / passes / passes with batches of two quads: 10.2 / 11.6 / 14.7 us,
+// fp32 15.7 / 20.8 / 21.0; 64 x 4096 4.2 / 5.9 / 5.7; 2112 x 5120, passes / batches of four quads / of two: 10.5 / 15.3 / 13.5.
+template <class T, int R, int U>
+hipError_t launch_length(const GemvParams<T> &p, int mode, int grid, size_t lds, hipStream_t stream) {
+    if (p.K <= 2048) return launch_mode<T, R, U, 2>(p, mode, grid, lds, stream);
+    if (p.K <= 4096) return launch_mode<T, R, U, 4>(p, mode, grid, lds, stream);
+    return launch_mode<T, R, U, 0>(p, mode, grid, lds, stream);
 }
 
 int rows_per_wave(int K, int N) { return K > 2048 || N < 512 ? 1 : K > 1024 ? 2 : 4; }
@@ -344,9 +369,9 @@ hipError_t launch_typed(const void *w, const RowIntake &in, void *out, float *ou
     const int need = (p.groups + kGemvWaves - 1) / kGemvWaves, grid = need < kMaxBlocks ? need : kMaxBlocks;
     const size_t lds = (size_t)((K + kPiece - 1) / kPiece) * kPiece * sizeof(T);
     switch (R) {
-        case 1: return launch_mode<T, 1, 8>(p, in.mode, grid, lds, stream);
-        case 2: return launch_mode<T, 2, 4>(p, in.mode, grid, lds, stream);
-        default: return launch_mode<T, 4, 2>(p, in.mode, grid, lds, stream);
+        case 1: return launch_length<T, 1, 8>(p, in.mode, grid, lds, stream);
+        case 2: return launch_length<T, 2, 4>(p, in.mode, grid, lds, stream);
+        default: return launch_mode<T, 4, 2, 2>(p, in.mode, grid, lds, stream);   // (K <= 1024)
     }
 }
 

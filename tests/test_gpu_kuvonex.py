@@ -119,6 +119,36 @@ def test_gemv_and_its_intakes(dense, dtype, N, K, width):
     close(out, W @ (host(emb)[5] * 1.7), dtype, "embedding product")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("K", [2048, 2112, 4096, 4160, 8256])
+def test_intakes_at_the_lengths_that_registers_hold(dense, dtype, K):
+    """x in registers up to 2048 and 4096 elements, asked for by every pass past that; one that is there already 8192 at a time."""
+    say("intake", dtype, K)
+    N, eps, width = 96, 1e-3, K - 5
+    w, x, emb = rnd((N, K), 1, K ** -0.5, dtype), rnd((K,), 2, dtype=dtype), rnd((3, K), 7, dtype=dtype)
+    res, y, nw, fw = (rnd((K,), 3 + i, dtype=F32) for i in range(4))
+    for t in (res, y, nw, fw):
+        t[width:] = 0
+    emb[:, width:] = 0
+    W, R, Y, F = host(w), host(res), host(y), host(fw)
+    norm = lambda v, f: v / np.sqrt((v ** 2).sum() / width + eps) * f
+    both, row, tok = R + norm(Y, host(nw)), host(emb)[1] * 0.7, torch.tensor([1], dtype=torch.int32, device="cuda")
+    close(dense.gemv(x, w, out_f32=True), W @ host(x), F32, "plain")
+    r, bare = dense.Residual(res, y, nw, eps, width), dense.Residual(res, None, None, eps, width)
+    out, left, h = dense.gemv_residual(r, w, out_f32=True, want_h=True)
+    close(left, both, F32, "residual"), close(h, both, dtype, "residual, element type"), close(out, W @ both, dtype, "residual product")
+    close(dense.gemv_final(r, fw, w), W @ norm(both, F), dtype, "final")
+    close(dense.gemv_final(bare, fw, w), W @ norm(R, F), dtype, "final without a pending output")
+    out, left, h = dense.gemv_embed(tok, emb, 0.7, w, want_h=True)
+    close(left, row, F32, "row"), close(out, W @ row, dtype, "row product")
+    for s, v in ((dense.Sum(res=res, y=y), R + Y), (dense.Sum(res=res), R), (dense.Sum(token=tok, embed=emb, scale=0.7), row)):
+        out, left = dense.gemv_normed(s, fw, eps, width, w, out_f32=True)
+        close(left, v, F32, "sum"), close(out, W @ norm(v, F), dtype, "normed sum")
+        out, left = dense.gemv_normed(s, fw, eps, width, w, gate=dense.GATE_SILU)
+        z = (W @ norm(v, F)).reshape(N // 32, 2, 16)
+        close(left, v, F32, "gated sum"), close(out, (okv.silu(z[:, 0]) * z[:, 1]).reshape(-1), dtype, "gate", f32=1e-4)   # (silu passes errors on times up to |up|)
+
+
 def test_argmax_takes_the_lowest_row_on_ties(dense):
     w = torch.zeros((700, 64), dtype=F32, device="cuda")
     w[[650, 33, 480]] = 1.0
