@@ -261,8 +261,8 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gate_up_gemv_kernel(const Moe
 // y[n] = sum_s weight_s (down_s h_s)[n]; a wave owns a row, the pieces of all slots run through one loop, U of them in flight.  What bounds it:
 // HBM, behind two round trips, the choice's and the weights'.  So h is asked for first, a wave's pieces at once, then
 // the choice, a slot to a lane, and the weights before h is stored to LDS, all of a row where it is U pieces.  (No branch and no wait between
-// the requests: addresses past the end are clamped.)  8 experts of 2048 x 1024 (33.5 MB): 10.1 -> 8.9 us (a round trip per slot
-// for h and two rounds of 8 pieces before).
+// the requests: addresses past the end are clamped.)  8 experts of 2048 x 1024 (33.5 MB), one product behind the other: 8.5 -> 8.0 us = 4.2 TB/s (a
+// round trip per slot for h before).
 template <class T, int U>
 __global__ void __launch_bounds__(kMoeThreads, 2) moe_down_gemv_kernel(const MoeGemv<T> p) {
     extern __shared__ __attribute__((aligned(16))) char moe_lds[];
@@ -390,7 +390,9 @@ hipError_t down(const void *h, const void *w, const int32_t *ids, const float *w
     p.N = N;
     p.top = top;
     const size_t lds = (size_t)top * ((ff + kMoePiece - 1) / kMoePiece) * kMoePiece * sizeof(T);
-    auto kernel = &moe_down_gemv_kernel<T, sizeof(T) == 2 ? 16 : 8>;
+    // Pieces in flight: 4 in fp32 (twice the registers) and where a row is no more, else 8.  (Requests past a row's end read its last piece again: with 16 for
+    // every row, 2 experts of 2048 x 1024 took 6.2 us, 4.0 with 4; 8 of them 8.65, 8.0 with 8.)
+    auto kernel = sizeof(T) == 4 || top * ((ff + kMoePiece - 1) / kMoePiece) <= 4 ? &moe_down_gemv_kernel<T, 4> : &moe_down_gemv_kernel<T, 8>;
     const hipError_t e = with_lds(kernel, lds);
     if (e != hipSuccess) return e;
     const int need = (N + kMoeWaves - 1) / kMoeWaves;

@@ -265,6 +265,13 @@ def test_mixture(dense, dtype, M, experts, top, groups, keep, K, ff, N):
     close(got, want, dtype, bf16=3e-2)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("experts,top,ff,N", [(6, 4, 512, 64), (6, 5, 448, 80), (9, 8, 64, 64), (12, 9, 576, 64), (24, 20, 576, 64), (4, 1, 64, 4160), (5, 3, 1088, 4160)])
+def test_one_token_mixture_by_pieces(dense, dtype, experts, top, ff, N):
+    """Pieces of 512 of all slots: as many as are in flight (4 or 8), one more, several rounds and turns of h with ragged ends; more rows than waves."""
+    test_mixture(dense, dtype, 1, experts, top, 1, 1, 64, ff, N)
+
+
 @pytest.mark.parametrize("ff", [64, 512, 576])
 def test_one_token_mixture_that_overflows(dense, ff):
     """An expert's activation beyond the element type stays an infinity: pieces that a row does not have add nothing, not 0 times it."""
