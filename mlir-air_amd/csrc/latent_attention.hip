@@ -380,15 +380,10 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
     Vec8<T> w_first[kRowsPerWave];
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) w_first[i] = 8 * lane < rank ? load8(w_row + (size_t)i * rank + 8 * lane) : zero8<T>();
-    // ... and so are the gate, every split's maximum and sum and the first 512 columns of up to 64 splits, whether the position uses them or not
+    // ... and so are the gate and every split's maximum and sum, whether the position uses them or not.  (Not the splits' latents: up to 64 of them asked for
+    // ahead of the position cost every workgroup 128 KB, 4.5 -> 5.2 us with 16 heads, 9.3 -> 26.9 with 128, and 5.1 -> 5.4 where 33 are in use.)
     const int quarter = tid >> 7, col = 4 * (tid & 127);
     constexpr int BATCH = 16;
-    floatx4 ahead[BATCH];
-#pragma unroll
-    for (int j = 0; j < BATCH; ++j) {
-        const int i = quarter + 4 * j;
-        ahead[j] = *reinterpret_cast<const floatx4 *>(part_o + (row * nsplit + (i < nsplit ? i : 0)) * rank + (col < rank ? col : 0));
-    }
     const float *ml = part_ml + (row * nsplit + (tid < nsplit ? tid : 0)) * 2;
     const float ml_m = ml[0], ml_l = ml[1];
     const int value = h * p.s.vdim + v0 + kRowsPerWave * wave + (lane < kRowsPerWave ? lane : 0);
@@ -421,12 +416,7 @@ __global__ void __launch_bounds__(kMergeThreads) latent_combine_kernel(const Lat
         floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
         if (r < rank) {
             const float *src = part_o + row * nsplit * rank + r;
-            if (r0 == 0) {
-#pragma unroll
-                for (int j = 0; j < BATCH; ++j)
-                    if (quarter + 4 * j < active) s += ahead[j] * f[quarter + 4 * j];
-            }
-            for (int i = quarter + (r0 == 0 ? 4 * BATCH : 0); i < active; i += 4 * BATCH) {
+            for (int i = quarter; i < active; i += 4 * BATCH) {
                 floatx4 v[BATCH];
 #pragma unroll
                 for (int j = 0; j < BATCH; ++j) v[j] = *reinterpret_cast<const floatx4 *>(src + (size_t)(i + 4 * j < active ? i + 4 * j : i) * rank);
