@@ -48,41 +48,26 @@ __device__ __forceinline__ void rotate_pair(const T *src, T *dst, const float *l
     dst[1] = from_float<T>(v * c + u * s);
 }
 
-// The cache row of token m: by one workgroup.  Padding columns of the projections are zeros and stay zeros.  (Up to 1024 columns are read
-// once, with the norm's weights, before the position is there.)
+// The cache row of token m: by one workgroup.  Padding columns of the projections are zeros and stay zeros.
 template <class T>
 __device__ __forceinline__ void append_row(const LatentArgs<T> &p, int m, int position, float *red) {
-    constexpr int NB = 4;
     const T *src = p.proj + (size_t)m * p.ld + p.kv_off;
     T *dst = p.cache + (size_t)position * (p.s.rank + p.s.rot);
-    float x[NB], w[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int at = (int)threadIdx.x + kLatThreads * b, i = at < p.s.rank ? at : p.s.rank - 1;
-        x[b] = to_float(src[i]);
-        w[b] = p.kv_norm[i];
-    }
     float ss = 0.f;
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        if ((int)threadIdx.x + kLatThreads * b < p.s.rank) ss = fmaf(x[b], x[b], ss);
-    for (int i = threadIdx.x + kLatThreads * NB; i < p.s.rank; i += kLatThreads) {
+    for (int i = threadIdx.x; i < p.s.rank; i += kLatThreads) {
         const float v = to_float(src[i]);
         ss = fmaf(v, v, ss);
     }
     ss = wave_reduce<false>(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.s.true_rank + p.eps);
+    for (int i = threadIdx.x; i < p.s.rank; i += kLatThreads) dst[i] = from_float<T>(to_float(src[i]) * rstd * p.kv_norm[i]);
     for (int i = threadIdx.x; i < p.s.rot / 2; i += kLatThreads) {
         T *d = dst + p.s.rank + 2 * i;
         if (i < p.s.rot_pairs) rotate_pair(src + p.s.rank + 2 * i, d, p.lut + ((size_t)position * p.s.rot_pairs + i) * 2);
         else d[0] = d[1] = from_float<T>(0.f);
     }
-    __syncthreads();
-    const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.s.true_rank + p.eps);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        if (const int i = (int)threadIdx.x + kLatThreads * b; i < p.s.rank) dst[i] = from_float<T>(x[b] * rstd * w[b]);
-    for (int i = threadIdx.x + kLatThreads * NB; i < p.s.rank; i += kLatThreads) dst[i] = from_float<T>(to_float(src[i]) * rstd * p.kv_norm[i]);
 }
 
 // one workgroup per token
@@ -117,30 +102,22 @@ __global__ void __launch_bounds__(kLatThreads) latent_absorb_kernel(const Latent
     T *out = qa + ((size_t)m * p.s.heads + h) * lq;
     const int col = r0 + 8 * (tid & 15), dg = tid >> 4;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // eight rows of W at a time, the first of them asked for with the query (past the end: the last row and column, not added)
-    constexpr int kRows = 8;
-    const T *w = w_uk + (size_t)h * p.s.dim * p.s.rank + (col < p.s.rank ? col : p.s.rank - 8);
-    Vec8<T> v[kRows];
-    auto request = [&](int d0) {
-#pragma unroll
-        for (int j = 0; j < kRows; ++j) {
-            const int d = d0 + dg + 16 * j;
-            v[j] = load8(w + (size_t)(d < p.s.dim ? d : p.s.dim - 1) * p.s.rank);
-        }
-    };
-    request(0);
     for (int i = tid; i < p.s.dim; i += kLatThreads) qs[i] = to_float(q[i]);
     __syncthreads();
-    for (int d0 = 0; d0 < p.s.dim; d0 += 16 * kRows) {
-        if (d0 > 0) request(d0);
+    if (col < p.s.rank) {
+        const T *w = w_uk + ((size_t)h * p.s.dim + dg) * p.s.rank + col;
+        for (int d = dg; d < p.s.dim; d += 64) {       // dim is a multiple of 32: two or four rows at a time
+            Vec8<T> v[4];
 #pragma unroll
-        for (int j = 0; j < kRows; ++j) {
-            const int d = d0 + dg + 16 * j;
-            if (d >= p.s.dim) continue;
-            float f[8];
-            unpack8(v[j], f);
+            for (int j = 0; j < 4; ++j) v[j] = d + 16 * j < p.s.dim ? load8(w + (size_t)(d - dg + 16 * j) * p.s.rank) : zero8<T>();
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = fmaf(qs[d], f[e], acc[e]);
+            for (int j = 0; j < 4; ++j) {
+                float f[8];
+                unpack8(v[j], f);
+                const float x = d + 16 * j < p.s.dim ? qs[d + 16 * j] : 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[e] = fmaf(x, f[e], acc[e]);
+            }
         }
     }
 #pragma unroll
