@@ -70,10 +70,10 @@ __global__ void __launch_bounds__(kStepThreads) gated_norm_heads_kernel(const Ga
 }
 
 // One long group: a workgroup per token.
-template <class T>
+template <class T, bool KEPT>
 __global__ void __launch_bounds__(kStepThreads) gated_norm_row_kernel(const GatedNorm g, const T *gate, T *out) {
     __shared__ float red[4];
-    gated_norm_row_step<T>(g, gate, out, blockIdx.x, red);
+    gated_norm_row_step<T, KEPT>(g, gate, out, blockIdx.x, red);
 }
 
 template <class T>
@@ -126,7 +126,8 @@ hipError_t launch_gated_norm(int dtype, const GatedNorm &g, const void *gate, vo
     const dim3 grid = row ? dim3(M) : dim3((g.groups + per - 1) / per, M);
     auto run = [&](auto tag) {
         using T = decltype(tag);
-        if (row) hipLaunchKernelGGL(gated_norm_row_kernel<T>, grid, dim3(kStepThreads), 0, stream, g, static_cast<const T *>(gate), static_cast<T *>(out));
+        const auto rows = gated_norm_kept(g, M) ? &gated_norm_row_kernel<T, true> : &gated_norm_row_kernel<T, false>;
+        if (row) hipLaunchKernelGGL(rows, grid, dim3(kStepThreads), 0, stream, g, static_cast<const T *>(gate), static_cast<T *>(out));
         else hipLaunchKernelGGL(gated_norm_heads_kernel<T>, grid, dim3(kStepThreads), 0, stream, g, static_cast<const T *>(gate), static_cast<T *>(out), lanes);
         return hipGetLastError();
     };

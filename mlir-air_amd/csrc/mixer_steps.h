@@ -309,50 +309,61 @@ __device__ __forceinline__ void recurrence_step(const LinearArgs &a, float *o, i
     for (int c = 0; c < ND; ++c) *reinterpret_cast<floatx4 *>(st + 64 * c) = s[c];
 }
 
-// One long group, token m; up to 2048 columns stay in registers.  red: 4 floats of LDS.
-template <class T>
+// One long group, token m; KEPT: of up to 2048 columns, which stay in registers from the sum to the use.  red: 4 floats of LDS.
+template <class T, bool KEPT>
 __device__ __forceinline__ void gated_norm_row_step(const GatedNorm &g, const T *gate, T *out, size_t m, float *red) {
     constexpr int NB = 2, kStep = 4 * kStepThreads;
     const float *o = g.o + m * g.cols;
+    const T *gates = gate + m * g.ld_gate;
+    T *dst = out + m * g.ld_out;
     floatx4 v[NB], w[NB];
     float z[NB][4];
-    auto load = [&](int q) {
+    if constexpr (KEPT) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int at = 4 * (int)threadIdx.x + (q * NB + b) * kStep, i = at < g.cols ? at : g.cols - 4;
+            const int at = 4 * (int)threadIdx.x + b * kStep, i = at < g.cols ? at : g.cols - 4;
             v[b] = *reinterpret_cast<const floatx4 *>(o + i);
             w[b] = *reinterpret_cast<const floatx4 *>(g.w + i);
-            load4(gate + m * g.ld_gate + i, z[b]);
+            load4(gates + i, z[b]);
         }
-    };
-    const int batches = (g.cols + NB * kStep - 1) / (NB * kStep);
-    load(0);
+    }
     float ss = 0.f;
-    for (int q = 0; q < batches; ++q) {
-        if (q > 0) load(q);
+    auto square = [&](const floatx4 x) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss = fmaf(x[j], x[j], ss);
+    };
+    if constexpr (KEPT) {
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-            if (4 * (int)threadIdx.x + (q * NB + b) * kStep < g.cols) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) ss = fmaf(v[b][j], v[b][j], ss);
-            }
+            if (4 * (int)threadIdx.x + b * kStep < g.cols) square(v[b]);
+    } else {
+        for (int i = 4 * threadIdx.x; i < g.cols; i += kStep) square(*reinterpret_cast<const floatx4 *>(o + i));
     }
     ss = wave_reduce<false>(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)g.true_cols + g.eps);
-    for (int q = 0; q < batches; ++q) {
-        if (batches > 1) load(q);
+    auto finish = [&](const floatx4 x, const floatx4 f, float (&y)[4], int i) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int i = 4 * (int)threadIdx.x + (q * NB + b) * kStep;
-            if (i >= g.cols) continue;
+        for (int j = 0; j < 4; ++j) y[j] = x[j] * rstd * f[j] * sigmoid_of<T>(y[j]);
+        store4(dst + i, y[0], y[1], y[2], y[3]);
+    };
+    if constexpr (KEPT) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) z[b][j] = v[b][j] * rstd * w[b][j] * sigmoid_of<T>(z[b][j]);
-            store4(out + m * g.ld_out + i, z[b][0], z[b][1], z[b][2], z[b][3]);
+        for (int b = 0; b < NB; ++b)
+            if (const int i = 4 * (int)threadIdx.x + b * kStep; i < g.cols) finish(v[b], w[b], z[b], i);
+    } else {
+        for (int i = 4 * threadIdx.x; i < g.cols; i += kStep) {
+            float y[4];
+            load4(gates + i, y);
+            finish(*reinterpret_cast<const floatx4 *>(o + i), *reinterpret_cast<const floatx4 *>(g.w + i), y, i);
         }
     }
 }
+// Whether the columns of a few tokens are kept: with two quads to a thread, 1 token of 2048 2.27 -> 2.14 us; up to 1024 columns it is the same (1.94), past 2048 a
+// second batch of them read more than the loops (2560 columns 2.63 -> 2.71, 2048 tokens of it 7.4 -> 9.6), and many tokens' workgroups fill each other's waits (2048
+// tokens of 1536 4.6 -> 4.8, of 512 2.9 -> 3.7).
+__host__ __device__ inline bool gated_norm_kept(const GatedNorm &g, int tokens) { return g.cols > 1024 && g.cols <= 2048 && tokens <= 64; }
 
 // out[row] = w[row] x for the rows `row0` .. of this workgroup (kRowsAtOnce per group of `lanes` lanes); x and the rows of w have K elements.
 constexpr int kRowsAtOnce = 4;

@@ -473,6 +473,21 @@ def test_gated_norm(dense, dtype, groups, cols, true):
     assert bool((out[:, :32] == 7.0).all()) and bool((out[:, -8:] == 7.0).all())
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("M,cols,true", [(1, 1028, 1028), (64, 2048, 2041), (65, 1600, 1600), (1, 2052, 2049), (3, 4128, 4100)])
+def test_gated_norm_of_a_long_row(dense, dtype, M, cols, true):
+    """Columns that stay in registers (1025 to 2048, up to 64 tokens), and the lengths and tokens around them."""
+    rng = np.random.default_rng(cols)
+    mask = np.arange(cols) < true
+    o, w, z = rng.standard_normal((M, cols)) * mask, (rng.standard_normal(cols) * mask).astype(np.float32), rounded(rng.standard_normal((M, cols)) * 3)
+    o = o.astype(np.float32)
+    out = torch.full((M, cols + 8), 7.0, dtype=dtype, device="cuda")
+    dense.gated_norm(gpu(o), gpu(w), 1e-3, 1, true, gpu(z, dtype), out)
+    o = o.astype(np.float64)
+    close(out[:, :cols], o / np.sqrt((o ** 2).sum(-1, keepdims=True) / true + 1e-3) * w * ost.sigmoid(z), dtype)
+    assert bool((out[:, cols:] == 7.0).all())
+
+
 # ---- the model ---------------------------------------------------------------------------------------------------------------
 def _model(config, seed, dtype, **kw):
     from air_hip import sitirax
