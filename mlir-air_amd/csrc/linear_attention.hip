@@ -45,24 +45,17 @@ __global__ void __launch_bounds__(kStepThreads) gated_norm_heads_kernel(const Ga
     if (grp >= g.groups) return;
     const size_t m = blockIdx.y;
     const float *o = g.o + (m * g.groups + grp) * g.cols;
-    const T *gates = gate + m * g.ld_gate + (size_t)grp * g.cols;
-    // (a group of up to 256 columns is one turn, whose operands are read once, before the sum)
-    const int i0 = 4 * lane < g.cols ? 4 * lane : g.cols - 4;
-    const floatx4 v0 = *reinterpret_cast<const floatx4 *>(o + i0), w0 = *reinterpret_cast<const floatx4 *>(g.w + i0);
-    float z0[4];
-    load4(gates + i0, z0);
     float ss = 0.f;
     for (int i = 4 * lane; i < g.cols; i += 4 * lanes) {
-        const floatx4 v = i == 4 * lane ? v0 : *reinterpret_cast<const floatx4 *>(o + i);
+        const floatx4 v = *reinterpret_cast<const floatx4 *>(o + i);
 #pragma unroll
         for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
     }
     const float rstd = 1.0f / sqrtf(group_sum(ss, lanes) / (float)g.true_cols + g.eps);
     for (int i = 4 * lane; i < g.cols; i += 4 * lanes) {
-        const bool first = i == 4 * lane;
-        const floatx4 v = first ? v0 : *reinterpret_cast<const floatx4 *>(o + i), w = first ? w0 : *reinterpret_cast<const floatx4 *>(g.w + i);
-        float z[4] = {z0[0], z0[1], z0[2], z0[3]};
-        if (!first) load4(gates + i, z);
+        const floatx4 v = *reinterpret_cast<const floatx4 *>(o + i), w = *reinterpret_cast<const floatx4 *>(g.w + i);
+        float z[4];
+        load4(gate + m * g.ld_gate + (size_t)grp * g.cols + i, z);
 #pragma unroll
         for (int j = 0; j < 4; ++j) z[j] = v[j] * rstd * w[j] * sigmoid_of<T>(z[j]);
         store4(out + m * g.ld_out + (size_t)grp * g.cols + i, z[0], z[1], z[2], z[3]);
