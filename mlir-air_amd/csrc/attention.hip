@@ -104,11 +104,13 @@ __device__ __forceinline__ float slots_reduce(float v) {
     return swap_reduce<32, MAX>(v, v);
 }
 
-// What bounds it: latencies in a row, at 64 positions a workgroup: the fresh qkv and the cache (requested together and without a branch between
-// them, qkv first, so that it is rotated while the cache is on its way; the new token's K and V are taken from registers, not read back), the scores' sums, one maximum per wave and head, and the sums over positions.  Those halve
+// What bounds it: latencies in a row, at 64 positions a workgroup: the fresh qkv and the cache (requested together, qkv first, so that it is rotated
+// while the cache is on its way; the new token's K and V are taken from registers, not read back), the scores' sums, one maximum per wave and head,
+// and the sums over positions.  Those halve
 // what a lane holds with every exchange (v_permlane*_swap: half the values go each way), 28 exchanges for a head group of 4, where full
 // butterflies of (m, l, acc) took 120 shuffles through LDS.   32 heads of 64 over 8, 1000 positions: 7.3 -> 4.9 us; -> 4.5 a layer of
-// the model since the new token's row and the queries are no longer asked for one after the other behind the cache.
+// the model since the new token's row and the queries are no longer asked for one after the other behind the cache.  Only the chunk that appends
+// the new K and V asks for them: with all chunks, merge included, 32 heads of 64 over 8 at 4000 positions 7.5 us, 32 heads of 128 at 2000 8.6; 7.2 and 7.8.
 template <int HD, int G>
 __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     constexpr int LPP = HD / 8;        // lanes per position
@@ -128,7 +130,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     uint16_t *kc = p.k_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
     uint16_t *vc = p.v_cache + (size_t)kvh * p.max_seq * HD + 8 * sub;
 
-    // rotation and this lane's slices of qkv, the new K and V also where the chunk does not own them
+    // rotation and this lane's slices of qkv; of the new K and V where the chunk that holds `pos` appends them
     const bool low = 8 * sub < HD / 2;
     const int other = low ? 8 * sub + HD / 2 : 8 * sub - HD / 2, turn = low ? 8 * sub : other;
     auto raw = [](const uint16_t *at) { return *reinterpret_cast<const u32x4 *>(at); };
@@ -141,7 +143,9 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
         qy[h] = raw(src + other);
     }
     const uint16_t *k_row = p.qkv + nq + kvh * HD;
-    const u32x4 kx = raw(k_row + 8 * sub), ky = raw(k_row + other), vnew = raw(k_row + nkv + 8 * sub);
+    const bool owner = t0 <= p.pos && p.pos < t1;
+    u32x4 kx, ky, knew, vnew;
+    if (owner) kx = raw(k_row + 8 * sub), ky = raw(k_row + other), vnew = raw(k_row + nkv + 8 * sub);
 
     u32x4 kraw[UN], vraw[UN];
     auto request = [&](int tb) {
@@ -160,10 +164,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     float cos[8], sin[8];
     unpack8(cos_raw, cos);
     unpack8(sin_raw, sin);
-    // the chunk that owns `pos` appends the new token's K (rotated) and V
-    const bool owner = t0 <= p.pos && p.pos < t1;
-    u32x4 knew;
-    {
+    if (owner) {
         float kr[8];
         rope8(kx, ky, cos, sin, low, kr);
 #pragma unroll
