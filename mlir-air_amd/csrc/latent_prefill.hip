@@ -11,8 +11,8 @@
 // The D layout gives a lane keys 4 g .. + 3 of each 16-key block; the k slots of the second product are defined as exactly
 // those keys, so P never moves between lanes.  Four waves of QB blocks of 16 queries each share the K and V rows going through
 // LDS; the next block of keys travels global -> registers while one is multiplied.  With SETS = 2 a second set of four waves
-// takes the odd key blocks for the same queries, and the two partial results are merged through LDS at the end, a block of queries by
-// each set: the longest rows take half as long, and two waves share a SIMD.  (2048 tokens, 16 heads of 128 + 64 / 128: merge, gates and stores by one
+// takes the odd key blocks for the same queries, and the two partial results are merged through LDS at the end (with gates a block of queries by
+// each set): the longest rows take half as long, and two waves share a SIMD.  (2048 tokens, 16 heads of 128 + 64 / 128: merge, gates and stores by one
 // set 7.8 of 65 us, gates by an exponential and a division each and asked for one by one; now 3.7 of 62.)  The grid puts the longest rows first.  The running maximum may lag the true one by 2^8 (as in prefill_attention.hip), so
 // rescaling is rare; the row sum is a product with a row of ones.
 //
@@ -243,9 +243,9 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
         __syncthreads();
     }
 
-    // The same wave and lane of the other set holds the same queries and output elements.  With two blocks of queries each set finishes one
-    // of them, so that both work on the gates.
-    constexpr bool kShare = SETS == 2 && QB == 2;
+    // The same wave and lane of the other set holds the same queries and output elements.  Where there are gates each set finishes one block
+    // of queries, so that both work on them; without, the exchange both ways costs more than it shares (4 heads of 64 over 2, 2048 tokens 15.3 -> 15.6 us).
+    constexpr bool kShare = SETS == 2 && QB == 2 && !WINDOW;
     if constexpr (SETS == 2) {
         constexpr int NREG = (kShare ? 1 : QB) * (4 * NV + 2);
         float *mine = reinterpret_cast<float *>(pf_lds) + (wave + (kShare ? 4 * set : 0)) * NREG * 64 + lane;   // what this wave takes
