@@ -271,17 +271,19 @@ __global__ void __launch_bounds__(kGemvThreads) dense_gemv_kernel(const GemvPara
     }
 }
 
+// AT keys of a thread at a time: a round trip for up to 4096 of them with 4, where fewer ask for one each
+template <int AT>
 __global__ void __launch_bounds__(1024) argmax_keys_kernel(const unsigned long long *keys, int n, int32_t *token, int32_t *position,
                                                            int32_t *history) {
     __shared__ unsigned long long part[16];
     const int32_t here = position ? position[0] : 0;   // (every thread: asked for with the keys)
     unsigned long long best = 0;
-    for (int i0 = threadIdx.x; i0 < n; i0 += 4 * 1024) {   // four at a time: a round trip for up to 4096 of them
-        unsigned long long k[4];
+    for (int i0 = threadIdx.x; i0 < n; i0 += AT * 1024) {
+        unsigned long long k[AT];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) k[j] = keys[i0 + 1024 * j < n ? i0 + 1024 * j : i0];
+        for (int j = 0; j < AT; ++j) k[j] = keys[i0 + 1024 * j < n ? i0 + 1024 * j : i0];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) best = k[j] > best ? k[j] : best;
+        for (int j = 0; j < AT; ++j) best = k[j] > best ? k[j] : best;
     }
     best = wave_max_u64(best);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
@@ -390,7 +392,7 @@ hipError_t launch_dense_gemv(int dtype, const void *w, const RowIntake &in, void
 }
 
 hipError_t launch_argmax_keys(const unsigned long long *keys, int n, int32_t *token, int32_t *position, int32_t *history, hipStream_t stream) {
-    hipLaunchKernelGGL(argmax_keys_kernel, dim3(1), dim3(1024), 0, stream, keys, n, token, position, history);
+    hipLaunchKernelGGL(n <= 1024 ? &argmax_keys_kernel<1> : &argmax_keys_kernel<4>, dim3(1), dim3(1024), 0, stream, keys, n, token, position, history);
     return hipGetLastError();
 }
 
