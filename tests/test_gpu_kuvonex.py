@@ -401,6 +401,38 @@ def test_latent_attention_forms_agree_token_by_token_and_with_the_position_on_th
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("sizes", [(16, 128, 64, 128, 512), (6, 64, 32, 64, 192), (5, 16, 6, 24, 40)])
+@pytest.mark.parametrize("form", ["rows", "absorbed"])
+def test_gates_that_are_not_finite(dense, dtype, sizes, form):
+    """A gate that is not a number makes its output one that is not, of minus infinity nothing passes and of infinity all, and no other output changes."""
+    say("gates", dtype, sizes, form)
+    T = 70 if form == "rows" else 3
+    x = Latents(dense, sizes, T, dtype, seed=9)
+    H, V, vp = sizes[0], sizes[3], x.spec.vdim_p
+    gates = x.proj[:, x.gate_off:x.gate_off + H * vp].view(T, H, vp)
+    base = x.run(form, 0, T).view(T, H, V).clone()
+    places = [(0, 0, 0), (1, H - 1, V - 1), (T - 1, 1, V // 2), (T // 2, H - 1, 3)]
+    full = torch.tensor([30.0]).to(dtype).cuda()                 # sigmoid 1 - 1e-13
+    for value in (float("nan"), float("inf"), -float("inf"), -200.0, 200.0):
+        keep = gates.clone()
+        for i in places:
+            gates[i] = full
+        whole = x.run(form, 0, T).view(T, H, V).clone()
+        for i in places:
+            gates[i] = value
+        got = x.run(form, 0, T).view(T, H, V)
+        rest = torch.ones((T, H, V), dtype=torch.bool, device="cuda")
+        for i in places:
+            rest[i] = False
+            if value != value:
+                assert bool(got[i].isnan()), (value, i)
+            else:
+                assert float(got[i]) == (float(whole[i]) if value > 0 else 0.0), (value, i)
+        assert torch.equal(got[rest], base[rest]) and torch.equal(whole[rest], base[rest])
+        gates.copy_(keep)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("sizes", [(2, 24, 8, 40, 56), (2, 24, 8, 32, 600)])
 def test_latent_attention_of_one_token_in_many_splits(dense, dtype, sizes):
     """One to many blocks of keys to a split (two of them ahead of the products), and more splits in use than the merge reads ahead (64)."""
