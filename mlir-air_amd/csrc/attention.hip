@@ -55,11 +55,6 @@ __device__ __forceinline__ float exp2_nonpos(float x) { return __builtin_amdgcn_
 // distances 1 and 2, half-row and row mirrors for 4 and 8: once the quads agree, mirroring meets the
 // partner quad), i.e. full-rate VALU adds instead of LDS-routed shuffles.  Bit-identical to the butterfly
 // with shuffles: every step adds the same two partial sums.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true);
-    return v + __builtin_bit_cast(float, moved);
-}
 template <int LPP>
 __device__ __forceinline__ float group_sum(float s) {
     static_assert(LPP == 8 || LPP == 16, "lane groups of 8 or 16");
@@ -83,16 +78,6 @@ __device__ __forceinline__ void rope8(const u32x4 xr, const u32x4 yr, const floa
     }
 }
 
-// Two lane halves (SWAP 32) or neighbouring rows of 16 lanes (SWAP 16): first + second of the values that each pair of lanes holds of `a`
-// in the one lane, of `b` in the other.
-template <int SWAP, bool MAX>
-__device__ __forceinline__ float swap_reduce(float a, float b) {
-    const auto r = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false)
-                              : __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-    const unsigned first = r[0], second = r[1];   // (a bit cast of an element itself reads the vector's first one)
-    const float x = __builtin_bit_cast(float, first), y = __builtin_bit_cast(float, second);
-    return MAX ? fmaxf(x, y) : x + y;
-}
 // Over the lanes with equal `sub` (one per position), every one of them receiving the result.
 template <int LPP, bool MAX>
 __device__ __forceinline__ float slots_reduce(float v) {

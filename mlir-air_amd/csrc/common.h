@@ -58,6 +58,22 @@ __device__ __forceinline__ void unpack8_f32(uint32_t w, float (&q)[8]) {
     q[7] = static_cast<float>(o >> 24);
 }
 
+// v + the value that the DPP control CTRL moves to this lane
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+
+// Two lane halves (SWAP 32) or neighbouring rows of 16 lanes (SWAP 16): first + second of the values that each pair of lanes holds of `a`
+// in the one lane, of `b` in the other.
+template <int SWAP, bool MAX>
+__device__ __forceinline__ float swap_reduce(float a, float b) {
+    const auto r = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false)
+                              : __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned first = r[0], second = r[1];   // (a bit cast of an element itself reads the vector's first one)
+    const float x = __builtin_bit_cast(float, first), y = __builtin_bit_cast(float, second);
+    return MAX ? fmaxf(x, y) : x + y;
+}
 // Maximum / sum over the 64 lanes of a wavefront, every lane receiving the result: the four steps inside a row of
 // 16 lanes on DPP moves (quad permutes for distances 1 and 2, half-row and row mirrors for 4 and 8: once the
 // quads agree, mirroring meets the partner quad), the two steps across rows by exchanging rows and halves of two copies, which then hold a
@@ -75,12 +91,8 @@ __device__ __forceinline__ float wave_reduce(float v) {
     dpp(std::integral_constant<int, 0x4E>());    // quad_perm [2, 3, 0, 1]
     dpp(std::integral_constant<int, 0x141>());   // row_half_mirror
     dpp(std::integral_constant<int, 0x140>());   // row_mirror
-    const uint32_t u = __builtin_bit_cast(uint32_t, v);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);   // rows (0, 1) and (2, 3) exchanged
-    v = op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
-    const uint32_t w = __builtin_bit_cast(uint32_t, v);
-    const auto h = __builtin_amdgcn_permlane32_swap(w, w, false, false);   // halves exchanged
-    return op(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1]));
+    v = swap_reduce<16, MAX>(v, v);   // rows (0, 1) and (2, 3) exchanged
+    return swap_reduce<32, MAX>(v, v);   // halves exchanged
 }
 
 // Maximum / sum over the 16 lanes of a DPP row, every lane of the row receiving it (the four in-row steps of wave_reduce).

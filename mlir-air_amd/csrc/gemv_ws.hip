@@ -48,19 +48,10 @@ __device__ __forceinline__ bf16x8 cell_operand(uint32_t w, uint32_t nib_mask, ui
     return __builtin_bit_cast(bf16x8, b);
 }
 
-// v + the value CTRL rotates to this lane inside its row of 16
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
 // sum over the four lanes ln, ln + 16, ln + 32, ln + 48: (first + second) + (third + fourth)
 __device__ __forceinline__ float row_groups_sum(float v) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, v);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    v = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
-    const uint32_t w = __builtin_bit_cast(uint32_t, v);
-    const auto h = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-    return __builtin_bit_cast(float, (uint32_t)h[0]) + __builtin_bit_cast(float, (uint32_t)h[1]);
+    v = swap_reduce<16, false>(v, v);
+    return swap_reduce<32, false>(v, v);
 }
 
 // Arguments that only some launches read; they follow the ones every wave needs at once, which fit the SGPRs
@@ -119,7 +110,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) gemv_ws_kernel(const uint16_t 
     for (int m = 0; m < NMAT; ++m) yv[m] = 0.f;
 
     // The residual is added last and asked for first: behind the sums it is a round trip of its own (O product of 2048 x 2048, 4.0 -> 3.8 us, down of 8192 x 2048 5.0 -> 4.7).
-    // Without one some x is read, and not used.
+    // Without one some x is read, and not used: that is free (4096 x 11008 6.3 us with and without), a branch around it costs the products with a residual 2 %.
     const uint32_t add = (residual ? residual + tile * kWsTileCols : x)[threadIdx.x & (kWsTileCols - 1)];
 
     // RMS: the partial sums are requested first and consumed only after the first task's loads have been requested
@@ -260,8 +251,8 @@ __global__ void __launch_bounds__(kMaxWaves * 64) gemv_ws_kernel(const uint16_t 
         else yv[0] += sum;
     }
 
-    // K-reduction: the 4 lane groups of a wave hold different groups of K for the same 16 columns and are added with
-    // wavefront shuffles, (lg 0 + lg 1) + (lg 2 + lg 3); only the waves' sums meet in LDS, added by the first 16 threads
+    // K-reduction: the 4 lane groups of a wave hold different groups of K for the same 16 columns and are added by exchanging
+    // rows and halves of the wave in registers, (lg 0 + lg 1) + (lg 2 + lg 3); only the waves' sums meet in LDS, added by the first 16 threads
 #pragma unroll
     for (int m = 0; m < NMAT; ++m) {
         const float v = row_groups_sum(yv[m]);
