@@ -411,7 +411,8 @@ def latent_attention_rows(spec, proj, kv_off, gate_off, lut, kv_norm, eps, cache
 
 def latent_splits(spec, M, total):
     """How many workgroups share the keys of 16 rows.  A workgroup's time grows with its blocks of 32 keys, the merge's with
-    the splits and rows: the square root balances them (constant measured at 16, 32 and 128 heads, 2k to 128k keys)."""
+    the splits and rows: the square root balances them (8 to 128 heads, 300 to 32k keys: within 5 % of the best of half to twice as many,
+    within 11 % with 128 heads, whose splits are few whole blocks)."""
     rows, blocks = M * spec.heads, (total + 31) // 32
     return max(1, min(256, 512 // ((rows + 15) // 16), blocks, round((512 * blocks / rows) ** 0.5)))
 
