@@ -264,8 +264,8 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
 // A wave's NT x MT tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
-// GROUPED without a pair, entries as rows of the result: out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
-template <int NT, int MT, int EPI, bool GROUPED>
+// SCATTER: rows of the result are entries; without a pair out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
+template <int NT, int MT, int EPI, bool GROUPED, bool SCATTER>
 __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first,
                                            const int (&out_rows)[2] = {0, 0}) {
     typedef typename std::conditional<EPI == kOutF32, float, bf16>::type Out;
@@ -295,11 +295,9 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
         for (int t = lane; t < kPieces; t += 64) {
             const int row = t / (kCols / kPiece), col = t % (kCols / kPiece) * kPiece, m = m_first + 16 * i + row;
             size_t to = m;
-            if constexpr (GROUPED && !kPair)
-                if (p.gather == 0) to = __shfl(out_rows[i / 4], 16 * (i % 4) + row);
+            if constexpr (SCATTER && !kPair) to = __shfl(out_rows[i / 4], 16 * (i % 4) + row);
             if (m >= m_end || n_out + col >= n_end) continue;
-            if constexpr (GROUPED && kPair)
-                if (p.gather == 0) to = p.order[m];   // (no product of the mixture: asked for here, the registers of out_rows are worth more)
+            if constexpr (SCATTER && kPair) to = p.order[m];   // (no product of the mixture)
             const long part = EPI == kOutF32 ? blockIdx.y * p.slice_stride : 0;
             *reinterpret_cast<u32x4 *>(static_cast<Out *>(p.out) + part + to * p.ldo + n_out + col) = *reinterpret_cast<const u32x4 *>(rows + row * kPitch + col);
         }
@@ -455,7 +453,7 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
     for (int j = 0; j < NT; ++j)
         asm volatile("" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
 
-    store_rows<NT, 8, EPI, false>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
+    store_rows<NT, 8, EPI, false, false>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
 }
 
 template <int WM, int NT, int EPI>
@@ -493,7 +491,7 @@ constexpr size_t expert_lds(int mt, bool few) { return (size_t)(expert_stages_a(
 // of `items` that are to be spread over the products [0, upto): the first one that goes behind product n or later
 __device__ constexpr int items_before(int n, int upto, int items) { return n >= upto ? items : n * items / upto; }
 
-template <int MT, int EPI, bool FEW>
+template <int MT, int EPI, bool SCATTER, bool FEW>
 __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, int first) {
     constexpr int kSideA = 64 * MT * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(MT, FEW), RW = kExpertStagesW;
     constexpr int kBehind = RA == RW ? (RA - 2) * (2 * MT + 4) : 4;   // copies that may be on their way at the wait
@@ -570,7 +568,7 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     // where the second product's rows go: asked for here, because a store that has to ask waits once per 16 rows (down of 64 experts of
     // 1024 x 2048, 16384 entries: 109 -> 101 us, with nothing read past the last K-step)
     int out_rows[2] = {0, 0};
-    if (EPI == kOutElem && p.gather == 0) {
+    if constexpr (SCATTER && EPI == kOutElem) {
         const int own = m0 + wave * 16 * MT;
         out_rows[0] = p.order[own + lane < m_end ? own + lane : m_end - 1];
         if (MT > 4) out_rows[1] = p.order[own + 64 + lane < m_end ? own + 64 + lane : m_end - 1];
@@ -641,10 +639,11 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
 #pragma unroll
     for (int i = 0; i < MT; ++i)
         asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]), "+a"(acc[4][i]), "+a"(acc[5][i]), "+a"(acc[6][i]), "+a"(acc[7][i]));
-    store_rows<8, MT, EPI, true>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0, out_rows);
+    store_rows<8, MT, EPI, true, SCATTER>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0, out_rows);
 }
 
-template <int EPI, bool FEW>
+// (SCATTER is gather == 0: asked at run time it cost gate and up 1.7 %)
+template <int EPI, bool SCATTER, bool FEW>
 __global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_kernel(const GemmKernelArgs<bf16> p) {
     extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
     const int tiles_m = p.tiles[4 * p.tiles_m];
@@ -656,19 +655,19 @@ __global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_k
     const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
     const int first = (5 * t[0] + 3 * (tile % p.tiles_n)) % (p.K / 64);
     if constexpr (FEW) {
-        if (t[2] <= 64) return expert_tile<1, EPI, true>(p, gemm_lds, w, m0, m_end, n0, first);
+        if (t[2] <= 64) return expert_tile<1, EPI, SCATTER, true>(p, gemm_lds, w, m0, m_end, n0, first);
         for (int m = m0; m < m_end; m += kFewRows) {   // (once, for a plan of the tile_rows that the launch was given)
             if (m > m0) __syncthreads();
-            expert_tile<2, EPI, true>(p, gemm_lds, w, m, m_end - m < kFewRows ? m_end : m + kFewRows, n0, first);
+            expert_tile<2, EPI, SCATTER, true>(p, gemm_lds, w, m, m_end - m < kFewRows ? m_end : m + kFewRows, n0, first);
         }
     } else {
         switch ((t[2] + 63) / 64) {
-            case 1: return expert_tile<1, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 2: return expert_tile<2, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 3: return expert_tile<3, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 4: return expert_tile<4, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 5: return expert_tile<5, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            default: return expert_tile<6, EPI, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 1: return expert_tile<1, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 2: return expert_tile<2, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 3: return expert_tile<3, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 4: return expert_tile<4, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 5: return expert_tile<5, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            default: return expert_tile<6, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
         }
     }
 }
@@ -742,8 +741,9 @@ hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
     constexpr size_t lds = FEW ? expert_lds(2, true) : expert_lds(6, false);
     static_assert(lds <= (FEW ? 80 : 160) * 1024 && 4 * kWideStore <= lds, "fits LDS, twice for few rows");
     static_assert(FEW ? expert_lds(1, true) <= lds : expert_lds(4, false) <= lds && expert_lds(5, false) <= lds, "the other heights too");
-    return g.epilogue == kOutSwiglu ? run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutSwiglu, FEW>, p, kWideThreads, lds, 1, stream)
-                                    : run_tiles<GemmKernelArgs<bf16>>(&dense_gemm_expert_kernel<kOutElem, FEW>, p, kWideThreads, lds, 1, stream);
+    auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, lds, 1, stream); };
+    if (g.epilogue == kOutSwiglu) return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutSwiglu, true, FEW>) : run(&dense_gemm_expert_kernel<kOutSwiglu, false, FEW>);
+    return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutElem, true, FEW>) : run(&dense_gemm_expert_kernel<kOutElem, false, FEW>);
 }
 
 // out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
