@@ -258,25 +258,25 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
             to[4 * NV * 64] = m[b];
             to[(4 * NV + 1) * 64] = l[b][0];
         };
-        // (set 0's part first, whoever adds them up: a query's result does not depend on it)
-        auto take = [&](int b, const float *from, auto own_first) {
+        // (own: this wave's part counts as set b's of block b.  Written out, so that a query's result does not depend on who adds the parts up.)
+        auto take = [&](int b, const float *from, auto own) {
             const float m1 = from[4 * NV * 64], l1 = from[(4 * NV + 1) * 64];
             const float mm = fmaxf(m[b], m1);
             const float f0 = __builtin_amdgcn_exp2f((m[b] - mm) * p.scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mm) * p.scale_log2);
-            auto sum = [&](float own, float got) { return own_first ? fmaf(own, f0, got * f1) : fmaf(got, f1, own * f0); };
+            auto sum = [&](float mine, float got, bool first) { return first ? fmaf(mine, f0, got * f1) : fmaf(got, f1, mine * f0); };
             m[b] = mm;
-            l[b][0] = sum(l[b][0], l1);
+            l[b][0] = sum(l[b][0], l1, !own);
 #pragma unroll
             for (int d = 0; d < NV; ++d)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) o[b][d][r] = sum(o[b][d][r], from[(d * 4 + r) * 64]);
+                for (int r = 0; r < 4; ++r) o[b][d][r] = sum(o[b][d][r], from[(d * 4 + r) * 64], own);
         };
         if constexpr (kShare) {
             if (set == 0) give(1, other);
             else give(0, other);
             __syncthreads();
             if (set == 0) take(0, mine, std::true_type());
-            else take(1, mine, std::false_type());
+            else take(1, mine, std::true_type());
         } else {
             if (set == 1) {
 #pragma unroll
@@ -284,8 +284,8 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
             }
             __syncthreads();
             if (set == 1) return;
-#pragma unroll
-            for (int b = 0; b < QB; ++b) take(b, mine + b * (4 * NV + 2) * 64, std::true_type());
+            take(0, mine, std::true_type());
+            if constexpr (QB == 2) take(1, mine + (4 * NV + 2) * 64, std::false_type());
         }
     }
 
