@@ -803,6 +803,8 @@ float gemm_time(const GemmKind &k, int M, int N, int steps, int epilogue, int sl
     if (epilogue == kOutF32 || slices > 1) t += slices * mb / k.store_tbs;
     // whoever adds them up: the next kernel where the parts are kept, else a launch (3.5 us on the GPU, 6 with its allocation on the host, which
     // short prompts wait for)
+    // (a router's parts: the choice of the experts waits for them, a wave to a token.  16384 x 32 x 512 13.1 us in one launch, 14.8 in two slices)
+    if (slices > 1 && kept && N <= 128) t += 1.5e-4f * M;
     if (slices > 1) t += kept ? (slices - 1) * mb / 5.f : 6.f + (slices + 0.5f) * mb / 4.f;
     return t;
 }

@@ -418,6 +418,7 @@ def test_slices_that_a_launch_adds_up_are_charged_for_it():
     lib = _lib.load_dense_library()
     assert [lib.dlm_gemm_slices(0, M, 64, 2048, 1) for M in (2048, 4096, 8192)] == [1] * 3
     assert lib.dlm_gemm_parts(0, 2048, 2048, 8192) > 1 and lib.dlm_gemm_parts(0, 64, 2048, 8192) > 1
+    assert lib.dlm_gemm_parts(0, 2048, 64, 2048) > 1 and lib.dlm_gemm_parts(0, 16384, 32, 512) == 1   # a router's: very many tokens' choices wait for parts
     assert lib.dlm_gemm_slices(0, 64, 2048, 8192, 1) > 1                                     # worth its launch
     assert lib.dlm_gemm_parts(1, 64, 2048, 8192) == 1 and lib.dlm_gemm_parts(0, 0, 64, 64) == 0   # fp32 weights, no rows
 
