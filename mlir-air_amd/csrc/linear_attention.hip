@@ -119,7 +119,7 @@ hipError_t launch_gated_norm(int dtype, const GatedNorm &g, const void *gate, vo
     const dim3 grid = row ? dim3(M) : dim3((g.groups + per - 1) / per, M);
     auto run = [&](auto tag) {
         using T = decltype(tag);
-        const auto rows = gated_norm_kept(g, M) ? &gated_norm_row_kernel<T, true> : &gated_norm_row_kernel<T, false>;
+        const auto rows = gated_norm_kept(g) ? &gated_norm_row_kernel<T, true> : &gated_norm_row_kernel<T, false>;
         if (row) hipLaunchKernelGGL(rows, grid, dim3(kStepThreads), 0, stream, g, static_cast<const T *>(gate), static_cast<T *>(out));
         else hipLaunchKernelGGL(gated_norm_heads_kernel<T>, grid, dim3(kStepThreads), 0, stream, g, static_cast<const T *>(gate), static_cast<T *>(out), lanes);
         return hipGetLastError();

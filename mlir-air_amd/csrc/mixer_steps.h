@@ -360,10 +360,10 @@ __device__ __forceinline__ void gated_norm_row_step(const GatedNorm &g, const T 
         }
     }
 }
-// Whether the columns of a few tokens are kept: with two quads to a thread, 1 token of 2048 2.27 -> 2.14 us; up to 1024 columns it is the same (1.94), past 2048 a
-// second batch of them read more than the loops (2560 columns 2.63 -> 2.71, 2048 tokens of it 7.4 -> 9.6), and many tokens' workgroups fill each other's waits (2048
-// tokens of 1536 4.6 -> 4.8, of 512 2.9 -> 3.7).
-__host__ __device__ inline bool gated_norm_kept(const GatedNorm &g, int tokens) { return g.cols > 1024 && g.cols <= 2048 && tokens <= 64; }
+// Whether the columns are kept: with two quads to a thread, 1 token of 2048 2.27 -> 2.14 us, 2048 tokens of it behind a recurrence, whose outputs have left L2,
+// 8.3 -> 7.4 (with everything in L2 5.4 either way, of 1536 4.6 -> 4.8).  Up to 1024 columns it is the same for a token (1.94) and slower for many (2048 of
+// 512 2.9 -> 3.7), past 2048 a second batch of them read more than the loops (2560 columns 2.63 -> 2.71, 2048 tokens of it 7.4 -> 9.6).
+__host__ __device__ inline bool gated_norm_kept(const GatedNorm &g) { return g.cols > 1024 && g.cols <= 2048; }
 
 // out[row] = w[row] x for the rows `row0` .. of this workgroup (kRowsAtOnce per group of `lanes` lanes); x and the rows of w have K elements.
 constexpr int kRowsAtOnce = 4;

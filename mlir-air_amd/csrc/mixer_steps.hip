@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(kStepThreads) head_state_end_kernel(const Head
     __shared__ float red[8];
     __shared__ floatx4 part[kStepThreads];
     if (blockIdx.x == 0) {
-        if (gated_norm_kept(g, 1)) gated_norm_row_step<T, true>(g, gate, norm_out, 0, red);
+        if (gated_norm_kept(g)) gated_norm_row_step<T, true>(g, gate, norm_out, 0, red);
         else gated_norm_row_step<T, false>(g, gate, norm_out, 0, red);
     } else {
         head_merge_step<T>(s, 1, pos_dev, pos, nsplit, kb, part_o, part_ml, out, 0, blockIdx.x - 1, 0, f, red, part);

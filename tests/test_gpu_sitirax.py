@@ -474,9 +474,9 @@ def test_gated_norm(dense, dtype, groups, cols, true):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
-@pytest.mark.parametrize("M,cols,true", [(1, 1028, 1028), (64, 2048, 2041), (65, 1600, 1600), (1, 2052, 2049), (3, 4128, 4100)])
+@pytest.mark.parametrize("M,cols,true", [(1, 1024, 1020), (1, 1028, 1028), (64, 2048, 2041), (65, 1600, 1600), (1, 2052, 2049), (3, 4128, 4100)])
 def test_gated_norm_of_a_long_row(dense, dtype, M, cols, true):
-    """Columns that stay in registers (1025 to 2048, up to 64 tokens), and the lengths and tokens around them."""
+    """Columns that stay in registers (1025 to 2048), and the lengths around them."""
     rng = np.random.default_rng(cols)
     mask = np.arange(cols) < true
     o, w, z = rng.standard_normal((M, cols)) * mask, (rng.standard_normal(cols) * mask).astype(np.float32), rounded(rng.standard_normal((M, cols)) * 3)
