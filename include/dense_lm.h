@@ -223,7 +223,7 @@ typedef struct {
     int32_t k_heads, heads, dim, vdim, q_off, k_off, v_off, M, pos;
 } dlm_recurrence_args;
 /* o fp32 [M, heads vdim].  _steps: token by token; _chunks: 64 tokens at a time, work of dlm_recurrence_chunk_bytes (0: no kernel for
- * this size). */
+ * this size; no less for a longer portion). */
 int dlm_recurrence_steps(int dtype, const dlm_recurrence_args *a, float *o, void *stream);
 size_t dlm_recurrence_chunk_bytes(const dlm_recurrence_args *a);
 int dlm_recurrence_chunks(int dtype, const dlm_recurrence_args *a, void *work, float *o, void *stream);
