@@ -20,13 +20,13 @@
 // Issue budget (measured with a loop of this kernel's instruction pattern): the MFMA occupies the matrix pipe for
 // 16 cycles and the issue port for 8; a wave issues in order, so exactly two VALU instructions fit behind an
 // MFMA for free, a third costs 4 cycles, and two dependent VALU instructions back to back stall on top of that.
-// Dequantising 8 weights takes 23 instructions, and with 16 row tiles one B operand feeds 16 MFMAs: the 23
-// instructions are cut into 12 slots of two independent instructions (DequantSlots), one slot behind each of the
-// first 12 MFMAs of the previous operand.  With 8 row tiles (2.9 instructions per MFMA) the same loop is bound by
-// the VALU: 128 x 448 tiles measured 288 us against 257 us for 256 x 256 with the same inner loop.
+// Dequantising 8 weights takes 17 instructions (Q4NX: 23), and with 16 row tiles one B operand feeds 16 MFMAs: the
+// instructions are cut into 9 (12) slots of two independent instructions (DequantSlots), one slot behind each of the
+// first 9 (12) MFMAs of the previous operand.  With 8 row tiles (2.9 instructions per MFMA) the same loop is bound by
+// the VALU: 128 x 448 tiles measured 288 us against 257 us for 256 x 256 with the same inner loop and 23 instructions.
 // Every other instruction (LDS read, memory request, s_add, s_nop, s_waitcnt) takes a slot of its own as well.
 //
-// Where the time goes at M = 2048, K = 4096, N = 14336 (same box, kernel parts compiled out one at a time): MFMAs alone
+// Where the time goes at M = 2048, K = 4096, N = 14336 (same box, kernel parts compiled out one at a time, 23 instructions a dequant): MFMAs alone
 // 143 us (the accumulators' pro- and epilogue included), with the dequant 153 us, with LDS reads, x tile copy and
 // cell loads 203 - 213 us; without the x tile copy 169 us, without the LDS reads 192 us, without the cell loads 194 us.
 // The x tile through registers instead (global_load_dwordx4, then ds_write_b128 a K-step later): 216 against 202 us.
@@ -45,9 +45,9 @@
 // slot ^ row % 16.  The A operand read of K-step t (lane (lg, ln): row 16 rt + ln, chunk 4 t + lg) then touches 16
 // distinct slots over 16 consecutive rows: conflict-free without padding.
 //
-// Dequant in registers: e = w & 0x0F0F0F0F and o = (w >> 4) & 0x0F0F0F0F put the eight nibbles of a dword into bytes,
-// v_cvt_f32_ubyteN converts each, fma(q, s, -z s) equals (q - z) * s exactly ((q - z) has 5 significant bits, s has 8),
-// v_cvt_pk_bf16_f32 rounds once.
+// Dequant in registers (wsdequant.h), AWQ order: two nibbles a mask behind the exponent of the half-precision 1024, v_fma_mix_f32 multiplies and adds the
+// half as it is (exact), v_cvt_pk_bf16_f32 rounds once.  Q4NX order: e = w & 0x0F0F0F0F and o = (w >> 4) & 0x0F0F0F0F put the eight nibbles of a dword
+// into bytes, v_cvt_f32_ubyteN converts each, fma(q, s, min').
 #include <algorithm>
 #include <functional>
 #include <mutex>
@@ -77,6 +77,8 @@ constexpr double kPfSlowdown128 = 1.4, kPfSlowdown64 = 2.0;   // time per column
 struct DequantSlots {
     uint32_t w;
     float sf, c0;
+    AwqScale d;
+    uint32_t n1, n2, w8;
     uint32_t e, o;
     float a0, a1, b0, b1;
     uint32_t p0, p1, p2, p3;
@@ -117,6 +119,40 @@ __device__ __forceinline__ void mfma_quarter(floatx4 &c0, floatx4 &c1, floatx4 &
                      : "+a"(c0), "+a"(c1), "+a"(c2), "+a"(c3), "+v"(d.a1), "=&v"(d.b0), "=&v"(d.b1), "=&v"(d.p2), "=&v"(d.p3)
                      : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b), "v"(d.a0), "v"(d.o), "v"(d.sf), "v"(d.c0));
     }
+}
+
+// The AWQ order's dequant (dequant_operand_awq) in the same way: 17 instructions, nine slots, so seven of the 16 MFMAs of an operand have
+// theirs free.  Quarters 0 and 1, and the first MFMA of quarter 2.
+template <int Q>
+__device__ __forceinline__ void mfma_quarter_awq(floatx4 &c0, floatx4 &c1, floatx4 &c2, floatx4 &c3, const bf16x8 &a0, const bf16x8 &a1,
+                                                 const bf16x8 &a2, const bf16x8 &a3, const bf16x8 &b, DequantSlots &d, uint32_t low, uint32_t high,
+                                                 uint32_t magic) {
+#define PF_MIX(dst, n, hi, s, c) "v_fma_mix_f32 %" #dst ", %" #n ", %" #s ", %" #c " op_sel:[" #hi ",0,0] op_sel_hi:[1,0,0]\n\t"
+    if constexpr (Q == 0) {
+        // %4 n0, %5 n1, %6 n2, %7 w8, %8 a0, %9 a1, %10 b0, %11 p0 | %12..%15 A, %16 B, %17 w, %18 s, %19 c, %20 s / 16, %21 its c, %22 low, %23 high, %24 magic
+        asm volatile(PF_MFMA(0, 12, 16) "v_lshrrev_b32 %7, 8, %17\n\tv_and_or_b32 %4, %17, %22, %24\n\t"
+                     PF_MFMA(1, 13, 16) "v_and_or_b32 %5, %17, %23, %24\n\t" PF_MIX(8, 4, 0, 18, 19)
+                     PF_MFMA(2, 14, 16) PF_MIX(9, 4, 1, 18, 19) "v_and_or_b32 %6, %7, %22, %24\n\t"
+                     PF_MFMA(3, 15, 16) PF_MIX(10, 5, 0, 20, 21) "v_cvt_pk_bf16_f32 %11, %8, %9"
+                     : "+a"(c0), "+a"(c1), "+a"(c2), "+a"(c3), "=&v"(d.e), "=&v"(d.n1), "=&v"(d.n2), "=&v"(d.w8), "=&v"(d.a0), "=&v"(d.a1), "=&v"(d.b0),
+                       "=&v"(d.p0)
+                     : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b), "v"(d.w), "v"(d.d.s), "v"(d.d.c), "v"(d.d.s16), "v"(d.d.c16), "s"(low), "s"(high),
+                       "v"(magic));
+    } else {
+        // %4 b1, %5 n3, %6 a0, %7 a1, %8 p1, %9 p2, %10 b0 | %11..%14 A, %15 B, %16 n1, %17 n2, %18 w8, %19 s, %20 c, %21 s / 16, %22 its c, %23 high, %24 magic
+        asm volatile(PF_MFMA(0, 11, 15) PF_MIX(4, 16, 1, 21, 22) "v_and_or_b32 %5, %18, %23, %24\n\t"
+                     PF_MFMA(1, 12, 15) PF_MIX(6, 17, 0, 19, 20) "v_cvt_pk_bf16_f32 %8, %10, %4\n\t"
+                     PF_MFMA(2, 13, 15) PF_MIX(7, 17, 1, 19, 20) PF_MIX(10, 5, 0, 21, 22)
+                     PF_MFMA(3, 14, 15) "v_cvt_pk_bf16_f32 %9, %6, %7\n\t"
+                     "v_fma_mix_f32 %4, %5, %21, %22 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+                     : "+a"(c0), "+a"(c1), "+a"(c2), "+a"(c3), "=&v"(d.b1), "=&v"(d.o), "=&v"(d.a0), "=&v"(d.a1), "=&v"(d.p1), "=&v"(d.p2), "+v"(d.b0)
+                     : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b), "v"(d.n1), "v"(d.n2), "v"(d.w8), "v"(d.d.s), "v"(d.d.c), "v"(d.d.s16), "v"(d.d.c16),
+                       "s"(high), "v"(magic));
+    }
+#undef PF_MIX
+}
+__device__ __forceinline__ void mfma_last_slot(floatx4 &acc, const bf16x8 &a, const bf16x8 &b, DequantSlots &d) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %2, %3, %0\n\tv_cvt_pk_bf16_f32 %1, %4, %5" : "+a"(acc), "=&v"(d.p3) : "v"(a), "v"(b), "v"(d.b0), "v"(d.b1));
 }
 
 __device__ __forceinline__ void mfma_one(floatx4 &acc, const bf16x8 &a, const bf16x8 &b) {
@@ -281,12 +317,17 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     // The A operands are double buffered: K-step t multiplies from a[t % 2] while a[(t + 1) % 2] is refilled.
     bf16x8 a[2][RT];
     bf16x8 b_cur;
-    float sf[NCB], c0[NCB];
+    AwqScale scale[Q4 ? 1 : NCB];
+    uint32_t low = kLowNibbles, high = kHighNibbles, magic = kHalf1024;
+    if constexpr (!Q4) {
+        asm volatile("" : "+s"(low), "+s"(high));
+        asm volatile("" : "+v"(magic));
+    }
 
     // One quantisation group, software-pipelined over (K-step t, tile c, quarter of the 16 row tiles).  Behind every
-    // MFMA of quarters 0..2 sits a slot of the next operand's dequant; those MFMAs have no issue slot to spare.  The
-    // memory requests are spread over the group, between the quarters and behind the MFMAs of quarter 3 (two free
-    // slots each): issued as a burst at the top of the group they leave the wave in the request queue with no MFMA
+    // MFMA of quarters 0 and 1 and the first of quarter 2 (Q4NX: 0..2) sits a slot of the next operand's dequant; those
+    // MFMAs have no issue slot to spare.  The memory requests are spread over the group, between the quarters and behind the
+    // other MFMAs (two free slots each): issued as a burst at the top of the group they leave the wave in the request queue with no MFMA
     // in flight (a third of the run time), and the four waves asking for their 16 A operands at once want twice what
     // the LDS delivers.
     //   - every K-step: the 16 LDS reads that fetch the A operands of the next K-step (K-step 3: of the next group's
@@ -329,16 +370,15 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
                 if constexpr (Q4) {
                     decode_md_q4(last ? md[set ^ 1][0][0] : md[set][cn][tn], dq.sf, dq.c0);
                 } else {
-                    if (last) decode_md(md[set ^ 1][0][0], sf[0], c0[0]);
-                    dq.sf = sf[cn];
-                    dq.c0 = c0[cn];
+                    if (last) scale[0] = awq_scale(md[set ^ 1][0][0]);
+                    dq.d = scale[cn];
                 }
                 const bf16x8(&ac)[RT] = a[t & 1];
                 // This tile's share of the LDS reads that fetch the next K-step's A operands: operands n0 .. n1 - 1, all of
                 // them issued by the last tile but one, so that one wait at the head of the next K-step (instead of one
-                // in front of every quarter, each an issue slot) finds them all arrived.  The first three go between
+                // in front of every quarter, each an issue slot) finds them all arrived.  The first ones go between
                 // the quarters, where the compiler would otherwise put an s_nop (it separates asm statements that hand
-                // a register on), the rest behind the MFMAs of quarter 3.
+                // a register on), the rest behind the MFMAs with free slots.
                 constexpr int kReadTiles = NCB > 1 ? NCB - 1 : 1;   // (one tile per K-step: the reads share it)
                 constexpr int kPerTile = (RT + kReadTiles - 1) / kReadTiles;
                 const int n0 = c < kReadTiles ? c * RT / kReadTiles : RT, n1 = c < kReadTiles ? (c + 1) * RT / kReadTiles : RT;
@@ -350,38 +390,63 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
                 auto fetch_a = [&](int n) {
                     if (n < n1) a[(t + 1) & 1][n] = t < 3 ? read_a(stage, t + 1, n) : read_a(stage ^ 1, 0, n);
                 };
-                __builtin_amdgcn_sched_barrier(0);
-                mfma_quarter<0>(acc[0][c], acc[1][c], acc[2][c], acc[3][c], ac[0], ac[1], ac[2], ac[3], b_cur, dq);
-                __builtin_amdgcn_sched_barrier(0);
-                fetch_a(n0);
-                __builtin_amdgcn_sched_barrier(0);
-                mfma_quarter<1>(acc[4][c], acc[5][c], acc[6][c], acc[7][c], ac[4], ac[5], ac[6], ac[7], b_cur, dq);
-                __builtin_amdgcn_sched_barrier(0);
-                fetch_a(n0 + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                mfma_quarter<2>(acc[8][c], acc[9][c], acc[10][c], acc[11][c], ac[8], ac[9], ac[10], ac[11], b_cur, dq);
-                __builtin_amdgcn_sched_barrier(0);
-                fetch_a(n0 + 2);
-                // quarter 3: the dequant is done, two issue slots are free behind each MFMA: the other requests
+                // behind an MFMA of the tile whose issue slots are free (j of `of`): the other requests
+                auto requests = [&](int j, int of, int reads) __attribute__((always_inline)) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    mfma_one(acc[12 + k][c], ac[12 + k], b_cur);
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int n = n0 + 3 + k * (kPerTile - 3) / 4; n < n0 + 3 + (k + 1) * (kPerTile - 3) / 4; ++n) fetch_a(n);
+                    for (int n = n0 + reads + j * (kPerTile - reads) / of; n < n0 + reads + (j + 1) * (kPerTile - reads) / of; ++n) fetch_a(n);
                     // the next group's x tile (K-steps 0 and 1: early enough to have landed before K-step 3) ...
                     if (t == 0 || t == 1) {
-                        const int j = (t * NCB + c) * 4 + k;
+                        const int i = (t * NCB + c) * of + j;
 #pragma unroll
-                        for (int n = j * RT / (8 * NCB); n < (j + 1) * RT / (8 * NCB); ++n) copy_x_part(stage ^ 1, xs, n);
+                        for (int n = i * RT / (2 * of * NCB); n < (i + 1) * RT / (2 * of * NCB); ++n) copy_x_part(stage ^ 1, xs, n);
                     }
                     // ... its cells and scale words (K-step 0) ...
-                    if (t == 0 && k == 3) load_w_tile(set ^ 1, wo, c);
+                    if (t == 0 && j == of - 1) load_w_tile(set ^ 1, wo, c);
                     // ... and the scale words of its other tiles, behind the last MFMA of the group
-                    if (!Q4 && last && k == 3) {
+                    if constexpr (!Q4) {
+                        if (last && j == of - 1) {
 #pragma unroll
-                        for (int n = 1; n < NCB; ++n) decode_md(md[set ^ 1][n][0], sf[n], c0[n]);
+                            for (int n = 1; n < NCB; ++n) scale[n] = awq_scale(md[set ^ 1][n][0]);
+                        }
+                    }
+                };
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (Q4) {
+                    mfma_quarter<0>(acc[0][c], acc[1][c], acc[2][c], acc[3][c], ac[0], ac[1], ac[2], ac[3], b_cur, dq);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch_a(n0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mfma_quarter<1>(acc[4][c], acc[5][c], acc[6][c], acc[7][c], ac[4], ac[5], ac[6], ac[7], b_cur, dq);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch_a(n0 + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mfma_quarter<2>(acc[8][c], acc[9][c], acc[10][c], acc[11][c], ac[8], ac[9], ac[10], ac[11], b_cur, dq);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch_a(n0 + 2);
+                    // quarter 3: the dequant is done, two issue slots are free behind each MFMA
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        mfma_one(acc[12 + k][c], ac[12 + k], b_cur);
+                        __builtin_amdgcn_sched_barrier(0);
+                        requests(k, 4, 3);
+                    }
+                } else {
+                    mfma_quarter_awq<0>(acc[0][c], acc[1][c], acc[2][c], acc[3][c], ac[0], ac[1], ac[2], ac[3], b_cur, dq, low, high, magic);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch_a(n0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mfma_quarter_awq<1>(acc[4][c], acc[5][c], acc[6][c], acc[7][c], ac[4], ac[5], ac[6], ac[7], b_cur, dq, low, high, magic);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch_a(n0 + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mfma_last_slot(acc[8][c], ac[8], b_cur, dq);
+#pragma unroll
+                    for (int k = 0; k < 7; ++k) {   // free slots behind the other seven
+                        __builtin_amdgcn_sched_barrier(0);
+                        mfma_one(acc[9 + k][c], ac[9 + k], b_cur);
+                        __builtin_amdgcn_sched_barrier(0);
+                        requests(k, 7, 2);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -399,14 +464,16 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     __syncthreads();
     take_w(0);
     if constexpr (Q4) {
-        decode_md_q4(md[0][0][0], sf[0], c0[0]);
+        float s, c;
+        decode_md_q4(md[0][0][0], s, c);
+        b_cur = dequant_operand(cell[0][0][0], s, c);
     } else {
 #pragma unroll
-        for (int c = 0; c < NCB; ++c) decode_md(md[0][c][0], sf[c], c0[c]);
+        for (int c = 0; c < NCB; ++c) scale[c] = awq_scale(md[0][c][0]);
+        b_cur = dequant_operand_awq(cell[0][0][0], scale[0], low, high, magic);
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r) a[0][r] = read_a(0, 0, r);
-    b_cur = dequant_operand(cell[0][0][0], sf[0], c0[0]);
 
     // two groups per trip (an even number of them): stage / register set 0, then 1
     for (int g = g_lo; g < g_hi; g += 2) {

@@ -125,9 +125,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         return *reinterpret_cast<const uint32_t *>(lds + stage + wave_lds + NT * (int)kWsCellBytes + (Q4 ? 256 * c + 64 * t : 64 * c) + 4 * ln);
     };
 
-    uint32_t nib_mask = 0x000F000Fu, magic = 0x43004300u;
+    uint32_t nib_mask = kLowNibbles, high_mask = kHighNibbles, magic = kExact ? 0x43004300u : kHalf1024;
     asm volatile("" : "+s"(nib_mask));
     asm volatile("" : "+v"(magic));
+    if constexpr (MODE == kSmAwqRounded) asm volatile("" : "+s"(high_mask));
     auto exact_operand = [&](uint32_t w) {   // rows (2 v, 2 v + 1) as bf16 (128 + q)
         u32x4 b;
 #pragma unroll
@@ -205,7 +206,11 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
                 for (int c = 0; c < NT; ++c) acc[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        float s[NT], low[NT];
+        AwqScale d[NT];
+        if constexpr (MODE == kSmAwqRounded) {
+#pragma unroll
+            for (int c = 0; c < NT; ++c) d[c] = awq_scale(word[c][0]);
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             if constexpr (AHEAD == 2) {
@@ -241,9 +246,14 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], low8, Y[rt][c], 0, 0, 0);
                 } else {
-                    if (Q4) decode_md_q4(word[c][Q4 ? t : 0], s[c], low[c]);
-                    else if (t == 0) decode_md(word[c][0], s[c], low[c]);
-                    const bf16x8 b = dequant_operand(cell[c][t], s[c], low[c]);
+                    bf16x8 b;
+                    if constexpr (Q4) {
+                        float s, low;
+                        decode_md_q4(word[c][t], s, low);
+                        b = dequant_operand(cell[c][t], s, low);
+                    } else {
+                        b = dequant_operand_awq(cell[c][t], d[c], nib_mask, high_mask, magic);
+                    }
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, Y[rt][c], 0, 0, 0);
                 }

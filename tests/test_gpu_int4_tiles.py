@@ -195,3 +195,30 @@ def test_tiled_products_in_slices(q4):
         prod = ops.w4a16_gemm_stream(h, w)
         both = (prod.float() + res1.float()).bfloat16()
         assert torch.equal(out.view(torch.int16), both.view(torch.int16))
+
+
+@pytest.mark.parametrize("nt,rt", [(1, 2), (2, 5), (3, 4)])
+def test_every_weight_of_rounded_tiles(nt, rt):
+    """One-hot rows of x return the rounded weights bit for bit: every pair of nibble and zero point, under scales of either sign, down to the
+    smallest numbers and up to 2^116."""
+    from air_hip import ops
+    print("every weight", nt, rt, flush=True)
+    K, N = 256, 256
+    k, n = np.arange(K)[:, None], np.arange(N)[None, :]
+    q = ((k + n // 16) % 16).astype(np.uint8)
+    z = np.broadcast_to((n % 16).astype(np.uint8), (K // 128, N))
+    values = np.array([1.0, -0.3711, 2.0**-120, 9.2e-41, -(2.0**-126), 2.0**116, -1.99 * 2.0**115, 0.0], np.float32)
+    s = f32_to_bf16_bits(np.ascontiguousarray(values[(n // 16 + np.arange(K // 128)[:, None]) % len(values)]))
+    tri = dev(oawq.pack_awq_int32(q)), dev(oawq.pack_awq_int32(np.ascontiguousarray(z))), dev(s)
+    x, w = torch.eye(K, dtype=torch.bfloat16, device="cuda"), ops.repack_stream(*tri)
+    want = bits(ops.awq_dequant(*tri))
+    keys = ("prefill_wsm", "gemm_wsm_nt", "gemm_wsm_rt")
+    try:
+        for values in ((1, nt, rt), (2, 0, 0)):   # the tile; the tiled kernel
+            for key, value in zip(keys, values):
+                ops.tune(key, value)
+            got = bits(ops.w4a16_gemm_stream(x, w))
+            assert np.array_equal(np.where(got == 0x8000, 0, got), np.where(want == 0x8000, 0, want))   # (a sum's zero has no sign)
+    finally:
+        for key in keys:
+            ops.tune(key, 0)
