@@ -1,12 +1,14 @@
 """ctypes bindings of libw4a16_hip.so (include/w4a16.h) and libdense_lm_hip.so (include/dense_lm.h)."""
 
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libw4a16_hip.so")
 DENSE_ABI = 2
 _DENSE_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libdense_lm_hip.so")
+_HOST_PATH = os.path.join(os.path.dirname(_HERE), "lib", "air_host.so")
 
 OK = 0
 ERR_NULL, ERR_SHAPE, ERR_GROUP, ERR_ALIGN, ERR_WORKSPACE, ERR_HIP, ERR_TUNE, ERR_TIMEOUT, ERR_TOO_LARGE, ERR_NOT_PREPARED = -1, -2, -3, -4, -5, -6, -7, -8, -9, -10
@@ -224,6 +226,8 @@ class DenseLmError(W4A16Error):
 
 _lib = None
 _dense = None
+_host = None
+_host_w4a16 = _host_dense = None   # the same module, once the library's entry points are known to it
 
 
 def library_path():
@@ -237,6 +241,44 @@ def _bind(path, symbols):
         fn.restype = restype
         fn.argtypes = argtypes
     return lib
+
+
+def _load_host():
+    global _host
+    if _host is None:
+        if not os.path.exists(_HOST_PATH):
+            raise LibraryNotBuiltError(f"{_HOST_PATH} is missing: build it with `python mlir-air_amd/build.py --only host`")
+        import torch  # noqa: F401  (whose libraries the module is linked against)
+
+        spec = importlib.util.spec_from_file_location("air_host", _HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
+
+
+def _addresses(lib, names):
+    return {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}
+
+
+def host_w4a16():
+    """The host module (csrc/host.cpp) for the int4 operators."""
+    global _host_w4a16
+    if _host_w4a16 is None:
+        host = _load_host()
+        host.bind_w4a16(_addresses(load_library(), host.w4a16_entries()))
+        _host_w4a16 = host
+    return _host_w4a16
+
+
+def host_dense():
+    """The host module for the dense-weight models."""
+    global _host_dense
+    if _host_dense is None:
+        host = _load_host()
+        host.bind_dense(_addresses(load_dense_library(), host.dense_entries()))
+        _host_dense = host
+    return _host_dense
 
 
 def load_dense_library():

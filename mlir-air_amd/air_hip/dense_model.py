@@ -9,7 +9,8 @@ with `_head(pending, keys)` (fp32 logits of one position) and `_head_rows(res, r
 
 import torch
 
-from . import dense, generation, weights as wmod
+from . import _lib, dense, generation, weights as wmod
+from .ops import _stream
 
 
 def place(t, shape):
@@ -50,6 +51,7 @@ class SequenceCache:
 
 
 class DenseModel(generation.CausalLM):
+    tail_intake = None       # how a one-token product norms the last row of a finished residual: an intake of dense.py
     max_portion = None       # most tokens that go through the layers at once (None: any number)
 
     @classmethod
@@ -113,7 +115,9 @@ class DenseModel(generation.CausalLM):
             return self._tail(self._one_token(cache, ids, pos))
         for a, b in self._portions(len(ids)):
             res = self._rows(cache, ids[a:b], pos + a)
-        return self._tail(self._pending(res[-1].contiguous()))
+        last, c = res[-1], self.config
+        out = _lib.host_dense().tail(self.tail_intake, last, self.final_norm, self.head, c.eps, c.width, self.vocab, _stream())
+        return (out[0][:self.vocab], out[1]) if out is not None else self._tail(self._pending(last.contiguous()))
 
     def decode_token(self, cache, token):
         pos = self._advance(cache, 1)

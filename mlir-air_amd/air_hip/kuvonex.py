@@ -18,8 +18,9 @@ from typing import List, Optional
 import numpy as np
 import torch
 
-from . import dense
+from . import _lib, dense
 from .dense_model import DenseModel, SequenceCache, place as _place
+from .ops import _stream
 
 # Up to this many tokens a portion attends over the latents: expanding keys and values of the whole cache costs
 # rank * (dim + vdim) per cached token and head whatever the portion's length, the latent form (2 rank + rot) instead
@@ -266,6 +267,12 @@ class KuvonexModel(DenseModel):
         """M tokens (device int32 [M]) through every layer; returns the fp32 residual [M, width].  `trace`: a list that
         receives a copy of the residual after every layer."""
         c = self.config
+        if trace is None:   # every launch from one native call
+            res = _lib.host_dense().latent_rows(self.layers, [cache.rows[l.source] for l in self.layers],
+                                                [cache.tables[(l.rot_base, l.spec.rot)] for l in self.layers], tokens, self.embed, c.embed_scale, c.eps,
+                                                c.width, pos, ABSORB_MAX_TOKENS, _stream())
+            if res is not None:
+                return res
         res, h = dense.embed_rows(tokens, self.embed, c.embed_scale)
         for l in self.layers:
             attn = self._attend(l, dense.gemm(h, l.w_in), cache, pos)
@@ -278,6 +285,8 @@ class KuvonexModel(DenseModel):
             if trace is not None:
                 trace.append(res.clone())
         return res
+
+    tail_intake = dense.FINAL
 
     def _pending(self, res):
         return dense.Residual(res, None, None, self.config.eps, self.config.width)

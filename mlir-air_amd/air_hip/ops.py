@@ -250,6 +250,10 @@ def repack_stream(qweight, qzeros, scales, group=GROUP):
 def w4a16_gemv_stream(x, w, residual=None, group=GROUP, out=None):
     """Decode GEMV on a StreamWeight: y[N] = bf16(x[K] . W), with `residual` y = bf16(x . W + R).
     Stateless (no workspace)."""
+    if residual is None and out is None and group == GROUP and w.order == "awq":
+        y = _lib.host_w4a16().linear(x, w.buf, w.K, w.N, False, True, _stream())
+        if y is not None:
+            return y
     lib = _lib.load_library()
     _need_cuda(x, w.buf)
     _need_order("awq", w)
@@ -276,6 +280,10 @@ def _gemm_scratch(nbytes, device):
 def w4a16_gemm_stream(x, w, group=GROUP, out=None):
     """y[M, N] = bf16(x[M, K] . W) on a StreamWeight; x may be a vector [K].  Batches of 17 rows and more run in slices of
     K where that is the faster way, their partial sums in plain scratch of the call."""
+    if out is None and group == GROUP and w.order == "awq":
+        y = _lib.host_w4a16().linear(x, w.buf, w.K, w.N, False, False, _stream())
+        if y is not None:
+            return y
     lib = _lib.load_library()
     _need_cuda(x, w.buf)
     _need_order("awq", w)
@@ -869,6 +877,10 @@ def q4nx_blocks_to_stream(blocks, M, K, mode=0):
 
 def q4nx_gemv_stream(x, w, residual=None, out=None):
     """y[N] = bf16(x[K] . W (+ residual)) on a Q4NX-order StreamWeight; stateless, no workspace."""
+    if residual is None and out is None and w.order == "q4nx":
+        y = _lib.host_w4a16().linear(x, w.buf, w.K, w.N, True, True, _stream())
+        if y is not None:
+            return y
     lib = _lib.load_library()
     _need_cuda(x, w.buf)
     _need_order("q4nx", w)
@@ -883,6 +895,10 @@ def q4nx_gemv_stream(x, w, residual=None, out=None):
 
 def q4nx_gemm_stream(x, w, residual=None, out=None):
     """y[M, N] = bf16(x[M, K] . W (+ residual [M, N])) on a Q4NX-order StreamWeight; x may be a vector [K]."""
+    if residual is None and out is None and w.order == "q4nx":
+        y = _lib.host_w4a16().linear(x, w.buf, w.K, w.N, True, False, _stream())
+        if y is not None:
+            return y
     lib = _lib.load_library()
     _need_cuda(x, w.buf)
     _need_order("q4nx", w)

@@ -19,8 +19,9 @@ from typing import List, Optional, Tuple, Union
 
 import torch
 
-from . import dense
+from . import _lib, dense
 from .dense_model import DenseModel, SequenceCache, place
+from .ops import _stream
 
 # Up to this many tokens a portion attends with its keys split over workgroups, like a single token.
 SPLIT_MAX_TOKENS = 16
@@ -399,6 +400,11 @@ class SitiraxModel(DenseModel):
         """M tokens (device int32 [M]) through every layer; returns the fp32 residual [M, width].  `trace`: a list that
         receives a copy of the residual after every layer."""
         c, M = self.config, tokens.numel()
+        if trace is None:   # every launch from one native call
+            res = _lib.host_dense().mixed_rows(self.layers, cache.layers, tokens, self.embed, c.eps, c.width, pos, SPLIT_MAX_TOKENS, dense.STEPS_MAX_TOKENS,
+                                               UNIT_EPS, _stream())
+            if res is not None:
+                return res
         res = torch.empty((M, self.width), dtype=torch.float32, device=self.device)
         y, embedding = None, dict(tokens=tokens, embed=self.embed)
         for i, l in enumerate(self.layers):
@@ -413,6 +419,8 @@ class SitiraxModel(DenseModel):
                 trace.append(res + y.sum(0))
         dense.add_norm_rows(res, y, None, c.eps, c.width, self.dtype, **embedding)
         return res
+
+    tail_intake = dense.NORMED
 
     def _pending(self, res):
         return dense.Sum(res)

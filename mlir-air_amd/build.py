@@ -25,10 +25,11 @@ LIBRARIES = {
                  "head_attention.hip", "linear_attention.hip", "linear_chunks.hip", "mixer_steps.hip"],
 }
 SOURCES = [s for sources in LIBRARIES.values() for s in sources]
+HOST = "host"   # csrc/host.cpp, a Python module on torch's C++ interface; no GPU code, loads without the other two
 
 
 def lib_path(name):
-    return os.path.join(LIB_DIR, f"lib{name}_hip.so")
+    return os.path.join(LIB_DIR, "air_host.so" if name == HOST else f"lib{name}_hip.so")
 
 
 LIB_PATH = lib_path("w4a16")
@@ -68,14 +69,34 @@ def _compile(src, extra):
     return obj, out
 
 
+def _build_host():
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = f"{lib_path(HOST)}.{os.getpid()}"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(a for d in include_paths() for a in ("-isystem", d)), "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "host.cpp"), "-o", tmp,
+           *(f"-L{d}" for d in library_paths()), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for host.cpp:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, lib_path(HOST))
+
+
 def build(jobs=4, extra=(), verbose=False, only=None):
     """Compile and link the libraries named in `only` (default: all); returns the path of the last one."""
-    names = list(only or LIBRARIES)
+    names = list(only or (*LIBRARIES, HOST))
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
+    host, names = HOST in names, [n for n in names if n != HOST]
     sources = [s for name in names for s in LIBRARIES[name]]
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_build_host) if host else None
         results = dict(zip(sources, pool.map(lambda s: _compile(s, list(extra)), sources)))
+        if host:
+            host.result()
     for _, out in results.values():
         if out.strip() and verbose:
             print(out)
@@ -84,7 +105,7 @@ def build(jobs=4, extra=(), verbose=False, only=None):
         tmp = f"{lib_path(name)}.{os.getpid()}"   # renamed when whole: nobody loads half a library
         subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs])
         os.replace(tmp, lib_path(name))
-    return lib_path(names[-1])
+    return lib_path(names[-1] if names else HOST)
 
 
 @contextlib.contextmanager
@@ -96,11 +117,12 @@ def _lock():
 
 
 def ensure(name, jobs=8):
-    """The library `name`, built first if there is none (one builder at a time)."""
-    if not os.path.exists(lib_path(name)):
+    """The library `name` and the host module, built first where there is none (one builder at a time)."""
+    if not all(os.path.exists(lib_path(n)) for n in (name, HOST)):
         with _lock():
-            if not os.path.exists(lib_path(name)):
-                build(jobs, only=[name])
+            missing = [n for n in (name, HOST) if not os.path.exists(lib_path(n))]
+            if missing:
+                build(jobs, only=missing)
     return lib_path(name)
 
 
@@ -108,7 +130,7 @@ if __name__ == "__main__":
     ap = argparse.ArgumentParser()
     ap.add_argument("-j", type=int, default=4)
     ap.add_argument("-v", action="store_true")
-    ap.add_argument("--only", nargs="*", choices=list(LIBRARIES), help="build these libraries only")
+    ap.add_argument("--only", nargs="*", choices=[*LIBRARIES, HOST], help="build these libraries only")
     ap.add_argument("--save-temps", action="store_true", help="keep ISA (.s) files under build/")
     a = ap.parse_args()
     extra = ["-save-temps=obj"] if a.save_temps else []
