@@ -20,6 +20,7 @@
 // row and never stored.
 #include "dense.h"
 #include "dense_kernels.h"
+#include <utility>
 
 namespace w4a16 {
 
@@ -264,10 +265,10 @@ __device__ constexpr int copy_behind(int n, int products, int items) {
 // A wave's NT x MT tiles by way of LDS, 16 rows at a time: what leaves is whole 16-byte pieces, as many rows' side by side as a wave
 // has lanes for.  (store_tile's pieces are 8 bytes, 32 together: 2048 x 6656 x 2048 took 61 us with them, 56 with these.)
 constexpr int kWideStore = 16 * (16 * 8 + 8) * (int)sizeof(float);   // of a wave: 16 rows and their padding
-// SCATTER: rows of the result are entries; without a pair out_rows holds where the wave's rows 0 .. 63 and 64 .. 127 go, a lane each.
+// SCATTER: rows of the result are entries; without a pair out_rows holds where the wave's rows go, 64 an element, a lane each.
 template <int NT, int MT, int EPI, bool GROUPED, bool SCATTER>
 __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx4 (&acc)[NT][MT], char *lds, int m_first, int m_end, int n_first,
-                                           const int (&out_rows)[2] = {0, 0}) {
+                                           const int (&out_rows)[3] = {0, 0, 0}) {
     typedef typename std::conditional<EPI == kOutF32, float, bf16>::type Out;
     constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
     constexpr int kCols = 16 * NT / (kPair ? 2 : 1), kPiece = 16 / (int)sizeof(Out), kPitch = kCols + kPiece;
@@ -472,12 +473,15 @@ __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const 
 
 
 // ---- experts, bf16 -----------------------------------------------------------------------------------------------------------
-// 64 MT rows of an expert (MT <= 6) x 128 columns, four waves one below the other, a wave 16 MT rows x 128 columns.
+// 32 R rows of an expert (R <= 12) x 128 columns, four waves two by two, a wave 16 R rows x 64 columns.
 //
 // What bounds it: an expert's W is read for its few hundred rows alone, so HBM (W once: 64 experts of 2048 x 2048 take 100 us) as well as the
-// matrix pipe.  A workgroup has all of an expert's rows where they are 384 or less (else even parts of them), so W leaves HBM once, in
-// 128 columns, so that there are many workgroups of even work, and does whole 64-row tiles' products only.
-// A K-step is two halves of 8 MT products of 16 cycles; each half's operands are read during the one before it.  One wait and barrier
+// matrix pipe, and LDS beside it: a K-step of 256 rows reads 96 KiB and fills 48, 1152 cycles of LDS for 1024 of products.  A workgroup has all of an
+// expert's rows where they are 384 or less (else even parts of them), so W leaves HBM once, in
+// 128 columns, so that there are many workgroups of even work, and does whole 32-row steps' products only.  (Four waves one below the other, 64-row
+// steps: the same reads from LDS at 256 rows, but 32 rows of padding an expert on average instead of 16, multiplied, copied and read.  64 experts
+// of 2 x 1024 x 2048 and 1024 x 2048, 16384 entries 196 + 111 -> 191.5 + 108 us; 8 experts of 2 x 1408 x 1024, 600 entries 13.2 + 13.2 -> 12.1 + 11.8.)
+// A K-step is two halves of 4 R products of 16 cycles; each half's operands are read during the one before it.  One wait and barrier
 // stand between the halves: all of the next K-step has landed, everybody has read all of this one, and the copies of a K-step two or three
 // on (buffers: W three, A three up to 256 rows, else two; more of them for few rows were no faster) go out behind the products after it.
 // Few rows (plans of 128 to a tile): two workgroups to a CU, whose starts and stores then stand beside each other's products; 80 KiB of LDS and
@@ -486,19 +490,25 @@ __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const 
 // expert on average and up to 188, 117 / 138 + 77 / 80, which is where the second reading of W costs more: up to 64 on average.
 constexpr int kExpertCols = 128, kExpertRows = 384, kFewRows = 128, kFewMean = 64;
 constexpr int kExpertStagesW = 3;
-constexpr int expert_stages_a(int mt, bool few) { return mt <= (few ? 1 : 4) ? 3 : 2; }
-constexpr size_t expert_lds(int mt, bool few) { return (size_t)(expert_stages_a(mt, few) * 64 * mt + kExpertStagesW * kExpertCols) * kRowBytes; }
+constexpr int expert_stages_a(int r, bool few) { return r <= (few ? 2 : 8) ? 3 : 2; }
+constexpr size_t expert_lds(int r, bool few) { return (size_t)(expert_stages_a(r, few) * 32 * r + kExpertStagesW * kExpertCols) * kRowBytes; }
+// f(0) .. f(N - 1), the number known to the compiler (which leaves long loops around loops as they are)
+template <class F, int... N>
+__device__ __forceinline__ void each_of(F &&f, std::integer_sequence<int, N...>) { (f(std::integral_constant<int, N>()), ...); }
+template <int N, class F>
+__device__ __forceinline__ void each(F &&f) { each_of(f, std::make_integer_sequence<int, N>()); }
 // of `items` that are to be spread over the products [0, upto): the first one that goes behind product n or later
 __device__ constexpr int items_before(int n, int upto, int items) { return n >= upto ? items : n * items / upto; }
 
-template <int MT, int EPI, bool SCATTER, bool FEW>
+template <int R, int EPI, bool SCATTER, bool FEW>
 __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, int first) {
-    constexpr int kSideA = 64 * MT * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(MT, FEW), RW = kExpertStagesW;
-    constexpr int kBehind = RA == RW ? (RA - 2) * (2 * MT + 4) : 4;   // copies that may be on their way at the wait
-    constexpr int CA = 2 * MT, CW = 4, V = CA + CW, kEarly = V / 2;   // copies of a wave and K-step; those right behind the barrier
-    constexpr int kProducts = 8 * MT, kReads = 8 + MT, kReadsUpto = MT == 1 ? 4 : kProducts * 3 / 4;
+    constexpr int kSideA = 32 * R * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(R, FEW), RW = kExpertStagesW;
+    constexpr int kBehind = RA == RW ? (RA - 2) * (R + 4) : 4;   // copies that may be on their way at the wait
+    constexpr int CA = R, CW = 4, V = CA + CW, kEarly = V / 2;   // copies of a wave and K-step; those right behind the barrier
+    constexpr int kProducts = 4 * R, kReads = 4 + R, kReadsUpto = kProducts * 3 / 4;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / 2, wn = wave % 2;
     const int ql = lane & 15, g = lane >> 4;
 
     // copies as in wide_tile: KiB i of the wave's part of a stage, eight rows, lane's chunk (lane % 8) ^ row % 8
@@ -560,43 +570,46 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
         const uint32_t o = ql * kRowBytes + 16 * ((4 * ks + g) ^ (ql & 7));
-        at_a[ks] = o + wave * 16 * MT * kRowBytes;
-        at_w[ks] = o + RA * kSideA;
+        at_a[ks] = o + wm * 16 * R * kRowBytes;
+        at_w[ks] = o + RA * kSideA + wn * 64 * kRowBytes;
     }
     auto read = [&](uint32_t at, int i) { return *reinterpret_cast<const bf16x8 *>(lds + at + i * 16 * kRowBytes); };
 
     // where the second product's rows go: asked for here, because a store that has to ask waits once per 16 rows (down of 64 experts of
     // 1024 x 2048, 16384 entries: 109 -> 101 us, with nothing read past the last K-step)
-    int out_rows[2] = {0, 0};
+    int out_rows[3] = {0, 0, 0};
     if constexpr (SCATTER && EPI == kOutElem) {
-        const int own = m0 + wave * 16 * MT;
-        out_rows[0] = p.order[own + lane < m_end ? own + lane : m_end - 1];
-        if (MT > 4) out_rows[1] = p.order[own + 64 + lane < m_end ? own + 64 + lane : m_end - 1];
+#pragma unroll
+        for (int i = 0; i < (R + 3) / 4; ++i) {
+            const int own = m0 + wm * 16 * R + 64 * i + lane;
+            out_rows[i] = p.order[own < m_end ? own : m_end - 1];
+        }
     }
 
-    floatx4 acc[8][MT];
+    floatx4 acc[4][R];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 a0[MT], a1[MT], w0[8], w1[8];
-    // 8 MT products with the reads of the next half and copies [c0, c1) of a K-step behind them
-    auto half = [&](const bf16x8 (&wh)[8], const bf16x8 (&ah)[MT], bf16x8 (&wn)[8], bf16x8 (&an)[MT], uint32_t from_wn, uint32_t from_an, auto c0, auto c1) {
-#pragma unroll
-        for (int n = 0; n < kProducts; ++n) {
+        for (int i = 0; i < R; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 a0[R], a1[R], w0[4], w1[4];
+    // 4 R products with the reads of the next half and copies [c0, c1) of a K-step behind them
+    auto half = [&](const bf16x8 (&wh)[4], const bf16x8 (&ah)[R], bf16x8 (&wx)[4], bf16x8 (&ax)[R], uint32_t from_wx, uint32_t from_ax, auto c0, auto c1) {
+        each<kProducts>([&](auto product) __attribute__((always_inline)) {
+            constexpr int n = decltype(product)::value;
+            constexpr int r0 = items_before(n, kReadsUpto, kReads), r1 = items_before(n + 1, kReadsUpto, kReads);
+            constexpr int k0 = decltype(c0)::value + items_before(n, kProducts, decltype(c1)::value - decltype(c0)::value);
+            constexpr int k1 = decltype(c0)::value + items_before(n + 1, kProducts, decltype(c1)::value - decltype(c0)::value);
             __builtin_amdgcn_sched_barrier(0);
-            mfma_in_place(acc[n % 8][n / 8], wh[n % 8], ah[n / 8]);
+            mfma_in_place(acc[n % 4][n / 4], wh[n % 4], ah[n / 4]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < kReads; ++r)
-                if (r >= items_before(n, kReadsUpto, kReads) && r < items_before(n + 1, kReadsUpto, kReads)) {
-                    if (r < 8) wn[r < 8 ? r : 0] = read(from_wn, r);
-                    else an[r < 8 ? 0 : r - 8] = read(from_an, r - 8);
-                }
+            for (int r = r0; r < r1; ++r) {
+                if (r < 4) wx[r < 4 ? r : 0] = read(from_wx, r);
+                else ax[r < 4 ? 0 : r - 4] = read(from_ax, r - 4);
+            }
 #pragma unroll
-            for (int c = 0; c < V; ++c)
-                if (c >= c0 + items_before(n, kProducts, c1 - c0) && c < c0 + items_before(n + 1, kProducts, c1 - c0)) step_copy(c);
-        }
+            for (int c = k0; c < k1; ++c) step_copy(c);
+        });
     };
 
     // All buffers but one each, and the first copies of the next K-step (with two buffers for A and three for W, A of K-step t + 2 goes with
@@ -611,9 +624,9 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 8; ++j) w0[j] = read(at_w[0], j);
+    for (int j = 0; j < 4; ++j) w0[j] = read(at_w[0], j);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) a0[i] = read(at_a[0], i);
+    for (int i = 0; i < R; ++i) a0[i] = read(at_a[0], i);
 
     int side_a = 0, side_w = 0;   // of the K-step that is multiplied
 #pragma unroll 1
@@ -637,9 +650,8 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-        asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]), "+a"(acc[4][i]), "+a"(acc[5][i]), "+a"(acc[6][i]), "+a"(acc[7][i]));
-    store_rows<8, MT, EPI, true, SCATTER>(p, acc, lds + wave * kWideStore, m0 + wave * 16 * MT, m_end, n0, out_rows);
+    for (int i = 0; i < R; ++i) asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]));
+    store_rows<4, R, EPI, true, SCATTER>(p, acc, lds + wave * kWideStore, m0 + wm * 16 * R, m_end, n0 + wn * 64, out_rows);
 }
 
 // (SCATTER is gather == 0: asked at run time it cost gate and up 1.7 %)
@@ -655,19 +667,30 @@ __global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_k
     const bf16 *w = p.w + (size_t)t[0] * p.w_stride;
     const int first = (5 * t[0] + 3 * (tile % p.tiles_n)) % (p.K / 64);
     if constexpr (FEW) {
-        if (t[2] <= 64) return expert_tile<1, EPI, SCATTER, true>(p, gemm_lds, w, m0, m_end, n0, first);
         for (int m = m0; m < m_end; m += kFewRows) {   // (once, for a plan of the tile_rows that the launch was given)
             if (m > m0) __syncthreads();
-            expert_tile<2, EPI, SCATTER, true>(p, gemm_lds, w, m, m_end - m < kFewRows ? m_end : m + kFewRows, n0, first);
+            const int end = m_end - m < kFewRows ? m_end : m + kFewRows;
+            switch ((end - m + 31) / 32) {
+                case 1: expert_tile<1, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
+                case 2: expert_tile<2, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
+                case 3: expert_tile<3, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
+                default: expert_tile<4, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
+            }
         }
     } else {
-        switch ((t[2] + 63) / 64) {
+        switch ((t[2] + 31) / 32) {
             case 1: return expert_tile<1, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
             case 2: return expert_tile<2, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
             case 3: return expert_tile<3, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
             case 4: return expert_tile<4, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
             case 5: return expert_tile<5, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            default: return expert_tile<6, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 6: return expert_tile<6, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 7: return expert_tile<7, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 8: return expert_tile<8, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 9: return expert_tile<9, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 10: return expert_tile<10, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 11: return expert_tile<11, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            default: return expert_tile<12, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
         }
     }
 }
@@ -738,9 +761,9 @@ hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
 template <bool FEW>
 hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
     const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, kExpertRows, kExpertCols);
-    constexpr size_t lds = FEW ? expert_lds(2, true) : expert_lds(6, false);
+    constexpr size_t lds = FEW ? expert_lds(4, true) : expert_lds(12, false);
     static_assert(lds <= (FEW ? 80 : 160) * 1024 && 4 * kWideStore <= lds, "fits LDS, twice for few rows");
-    static_assert(FEW ? expert_lds(1, true) <= lds : expert_lds(4, false) <= lds && expert_lds(5, false) <= lds, "the other heights too");
+    static_assert(FEW ? expert_lds(2, true) <= lds : expert_lds(8, false) <= lds, "the heights with a buffer more too");
     auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, lds, 1, stream); };
     if (g.epilogue == kOutSwiglu) return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutSwiglu, true, FEW>) : run(&dense_gemm_expert_kernel<kOutSwiglu, false, FEW>);
     return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutElem, true, FEW>) : run(&dense_gemm_expert_kernel<kOutElem, false, FEW>);

@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(1024) moe_plan_kernel(const int32_t *ids, int 
         total += sums[1][w];
     }
     first[t] = runs;
-    const int each = bm > 256 && bm % 64 == 0 && n ? ((n + parts - 1) / parts + 63) / 64 * 64 : bm;
+    const int each = bm > 256 && bm % 64 == 0 && n ? ((n + parts - 1) / parts + 31) / 32 * 32 : bm;
     if (t < experts)
         for (int i = 0; i < parts; ++i) {
             int32_t *row = tiles + 4 * (cut + i);

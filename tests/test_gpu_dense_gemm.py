@@ -183,6 +183,12 @@ def test_experts_with_tiles_of_every_fill(dense, counts, tile_rows, launched):
         close(out[at], got.double() @ w2[i].double().t(), True, ("down", i))
 
 
+@pytest.mark.parametrize("tile_rows", [128, 384])
+@pytest.mark.parametrize("past", [-1, 0, 1])
+def test_experts_with_tiles_of_every_height(dense, tile_rows, past):
+    test_experts_with_tiles_of_every_fill(dense, [32 * r + past for r in range(1, 1 + tile_rows // 32)], tile_rows, tile_rows)
+
+
 @pytest.mark.parametrize("dtype,tile_rows", [(torch.bfloat16, 32), (torch.bfloat16, 128), (torch.bfloat16, 384), (torch.float32, 32), (torch.float32, 128)])
 @pytest.mark.parametrize("pair", [False, True])
 def test_grouped_products_with_rows_in_either_order(dense, dtype, tile_rows, pair):
