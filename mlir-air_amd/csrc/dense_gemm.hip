@@ -500,7 +500,9 @@ __device__ __forceinline__ void each(F &&f) { each_of(f, std::make_integer_seque
 // of `items` that are to be spread over the products [0, upto): the first one that goes behind product n or later
 __device__ constexpr int items_before(int n, int upto, int items) { return n >= upto ? items : n * items / upto; }
 
-template <int R, int EPI, bool SCATTER, bool FEW>
+// (LONG: rows of A further apart than 32-bit offsets reach; a 64-bit address a copy, added up in two steps, holds the products up.  4096 tokens of 8
+// experts, 64 of 2 x 1024 x 2048 and 1024 x 2048: 308 + 173 us with them, 294 + 166 without.)
+template <int R, int EPI, bool SCATTER, bool FEW, bool LONG>
 __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, int first) {
     constexpr int kSideA = 32 * R * kRowBytes, kSideW = kExpertCols * kRowBytes, RA = expert_stages_a(R, FEW), RW = kExpertStagesW;
     constexpr int kBehind = RA == RW ? (RA - 2) * (R + 4) : 4;   // copies that may be on their way at the wait
@@ -512,15 +514,18 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     const int ql = lane & 15, g = lane >> 4;
 
     // copies as in wide_tile: KiB i of the wave's part of a stage, eight rows, lane's chunk (lane % 8) ^ row % 8
-    const char *row_a[CA];
-    uint32_t off_w[CW];
+    uint32_t off_a[CA], off_w[CW];
+    size_t far_a[LONG ? CA : 1];
+    const int m_wave = p.gather > 0 ? 0 : m0 + 8 * CA * wave < m_end ? m0 + 8 * CA * wave : m_end - 1;
     const int n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
         const int row = 8 * (CA * wave + i) + (lane >> 3);
         int m = m0 + row < m_end ? m0 + row : m_end - 1;
         if (p.gather > 0) m = p.order[m] / p.gather;
-        row_a[i] = reinterpret_cast<const char *>(p.a + (size_t)m * p.lda) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+        const uint32_t chunk = 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+        if constexpr (LONG) far_a[i] = (size_t)(m - m_wave) * (p.lda * sizeof(bf16)) + chunk;
+        else off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + chunk;
     }
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
@@ -529,8 +534,9 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
         off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
     }
     const int steps = p.K / 64;
-    ptrdiff_t from_a = (ptrdiff_t)first * kRowBytes - 4096;
-    gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from_a);
+    const ptrdiff_t from = (ptrdiff_t)first * kRowBytes - 4096;
+    gptr base_a = scalar_ptr(reinterpret_cast<const char *>(p.a + (size_t)m_wave * p.lda) + from);
+    gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from);
     auto copy = [&](gptr from, int at, int i) {
         const auto *src = (const __attribute__((address_space(1))) void *)from;
         auto *dst = (__attribute__((address_space(3))) void *)(lds + at + 1024 * (i & ~3));
@@ -547,11 +553,12 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
     int next_a = first, next_w = first, left_a = steps - 1, left_w = steps - 1;
     auto step_copy = [&](int i) {
         if (i < CA) {
-            copy((gptr)(row_a[i < CA ? i : 0] + from_a), fill_a + 1024 * CA * wave, i);
+            if constexpr (LONG) copy((gptr)(base_a + far_a[i < CA ? i : 0]), fill_a + 1024 * CA * wave, i);
+            else copy(base_a + off_a[i < CA ? i : 0], fill_a + 1024 * CA * wave, i);
             if (i == CA - 1) {
                 const bool more = left_a-- > 0, wrap = next_a + 1 == steps;
                 next_a = wrap ? 0 : next_a + 1;
-                from_a += !more ? 0 : wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
+                base_a += !more ? 0 : wrap ? kRowBytes - steps * kRowBytes : kRowBytes;
                 fill_a = fill_a == (RA - 1) * kSideA ? 0 : fill_a + kSideA;
             }
         } else {
@@ -600,7 +607,9 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
             constexpr int k0 = decltype(c0)::value + items_before(n, kProducts, decltype(c1)::value - decltype(c0)::value);
             constexpr int k1 = decltype(c0)::value + items_before(n + 1, kProducts, decltype(c1)::value - decltype(c0)::value);
             __builtin_amdgcn_sched_barrier(0);
-            mfma_in_place(acc[n % 4][n / 4], wh[n % 4], ah[n / 4]);
+            // (the last ones are the compiler's: what it puts behind the loop, a move of the accumulators say, it then makes wait for them)
+            if constexpr (n < kProducts - 4) mfma_in_place(acc[n % 4][n / 4], wh[n % 4], ah[n / 4]);
+            else acc[n % 4][n / 4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[n % 4], ah[n / 4], acc[n % 4][n / 4], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int r = r0; r < r1; ++r) {
@@ -632,6 +641,9 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
 #pragma unroll 1
     for (int kt = 0; kt < steps; ++kt) {
 #pragma unroll
+        for (int i = 0; i < CA; ++i)
+            if constexpr (!LONG) asm volatile("" : "+v"(off_a[i]));
+#pragma unroll
         for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
         half(w0, a0, w1, a1, at_w[1], at_a[1], std::integral_constant<int, kEarly>(), std::integral_constant<int, V>());
         __builtin_amdgcn_sched_barrier(0);
@@ -645,17 +657,15 @@ __device__ __forceinline__ void expert_tile(const GemmKernelArgs<bf16> &p, char 
         for (int ks = 0; ks < 2; ++ks) at_a[ks] += by_a, at_w[ks] += by_w;
         half(w1, a1, w0, a0, at_w[0], at_a[0], std::integral_constant<int, 0>(), std::integral_constant<int, kEarly>());
     }
-    // no copy, of any wave, is on its way to LDS any more; the products have left the matrix pipe
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    // no copy, of any wave, is on its way to LDS any more
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < R; ++i) asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i]));
     store_rows<4, R, EPI, true, SCATTER>(p, acc, lds + wave * kWideStore, m0 + wm * 16 * R, m_end, n0 + wn * 64, out_rows);
 }
 
 // (SCATTER is gather == 0: asked at run time it cost gate and up 1.7 %)
-template <int EPI, bool SCATTER, bool FEW>
+template <int EPI, bool SCATTER, bool FEW, bool LONG>
 __global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_kernel(const GemmKernelArgs<bf16> p) {
     extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
     const int tiles_m = p.tiles[4 * p.tiles_m];
@@ -671,26 +681,28 @@ __global__ void __launch_bounds__(kWideThreads, FEW ? 2 : 1) dense_gemm_expert_k
             if (m > m0) __syncthreads();
             const int end = m_end - m < kFewRows ? m_end : m + kFewRows;
             switch ((end - m + 31) / 32) {
-                case 1: expert_tile<1, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
-                case 2: expert_tile<2, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
-                case 3: expert_tile<3, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
-                default: expert_tile<4, EPI, SCATTER, true>(p, gemm_lds, w, m, end, n0, first); break;
+                case 1: expert_tile<1, EPI, SCATTER, true, false>(p, gemm_lds, w, m, end, n0, first); break;
+                case 2: expert_tile<2, EPI, SCATTER, true, false>(p, gemm_lds, w, m, end, n0, first); break;
+                case 3: expert_tile<3, EPI, SCATTER, true, false>(p, gemm_lds, w, m, end, n0, first); break;
+                default: expert_tile<4, EPI, SCATTER, true, false>(p, gemm_lds, w, m, end, n0, first); break;
             }
         }
+    } else if constexpr (LONG) {
+        expert_tile<12, EPI, SCATTER, false, true>(p, gemm_lds, w, m0, m_end, n0, first);
     } else {
         switch ((t[2] + 31) / 32) {
-            case 1: return expert_tile<1, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 2: return expert_tile<2, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 3: return expert_tile<3, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 4: return expert_tile<4, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 5: return expert_tile<5, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 6: return expert_tile<6, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 7: return expert_tile<7, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 8: return expert_tile<8, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 9: return expert_tile<9, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 10: return expert_tile<10, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            case 11: return expert_tile<11, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
-            default: return expert_tile<12, EPI, SCATTER, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 1: return expert_tile<1, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 2: return expert_tile<2, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 3: return expert_tile<3, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 4: return expert_tile<4, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 5: return expert_tile<5, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 6: return expert_tile<6, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 7: return expert_tile<7, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 8: return expert_tile<8, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 9: return expert_tile<9, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 10: return expert_tile<10, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            case 11: return expert_tile<11, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
+            default: return expert_tile<12, EPI, SCATTER, false, false>(p, gemm_lds, w, m0, m_end, n0, first);
         }
     }
 }
@@ -758,15 +770,15 @@ hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
     }
 }
 
-template <bool FEW>
+template <bool FEW, bool LONG>
 hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
     const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, kExpertRows, kExpertCols);
     constexpr size_t lds = FEW ? expert_lds(4, true) : expert_lds(12, false);
     static_assert(lds <= (FEW ? 80 : 160) * 1024 && 4 * kWideStore <= lds, "fits LDS, twice for few rows");
     static_assert(FEW ? expert_lds(2, true) <= lds : expert_lds(8, false) <= lds, "the heights with a buffer more too");
     auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, lds, 1, stream); };
-    if (g.epilogue == kOutSwiglu) return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutSwiglu, true, FEW>) : run(&dense_gemm_expert_kernel<kOutSwiglu, false, FEW>);
-    return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutElem, true, FEW>) : run(&dense_gemm_expert_kernel<kOutElem, false, FEW>);
+    if (g.epilogue == kOutSwiglu) return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutSwiglu, true, FEW, LONG>) : run(&dense_gemm_expert_kernel<kOutSwiglu, false, FEW, LONG>);
+    return g.gather == 0 ? run(&dense_gemm_expert_kernel<kOutElem, true, FEW, LONG>) : run(&dense_gemm_expert_kernel<kOutElem, false, FEW, LONG>);
 }
 
 // out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
@@ -881,7 +893,10 @@ hipError_t launch_dense_gemm(int dtype, const GemmArgs &g, int tile_rows, hipStr
     if (dtype == kF32) return tile_rows == 32 ? launch_tile<float, 32, 128, 1, 4, 4>(g, 1, stream) : launch_tile<float, 128, 128, 2, 2, 2>(g, 1, stream);
     if (g.tiles) {   // (any plan: its tiles are 384 rows or less)
         if (g.K >= 1 << 26) return hipErrorInvalidValue;
-        return tile_rows <= kFewRows ? launch_experts<true>(g, stream) : launch_experts<false>(g, stream);
+        // the copies' 32-bit offsets: from the first row of A where rows are gathered, else within a wave's part of a tile
+        const long rows = g.gather > 0 ? (g.M + g.gather - 1) / g.gather : kExpertRows;
+        if (rows * g.lda >= (1L << 31) - 4096) return launch_experts<false, true>(g, stream);
+        return tile_rows <= kFewRows ? launch_experts<true, false>(g, stream) : launch_experts<false, false>(g, stream);
     }
     if (tile_rows == 32) return launch_tile<bf16, 32, 128, 1, 4, 4>(g, 1, stream);
     return launch_kind(g, tile_rows == 256 ? kWide256 : kWide128, 1, stream);

@@ -189,6 +189,31 @@ def test_experts_with_tiles_of_every_height(dense, tile_rows, past):
     test_experts_with_tiles_of_every_fill(dense, [32 * r + past for r in range(1, 1 + tile_rows // 32)], tile_rows, tile_rows)
 
 
+@pytest.mark.parametrize("gather,lda", [(1, 1 << 30), (2, 1 << 29), (0, 6 << 20)])   # 3 tokens' rows past 2^32 bytes, below them, a tile's past them
+def test_experts_with_rows_far_apart(dense, gather, lda):
+    print("experts with rows of", lda, "gathered", gather, flush=True)
+    from air_hip import _lib
+    lib, stream = _lib.load_dense_library(), torch.cuda.current_stream().cuda_stream
+    E, K, N, tokens = 3, 128, 144, 3
+    entries = tokens * max(gather, 1)
+    ids = torch.tensor([2, 0, 2, 0, 0, 2][:entries], dtype=torch.int32, device="cuda")
+    a = torch.empty(((tokens if gather else entries) - 1) * lda + K, dtype=torch.bfloat16, device="cuda").as_strided((tokens if gather else entries, K), (lda, 1))
+    a.copy_(rand(1, *a.shape))
+    w = (rand(2, E, N, K) * K ** -0.5).bfloat16()
+    order = torch.empty((entries,), dtype=torch.int32, device="cuda")
+    n_tiles = lib.dlm_moe_max_tiles(entries, E, 128)
+    tiles = torch.empty((n_tiles + 1, 4), dtype=torch.int32, device="cuda")
+    _lib.check_dense(lib.dlm_moe_plan(ids.data_ptr(), entries, E, 128, order.data_ptr(), tiles.data_ptr(), stream))
+    out = torch.full((entries, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    g = _lib.GemmArgs(a=a.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), lda=lda, ldo=N, w_stride=N * K, N=N, K=K, gather=gather, tiles=tiles.data_ptr(),
+                      epilogue=dense.OUT_ELEM, order=order.data_ptr(), M=entries, n_tiles=n_tiles, tile_rows=128)
+    _lib.check_dense(lib.dlm_gemm(0, ctypes.byref(g), stream))
+    at = order.long()
+    rows = a[at // gather] if gather else a
+    want = torch.stack([w[e].double() @ r.double() for e, r in zip(ids[at].tolist(), rows)])
+    close(out if gather else out[at], want, True, (gather, lda))
+
+
 @pytest.mark.parametrize("dtype,tile_rows", [(torch.bfloat16, 32), (torch.bfloat16, 128), (torch.bfloat16, 384), (torch.float32, 32), (torch.float32, 128)])
 @pytest.mark.parametrize("pair", [False, True])
 def test_grouped_products_with_rows_in_either_order(dense, dtype, tile_rows, pair):
