@@ -477,6 +477,10 @@ int w4a16_prefill_rms_qkv_rope_bf16(const uint16_t *x, const uint16_t *attn_norm
 int w4a16_prefill_attention_bf16(const uint16_t *qkv, uint16_t *attn_out, int M, int n_heads, int n_kv_heads,
                                  int head_dim, void *stream);
 
+/* The same, and rows 0 .. M - 1 of the caches [n_kv_heads, max_seq, head_dim] become the K and V of qkv; max_seq >= M. */
+int w4a16_prefill_attention_cache_bf16(const uint16_t *qkv, uint16_t *k_cache, uint16_t *v_cache, uint16_t *attn_out, int M,
+                                       int max_seq, int n_heads, int n_kv_heads, int head_dim, void *stream);
+
 /*
  * Tail of a decode step: final RMSNorm, bf16 lm_head GEMV and argmax in one call
  * (run_npu_decode_step, programming_examples/llms/llama32_1b_int4/llama32_1b_int4_inference.py:459-486:

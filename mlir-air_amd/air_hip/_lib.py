@@ -47,6 +47,7 @@ SYMBOLS = {
     "w4a16_q4nx_prefill_rms_qkv_rope_stream_bf16": (_ci, [_vp, _vp, _cf, _vp, _vp, _ci, _ci, _vp] + [_ci] * 5 + [_vp, _sz, _vp]),
     "w4a16_q4nx_prefill_o_ffn_stream_bf16": (_ci, [_vp, _vp, _vp, _cf] + [_vp] * 7 + [_ci, _ci, _ci, _vp, _sz, _vp]),
     "w4a16_prefill_attention_bf16": (_ci, [_vp, _vp, _ci, _ci, _ci, _ci, _vp]),
+    "w4a16_prefill_attention_cache_bf16": (_ci, [_vp] * 4 + [_ci] * 5 + [_vp]),
     "lm_head_workspace_bytes": (_sz, [_ci]),
     "w4a16_decode_attn_o_gemv_ffn_bf16": (_ci, [_vp] * 5 + [_ci] * 5 + [_vp, _sz, _vp, _vp, _cf] + [_vp] * 12 + [_vp, _vp, _ci, _ci, _ci, _vp, _sz, _vp]),
     "w4a16_rms_gemv_sumsq_bf16": (_ci, [_vp, _vp, _ci, _vp, _cf, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _vp, _sz, _vp]),

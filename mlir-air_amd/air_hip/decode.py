@@ -213,10 +213,7 @@ def run_prefill_layer(x, layer: DecodeLayer, config, k_cache_layer, v_cache_laye
                                               codec=layer.codec)
     else:
         qkv = ops.prefill_rms_qkv_rope(x, layer.attn_norm, layer.wqkv, rope_lut, 0, nh, nkv, hd, eps=config.rms_eps)
-    nq, nk = nh * hd, nkv * hd
-    k_cache_layer[:, :M].copy_(qkv[:, nq:nq + nk].reshape(M, nkv, hd).transpose(0, 1))
-    v_cache_layer[:, :M].copy_(qkv[:, nq + nk:].reshape(M, nkv, hd).transpose(0, 1))
-    attn_out = ops.prefill_attention(qkv, nh, nkv, hd)
+    attn_out = ops.prefill_attention(qkv, nh, nkv, hd, k_cache_layer, v_cache_layer)
     if sw is not None:
         return ops.prefill_o_ffn_stream(attn_out, x, layer.ffn_norm, sw["wo"], sw["w_gate"], sw["w_up"], sw["w_down"], eps=config.rms_eps,
                                         codec=layer.codec)

@@ -630,15 +630,25 @@ def prefill_rms_qkv_rope(x, attn_norm_weight, wqkv, rope_lut, pos0, n_heads, n_k
     return out
 
 
-def prefill_attention(qkv, n_heads, n_kv_heads, head_dim):
+def prefill_attention(qkv, n_heads, n_kv_heads, head_dim, k_cache=None, v_cache=None):
     """Causal GQA attention over the M rows of qkv bf16 [M, (n_heads + 2 n_kv_heads) * head_dim] (roped Q | roped K | V):
-    returns bf16 [M, n_heads * head_dim]."""
+    returns bf16 [M, n_heads * head_dim].  Rows 0 .. M - 1 of the caches [n_kv_heads, max_seq, head_dim], if given, become the K and V of qkv."""
     lib = _lib.load_library()
     _need_cuda(qkv)
     M = qkv.shape[0]
     if qkv.shape[1] != (n_heads + 2 * n_kv_heads) * head_dim:
         raise ValueError("qkv must be [M, (n_heads + 2 n_kv_heads) * head_dim]")
     out = torch.empty((M, n_heads * head_dim), dtype=torch.bfloat16, device=qkv.device)
+    if k_cache is not None:
+        if all(c.dtype == torch.bfloat16 and c.device == qkv.device and c.dim() == 3 and (c.shape[0], c.shape[2]) == (n_kv_heads, head_dim) and c.is_contiguous()
+               and c.data_ptr() % 16 == 0 for c in (k_cache, v_cache)) and M <= k_cache.shape[1] == v_cache.shape[1]:
+            _lib.check(lib.w4a16_prefill_attention_cache_bf16(_ptr(_bits(qkv)), _ptr(k_cache), _ptr(v_cache), _ptr(out), M, k_cache.shape[1], n_heads,
+                                                              n_kv_heads, head_dim, _stream()))
+            return out
+        # caches of another type, parts of larger ones and the like
+        nq, nk = n_heads * head_dim, n_kv_heads * head_dim
+        k_cache[:, :M].copy_(qkv[:, nq:nq + nk].reshape(M, n_kv_heads, head_dim).transpose(0, 1))
+        v_cache[:, :M].copy_(qkv[:, nq + nk:].reshape(M, n_kv_heads, head_dim).transpose(0, 1))
     _lib.check(lib.w4a16_prefill_attention_bf16(_ptr(_bits(qkv)), _ptr(out), M, n_heads, n_kv_heads, head_dim, _stream()))
     return out
 

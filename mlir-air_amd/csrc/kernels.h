@@ -170,8 +170,9 @@ bool prefill_block_supported(int M, int E, int H);
 size_t prefill_block_scratch_bytes(int M, int E, int H);   // sized for split-K on a 256-CU device
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream);
 // Causal GQA attention over the M rows of a prefill (prefill_attention.hip); qkv is [M, (n_heads + 2 n_kv) * head_dim].
+// With caches [n_kv, max_seq, head_dim] their rows 0 .. M - 1 become the K and V of qkv.
 hipError_t launch_prefill_attention(const uint16_t *qkv, uint16_t *attn_out, int M, int n_heads, int n_kv, int head_dim,
-                                    hipStream_t stream);
+                                    hipStream_t stream, uint16_t *k_cache = nullptr, uint16_t *v_cache = nullptr, int max_seq = 0);
 // RMSNorm rows + fused Q|K|V GEMM + RoPE on the Q and K heads (prefill_block.hip); `normed` [M, E] is scratch.
 hipError_t launch_prefill_rms_qkv_rope(const uint16_t *x, const uint16_t *norm_w, float eps, const PrefillLinear &wqkv,
                                        const uint16_t *rope_lut, int pos0, uint16_t *qkv_out, int M, int E, int n_heads,

@@ -268,6 +268,26 @@ def test_prefill_attention(ops, M, nh, nkv, hd):
     assert np.array_equal(bits(out)[0], v0)
 
 
+@pytest.mark.parametrize("M,nh,nkv,hd", [(1, 2, 1, 64), (31, 4, 1, 128), (33, 3, 3, 64), (65, 8, 2, 128), (127, 8, 1, 64), (129, 2, 2, 128), (300, 6, 2, 64), (513, 8, 1, 128)])
+def test_prefill_attention_fills_the_caches(ops, M, nh, nkv, hd):
+    """Once per KV head whatever the number of workgroups that share it, and the rows behind the prompt stay as they are; caches that are parts of
+    larger ones, of another type or not aligned go by copies."""
+    print(f"prefill attention into caches M={M} heads {nh}/{nkv} hd={hd}", flush=True)
+    qkv = torch.randn((M, (nh + 2 * nkv) * hd), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M)).bfloat16()
+    want = ops.prefill_attention(qkv, nh, nkv, hd)
+    k, v = (qkv[:, (nh + i * nkv) * hd:(nh + (i + 1) * nkv) * hd].reshape(M, nkv, hd).transpose(0, 1) for i in (0, 1))
+    new = lambda rows, width=hd, dtype=torch.bfloat16: torch.full((nkv, rows, width), 7.0, dtype=dtype, device="cuda")
+    shifted = lambda: torch.full((nkv * (M + 3) * hd + 4,), 7.0, dtype=torch.bfloat16, device="cuda")[4:].view(nkv, M + 3, hd)
+    for make in (lambda: new(M), lambda: new(M + 5), lambda: new(M + 5, hd + 8)[:, :, :hd], lambda: new(M + 5, dtype=torch.float32), shifted):
+        kc, vc = make(), make()
+        assert torch.equal(ops.prefill_attention(qkv, nh, nkv, hd, kc, vc), want)
+        assert torch.equal(kc[:, :M].bfloat16(), k) and torch.equal(vc[:, :M].bfloat16(), v)
+        assert bool((kc[:, M:] == 7).all()) and bool((vc[:, M:] == 7).all())
+    if M > 1:
+        with pytest.raises(RuntimeError):
+            ops.prefill_attention(qkv, nh, nkv, hd, new(M - 1), new(M - 1))
+
+
 def test_prefill_attention_scores_of_wide_range(ops):
     """Scores spread over hundreds of log2 units: the kernel's reference maximum, which follows the true one in steps,
     must not lose the small terms or overflow; and a second call returns the same bits."""
