@@ -3,10 +3,10 @@
 //
 // Input is the fresh, un-rotated projection vector qkv = [Q (n_heads * HD) | K (n_kv * HD) |
 // V (n_kv * HD)] of the current token.  HBM-bound on the cache: every cached K and V element is
-// read once, by the one workgroup that owns its (kv head, sequence chunk), and used for all G
-// query heads of the group.
+// read by the workgroups of its (kv head, sequence chunk), as few or as many as there is room for
+// (launch_decode_attention), and used for the G query heads that each has.
 //
-//   grid  = (nsplit sequence chunks, n_kv heads), 4 waves per workgroup
+//   grid  = (nsplit sequence chunks, n_kv heads x groups of G of their query heads), 4 waves per workgroup
 //   lanes = HD / 8 lanes share one cache position (16-byte loads), so a wave covers 64 / (HD / 8)
 //           positions per load; each lane group keeps a private online-softmax state
 //           (m, l, acc[8]) per query head and the states are merged at the end: across lane
@@ -35,6 +35,7 @@ struct AttnParams {
     float *part_ml;           // [n_heads, nsplit, 2]
     float *part_acc;          // [n_heads, nsplit, HD]
     int pos, max_seq, n_heads, n_kv, nsplit, chunk;
+    int log2_sharers;         // of the workgroups that have query heads of one KV head
     float scale;
 };
 
@@ -96,17 +97,17 @@ __device__ __forceinline__ float slots_reduce(float v) {
 // butterflies of (m, l, acc) took 120 shuffles through LDS.   32 heads of 64 over 8, 1000 positions: 7.3 -> 4.9 us; -> 4.5 a layer of
 // the model since the new token's row and the queries are no longer asked for one after the other behind the cache.  Only the chunk that appends
 // the new K and V asks for them: with all chunks, merge included, 32 heads of 64 over 8 at 4000 positions 7.5 us, 32 heads of 128 at 2000 8.6; 7.2 and 7.8.
-template <int HD, int G>
+template <int HD, int G, int UN>
 __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     constexpr int LPP = HD / 8;        // lanes per position
     constexpr int PPW = 64 / LPP;      // positions per wave and load
     constexpr int STATE = 4 + HD;      // m, l, -, -, acc[HD] per head
-    constexpr int UN = 2, STEP = UN * 4 * PPW;   // positions per lane and trip, per workgroup and trip
+    constexpr int STEP = UN * 4 * PPW;   // positions per lane and trip, per workgroup and trip
     __shared__ __attribute__((aligned(16))) float sh[4 * G * STATE];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPP, slot = lane / LPP;
-    const int split = blockIdx.x, kvh = blockIdx.y;
+    const int split = blockIdx.x, kvh = blockIdx.y >> p.log2_sharers, head0 = blockIdx.y * G;
     const int seq_len = p.pos + 1;
     const int t0 = split * p.chunk;
     const int t1 = min(seq_len, t0 + p.chunk);
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
     u32x4 qx[G], qy[G];
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-        const uint16_t *src = p.qkv + (size_t)(kvh * G + h) * HD;
+        const uint16_t *src = p.qkv + (size_t)(head0 + h) * HD;
         qx[h] = raw(src + 8 * sub);
         qy[h] = raw(src + other);
     }
@@ -211,7 +212,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
         }
     }
 
-    if (owner && threadIdx.x < LPP) {   // (behind the loop: no wait in it counts stores)
+    if (owner && blockIdx.y == kvh << p.log2_sharers && threadIdx.x < LPP) {   // (behind the loop: no wait in it counts stores)
         *reinterpret_cast<u32x4 *>(kc + (size_t)p.pos * HD) = knew;
         *reinterpret_cast<u32x4 *>(vc + (size_t)p.pos * HD) = vnew;
     }
@@ -256,7 +257,7 @@ __global__ void __launch_bounds__(256) attn_partial_kernel(const AttnParams p) {
             ls += src[1] * c;
             as += src[4 + e] * c;
         }
-        const int head = kvh * G + h;
+        const int head = head0 + h;
         if (p.nsplit == 1) {
             p.out[(size_t)head * HD + e] = float_to_bf16_bits(as / ls);
         } else {
@@ -299,12 +300,14 @@ __global__ void attn_combine_kernel(const float *part_ml, const float *part_acc,
 }
 
 template <int HD>
-hipError_t launch_g(int g, const AttnParams &p, dim3 grid, hipStream_t stream) {
+hipError_t launch_g(int g, bool longer, const AttnParams &p, dim3 grid, hipStream_t stream) {
     switch (g) {
-        case 1: hipLaunchKernelGGL((attn_partial_kernel<HD, 1>), grid, dim3(256), 0, stream, p); break;
-        case 2: hipLaunchKernelGGL((attn_partial_kernel<HD, 2>), grid, dim3(256), 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((attn_partial_kernel<HD, 4>), grid, dim3(256), 0, stream, p); break;
-        case 8: hipLaunchKernelGGL((attn_partial_kernel<HD, 8>), grid, dim3(256), 0, stream, p); break;
+        case 1:
+            if (longer) hipLaunchKernelGGL((attn_partial_kernel<HD, 1, 4>), grid, dim3(256), 0, stream, p);
+            else hipLaunchKernelGGL((attn_partial_kernel<HD, 1, 2>), grid, dim3(256), 0, stream, p);
+            break;
+        case 2: hipLaunchKernelGGL((attn_partial_kernel<HD, 2, 2>), grid, dim3(256), 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((attn_partial_kernel<HD, 4, 2>), grid, dim3(256), 0, stream, p); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -312,10 +315,18 @@ hipError_t launch_g(int g, const AttnParams &p, dim3 grid, hipStream_t stream) {
 
 }  // namespace
 
-int attention_nsplit(int seq_len) {
+// Whether one workgroup a query head takes all positions, two or four a lane and trip, and writes the result: every trip takes a chain of 0.6 us, chunks end in a
+// launch that merges them.  us of the whole attention in a graph, 32 heads of 64 over 8, in chunks (four heads of a KV head to a workgroup, then the rule
+// of launch_decode_attention) / whole: 64 positions 3.8 / 2.9 (one chunk), 128 5.9, 4.7 / 3.2, 256 5.9, 4.9 / 4.1, 384 6.0, 5.2 / 4.8,
+// 512 5.9, 5.0 / 5.5.  Heads of 128: 64 4.8 / 3.2, 128 7.0, 5.6 / 4.1, 256 7.0, 5.8 / 5.5, 300 7.2, 6.1 / 6.2.  (16 waves instead of four 1.8 more, 8 waves
+// 0.4 to 0.9.)
+static bool attention_whole(int seq_len, int head_dim) { return seq_len <= (head_dim == 64 ? 384 : 256); }
+
+int attention_nsplit(int seq_len, int head_dim) {
+    if (attention_whole(seq_len, head_dim)) return 1;
     int n = (seq_len + 63) / 64;   // >= 64 positions per chunk
     if (n > kMaxAttnSplit) n = kMaxAttnSplit;
-    return n < 1 ? 1 : n;
+    return n;
 }
 
 size_t attention_workspace_bytes(int n_heads, int head_dim) {
@@ -335,15 +346,26 @@ hipError_t launch_decode_attention(const uint16_t *qkv, const uint16_t *lut_row,
     p.max_seq = max_seq;
     p.n_heads = n_heads;
     p.n_kv = n_kv;
-    p.nsplit = attention_nsplit(pos + 1);
+    p.nsplit = attention_nsplit(pos + 1, head_dim);
     const int ppb = 4 * (64 / (head_dim / 8));   // positions per workgroup iteration
     p.chunk = (((pos + 1 + p.nsplit - 1) / p.nsplit + ppb - 1) / ppb) * ppb;
     p.scale = 1.0f / sqrtf((float)head_dim);
     p.part_ml = reinterpret_cast<float *>(workspace);
     p.part_acc = p.part_ml + (size_t)n_heads * kMaxAttnSplit * 2;
-    const dim3 grid(p.nsplit, n_kv);
-    hipError_t e = head_dim == 64 ? launch_g<64>(n_heads / n_kv, p, grid, stream)
-                                  : launch_g<128>(n_heads / n_kv, p, grid, stream);
+    // Query heads of a KV head to a workgroup: one if that makes a workgroup a CU at most, else two or four (a head costs a workgroup 0.3 to 0.9 us, but each that is not
+    // there reads the cache again).  us with 4 / 2 / 1 heads, merge included: 32 heads of 64 over 8, 512 positions (64 / 128 / 256 workgroups) 6.0 / 5.2 / 5.0, 1000 (128 / 256 / 512)
+    // 6.4 / 5.7 / 5.9, 1700 6.8 / 6.9 / 7.6; 32 of 128 over 4 at 1000 7.3 / 6.1 / 6.3, with all eight heads 9.7; 64 of 128 over 8 at 4000 12.8 / 13.1 / 14.4, with eight 13.3.
+    const int group = n_heads / n_kv;
+    int g = 1;
+    while (g < group && g < 4 && p.nsplit * n_heads / g > 256) g *= 2;
+    if (p.nsplit == 1) {
+        p.chunk = pos + 1;
+        g = 1;
+    }
+    p.log2_sharers = __builtin_ctz(group / g);
+    const dim3 grid(p.nsplit, n_heads / g);
+    const bool longer = p.nsplit == 1 && pos >= ppb * 2;   // than two positions a lane
+    hipError_t e = head_dim == 64 ? launch_g<64>(g, longer, p, grid, stream) : launch_g<128>(g, longer, p, grid, stream);
     if (e != hipSuccess || p.nsplit == 1 || !combine) return e;
     hipLaunchKernelGGL(attn_combine_kernel, dim3(n_heads), dim3(head_dim), 0, stream, p.part_ml, p.part_acc, out,
                        p.nsplit, head_dim);

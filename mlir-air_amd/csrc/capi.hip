@@ -949,7 +949,7 @@ int w4a16_decode_attn_o_gemv_ffn_bf16(const uint16_t *qkv, const uint16_t *rope_
     // With several sequence chunks and an O projection whose units lie inside one head, the projection merges the
     // chunk partials itself and the merge launch is dropped; attn_out is then not written.
     AttnPartials ap;
-    ap.nsplit = attention_nsplit(pos + 1);
+    ap.nsplit = attention_nsplit(pos + 1, head_dim);
     ap.hd = head_dim;
     attention_partials(attn_workspace, n_heads, &ap.ml, &ap.acc);
     const bool fuse = !g_stream_tune.no_attn_fuse && stream_attn_fusable(E, E, head_dim, ap.nsplit);

@@ -208,7 +208,7 @@ hipError_t launch_lm_head(const uint16_t *x, const uint16_t *norm_w, float eps, 
 // Decode attention (attention.hip).  The scratch buffer holds per-chunk softmax partials and
 // needs no initialisation.
 constexpr int kMaxAttnSplit = 32;
-int attention_nsplit(int seq_len);
+int attention_nsplit(int seq_len, int head_dim);
 size_t attention_workspace_bytes(int n_heads, int head_dim);
 hipError_t launch_decode_attention(const uint16_t *qkv, const uint16_t *lut_row, uint16_t *k_cache, uint16_t *v_cache,
                                    uint16_t *out, int pos, int max_seq, int n_heads, int n_kv, int head_dim,

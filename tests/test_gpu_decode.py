@@ -250,6 +250,17 @@ def test_generate_is_prefill_plus_greedy_decoding_and_stops_at_eos(ops):
         decode.generate(prompt, layers, embed, final_norm, embed, cfg, lut, n_tokens=60)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,positions", [
+    (4, 4, 64, [64, 127, 128, 255, 383, 384, 400]),       # two positions a lane, four, several trips, then chunks
+    (8, 4, 64, [63, 129, 382, 511]),                      # two heads read one KV head's rows, one of them appends
+    (32, 8, 64, [64, 383, 384, 512, 1100]),               # one, two and four heads to a workgroup
+    (16, 2, 128, [31, 32, 63, 64, 255, 256, 500]),        # eight heads of a KV head
+    (64, 8, 128, [256, 513, 700]),
+])
+def test_decode_attention_whole_and_in_chunks(ops, n_heads, n_kv, hd, positions):
+    test_decode_attention(ops, n_heads, n_kv, hd, positions[-1] + 3, positions)
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,H,max_seq,positions", [
     (32, 8, 128, 14336, 2048, [0, 63, 64, 500, 2047]),   # Llama-3-8B layer: fused from position 64 on (2 .. 32 chunks)
     (32, 8, 64, 8192, 2048, [100, 2047]),                # Llama-3.2-1B layer
