@@ -169,19 +169,6 @@ __device__ __forceinline__ float sigmoid_of(float z) {
     if constexpr (sizeof(T) == 2) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
     return sigmoid_f32(z);
 }
-// z sigmoid(v) with the error of z / (1 + expf(-v)) in fp32 (half a unit of 2^-24 on average, two and a half at most) over its whole range,
-// in 19 instructions instead of 27, none of them a division's.  A wide tile's store has up to 256 of them to a lane, alone on its SIMD:
-// 2048 x 11264 x 2048 with silu on 4096 columns 96 us with the division, 91 with this, 83 with the bare hardware exponential and
-// reciprocal, whose argument is rounded behind log2 e (30 units at v = -60).
-// e = e^-|v|: the product with log2 e is cut at a whole number n before it is rounded; s / (1 + e), s = 1 or for v < 0 e, by the hardware's
-// reciprocal and one step that takes back its error and that of 1 + e.  (Past 150 e is 0.)
-__device__ __forceinline__ float gated_f32(float z, float v) {
-    const float a = __builtin_amdgcn_fmed3f(fabsf(v), 0.0f, 150.0f);
-    const float n = rintf(-1.44269502f * a), x = fmaf(-1.92596303e-8f, a, fmaf(-1.44269502f, a, -n));   // log2 e in two parts
-    const float e = ldexpf(__builtin_amdgcn_exp2f(x), (int)n), s = v < 0.0f ? e : 1.0f;
-    const float d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), q = s * r;
-    return z * fmaf(fmaf(-q, e - (d - 1.0f), fmaf(-d, q, s)), r, q);
-}
 template <class T>
 __device__ __forceinline__ float silu_of(float z) {
     if constexpr (sizeof(T) == 2) return gated_f32(z, z);

@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(kThreads, 1) gemm_kernel(const GemmParams p) {
                         v[e] = pack_bf16x2(v0 + a0, v1 + a1);
                     } else {
                         // y = bf16(silu(G) * bf16(x . W)), silu(g) = g / (1 + exp(-g)) in fp32
-                        v[e] = pack_bf16x2(a0 / (1.0f + expf(-a0)) * v0, a1 / (1.0f + expf(-a1)) * v1);
+                        v[e] = pack_bf16x2(gated_f32(a0, a0) * v0, gated_f32(a1, a1) * v1);
                     }
                 }
             }
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *__restr
             out[e] = float_to_bf16_bits(bf16_bits_to_float(out[e]) + bf16_bits_to_float(aux[at + e]));
         } else if (epi == kEpiSiluGateMul) {
             const float g = bf16_bits_to_float(aux[at + e]);
-            out[e] = float_to_bf16_bits(g / (1.0f + expf(-g)) * bf16_bits_to_float(out[e]));
+            out[e] = float_to_bf16_bits(gated_f32(g, g) * bf16_bits_to_float(out[e]));
         }
     }
     *reinterpret_cast<uint2 *>(y + at) = uint2{(uint32_t)out[0] | ((uint32_t)out[1] << 16), (uint32_t)out[2] | ((uint32_t)out[3] << 16)};

@@ -560,7 +560,7 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
                     const float v0 = bf16_bits_to_float(vw & 0xFFFFu), v1 = bf16_bits_to_float(vw >> 16);
                     const float a0 = bf16_bits_to_float(aw & 0xFFFFu), a1 = bf16_bits_to_float(aw >> 16);
                     if constexpr (kEpi == kEpiAddRounded) v[e] = pack_bf16x2(v0 + a0, v1 + a1);
-                    else v[e] = pack_bf16x2(a0 / (1.0f + expf(-a0)) * v0, a1 / (1.0f + expf(-a1)) * v1);
+                    else v[e] = pack_bf16x2(gated_f32(a0, a0) * v0, gated_f32(a1, a1) * v1);
                 }
             }
             __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p.y + at));   // y is not read again here: keep x and W in L2
@@ -580,7 +580,7 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
                 for (int e = 0; e < 4; ++e) {
                     const float g0 = bf16_bits_to_float(gv[e] & 0xFFFFu), g1 = bf16_bits_to_float(gv[e] >> 16);
                     const float u0 = bf16_bits_to_float(uv[e] & 0xFFFFu), u1 = bf16_bits_to_float(uv[e] >> 16);
-                    v[e] = pack_bf16x2(g0 / (1.0f + expf(-g0)) * u0, g1 / (1.0f + expf(-g1)) * u1);
+                    v[e] = pack_bf16x2(gated_f32(g0, g0) * u0, gated_f32(g1, g1) * u1);
                 }
                 *reinterpret_cast<u32x4 *>(p.y + (size_t)(m0 + row) * Nout + ocol0 + oc) = v;
             }
