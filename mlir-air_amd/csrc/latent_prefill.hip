@@ -18,6 +18,8 @@
 //
 // Head sizes that are common have kernels of their own (EXACT: everything unrolled); any other size runs on the next
 // larger register allotment with uniform bounds.
+#include <algorithm>
+
 #include "dense.h"
 #include "dense_kernels.h"
 
@@ -396,6 +398,23 @@ PrefillArgs<T> args_of(const HeadShape &s, const HeadRows &r, const void *q, voi
     return p;
 }
 
+// Whether a workgroup takes 64 queries, 16 to a wave, instead of 128, for heads of 128 + 64 / 128 and of 128 / 128 behind long windows.  A block of 64 keys takes a wave set 2.75 us
+// with 16 queries to a wave and 3.3 with 32 (staging, scores, softmax and outputs are a chain between two barriers, a workgroup has its CU to itself): the longest item is done
+// sooner, all of them together take 1.7 times as long.  So where they are no more than 256 CUs have room for beside the longest.  us, 128 / 64 queries, 16 heads of 128 + 64 / 128:
+// 128 tokens 12.3 / 8.4, 1024 33.0 / 26.3, 1500 45.5 / 36.9, 3000 81.1 / 112.8, 500 behind 500 31.6 / 24.1, 1000 behind 3000 104.1 / 94.0, 2048 behind 2048 107.9 / 145.9; 64 heads: 300
+// 16.1 / 13.5, 1024 47.7 / 61.6.  (On the line, 16 heads and 2048 tokens, 58.9 / 54.1 alone, but 3 us more between a model's products.)
+template <class T>
+bool few_queries(const PrefillArgs<T> &p) {
+    long longest = 0, all = 0;   // blocks of 64 keys
+    for (long first = p.total - p.M; first < p.total; first += 64) {
+        const long end = std::min<long>(first + 64, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
+        const long blocks = (end + 63) / 64 - unseen;
+        longest = std::max(longest, blocks);
+        all += blocks;
+    }
+    return all * p.heads <= 256 * longest;
+}
+
 }  // namespace
 
 bool latent_prefill_supported(int dtype, const LatentShape &s) {
@@ -414,8 +433,9 @@ hipError_t launch_latent_prefill(int dtype, const LatentShape &s, const LatentRo
     }
     const PrefillArgs<bf16> p = args_of<bf16>(s, r, kv, ldkv, sink, out, ldo);
     if ((double)p.total * ldkv * sizeof(bf16) < 4e9) {
-        if (nq == 6 && nv == 8) return launch<bf16, 6, 8, 2, 64, 2, true>(p, stream);
-        if (nq == 3 && nv == 4) return launch<bf16, 3, 4, 2, 64, 2, true>(p, stream);
+        if (nq == 6 && nv == 8) return few_queries(p) ? launch<bf16, 6, 8, 1, 32, 2, true>(p, stream) : launch<bf16, 6, 8, 2, 64, 2, true>(p, stream);
+        // (two workgroups to a CU: 4 to 64 heads, 128 to 4096 tokens 1.0 to 1.4 times as fast as with 128 queries)
+        if (nq == 3 && nv == 4) return launch<bf16, 3, 4, 1, 64, 2, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false>(p, stream);
     if (nq <= 8 && nv <= 8) return launch<bf16, 8, 8, 1, 64, 1, false>(p, stream);
@@ -437,8 +457,11 @@ hipError_t launch_head_prefill(int dtype, const HeadShape &s, const HeadRows &r,
     }
     const PrefillArgs<bf16> p = args_of<bf16>(s, r, q, out, ldo);
     if ((double)s.ring * (s.dim + s.vdim) * sizeof(bf16) < 4e9) {
-        if (nq == 4 && nv == 8) return launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
-        if (nq == 2 && nv == 4) return launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream);
+        // (windows of few blocks are mostly start and end, which the smaller items share a CU for: 16 to 64 heads, 1024 to 4096 tokens, windows of 64 to 256 1.03 to 1.4 times
+        // as fast, of 384 to 700 0.99 to 1.3; heads of 64 at any window 0.96 to 1.5, 1.2 on average)
+        if (nq == 4 && nv == 8)
+            return p.window <= 768 || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
+        if (nq == 2 && nv == 4) return launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false, true>(p, stream);
     if (nq <= 8 && nv <= 8) return launch<bf16, 8, 8, 1, 64, 1, false, true>(p, stream);

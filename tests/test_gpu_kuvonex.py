@@ -382,6 +382,17 @@ def test_latent_attention(dense, dtype, sizes, form):
     close(x.run(form, 0, T), want, dtype, "whole", **tol)
 
 
+@pytest.mark.parametrize("T,cut", [(1100, 256), (1025, 65)])
+def test_latent_attention_of_many_heads_whole_and_in_portions(dense, T, cut):
+    """Items of 128 queries, which many heads with many tokens take, against those of 64 that portions take: each is within 2^-8 of the exact result (weights and
+    outputs in bf16, 2^-9 each), by the norm of a row."""
+    say("latent attention, 64 heads", T, cut)
+    x = Latents(dense, (64, 128, 64, 128, 64), T, BF16, seed=T)
+    whole = x.run("rows", 0, T).double()
+    parts = torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]).double()
+    assert bool(whole.isfinite().all()) and bool(((whole - parts).norm(dim=1) <= 2.0 ** -7 * whole.norm(dim=1)).all())
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 def test_latent_attention_forms_agree_token_by_token_and_with_the_position_on_the_device(dense, dtype):
     x = Latents(dense, (6, 64, 32, 64, 192), 140, dtype, seed=4, far=[(139, 63), (138, 64)])

@@ -215,6 +215,18 @@ def test_windowed_attention(dense, dtype, sizes, form):
         close(parts[i], want[i], dtype, i, **tol)
 
 
+@pytest.mark.parametrize("sizes", [(64, 8, 128, 128, 1000), (64, 8, 128, 128, 768), (64, 16, 64, 64, 1000)])
+@pytest.mark.parametrize("T,cut", [(1100, 256), (1025, 65)])
+def test_windowed_attention_of_many_heads_whole_and_in_portions(dense, sizes, T, cut):
+    """Items of 128 queries (long windows, many heads and tokens) and of 64 (portions): each is within 2^-8 of the exact result, by the norm of a row."""
+    say("windowed attention, many heads", sizes, T, cut)
+    x = Heads(dense, sizes, T, BF16, 1152, seed=T)
+    whole = x.run("rows", 0, T).double()
+    x.cache.fill_(float("nan"))
+    parts = torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]).double()
+    assert bool(whole.isfinite().all()) and bool(((whole - parts).norm(dim=1) <= 2.0 ** -7 * whole.norm(dim=1)).all())
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("sizes", [(4, 2, 24, 40, 37), (8, 2, 128, 128, 65), (3, 3, 64, 64, 64), (2, 1, 32, 32, 1)])
 def test_ring_of_rows_and_positions_on_the_device(dense, dtype, sizes):
