@@ -233,6 +233,8 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_gemm_kernel(const GemmKern
 // bursts stopped the products (215 -> 197 us below).
 // Two waves per SIMD with 128 x 64 each (the kernel before) read half as much again from LDS: 1536 + 512 cycles of reads and copies for
 // 2048 of products.  2048 x 8192 x 8192 236 -> 197 us = 1.39 PFLOP/s, 4096^3 122 -> 100 us = 1.38, 2048 x 16384 x 2048 with gelu 135 -> 106.
+// More tiles than CUs: a workgroup takes one after the other, and asks for a tile's first K-steps before it stores the one before (that waited for a workgroup's
+// start, its addresses and HBM: 2048 x 16384 x 2048 with gelu, two tiles each, 110.7 -> 108.2 us, 2048 x 11264 x 2048 77.2 -> 75.4, 2048 x 28672 x 4096 with silu 383.7 -> 372.0).
 constexpr int kWideThreads = 256, kWideStagesW = 3;
 constexpr size_t wide_lds(int wm, int nt) { return (2 * (size_t)(128 * wm) + kWideStagesW * (size_t)(4 / wm * 16 * nt)) * kRowBytes; }
 
@@ -241,12 +243,14 @@ __device__ __forceinline__ void mfma_in_place(floatx4 &acc, const bf16x8 &w, con
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
 }
 // COLS x 8 products, `behind(n)` issued behind the n-th of them
-template <int COLS, int W, class F>
+// (LAST: the last of them are the compiler's, so that what it puts behind the loop, a move of the accumulators say, waits for them)
+template <int COLS, bool LAST = false, int W, class F>
 __device__ __forceinline__ void quarter(floatx4 (*acc)[8], const bf16x8 (&w)[W], const bf16x8 (&a)[8], F behind) {
 #pragma unroll
     for (int n = 0; n < 8 * COLS; ++n) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma_in_place(acc[n / 8][n % 8], w[n / 8], a[n % 8]);
+        if (LAST && n >= 8 * COLS - 4) acc[n / 8][n % 8] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n / 8], a[n % 8], acc[n / 8][n % 8], 0, 0, 0);
+        else mfma_in_place(acc[n / 8][n % 8], w[n / 8], a[n % 8]);
         __builtin_amdgcn_sched_barrier(0);
         behind(n);
     }
@@ -306,8 +310,11 @@ __device__ __forceinline__ void store_rows(const GemmKernelArgs<bf16> &p, floatx
     }
 }
 
+// (fp32 rows need more LDS for their stores than is free then; with 256 accumulators and silu on some columns there are no registers for both)
+constexpr bool wide_loops(int nt, int epi) { return epi != kOutF32 && !(nt == 8 && epi == kOutElem); }
+
 template <int WM, int NT, int EPI>
-__device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *lds, const bf16 *w, int m0, int m_end, int n0, KSlice slice) {
+__device__ __forceinline__ void wide_tiles(const GemmKernelArgs<bf16> &p, char *lds, int tile, int tiles_end, int stride, KSlice slice) {
     constexpr int WN = 4 / WM, BM = 128 * WM, BN = 16 * NT * WN;
     constexpr int H0 = (NT + 1) / 2, H1 = NT - H0;        // column tiles of the two halves of a wave's columns
     static_assert(H1 >= 2, "room for a quarter's LDS reads");
@@ -323,23 +330,31 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
     // their LDS base (M0) and differ in the instruction's offset, which the hardware adds to both addresses: the source takes it back.
     // (Offsets from the wave's first row, 64 rows at most.)
     uint32_t off_a[CA], off_w[CW];
-    const int m_wave = m0 + 8 * CA * wave < m_end ? m0 + 8 * CA * wave : m_end - 1, n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
+    gptr base_a, base_w;
+    int m0, n0;
+    const int m_end = p.M;
+    auto place = [&](int tile) {   // where a tile is, and the offsets of its copies; then the copies' bases
+        const int band = tile / (4 * p.tiles_n), in_band = tile % (4 * p.tiles_n);
+        const int rows_in_band = p.tiles_m - 4 * band < 4 ? p.tiles_m - 4 * band : 4;
+        m0 = (4 * band + in_band % rows_in_band) * BM, n0 = in_band / rows_in_band * BN;
+        const int m_wave = m0 + 8 * CA * wave < m_end ? m0 + 8 * CA * wave : m_end - 1, n_wave = n0 + 8 * CW * wave < p.N ? n0 + 8 * CW * wave : p.N - 1;
 #pragma unroll
-    for (int i = 0; i < CA; ++i) {
-        const int row = 8 * (CA * wave + i) + (lane >> 3);
-        const uint32_t chunk = 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
-        const int m = m0 + row < m_end ? m0 + row : m_end - 1;
-        off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + chunk;
-    }
+        for (int i = 0; i < CA; ++i) {
+            const int row = 8 * (CA * wave + i) + (lane >> 3), m = m0 + row < m_end ? m0 + row : m_end - 1;
+            off_a[i] = (uint32_t)(m - m_wave) * (uint32_t)(p.lda * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+        }
 #pragma unroll
-    for (int i = 0; i < CW; ++i) {
-        const int row = 8 * (CW * wave + i) + (lane >> 3);
-        const int n = n0 + row < p.N ? n0 + row : p.N - 1;
-        off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
-    }
-    const size_t from = (size_t)slice.first * kRowBytes;
-    gptr base_a = scalar_ptr(reinterpret_cast<const char *>(p.a + (size_t)m_wave * p.lda) + from - 4096);
-    gptr base_w = scalar_ptr(reinterpret_cast<const char *>(w + (size_t)n_wave * p.K) + from - 4096);
+        for (int i = 0; i < CW; ++i) {
+            const int row = 8 * (CW * wave + i) + (lane >> 3), n = n0 + row < p.N ? n0 + row : p.N - 1;
+            off_w[i] = (uint32_t)(n - n_wave) * (uint32_t)(p.K * sizeof(bf16)) + 16 * ((lane & 7) ^ (row & 7)) + 4096 - 1024 * (i & 3);
+        }
+        return int2{m_wave, n_wave};
+    };
+    auto begin = [&](int2 at) {
+        const size_t from = (size_t)slice.first * kRowBytes;
+        base_a = scalar_ptr(reinterpret_cast<const char *>(p.a + (size_t)at.x * p.lda) + from - 4096);
+        base_w = scalar_ptr(reinterpret_cast<const char *>(p.w + (size_t)at.y * p.K) + from - 4096);
+    };
     auto copy = [&](gptr from, int at, int i) {
         const auto *src = (const __attribute__((address_space(1))) void *)from;
         auto *dst = (__attribute__((address_space(3))) void *)(lds + at + 1024 * (i & ~3));
@@ -354,121 +369,137 @@ __device__ __forceinline__ void wide_tile(const GemmKernelArgs<bf16> &p, char *l
     auto copy_w = [&](int side, int i) { copy(base_w + off_w[i], 2 * kSideA + side + 1024 * CW * wave, i); };
 
     const int steps = slice.steps;
-    // operand addresses of the two halves (32 k) of a K-step; tile i is the instruction's offset
-    uint32_t at_a[2], at_w[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        const uint32_t o = ql * kRowBytes + 16 * ((4 * ks + g) ^ (ql & 7));
-        at_a[ks] = o + wm * 128 * kRowBytes;
-        at_w[ks] = o + 2 * kSideA + wn * 16 * NT * kRowBytes;
-    }
     auto read = [&](uint32_t at, int i) { return *reinterpret_cast<const bf16x8 *>(lds + at + i * 16 * kRowBytes); };
-
-    floatx4 acc[NT][8];
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // A of K-steps 0 and 1, W of 0, 1 and 2 are on their way when the loop begins (past the end: the last K-step's once more, into
     // a buffer that nobody reads)
-    int next_a = 0, next_w = 0;   // K-steps that the sources stand at
+    int next_a, next_w;   // K-steps that the sources stand at
     auto step_a = [&]() { return next_a + 1 < steps ? (++next_a, kRowBytes) : 0; };
     auto step_w = [&]() { return next_w + 1 < steps ? (++next_w, kRowBytes) : 0; };
+    auto ask = [&] {
+        next_a = next_w = 0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+        for (int s = 0; s < 2; ++s) {
 #pragma unroll
-        for (int i = 0; i < CW; ++i) copy_w(s * kSideW, i);
-        base_w += step_w();
+            for (int i = 0; i < CW; ++i) copy_w(s * kSideW, i);
+            base_w += step_w();
 #pragma unroll
-        for (int i = 0; i < (s == 0 ? CA : CA0); ++i) copy_a(s * kSideA, i);
-        if (s == 0) base_a += step_a();
-    }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CW + CA0) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+            for (int i = 0; i < (s == 0 ? CA : CA0); ++i) copy_a(s * kSideA, i);
+            if (s == 0) base_a += step_a();
+        }
+    };
+    begin(place(tile));
+    ask();
+    for (;;) {
+        floatx4 acc[NT][8];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    bf16x8 a0[8], a1[8], w0[H0], w1[H0];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a0[i] = read(at_a[0], i);
-#pragma unroll
-    for (int j = 0; j < H0; ++j) w0[j] = read(at_w[0], j);
-
-    int side_a = 0, side_w = 0, fill_w = 2 * kSideW;   // of the K-step that is multiplied; of the one that W is copied for
-#pragma unroll 1
-    for (int kt = 0; kt < steps; ++kt) {
-        // (opaque in this block: the offsets' zero extension folds into the copies only if it is not taken out of the loop)
-#pragma unroll
-        for (int i = 0; i < CA; ++i) asm volatile("" : "+v"(off_a[i]));
-#pragma unroll
-        for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
-        // first columns, first half of the K-step; the other half of A's copies for the next K-step
-        quarter<H0>(acc, w0, a0, [&](int n) {
-            if (const int r = read_behind(n, 8 * H0, H0 + 8); r >= 0) {
-                if (r < H0) w1[r] = read(at_w[1], r);
-                else a1[r - H0] = read(at_a[1], r - H0);
-            }
-            if (const int i = copy_behind(n, 8 * H0, CA - CA0); i >= 0) copy_a(side_a ^ kSideA, CA0 + i);
-        });
-        base_a += step_a();
-        // second half; W two K-steps on
-        quarter<H0>(acc, w1, a1, [&](int n) {
-            if (const int r = read_behind(n, 8 * H0, H1); r >= 0) w0[r] = read(at_w[0], H0 + r);
-            if (const int i = copy_behind(n, 8 * H0, CW0); i >= 0) copy_w(fill_w, i);
-        });
-        // the other columns, first half
-        quarter<H1>(acc + H0, w0, a0, [&](int n) {
-            if (const int r = read_behind(n, 8 * H1, H1); r >= 0) w1[r] = read(at_w[1], H0 + r);
-            if (const int i = copy_behind(n, 8 * H1, CW - CW0); i >= 0) copy_w(fill_w, CW0 + i);
-        });
-        base_w += step_w();
-        __builtin_amdgcn_sched_barrier(0);
-        // everything of the next K-step has landed (W of the one after it need not have), everybody has read all of this one
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(CW) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const int filled = side_a;
-        side_a ^= kSideA;
-        const int ahead = side_w == 2 * kSideW ? -2 * kSideW : kSideW;
-        side_w += ahead;
-        fill_w = fill_w == 2 * kSideW ? 0 : fill_w + kSideW;
+        // operand addresses of the two halves (32 k) of a K-step; tile i is the instruction's offset
+        uint32_t at_a[2], at_w[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            at_a[ks] ^= kSideA;
-            at_w[ks] += ahead;
+            const uint32_t o = ql * kRowBytes + 16 * ((4 * ks + g) ^ (ql & 7));
+            at_a[ks] = o + wm * 128 * kRowBytes;
+            at_w[ks] = o + 2 * kSideA + wn * 16 * NT * kRowBytes;
         }
-        // second half; A two K-steps on
-        quarter<H1>(acc + H0, w1, a1, [&](int n) {
-            if (const int r = read_behind(n, 8 * H1, H0 + 8); r >= 0) {
-                if (r < H0) w0[r] = read(at_w[0], r);
-                else a0[r - H0] = read(at_a[0], r - H0);
-            }
-            if (const int i = copy_behind(n, 8 * H1, CA0); i >= 0) copy_a(filled, i);
-        });
-    }
-    // no copy, of any wave, is on its way to LDS any more; the products have left the matrix pipe
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-        asm volatile("" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CW + CA0) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
 
-    store_rows<NT, 8, EPI, false, false>(p, acc, lds + wave * kWideStore, m0 + wm * 128, m_end, n0 + wn * 16 * NT);
+        // (the zeros have been written when the first product, of which the compiler does not know, adds to them)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            asm volatile("s_nop 1" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
+        bf16x8 a0[8], a1[8], w0[H0], w1[H0];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a0[i] = read(at_a[0], i);
+#pragma unroll
+        for (int j = 0; j < H0; ++j) w0[j] = read(at_w[0], j);
+
+        int side_a = 0, side_w = 0, fill_w = 2 * kSideW;   // of the K-step that is multiplied; of the one that W is copied for
+#pragma unroll 1
+        for (int kt = 0; kt < steps; ++kt) {
+            // (opaque in this block: the offsets' zero extension folds into the copies only if it is not taken out of the loop)
+#pragma unroll
+            for (int i = 0; i < CA; ++i) asm volatile("" : "+v"(off_a[i]));
+#pragma unroll
+            for (int i = 0; i < CW; ++i) asm volatile("" : "+v"(off_w[i]));
+            // first columns, first half of the K-step; the other half of A's copies for the next K-step
+            quarter<H0>(acc, w0, a0, [&](int n) {
+                if (const int r = read_behind(n, 8 * H0, H0 + 8); r >= 0) {
+                    if (r < H0) w1[r] = read(at_w[1], r);
+                    else a1[r - H0] = read(at_a[1], r - H0);
+                }
+                if (const int i = copy_behind(n, 8 * H0, CA - CA0); i >= 0) copy_a(side_a ^ kSideA, CA0 + i);
+            });
+            base_a += step_a();
+            // second half; W two K-steps on
+            quarter<H0>(acc, w1, a1, [&](int n) {
+                if (const int r = read_behind(n, 8 * H0, H1); r >= 0) w0[r] = read(at_w[0], H0 + r);
+                if (const int i = copy_behind(n, 8 * H0, CW0); i >= 0) copy_w(fill_w, i);
+            });
+            // the other columns, first half
+            quarter<H1>(acc + H0, w0, a0, [&](int n) {
+                if (const int r = read_behind(n, 8 * H1, H1); r >= 0) w1[r] = read(at_w[1], H0 + r);
+                if (const int i = copy_behind(n, 8 * H1, CW - CW0); i >= 0) copy_w(fill_w, CW0 + i);
+            });
+            base_w += step_w();
+            __builtin_amdgcn_sched_barrier(0);
+            // everything of the next K-step has landed (W of the one after it need not have), everybody has read all of this one
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(CW) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int filled = side_a;
+            side_a ^= kSideA;
+            const int ahead = side_w == 2 * kSideW ? -2 * kSideW : kSideW;
+            side_w += ahead;
+            fill_w = fill_w == 2 * kSideW ? 0 : fill_w + kSideW;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                at_a[ks] ^= kSideA;
+                at_w[ks] += ahead;
+            }
+            // second half; A two K-steps on
+            quarter<H1, wide_loops(NT, EPI)>(acc + H0, w1, a1, [&](int n) {
+                if (const int r = read_behind(n, 8 * H1, H0 + 8); r >= 0) {
+                    if (r < H0) w0[r] = read(at_w[0], r);
+                    else a0[r - H0] = read(at_a[0], r - H0);
+                }
+                if (const int i = copy_behind(n, 8 * H1, CA0); i >= 0) copy_a(filled, i);
+            });
+        }
+        // no copy, of any wave, is on its way to LDS any more; the products have left the matrix pipe
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            asm volatile("" : "+a"(acc[j][0]), "+a"(acc[j][1]), "+a"(acc[j][2]), "+a"(acc[j][3]), "+a"(acc[j][4]), "+a"(acc[j][5]), "+a"(acc[j][6]), "+a"(acc[j][7]));
+        const int m_store = m0 + wm * 128, n_store = n0 + wn * 16 * NT;
+        tile += stride;
+        const bool more = wide_loops(NT, EPI) && tile < tiles_end;
+        if (more) {
+            begin(place(tile));
+            ask();
+        }
+        // (the third buffer of W, which nothing is on its way to; fp32 rows, of one tile only, need more)
+        store_rows<NT, 8, EPI, false, false>(p, acc, lds + (wide_loops(NT, EPI) ? 2 * kSideA + 2 * kSideW + wave * (kWideStore / 2) : wave * kWideStore), m_store, m_end, n_store);
+        if (!more) return;
+        // the offsets once more, so that they need no registers beside the rows that are stored
+        asm volatile("" : "+s"(tile));
+        place(tile);
+    }
 }
 
 template <int WM, int NT, int EPI>
 __global__ void __launch_bounds__(kWideThreads, 1) dense_gemm_wide_kernel(const GemmKernelArgs<bf16> p) {
     extern __shared__ __attribute__((aligned(16))) char gemm_lds[];
-    constexpr int BM = 128 * WM, BN = 16 * NT * (4 / WM);
-    const int tiles_m = p.tiles_m;
-    const int total = tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= total) return;
-    const int band = tile / (4 * p.tiles_n), in_band = tile % (4 * p.tiles_n);
-    const int rows_in_band = tiles_m - 4 * band < 4 ? tiles_m - 4 * band : 4;
-    const int tm = 4 * band + in_band % rows_in_band, tn = in_band / rows_in_band;
-    wide_tile<WM, NT, EPI>(p, gemm_lds, p.w, tm * BM, p.M, tn * BN, k_slice(p.K / 64));
+    const int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8, total = p.tiles_m * p.tiles_n;
+    const int first = (blockIdx.x & 7) * per_xcd, end = first + per_xcd < total ? first + per_xcd : total, tile = first + (blockIdx.x >> 3);
+    if (tile < end) wide_tiles<WM, NT, EPI>(p, gemm_lds, tile, end, gridDim.x / 8, k_slice(p.K / 64));
 }
 
 
@@ -731,13 +762,13 @@ GemmKernelArgs<T> kernel_args(const GemmArgs &g, int bm, int bn) {
 }
 
 template <class P>
-hipError_t run_tiles(void (*kernel)(P), const P &p, int threads, size_t lds, int slices, hipStream_t stream) {
+hipError_t run_tiles(void (*kernel)(P), const P &p, int threads, size_t lds, int slices, hipStream_t stream, int most = 1 << 30) {
     if (lds > 48 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    const int total = p.tiles_m * p.tiles_n;
-    hipLaunchKernelGGL(kernel, dim3((total + 7) / 8 * 8, slices), dim3(threads), lds, stream, p);
+    const int total = (p.tiles_m * p.tiles_n + 7) / 8 * 8;
+    hipLaunchKernelGGL(kernel, dim3(total < most ? total : most, slices), dim3(threads), lds, stream, p);
     return hipGetLastError();
 }
 
@@ -761,7 +792,7 @@ hipError_t launch_tile(const GemmArgs &g, int slices, hipStream_t stream) {
 template <int WM, int NT>
 hipError_t launch_wide(const GemmArgs &g, int slices, hipStream_t stream) {
     const GemmKernelArgs<bf16> p = kernel_args<bf16>(g, 128 * WM, 16 * NT * (4 / WM));
-    auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, wide_lds(WM, NT), slices, stream); };
+    auto run = [&](auto kernel) { return run_tiles<GemmKernelArgs<bf16>>(kernel, p, kWideThreads, wide_lds(WM, NT), slices, stream, wide_loops(NT, g.epilogue) ? 256 : 1 << 30); };
     switch (g.epilogue) {
         case kOutF32: return run(&dense_gemm_wide_kernel<WM, NT, kOutF32>);
         case kOutSwiglu: return run(&dense_gemm_wide_kernel<WM, NT, kOutSwiglu>);

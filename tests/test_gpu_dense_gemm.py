@@ -85,6 +85,14 @@ def test_every_tile(dense, tile, M, N, K):
     products(dense, M, N, K, {1, min(3, K // 64)}, -tile)
 
 
+@pytest.mark.parametrize("tile", [4, 5, 6])
+@pytest.mark.parametrize("M,N,K", [(2100, 8208, 64), (1300, 12304, 320), (513, 33296, 128)])
+def test_wide_tiles_one_after_the_other(dense, tile, M, N, K):
+    """More tiles than CUs, whole ones and those at the edges in turn, one to five K-steps each."""
+    print("wide tiles", tile, M, N, K, flush=True)
+    products(dense, M, N, K, {1, 2} if K > 64 else {1}, -tile)
+
+
 @pytest.mark.parametrize("M,N,K,slices", [(64, 4096, 64, 1), (260, 2048, 128, 2), (1040, 512, 64, 1)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_silu_behind_a_product_is_an_fp32_one(dense, gated, M, N, K, slices):
