@@ -127,23 +127,23 @@ __device__ __forceinline__ void head_merge_step(const HeadShape &s, int M, const
 }
 
 constexpr int kConvTokens = 4;   // tokens per thread
+constexpr int kConvTaps = 4;     // taps whose operands are in flight together
 
 // The convolution of one token at eight channels: up to four taps at a time.
 template <class T>
 __device__ __forceinline__ void one_token_conv(const ConvArgs &c, const T *proj, T *history, int ch, int C, int pos0, float (&acc)[8]) {
-    constexpr int kTaps = 4;
     const Vec8<T> mine = load8(proj + ch);
-    for (int j0 = 0; j0 < c.taps; j0 += kTaps) {
-        Vec8<float> w[kTaps];
-        Vec8<T> x[kTaps];
+    for (int j0 = 0; j0 < c.taps; j0 += kConvTaps) {
+        Vec8<float> w[kConvTaps];
+        Vec8<T> x[kConvTaps];
 #pragma unroll
-        for (int t = 0; t < kTaps; ++t) {
+        for (int t = 0; t < kConvTaps; ++t) {
             const int j = j0 + t < c.taps ? j0 + t : c.taps - 1, at = pos0 + j - (c.taps - 1);   // the tap's position; the last tap's is this token's
             w[t] = load8(c.w + (size_t)j * C + ch);
             x[t] = load8(history + (size_t)(at >= 0 ? at % c.taps : 0) * C + ch);
         }
 #pragma unroll
-        for (int t = 0; t < kTaps; ++t) {
+        for (int t = 0; t < kConvTaps; ++t) {
             const int j = j0 + t;
             if (j >= c.taps || pos0 + j - (c.taps - 1) < 0) continue;
             float f[8], v[8];
@@ -158,6 +158,10 @@ __device__ __forceinline__ void one_token_conv(const ConvArgs &c, const T *proj,
 
 // Vectors (q and k heads, then v heads) by groups of `lanes` lanes, eight channels per lane at a time; tokens m0 .. m0 + kConvTokens - 1.
 // Rows in front of the portion come from the history, a ring of `taps` rows by position.
+// Latency and the reads bind it: the rows that four tokens meet at four taps (seven) and the four rows of filters are asked for together,
+// and a row is read once for four tokens.  With a wait after each tap, and a row at a time at a portion's two ends, 16 q, k and v heads of
+// 128 took, with the history's launch, 9.9 us at 8 tokens, 10.6 at 300, 19.6 at 2048 and 37.4 at 4096; so 7.0, 7.6, 17.3 and 29.6.
+// Eight tokens a thread: 9.8, 10.4, 17.3 and 30.0 (half as many workgroups, each with more behind it).
 template <class T>
 __device__ __forceinline__ void short_conv_step(const ConvArgs &c, const T *proj, T *history, T *act, int lanes, int block, int m0) {
     const int lane = threadIdx.x % lanes, unit = block * (kStepThreads / lanes) + threadIdx.x / lanes;
@@ -166,8 +170,7 @@ __device__ __forceinline__ void short_conv_step(const ConvArgs &c, const T *proj
     const bool is_v = unit >= 2 * c.k_heads;
     const int c0 = is_v ? 2 * c.k_heads * c.dim + (unit - 2 * c.k_heads) * c.vdim : unit * c.dim, n = is_v ? c.vdim : c.dim;
     const int pos0 = c.pos_dev ? c.pos_dev[0] : c.pos;
-    const bool inside = m0 >= c.taps - 1 && m0 + kConvTokens <= c.M;   // every row is one of the portion
-    float ss[kConvTokens] = {0.f, 0.f, 0.f, 0.f};
+    float ss[kConvTokens] = {};
     for (int i = 8 * lane; i < n; i += 8 * lanes) {
         const int ch = c0 + i;
         float acc[kConvTokens][8];
@@ -177,34 +180,32 @@ __device__ __forceinline__ void short_conv_step(const ConvArgs &c, const T *proj
             for (int e = 0; e < 8; ++e) acc[t][e] = 0.f;
         if (c.M == 1) {
             one_token_conv<T>(c, proj, history, ch, C, pos0, acc[0]);
-        } else if (inside) {
-            for (int j = 0; j < c.taps; ++j) {
-                const T *row = proj + (size_t)(m0 + j - (c.taps - 1)) * c.ld + ch;
-                float w[8];
-                unpack8(load8(c.w + (size_t)j * C + ch), w);
-                Vec8<T> v[kConvTokens];
-#pragma unroll
-                for (int t = 0; t < kConvTokens; ++t) v[t] = load8(row + (size_t)t * c.ld);
-#pragma unroll
-                for (int t = 0; t < kConvTokens; ++t) {
-                    float x[8];
-                    unpack8(v[t], x);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[t][e] = fmaf(w[e], x[e], acc[t][e]);
-                }
-            }
         } else {
-            for (int j = 0; j < c.taps; ++j) {
-                float w[8];
-                unpack8(load8(c.w + (size_t)j * C + ch), w);
+            for (int j0 = 0; j0 < c.taps; j0 += kConvTaps) {
+                constexpr int kRows = kConvTokens + kConvTaps - 1;
+                const int r0 = m0 + j0 - (c.taps - 1);                   // the row that the first token meets at tap j0
+                Vec8<float> w[kConvTaps];
+                Vec8<T> v[kRows];
 #pragma unroll
-                for (int t = 0; t < kConvTokens; ++t) {
-                    const int m = m0 + t, r = m + j - (c.taps - 1);       // row of the portion that meets this tap
-                    if (m >= c.M || pos0 + r < 0) continue;
+                for (int t = 0; t < kConvTaps; ++t) w[t] = load8(c.w + (size_t)(j0 + t < c.taps ? j0 + t : c.taps - 1) * C + ch);
+#pragma unroll
+                for (int k = 0; k < kRows; ++k) {
+                    const int r = r0 + k < c.M ? r0 + k : c.M - 1, at = pos0 + r;
+                    v[k] = load8((r >= 0 ? proj + (size_t)r * c.ld : history + (size_t)(at >= 0 ? at % c.taps : 0) * C) + ch);
+                }
+#pragma unroll
+                for (int k = 0; k < kRows; ++k) {
                     float x[8];
-                    unpack8(load8(r >= 0 ? proj + (size_t)r * c.ld + ch : history + (size_t)((pos0 + r) % c.taps) * C + ch), x);
+                    unpack8(v[k], x);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[t][e] = fmaf(w[e], x[e], acc[t][e]);
+                    for (int t = 0; t < kConvTaps; ++t) {                // row k meets tap j0 + t at token k - t
+                        if (k - t < 0 || k - t >= kConvTokens) continue;
+                        if (j0 + t >= c.taps || pos0 + r0 + k < 0) continue;
+                        float f[8];
+                        unpack8(w[t], f);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) acc[k - t][e] = fmaf(f[e], x[e], acc[k - t][e]);
+                    }
                 }
             }
         }

@@ -300,6 +300,12 @@ def test_short_convolution(dense, dtype, heads, k_heads, dim, vdim, taps):
             at += h * padded(n)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("taps", [2, 5, 8, 9])
+def test_short_convolution_at_the_remainders_of_four_taps(dense, dtype, taps):
+    test_short_convolution(dense, dtype, 3, 1, 72, 40, taps)
+
+
 # ---- recurrences -----------------------------------------------------------------------------------------------------------------
 class Recurrence:
     """Random inputs of one recurrence.  `far`: (query, key) pairs with a channel of their own, so that what the key wrote is
