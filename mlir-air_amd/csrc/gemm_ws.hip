@@ -490,6 +490,38 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int c = 0; c < NCB; ++c) asm volatile("" : "+a"(acc[r][c]));   // and no read of them moves above that wait
+    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, in the same order, operand by operand from memory.  (Nothing of it stands in the
+    // loop; few registers, so that those of the loop decide.)
+    if constexpr (!Q4) {
+        bool over = false;
+#pragma unroll
+        for (int c = 0; c < NCB; ++c) over |= awq_overflowed(acc[0][c][0], acc[RT - 1][c][0]);
+        if (__ballot(over)) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int c = 0; c < NCB; ++c) acc[r][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = 4 * g_lo; k < 4 * g_hi; ++k) {   // K-steps
+                const WOffsets at = w_offsets(k >> 2);
+#pragma unroll
+                for (int c = 0; c < NCB; ++c) {
+                    typedef const __attribute__((address_space(1))) uint32_t *Word;
+                    float s, low;
+                    decode_md(*reinterpret_cast<Word>(tile_base[c] + at.md), s, low);
+                    const bf16x8 b = dequant_operand(*reinterpret_cast<Word>(tile_base[c] + at.cell + 4 * (k & 3)), s, low);
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) {
+                        int row = m0 + 16 * r + ln;
+                        asm volatile("" : "+v"(row));   // (no addresses kept)
+                        const bf16x8 x = *reinterpret_cast<const bf16x8 *>(p.x + (size_t)min(row, M - 1) * K + 32 * k + 8 * lg);
+                        acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b, acc[r][c], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+    }
     __syncthreads();                                      // every wave is done reading the last x tile
     if constexpr (PARTS) {   // whole rows of the tile's columns, 128 rows at a time
         constexpr int LDF = TN + 4;

@@ -307,6 +307,38 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         half ^= 1;
     }
 
+    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, in the same order, operand by operand from memory.
+    if constexpr (MODE == kSmAwqRounded) {
+        static_assert(KW == 1, "a wave has all of the slice");
+        bool over = false;
+#pragma unroll
+        for (int c = 0; c < NT; ++c) over |= awq_overflowed(Y[0][c][0], Y[RT - 1][c][0]);
+        if (__ballot(over)) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int c = 0; c < NT; ++c) Y[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = 4 * g_lo; k < 4 * g_hi; ++k) {   // K-steps
+                const int g = k >> 2;
+                const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
+                const uint32_t cell = lane16 + blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes + 4 * (k & 3), word = 16 * ln + blk + 64 * (g & 12) + 4 * (g & 3);
+#pragma unroll
+                for (int c = 0; c < NT; ++c) {
+                    typedef const __attribute__((address_space(1))) uint32_t *Word;
+                    float s, low;
+                    decode_md(*reinterpret_cast<Word>(tb[c] + word), s, low);
+                    const bf16x8 b = dequant_operand(*reinterpret_cast<Word>(tb[c] + cell), s, low);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) {
+                        const bf16x8 x = *reinterpret_cast<const bf16x8 *>(p.x + (size_t)(m0 + min(16 * rt + ln, rows - 1)) * p.K + 32 * k + 8 * lg);
+                        Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b, Y[rt][c], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+
     // The parts of K meet, then the sums leave through LDS, so that a store is whole rows of the workgroup's columns.  (No copy of
     // any wave may still be on its way into it.)
     constexpr int LDP = CW + 4;

@@ -5,7 +5,7 @@
 
 namespace w4a16 {
 
-// Q4NX order: eight weights of one dword (rows 8 lg .. 8 lg + 7 of the lane's column) as the four registers of a B operand, bf16(s q + min')
+// Eight weights of one dword (rows 8 lg .. 8 lg + 7 of the lane's column) as the four registers of a B operand, bf16(sf q + c0): any scale of either order
 __device__ __forceinline__ bf16x8 dequant_operand(uint32_t w, float sf, float c0) {
     uint32_t e = w & 0x0F0F0F0Fu;          // nibbles 0, 2, 4, 6 -> rows 0, 4, 1, 5
     uint32_t o = (w >> 4) & 0x0F0F0F0Fu;   // nibbles 1, 3, 5, 7 -> rows 2, 6, 3, 7
@@ -22,8 +22,10 @@ __device__ __forceinline__ bf16x8 dequant_operand(uint32_t w, float sf, float c0
 
 // The same eight weights of the AWQ order in 17 vector instructions instead of 23.  A nibble behind the exponent of the half-precision 1024 is 1024 + q
 // (bits 0 .. 3 of a half) or 1024 + 16 q (bits 4 .. 7), two weights a mask, and a multiply-add that takes a half as it is does conversion and scale in
-// one: (1024 + q) s - (1024 + z) s = (q - z) s and (1024 + 16 q) s / 16 - (64 + z) s, exact in fp32 (11 x 8 bits; scales below 2^117), so
-// the rounded weights are the same bits.  300 rows of 4096 x 11008 48.2 -> 44.5 us, 512 of 4096 x 4096 30.4 -> 29.1, tiled 2048 of 4096 x 14336
+// one: (1024 + q) s - (1024 + z) s = (q - z) s and (1024 + 16 q) s / 16 - (64 + z) s, exact in fp32 (11 x 8 bits), so
+// the rounded weights are the same bits.  From scales of 2^117 on the offsets may be infinite, and then so is, or no number at all, every weight of the group and
+// every result of its column: the kernels look for that behind their loop (awq_overflowed) and take such columns again with the form above
+// (without such scales 300 rows of 4096 x 11008 and 2048 of 4096 x 14336 take as long as without the look).  300 rows of 4096 x 11008 48.2 -> 44.5 us, 512 of 4096 x 4096 30.4 -> 29.1, tiled 2048 of 4096 x 14336
 // 178.5 -> 176.6.  (Q4NX keeps the 23: min' - 1024 s is not exact for a minimum that is small against the scale.)
 struct AwqScale {
     float s, c, s16, c16;   // s, -(1024 + z) s, s / 16, -(64 + z) s
@@ -45,6 +47,16 @@ __device__ __forceinline__ bf16x8 dequant_operand_awq(uint32_t w, const AwqScale
                      pair((w8 & high) | magic, d.s16, d.c16)};
     return __builtin_bit_cast(bf16x8, b);
 }
+
+// AWQ order: scale word -> scale s and -z s (exact: (128 + z) - 128 and an 8 x 8 bit product), for dequant_operand
+__device__ __forceinline__ void decode_md(uint32_t md, float &sf, float &c0) {
+    sf = __builtin_bit_cast(float, md << 16);
+    const float nz = __builtin_bit_cast(float, md & 0xFFFF0000u);   // -(128 + z)
+    c0 = (nz + 128.0f) * sf;
+}
+// Whether a column of the wave may have had a weight of AwqScale that is not finite, by two results of it, of different rows of x (one row may itself hold
+// an infinity).
+__device__ __forceinline__ bool awq_overflowed(float a, float b) { return !__builtin_isfinite(a) && !__builtin_isfinite(b); }
 
 // Q4NX order: scale word -> scale s and min' (two bf16 halves)
 __device__ __forceinline__ void decode_md_q4(uint32_t md, float &sf, float &c0) {

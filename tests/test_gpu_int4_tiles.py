@@ -222,3 +222,58 @@ def test_every_weight_of_rounded_tiles(nt, rt):
     finally:
         for key in keys:
             ops.tune(key, 0)
+
+
+@pytest.mark.parametrize("M,K,N,forms", [(257, 512, 384, [(1, nt, rt, 0) for nt, rt in ((1, 2), (1, 7), (2, 4), (2, 6), (3, 3), (3, 5))] + [(2, 0, 0, tile) for tile in (1, 2, 3, 4)]),
+                                         (1500, 14336, 4096, [(2, 0, 0, 0)])])   # (the last one in slices of K)
+def test_scales_up_to_the_largest(M, K, N, forms):
+    """Scales of 2^118 to 2^124, whose offsets are past fp32, in half of the columns: a power of two on scales and off x changes no bit of what is
+    added up, here or in the other columns.  The kernels of fewer rows take any scale as it is."""
+    from air_hip import ops
+    print("largest scales", M, K, N, flush=True)
+    rng = np.random.default_rng(M)
+    q, z = rng.integers(0, 16, (K, N), dtype=np.uint8), rng.integers(0, 16, (K // 128, N), dtype=np.uint8)
+    s = np.exp2(rng.uniform(8, 14, (K // 128, N))).astype(np.float32) * rng.choice([-1, 1], (K // 128, N))
+    x = (rng.uniform(0.125, 4, (M, K)) * rng.choice([-1, 1], (M, K))).astype(np.float32)
+    exact = lambda b, by: f32_to_bf16_bits(bf16_bits_to_f32(b) * by)
+    s, x = (f32_to_bf16_bits(np.ascontiguousarray(t.astype(np.float32))) for t in (s, x))
+    large = np.broadcast_to(np.arange(N) // 16 % 2 == 0, (K // 128, N))
+    qz = dev(oawq.pack_awq_int32(q)), dev(oawq.pack_awq_int32(z))
+    w, w_large = (ops.repack_stream(*qz, dev(t)) for t in (s, exact(s, np.where(large, 2.0**110, 1.0).astype(np.float32))))
+    small_x = exact(x, np.float32(2.0**-110))
+    keys = ("prefill_wsm", "gemm_wsm_nt", "gemm_wsm_rt", "prefill_tile")
+    try:
+        for values in forms:
+            for key, value in zip(keys, values):
+                ops.tune(key, value)
+            want = bits(ops.w4a16_gemm_stream(dev(x), w))
+            got = bits(ops.w4a16_gemm_stream(dev(small_x), w_large))
+            assert np.array_equal(got, np.where(large[0], want, exact(want, np.float32(2.0**-110)))), values
+    finally:
+        for key in keys:
+            ops.tune(key, 0)
+
+
+@pytest.mark.parametrize("form", [(1, 1, 2, 0), (1, 3, 4, 0), (2, 0, 0, 1), (2, 0, 0, 3)])
+def test_every_weight_under_the_largest_scales(form):
+    """One-hot rows of x, small and largest scales in one column: the dequantised weights bit for bit."""
+    from air_hip import ops
+    print("every weight, largest scales", form, flush=True)
+    K, N = 256, 256
+    k, n = np.arange(K)[:, None], np.arange(N)[None, :]
+    q = ((k + n // 16) % 16).astype(np.uint8)
+    z = np.broadcast_to((n % 16).astype(np.uint8), (K // 128, N))
+    values = np.array([1.0, 2.0**118, 2.0**-120, -1.99 * 2.0**117, 2.0**122, 2.0**117, -(2.0**124)], np.float32)
+    s = f32_to_bf16_bits(np.ascontiguousarray(values[(n // 16 + 3 * np.arange(K // 128)[:, None]) % len(values)]))
+    tri = dev(oawq.pack_awq_int32(q)), dev(oawq.pack_awq_int32(np.ascontiguousarray(z))), dev(s)
+    x, w = torch.eye(K, dtype=torch.bfloat16, device="cuda"), ops.repack_stream(*tri)
+    want = bits(ops.awq_dequant(*tri))
+    keys = ("prefill_wsm", "gemm_wsm_nt", "gemm_wsm_rt", "prefill_tile")
+    try:
+        for key, value in zip(keys, form):
+            ops.tune(key, value)
+        got = bits(ops.w4a16_gemm_stream(x, w))
+        assert np.array_equal(np.where(got == 0x8000, 0, got), np.where(want == 0x8000, 0, want))   # (a sum's zero has no sign)
+    finally:
+        for key in keys:
+            ops.tune(key, 0)
