@@ -308,6 +308,7 @@ hipError_t launch_g(int g, bool longer, const AttnParams &p, dim3 grid, hipStrea
             break;
         case 2: hipLaunchKernelGGL((attn_partial_kernel<HD, 2, 2>), grid, dim3(256), 0, stream, p); break;
         case 4: hipLaunchKernelGGL((attn_partial_kernel<HD, 4, 2>), grid, dim3(256), 0, stream, p); break;
+        case 8: hipLaunchKernelGGL((attn_partial_kernel<HD, 8, 2>), grid, dim3(256), 0, stream, p); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -355,9 +356,13 @@ hipError_t launch_decode_attention(const uint16_t *qkv, const uint16_t *lut_row,
     // Query heads of a KV head to a workgroup: one if that makes a workgroup a CU at most, else two or four (a head costs a workgroup 0.3 to 0.9 us, but each that is not
     // there reads the cache again).  us with 4 / 2 / 1 heads, merge included: 32 heads of 64 over 8, 512 positions (64 / 128 / 256 workgroups) 6.0 / 5.2 / 5.0, 1000 (128 / 256 / 512)
     // 6.4 / 5.7 / 5.9, 1700 6.8 / 6.9 / 7.6; 32 of 128 over 4 at 1000 7.3 / 6.1 / 6.3, with all eight heads 9.7; 64 of 128 over 8 at 4000 12.8 / 13.1 / 14.4, with eight 13.3.
+    // All eight heads of a KV head where that leaves two workgroups a CU and the cache is so long that reading it is what takes the time: with eight / four, 128 heads of
+    // 128 over 16 at 3000 17.3 / 16.4, 6000 25.5 / 26.1, 12000 37.7 / 39.5, 32000 83.9 / 89.9, of 64 8000 18.6 / 18.1, 12200 23.4 / 24.1, 32000 47.0 / 49.0; 64 of 128 over 8 (one
+    // workgroup a CU) at 32000 52.0 / 50.8.
     const int group = n_heads / n_kv;
     int g = 1;
     while (g < group && g < 4 && p.nsplit * n_heads / g > 256) g *= 2;
+    if (g == 4 && group == 8 && p.nsplit * n_kv >= 512 && (long)pos * head_dim >= 5120 * 128) g = 8;
     if (p.nsplit == 1) {
         p.chunk = pos + 1;
         g = 1;

@@ -256,6 +256,8 @@ def test_generate_is_prefill_plus_greedy_decoding_and_stops_at_eos(ops):
     (32, 8, 64, [64, 383, 384, 512, 1100]),               # one, two and four heads to a workgroup
     (16, 2, 128, [31, 32, 63, 64, 255, 256, 500]),        # eight heads of a KV head
     (64, 8, 128, [256, 513, 700]),
+    (128, 16, 128, [5119, 5120, 5150]),                   # four, then all eight heads to a workgroup
+    (128, 16, 64, [10239, 10240]),
 ])
 def test_decode_attention_whole_and_in_chunks(ops, n_heads, n_kv, hd, positions):
     test_decode_attention(ops, n_heads, n_kv, hd, positions[-1] + 3, positions)
