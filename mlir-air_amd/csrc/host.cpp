@@ -63,42 +63,60 @@ py::list w4a16_entries() {
 }
 #undef NAME
 
-void raise(const char *check, int code) { py::module_::import("air_hip._lib").attr(check)(code); }
-void must(int code) {
-    if (code) raise("check_dense", code);
+// What an entry point refused, on its way to the errors of _lib.py: `check` raises the code's.
+struct Refused {
+    const char *check;
+    int code;
+};
+void must(int code, const char *check = "check_dense") {
+    if (code) throw Refused{check, code};
+}
+// f, which allocates and launches, without Python's lock, as ctypes calls the entry points: other threads go on, also where the launch queue is full.
+// (It takes and gives back no Python objects.  One row of 1024 x 1024, a call: 3.77 us with the lock held, 3.78 so.)
+template <class F>
+auto unlocked(F f) {
+    try {
+        py::gil_scoped_release others;
+        return f();
+    } catch (const Refused &r) {
+        py::module_::import("air_hip._lib").attr(r.check)(r.code);
+        throw;
+    }
 }
 
 bool on_gpu(const Tensor &t) { return t.defined() && t.is_cuda() && t.is_contiguous(); }
 bool shaped(const Tensor &t, at::IntArrayRef sizes) { return on_gpu(t) && t.sizes() == sizes; }
 
 // ---- int4 Linear ---------------------------------------------------------------------------------------------------------------
-// y = bf16(x . W (+ residual)) of a stream-order matrix; `vector`: the form of one row, whose result is [N]
+// y = bf16(x . W) of a stream-order matrix; `vector`: the form of one row, whose result is [N]
 std::optional<Tensor> linear(const Tensor &x, const Tensor &w, int64_t K, int64_t N, bool q4, bool vector, uintptr_t stream) {
     if (!on_gpu(x) || !on_gpu(w) || x.scalar_type() != at::kBFloat16) return std::nullopt;
     const int64_t dims = x.dim();
     if (vector ? x.numel() != K : (dims != 1 && dims != 2) || x.size(-1) != K) return std::nullopt;
     const int64_t M = vector || dims == 1 ? 1 : x.size(0);
     if (M < 1 || M > INT32_MAX || K > INT32_MAX || N > INT32_MAX) return std::nullopt;
-    Tensor y = vector || dims == 1 ? at::empty({N}, x.options()) : at::empty({M, N}, x.options());
-    const auto *xp = static_cast<const uint16_t *>(x.data_ptr());
-    auto *yp = static_cast<uint16_t *>(y.data_ptr());
-    void *st = reinterpret_cast<void *>(stream);
-    const int m = (int)M, k = (int)K, n = (int)N;
-    int rc;
-    if (M == 1) {
-        rc = q4 ? w4a16.w4a16_q4nx_gemv_stream_bf16(xp, w.data_ptr(), nullptr, yp, k, n, st) : w4a16.w4a16_gemv_stream_bf16(xp, w.data_ptr(), yp, k, n, 128, st);
-    } else {
-        // plain scratch of the call: of the caller's stream and, in a capture, of its graph
-        const size_t bytes = M <= 16 ? 0 : q4 ? w4a16.w4a16_q4nx_gemm_stream_best_scratch_bytes(m, k, n, 0) : w4a16.w4a16_gemm_stream_best_scratch_bytes(m, k, n);
-        Tensor scratch;
-        if (bytes) scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
-        void *sp = bytes ? scratch.data_ptr() : nullptr;
-        if (q4) rc = w4a16.w4a16_q4nx_gemm_stream_scratch_bf16(xp, w.data_ptr(), nullptr, yp, m, k, n, sp, bytes, st);
-        else if (bytes) rc = w4a16.w4a16_gemm_stream_scratch_bf16(xp, w.data_ptr(), yp, m, k, n, 128, sp, bytes, st);
-        else rc = w4a16.w4a16_gemm_stream_bf16(xp, w.data_ptr(), yp, m, k, n, 128, st);
-    }
-    if (rc) raise("check", rc);
-    return y;
+    return unlocked([&]() -> std::optional<Tensor> {
+        Tensor y = vector || dims == 1 ? at::empty({N}, x.options()) : at::empty({M, N}, x.options());
+        const auto *xp = static_cast<const uint16_t *>(x.data_ptr());
+        auto *yp = static_cast<uint16_t *>(y.data_ptr());
+        void *st = reinterpret_cast<void *>(stream);
+        const int m = (int)M, k = (int)K, n = (int)N;
+        int rc;
+        if (M == 1) {
+            rc = q4 ? w4a16.w4a16_q4nx_gemv_stream_bf16(xp, w.data_ptr(), nullptr, yp, k, n, st) : w4a16.w4a16_gemv_stream_bf16(xp, w.data_ptr(), yp, k, n, 128, st);
+        } else {
+            // plain scratch of the call: of the caller's stream and, in a capture, of its graph
+            const size_t bytes = M <= 16 ? 0 : q4 ? w4a16.w4a16_q4nx_gemm_stream_best_scratch_bytes(m, k, n, 0) : w4a16.w4a16_gemm_stream_best_scratch_bytes(m, k, n);
+            Tensor scratch;
+            if (bytes) scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+            void *sp = bytes ? scratch.data_ptr() : nullptr;
+            if (q4) rc = w4a16.w4a16_q4nx_gemm_stream_scratch_bf16(xp, w.data_ptr(), nullptr, yp, m, k, n, sp, bytes, st);
+            else if (bytes) rc = w4a16.w4a16_gemm_stream_scratch_bf16(xp, w.data_ptr(), yp, m, k, n, 128, sp, bytes, st);
+            else rc = w4a16.w4a16_gemm_stream_bf16(xp, w.data_ptr(), yp, m, k, n, 128, st);
+        }
+        must(rc, "check");
+        return y;
+    });
 }
 
 // ---- dense-weight models: many tokens through every layer ----------------------------------------------------------------------
@@ -261,21 +279,23 @@ std::optional<Tensor> latent_rows(py::list layers, std::vector<Tensor> caches, s
         ls[i].eps = eps;
         if (!ls[i].read(layers[i], caches[i], tables[i], p, W, pos, absorb_most)) return std::nullopt;
     }
-    const Tensor res = p.floats({M, W});
-    float *rp = res.data_ptr<float>();
-    Tensor h = p.elems(M, W);
-    must(dense.dlm_embed_rows(p.dt, tokens.data_ptr<int>(), embed.data_ptr(), embed_scale, rp, h.data_ptr(), (int)M, (int)W, p.stream));
-    for (const LatentLayer &l : ls) {
-        const Tensor attn = l.attend(p, p.gemm(h.data_ptr(), W, l.w_in, 0), pos), y = p.parts(attn, l.w_o);
-        h = p.elems(M, W);
-        must(dense.dlm_residual_norm_parts(p.dt, rp, y.data_ptr<float>(), (int)y.size(0), l.norm1.data_ptr<float>(), eps, width, h.data_ptr(), (int)M, (int)W, p.stream));
-        if (!l.experts.top) continue;
-        const auto [out, weights] = l.experts.run(p, h, p.parts(h, l.experts.w_router));
-        h = p.elems(M, W);
-        must(dense.dlm_residual_norm_rows(p.dt, rp, out.data_ptr(), weights.data_ptr<float>(), l.experts.top, l.norm2.data_ptr<float>(), eps, width, h.data_ptr(), (int)M,
-                                          (int)W, p.stream));
-    }
-    return res;
+    return unlocked([&]() -> std::optional<Tensor> {
+        const Tensor res = p.floats({M, W});
+        float *rp = res.data_ptr<float>();
+        Tensor h = p.elems(M, W);
+        must(dense.dlm_embed_rows(p.dt, tokens.data_ptr<int>(), embed.data_ptr(), embed_scale, rp, h.data_ptr(), (int)M, (int)W, p.stream));
+        for (const LatentLayer &l : ls) {
+            const Tensor attn = l.attend(p, p.gemm(h.data_ptr(), W, l.w_in, 0), pos), y = p.parts(attn, l.w_o);
+            h = p.elems(M, W);
+            must(dense.dlm_residual_norm_parts(p.dt, rp, y.data_ptr<float>(), (int)y.size(0), l.norm1.data_ptr<float>(), eps, width, h.data_ptr(), (int)M, (int)W, p.stream));
+            if (!l.experts.top) continue;
+            const auto [out, weights] = l.experts.run(p, h, p.parts(h, l.experts.w_router));
+            h = p.elems(M, W);
+            must(dense.dlm_residual_norm_rows(p.dt, rp, out.data_ptr(), weights.data_ptr<float>(), l.experts.top, l.norm2.data_ptr<float>(), eps, width, h.data_ptr(), (int)M,
+                                              (int)W, p.stream));
+        }
+        return res;
+    });
 }
 
 // One layer of windowed attention beside a recurrence, or of the delta rule (sitirax.SitiraxLayer)
@@ -405,49 +425,53 @@ std::optional<Tensor> mixed_rows(py::list layers, py::list caches, const Tensor 
     std::vector<MixedLayer> ls(layers.size());
     for (size_t i = 0; i < ls.size(); ++i)
         if (!ls[i].read(layers[i], caches[i].cast<py::dict>(), p, W, pos, split_most)) return std::nullopt;
-    const Tensor res = p.floats({M, W});
-    Tensor y;
-    bool first = true;
-    // the residual brought up to date (from the embedding first), and its norm
-    auto add_norm = [&](const Tensor *norm) {
-        Tensor h;
-        if (norm) h = p.elems(M, W);
-        void *hp = norm ? h.data_ptr() : nullptr;
-        const float *np = norm ? norm->data_ptr<float>() : nullptr;
-        if (y.defined())
-            must(dense.dlm_add_norm_parts(p.dt, res.data_ptr<float>(), y.data_ptr<float>(), (int)y.size(0), np, eps, width, hp, (int)M, (int)W, p.stream));
-        else
-            must(dense.dlm_add_norm_rows(p.dt, res.data_ptr<float>(), nullptr, first ? tokens.data_ptr<int>() : nullptr, first ? embed.data_ptr() : nullptr, 1.0f, np, eps, width, hp,
-                                         (int)M, (int)W, p.stream));
-        first = false;
-        return h;
-    };
-    for (const MixedLayer &l : ls) {
-        const Tensor h = add_norm(&l.norm1);
-        const Tensor out = l.mix(p, p.gemm(h.data_ptr(), W, l.w_in, 0, -1, l.silu[0], l.silu[1]), pos, eps, unit_eps, steps_most);
-        y = p.parts(out, l.w_o);
-        if (l.norm2.defined()) {
-            const Tensor h2 = add_norm(&l.norm2), a = p.gemm(h2.data_ptr(), W, l.w_gate_up, 3);
-            y = p.parts(a, l.w_down);
+    return unlocked([&]() -> std::optional<Tensor> {
+        const Tensor res = p.floats({M, W});
+        Tensor y;
+        bool first = true;
+        // the residual brought up to date (from the embedding first), and its norm
+        auto add_norm = [&](const Tensor *norm) {
+            Tensor h;
+            if (norm) h = p.elems(M, W);
+            void *hp = norm ? h.data_ptr() : nullptr;
+            const float *np = norm ? norm->data_ptr<float>() : nullptr;
+            if (y.defined())
+                must(dense.dlm_add_norm_parts(p.dt, res.data_ptr<float>(), y.data_ptr<float>(), (int)y.size(0), np, eps, width, hp, (int)M, (int)W, p.stream));
+            else
+                must(dense.dlm_add_norm_rows(p.dt, res.data_ptr<float>(), nullptr, first ? tokens.data_ptr<int>() : nullptr, first ? embed.data_ptr() : nullptr, 1.0f, np, eps, width, hp,
+                                             (int)M, (int)W, p.stream));
+            first = false;
+            return h;
+        };
+        for (const MixedLayer &l : ls) {
+            const Tensor h = add_norm(&l.norm1);
+            const Tensor out = l.mix(p, p.gemm(h.data_ptr(), W, l.w_in, 0, -1, l.silu[0], l.silu[1]), pos, eps, unit_eps, steps_most);
+            y = p.parts(out, l.w_o);
+            if (l.norm2.defined()) {
+                const Tensor h2 = add_norm(&l.norm2), a = p.gemm(h2.data_ptr(), W, l.w_gate_up, 3);
+                y = p.parts(a, l.w_down);
+            }
         }
-    }
-    add_norm(nullptr);
-    return res;
+        add_norm(nullptr);
+        return res;
+    });
 }
 
 // Logits fp32 [rows of the head] of one row of a finished residual and its greedy choice [1]; mode: the intake of dlm_gemv, 3 or 4
 std::optional<std::pair<Tensor, Tensor>> tail(int mode, const Tensor &res, const Tensor &final_w, const Tensor &head, float eps, int width, int n_valid, uintptr_t stream) {
     if (!on_gpu(res) || !on_gpu(final_w) || !on_gpu(head) || head.dim() != 2 || res.numel() != head.size(1) || final_w.numel() != head.size(1)) return std::nullopt;
     if (res.scalar_type() != at::kFloat || final_w.scalar_type() != at::kFloat || (head.scalar_type() != at::kBFloat16 && head.scalar_type() != at::kFloat)) return std::nullopt;
-    const Pass p(1, head, stream);
-    const int K = (int)head.size(1), N = (int)head.size(0), n_keys = dense.dlm_gemv_keys(K, N);
-    const Tensor logits = p.floats({N}), keys = at::empty({n_keys}, p.elem.dtype(at::kLong)), best = at::empty({1}, p.i32);
-    dlm_intake in{};
-    in.mode = mode, in.width = width, in.eps = eps, in.scale = 1.0f, in.res = res.data_ptr<float>(), in.final_w = final_w.data_ptr<float>();
-    auto *kp = reinterpret_cast<uint64_t *>(keys.data_ptr<int64_t>());
-    must(dense.dlm_gemv(p.dt, head.data_ptr(), &in, nullptr, logits.data_ptr<float>(), kp, n_valid, K, N, p.stream));
-    must(dense.dlm_argmax(kp, n_keys, best.data_ptr<int>(), nullptr, nullptr, p.stream));
-    return std::make_pair(logits, best);
+    return unlocked([&]() -> std::optional<std::pair<Tensor, Tensor>> {
+        const Pass p(1, head, stream);
+        const int K = (int)head.size(1), N = (int)head.size(0), n_keys = dense.dlm_gemv_keys(K, N);
+        const Tensor logits = p.floats({N}), keys = at::empty({n_keys}, p.elem.dtype(at::kLong)), best = at::empty({1}, p.i32);
+        dlm_intake in{};
+        in.mode = mode, in.width = width, in.eps = eps, in.scale = 1.0f, in.res = res.data_ptr<float>(), in.final_w = final_w.data_ptr<float>();
+        auto *kp = reinterpret_cast<uint64_t *>(keys.data_ptr<int64_t>());
+        must(dense.dlm_gemv(p.dt, head.data_ptr(), &in, nullptr, logits.data_ptr<float>(), kp, n_valid, K, N, p.stream));
+        must(dense.dlm_argmax(kp, n_keys, best.data_ptr<int>(), nullptr, nullptr, p.stream));
+        return std::make_pair(logits, best);
+    });
 }
 
 }  // namespace

@@ -1,5 +1,7 @@
 """Passes and operators whose host side is native code (csrc/host.cpp) against the operators in Python, bit for bit (the same launches), and the calls
 that are left to those."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -88,3 +90,38 @@ def test_linear_forms(monkeypatch, q4):
         for op in (gemv, gemm):
             with pytest.raises(error):
                 op(bad, w)
+
+
+def test_other_threads_run_while_a_call_launches():
+    """Entry points are called without Python's lock: PyGILState_Check in their place, which returns 0 then, and 1, an error's code, where it is held.
+    (Nothing is launched.)"""
+    from air_hip import _lib, ops
+    held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    asked = ("_slices", "gemm_parts", "_tile_rows", "_max_tiles", "gemv_keys", "_supported", "_bytes")   # (these launch nothing)
+    stream = torch.cuda.current_stream().cuda_stream
+    models = [mod._model(config, 5, torch.bfloat16)[0] for mod, config in ((tk, KUVONEX_MIXED), (ts, SITIRAX_MIXED))]
+    w = ops.repack_stream(*map(dev, make_awq(256, 128, seed=1)))
+    for bind, lib, names in ((_lib.host_dense().bind_dense, _lib.load_dense_library(), _lib.host_dense().dense_entries()),
+                             (_lib.host_w4a16().bind_w4a16, _lib.load_library(), _lib.host_w4a16().w4a16_entries())):
+        real = _lib._addresses(lib, names)
+        bind({n: at if n.endswith(asked) else held for n, at in real.items()})
+        try:
+            if lib is _lib.load_library():
+                for M in (1, 2, 17, 130):
+                    assert _lib.host_w4a16().linear(dev(make_x((M, 256), seed=M)), w.buf, 256, 128, False, False, stream) is not None
+                continue
+            for m in models:
+                for n in (2, 70):
+                    assert m._rows(m.new_cache(80), torch.zeros(n, dtype=torch.int32, device="cuda"), 0).shape == (n, m.embed.shape[1])
+                c = m.config
+                assert _lib.host_dense().tail(m.tail_intake, torch.zeros(m.embed.shape[1], device="cuda"), m.final_norm, m.head, c.eps, c.width, m.vocab, stream) is not None
+        finally:
+            bind(real)
+
+
+def test_errors_of_a_call():
+    """What an entry point refuses is the same error as from Python."""
+    from air_hip import _lib, ops
+    w = ops.repack_stream(*map(dev, make_awq(256, 128, seed=1)))
+    with pytest.raises(_lib.W4A16Error):
+        _lib.host_w4a16().linear(dev(make_x((1, 192), seed=1)), w.buf, 192, 128, False, True, torch.cuda.current_stream().cuda_stream)   # no whole groups
