@@ -3,6 +3,7 @@
 import ctypes
 import importlib.util
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libw4a16_hip.so")
@@ -244,7 +245,8 @@ def _bind(path, symbols):
     return lib
 
 
-def _load_host():
+def load_host():
+    """The host module (csrc/host.cpp); raises LibraryNotBuiltError where it is missing, ImportError where it does not load."""
     global _host
     if _host is None:
         if not os.path.exists(_HOST_PATH):
@@ -262,23 +264,39 @@ def _addresses(lib, names):
     return {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}
 
 
+class _NoHost:
+    """In the host module's place: leaves every call to the operators in Python, which make the same launches."""
+
+    linear = latent_rows = mixed_rows = tail = staticmethod(lambda *args: None)
+
+
+def _host_or_none():
+    try:
+        return load_host()
+    except (LibraryNotBuiltError, ImportError) as e:
+        warnings.warn(f"the host side of small calls runs in Python, which takes longer: {e}", RuntimeWarning, stacklevel=4)
+        return None
+
+
 def host_w4a16():
-    """The host module (csrc/host.cpp) for the int4 operators."""
+    """The host module for the int4 operators, or what leaves them to Python."""
     global _host_w4a16
     if _host_w4a16 is None:
-        host = _load_host()
-        host.bind_w4a16(_addresses(load_library(), host.w4a16_entries()))
-        _host_w4a16 = host
+        lib, host = load_library(), _host_or_none()
+        if host is not None:
+            host.bind_w4a16(_addresses(lib, host.w4a16_entries()))
+        _host_w4a16 = host or _NoHost
     return _host_w4a16
 
 
 def host_dense():
-    """The host module for the dense-weight models."""
+    """The host module for the dense-weight models, or what leaves them to Python."""
     global _host_dense
     if _host_dense is None:
-        host = _load_host()
-        host.bind_dense(_addresses(load_dense_library(), host.dense_entries()))
-        _host_dense = host
+        lib, host = load_dense_library(), _host_or_none()
+        if host is not None:
+            host.bind_dense(_addresses(lib, host.dense_entries()))
+        _host_dense = host or _NoHost
     return _host_dense
 
 

@@ -6,7 +6,7 @@
 // addresses.
 //
 // Functions return None, with nothing launched, where tensors are not of the form that they take: the operators in Python (ops.py, dense.py) say
-// then what is wrong with them.
+// then what is wrong with them.  (Without the module they run always.)
 #include <torch/extension.h>
 
 #include <cmath>

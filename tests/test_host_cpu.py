@@ -3,6 +3,7 @@ comparator, backend argument checks, and the C ABI's symbols and error paths."""
 import ctypes
 import os
 import re
+import warnings
 
 import numpy as np
 import pytest
@@ -431,3 +432,21 @@ def test_int4_slices_are_ranked_by_time_and_advised_past_what_their_launch_costs
     assert slices(64, 4096, 1024) > 4 and slices(20, 5120, 1280) > 4 and slices(33, 128 * 19, 272) == 0   # (four were the first below 12 us)
     assert lib.w4a16_gemm_stream_best_scratch_bytes(30, 3328, 1472) == 0 and lib.w4a16_gemm_stream_best_scratch_bytes(20, 5120, 1280) == 0
     assert lib.w4a16_gemm_stream_best_scratch_bytes(64, 14336, 4096) >= lib.w4a16_gemm_stream_scratch_bytes(64, 14336, 4096)
+
+
+@pytest.mark.parametrize("broken", [False, True])
+def test_without_the_host_module_the_operators_run_in_python(monkeypatch, tmp_path, broken):
+    """A missing module, or one that does not load (built against another torch, say), leaves every call to Python, and says so once a library."""
+    path = tmp_path / "air_host.so"
+    if broken:
+        path.write_bytes(b"not a library")
+    monkeypatch.setattr(_lib, "_HOST_PATH", str(path))
+    for name in ("_host", "_host_w4a16", "_host_dense"):
+        monkeypatch.setattr(_lib, name, None)
+    for get in (_lib.host_w4a16, _lib.host_dense):
+        with pytest.warns(RuntimeWarning, match="air_host"):
+            host = get()
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            assert get() is host
+    assert all(f(1, 2, 3) is None for f in (host.linear, host.latent_rows, host.mixed_rows, host.tail))
