@@ -86,7 +86,8 @@ def _build_host():
 
 
 def build(jobs=4, extra=(), verbose=False, only=None):
-    """Compile and link the libraries named in `only` (default: all); returns the path of the last one."""
+    """Compile and link the libraries named in `only` (default: all, and the host module); returns the path of the last one.  What the host module needs beside
+    hipcc (g++, torch and its headers) may be missing: the libraries are linked first, then that is an error."""
     names = list(only or (*LIBRARIES, HOST))
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -95,8 +96,6 @@ def build(jobs=4, extra=(), verbose=False, only=None):
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         host = pool.submit(_build_host) if host else None
         results = dict(zip(sources, pool.map(lambda s: _compile(s, list(extra)), sources)))
-        if host:
-            host.result()
     for _, out in results.values():
         if out.strip() and verbose:
             print(out)
@@ -105,6 +104,8 @@ def build(jobs=4, extra=(), verbose=False, only=None):
         tmp = f"{lib_path(name)}.{os.getpid()}"   # renamed when whole: nobody loads half a library
         subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs])
         os.replace(tmp, lib_path(name))
+    if host:
+        host.result()
     return lib_path(names[-1] if names else HOST)
 
 
@@ -117,12 +118,20 @@ def _lock():
 
 
 def ensure(name, jobs=8):
-    """The library `name` and the host module, built first where there is none (one builder at a time)."""
-    if not all(os.path.exists(lib_path(n)) for n in (name, HOST)):
+    """The library `name` and the host module, built first where there is none (one builder at a time).  Without what the host module is built with, the library
+    alone: the package runs without the module."""
+    for n in (name, HOST):
+        if os.path.exists(lib_path(n)):
+            continue
         with _lock():
-            missing = [n for n in (name, HOST) if not os.path.exists(lib_path(n))]
-            if missing:
-                build(jobs, only=missing)
+            if os.path.exists(lib_path(n)):
+                continue
+            try:
+                build(jobs, only=[n])
+            except Exception as e:
+                if n != HOST:
+                    raise
+                print(f"no host module: {e}", file=sys.stderr)
     return lib_path(name)
 
 

@@ -1,6 +1,7 @@
 """Host logic of the product package (no GPU): layout tools against the oracle, the runner's
 comparator, backend argument checks, and the C ABI's symbols and error paths."""
 import ctypes
+import importlib.util
 import os
 import re
 import warnings
@@ -450,3 +451,26 @@ def test_without_the_host_module_the_operators_run_in_python(monkeypatch, tmp_pa
             warnings.simplefilter("error")
             assert get() is host
     assert all(f(1, 2, 3) is None for f in (host.linear, host.latent_rows, host.mixed_rows, host.tail))
+
+
+def test_build_links_the_libraries_where_the_host_module_cannot_be_built(monkeypatch, tmp_path, capsys):
+    """Without g++ or torch's headers: an error behind the link, and a library that is asked for alone is built without one."""
+    spec = importlib.util.spec_from_file_location("build_under_test", os.path.join(ROOT, "mlir-air_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    for name in ("LIB_DIR", "OBJ_DIR"):
+        monkeypatch.setattr(build, name, str(tmp_path / name))
+
+    def no_host():
+        raise RuntimeError("no compiler for the host module")
+
+    monkeypatch.setattr(build, "_build_host", no_host)
+    monkeypatch.setattr(build, "_compile", lambda src, extra: (src, ""))
+    monkeypatch.setattr(build.subprocess, "check_call", lambda cmd: open(cmd[cmd.index("-o") + 1], "w").close())
+    with pytest.raises(RuntimeError, match="no compiler"):
+        build.build()
+    for name in build.LIBRARIES:
+        assert os.path.exists(build.lib_path(name))
+        os.remove(build.lib_path(name))
+        assert build.ensure(name) == build.lib_path(name) and os.path.exists(build.lib_path(name))
+        assert "no compiler" in capsys.readouterr().err
