@@ -7,6 +7,7 @@ import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libw4a16_hip.so")
+W4A16_ABI = 1
 DENSE_ABI = 2
 _DENSE_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libdense_lm_hip.so")
 _HOST_PATH = os.path.join(os.path.dirname(_HERE), "lib", "air_host.so")
@@ -246,7 +247,8 @@ def _bind(path, symbols):
 
 
 def load_host():
-    """The host module (csrc/host.cpp); raises LibraryNotBuiltError where it is missing, ImportError where it does not load."""
+    """The host module (csrc/host.cpp); raises LibraryNotBuiltError where it is missing or older than the libraries'
+    interface, ImportError where it does not load."""
     global _host
     if _host is None:
         if not os.path.exists(_HOST_PATH):
@@ -256,8 +258,19 @@ def load_host():
         spec = importlib.util.spec_from_file_location("air_host", _HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        wrong = _host_misfits(module)
+        if wrong:
+            raise LibraryNotBuiltError(f"{_HOST_PATH} was built against other headers ({wrong}): build it again")
         _host = module
     return _host
+
+
+def _host_misfits(module):
+    """What of the C ABI the host module was compiled for in another form than the libraries are called here: versions and struct sizes."""
+    if not hasattr(module, "compiled_for"):
+        return "no record of them"
+    here = {"w4a16": W4A16_ABI, "dense_lm": DENSE_ABI}
+    return ", ".join(f"{k} {v}" for k, v in module.compiled_for().items() if v != (here[k] if k in here else ctypes.sizeof(globals()[k])))
 
 
 def _addresses(lib, names):
@@ -335,8 +348,8 @@ def load_library():
             "(there is no CPU fallback for the W4A16 kernels)"
         )
     lib = _bind(_LIB_PATH, SYMBOLS)
-    if lib.w4a16_abi_version() != 1:
-        raise LibraryNotBuiltError(f"{_LIB_PATH}: ABI version {lib.w4a16_abi_version()} != 1, rebuild")
+    if lib.w4a16_abi_version() != W4A16_ABI:
+        raise LibraryNotBuiltError(f"{_LIB_PATH}: ABI version {lib.w4a16_abi_version()} != {W4A16_ABI}, rebuild")
     _lib = lib
     return lib
 

@@ -62,6 +62,15 @@ py::list w4a16_entries() {
     return names;
 }
 #undef NAME
+// What the module was compiled against: the ABI versions and the size of every struct that crosses, as _lib.py has them, which compares.
+py::dict compiled_for() {
+    py::dict d;
+    d["w4a16"] = W4A16_ABI_VERSION, d["dense_lm"] = DLM_ABI_VERSION;
+    d["Intake"] = sizeof(dlm_intake), d["Router"] = sizeof(dlm_router), d["GemmArgs"] = sizeof(dlm_gemm_args), d["LatentShape"] = sizeof(dlm_latent_shape);
+    d["LatentRows"] = sizeof(dlm_latent_rows), d["HeadShape"] = sizeof(dlm_head_shape), d["HeadRows"] = sizeof(dlm_head_rows);
+    d["ShortConvArgs"] = sizeof(dlm_short_conv_args), d["RecurrenceArgs"] = sizeof(dlm_recurrence_args);
+    return d;
+}
 
 // What an entry point refused, on its way to the errors of _lib.py: `check` raises the code's.
 struct Refused {
@@ -481,6 +490,7 @@ PYBIND11_MODULE(air_host, m) {
     m.def("bind_w4a16", &bind_w4a16);
     m.def("dense_entries", &dense_entries);
     m.def("w4a16_entries", &w4a16_entries);
+    m.def("compiled_for", &compiled_for);
     m.def("linear", &linear);
     m.def("latent_rows", &latent_rows);
     m.def("mixed_rows", &mixed_rows);

@@ -474,3 +474,25 @@ def test_build_links_the_libraries_where_the_host_module_cannot_be_built(monkeyp
         os.remove(build.lib_path(name))
         assert build.ensure(name) == build.lib_path(name) and os.path.exists(build.lib_path(name))
         assert "no compiler" in capsys.readouterr().err
+
+
+def test_a_host_module_built_against_other_headers_is_not_used(monkeypatch):
+    """Versions and struct sizes are those of the ctypes side, and one that differs leaves the calls to Python."""
+    module = _lib.load_host()
+    compiled = module.compiled_for()
+    assert compiled["w4a16"] == _lib.load_library().w4a16_abi_version() and compiled["dense_lm"] == _lib.load_dense_library().dlm_abi_version()
+    text = open(os.path.join(ROOT, "mlir-air_amd", "csrc", "host.cpp")).read()
+    handed_over = set(re.findall(r"\bdlm_(\w+) \w+{", text)) | {"latent_shape", "head_shape"}
+    assert {n.title().replace("_", "") for n in handed_over} <= set(compiled)   # every struct that it fills in
+    assert _lib._host_misfits(module) == "" and "no record" in _lib._host_misfits(object())
+    for name in ("GemmArgs", "HeadRows"):
+        class Longer(getattr(_lib, name)):
+            _fields_ = [("more", ctypes.c_int64)]
+        with monkeypatch.context() as m:
+            m.setattr(_lib, name, Longer)
+            for cached in ("_host", "_host_dense"):
+                m.setattr(_lib, cached, None)
+            with pytest.raises(_lib.LibraryNotBuiltError, match=name):
+                _lib.load_host()
+            with pytest.warns(RuntimeWarning, match="other headers"):
+                assert _lib.host_dense().latent_rows(1) is None
