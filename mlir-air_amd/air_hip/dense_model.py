@@ -51,8 +51,15 @@ class SequenceCache:
 
 
 class DenseModel(generation.CausalLM):
-    tail_intake = None       # how a one-token product norms the last row of a finished residual: an intake of dense.py
+    # How the product of `_head(_pending(row))` norms a row of a finished residual, an intake of dense.py: a prompt's tail is then one native call.
+    # None: by `_tail`.  (So it is where a class has a form of one of the three of its own and does not say otherwise.)
+    tail_intake = None
     max_portion = None       # most tokens that go through the layers at once (None: any number)
+
+    def __init_subclass__(cls, **kwargs):
+        super().__init_subclass__(**kwargs)
+        if {"_head", "_pending", "_tail"} & cls.__dict__.keys() and "tail_intake" not in cls.__dict__:
+            cls.tail_intake = None
 
     @classmethod
     def load(cls, path, config_json, dtype=torch.bfloat16, device="cuda"):
@@ -115,9 +122,13 @@ class DenseModel(generation.CausalLM):
             return self._tail(self._one_token(cache, ids, pos))
         for a, b in self._portions(len(ids)):
             res = self._rows(cache, ids[a:b], pos + a)
-        last, c = res[-1], self.config
-        out = _lib.host_dense().tail(self.tail_intake, last, self.final_norm, self.head, c.eps, c.width, self.vocab, _stream())
-        return (out[0][:self.vocab], out[1]) if out is not None else self._tail(self._pending(last.contiguous()))
+        last = res[-1]
+        if self.tail_intake is not None:
+            c = self.config
+            out = _lib.host_dense().tail(self.tail_intake, last, self.final_norm, self.head, c.eps, c.width, self.vocab, _stream())
+            if out is not None:
+                return out[0][:self.vocab], out[1]
+        return self._tail(self._pending(last.contiguous()))
 
     def decode_token(self, cache, token):
         pos = self._advance(cache, 1)

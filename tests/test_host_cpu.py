@@ -496,3 +496,44 @@ def test_a_host_module_built_against_other_headers_is_not_used(monkeypatch):
                 _lib.load_host()
             with pytest.warns(RuntimeWarning, match="other headers"):
                 assert _lib.host_dense().latent_rows(1) is None
+
+
+def test_a_model_with_a_tail_of_its_own():
+    """A further dense-weight model gives its passes and the tail's two steps; a prompt goes by those unless the class names the native tail's form."""
+    import torch
+    from air_hip import dense
+    from air_hip.dense_model import DenseModel, SequenceCache
+    from air_hip.kuvonex import KuvonexModel
+    from air_hip.sitirax import SitiraxModel
+
+    class Own(DenseModel):
+        device, vocab = torch.device("cpu"), 9
+
+        def _rows(self, cache, tokens, pos, trace=None):
+            return tokens.float()[:, None].expand(-1, 4)
+
+        def _pending(self, row):
+            return row + 1
+
+        def _tail(self, pending):
+            return pending, pending.argmax().reshape(1)
+
+    model = Own()
+    cache = SequenceCache(model, 8)
+    for tokens in ([3, 5], torch.tensor([1, 5], dtype=torch.int32)):
+        row, _ = model.prefill(cache, tokens)
+        assert row.tolist() == [6.0] * 4
+
+    class Scaled(KuvonexModel):
+        def _head(self, r, keys=None):
+            return super()._head(r, keys)
+
+    class Kept(SitiraxModel):
+        def _tail(self, pending):
+            return super()._tail(pending)
+
+    class Longer(SitiraxModel):
+        max_portion = 64
+
+    assert Kept.tail_intake is None and Scaled.tail_intake is None and KuvonexModel.tail_intake == dense.FINAL
+    assert Longer.tail_intake == SitiraxModel.tail_intake == dense.NORMED
