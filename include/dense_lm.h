@@ -157,7 +157,8 @@ int dlm_latent_prepare(int dtype, const dlm_latent_shape *s, const dlm_latent_ro
 int dlm_latent_prefill(int dtype, const dlm_latent_shape *s, const dlm_latent_rows *r, const void *kv, int64_t ldkv, const float *sink,
                        void *out, int64_t ldo, void *stream);
 /* One token or short portions: qa [M * heads, rank + rot]; part_o fp32 [M * heads, nsplit, rank], part_ml
- * [M * heads, nsplit, 2]; nsplit <= 256. */
+ * [M * heads, nsplit, 2]; nsplit <= 256, dlm_latent_splits of `total` cached tokens (the M among them) for speed. */
+int dlm_latent_splits(int heads, int M, int64_t total);
 int dlm_latent_absorb(int dtype, const dlm_latent_shape *s, const dlm_latent_rows *r, const void *w_uk, void *qa, void *stream);
 int dlm_latent_decode(int dtype, const dlm_latent_shape *s, const dlm_latent_rows *r, const void *qa, int nsplit, float *part_o,
                       float *part_ml, void *stream);
@@ -181,6 +182,7 @@ typedef struct {
     int32_t off, M, pos;
     float eps;
 } dlm_head_rows;
+int dlm_head_splits(int heads, int kv_heads, int64_t window, int M, int64_t total); /* an nsplit for speed, `total` tokens cached */
 int dlm_head_decode_supported(int dtype, const dlm_head_shape *s);
 int dlm_head_prefill_supported(int dtype, const dlm_head_shape *s);
 /* Normed queries q [kv_heads, M, heads / kv_heads, dim] and the cache rows; then either the attention of many rows, or of few with

@@ -202,6 +202,8 @@ DENSE_SYMBOLS = {
     "dlm_latent_prepare": (_ci, [_ci, _vp, _vp, _vp]),
     "dlm_latent_prefill": (_ci, [_ci, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp]),
     "dlm_latent_absorb": (_ci, [_ci] + [_vp] * 5),
+    "dlm_latent_splits": (_ci, [_ci, _ci, _i64]),
+    "dlm_head_splits": (_ci, [_ci, _ci, _i64, _ci, _i64]),
     "dlm_latent_decode": (_ci, [_ci, _vp, _vp, _vp, _ci, _vp, _vp, _vp]),
     "dlm_latent_combine": (_ci, [_ci, _vp, _vp, _ci] + [_vp] * 5 + [_i64, _vp]),
 }

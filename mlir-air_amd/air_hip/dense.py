@@ -410,11 +410,8 @@ def latent_attention_rows(spec, proj, kv_off, gate_off, lut, kv_norm, eps, cache
 
 
 def latent_splits(spec, M, total):
-    """How many workgroups share the keys of 16 rows.  A workgroup's time grows with its blocks of 32 keys, the merge's with
-    the splits and rows: the square root balances them (8 to 128 heads, 300 to 32k keys: within 5 % of the best of half to twice as many,
-    within 11 % with 128 heads, whose splits are few whole blocks)."""
-    rows, blocks = M * spec.heads, (total + 31) // 32
-    return max(1, min(256, 512 // ((rows + 15) // 16), blocks, round((512 * blocks / rows) ** 0.5)))
+    """How many workgroups share the keys of 16 rows where `total` tokens are cached."""
+    return _lib.load_dense_library().dlm_latent_splits(spec.heads, M, total)
 
 
 def latent_attention_absorbed(spec, proj, kv_off, gate_off, lut, kv_norm, eps, cache, pos, w_ukv, sink, pos_dev=None, nsplit=None):
@@ -473,11 +470,8 @@ class HeadSpec:
 
 
 def head_splits(spec, M, total):
-    """How many workgroups share the keys of 16 query rows of a key / value head: enough of them to fill the GPU twice, as far as
-    there are blocks of 32 keys."""
-    tiles = spec.kv_heads * ((M * (spec.heads // spec.kv_heads) + 15) // 16)
-    blocks = (min(total, spec.window + M - 1) + 31) // 32 + 1
-    return max(1, min(256, 512 // tiles, blocks))
+    """How many workgroups share the keys of 16 query rows of a key / value head where `total` tokens are cached."""
+    return _lib.load_dense_library().dlm_head_splits(spec.heads, spec.kv_heads, min(spec.window, 1 << 30), M, total)
 
 
 def head_attention(spec, proj, off, q_norm, k_norm, eps, cache, pos, out, pos_dev=None, nsplit=None, rows_form=False):

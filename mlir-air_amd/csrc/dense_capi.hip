@@ -1,6 +1,8 @@
 // C ABI of the dense-weight library (include/dense_lm.h): argument checks, then the launches of dense_kernels.h.
 #include "../../include/dense_lm.h"
 
+#include <algorithm>
+#include <cmath>
 #include <string>
 
 #include "dense_kernels.h"
@@ -169,6 +171,23 @@ const char *dlm_strerror(int code) {
 }
 
 const char *dlm_last_hip_error(void) { return g_error.c_str(); }
+
+// How many workgroups share the keys of 16 rows.  A workgroup's time grows with its blocks of 32 keys, the merge's with
+// the splits and rows: the square root balances them (8 to 128 heads, 300 to 32k keys: within 5 % of the best of half to twice as many,
+// within 11 % with 128 heads, whose splits are few whole blocks).
+int dlm_latent_splits(int heads, int M, int64_t total) {
+    if (heads <= 0 || M <= 0) return 1;
+    const int64_t rows = (int64_t)M * heads, blocks = (total + 31) / 32;
+    const int64_t balance = (int64_t)std::nearbyint(std::sqrt((double)(512 * blocks) / (double)rows));
+    return (int)std::max<int64_t>(1, std::min({(int64_t)256, 512 / ((rows + 15) / 16), blocks, balance}));
+}
+// How many workgroups share the keys of 16 query rows of a key / value head: enough of them to fill the GPU twice, as far as
+// there are blocks of 32 keys.
+int dlm_head_splits(int heads, int kv_heads, int64_t window, int M, int64_t total) {
+    if (heads <= 0 || kv_heads <= 0 || M <= 0) return 1;
+    const int64_t tiles = kv_heads * (((int64_t)M * (heads / kv_heads) + 15) / 16), blocks = (std::min(total, window + M - 1) + 31) / 32 + 1;
+    return (int)std::max<int64_t>(1, std::min({(int64_t)256, 512 / std::max<int64_t>(tiles, 1), blocks}));
+}
 
 int dlm_gemv_keys(int K, int N) { return K > 0 && N > 0 ? 4 * dense_gemv_blocks(K, N) : 0; }
 

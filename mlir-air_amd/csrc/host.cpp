@@ -9,7 +9,6 @@
 // then what is wrong with them.  (Without the module they run always.)
 #include <torch/extension.h>
 
-#include <cmath>
 #include <string>
 #include <vector>
 
@@ -26,9 +25,9 @@ namespace {
     X(dlm_gemm) X(dlm_gemm_slices) X(dlm_gemm_parts) X(dlm_gemm_sliced) X(dlm_gemm_tile_rows) X(dlm_moe_select_parts) X(dlm_moe_max_tiles) \
     X(dlm_moe_plan) X(dlm_residual_norm_parts) X(dlm_residual_norm_rows) X(dlm_add_norm_parts) X(dlm_add_norm_rows) X(dlm_embed_rows)      \
     X(dlm_gemv) X(dlm_gemv_keys) X(dlm_argmax) X(dlm_latent_decode_supported) X(dlm_latent_prefill_supported) X(dlm_latent_prepare)        \
-    X(dlm_latent_prefill) X(dlm_latent_absorb) X(dlm_latent_decode) X(dlm_latent_combine) X(dlm_head_decode_supported)                     \
-    X(dlm_head_prefill_supported) X(dlm_head_prepare) X(dlm_head_prefill) X(dlm_head_decode) X(dlm_head_merge) X(dlm_short_conv)           \
-    X(dlm_recurrence_steps) X(dlm_recurrence_chunk_bytes) X(dlm_recurrence_chunks) X(dlm_gated_norm)
+    X(dlm_latent_prefill) X(dlm_latent_splits) X(dlm_latent_absorb) X(dlm_latent_decode) X(dlm_latent_combine) X(dlm_head_splits)          \
+    X(dlm_head_decode_supported) X(dlm_head_prefill_supported) X(dlm_head_prepare) X(dlm_head_prefill) X(dlm_head_decode)                  \
+    X(dlm_head_merge) X(dlm_short_conv) X(dlm_recurrence_steps) X(dlm_recurrence_chunk_bytes) X(dlm_recurrence_chunks) X(dlm_gated_norm)
 #define W4A16_ENTRIES(X)                                                                                                   \
     X(w4a16_gemv_stream_bf16) X(w4a16_gemm_stream_bf16) X(w4a16_gemm_stream_best_scratch_bytes) X(w4a16_gemm_stream_scratch_bf16) \
     X(w4a16_q4nx_gemv_stream_bf16) X(w4a16_q4nx_gemm_stream_best_scratch_bytes) X(w4a16_q4nx_gemm_stream_scratch_bf16)
@@ -263,8 +262,8 @@ struct LatentLayer {
             must(dense.dlm_latent_prefill(p.dt, &shape, &r, kv.data_ptr(), kv.size(1), sink.data_ptr<float>(), out.data_ptr(), out_width, p.stream));
             return out;
         }
-        const int64_t rows = M * H, blocks = (pos + M + 31) / 32;   // (dense.latent_splits)
-        const int nsplit = (int)std::max<int64_t>(1, std::min({(int64_t)256, 512 / ((rows + 15) / 16), blocks, (int64_t)std::nearbyint(std::sqrt((double)(512 * blocks) / (double)rows))}));
+        const int64_t rows = M * H;
+        const int nsplit = dense.dlm_latent_splits(shape.heads, (int)M, pos + M);
         const Tensor qa = p.elems(rows, shape.rank + shape.rot), part_o = p.floats({rows, nsplit, shape.rank}), part_ml = p.floats({rows, nsplit, 2}), out = result();
         const char *uk = static_cast<const char *>(w_ukv.data_ptr());
         must(dense.dlm_latent_absorb(p.dt, &shape, &r, uk, qa.data_ptr(), p.stream));
@@ -393,9 +392,8 @@ struct MixedLayer {
             must(dense.dlm_head_prepare(p.dt, &heads, &r, q.data_ptr(), p.stream));
             if (!few) {
                 must(dense.dlm_head_prefill(p.dt, &heads, &r, q.data_ptr(), out.data_ptr(), ldo, p.stream));
-            } else {   // (dense.head_splits)
-                const int64_t tiles = heads.kv_heads * ((M * (heads.heads / heads.kv_heads) + 15) / 16), blocks = (std::min<int64_t>(pos + M, heads.window + M - 1) + 31) / 32 + 1;
-                const int n = (int)std::max<int64_t>(1, std::min({(int64_t)256, 512 / tiles, blocks}));
+            } else {
+                const int n = dense.dlm_head_splits(heads.heads, heads.kv_heads, heads.window, (int)M, pos + M);
                 const Tensor part_o = p.floats({M * heads.heads, n, heads.vdim}), part_ml = p.floats({M * heads.heads, n, 2});
                 must(dense.dlm_head_decode(p.dt, &heads, &r, q.data_ptr(), n, part_o.data_ptr<float>(), part_ml.data_ptr<float>(), p.stream));
                 must(dense.dlm_head_merge(p.dt, &heads, &r, n, part_o.data_ptr<float>(), part_ml.data_ptr<float>(), out.data_ptr(), ldo, p.stream));

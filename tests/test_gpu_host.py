@@ -97,7 +97,7 @@ def test_other_threads_run_while_a_call_launches():
     (Nothing is launched.)"""
     from air_hip import _lib, ops
     held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
-    asked = ("_slices", "gemm_parts", "_tile_rows", "_max_tiles", "gemv_keys", "_supported", "_bytes")   # (these launch nothing)
+    asked = ("_slices", "_splits", "gemm_parts", "_tile_rows", "_max_tiles", "gemv_keys", "_supported", "_bytes")   # (these launch nothing)
     stream = torch.cuda.current_stream().cuda_stream
     models = [mod._model(config, 5, torch.bfloat16)[0] for mod, config in ((tk, KUVONEX_MIXED), (ts, SITIRAX_MIXED))]
     w = ops.repack_stream(*map(dev, make_awq(256, 128, seed=1)))

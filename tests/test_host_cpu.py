@@ -537,3 +537,23 @@ def test_a_model_with_a_tail_of_its_own():
 
     assert Kept.tail_intake is None and Scaled.tail_intake is None and KuvonexModel.tail_intake == dense.FINAL
     assert Longer.tail_intake == SitiraxModel.tail_intake == dense.NORMED
+
+
+def test_splits_of_the_keys():
+    """One rule for passes in Python and in native code: what the operators have always launched."""
+    lib = _lib.load_dense_library()
+    lengths = [1, 2, 17, 31, 32, 33, 64, 100, 300, 511, 513, 1000, 2048, 4097, 10000, 32768, 65537, 1 << 20]
+    for heads in (1, 2, 3, 4, 8, 12, 16, 24, 32, 64, 128, 255):
+        for M in (1, 2, 3, 5, 8, 16, 17, 33, 64, 1000):
+            rows = M * heads
+            for total in lengths:
+                blocks = (total + 31) // 32
+                assert lib.dlm_latent_splits(heads, M, total) == max(1, min(256, 512 // ((rows + 15) // 16), blocks, round((512 * blocks / rows) ** 0.5))), (heads, M, total)
+            for kv_heads in {1, heads, max(1, heads // 4)}:
+                if heads % kv_heads:
+                    continue
+                tiles = kv_heads * ((M * (heads // kv_heads) + 15) // 16)
+                for window in (1, 64, 1000, 1 << 30):
+                    for total in lengths:
+                        assert lib.dlm_head_splits(heads, kv_heads, window, M, total) == max(1, min(256, 512 // tiles, (min(total, window + M - 1) + 31) // 32 + 1))
+    assert lib.dlm_latent_splits(0, 1, 5) == lib.dlm_head_splits(4, 0, 5, 1, 5) == 1
