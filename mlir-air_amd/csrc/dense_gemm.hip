@@ -321,6 +321,7 @@ __device__ __forceinline__ void wide_tiles(const GemmKernelArgs<bf16> &p, char *
     constexpr int CA = BM / 32, CW = BN / 32;             // copies of a wave and K-step
     constexpr int CA0 = CA / 2, CW0 = (CW + 1) / 2;
     constexpr int kSideA = BM * kRowBytes, kSideW = BN * kRowBytes;
+    static_assert(!wide_loops(NT, EPI) || 4 * (kWideStore / 2) <= kSideW, "rows on their way out fit the buffer that no copy goes to");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
@@ -463,7 +464,7 @@ __device__ __forceinline__ void wide_tiles(const GemmKernelArgs<bf16> &p, char *
                 at_w[ks] += ahead;
             }
             // second half; A two K-steps on
-            quarter<H1, wide_loops(NT, EPI)>(acc + H0, w1, a1, [&](int n) {
+            quarter<H1, true>(acc + H0, w1, a1, [&](int n) {
                 if (const int r = read_behind(n, 8 * H1, H0 + 8); r >= 0) {
                     if (r < H0) w0[r] = read(at_w[0], r);
                     else a0[r - H0] = read(at_a[0], r - H0);
