@@ -170,3 +170,16 @@ SITIRAX_MIXED = sitirax_config([
     sitirax_delta(heads=2, kv_heads=1, dim=40, vdim=72, conv=5),
     sitirax_parallel(heads=2, kv_heads=2, dim=72, vdim=24, window=70, scale=0.4, right_heads=4, right_dim=72, right_vdim=8, ff=24),
 ], vocab=67, width=72)
+
+
+def items_of_64(heads, M, total, window=0):
+    """The rule by which launches of the larger heads take 64 queries to a workgroup instead of 128."""
+    blocks = [(min(f + 64, total) + 63) // 64 - ((f - window + 1) // 64 if window and f >= window else 0) for f in range(total - M, total, 64)]
+    return sum(blocks) * heads <= 256 * max(blocks)
+
+
+def each_head_close(got, want, heads, tol, what):
+    """Every head of every row against its own size."""
+    got, want = got.double().cpu().numpy().reshape(len(want), heads, -1), want.reshape(len(want), heads, -1)
+    off = np.linalg.norm(got - want, axis=2) / np.linalg.norm(want, axis=2)
+    assert np.isfinite(got).all() and off.max() <= tol, (what, off.max(), np.unravel_index(off.argmax(), off.shape))

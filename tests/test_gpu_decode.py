@@ -264,9 +264,9 @@ def test_decode_attention_whole_and_in_chunks(ops, n_heads, n_kv, hd, positions)
 
 
 @pytest.mark.parametrize("n_heads,n_kv,hd,H,max_seq,positions", [
-    (32, 8, 128, 14336, 2048, [0, 63, 64, 500, 2047]),   # Llama-3-8B layer: fused from position 64 on (2 .. 32 chunks)
-    (32, 8, 64, 8192, 2048, [100, 2047]),                # Llama-3.2-1B layer
-    (8, 2, 64, 1024, 300, [10, 299]),                    # small E
+    (32, 8, 128, 14336, 2048, [0, 63, 64, 255, 256, 500, 2047]),   # Llama-3-8B layer: whole up to 256 positions, then 5 .. 32 chunks that the O projection merges
+    (32, 8, 64, 8192, 2048, [100, 383, 384, 2047]),                # Llama-3.2-1B layer: whole up to 384, then 7 .. 32 chunks
+    (8, 2, 64, 1024, 450, [10, 299, 383, 384, 449]),               # small E
 ])
 def test_attention_and_block_in_one_call_equal_the_two_calls(ops, n_heads, n_kv, hd, H, max_seq, positions):
     """w4a16_decode_attn_o_gemv_ffn_bf16 against w4a16_decode_attention_bf16 + w4a16_o_gemv_ffn_bf16: the same output bit
@@ -302,7 +302,7 @@ def test_attention_and_block_in_one_call_equal_the_two_calls(ops, n_heads, n_kv,
 def test_sum_of_squares_chained_into_the_next_norm(ops, n_heads, n_kv, hd, H):
     """The block's y_sumsq is the sum of squares of its bf16 output per 256-column tile, and w4a16_rms_gemv fed with it
     equals the plain call up to the summation order of the mean (one-ulp flips of the normalised vector)."""
-    E, pos, max_seq = n_heads * hd, 70, 128
+    E, pos, max_seq = n_heads * hd, 400, 512   # (attention in chunks)
     rng = np.random.default_rng(E + H)
     small = lambda w: (w[0], w[1], (w[2].float() * 0.05).to(torch.bfloat16))
     wo, wg, wu, wd = (small(tuple(map(dev, make_awq(a, b, seed=80 + i)))) for i, (a, b) in enumerate([(E, E), (E, H), (E, H), (H, E)]))

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import KUVONEX_MIXED, kuvonex_config, kuvonex_layer, kuvonex_weights, kuvonex_write
+from helpers import KUVONEX_MIXED, each_head_close, items_of_64, kuvonex_config, kuvonex_layer, kuvonex_weights, kuvonex_write
 from oracle import kuvonex as okv
 
 pytestmark = pytest.mark.gpu
@@ -384,13 +384,26 @@ def test_latent_attention(dense, dtype, sizes, form):
 
 @pytest.mark.parametrize("T,cut", [(1100, 256), (1025, 65)])
 def test_latent_attention_of_many_heads_whole_and_in_portions(dense, T, cut):
-    """Items of 128 queries, which many heads with many tokens take, against those of 64 that portions take: each is within 2^-8 of the exact result (weights and
-    outputs in bf16, 2^-9 each), by the norm of a row."""
+    """Items of 128 queries, which many heads with many tokens take, against those of 64 that portions take, by the norm of a row: the two differ by what weights and
+    outputs are rounded to, 2^-9 each on either side.  (Against the exact result, head by head: the next test.)"""
     say("latent attention, 64 heads", T, cut)
     x = Latents(dense, (64, 128, 64, 128, 64), T, BF16, seed=T)
     whole = x.run("rows", 0, T).double()
     parts = torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]).double()
     assert bool(whole.isfinite().all()) and bool(((whole - parts).norm(dim=1) <= 2.0 ** -7 * whole.norm(dim=1)).all())
+
+
+@pytest.mark.parametrize("heads,T", [(128, 330), (64, 1000)])
+def test_latent_attention_by_items_of_128_and_of_64_queries(dense, heads, T):
+    """Both kernels of heads of 128 + 64 / 128 against the plain result, far keys around the edges of blocks of 64 keys and of items.  2^-5 a head: queries, keys and
+    latents are bf16, so a score of size 8 is off by up to 8 / 2^9 and its weight by 2^-6; keys, values, weights and outputs are rounded to 2^-9 each."""
+    assert not items_of_64(heads, T, T) and items_of_64(heads, 70, T)
+    far = [(40, 0), (64, 31), (65, 32), (127, 64), (128, 63), (129, 65), (191, 191), (192, 127), (255, 128), (256, 193), (319, 255), (320, 256), (329, 1), (328, 327)]
+    x = Latents(dense, (heads, 128, 64, 128, 64), T, BF16, seed=T, far=far)
+    want = x.want()
+    for cut in (T, 70):
+        say("latent attention, items", heads, T, cut)
+        each_head_close(torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]), want, heads, 2.0 ** -5, cut)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])

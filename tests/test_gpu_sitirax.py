@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import SITIRAX_MIXED, sitirax_config, sitirax_delta, sitirax_parallel, sitirax_weights, sitirax_write
+from helpers import SITIRAX_MIXED, each_head_close, items_of_64, sitirax_config, sitirax_delta, sitirax_parallel, sitirax_weights, sitirax_write
 from oracle import sitirax as ost
 
 pytestmark = pytest.mark.gpu
@@ -218,13 +218,34 @@ def test_windowed_attention(dense, dtype, sizes, form):
 @pytest.mark.parametrize("sizes", [(64, 8, 128, 128, 1000), (64, 8, 128, 128, 768), (64, 16, 64, 64, 1000)])
 @pytest.mark.parametrize("T,cut", [(1100, 256), (1025, 65)])
 def test_windowed_attention_of_many_heads_whole_and_in_portions(dense, sizes, T, cut):
-    """Items of 128 queries (long windows, many heads and tokens) and of 64 (portions): each is within 2^-8 of the exact result, by the norm of a row."""
+    """Items of 128 queries (long windows, many heads and tokens) and of 64 (portions), by the norm of a row: the two differ by what weights and outputs are rounded
+    to, 2^-9 each on either side.  (Against the exact result, head by head: the next test.)"""
     say("windowed attention, many heads", sizes, T, cut)
     x = Heads(dense, sizes, T, BF16, 1152, seed=T)
     whole = x.run("rows", 0, T).double()
     x.cache.fill_(float("nan"))
     parts = torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]).double()
     assert bool(whole.isfinite().all()) and bool(((whole - parts).norm(dim=1) <= 2.0 ** -7 * whole.norm(dim=1)).all())
+
+
+@pytest.mark.parametrize("sizes,T,items", [((64, 8, 128, 128, 769), 900, 128), ((64, 8, 128, 128, 1000), 1100, 128), ((64, 8, 128, 128, 768), 900, 64),
+                                           ((64, 16, 64, 64, 1000), 900, 64)])
+def test_windowed_attention_by_items_of_128_and_of_64_queries(dense, sizes, T, items):
+    """Heads of 128 / 128 by either kernel, of 64 / 64 by theirs, against the plain result, far keys around the edges of the window, of blocks of 64 keys and of items.
+    2^-5 a head: a component of a query or key that is rounded the other way moves a score by 30 / 64 x 3 x 3 / 2^8 = 2^-5.9 at most (heads of 64), weights and
+    outputs are rounded to 2^-9 each."""
+    heads, window = sizes[0], sizes[4]
+    assert (items == 128) == (sizes[2] == 128 and window > 768 and not items_of_64(heads, T, T, window)) and items_of_64(heads, 70, T, window)
+    far = []
+    for i, j in borders(window, T) + [(127, 64), (128, 63), (255, 128), (256, 191), (319, 255), (383, 320), (384, 256), (511, 448), (639, 127), (640, 1), (767, 0), (768, 704), (895, 831)]:
+        if i < T and not any(i == a or j == b for a, b in far):
+            far.append((i, j))
+    x = Heads(dense, sizes, T, BF16, 1152, seed=T, far=far)
+    want = x.want()
+    for cut in (T, 70):
+        say("windowed attention, items", sizes, T, cut)
+        x.cache.fill_(float("nan"))
+        each_head_close(torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]), want, heads, 2.0 ** -5, cut)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
