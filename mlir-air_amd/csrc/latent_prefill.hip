@@ -404,15 +404,34 @@ PrefillArgs<T> args_of(const HeadShape &s, const HeadRows &r, const void *q, voi
 // 128 tokens 12.3 / 8.4, 1024 33.0 / 26.3, 1500 45.5 / 36.9, 3000 81.1 / 112.8, 500 behind 500 31.6 / 24.1, 1000 behind 3000 104.1 / 94.0, 2048 behind 2048 107.9 / 145.9; 64 heads: 300
 // 16.1 / 13.5, 1024 47.7 / 61.6.  (On the line, 16 heads and 2048 tokens, 58.9 / 54.1 alone, but 3 us more between a model's products.)
 template <class T>
+long item_blocks(const PrefillArgs<T> &p, long first) {   // blocks of 64 keys of the item of 64 queries from position `first` on
+    const long end = std::min<long>(first + 64, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
+    return (end + 63) / 64 - unseen;
+}
+template <class T>
 bool few_queries(const PrefillArgs<T> &p) {
-    long longest = 0, all = 0;   // blocks of 64 keys
+    long longest = 0, all = 0;
     for (long first = p.total - p.M; first < p.total; first += 64) {
-        const long end = std::min<long>(first + 64, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
-        const long blocks = (end + 63) / 64 - unseen;
+        const long blocks = item_blocks(p, first);
         longest = std::max(longest, blocks);
         all += blocks;
     }
     return all * p.heads <= 256 * longest;
+}
+
+// Whether heads of 64 / 64 take 128 queries to a workgroup after all: 512 items of 64 or fewer, two to a CU, of which more than 256 are nearly as long as the longest.  Two long
+// ones on a CU take 1.02 us a block of keys together, one alone 0.76, an item of 128 queries 0.93; where lengths differ a long one shares with short ones.  us, 128 / 64 queries:
+// 8 heads, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16 heads, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3; but 6 heads, window
+// 2048, 4096 tokens 31.0 / 27.6 (384 and 210), 16 heads, window 1024, 3000 tokens 32.2 / 24.4 (752 items).  Over 352 sizes 64 queries were 1.195 times as fast as 128, so 1.199, and more than
+// 2 % slower at 35 and 6 of them.  Windows of few blocks take as long either way.
+template <class T>
+bool even_round(const PrefillArgs<T> &p) {
+    const long items = (p.M + 63) / 64 * (long)p.heads;
+    if (items <= 256 || items > 512) return false;
+    long longest = 0, tall = 0;
+    for (long first = p.total - p.M; first < p.total; first += 64) longest = std::max(longest, item_blocks(p, first));
+    for (long first = p.total - p.M; first < p.total; first += 64) tall += 10 * item_blocks(p, first) >= 9 * longest;
+    return longest >= 14 && tall * p.heads > 256;
 }
 
 }  // namespace
@@ -458,10 +477,10 @@ hipError_t launch_head_prefill(int dtype, const HeadShape &s, const HeadRows &r,
     const PrefillArgs<bf16> p = args_of<bf16>(s, r, q, out, ldo);
     if ((double)s.ring * (s.dim + s.vdim) * sizeof(bf16) < 4e9) {
         // (windows of few blocks are mostly start and end, which the smaller items share a CU for: 16 to 64 heads, 1024 to 4096 tokens, windows of 64 to 256 1.03 to 1.4 times
-        // as fast, of 384 to 700 0.99 to 1.3; heads of 64 at any window 0.96 to 1.5, 1.2 on average)
+        // as fast, of 384 to 700 0.99 to 1.3)
         if (nq == 4 && nv == 8)
             return p.window <= 768 || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
-        if (nq == 2 && nv == 4) return launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
+        if (nq == 2 && nv == 4) return even_round(p) ? launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream) : launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false, true>(p, stream);
     if (nq <= 8 && nv <= 8) return launch<bf16, 8, 8, 1, 64, 1, false, true>(p, stream);

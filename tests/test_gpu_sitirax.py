@@ -248,6 +248,23 @@ def test_windowed_attention_by_items_of_128_and_of_64_queries(dense, sizes, T, i
         each_head_close(torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]), want, heads, 2.0 ** -5, cut)
 
 
+@pytest.mark.parametrize("cut", [1000, 1300 - 257])
+def test_windowed_attention_of_64_channels_by_items_of_128_queries(dense, cut):
+    """A portion behind a whole window: 320 items of 64 queries (5 a head), all of 17 or 18 blocks of keys, so more than a CU each and no more than two.  The tolerance is
+    that of the test above."""
+    sizes, T = (64, 16, 64, 64, 1000), 1300
+    heads, window = sizes[0], sizes[4]
+    blocks = [(min(f + 64, T) + 63) // 64 - (f - window + 1) // 64 for f in range(cut, T, 64)]
+    assert 256 < heads * len(blocks) <= 512 and min(blocks) >= 0.9 * max(blocks) >= 14
+    far = [(cut - 1, 3), (cut, cut - 999), (cut + 1, cut - 64), (cut + 63, cut + 62), (cut + 64, 127 + cut // 64), (cut + 127, cut + 65), (cut + 128, 320), (cut + 191, cut - 800),
+           (T - 2, T - 1001), (T - 1, T - 1002 + 2)]
+    x = Heads(dense, sizes, T, BF16, 1344, seed=cut, far=far)
+    want = x.want()
+    say("windowed attention, a portion behind a window", cut)
+    got = torch.cat([x.run("rows", 0, cut), x.run("rows", cut, T)])
+    each_head_close(got, want, heads, 2.0 ** -5, cut)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("sizes", [(4, 2, 24, 40, 37), (8, 2, 128, 128, 65), (3, 3, 64, 64, 64), (2, 1, 32, 32, 1)])
 def test_ring_of_rows_and_positions_on_the_device(dense, dtype, sizes):
