@@ -404,8 +404,8 @@ PrefillArgs<T> args_of(const HeadShape &s, const HeadRows &r, const void *q, voi
 // 128 tokens 12.3 / 8.4, 1024 33.0 / 26.3, 1500 45.5 / 36.9, 3000 81.1 / 112.8, 500 behind 500 31.6 / 24.1, 1000 behind 3000 104.1 / 94.0, 2048 behind 2048 107.9 / 145.9; 64 heads: 300
 // 16.1 / 13.5, 1024 47.7 / 61.6.  (On the line, 16 heads and 2048 tokens, 58.9 / 54.1 alone, but 3 us more between a model's products.)
 template <class T>
-long item_blocks(const PrefillArgs<T> &p, long first) {   // blocks of 64 keys of the item of 64 queries from position `first` on
-    const long end = std::min<long>(first + 64, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
+long item_blocks(const PrefillArgs<T> &p, long first, long queries = 64) {   // blocks of 64 keys of the item of so many queries from position `first` on
+    const long end = std::min<long>(first + queries, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
     return (end + 63) / 64 - unseen;
 }
 template <class T>
@@ -419,19 +419,21 @@ bool few_queries(const PrefillArgs<T> &p) {
     return all * p.heads <= 256 * longest;
 }
 
-// Whether heads of 64 / 64 take 128 queries to a workgroup after all: 512 items of 64 or fewer, two to a CU, of which more than 256 are nearly as long as the longest.  Two long
-// ones on a CU take 1.02 us a block of keys together, one alone 0.76, an item of 128 queries 0.93; where lengths differ a long one shares with short ones.  us, 128 / 64 queries:
-// 8 heads, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16 heads, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3; but 6 heads, window
-// 2048, 4096 tokens 31.0 / 27.6 (384 and 210), 16 heads, window 1024, 3000 tokens 32.2 / 24.4 (752 items).  Over 352 sizes 64 queries were 1.195 times as fast as 128, so 1.199, and more than
-// 2 % slower at 35 and 6 of them.  Windows of few blocks take as long either way.
+// Whether windowed heads that otherwise take 64 queries to a workgroup take 128 after all: 512 items of 64 or fewer, two to a CU, of which more than 256 are nearly as long as the
+// longest.  Two long ones on a CU take 1.02 us a block of keys together, one alone 0.76, an item of 128 queries 0.93 (heads of 64); where lengths differ a long one shares with short ones.
+// Its two wave sets take blocks in turn, so an odd number costs it one more, which only long items make up for.  us, 128 / 64 queries,
+// heads of 64: 8, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3; but 6, window 2048, 4096
+// tokens 31.0 / 27.6 (384 and 210), 16, window 1024, 3000 tokens 32.2 / 24.4 (752 items).  Heads of 128, 16 of them, 2048 tokens: windows of 576 22.1 / 21.6, 640 22.3 / 22.9, 704 24.6 / 23.2,
+// 768 24.5 / 25.7; below 10 blocks both take as long.
 template <class T>
 bool even_round(const PrefillArgs<T> &p) {
-    const long items = (p.M + 63) / 64 * (long)p.heads;
+    const long items = (p.M + 63) / 64 * (long)p.heads, start = p.total - p.M;
     if (items <= 256 || items > 512) return false;
-    long longest = 0, tall = 0;
-    for (long first = p.total - p.M; first < p.total; first += 64) longest = std::max(longest, item_blocks(p, first));
-    for (long first = p.total - p.M; first < p.total; first += 64) tall += 10 * item_blocks(p, first) >= 9 * longest;
-    return longest >= 14 && tall * p.heads > 256;
+    long longest = 0, tall = 0, longest128 = 0;
+    for (long first = start; first < p.total; first += 64) longest = std::max(longest, item_blocks(p, first));
+    for (long first = start; first < p.total; first += 64) tall += 10 * item_blocks(p, first) >= 9 * longest;
+    for (long first = start; first < p.total; first += 128) longest128 = std::max(longest128, item_blocks(p, first, 128));
+    return longest >= (longest128 % 2 ? 22 : 10) && tall * p.heads > 256;
 }
 
 }  // namespace
@@ -479,7 +481,7 @@ hipError_t launch_head_prefill(int dtype, const HeadShape &s, const HeadRows &r,
         // (windows of few blocks are mostly start and end, which the smaller items share a CU for: 16 to 64 heads, 1024 to 4096 tokens, windows of 64 to 256 1.03 to 1.4 times
         // as fast, of 384 to 700 0.99 to 1.3)
         if (nq == 4 && nv == 8)
-            return p.window <= 768 || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
+            return (p.window <= 768 && !even_round(p)) || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
         if (nq == 2 && nv == 4) return even_round(p) ? launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream) : launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false, true>(p, stream);

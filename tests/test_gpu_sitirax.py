@@ -248,19 +248,18 @@ def test_windowed_attention_by_items_of_128_and_of_64_queries(dense, sizes, T, i
         each_head_close(torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]), want, heads, 2.0 ** -5, cut)
 
 
-@pytest.mark.parametrize("cut", [1000, 1300 - 257])
-def test_windowed_attention_of_64_channels_by_items_of_128_queries(dense, cut):
-    """A portion behind a whole window: 320 items of 64 queries (5 a head), all of 17 or 18 blocks of keys, so more than a CU each and no more than two.  The tolerance is
-    that of the test above."""
-    sizes, T = (64, 16, 64, 64, 1000), 1300
-    heads, window = sizes[0], sizes[4]
-    blocks = [(min(f + 64, T) + 63) // 64 - (f - window + 1) // 64 for f in range(cut, T, 64)]
-    assert 256 < heads * len(blocks) <= 512 and min(blocks) >= 0.9 * max(blocks) >= 14
-    far = [(cut - 1, 3), (cut, cut - 999), (cut + 1, cut - 64), (cut + 63, cut + 62), (cut + 64, 127 + cut // 64), (cut + 127, cut + 65), (cut + 128, 320), (cut + 191, cut - 800),
-           (T - 2, T - 1001), (T - 1, T - 1002 + 2)]
-    x = Heads(dense, sizes, T, BF16, 1344, seed=cut, far=far)
+@pytest.mark.parametrize("sizes,cut", [((64, 16, 64, 64, 1000), 1000), ((64, 16, 64, 64, 1000), 1024), ((64, 8, 128, 128, 768), 832), ((64, 8, 128, 128, 640), 1024)])
+def test_windowed_attention_of_a_portion_by_items_of_128_queries(dense, sizes, cut):
+    """A portion behind a whole window: 320 items of 64 queries (5 a head), about as long, so more than one a CU and no more than two, and an even number of blocks of keys for
+    128 queries.  The tolerance is that of the test above."""
+    heads, window, T = sizes[0], sizes[4], cut + 300
+    blocks = lambda n: [(min(f + n, T) + 63) // 64 - max(f - window + 1, 0) // 64 for f in range(cut, T, n)]
+    assert 256 < heads * len(blocks(64)) <= 512 and min(blocks(64)) >= 0.9 * max(blocks(64)) >= 9 and max(blocks(128)) % 2 == 0
+    far = [(cut - 1, 300), (cut, cut - window + 1), (cut + 1, cut - 64), (cut + 63, cut + 62), (cut + 64, cut - 513), (cut + 127, cut + 65), (cut + 128, cut - 300), (cut + 191, cut - 400),
+           (T - 2, T - 1 - window), (T - 1, T - 127)]
+    x = Heads(dense, sizes, T, BF16, -(-T // 64) * 64, seed=cut, far=far)
     want = x.want()
-    say("windowed attention, a portion behind a window", cut)
+    say("windowed attention, a portion behind a window", sizes, cut)
     got = torch.cat([x.run("rows", 0, cut), x.run("rows", cut, T)])
     each_head_close(got, want, heads, 2.0 ** -5, cut)
 
