@@ -307,35 +307,35 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         half ^= 1;
     }
 
-    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, in the same order, operand by operand from memory.
+    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, a tile at a time in the same order, operand by operand from memory.  Where that stands decides
+    // how the compiler schedules the loop above: here for two tiles side by side, at the stores for one and three (15 forms and 6 sizes, against the kernel without: 0.98 to 1.04, 1.01
+    // for what the sizes take; all tiles at once behind the loop in every form 0.98 to 1.05 and 1.006).
+    bool over = false;
+    auto again = [&](int rt, int c) {
+        typedef const __attribute__((address_space(1))) uint32_t *Word;
+        const gptr tile = (gptr)(p.w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
+        const uint16_t *x = p.x + (size_t)(m0 + min(16 * rt + ln, rows - 1)) * p.K + 8 * lg;
+        floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k = 0; k < 4 * p.G; ++k) {   // K-steps (slices are for the exact modes)
+            const int g = k >> 2;
+            const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
+            const uint32_t cell = lane16 + blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes + 4 * (k & 3), word = 16 * ln + blk + 64 * (g & 12) + 4 * (g & 3);
+            float s, low;
+            decode_md(*reinterpret_cast<Word>(tile + word), s, low);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(x + 32 * k), dequant_operand(*reinterpret_cast<Word>(tile + cell), s, low), acc, 0, 0, 0);
+        }
+        return acc;
+    };
     if constexpr (MODE == kSmAwqRounded) {
-        static_assert(KW == 1, "a wave has all of the slice");
-        bool over = false;
+        static_assert(KW == 1, "a wave has all of K");
 #pragma unroll
         for (int c = 0; c < NT; ++c) over |= awq_overflowed(Y[0][c][0], Y[RT - 1][c][0]);
-        if (__ballot(over)) {
+        if (NT == 2 && __ballot(over)) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int c = 0; c < NT; ++c) Y[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-            for (int k = 4 * g_lo; k < 4 * g_hi; ++k) {   // K-steps
-                const int g = k >> 2;
-                const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
-                const uint32_t cell = lane16 + blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes + 4 * (k & 3), word = 16 * ln + blk + 64 * (g & 12) + 4 * (g & 3);
-#pragma unroll
-                for (int c = 0; c < NT; ++c) {
-                    typedef const __attribute__((address_space(1))) uint32_t *Word;
-                    float s, low;
-                    decode_md(*reinterpret_cast<Word>(tb[c] + word), s, low);
-                    const bf16x8 b = dequant_operand(*reinterpret_cast<Word>(tb[c] + cell), s, low);
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-                        const bf16x8 x = *reinterpret_cast<const bf16x8 *>(p.x + (size_t)(m0 + min(16 * rt + ln, rows - 1)) * p.K + 32 * k + 8 * lg);
-                        Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b, Y[rt][c], 0, 0, 0);
-                    }
-                }
-            }
+                for (int c = 0; c < NT; ++c) Y[rt][c] = again(rt, c);
         }
     }
 
@@ -368,6 +368,17 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
             for (int c = 0; c < NT; ++c)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) yt[(16 * rt + 4 * lg + i) * LDP + (NT * wq + c) * kWsTileCols + ln] = Y[rt][c][i];
+    }
+    if constexpr (MODE == kSmAwqRounded && NT != 2) {
+        if (__ballot(over)) {
+#pragma unroll 1
+            for (int n = 0; n < RT * NT; ++n) {
+                const int rt = n / NT, c = n % NT;
+                const floatx4 acc = again(rt, c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) yt[(16 * rt + 4 * lg + i) * LDP + (NT * wq + c) * kWsTileCols + ln] = acc[i];
+            }
+        }
     }
     __syncthreads();
     const int col0 = set * CW, ncols = min(CW, p.N - col0);   // a multiple of 16
