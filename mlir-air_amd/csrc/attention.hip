@@ -11,8 +11,8 @@
 //           positions per load; each lane group keeps a private online-softmax state
 //           (m, l, acc[8]) per query head and the states are merged at the end: across lane
 //           groups with shuffles, across waves through LDS, across chunks by the combine kernel
-//   the chunk that holds `pos` first rotates K, stores K and V of the new token into the caches,
-//   and then reads them back like any other position
+//   the chunk that holds `pos` rotates K, takes the new token's K and V from registers and stores
+//   them into the caches at its end, once per KV head
 //
 // Rounding points follow the reference's decode step: Q and K are rounded to bf16 after RoPE,
 // scores, softmax and the weighted sum are fp32, the output is rounded to bf16 once.

@@ -458,7 +458,8 @@ hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t str
 
 // The time of a launch on the GPU.  Exact modes: fitted to 3900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows,
 // every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 0.5 % more than the best of them on average, 10 % at worst); rounded: to
-// 2500 (13 matrices, 65 .. 3500 rows; rms error 10 %, 24 % at worst).  Microseconds of start, of a workgroup, and of a step alone on the chip
+// 2500 (13 matrices, 65 .. 3500 rows; rms error 10 %, 24 % at worst) of kernels with 23 instructions a dequantisation, which the AWQ order's no longer have: they
+// take up to 9 % less than this says, the tiled kernel that they are weighed against (0.95 of its estimate, which is from then as well) up to 2 %.  Microseconds of start, of a workgroup, and of a step alone on the chip
 // (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of one of two.  The launch that
 // adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
 struct SmCost {
