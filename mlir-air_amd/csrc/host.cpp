@@ -427,6 +427,7 @@ std::optional<Tensor> mixed_rows(py::list layers, py::list caches, const Tensor 
                                  int64_t steps_most, float unit_eps, uintptr_t stream) {
     if (!on_gpu(embed) || embed.dim() != 2 || !on_gpu(tokens) || tokens.scalar_type() != at::kInt || tokens.numel() < 1 || pos < 0) return std::nullopt;
     if (embed.scalar_type() != at::kBFloat16 && embed.scalar_type() != at::kFloat) return std::nullopt;
+    if (tokens.numel() == 1) return std::nullopt;   // (mixers of one token share launches, which are the operators')
     const Pass p(tokens.numel(), embed, stream);
     const int64_t M = p.M, W = embed.size(1);
     std::vector<MixedLayer> ls(layers.size());
