@@ -421,19 +421,19 @@ bool few_queries(const PrefillArgs<T> &p) {
 
 // Whether windowed heads that otherwise take 64 queries to a workgroup take 128 after all: 512 items of 64 or fewer, two to a CU, of which more than 256 are nearly as long as the
 // longest.  Two long ones on a CU take 1.02 us a block of keys together, one alone 0.76, an item of 128 queries 0.93 (heads of 64); where lengths differ a long one shares with short ones.
-// Its two wave sets take blocks in turn, so an odd number costs it one more, which only long items make up for.  us, 128 / 64 queries,
-// heads of 64: 8, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3; but 6, window 2048, 4096
-// tokens 31.0 / 27.6 (384 and 210), 16, window 1024, 3000 tokens 32.2 / 24.4 (752 items).  Heads of 128, 16 of them, 2048 tokens: windows of 576 22.1 / 21.6, 640 22.3 / 22.9, 704 24.6 / 23.2,
-// 768 24.5 / 25.7; below 10 blocks both take as long.
+// us, 128 / 64 queries, heads of 64: 8, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3;
+// but 6, window 2048, 4096 tokens 31.0 / 27.6 (384 and 210), 16, window 1024, 3000 tokens 32.2 / 24.4 (752 items); below 17 blocks 0.95 to 1.01 times.  Heads of 128 (windows up to 768): 16
+// of them, 2048 tokens, windows of 640 22.1 / 22.9, 768 24.5 / 25.7, but 576 22.1 / 21.6, 704 24.6 / 23.2: the two wave sets of 128 queries take blocks in turn, so an odd number costs
+// them one more.
 template <class T>
-bool even_round(const PrefillArgs<T> &p) {
+bool even_round(const PrefillArgs<T> &p, bool wide) {
     const long items = (p.M + 63) / 64 * (long)p.heads, start = p.total - p.M;
     if (items <= 256 || items > 512) return false;
     long longest = 0, tall = 0, longest128 = 0;
     for (long first = start; first < p.total; first += 64) longest = std::max(longest, item_blocks(p, first));
     for (long first = start; first < p.total; first += 64) tall += 10 * item_blocks(p, first) >= 9 * longest;
     for (long first = start; first < p.total; first += 128) longest128 = std::max(longest128, item_blocks(p, first, 128));
-    return longest >= (longest128 % 2 ? 22 : 10) && tall * p.heads > 256;
+    return tall * p.heads > 256 && (wide ? longest >= 10 && longest128 % 2 == 0 : longest >= 17);
 }
 
 }  // namespace
@@ -481,8 +481,8 @@ hipError_t launch_head_prefill(int dtype, const HeadShape &s, const HeadRows &r,
         // (windows of few blocks are mostly start and end, which the smaller items share a CU for: 16 to 64 heads, 1024 to 4096 tokens, windows of 64 to 256 1.03 to 1.4 times
         // as fast, of 384 to 700 0.99 to 1.3)
         if (nq == 4 && nv == 8)
-            return (p.window <= 768 && !even_round(p)) || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
-        if (nq == 2 && nv == 4) return even_round(p) ? launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream) : launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
+            return (p.window <= 768 && !even_round(p, true)) || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
+        if (nq == 2 && nv == 4) return even_round(p, false) ? launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream) : launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false, true>(p, stream);
     if (nq <= 8 && nv <= 8) return launch<bf16, 8, 8, 1, 64, 1, false, true>(p, stream);

@@ -250,11 +250,12 @@ def test_windowed_attention_by_items_of_128_and_of_64_queries(dense, sizes, T, i
 
 @pytest.mark.parametrize("sizes,cut", [((64, 16, 64, 64, 1000), 1000), ((64, 16, 64, 64, 1000), 1024), ((64, 8, 128, 128, 768), 832), ((64, 8, 128, 128, 640), 1024)])
 def test_windowed_attention_of_a_portion_by_items_of_128_queries(dense, sizes, cut):
-    """A portion behind a whole window: 320 items of 64 queries (5 a head), about as long, so more than one a CU and no more than two, and an even number of blocks of keys for
-    128 queries.  The tolerance is that of the test above."""
+    """A portion behind a whole window: 320 items of 64 queries (5 a head), about as long, so more than one a CU and no more than two; blocks of keys enough (heads of 64) or an even
+    number for 128 queries (of 128).  The tolerance is that of the test above."""
     heads, window, T = sizes[0], sizes[4], cut + 300
     blocks = lambda n: [(min(f + n, T) + 63) // 64 - max(f - window + 1, 0) // 64 for f in range(cut, T, n)]
-    assert 256 < heads * len(blocks(64)) <= 512 and min(blocks(64)) >= 0.9 * max(blocks(64)) >= 9 and max(blocks(128)) % 2 == 0
+    assert 256 < heads * len(blocks(64)) <= 512 and min(blocks(64)) >= 0.9 * max(blocks(64))
+    assert max(blocks(64)) >= 17 if sizes[2] == 64 else max(blocks(64)) >= 10 and max(blocks(128)) % 2 == 0
     far = [(cut - 1, 300), (cut, cut - window + 1), (cut + 1, cut - 64), (cut + 63, cut + 62), (cut + 64, cut - 513), (cut + 127, cut + 65), (cut + 128, cut - 300), (cut + 191, cut - 400),
            (T - 2, T - 1 - window), (T - 1, T - 127)]
     x = Heads(dense, sizes, T, BF16, -(-T // 64) * 64, seed=cut, far=far)
