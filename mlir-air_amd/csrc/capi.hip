@@ -1181,7 +1181,7 @@ int w4a16_tune(const char *key, int value) {
         if (value < 0 || value > 2) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.splitk = value;
     } else if (!strcmp(key, "gemm_wsm_rt")) {
-        if (value == 1 || value > 7) return W4A16_ERR_TUNE;
+        if (value == 1 || value > 10) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.wsm_rt = value;
     } else if (!strcmp(key, "gemm_wsm_nt")) {
         if (value > 3) return W4A16_ERR_TUNE;

@@ -18,9 +18,16 @@
 //                into two bf16, and the minimum is an operand of its own: three MFMAs per K-step with every product exact, as s sum q x +
 //                min sum x has them.  (s q + min in two operands keeps 16 bits of it, which loses minima small against the scale.)
 //   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits, and a residual is
-//                added to the rounded product as its epilogue does
+//                added to the rounded product as its epilogue does.  KW = 1, and an accumulator's products follow each other, so what hides a wave's LDS reads and
+//                dequantisation are its own products: those of a K-step run beside the reads and the dequantisation of the next one (sm_interleave), across
+//                groups too, for which a group has landed one group ahead.  What bounds it then is issue, 4 cycles an instruction: a group of 5 x 3 tiles has 240
+//                vector, 60 matrix and 110 other ones.  Tall and wide forms (up to 10 x 2 and 7 x 3 tiles, one workgroup to a CU, rings of 160 KB) need the fewest.
+//                us before / with: 300 rows of 4096 x 11008 40.7 / 36.4 (5 x 3 tiles instead of 4 x 2), 256 of 4096 x 14336 41.0 / 35.4 (8 x 2), 160 of 4096 x 11008 28.4 / 27.1,
+//                300 of 14336 x 4096 68.0 / 62.9; 120 random products of 66 to 1400 rows 1.049 times as fast.  (Every instruction in its place by volatile asm, none behind one that it
+//                depends on: 38.3, 34.6, 27.3, 72: not taken.)
 //   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
 #include <algorithm>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -44,13 +51,32 @@ struct SmArgs {
     int sets, slices, blocks;      // column sets, slices of K, blocks of rows
 };
 
+// (rounded: two workgroups to a CU where three stages of each fit LDS, else one with all of it)
 // A step in LDS: the x tiles of its groups, then per wave its cells and its scale words ([64]: tile lane / 16, column lane % 16; Q4NX:
 // [NT][64], K-step lane / 16)
 constexpr int sm_wave_bytes(int nt, bool q4) { return nt * (int)kWsCellBytes + (q4 ? nt : 1) * 256; }
 constexpr int sm_stage(int rt, int nt, int kw, bool q4) { return kw * (16 * rt * 256 + 4 * sm_wave_bytes(nt, q4)); }
+constexpr bool sm_together(int rt, int nt, bool q4) { return 3 * sm_stage(rt, nt, 1, q4) <= kSmLds / 2; }
 constexpr int sm_ring(int rt, int nt, int kw, bool q4) {
-    const int n = ((kw == 1 ? kSmLds / 2 : kSmLds) - (q4 || rt > 4 ? 0 : 2 * kw * 16 * rt * 4)) / sm_stage(rt, nt, kw, q4);
+    const int n = ((kw == 1 && sm_together(rt, nt, q4) ? kSmLds / 2 : kSmLds) - (q4 || rt > 4 ? 0 : 2 * kw * 16 * rt * 4)) / sm_stage(rt, nt, kw, q4);
     return n < 4 ? n : 4;
+}
+
+// The compiler's schedule of P products: behind each its share of VALU vector instructions; the READS LDS reads behind the first half, so that they are there when the
+// next K-step begins; the COPIES requests, which may not pass them, behind the other.  (Reads behind all of the products, copies first: 300 x 4096 x 11008 38 us, 36.4 so.)
+template <int P, int VALU, int READS, int COPIES, int... I>
+__device__ __forceinline__ void sm_interleave(std::integer_sequence<int, I...>) {
+    auto one = [](auto n) __attribute__((always_inline)) {
+        constexpr int i = decltype(n)::value;
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        constexpr int E = P / 2;
+        constexpr int r = (i + 1 < E ? (i + 1) * READS / E : READS) - (i < E ? i * READS / E : READS);
+        constexpr int c = (i < E ? 0 : (i + 1 - E) * COPIES / (P - E)) - (i <= E ? 0 : (i - E) * COPIES / (P - E)), v = (i + 1) * VALU / P - i * VALU / P;
+        if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
+        if constexpr (v > 0) __builtin_amdgcn_sched_group_barrier(0x2, v, 0);
+        if constexpr (c > 0) __builtin_amdgcn_sched_group_barrier(0x20, c, 0);
+    };
+    (one(std::integral_constant<int, I>()), ...);
 }
 
 template <int RT, int NT, int KW, int MODE>
@@ -95,7 +121,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 
     // copy j of the wave: rows 4 q .. + 3 of its group's x, q = 4 j + wq; lane l fetches chunk (l % 16) ^ row % 16 of row l / 16
     const gptr xbase = scalar_ptr(p.x + (size_t)m0 * p.K);
-    uint32_t xoff[RT];   // (at most 111 rows: the host keeps K below 2^24)
+    uint32_t xoff[RT];   // (at most 127 rows: the host keeps K below 2^24; 2^23 with more)
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
         const int row = 4 * (4 * j + wq) + lg;
@@ -108,10 +134,13 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     auto copy4 = [&](gptr src, int dst) {
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)(lds + dst), 4, 0, 0);
     };
-    auto request = [&](int g, int stage) {
+    auto request_x = [&](int g, int stage, int j0, int j1) {
         const gptr xs = xbase + (size_t)g * 256;
 #pragma unroll
-        for (int j = 0; j < RT; ++j) copy16(xs + xoff[j], stage + x_lds + 1024 * (4 * j + wq));
+        for (int j = 0; j < RT; ++j)
+            if (j >= j0 && j < j1) copy16(xs + xoff[j], stage + x_lds + 1024 * (4 * j + wq));
+    };
+    auto request_w = [&](int g, int stage) {
         const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
         uint32_t cell = lane16 + (blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes), word = word_off + (blk + 64 * (g & 12) + 4 * (g & 3));
         asm volatile("" : "+v"(cell), "+v"(word));   // (a 32-bit sum: folds into the copies as their offset)
@@ -119,6 +148,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         for (int c = 0; c < NT; ++c) copy16(tb[c] + cell, stage + wave_lds + c * (int)kWsCellBytes);
 #pragma unroll
         for (int c = 0; c < MC; ++c) copy4(tb[c] + word, stage + wave_lds + NT * (int)kWsCellBytes + 256 * c);
+    };
+    auto request = [&](int g, int stage) {
+        request_x(g, stage, 0, RT);
+        request_w(g, stage);
     };
     auto cell_at = [&](int stage, int c) { return *reinterpret_cast<const u32x4 *>(lds + stage + wave_lds + c * (int)kWsCellBytes + 16 * lane); };
     auto word_at = [&](int stage, int c, int t) {   // (AWQ: t = 0)
@@ -291,6 +324,112 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     }
 
     int stage = 0, half = 0;
+    if constexpr (MODE >= kSmAwqRounded) {
+        // Products of K-step t from one side of a and b, while the other one is made.  Between K-steps 1 and 2 the next group has landed for everybody, and nobody
+        // reads the one before this any more: its stage is filled from there on.
+        bf16x8 a[2][RT], b[2][NT];
+        u32x4 cell[NT];
+        uint32_t word[NT][Q4 ? 4 : 1];
+        AwqScale d[NT];
+        auto read_a = [&](int at, int t, int side) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) a[side][rt] = operand_a(at, t, rt);
+        };
+        auto read_w = [&](int at) {
+#pragma unroll
+            for (int c = 0; c < NT; ++c) cell[c] = cell_at(at, c);
+#pragma unroll
+            for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int t = 0; t < (Q4 ? 4 : 1); ++t) word[c][t] = word_at(at, c, t);
+        };
+        auto scales = [&]() {
+            if constexpr (!Q4) {
+#pragma unroll
+                for (int c = 0; c < NT; ++c) d[c] = awq_scale(word[c][0]);
+            }
+        };
+        uint32_t last[NT], last_word[NT];   // of K-step 3, while the next group's are read
+        auto keep_last = [&]() {
+#pragma unroll
+            for (int c = 0; c < NT; ++c) {
+                last[c] = cell[c][3];
+                asm volatile("" : "+v"(last[c]));
+                if constexpr (Q4) {
+                    last_word[c] = word[c][Q4 ? 3 : 0];
+                    asm volatile("" : "+v"(last_word[c]));
+                }
+            }
+        };
+        auto dequant = [&](int t, int side) {
+#pragma unroll
+            for (int c = 0; c < NT; ++c) {
+                const uint32_t v = t == 3 ? last[c] : cell[c][t];
+                if constexpr (Q4) {
+                    float s, low;
+                    decode_md_q4(t == 3 ? last_word[c] : word[c][t], s, low);
+                    b[side][c] = dequant_operand(v, s, low);
+                } else {
+                    b[side][c] = dequant_operand_awq(v, d[c], nib_mask, high_mask, magic);
+                }
+            }
+        };
+        auto products = [&](int side) {
+#pragma unroll
+            for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[side][rt], b[side][c], Y[rt][c], 0, 0, 0);
+        };
+        auto interleave = [&](auto valu, auto reads, auto copies) {
+            constexpr int P = RT * NT, VALU = decltype(valu)::value, READS = decltype(reads)::value, COPIES = decltype(copies)::value;
+            sm_interleave<P, VALU, READS, COPIES>(std::make_integer_sequence<int, P>());
+        };
+        constexpr int kDq = NT * (Q4 ? 25 : 17);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * V) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read_w(0);
+        read_a(0, 0, 0);
+        scales();
+        dequant(0, 0);
+        for (int g = g_lo; g < g_hi; ++g) {
+#pragma unroll
+            for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
+            const int fill = stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
+            const int gn = min(g + R - 1, g_last);
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(stage, 1, 1);
+            dequant(1, 1);
+            products(0);
+            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(stage, 2, 0);
+            dequant(2, 0);
+            keep_last();
+            products(1);
+            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            __builtin_amdgcn_sched_barrier(0);
+            // the next group has landed for everybody, and nobody reads the one before this any more
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 3) * V) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            read_a(stage, 3, 1);
+            read_w(next);
+            dequant(3, 1);
+            products(0);
+            request_x(gn, fill, 0, RT);
+            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT + NT * (Q4 ? 5 : 2)>(), std::integral_constant<int, RT>());
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(next, 0, 0);
+            scales();
+            dequant(0, 0);
+            products(1);
+            request_w(gn, fill);
+            interleave(std::integral_constant<int, kDq + (Q4 ? 0 : 4 * NT)>(), std::integral_constant<int, RT>(), std::integral_constant<int, NT + MC>());
+            __builtin_amdgcn_sched_barrier(0);
+            stage = next;
+        }
+    } else {
     for (int g0 = g_lo; g0 < g_hi; g0 += KW) {
         // This step's requests and, for the sums, the next step's x have landed (younger ones: R - 2 steps, less that x); this wave is done
         // with the step before, and behind the barrier so is everybody.
@@ -305,6 +444,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         if (KW == 1 || g0 + kq < g_hi) multiply(half, stage, next);
         stage = next;
         half ^= 1;
+    }
     }
 
     // Scales from 2^117 on (wsdequant.h): the wave's columns once more, a tile at a time in the same order, operand by operand from memory.  Where that stands decides
@@ -445,34 +585,69 @@ hipError_t launch_wsm_rt(int rt, const SmArgs &p, hipStream_t stream) {
         case 4: return launch_wsm<4, NT, KW, MODE>(p, stream);
         case 5: return launch_wsm<5, NT, KW, MODE>(p, stream);
         case 6: return launch_wsm<6, NT, KW, MODE>(p, stream);
-        default: return launch_wsm<7, NT, KW, MODE>(p, stream);
+        case 7: return launch_wsm<7, NT, KW, MODE>(p, stream);
+        default:
+            if constexpr (MODE >= kSmAwqRounded && NT == 2) return rt == 8 ? launch_wsm<8, NT, KW, MODE>(p, stream) : launch_wsm<10, NT, KW, MODE>(p, stream);
+            else return hipErrorInvalidValue;
     }
 }
 
 template <int MODE>
 hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t stream) {
-    if constexpr (MODE >= kSmAwqRounded)
-        if (plan.nt == 3) return plan.rt == 3 ? launch_wsm<3, 3, 1, MODE>(p, stream) : plan.rt == 4 ? launch_wsm<4, 3, 1, MODE>(p, stream) : launch_wsm<5, 3, 1, MODE>(p, stream);
+    if constexpr (MODE >= kSmAwqRounded) {
+        if (plan.nt == 3) {
+            switch (plan.rt) {
+                case 3: return launch_wsm<3, 3, 1, MODE>(p, stream);
+                case 4: return launch_wsm<4, 3, 1, MODE>(p, stream);
+                case 5: return launch_wsm<5, 3, 1, MODE>(p, stream);
+                case 6: return launch_wsm<6, 3, 1, MODE>(p, stream);
+                default: return launch_wsm<7, 3, 1, MODE>(p, stream);
+            }
+        }
+    }
     return plan.nt == 1 ? launch_wsm_rt<1, MODE>(plan.rt, p, stream) : launch_wsm_rt<2, MODE>(plan.rt, p, stream);
 }
 
 // The time of a launch on the GPU.  Exact modes: fitted to 3900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows,
-// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 0.5 % more than the best of them on average, 10 % at worst); rounded: to
-// 2500 (13 matrices, 65 .. 3500 rows; rms error 10 %, 24 % at worst) of kernels with 23 instructions a dequantisation, which the AWQ order's no longer have: they
-// take up to 9 % less than this says, the tiled kernel that they are weighed against (0.95 of its estimate, which is from then as well) up to 2 %.  Microseconds of start, of a workgroup, and of a step alone on the chip
-// (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of one of two.  The launch that
-// adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
+// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 0.5 % more than the best of them on average, 10 % at worst).  Microseconds of start, of a
+// workgroup, and of a step alone on the chip (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of
+// one of two.  The launch that adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
 struct SmCost {
     double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, part, tb_s;
 };
-constexpr SmCost kSmCost[3] = {{2.94, 1.70, 0.184, 0.065, 0.055, 0.083, 0.154, 0, 0, 0, 0.65, 0.91, 0.23, 5.0},
-                               {3.79, 1.28, 0, 0.018, 0.422, 0.165, 0.138, 0.019, 0.089, 0, 0.83, 0.60, 0.21, 5.6},
-                               {1.8, 2.5, 0, 0.030, 0.150, 0.035, 0.07, 0.018, 0.09, 0.03, 0, 0, 0, 1}};
+constexpr SmCost kSmCost[2] = {{2.94, 1.70, 0.184, 0.065, 0.055, 0.083, 0.154, 0, 0, 0, 0.65, 0.91, 0.23, 5.0},
+                               {3.79, 1.28, 0, 0.018, 0.422, 0.165, 0.138, 0.019, 0.089, 0, 0.83, 0.60, 0.21, 5.6}};
+// Rounded weights: what a group takes a workgroup that is alone, and what is added with every CU full, for each form there is (AWQ, Q4NX).  Fitted to 1600 timings a codec
+// in a graph (14 matrices from 1024 x 4096 to 10240 x 8192, 66 .. 1600 rows, every form; rms error 5 to 6 %; the form it picks takes 1.2 % more than the best of them on
+// average, 15 % at worst: few columns and much K).
+struct SmForm {
+    int rt, nt;
+    float alone[2], more[2];
+};
+constexpr SmForm kSmForms[] = {{2, 1, {0.248f, 0.281f}, {0.184f, 0.187f}}, {3, 1, {0.340f, 0.363f}, {0.251f, 0.267f}}, {4, 1, {0.421f, 0.461f}, {0.266f, 0.274f}},
+                               {5, 1, {0.488f, 0.496f}, {0.280f, 0.326f}}, {6, 1, {0.456f, 0.488f}, {0.095f, 0.095f}}, {7, 1, {0.491f, 0.531f}, {0.094f, 0.086f}},
+                               {2, 2, {0.484f, 0.555f}, {0.332f, 0.367f}}, {3, 2, {0.559f, 0.655f}, {0.389f, 0.407f}}, {4, 2, {0.613f, 0.685f}, {0.476f, 0.502f}},
+                               {5, 2, {0.679f, 0.794f}, {0.100f, 0.075f}}, {6, 2, {0.741f, 0.847f}, {0.104f, 0.097f}}, {7, 2, {0.805f, 0.991f}, {0.123f, 0.086f}},
+                               {8, 2, {0.866f, 0.951f}, {0.146f, 0.135f}}, {10, 2, {0.974f, 1.166f}, {0.196f, 0.160f}}, {3, 3, {0.745f, 0.966f}, {0.593f, 0.053f}},
+                               {4, 3, {0.861f, 0.969f}, {0.102f, 0.100f}}, {5, 3, {0.912f, 1.058f}, {0.115f, 0.112f}}, {6, 3, {0.951f, 1.157f}, {0.174f, 0.148f}},
+                               {7, 3, {1.006f, 1.268f}, {0.212f, 0.149f}}};
 
-double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
-    const SmCost &c = kSmCost[rounded ? 2 : q4];
-    const bool four = !rounded && p.rt <= 2;
-    const int kw = rounded ? 1 : four ? 4 : 2, chip = rounded ? 512 : 256;   // (two workgroups a CU where one has a wave per SIMD)
+double wsm_rounded_us(const SmForm &f, int blocks, int K, int N, bool q4) {
+    const bool two = sm_together(f.rt, f.nt, q4);   // workgroups to a CU
+    const int chip = two ? 512 : 256, groups = K / kGroup;
+    const long wgs = (long)((N + 64 * f.nt - 1) / (64 * f.nt)) * blocks, full = wgs / chip;
+    const double rest = (double)(wgs % chip) / chip, start = q4 ? 3.75 : 3.5, each = q4 ? 2.02 : 2.13;
+    double us = start + full * (each + groups * (f.alone[q4] + f.more[q4]));
+    // (from half of them on some CUs have two, which take most of `more`)
+    const double share = !two ? rest : rest <= 0.5 ? 0.45 * rest : 0.95 + 0.1 * (rest - 0.5);
+    if (rest > 0) us += each + groups * (f.alone[q4] + f.more[q4] * share);
+    return us;
+}
+
+double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4) {
+    const SmCost &c = kSmCost[q4];
+    const bool four = p.rt <= 2;
+    const int kw = four ? 4 : 2, chip = 256;
     const int groups = (K / kGroup + p.slices - 1) / p.slices, steps = (groups + kw - 1) / kw;
     const double alone = c.a0 + c.a1 * p.rt + c.a2 * p.nt + c.a3 * p.rt * p.nt, more = c.b0 + c.b1 * p.rt + c.b2 * p.nt + c.b3 * p.rt * p.nt;
     const long wgs = (long)((N + 64 * p.nt - 1) / (64 * p.nt)) * p.blocks * p.slices, full = wgs / chip;
@@ -485,16 +660,42 @@ double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4, bool rounded) {
 
 }  // namespace
 
-WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch_bytes) {
+static WsmPlan plan_wsm_rounded(int M, int K, int N, bool q4) {
     const auto &tune = g_gemv_ws_tune;
-    const int tiles = (M + 15) / 16, G = K / kGroup, most_nt = rounded ? 3 : 2;
-    const int only_nt = tune.wsm_nt <= most_nt ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
+    const int tiles = (M + 15) / 16;
+    WsmPlan best;
+    best.us = -1;
+    // a tune key's form, or the tallest of its width where there is none so tall
+    int only_rt = tune.wsm_rt, only_nt = tune.wsm_nt;
+    if (only_rt || only_nt) {
+        int tallest = 0, fits = 0;
+        for (const SmForm &f : kSmForms) {
+            if (f.nt != (only_nt ? only_nt : f.nt)) continue;
+            tallest = std::max(tallest, f.rt);
+            if (f.rt >= only_rt && (!fits || f.rt < fits)) fits = f.rt;
+        }
+        if (only_rt) only_rt = fits ? fits : tallest;
+    }
+    for (const SmForm &f : kSmForms) {
+        if ((only_rt && f.rt != only_rt) || (only_nt && f.nt != only_nt) || (f.rt > 8 && K >= 1 << 23)) continue;   // (the copies' 32-bit offsets)
+        WsmPlan p;
+        p.rt = f.rt, p.nt = f.nt, p.slices = 1, p.blocks = (tiles + f.rt - 1) / f.rt;
+        p.us = wsm_rounded_us(f, p.blocks, K, N, q4);
+        if (best.us < 0 || p.us < best.us) best = p;
+    }
+    return best;
+}
+
+WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch_bytes) {
+    if (rounded) return plan_wsm_rounded(M, K, N, q4);
+    const auto &tune = g_gemv_ws_tune;
+    const int tiles = (M + 15) / 16, G = K / kGroup, most = 7, least = 2, few = (tiles + most - 1) / most;
+    const int only_nt = tune.wsm_nt <= 2 ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
     WsmPlan best;
     best.us = -1;
     double best_rank = 0;   // slices have to be 4 % faster: the estimate is no better than that
-    for (int nt = 1; nt <= most_nt; ++nt) {
+    for (int nt = 1; nt <= 2; ++nt) {
         if (only_nt && nt != only_nt) continue;
-        const int most = nt == 3 ? 5 : 7, least = nt == 3 ? 3 : 2, few = (tiles + most - 1) / most;
         const int options[3] = {few, few + 1, (tiles + 3) / 4};   // blocks of rows
         for (int blocks : options) {
             WsmPlan p;
@@ -504,8 +705,8 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
             p.blocks = (tiles + p.rt - 1) / p.rt;
             auto try_slices = [&](int slices) {   // false: no room for so many
                 p.slices = slices;
-                if (slices > 1 && (rounded || gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes)) return false;
-                p.us = wsm_us(p, M, K, N, q4, rounded);
+                if (slices > 1 && gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes) return false;
+                p.us = wsm_us(p, M, K, N, q4);
                 const double rank = slices > 1 ? 1.04 * p.us : p.us;
                 if (best.us < 0 || rank < best_rank) best = p, best_rank = rank;
                 return true;

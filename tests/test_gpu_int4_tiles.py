@@ -277,3 +277,32 @@ def test_every_weight_under_the_largest_scales(form):
     finally:
         for key in keys:
             ops.tune(key, 0)
+
+
+@pytest.mark.parametrize("codec", ["awq", "q4nx"])
+@pytest.mark.parametrize("rt,nt", [(2, 1), (4, 2), (5, 2), (8, 2), (10, 2), (3, 3), (6, 3), (7, 3)])
+def test_rounded_tiles_of_every_ring(codec, rt, nt):
+    """Forms with two and with one workgroup to a CU, rings of three and four stages, from fewer groups than stages on; a ragged last block of rows and set of columns:
+    the tiled kernel's bits."""
+    from air_hip import ops
+    for K in (256, 512, 1280):
+        for M in (16 * rt * max(2, 144 // (16 * rt)) - 7, 16 * rt * 9 + 1):
+            N = 64 * nt + 64
+            print("rounded ring", codec, rt, nt, M, K, N, flush=True)
+            if codec == "awq":
+                w, product = ops.repack_stream(*map(dev, make_awq(K, N, seed=rt))), ops.w4a16_gemm_stream
+            else:
+                q, s, m = make(N, K, seed=rt)
+                w, product = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T)), ops.q4nx_gemm_stream
+            x = dev(make_x((M, K), seed=K))
+            keys = ("prefill_min_m", "prefill_wsm", "gemm_wsm_rt", "gemm_wsm_nt")
+            try:
+                results = []
+                for values in ((17, 1, rt, nt), (17, 2, 0, 0)):
+                    for key, value in zip(keys, values):
+                        ops.tune(key, value)
+                    results.append(product(x, w))
+                assert torch.equal(*(r.view(torch.int16) for r in results)), (codec, rt, nt, M, K)
+            finally:
+                for key in keys:
+                    ops.tune(key, 0)
