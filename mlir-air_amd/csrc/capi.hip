@@ -560,7 +560,8 @@ static WsmPlan gemm_stream_plan(int M, int K, int N, bool q4, bool residual, siz
     if (!gemm_wsm_supported(M, K, N) || (rounded ? tune.prefill_tile || tune.prefill_wsm == 2 : tune.gemm_rows || tune.cb || tune.splitk == 2)) return p;
     p = plan_gemm_wsm(M, K, N, q4, rounded, scratch_bytes);
     const bool always = rounded ? tune.prefill_wsm == 1 : tune.splitk == 1;
-    if (!always && p.us > 0.95 * (rounded ? gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
+    // (rougher estimates have to differ by 5 %)
+    if (!always && p.us > (rounded ? 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : (q4 || residual ? 0.95 : 1.0) * gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
     return p;
 }
 

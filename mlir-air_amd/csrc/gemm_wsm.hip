@@ -1,19 +1,19 @@
 // Products of 17 rows and more on stream-order weights (wstream.h), both codecs, any K % 128 == 0 and N % 16 == 0:
 // y[M, N] = bf16(x[M, K] . W (+ residual)) with the exact weights, fp32 accumulation.
 //
-// A wave goes through a group of 128 k in about 1900 cycles, of which the matrix pipe works a third: LDS reads, 145 vector and 60
+// A wave alone goes through a group of 128 k (4 x 2 tiles, exact) in about 1900 cycles, of which the matrix pipe works a third: LDS reads, 145 vector and 60
 // scalar instructions and the barrier are a chain.  So a workgroup puts KW waves on every SIMD, each set of four on a group of its own
-// (their sums meet in LDS at the end), and K is cut into slices besides where there are few columns.  64 rows, K = 14336, N = 4096: one
-// wave per SIMD 22.9 us, two 18.2 us, the launches of 64 whole-K rows that ran before 27.3 us (split along K) and 54.9 us; 300 rows of
-// K = 4096, N = 11008 43 us (tiled kernel: 54 us); Q4NX, 2000 rows of the ragged K = 2176, N = 5744 151 us (16 rows a launch: 949 us).
+// (their sums meet in LDS at the end), and K is cut into slices besides where there are few columns; and two waves make a K-step's operands beside the products
+// of the one before (AWQ).  64 rows, K = 14336, N = 4096: 18.4 us, the launches of 64 whole-K rows that ran before there was this kernel 27.3 us (split along K) and 54.9 us;
+// Q4NX, 2000 rows of the ragged K = 2176, N = 5744 151 us (16 rows a launch: 949 us).
 //
 //   workgroup  = 16 RT rows x 64 NT columns; wave (part kq < KW of K, wq < 4): row tiles all, stream tiles NT wq .. of the column set
 //   step       = KW groups; x goes global -> LDS once per workgroup (global_load_lds_dwordx4) and so do a wave's cells and scale words
 //                (a cell is the B operand of four K-steps), R - 1 steps ahead, in a ring of R.  (Cells in registers instead: the
 //                compiler waits for every request in flight once per turn of a loop that carries loads from one turn to the next.)
-//   AWQ        : operands are (128 + q) exactly, flushed per group: y += s (sum (128 + q) x - (128 + z) sum x); the sums of x of the
-//                next step are taken by one wave per row tile with an MFMA against ones and handed round through LDS, with R = 2 by
-//                every wave for itself
+//   AWQ        : operands are (128 + q) exactly, flushed per group: y += s (sum (128 + q) x - (128 + z) sum x); the sums of x are taken by one wave per row
+//                tile with an MFMA against ones and handed round through LDS (by every wave for itself with four waves a SIMD and R = 2).  Two waves a SIMD, one group
+//                after the other / pipelined, us: 64 rows of 4096 x 14336 in 4 x 2 tiles 25.8 / 22.8, 4 x 1 20.6 / 19.1; 128 of 4096 x 11008 26.2 / 23.3; 3 x 2 of 64 of 14336 x 4096 24.4 / 22.2
 //   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: s q, which has 12 significant bits, is cut
 //                into two bf16, and the minimum is an operand of its own: three MFMAs per K-step with every product exact, as s sum q x +
 //                min sum x has them.  (s q + min in two operands keeps 16 bits of it, which loses minima small against the scale.)
@@ -56,9 +56,10 @@ struct SmArgs {
 // [NT][64], K-step lane / 16)
 constexpr int sm_wave_bytes(int nt, bool q4) { return nt * (int)kWsCellBytes + (q4 ? nt : 1) * 256; }
 constexpr int sm_stage(int rt, int nt, int kw, bool q4) { return kw * (16 * rt * 256 + 4 * sm_wave_bytes(nt, q4)); }
+constexpr int sm_sums(int rt, int kw, bool q4) { return q4 ? 0 : 2 * kw * 16 * rt * 4; }   // bytes of the sums of x of two steps
 constexpr bool sm_together(int rt, int nt, bool q4) { return 3 * sm_stage(rt, nt, 1, q4) <= kSmLds / 2; }
 constexpr int sm_ring(int rt, int nt, int kw, bool q4) {
-    const int n = ((kw == 1 && sm_together(rt, nt, q4) ? kSmLds / 2 : kSmLds) - (q4 || rt > 4 ? 0 : 2 * kw * 16 * rt * 4)) / sm_stage(rt, nt, kw, q4);
+    const int n = ((kw == 1 && sm_together(rt, nt, q4) ? kSmLds / 2 : kSmLds) - sm_sums(rt, kw, q4)) / sm_stage(rt, nt, kw, q4);
     return n < 4 ? n : 4;
 }
 
@@ -86,7 +87,9 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     constexpr int MC = Q4 ? NT : 1;                                    // copies (256 bytes) of a wave's scale words
     constexpr int V = RT + NT + MC;                                    // requests of a wave and step: x, cells, scale words
     constexpr int kWave = sm_wave_bytes(NT, Q4), kStage = sm_stage(RT, NT, KW, Q4), R = sm_ring(RT, NT, KW, Q4);
-    constexpr bool kSums = kExact && R > 2 && RT <= 4;                 // sums of x handed round; else a wave takes its own
+    // Exact AWQ by two waves a SIMD: pipelined.  (Four waves hide each other's latencies, and there are few registers: 2 x 2 tiles 16.0 us without, 17.0 with, 64 rows of 4096 x 14336.)
+    constexpr bool kAhead = kExact && KW == 2 && RT * NT <= 12;
+    constexpr bool kSums = kExact && !kAhead && R > 2 && RT <= 4;      // sums of x handed round, taken a step ahead; else a wave takes its own
     constexpr int CW = 64 * NT, kThreads = 256 * KW;
     static_assert(R >= 2, "two steps fit LDS");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -210,121 +213,149 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
         for (int c = 0; c < NT; ++c) Y[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // One group.  A wave's LDS reads are in flight long before their products: everything at the head of the group where there are
-    // registers for it (four row tiles or less), else the operands of a K-step while the one before it multiplies.
-    constexpr int AHEAD = RT <= 4 ? 4 : 2;
-    auto multiply = [&](int half, int stage, int next) {
+    // The first steps are requested; past the slice's end its last group once more (into a stage that nobody reads again).
+    const int g_wave = g_lo + kq, g_last = g_hi - 1;
+    constexpr int kFirst = kAhead ? R : R - 1;
+#pragma unroll
+    for (int i = 0; i < kFirst; ++i) request(min(g_wave + i * KW, g_last), i * kStage);
+    // VALU instructions, LDS reads and copies of a K-step
+    auto interleave = [&](auto products, auto valu, auto reads, auto copies) {
+        constexpr int P = decltype(products)::value;
+        sm_interleave<P, decltype(valu)::value, decltype(reads)::value, decltype(copies)::value>(std::make_integer_sequence<int, P>());
+    };
+
+    int stage = 0;
+    if constexpr (kAhead) {
+        // Products of K-step t from one side of a and b, while the other one is made.  A group's accumulators are flushed beside the first products of the next, and
+        // its sums of x are taken by four waves, row tiles wq and wq + 4 each.  Between K-steps 2 and 3 the next group has landed for everybody, and nobody
+        // reads this one any more: its stage is filled from there on.
+        constexpr int ST = (RT + 3) / 4, P = RT * NT;
+        const uint32_t one = 0x3F803F80u;
+        const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
+        const floatx4 zero = floatx4{0.f, 0.f, 0.f, 0.f};
+        floatx4 acc[RT][NT], xs[RT];
+        bf16x8 a[2][RT], b[2][NT], as[ST][4];
         u32x4 cell[NT];
-        uint32_t word[NT][Q4 ? 4 : 1];
-        bf16x8 a[AHEAD][RT], as[4];
+        uint32_t word[NT];
+        float sc[NT], nz[NT];
+        int half = 0;
+        auto read_a = [&](int at, int t, int side) {
 #pragma unroll
-        for (int c = 0; c < NT; ++c) cell[c] = cell_at(stage, c);
+            for (int rt = 0; rt < RT; ++rt) a[side][rt] = operand_a(at, t, rt);
+        };
+        auto read_next = [&](int at) {   // cells, words and what the sums are taken of
 #pragma unroll
-        for (int t = 0; t < (AHEAD == 4 ? 4 : 1); ++t)
+            for (int c = 0; c < NT; ++c) cell[c] = cell_at(at, c), word[c] = word_at(at, c, 0);
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) a[t][rt] = operand_a(stage, t, rt);
+            for (int i = 0; i < ST; ++i)
 #pragma unroll
-        for (int c = 0; c < NT; ++c)
+                for (int t = 0; t < 4; ++t) as[i][t] = operand_a(at, t, min(wq + 4 * i, RT - 1));
+        };
+        auto dequant = [&](int t, int side) {
 #pragma unroll
-            for (int t = 0; t < (Q4 ? 4 : 1); ++t) word[c][t] = word_at(stage, c, t);
-        __builtin_amdgcn_sched_barrier(0);
-        floatx4 acc[RT][NT], own[RT];
-        if constexpr (kExact && !kSums) {
+            for (int c = 0; c < NT; ++c) b[side][c] = exact_operand(cell[c][t]);
+        };
+        auto products = [&](int t) {
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) own[rt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-        if constexpr (MODE == kSmAwq) {
+            for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t & 1][rt], b[t & 1][c], t ? acc[rt][c] : zero, 0, 0, 0);
+        };
+        auto sums_at = [&](int rt) { return reinterpret_cast<floatx4 *>(xs_lds + (half * KW + kq) * ROWS + 16 * rt + 4 * lg); };   // register i of lane group lg is row 16 rt + 4 lg + i
+        auto sum_rows = [&]() {
+#pragma unroll
+            for (int i = 0; i < ST; ++i) {
+                floatx4 s = zero;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as[i][t], ones, s, 0, 0, 0);
+                *sums_at(min(wq + 4 * i, RT - 1)) = s;   // (the same from every column, and from every wave that takes the tile)
+            }
+        };
+        auto flush = [&](const floatx4 (&x)[RT]) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int c = 0; c < NT; ++c) acc[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+                for (int c = 0; c < NT; ++c)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) Y[rt][c][i] = fmaf(sc[c], fmaf(nz[c], x[rt][i], acc[rt][c][i]), Y[rt][c][i]);
+        };
+        auto scales = [&]() {
+#pragma unroll
+            for (int c = 0; c < NT; ++c) sc[c] = __builtin_bit_cast(float, word[c] << 16), nz[c] = __builtin_bit_cast(float, word[c] & 0xFFFF0000u);
+        };
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            xs[rt] = zero;
+#pragma unroll
+            for (int c = 0; c < NT; ++c) acc[rt][c] = zero;
         }
-        AwqScale d[NT];
-        if constexpr (MODE == kSmAwqRounded) {
 #pragma unroll
-            for (int c = 0; c < NT; ++c) d[c] = awq_scale(word[c][0]);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if constexpr (AHEAD == 2) {
-                if (t < 3) {
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) a[(t + 1) & 1][rt] = operand_a(stage, t + 1, rt);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            if (t == 2 && sums) read_sum_operands(next, as);
-            if constexpr (kExact && !kSums) {
-                const uint32_t one = 0x3F803F80u;
-                const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) own[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t % AHEAD][rt], ones, own[rt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int c = 0; c < NT; ++c) {
-                const bf16x8(&at)[RT] = a[t % AHEAD];
-                if constexpr (MODE == kSmAwq) {
-                    const bf16x8 b = exact_operand(cell[c][t]);
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, acc[rt][c], 0, 0, 0);
-                } else if constexpr (MODE == kSmQ4) {
-                    bf16x8 high, rest;
-                    two_operands(cell[c][t], __builtin_bit_cast(float, word[c][t] << 16), high, rest);
-                    const uint32_t min2 = __builtin_amdgcn_perm(word[c][t], word[c][t], 0x03020302u);
-                    const bf16x8 low8 = __builtin_bit_cast(bf16x8, u32x4{min2, min2, min2, min2});
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], high, Y[rt][c], 0, 0, 0);
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], rest, Y[rt][c], 0, 0, 0);
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], low8, Y[rt][c], 0, 0, 0);
-                } else {
-                    bf16x8 b;
-                    if constexpr (Q4) {
-                        float s, low;
-                        decode_md_q4(word[c][t], s, low);
-                        b = dequant_operand(cell[c][t], s, low);
-                    } else {
-                        b = dequant_operand_awq(cell[c][t], d[c], nib_mask, high_mask, magic);
-                    }
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, Y[rt][c], 0, 0, 0);
-                }
-            }
-            if (AHEAD == 2) __builtin_amdgcn_sched_barrier(0);
-        }
-        if (sums) sum_rows(as, half ^ 1);
-        if constexpr (MODE == kSmAwq) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {   // register i of lane group lg is row 16 rt + 4 lg + i
-                const floatx4 xs = kSums ? *reinterpret_cast<const floatx4 *>(xs_lds + (half * KW + kq) * ROWS + 16 * rt + 4 * lg) : own[rt];
-#pragma unroll
-                for (int c = 0; c < NT; ++c) {
-                    const float sc = __builtin_bit_cast(float, word[c][0] << 16), nz = __builtin_bit_cast(float, word[c][0] & 0xFFFF0000u);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) Y[rt][c][i] = fmaf(sc, fmaf(nz, xs[i], acc[rt][c][i]), Y[rt][c][i]);
-                }
-            }
-        }
-    };
-
-    // The first R - 1 steps are requested; past the slice's end its last group once more (into a stage that nobody reads again).
-    const int g_wave = g_lo + kq, g_last = g_hi - 1;
-#pragma unroll
-    for (int i = 0; i < R - 1; ++i) request(min(g_wave + i * KW, g_last), i * kStage);
-    if (kSums) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * V - RT) : "memory");
+        for (int c = 0; c < NT; ++c) sc[c] = nz[c] = 0.f;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * V) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        bf16x8 as[4];
-        if (sums) {
-            read_sum_operands(0, as);
-            sum_rows(as, 0);
+        read_next(0);
+        read_a(0, 0, 0);
+        dequant(0, 0);
+        const int whole = (g_hi - g_lo) / KW;   // steps in which every set of four waves has a group
+        for (int step = 0; step < whole; ++step) {
+            const int next = stage == (R - 1) * kStage ? 0 : stage + kStage, gn = min(g_wave + (step + R) * KW, g_last);
+#pragma unroll
+            for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
+            __builtin_amdgcn_sched_barrier(0);
+            flush(xs);
+            read_a(stage, 1, 1);
+            dequant(1, 1);
+            products(0);
+            sum_rows();
+            interleave(std::integral_constant<int, P + 4 * ST>(), std::integral_constant<int, 7 * NT + 8 * P>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(stage, 2, 0);
+            dequant(2, 0);
+            products(1);
+            interleave(std::integral_constant<int, P>(), std::integral_constant<int, 7 * NT>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(stage, 3, 1);
+            dequant(3, 1);
+            products(2);
+            interleave(std::integral_constant<int, P>(), std::integral_constant<int, 7 * NT>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * V) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            scales();
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) xs[rt] = *sums_at(rt);
+            read_next(next);
+            read_a(next, 0, 0);
+            dequant(0, 0);
+            products(3);
+            request(gn, stage);
+            interleave(std::integral_constant<int, P>(), std::integral_constant<int, 9 * NT>(), std::integral_constant<int, 2 * RT + 2 * NT + 4 * ST>(), std::integral_constant<int, V>());
+            __builtin_amdgcn_sched_barrier(0);
+            stage = next;
+            half ^= 1;
         }
-    }
-
-    int stage = 0, half = 0;
-    if constexpr (MODE >= kSmAwqRounded) {
+        flush(xs);
+        // the groups that are not a whole step: a set's own sums of x
+        if (g_wave + whole * KW < g_hi) {
+            floatx4 own[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) own[rt] = zero;
+            scales();
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t > 0) {
+                    read_a(stage, t, t & 1);
+                    dequant(t, t & 1);
+                }
+                products(t);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) own[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t & 1][rt], ones, own[rt], 0, 0, 0);
+            }
+            flush(own);
+        }
+    } else if constexpr (MODE >= kSmAwqRounded) {
         // Products of K-step t from one side of a and b, while the other one is made.  Between K-steps 1 and 2 the next group has landed for everybody, and nobody
         // reads the one before this any more: its stage is filled from there on.
         bf16x8 a[2][RT], b[2][NT];
@@ -380,11 +411,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[side][rt], b[side][c], Y[rt][c], 0, 0, 0);
         };
-        auto interleave = [&](auto valu, auto reads, auto copies) {
-            constexpr int P = RT * NT, VALU = decltype(valu)::value, READS = decltype(reads)::value, COPIES = decltype(copies)::value;
-            sm_interleave<P, VALU, READS, COPIES>(std::make_integer_sequence<int, P>());
-        };
         constexpr int kDq = NT * (Q4 ? 25 : 17);
+        constexpr std::integral_constant<int, RT * NT> P;
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * V) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -401,13 +429,13 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
             read_a(stage, 1, 1);
             dequant(1, 1);
             products(0);
-            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
             __builtin_amdgcn_sched_barrier(0);
             read_a(stage, 2, 0);
             dequant(2, 0);
             keep_last();
             products(1);
-            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
             __builtin_amdgcn_sched_barrier(0);
             // the next group has landed for everybody, and nobody reads the one before this any more
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 3) * V) : "memory");
@@ -418,33 +446,127 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
             dequant(3, 1);
             products(0);
             request_x(gn, fill, 0, RT);
-            interleave(std::integral_constant<int, kDq>(), std::integral_constant<int, RT + NT * (Q4 ? 5 : 2)>(), std::integral_constant<int, RT>());
+            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT + NT * (Q4 ? 5 : 2)>(), std::integral_constant<int, RT>());
             __builtin_amdgcn_sched_barrier(0);
             read_a(next, 0, 0);
             scales();
             dequant(0, 0);
             products(1);
             request_w(gn, fill);
-            interleave(std::integral_constant<int, kDq + (Q4 ? 0 : 4 * NT)>(), std::integral_constant<int, RT>(), std::integral_constant<int, NT + MC>());
+            interleave(P, std::integral_constant<int, kDq + (Q4 ? 0 : 4 * NT)>(), std::integral_constant<int, RT>(), std::integral_constant<int, NT + MC>());
             __builtin_amdgcn_sched_barrier(0);
             stage = next;
         }
     } else {
-    for (int g0 = g_lo; g0 < g_hi; g0 += KW) {
-        // This step's requests and, for the sums, the next step's x have landed (younger ones: R - 2 steps, less that x); this wave is done
-        // with the step before, and behind the barrier so is everybody.
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kSums ? (R - 2) * V - RT : (R - 2) * V) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        int half = 0;
+        // One group.  A wave's LDS reads are in flight long before their products: everything at the head of the group where there are
+        // registers for it (four row tiles or less), else the operands of a K-step while the one before it multiplies.
+        constexpr int AHEAD = RT <= 4 ? 4 : 2;
+        auto multiply = [&](int half, int stage, int next) {
+            u32x4 cell[NT];
+            uint32_t word[NT][Q4 ? 4 : 1];
+            bf16x8 a[AHEAD][RT], as[4];
 #pragma unroll
-        for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
-        const int fill = stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
-        request(min(g0 + kq + (R - 1) * KW, g_last), fill);
-        __builtin_amdgcn_sched_barrier(0);
-        if (KW == 1 || g0 + kq < g_hi) multiply(half, stage, next);
-        stage = next;
-        half ^= 1;
-    }
+            for (int c = 0; c < NT; ++c) cell[c] = cell_at(stage, c);
+#pragma unroll
+            for (int t = 0; t < (AHEAD == 4 ? 4 : 1); ++t)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) a[t][rt] = operand_a(stage, t, rt);
+#pragma unroll
+            for (int c = 0; c < NT; ++c)
+#pragma unroll
+                for (int t = 0; t < (Q4 ? 4 : 1); ++t) word[c][t] = word_at(stage, c, t);
+            __builtin_amdgcn_sched_barrier(0);
+            floatx4 acc[RT][NT], own[RT];
+            if constexpr (kExact && !kSums) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) own[rt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+            if constexpr (MODE == kSmAwq) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int c = 0; c < NT; ++c) acc[rt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if constexpr (AHEAD == 2) {
+                    if (t < 3) {
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) a[(t + 1) & 1][rt] = operand_a(stage, t + 1, rt);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                if (t == 2 && sums) read_sum_operands(next, as);
+                if constexpr (kExact && !kSums) {
+                    const uint32_t one = 0x3F803F80u;
+                    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) own[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t % AHEAD][rt], ones, own[rt], 0, 0, 0);
+                }
+#pragma unroll
+                for (int c = 0; c < NT; ++c) {
+                    const bf16x8(&at)[RT] = a[t % AHEAD];
+                    if constexpr (MODE == kSmAwq) {
+                        const bf16x8 b = exact_operand(cell[c][t]);
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], b, acc[rt][c], 0, 0, 0);
+                    } else {
+                        bf16x8 high, rest;
+                        two_operands(cell[c][t], __builtin_bit_cast(float, word[c][t] << 16), high, rest);
+                        const uint32_t min2 = __builtin_amdgcn_perm(word[c][t], word[c][t], 0x03020302u);
+                        const bf16x8 low8 = __builtin_bit_cast(bf16x8, u32x4{min2, min2, min2, min2});
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], high, Y[rt][c], 0, 0, 0);
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], rest, Y[rt][c], 0, 0, 0);
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[rt], low8, Y[rt][c], 0, 0, 0);
+                    }
+                }
+                if (AHEAD == 2) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (sums) sum_rows(as, half ^ 1);
+            if constexpr (MODE == kSmAwq) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {   // register i of lane group lg is row 16 rt + 4 lg + i
+                    const floatx4 xs = kSums ? *reinterpret_cast<const floatx4 *>(xs_lds + (half * KW + kq) * ROWS + 16 * rt + 4 * lg) : own[rt];
+#pragma unroll
+                    for (int c = 0; c < NT; ++c) {
+                        const float sc = __builtin_bit_cast(float, word[c][0] << 16), nz = __builtin_bit_cast(float, word[c][0] & 0xFFFF0000u);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) Y[rt][c][i] = fmaf(sc, fmaf(nz, xs[i], acc[rt][c][i]), Y[rt][c][i]);
+                    }
+                }
+            }
+        };
+
+        if (kSums) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * V - RT) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            bf16x8 as[4];
+            if (sums) {
+                read_sum_operands(0, as);
+                sum_rows(as, 0);
+            }
+        }
+
+        for (int g0 = g_lo; g0 < g_hi; g0 += KW) {
+            // This step's requests and, for the sums, the next step's x have landed (younger ones: R - 2 steps, less that x); this wave is done
+            // with the step before, and behind the barrier so is everybody.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kSums ? (R - 2) * V - RT : (R - 2) * V) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
+            const int fill = stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
+            request(min(g0 + kq + (R - 1) * KW, g_last), fill);
+            __builtin_amdgcn_sched_barrier(0);
+            if (KW == 1 || g0 + kq < g_hi) multiply(half, stage, next);
+            stage = next;
+            half ^= 1;
+        }
     }
 
     // Scales from 2^117 on (wsdequant.h): the wave's columns once more, a tile at a time in the same order, operand by operand from memory.  Where that stands decides
@@ -544,15 +666,24 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     }
 }
 
-// y = bf16(sum over the slices, in slice order (+ residual)); four columns per thread
+// y = bf16(sum over the slices, in slice order (+ residual)); four columns per thread.  Up to eight slices are asked for together: one after the other each costs a round trip
+// (64 x 4096 in 4 slices, 3.4 -> 2.7 us; in 8, 5.4 -> 3.6).
+template <int AT>
 __global__ void __launch_bounds__(256) gemm_wsm_sum_kernel(const float *__restrict__ partial, const uint16_t *__restrict__ residual,
                                                            uint16_t *__restrict__ y, size_t mn, int slices) {
     const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (at >= mn) return;
-    floatx4 s = *reinterpret_cast<const floatx4 *>(partial + at);
-    for (int k = 1; k < slices; ++k) s += *reinterpret_cast<const floatx4 *>(partial + (size_t)k * mn + at);
+    uint2 r = uint2{0u, 0u};
+    if (residual) r = *reinterpret_cast<const uint2 *>(residual + at);
+    floatx4 s;
+    for (int k0 = 0; k0 < slices; k0 += AT) {
+        floatx4 v[AT];
+#pragma unroll
+        for (int k = 0; k < AT; ++k) v[k] = *reinterpret_cast<const floatx4 *>(partial + (size_t)min(k0 + k, slices - 1) * mn + at);
+#pragma unroll
+        for (int k = 0; k < AT; ++k) s = k0 + k == 0 ? v[k] : k0 + k < slices ? s + v[k] : s;
+    }
     if (residual) {
-        const uint2 r = *reinterpret_cast<const uint2 *>(residual + at);
         s[0] += bf16_bits_to_float(r.x & 0xFFFFu), s[1] += bf16_bits_to_float(r.x >> 16);
         s[2] += bf16_bits_to_float(r.y & 0xFFFFu), s[3] += bf16_bits_to_float(r.y >> 16);
     }
@@ -562,7 +693,7 @@ __global__ void __launch_bounds__(256) gemm_wsm_sum_kernel(const float *__restri
 template <int RT, int NT, int KW, int MODE>
 hipError_t launch_wsm(const SmArgs &p, hipStream_t stream) {
     constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded;
-    constexpr size_t ring = (size_t)sm_ring(RT, NT, KW, Q4) * sm_stage(RT, NT, KW, Q4) + (Q4 || RT > 4 ? 0 : 2 * KW * 16 * RT * sizeof(float));
+    constexpr size_t ring = (size_t)sm_ring(RT, NT, KW, Q4) * sm_stage(RT, NT, KW, Q4) + sm_sums(RT, KW, Q4);
     constexpr size_t out = (size_t)16 * RT * (64 * NT + 4) * sizeof(float), parts = (size_t)(KW - 1) * 4 * RT * NT * 1024;
     constexpr size_t lds = ring > out ? (ring > parts ? ring : parts) : out > parts ? out : parts;
     static_assert(lds <= kSmLds, "fits LDS");
@@ -608,15 +739,22 @@ hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t str
     return plan.nt == 1 ? launch_wsm_rt<1, MODE>(plan.rt, p, stream) : launch_wsm_rt<2, MODE>(plan.rt, p, stream);
 }
 
-// The time of a launch on the GPU.  Exact modes: fitted to 3900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows,
-// every tile, 1 .. 16 slices; rms error 5 %; the plan it picks takes 0.5 % more than the best of them on average, 10 % at worst).  Microseconds of start, of a
-// workgroup, and of a step alone on the chip (a0 + a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + ..) with every CU busy; a step of four groups costs 1 + four of
-// one of two.  The launch that adds up: sum, and per slice a read that waits for the one before it (part) and its bytes.
+// The time of a launch on the GPU in microseconds.
+// Exact Q4NX: fitted to 1900 timings in a graph (11 matrices from 2432 x 272 to 13056 x 5744, 17 .. 700 rows, every tile, 1 .. 16 slices; rms error 5 %).  Start, a
+// workgroup, a step alone on the chip (a1 rt + a2 nt + a3 rt nt), plus (b0 + b1 rt + b2 nt) with every CU busy; a step of four groups costs 1 + four of one of
+// two.  The launch that adds up: sum, and per slice `part` and its bytes.
 struct SmCost {
-    double start, group, a0, a1, a2, a3, b0, b1, b2, b3, four, sum, part, tb_s;
+    double start, group, a1, a2, a3, b0, b1, b2, four, sum, part, tb_s;
 };
-constexpr SmCost kSmCost[2] = {{2.94, 1.70, 0.184, 0.065, 0.055, 0.083, 0.154, 0, 0, 0, 0.65, 0.91, 0.23, 5.0},
-                               {3.79, 1.28, 0, 0.018, 0.422, 0.165, 0.138, 0.019, 0.089, 0, 0.83, 0.60, 0.21, 5.6}};
+constexpr SmCost kSmCostQ4 = {3.79, 1.28, 0.018, 0.422, 0.165, 0.138, 0.019, 0.089, 0.83, 0.60, 0.21, 5.6};
+// Exact AWQ: a step's time for each form, fitted to 3000 timings (14 matrices from 1024 x 4096 to 10240 x 8192, 17 .. 128 rows, every form and number of slices;
+// rms error 4 %; the plan it picks takes 0.5 % more than the best of them on average, 5 % at worst).  Of 64 rows of 14336 x 4096 in 4 slices start and end are 5.5 us, seven steps 10, the
+// parts and their sum 3.6.
+struct SmExactForm {
+    float alone, more;
+};
+constexpr SmExactForm kSmExact[2][6] = {{{0.874f, 0.172f}, {0.690f, 0.044f}, {0.827f, 0.023f}, {1.013f, 0.067f}, {1.072f, 0.082f}, {1.256f, 0.116f}},
+                                        {{1.208f, 0.206f}, {0.866f, 0.057f}, {1.077f, 0.066f}, {1.336f, 0.085f}, {1.620f, 0.102f}, {2.023f, 0.f}}};   // [nt - 1][rt - 2]
 // Rounded weights: what a group takes a workgroup that is alone, and what is added with every CU full, for each form there is (AWQ, Q4NX).  Fitted to 1600 timings a codec
 // in a graph (14 matrices from 1024 x 4096 to 10240 x 8192, 66 .. 1600 rows, every form; rms error 5 to 6 %; the form it picks takes 1.2 % more than the best of them on
 // average, 15 % at worst: few columns and much K).
@@ -645,16 +783,23 @@ double wsm_rounded_us(const SmForm &f, int blocks, int K, int N, bool q4) {
 }
 
 double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4) {
-    const SmCost &c = kSmCost[q4];
-    const bool four = p.rt <= 2;
+    const bool four = p.rt <= 2;   // groups to a step
     const int kw = four ? 4 : 2, chip = 256;
     const int groups = (K / kGroup + p.slices - 1) / p.slices, steps = (groups + kw - 1) / kw;
-    const double alone = c.a0 + c.a1 * p.rt + c.a2 * p.nt + c.a3 * p.rt * p.nt, more = c.b0 + c.b1 * p.rt + c.b2 * p.nt + c.b3 * p.rt * p.nt;
     const long wgs = (long)((N + 64 * p.nt - 1) / (64 * p.nt)) * p.blocks * p.slices, full = wgs / chip;
-    const double rest = (double)(wgs % chip) / chip, step = steps * (four ? 1 + c.four : 1.0);
+    const double rest = (double)(wgs % chip) / chip, mb = (double)M * N * 8e-6;   // a part written and read
+    if (!q4) {
+        const SmExactForm &f = kSmExact[p.nt - 1][p.rt - 2];
+        double us = 3.26 + full * (2.24 + steps * (f.alone + f.more));
+        if (rest > 0) us += 2.24 + steps * (f.alone + f.more * rest);
+        if (p.slices > 1) us += 0.98 + 0.21 * ((p.slices + 7) / 8) + p.slices * mb / 3.52;
+        return us;
+    }
+    const SmCost &c = kSmCostQ4;
+    const double alone = c.a1 * p.rt + c.a2 * p.nt + c.a3 * p.rt * p.nt, more = c.b0 + c.b1 * p.rt + c.b2 * p.nt, step = steps * (four ? 1 + c.four : 1.0);
     double us = c.start + full * (c.group + step * (alone + more));
     if (rest > 0) us += c.group + step * (alone + more * rest);
-    if (p.slices > 1) us += c.sum + p.slices * (c.part + (double)M * N * 8e-6 / c.tb_s);
+    if (p.slices > 1) us += c.sum + p.slices * (c.part + mb / c.tb_s);
     return us;
 }
 
@@ -740,7 +885,7 @@ hipError_t launch_gemm_wsm(const WsmPlan &plan, const uint16_t *x, const void *w
                             : (rounded ? launch_wsm_mode<kSmAwqRounded>(plan, p, stream) : launch_wsm_mode<kSmAwq>(plan, p, stream));
     if (e != hipSuccess || plan.slices == 1) return e;
     const size_t mn = (size_t)M * N;   // N % 16 == 0: whole groups of four columns
-    hipLaunchKernelGGL(gemm_wsm_sum_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, residual, y, mn, plan.slices);
+    hipLaunchKernelGGL(plan.slices <= 2 ? &gemm_wsm_sum_kernel<2> : plan.slices <= 4 ? &gemm_wsm_sum_kernel<4> : &gemm_wsm_sum_kernel<8>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, residual, y, mn, plan.slices);
     return hipGetLastError();
 }
 

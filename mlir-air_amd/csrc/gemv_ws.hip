@@ -840,13 +840,12 @@ static int gemm_ws_cb(int tiles) {
     return tiles % cb ? 1 : cb;
 }
 
-// Each launch rounds of workgroups over the chip, a group of K a cost by rows and tile columns (fitted to 13 matrices at 8 .. 128 rows;
-// AWQ, 17 / 64 rows: K = 4096, N = 4096 7.3 estimated / 7.5 measured and 18.6 / 19.1 us, K = 14336, N = 4096 20.0 / 22.1 and 58.9 / 54.9;
-// Q4NX, 32 rows: K = 4096, N = 14336 26.1 / 24.1)
+// Each launch rounds of workgroups over the chip, a group of K a cost by rows and tile columns.  Launches of up to 64 rows: fitted to 360 timings (60 matrices of K = 1024 ..
+// 14336, 17 .. 128 rows; rms error 6 %); of 16 (Q4NX, or with a residual): to 13 matrices (Q4NX, 32 rows of K = 4096, N = 14336 26.1 estimated / 24.1 measured)
 double gemm_ws_us(int M, int K, int N, bool q4, bool residual) {
     const int tiles = N / kWsTileCols, cb = gemm_ws_cb(tiles), most = q4 || residual ? 16 : 64, G = K / kGroup;
-    const double rounds = (tiles / cb + 255) / 256, wide = cb == 4 ? 0.14 : cb == 2 ? 0.06 : 0.03, step16 = cb == 4 ? 0.33 : cb == 2 ? 0.20 : 0.15;
-    auto launch = [&](int rows) { return 2.5 + G * rounds * (most == 16 ? step16 * (0.5 + rows / 32.0) : wide + 0.0074 * rows); };
+    const double rounds = (tiles / cb + 255) / 256, wide = cb == 4 ? 0.136 : cb == 2 ? 0.076 : 0.042, step16 = cb == 4 ? 0.33 : cb == 2 ? 0.20 : 0.15;
+    auto launch = [&](int rows) { return most == 16 ? 2.5 + G * rounds * step16 * (0.5 + rows / 32.0) : 3.3 + G * rounds * (wide + 0.007 * rows); };
     return (M / most) * launch(most) + (M % most ? launch(M % most) : 0);
 }
 

@@ -306,3 +306,29 @@ def test_rounded_tiles_of_every_ring(codec, rt, nt):
             finally:
                 for key in keys:
                     ops.tune(key, 0)
+
+
+@pytest.mark.parametrize("rt,nt", [(3, 1), (4, 1), (7, 1), (3, 2), (4, 2), (6, 2)])
+def test_exact_tiles_of_few_groups(rt, nt):
+    """Pipelined exact tiles with fewer groups than sets of waves, than stages, and one more than whole steps: one bf16 rounding of an fp32 sum; a row of infinities stays
+    in its row."""
+    from air_hip import ops
+    keys = {"gemm_splitk": 1, "gemm_wsm_rt": rt, "gemm_wsm_nt": nt, "gemm_wsm_slices": 1}
+    M, N = 16 * rt - 5, 64 * nt + 48
+    for K in (128, 256, 384, 640, 896):
+        print("exact tiles of few groups", rt, nt, M, K, N, flush=True)
+        tri = make_awq(K, N, seed=K)
+        x = make_x((M, K), seed=rt)
+        want = bf16_bits_to_f32(x).astype(np.float64) @ dense_f64(*tri)
+        x[3, 5] = 0x7F80
+        w, xd = ops.repack_stream(*map(dev, tri)), dev(x)
+        try:
+            for key, value in keys.items():
+                ops.tune(key, value)
+            got = bits(ops.w4a16_gemm_stream(xd, w))
+        finally:
+            for key in keys:
+                ops.tune(key, 0)
+        rows = np.arange(M) != 3
+        assert not np.isfinite(bf16_bits_to_f32(got[3])).any()
+        assert_bf16_close(np.ascontiguousarray(got[rows]), want[rows], ulps=1.0, atol=2e-3, what=f"{rt} {nt} {K}")
