@@ -121,6 +121,20 @@ __device__ __forceinline__ float max_over_lane_groups(float v) {
     return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
 }
 
+// Sum of n matrices `stride` floats apart at one place, in their order, AT of them asked for together (one after the other each costs a round trip to the last-level cache)
+template <int AT>
+__device__ __forceinline__ floatx4 sum_parts(const float *p, size_t stride, int n) {
+    floatx4 sum;
+    for (int k0 = 0; k0 < n; k0 += AT) {
+        floatx4 v[AT];
+#pragma unroll
+        for (int k = 0; k < AT; ++k) v[k] = *reinterpret_cast<const floatx4 *>(p + (size_t)(k0 + k < n ? k0 + k : n - 1) * stride);
+#pragma unroll
+        for (int k = 0; k < AT; ++k) sum = k0 + k == 0 ? v[k] : k0 + k < n ? sum + v[k] : sum;
+    }
+    return sum;
+}
+
 // silu(g) in the reference's tanh form (matvec_int4_swiglu_rms.py:512-514), fp32
 __device__ __forceinline__ float silu_tanh(float g) { return g * 0.5f * (tanhf(g * 0.5f) + 1.0f); }
 

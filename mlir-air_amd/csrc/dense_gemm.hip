@@ -20,6 +20,7 @@
 // row and never stored.
 #include "dense.h"
 #include "dense_kernels.h"
+#include <type_traits>
 #include <utility>
 
 namespace w4a16 {
@@ -814,7 +815,7 @@ hipError_t launch_experts(const GemmArgs &g, hipStream_t stream) {
 }
 
 // out = the epilogue of the sum of `slices` parts [M][N]; a thread has four neighbouring columns of out
-template <int EPI>
+template <int EPI, int AT>
 __global__ void __launch_bounds__(256) gemm_sum_kernel(const float *parts, int slices, int M, int N, void *out, long ldo, int silu_begin, int silu_end) {
     constexpr bool kPair = EPI == kOutSwiglu || EPI == kOutGeglu;
     const int quads = (kPair ? N / 2 : N) / 4;
@@ -823,14 +824,9 @@ __global__ void __launch_bounds__(256) gemm_sum_kernel(const float *parts, int s
     const long m = t / quads;
     const int col = (int)(t % quads) * 4;
     const float *p = parts + m * N + (kPair ? col / 16 * 32 + col % 16 : col);
-    auto sum = [&](const float *q) {
-        floatx4 v = *reinterpret_cast<const floatx4 *>(q);
-        for (int s = 1; s < slices; ++s) v += *reinterpret_cast<const floatx4 *>(q + s * size);
-        return v;
-    };
-    floatx4 v = sum(p);
+    floatx4 v = sum_parts<AT>(p, size, slices);
     if constexpr (kPair) {
-        const floatx4 up = sum(p + 16);
+        const floatx4 up = sum_parts<AT>(p + 16, size, slices);
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (EPI == kOutGeglu ? gelu_tanh_of<bf16>(v[r]) : silu_of<bf16>(v[r])) * up[r];
     } else if (EPI == kOutElem && col >= silu_begin && col < silu_end) {
@@ -953,11 +949,15 @@ hipError_t launch_dense_gemm_sliced(int dtype, const GemmArgs &g, int slices, fl
         hipLaunchKernelGGL(kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, parts, slices, g.M, g.N, g.out, g.ldo, g.silu_begin, g.silu_end);
         return hipGetLastError();
     };
+    auto pick = [&](auto epi) {
+        constexpr int EPI = decltype(epi)::value;
+        return slices <= 2 ? add(&gemm_sum_kernel<EPI, 2>) : slices <= 4 ? add(&gemm_sum_kernel<EPI, 4>) : add(&gemm_sum_kernel<EPI, 8>);
+    };
     switch (g.epilogue) {
-        case kOutF32: return add(&gemm_sum_kernel<kOutF32>);
-        case kOutSwiglu: return add(&gemm_sum_kernel<kOutSwiglu>);
-        case kOutGeglu: return add(&gemm_sum_kernel<kOutGeglu>);
-        default: return add(&gemm_sum_kernel<kOutElem>);
+        case kOutF32: return pick(std::integral_constant<int, kOutF32>());
+        case kOutSwiglu: return pick(std::integral_constant<int, kOutSwiglu>());
+        case kOutGeglu: return pick(std::integral_constant<int, kOutGeglu>());
+        default: return pick(std::integral_constant<int, kOutElem>());
     }
 }
 

@@ -757,12 +757,12 @@ hipError_t launch_wsp(const PfArgs &p, hipStream_t stream, int slices = 1) {
 }
 
 // y = bf16(the sum over the slices, in their order), or that added to aux and rounded again; four columns per thread
+template <int AT>
 __global__ void __launch_bounds__(256) gemm_wsp_sum_kernel(const float *__restrict__ parts, const uint16_t *__restrict__ aux, uint16_t *__restrict__ y,
                                                            size_t mn, int slices) {
     const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (at >= mn) return;
-    floatx4 v = *reinterpret_cast<const floatx4 *>(parts + at);
-    for (int k = 1; k < slices; ++k) v += *reinterpret_cast<const floatx4 *>(parts + (size_t)k * mn + at);
+    const floatx4 v = sum_parts<AT>(parts + at, mn, slices);
     uint2 o = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     if (aux) {
         const uint2 a = *reinterpret_cast<const uint2 *>(aux + at);
@@ -838,7 +838,7 @@ hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y,
         const hipError_t e = launch_wsp<4, 0, true>(p, stream, slices);
         if (e != hipSuccess) return e;
         const size_t mn = (size_t)M * N;
-        hipLaunchKernelGGL(gemm_wsp_sum_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, aux, y, mn, slices);
+        hipLaunchKernelGGL(slices <= 2 ? &gemm_wsp_sum_kernel<2> : slices <= 4 ? &gemm_wsp_sum_kernel<4> : &gemm_wsp_sum_kernel<8>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, aux, y, mn, slices);
         return hipGetLastError();
     }
     Widths wd = pick_widths(p.tiles_m, U, 256, heads128);

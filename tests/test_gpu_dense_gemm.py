@@ -146,6 +146,29 @@ def test_parts_meet_in_the_row_kernels(dense, M, K):
     assert dense.gemm(a, w, out_f32=True, parts=True).shape[1:] == (M, K)
 
 
+@pytest.mark.parametrize("width", [64, 1024, 1088, 2048, 2112, 4096, 4160])
+def test_row_kernels_of_every_form(dense, width):
+    """Few rows (loads together, sums in registers) and many (loads in turn, sums by way of LDS) add up in the same order: the same bits."""
+    many = 1100
+    res, nw = rand(1, many, width), 1.0 + 0.1 * rand(2, width)
+    norm = lambda v: v / torch.sqrt(v.square().mean(-1, keepdim=True) + 1e-5) * nw.double()
+    for n in (1, 2, 3, 5, 9):
+        y, ys, wt = rand(n, n, many, width), rand(n + 20, many, n, width).bfloat16(), rand(n + 40, many, n).abs()
+        calls = {"residual": lambda r, m: dense.residual_norm_rows(r, y[:, :m].contiguous(), nw, 1e-5, width, torch.bfloat16),
+                 "sum": lambda r, m: dense.add_norm_rows(r, y[:, :m].contiguous(), nw, 1e-5, width, torch.bfloat16),
+                 "experts": lambda r, m: dense.residual_norm_rows(r, ys[:m].reshape(m * n, width), nw, 1e-5, width, torch.bfloat16, weights=wt[:m].contiguous())}
+        wants = {"residual": res.double() + norm(y.double().sum(0)), "sum": res.double() + y.double().sum(0),
+                 "experts": res.double() + norm((wt.double()[..., None] * ys.double()).sum(1))}
+        for name, call in calls.items():
+            all_r = res.clone()
+            all_h = call(all_r, many)
+            close(all_r, wants[name], False, (name, n))
+            for m in (1, 512, 513):
+                r = res[:m].clone()
+                h = call(r, m)
+                assert torch.equal(r, all_r[:m]) and torch.equal(h, all_h[:m]), (name, n, m)
+
+
 COUNTS = [(0, 1, 15, 128, 129, 255, 256, 257), (512, 0, 0, 300, 64, 127, 383, 385), (16, 16, 16, 16, 16, 16, 16, 16), (0, 0, 0, 700, 0, 0, 0, 0), [384, 385, 320, 770, 192, 321]]
 
 

@@ -332,3 +332,20 @@ def test_exact_tiles_of_few_groups(rt, nt):
         rows = np.arange(M) != 3
         assert not np.isfinite(bf16_bits_to_f32(got[3])).any()
         assert_bf16_close(np.ascontiguousarray(got[rows]), want[rows], ulps=1.0, atol=2e-3, what=f"{rt} {nt} {K}")
+
+
+@pytest.mark.parametrize("slices", [4, 5, 8, 9, 16])
+def test_sums_of_many_slices(slices):
+    """Parts asked for several at a time, with and without some left over, against the float64 product."""
+    from air_hip import ops
+    M, K, N = 33, 34 * 128, 80
+    qw, qz, s = make_awq(K, N, seed=slices)
+    x = make_x((M, K), seed=slices)
+    try:
+        for key, value in (("gemm_splitk", 1), ("gemm_wsm_slices", slices)):
+            ops.tune(key, value)
+        got = ops.w4a16_gemm_stream(dev(x), ops.repack_stream(dev(qw), dev(qz), dev(s)))
+        assert_bf16_close(bits(got), bf16_bits_to_f32(x).astype(np.float64) @ dense_f64(qw, qz, s), ulps=1.0, atol=2e-3, what=f"{slices} slices")
+    finally:
+        for key in ("gemm_splitk", "gemm_wsm_slices"):
+            ops.tune(key, 0)
