@@ -597,7 +597,8 @@ static size_t gemm_stream_best_scratch(int M, int K, int N, bool q4, bool residu
     if (p.slices == 1) return 0;
     if (g_gemv_ws_tune.splitk != 1) {
         const WsmPlan none = gemm_stream_plan(M, K, N, q4, residual, 0);
-        if (0.95 * (none.us >= 0 ? none.us : gemm_ws_us(M, K, N, q4, residual)) <= std::max(p.us, kTwoLaunchesUs)) return 0;
+        const double whole = gemm_stream_rounded(M, K, N, q4, residual) ? gemm_prefill_ws_us(M, K, N, q4, 0) : gemm_ws_us(M, K, N, q4, residual);
+        if (0.95 * (none.us >= 0 ? none.us : whole) <= std::max(p.us, kTwoLaunchesUs)) return 0;
     }
     return gemm_wsm_scratch_bytes(p, M, N);
 }
@@ -741,7 +742,7 @@ int rms_norm_rows_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps
 }
 
 size_t w4a16_prefill_qkv_workspace_bytes(int M, int E) {
-    return prefill_block_supported(M, E, 8) ? round256((size_t)M * E * sizeof(uint16_t)) : 0;
+    return prefill_block_supported(M, E, 8) ? prefill_qkv_scratch_bytes(M, E) : 0;
 }
 
 int w4a16_prefill_rms_qkv_rope_bf16(const uint16_t *x, const uint16_t *attn_norm_weight, float eps,
@@ -832,8 +833,7 @@ int prefill_qkv_stream_call(const uint16_t *x, const uint16_t *attn_norm_weight,
     if (!workspace || workspace_bytes < w4a16_prefill_qkv_workspace_bytes(M, E)) return W4A16_ERR_WORKSPACE;
     if (misaligned(workspace)) return W4A16_ERR_ALIGN;
     hipError_t e = launch_prefill_rms_qkv_rope_stream(x, attn_norm_weight, eps, qkv_wstream, rope_lut, pos0, qkv_out, M, E, n_heads,
-                                                      n_kv_heads, head_dim, static_cast<uint16_t *>(workspace),
-                                                      static_cast<hipStream_t>(stream), q4);
+                                                      n_kv_heads, head_dim, workspace, static_cast<hipStream_t>(stream), q4);
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
 

@@ -778,12 +778,13 @@ __global__ void __launch_bounds__(256) gemm_wsp_sum_kernel(const float *__restri
 
 bool gemm_prefill_ws_supported(int M, int K, int N) { return M > 0 && K > 0 && K % (2 * kGroup) == 0 && N > 0 && N % 64 == 0; }
 
-// Rounds of tiles over the chip, each K steps of a cost linear in the tile's width and growing with the share of the CUs that are busy
-// (fitted to 300 .. 2048 rows of twelve matrices, within 20 %: estimated / measured us at K = 4096, N = 4096, 300 rows 43 / 43; N = 11008,
-// 300 rows 58 / 54; K = 14336, N = 4096, 1024 rows 174 / 189, 2048 rows 221 / 218)
+// Rounds of tiles over the chip, each a start and K steps of a cost linear in the tile's width and growing a little with the share of the CUs that are busy (fitted to 1044
+// timings in a graph, 40 .. 1500 rows of 36 matrices from 512 x 512 to 14336 x 14336 in tiles of 64, 128 and 256 columns; rms error 6 %, Q4NX 4.5 %)
 static double wsp_us(int K, long tiles, int ncb, bool q4) {
     const long rounds = (tiles + 255) / 256;
-    return 2.5 + 1e-3 * K * rounds * (0.8 + 0.4 * tiles / (256.0 * rounds)) * (q4 ? 8.3 + 3.1 * ncb : 7.3 + 2.7 * ncb);
+    const double share = (double)tiles / (256.0 * rounds);
+    return q4 ? 2.1 + rounds * (0.8 + 2.05 * ncb + 1e-3 * K * (0.88 + 0.12 * share) * (8.15 + 3.2 * ncb))
+              : 1.8 + rounds * (0.9 + 2.0 * ncb + 1e-3 * K * (0.85 + 0.15 * share) * (7.45 + 2.6 * ncb));
 }
 
 // Slices of K (1: none) in tiles of 256 columns for products of many rows that have too few of them for the chip, where the whole-K
@@ -807,6 +808,11 @@ static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) 
     return best;
 }
 double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes) { return wsp_slices(M, K, N, q4, scratch_bytes).us; }
+double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4) {
+    const int tiles_m = (M + kPfRows - 1) / kPfRows;
+    const Widths wd = pick_widths(tiles_m, 2 * H / 64, 256, true);
+    return wsp_us(K, (long)tiles_m * (wd.wide + (wd.ncb == 4 ? wd.narrow : 0)), wd.ncb, q4);
+}
 size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most) {
     const int s = wsp_slices(M, K, N, q4, most).slices;
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;

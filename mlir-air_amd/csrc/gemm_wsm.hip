@@ -43,12 +43,13 @@ enum : int { kSmAwq, kSmQ4, kSmAwqRounded, kSmQ4Rounded };
 
 struct SmArgs {
     const uint16_t *x;
-    const char *w;
-    float *partial;
-    uint16_t *y;
+    const char *w, *w2;            // w2: a second matrix of the same shape, whose product goes to y2 (rounded weights)
+    float *partial;                // [slices][matrices][M][N]
+    uint16_t *y, *y2;
     const uint16_t *residual;
     int M, K, N, G, NB;
-    int sets, slices, blocks;      // column sets, slices of K, blocks of rows
+    int sets, slices, blocks;      // column sets of all matrices, slices of K, blocks of rows
+    int own_sets;                  // column sets of one matrix
 };
 
 // (rounded: two workgroups to a CU where three stages of each fit LDS, else one with all of it)
@@ -80,6 +81,12 @@ __device__ __forceinline__ void sm_interleave(std::integer_sequence<int, I...>) 
     (one(std::integral_constant<int, I>()), ...);
 }
 
+__device__ __forceinline__ floatx4 widen4(uint2 v) {
+    return floatx4{bf16_bits_to_float(v.x & 0xFFFFu), bf16_bits_to_float(v.x >> 16), bf16_bits_to_float(v.y & 0xFFFFu), bf16_bits_to_float(v.y >> 16)};
+}
+__device__ __forceinline__ uint2 narrow4(floatx4 v) { return uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}; }
+__device__ __forceinline__ floatx4 rounded4(floatx4 v) { return widen4(narrow4(v)); }
+
 template <int RT, int NT, int KW, int MODE>
 __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(const SmArgs p) {
     constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded, kExact = MODE == kSmAwq;
@@ -105,7 +112,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     const int total = p.sets * p.slices * p.blocks, per_xcd = (total + 7) / 8;
     const int id = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per_xcd || id >= total) return;
-    const int block = id % p.blocks, set = id / p.blocks % p.sets, slice = id / (p.blocks * p.sets);
+    const int block = id % p.blocks, set_of_all = id / p.blocks % p.sets, slice = id / (p.blocks * p.sets);
+    const bool second = MODE >= kSmAwqRounded && set_of_all >= p.own_sets;
+    const int set = second ? set_of_all - p.own_sets : set_of_all;
+    const char *const w = second ? p.w2 : p.w;
     const int g_lo = (int)((long)p.G * slice / p.slices), g_hi = (int)((long)p.G * (slice + 1) / p.slices);
     const int m0 = block * ROWS, rows = min(ROWS, p.M - m0);
 
@@ -116,7 +126,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     const int first = min((set * 4 + wq) * NT, ntiles - 1);
     gptr tb[NT];
 #pragma unroll
-    for (int c = 0; c < NT; ++c) tb[c] = scalar_ptr(p.w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
+    for (int c = 0; c < NT; ++c) tb[c] = scalar_ptr(w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
     // this lane's cell and scale words: 32-bit offsets from a tile's start (from the first tile's for the AWQ words, one copy of which
     // serves all the wave's tiles)
     const uint32_t lane16 = 16 * lane;
@@ -575,11 +585,11 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
     bool over = false;
     auto again = [&](int rt, int c) {
         typedef const __attribute__((address_space(1))) uint32_t *Word;
-        const gptr tile = (gptr)(p.w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
+        const gptr tile = (gptr)(w + (size_t)min(first + c, ntiles - 1) * tile_bytes);
         const uint16_t *x = p.x + (size_t)(m0 + min(16 * rt + ln, rows - 1)) * p.K + 8 * lg;
         floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-        for (int k = 0; k < 4 * p.G; ++k) {   // K-steps (slices are for the exact modes)
+        for (int k = 4 * g_lo; k < 4 * g_hi; ++k) {   // K-steps
             const int g = k >> 2;
             const uint32_t blk = (uint32_t)(g >> 4) * (uint32_t)((kWsBlockGroups + kMd) * kWsCellBytes);
             const uint32_t cell = lane16 + blk + (uint32_t)(kMd + (g & 15)) * (uint32_t)kWsCellBytes + 4 * (k & 3), word = 16 * ln + blk + 64 * (g & 12) + 4 * (g & 3);
@@ -650,7 +660,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         floatx4 v = *reinterpret_cast<const floatx4 *>(yt + row * LDP + col);
         const size_t at = (size_t)(m0 + row) * p.N + col0 + col;
         if (p.slices > 1) {
-            *reinterpret_cast<floatx4 *>(p.partial + (size_t)slice * p.M * p.N + at) = v;
+            const int part = MODE >= kSmAwqRounded ? (p.w2 ? 2 * slice + second : slice) : slice;
+            *reinterpret_cast<floatx4 *>(p.partial + (size_t)part * p.M * p.N + at) = v;
             continue;
         }
         if (p.residual) {
@@ -662,13 +673,13 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
             v[0] += bf16_bits_to_float(q.x & 0xFFFFu), v[1] += bf16_bits_to_float(q.x >> 16);
             v[2] += bf16_bits_to_float(q.y & 0xFFFFu), v[3] += bf16_bits_to_float(q.y >> 16);
         }
-        *reinterpret_cast<uint2 *>(p.y + at) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        *reinterpret_cast<uint2 *>((second ? p.y2 : p.y) + at) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }
 }
 
 // y = bf16(sum over the slices, in slice order (+ residual)); four columns per thread.  With their loads in flight together, not in turn, the whole of 64 x 14336 x 4096 in 4 slices
-// takes 18.6 us instead of 19.5, in 8 18.8 instead of 19.6, and 100 x 8192 x 2048 in 8 15.8 instead of 16.7.
-template <int AT>
+// takes 18.6 us instead of 19.5, in 8 18.8 instead of 19.6, and 100 x 8192 x 2048 in 8 15.8 instead of 16.7.  ROUNDED: the residual is added to the rounded sum.
+template <int AT, bool ROUNDED>
 __global__ void __launch_bounds__(256) gemm_wsm_sum_kernel(const float *__restrict__ partial, const uint16_t *__restrict__ residual,
                                                            uint16_t *__restrict__ y, size_t mn, int slices) {
     const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
@@ -677,10 +688,68 @@ __global__ void __launch_bounds__(256) gemm_wsm_sum_kernel(const float *__restri
     if (residual) r = *reinterpret_cast<const uint2 *>(residual + at);
     floatx4 s = sum_parts<AT>(partial + at, mn, slices);
     if (residual) {
-        s[0] += bf16_bits_to_float(r.x & 0xFFFFu), s[1] += bf16_bits_to_float(r.x >> 16);
-        s[2] += bf16_bits_to_float(r.y & 0xFFFFu), s[3] += bf16_bits_to_float(r.y >> 16);
+        if constexpr (ROUNDED) s = rounded4(s);
+        s += widen4(r);
     }
-    *reinterpret_cast<uint2 *>(y + at) = uint2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+    *reinterpret_cast<uint2 *>(y + at) = narrow4(s);
+}
+
+// What the tiled prompt kernel does to a bf16 product where it stores it, as launches of their own (2 to 5 us): its tiles of 256 rows leave few rows most of the chip idle, and these kernels'
+// narrower ones, cut along K besides, have no columns' partners at hand.  A layer of 4096 x 14336, 40 rows, projections / O / gate and up / down: 56 / 16 / 61 / 75 us in the tiled
+// kernel, 16 / 14 / 32 / 19 with these launches (under the profiler); four such layers and the head 835 -> 393 us, of 3 rows 1369 -> 328, 100 rows 916 -> 536, 300 rows 1195 -> 979.
+// Half-split RoPE on the heads of the first `rope_cols` columns; a thread has four columns of a head's lower half and the four they pair with.  AT = 0: in place.
+template <int AT>
+__global__ void __launch_bounds__(256) gemm_wsm_rope_kernel(const float *__restrict__ partial, int slices, const uint16_t *__restrict__ lut, uint16_t *y, int M, int N, int cols,
+                                                            int rope_cols, int hd, int pos0) {
+    const int half = hd >> 1, quads = half >> 2, per_row = cols / hd * quads;
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int m = (int)(t / per_row), q = (int)(t % per_row), i = q % quads * 4, col = q / quads * hd + i;
+    if (m >= M) return;
+    const size_t at = (size_t)m * N + col;
+    const uint16_t *angles = lut + (size_t)(pos0 + m) * hd + i;
+    const floatx4 cs = widen4(*reinterpret_cast<const uint2 *>(angles)), sn = widen4(*reinterpret_cast<const uint2 *>(angles + half));
+    floatx4 lo, hi;
+    if constexpr (AT > 0) {
+        lo = rounded4(sum_parts<AT>(partial + at, (size_t)M * N, slices));
+        hi = rounded4(sum_parts<AT>(partial + at + half, (size_t)M * N, slices));
+    } else {
+        lo = widen4(*reinterpret_cast<const uint2 *>(y + at));
+        hi = widen4(*reinterpret_cast<const uint2 *>(y + at + half));
+    }
+    if (col < rope_cols) {
+        const floatx4 x = lo, z = hi;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lo[e] = x[e] * cs[e] - z[e] * sn[e], hi[e] = z[e] * cs[e] + x[e] * sn[e];
+    }
+    *reinterpret_cast<uint2 *>(y + at) = narrow4(lo);
+    *reinterpret_cast<uint2 *>(y + at + half) = narrow4(hi);
+}
+
+// h = bf16(silu(bf16 gate) * bf16 up) from both products' parts, or (AT = 0) from the products, `gate` and what is in h
+template <int AT>
+__global__ void __launch_bounds__(256) gemm_wsm_swiglu_kernel(const float *__restrict__ partial, int slices, const uint16_t *__restrict__ gate, uint16_t *h, size_t mn) {
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (at >= mn) return;
+    floatx4 g, u;
+    if constexpr (AT > 0) {
+        g = rounded4(sum_parts<AT>(partial + at, 2 * mn, slices));
+        u = rounded4(sum_parts<AT>(partial + mn + at, 2 * mn, slices));
+    } else {
+        g = widen4(*reinterpret_cast<const uint2 *>(gate + at));
+        u = widen4(*reinterpret_cast<const uint2 *>(h + at));
+    }
+    floatx4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = gated_f32(g[e], g[e]) * u[e];
+    *reinterpret_cast<uint2 *>(h + at) = narrow4(v);
+}
+
+// f(parts asked for at a time)
+template <class F>
+void parts_at_a_time(int slices, F f) {
+    if (slices <= 2) f(std::integral_constant<int, 2>());
+    else if (slices <= 4) f(std::integral_constant<int, 4>());
+    else f(std::integral_constant<int, 8>());
 }
 
 template <int RT, int NT, int KW, int MODE>
@@ -798,11 +867,20 @@ double wsm_us(const WsmPlan &p, int M, int K, int N, bool q4) {
 
 }  // namespace
 
-static WsmPlan plan_wsm_rounded(int M, int K, int N, bool q4) {
+size_t gemm_wsm_scratch_bytes(const WsmPlan &p, int M, int N) { return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0; }
+
+// Parts of products of rounded weights: within 12 MB, as they are where there are fewer workgroups than the chip takes (512 of 64 x 64 results are 8 MB)
+size_t gemm_wsm_parts_bytes(int M, int N) { return M > kWsmSliceRows ? 0 : std::min((size_t)16 * M * N * sizeof(float), (size_t)12 << 20); }
+
+// Slices where few rows leave the chip idle: at least eight groups each, and no more parts than the workspace of a prompt pass always has (gemm_wsm_parts_bytes),
+// so that a plain product and the same one inside such a pass run the same slices.  Whole K / slices: 297 x 8704 x 1280 36.8 / 19.5 us, 369 x 13568 x 1088 53.7 / 23.5,
+// Q4NX 108 x 8448 x 1664 38.8 / 14.0.
+WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scratch_bytes) {
     const auto &tune = g_gemv_ws_tune;
     const int tiles = (M + 15) / 16;
     WsmPlan best;
     best.us = -1;
+    double best_rank = 0;   // slices have to be 4 % faster: the estimate is no better than that
     // a tune key's form, or the tallest of its width where there is none so tall
     int only_rt = tune.wsm_rt, only_nt = tune.wsm_nt;
     if (only_rt || only_nt) {
@@ -817,15 +895,28 @@ static WsmPlan plan_wsm_rounded(int M, int K, int N, bool q4) {
     for (const SmForm &f : kSmForms) {
         if ((only_rt && f.rt != only_rt) || (only_nt && f.nt != only_nt) || (f.rt > 8 && K >= 1 << 23)) continue;   // (the copies' 32-bit offsets)
         WsmPlan p;
-        p.rt = f.rt, p.nt = f.nt, p.slices = 1, p.blocks = (tiles + f.rt - 1) / f.rt;
-        p.us = wsm_rounded_us(f, p.blocks, K, N, q4);
-        if (best.us < 0 || p.us < best.us) best = p;
+        p.rt = f.rt, p.nt = f.nt, p.blocks = (tiles + f.rt - 1) / f.rt;
+        auto fits = [&](int slices) {
+            p.slices = slices;
+            return slices <= 1 || (K / kGroup / slices >= 8 && M <= kWsmSliceRows &&
+                                   gemm_wsm_scratch_bytes(p, M, N * matrices) <= std::min(scratch_bytes, gemm_wsm_parts_bytes(M, N * matrices)));
+        };
+        const int only = tune.wsm_slices && fits(tune.wsm_slices) ? tune.wsm_slices : 0;
+        for (int slices : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (only) slices = only;
+            if (!fits(slices)) break;
+            p.us = wsm_rounded_us(f, p.blocks * slices * matrices, (K / kGroup + slices - 1) / slices * kGroup, N, q4);
+            if (slices > 1) p.us += 0.98 + 0.21 * ((slices + 7) / 8) + slices * matrices * ((double)M * N * 8e-6 / 3.52);
+            const double rank = slices > 1 ? 1.04 * p.us : p.us;
+            if (best.us < 0 || rank < best_rank) best = p, best_rank = rank;
+            if (only) break;
+        }
     }
     return best;
 }
 
 WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch_bytes) {
-    if (rounded) return plan_wsm_rounded(M, K, N, q4);
+    if (rounded) return plan_wsm_rounded(M, K, N, 1, q4, scratch_bytes);
     const auto &tune = g_gemv_ws_tune;
     const int tiles = (M + 15) / 16, G = K / kGroup, most = 7, least = 2, few = (tiles + most - 1) / most;
     const int only_nt = tune.wsm_nt <= 2 ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
@@ -859,26 +950,60 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
 
 bool gemm_wsm_supported(int M, int K, int N) { return M > 16 && K > 0 && K % kGroup == 0 && K < 1 << 24 && N > 0 && N % kWsTileCols == 0; }
 
-size_t gemm_wsm_scratch_bytes(const WsmPlan &p, int M, int N) { return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0; }
+// (a second matrix: rounded weights; both products' parts, or each to its own y)
+static hipError_t launch_wsm_products(const WsmPlan &plan, const uint16_t *x, const void *w, const void *w2, uint16_t *y, uint16_t *y2, const uint16_t *residual, float *scratch, int M,
+                                      int K, int N, bool q4, bool rounded, hipStream_t stream) {
+    SmArgs p;
+    p.x = x;
+    p.w = static_cast<const char *>(w), p.w2 = static_cast<const char *>(w2);
+    p.partial = scratch;
+    p.y = y, p.y2 = y2;
+    p.residual = residual;
+    p.M = M, p.K = K, p.N = N, p.G = K / kGroup, p.NB = ws_blocks(K);
+    if (M < 1 || !gemm_wsm_supported(std::max(M, 17), K, N) || (w2 && !rounded)) return hipErrorInvalidValue;   // (the smallest products have other kernels, not other limits)
+    p.own_sets = (N + 64 * plan.nt - 1) / (64 * plan.nt);
+    p.sets = w2 ? 2 * p.own_sets : p.own_sets;
+    p.slices = plan.slices, p.blocks = plan.blocks;
+    if (plan.slices > 1 && !scratch) return hipErrorInvalidValue;
+    return q4 ? (rounded ? launch_wsm_mode<kSmQ4Rounded>(plan, p, stream) : launch_wsm_mode<kSmQ4>(plan, p, stream))
+              : (rounded ? launch_wsm_mode<kSmAwqRounded>(plan, p, stream) : launch_wsm_mode<kSmAwq>(plan, p, stream));
+}
 
 hipError_t launch_gemm_wsm(const WsmPlan &plan, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *residual, float *scratch, int M, int K, int N,
                            bool q4, bool rounded, hipStream_t stream) {
-    SmArgs p;
-    p.x = x;
-    p.w = static_cast<const char *>(w);
-    p.partial = scratch;
-    p.y = y;
-    p.residual = residual;
-    p.M = M, p.K = K, p.N = N, p.G = K / kGroup, p.NB = ws_blocks(K);
-    if (!gemm_wsm_supported(M, K, N)) return hipErrorInvalidValue;
-    p.sets = (N + 64 * plan.nt - 1) / (64 * plan.nt);
-    p.slices = plan.slices, p.blocks = plan.blocks;
-    if (plan.slices > 1 && !scratch) return hipErrorInvalidValue;
-    const hipError_t e = q4 ? (rounded ? launch_wsm_mode<kSmQ4Rounded>(plan, p, stream) : launch_wsm_mode<kSmQ4>(plan, p, stream))
-                            : (rounded ? launch_wsm_mode<kSmAwqRounded>(plan, p, stream) : launch_wsm_mode<kSmAwq>(plan, p, stream));
+    const hipError_t e = launch_wsm_products(plan, x, w, nullptr, y, nullptr, residual, scratch, M, K, N, q4, rounded, stream);
     if (e != hipSuccess || plan.slices == 1) return e;
     const size_t mn = (size_t)M * N;   // N % 16 == 0: whole groups of four columns
-    hipLaunchKernelGGL(plan.slices <= 2 ? &gemm_wsm_sum_kernel<2> : plan.slices <= 4 ? &gemm_wsm_sum_kernel<4> : &gemm_wsm_sum_kernel<8>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, residual, y, mn, plan.slices);
+    parts_at_a_time(plan.slices, [&](auto at) {
+        constexpr int AT = decltype(at)::value;
+        hipLaunchKernelGGL((rounded ? &gemm_wsm_sum_kernel<AT, true> : &gemm_wsm_sum_kernel<AT, false>), dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, scratch, residual, y, mn,
+                           plan.slices);
+    });
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_wsm_rope(const WsmPlan &plan, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *lut, const GemmRope &rope, float *scratch, int M, int K, int N,
+                                bool q4, hipStream_t stream) {
+    if (rope.head_dim % 8 || rope.head_dim <= 0 || rope.cols % rope.head_dim || N % rope.head_dim) return hipErrorInvalidValue;
+    const hipError_t e = launch_wsm_products(plan, x, w, nullptr, y, nullptr, nullptr, scratch, M, K, N, q4, true, stream);
+    if (e != hipSuccess) return e;
+    const int cols = plan.slices > 1 ? N : rope.cols;
+    const unsigned grid = (unsigned)(((size_t)M * (cols / 8) + 255) / 256);
+    auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, scratch, plan.slices, lut, y, M, N, cols, rope.cols, rope.head_dim, rope.pos0); };
+    if (plan.slices == 1) run(&gemm_wsm_rope_kernel<0>);
+    else parts_at_a_time(plan.slices, [&](auto at) { run(&gemm_wsm_rope_kernel<decltype(at)::value>); });
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_wsm_swiglu(const WsmPlan &plan, const uint16_t *x, const void *w_gate, const void *w_up, uint16_t *gate, uint16_t *h, float *scratch, int M, int K, int H, bool q4,
+                                  hipStream_t stream) {
+    const hipError_t e = launch_wsm_products(plan, x, w_gate, w_up, gate, h, nullptr, scratch, M, K, H, q4, true, stream);
+    if (e != hipSuccess) return e;
+    const size_t mn = (size_t)M * H;
+    const unsigned grid = (unsigned)((mn / 4 + 255) / 256);
+    auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, scratch, plan.slices, gate, h, mn); };
+    if (plan.slices == 1) run(&gemm_wsm_swiglu_kernel<0>);
+    else parts_at_a_time(plan.slices, [&](auto at) { run(&gemm_wsm_swiglu_kernel<decltype(at)::value>); });
     return hipGetLastError();
 }
 

@@ -140,8 +140,18 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
 size_t gemm_wsm_scratch_bytes(const WsmPlan &p, int M, int N);
 hipError_t launch_gemm_wsm(const WsmPlan &p, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *residual, float *scratch, int M, int K, int N,
                            bool q4, bool rounded, hipStream_t stream);
+// Rounded weights, any number of rows: for one or two matrices of a shape in one launch, and the same with RoPE or SwiGLU behind it (the bits of the tiled kernel's
+// epilogues on this product); `gate` [M, H] is scratch.
+WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scratch_bytes);
+constexpr int kWsmSliceRows = 512;           // more rows run whole K
+size_t gemm_wsm_parts_bytes(int M, int N);   // the most scratch that such a plan asks for
+hipError_t launch_gemm_wsm_rope(const WsmPlan &p, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *lut, const GemmRope &rope, float *scratch, int M, int K, int N,
+                                bool q4, hipStream_t stream);
+hipError_t launch_gemm_wsm_swiglu(const WsmPlan &p, const uint16_t *x, const void *w_gate, const void *w_up, uint16_t *gate, uint16_t *h, float *scratch, int M, int K, int H, bool q4,
+                                  hipStream_t stream);
 // Prefill GEMM on stream-order weights (gemm_ws.hip): bf16-rounded weights dequantised in registers, x through LDS.
 bool gemm_prefill_ws_supported(int M, int K, int N);   // K % 256 == 0, N % 64 == 0
+double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4);
 double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes);   // its time without an epilogue, an estimate for choosing between the kernels
 size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most);   // plain scratch that makes it faster (0: none)
 // Epilogues as for launch_gemm_prefill (kEpi*); kEpiRope with heads of 128 needs N % 128 == 0.
@@ -168,6 +178,7 @@ struct PrefillLinear {
 };
 bool prefill_block_supported(int M, int E, int H);
 size_t prefill_block_scratch_bytes(int M, int E, int H);   // sized for split-K on a 256-CU device
+size_t prefill_qkv_scratch_bytes(int M, int E);
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream);
 // Causal GQA attention over the M rows of a prefill (prefill_attention.hip); qkv is [M, (n_heads + 2 n_kv) * head_dim].
 // With caches [n_kv, max_seq, head_dim] their rows 0 .. M - 1 become the K and V of qkv.
@@ -181,11 +192,12 @@ hipError_t launch_prefill_o_ffn(const uint16_t *attn_out, const uint16_t *x_resi
                                 const PrefillLinear &wo, const PrefillLinear &wg, const PrefillLinear &wu,
                                 const PrefillLinear &wd, uint16_t *y, uint16_t *res1_out, uint16_t *h_out, int M, int E,
                                 int H, void *workspace, int cus, hipStream_t stream);
-// The same blocks on stream-order weights (every matrix re-packed with launch_repack_ws; `q4`: with launch_repack_ws_q4).
+// The same blocks on stream-order weights (every matrix re-packed with launch_repack_ws; `q4`: with launch_repack_ws_q4); workspaces of prefill_qkv_scratch_bytes
+// and prefill_block_scratch_bytes.
 bool prefill_block_stream_supported(int M, int E, int H);
 hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t *norm_w, float eps, const void *wqkv,
                                               const uint16_t *rope_lut, int pos0, uint16_t *qkv_out, int M, int E, int n_heads,
-                                              int n_kv, int head_dim, uint16_t *normed, hipStream_t stream, bool q4 = false);
+                                              int n_kv, int head_dim, void *workspace, hipStream_t stream, bool q4 = false);
 hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t *x_residual, const uint16_t *ffn_norm_w, float eps,
                                        const void *wo, const void *wg, const void *wu, const void *wd, uint16_t *y,
                                        uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace,

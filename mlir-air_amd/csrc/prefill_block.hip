@@ -9,6 +9,8 @@
 // A GEMM whose 256 x 256 tiles number less than half the CUs (the O and down projections at the 1B
 // model's width) runs split along K, and a small kernel sums the fp32 slices and applies the epilogue.
 // The reference's separate add, SwiGLU and up-projection outputs never reach HBM on their own.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -84,9 +86,20 @@ static size_t splitk_bytes(int M, int E, int H, int cus) {
     return d > b ? d : b;
 }
 
+static size_t tail_bytes(int M, int E, int H) { return std::max(splitk_bytes(M, E, H, kPlanCus), gemm_wsm_parts_bytes(M, std::max(E, 2 * H))); }
+static size_t block_rows_bytes(int M, int E, int H) { return 2 * round256((size_t)M * E * sizeof(uint16_t)) + 2 * round256((size_t)M * H * sizeof(uint16_t)); }
+
+// (a workspace for many rows also serves fewer of them, whose products run in slices)
 size_t prefill_block_scratch_bytes(int M, int E, int H) {
-    return 2 * round256((size_t)M * E * sizeof(uint16_t)) + 2 * round256((size_t)M * H * sizeof(uint16_t)) +
-           round256(splitk_bytes(M, E, H, kPlanCus));
+    const int few = std::min(M, kWsmSliceRows);
+    return std::max(block_rows_bytes(M, E, H) + round256(tail_bytes(M, E, H)), block_rows_bytes(few, E, H) + round256(gemm_wsm_parts_bytes(few, std::max(E, 2 * H))));
+}
+
+// Behind the normed rows: parts of the projections of few rows (how wide those are the call says; three times E where every head has keys of its own)
+static size_t qkv_parts_bytes(int M, int E) { return round256(gemm_wsm_parts_bytes(M, 3 * E)); }
+size_t prefill_qkv_scratch_bytes(int M, int E) {
+    const int few = std::min(M, kWsmSliceRows);
+    return std::max(round256((size_t)M * E * sizeof(uint16_t)) + qkv_parts_bytes(M, E), round256((size_t)few * E * sizeof(uint16_t)) + qkv_parts_bytes(few, E));
 }
 
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream) {
@@ -144,23 +157,39 @@ bool prefill_block_stream_supported(int M, int E, int H) {
            gemm_prefill_ws_supported(M, H, E);
 }
 
+// Whether gemm_wsm.hip takes a product of rounded weights: by time (tune keys: always, never).  What it does in a second launch - adding slices up, `elements` bf16 numbers read and written
+// where the tiled kernel has them at hand - counts what it takes the GPU, and where the GPU is soon done the 4 us that a launch takes the host.
+static bool by_wsm(const WsmPlan &plan, double elements, double tiled_us) {
+    const auto &tune = g_gemv_ws_tune;
+    double more = plan.slices == 1 && elements > 0 ? 1.2 + elements * 4e-6 / 3.5 : 0.0;   // (the sum of slices is part of the plan's time)
+    if ((plan.slices > 1 || elements > 0) && plan.us < 12) more += 2.8;
+    return plan.us >= 0 && !tune.prefill_tile && tune.prefill_wsm != 2 && (tune.prefill_wsm == 1 || plan.us + more < 0.95 * tiled_us);
+}
+
 hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t *norm_w, float eps, const void *wqkv,
                                               const uint16_t *rope_lut, int pos0, uint16_t *qkv_out, int M, int E, int n_heads,
-                                              int n_kv, int head_dim, uint16_t *normed, hipStream_t stream, bool q4) {
+                                              int n_kv, int head_dim, void *workspace, hipStream_t stream, bool q4) {
+    uint16_t *normed = static_cast<uint16_t *>(workspace);
+    const size_t own_e = round256((size_t)M * E * sizeof(uint16_t));
     hipError_t e = launch_rmsnorm_rows(x, norm_w, normed, M, E, eps, stream);
     if (e != hipSuccess) return e;
     const GemmRope rope = {(n_heads + n_kv) * head_dim, head_dim, pos0};
-    return launch_gemm_prefill_ws(normed, wqkv, qkv_out, M, E, (n_heads + 2 * n_kv) * head_dim, stream, kEpiRope, rope_lut, &rope, q4);
+    const int N = (n_heads + 2 * n_kv) * head_dim;
+    if (gemm_wsm_supported(17, E, N)) {
+        const WsmPlan plan = plan_wsm_rounded(M, E, N, 1, q4, qkv_parts_bytes(M, E));
+        if (by_wsm(plan, (double)M * rope.cols, gemm_prefill_ws_us(M, E, N, q4, 0)))
+            return launch_gemm_wsm_rope(plan, normed, wqkv, qkv_out, rope_lut, rope, reinterpret_cast<float *>(static_cast<char *>(workspace) + own_e), M, E, N, q4, stream);
+    }
+    return launch_gemm_prefill_ws(normed, wqkv, qkv_out, M, E, N, stream, kEpiRope, rope_lut, &rope, q4);
 }
 
-// y = bf16(bf16(x . W) + aux): the kernel for a few hundred rows where it is the faster one (same bits), else the tiled one, with slices of
-// K where they pay and fit `scratch`
-static hipError_t product_add(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, const uint16_t *aux, void *scratch, size_t scratch_bytes,
-                              hipStream_t stream, bool q4) {
-    const auto &tune = g_gemv_ws_tune;
-    if (gemm_wsm_supported(M, K, N) && !tune.prefill_tile && tune.prefill_wsm != 2) {
-        const WsmPlan plan = plan_gemm_wsm(M, K, N, q4, true, 0);
-        if (tune.prefill_wsm == 1 || plan.us < 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes)) return launch_gemm_wsm(plan, x, w, y, aux, nullptr, M, K, N, q4, true, stream);
+// y = bf16(bf16(x . W) + aux): the kernel for a few hundred rows where it is the faster one, with slices of K for few rows (their parts in `tail`), else the tiled one, with slices
+// where they pay and fit `scratch`
+static hipError_t product_add(const uint16_t *x, const void *w, uint16_t *y, int M, int K, int N, const uint16_t *aux, void *scratch, size_t scratch_bytes, void *tail,
+                              size_t tail_bytes, hipStream_t stream, bool q4) {
+    if (gemm_wsm_supported(17, K, N)) {
+        const WsmPlan plan = plan_wsm_rounded(M, K, N, 1, q4, tail_bytes);
+        if (by_wsm(plan, 0.0, gemm_prefill_ws_us(M, K, N, q4, scratch_bytes))) return launch_gemm_wsm(plan, x, w, y, aux, static_cast<float *>(tail), M, K, N, q4, true, stream);
     }
     return launch_gemm_prefill_ws(x, w, y, M, K, N, stream, kEpiAddRounded, aux, nullptr, q4, static_cast<float *>(scratch), scratch_bytes);
 }
@@ -177,11 +206,14 @@ hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t 
     uint16_t *gate = reinterpret_cast<uint16_t *>(base);
     base += round256((size_t)M * H * sizeof(uint16_t));
     uint16_t *h = reinterpret_cast<uint16_t *>(base);
+    base += round256((size_t)M * H * sizeof(uint16_t));
+    float *tail = reinterpret_cast<float *>(base);
+    const size_t most = tail_bytes(M, E, H);
     // scratch of the two products with a residual: what is not in use yet (gate, h) or any more (normed, gate)
     const size_t own_h = round256((size_t)M * H * sizeof(uint16_t)), own_e = round256((size_t)M * E * sizeof(uint16_t));
     if (res1_out) res1 = res1_out;
     if (h_out) h = h_out;
-    hipError_t e = product_add(attn_out, wo, res1, M, E, E, x_residual, gate, 2 * own_h, stream, q4);
+    hipError_t e = product_add(attn_out, wo, res1, M, E, E, x_residual, gate, 2 * own_h, tail, most, stream, q4);
     if (e != hipSuccess) return e;
     e = launch_rmsnorm_rows(res1, ffn_norm_w, normed, M, E, eps, stream);
     if (e != hipSuccess) return e;
@@ -190,10 +222,14 @@ hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t 
         if (e != hipSuccess) return e;
         e = launch_gemm_prefill_ws(normed, wu, h, M, E, H, stream, kEpiSiluGateMul, gate, nullptr, q4);
     } else {
-        e = launch_gemm_prefill_ws_swiglu(normed, wg, wu, h, M, E, H, stream, q4);
+        WsmPlan plan;
+        plan.us = -1;
+        if (gemm_wsm_supported(17, E, H)) plan = plan_wsm_rounded(M, E, H, 2, q4, most);
+        if (by_wsm(plan, 1.5 * M * H, gemm_prefill_ws_swiglu_us(M, E, H, q4))) e = launch_gemm_wsm_swiglu(plan, normed, wg, wu, gate, h, tail, M, E, H, q4, stream);
+        else e = launch_gemm_prefill_ws_swiglu(normed, wg, wu, h, M, E, H, stream, q4);
     }
     if (e != hipSuccess) return e;
-    return product_add(h, wd, y, M, H, E, res1, normed, own_e + own_h, stream, q4);
+    return product_add(h, wd, y, M, H, E, res1, normed, own_e + own_h, tail, most, stream, q4);
 }
 
 }  // namespace w4a16

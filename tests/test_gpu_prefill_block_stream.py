@@ -362,3 +362,62 @@ def test_prompt_layer_on_stream_order_weights_replays_from_a_hip_graph(ops):
             for name, a, b in zip(("qkv", "attention", "block"), outs, want):
                 assert torch.isfinite(a.float()).all(), (name, j)
                 assert torch.equal(a.view(torch.int16), b.view(torch.int16)), (name, j)
+
+
+@pytest.mark.parametrize("codec", ["awq", "q4nx"])
+@pytest.mark.parametrize("M,E,H,nh,nkv,hd", [(1, 2048, 4096, 4, 2, 64), (16, 2048, 1024, 5, 1, 128), (33, 4096, 2048, 3, 1, 64), (130, 2048, 2304, 2, 1, 128), (512, 2048, 256, 2, 2, 64)])
+def test_prompt_blocks_of_few_rows(ops, codec, M, E, H, nh, nkv, hd):
+    """Products of few rows behind which RoPE, SwiGLU and the residual are launches of their own.  On whole K they have the tiled kernel's bits.  In slices the fp32 sum meets in another order: a
+    product differs by its rounding (half an ulp and what the order moves, less than 2^-16 of the sum's magnitude, together less than an ulp), which each stage passes on."""
+    from oracle import decode as odec
+    print(f"prompt blocks of few rows {codec} M={M} E={E} H={H} heads {nh}/{nkv} of {hd}", flush=True)
+    N = (nh + 2 * nkv) * hd
+
+    def weight(K, n, seed):
+        if codec == "awq":
+            return _sw(ops, _scaled(K, n, seed, 0.1))
+        from test_gpu_q4nx import make
+        q, s, m = make(n, K, seed=seed)
+        return ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+
+    wqkv, wo, wg, wu, wd = (weight(*a) for a in ((E, N, 1), (E, E, 2), (E, H, 3), (E, H, 4), (H, E, 5)))
+    attn, xres, nw = make_x((M, E), seed=6), make_x((M, E), seed=7), _norm_w(E, 8)
+    lut = odec.generate_rope_lut(hd, 500000.0, M + 3)
+
+    def blocks(wsm, slices):
+        ops.tune("prefill_wsm", wsm)
+        ops.tune("gemm_wsm_slices", slices)
+        try:
+            qkv = ops.prefill_rms_qkv_rope_stream(dev(xres), dev(nw), wqkv, dev(lut), 3, nh, nkv, hd, codec=codec)
+            return [qkv, *ops.prefill_o_ffn_stream(dev(attn), dev(xres), dev(nw), wo, wg, wu, wd, return_intermediates=True, codec=codec)]
+        finally:
+            ops.tune("prefill_wsm", 0)
+            ops.tune("gemm_wsm_slices", 0)
+
+    tiled = blocks(2, 0)
+    for got, want in zip(blocks(1, 1), tiled):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for slices in (2, 0):
+        qkv, y, res1, h = blocks(1, slices)
+        for got, want in ((qkv, tiled[0]), (res1, tiled[2])):
+            # pairs of columns half a head apart share their products; res1: the residual's ulp besides
+            bound = 2.0**-7 * want.float().abs().amax(1, keepdim=True)
+            assert bool(((got.float() - want.float()).abs() <= bound).all())
+            assert float((got != want).float().mean()) < 0.02
+        # behind the norm of other roundings: from the kernel's own intermediates, on whole K
+        normed = ops.rms_norm_rows(res1, dev(nw))
+        f = lambda t: t.double().cpu().numpy()
+        plain = ops.q4nx_gemm_stream if codec == "q4nx" else ops.w4a16_gemm_stream
+        ops.tune("prefill_min_m", 17)
+        ops.tune("prefill_wsm", 2)
+        try:
+            pad = lambda t: torch.cat([t, torch.zeros((max(0, 17 - M), t.shape[1]), dtype=t.dtype, device="cuda")])   # (fewer rows have another kernel)
+            g, u, d = (plain(pad(t), w)[:M] for t, w in ((normed, wg), (normed, wu), (h, wd)))
+        finally:
+            ops.tune("prefill_min_m", 0)
+            ops.tune("prefill_wsm", 0)
+        g, u = f(g), f(u)
+        want = g / (1.0 + np.exp(-g)) * u
+        assert np.all(np.abs(f(h) - want) <= 2 * bf16_ulp(want) + 1.2 * bf16_ulp(g) * np.abs(u) + bf16_ulp(u) * np.abs(g) + 1e-3)
+        want = f(d) + f(res1)
+        assert np.all(np.abs(f(y) - want) <= bf16_ulp(want) + bf16_ulp(f(d)) + 2e-3)
