@@ -246,6 +246,10 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
     constexpr int MDK = Q4 ? kWsQ4MdKiB : 1;   // KiB of scale words in front of a block's cells, words per (group, column)
     const size_t tile_bytes = (size_t)(MDK * p.NB + G) * kWsCellBytes;
     const bool pair = p.epi == kEpiSwigluPair;
+    // 192 columns of a pair or of heads of 128: six 16-column tiles in the left half, their partners in the right one, so that the two can meet in the
+    // LDS tile though a wave's three cannot be halved.  The q-th pair is tile q of either matrix, or the tiles 8 (q / 4) + q % 4 and four further on, which
+    // RoPE turns together (a tile of 192 columns then holds a head and half of one).
+    const bool halves = NCB == 3 && (pair || (p.epi == kEpiRope && p.rope_hd == 128));
     const char *wt = p.w + (size_t)((pair ? n0 / 2 : n0) / kWsTileCols) * tile_bytes;
     u32x4 cell[2][NCB];
     uint32_t md[2][NCB][MDK];
@@ -260,6 +264,11 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
         const char *t = wt + (size_t)c * tile_bytes;
         if (pair && NCB % 2 == 0)   // tiles NCB / 2 .. NCB - 1 of the wave: the same columns of the second matrix
             t = c < NCB / 2 ? t : p.w_up + (t - p.w) - (size_t)(NCB / 2) * tile_bytes;
+        if (halves) {
+            const int q = col0 / 32 + wave % 2 * NCB + c;
+            if (pair) t = (wave < 2 ? p.w : p.w_up) + (size_t)q * tile_bytes;
+            else t = p.w + (size_t)(8 * (q / 4) + q % 4 + (wave < 2 ? 0 : 4)) * tile_bytes;
+        }
         tile_base[c] = scalar_ptr(t);
     }
     struct WOffsets {
@@ -563,14 +572,19 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
             const int row = chunk / CPR, cc = chunk % CPR;
             if (m0 + row >= M) continue;
             u32x4 v = *reinterpret_cast<const u32x4 *>(&ct[row * LDC + 8 * cc]);
-            const int grow = m0 + row, gcol = col0 + 8 * cc;
+            int gcol = col0 + 8 * cc;
+            if (kEpi == kEpiRope && halves) {   // (where the chunk's tile is: see above)
+                const int q = col0 / 32 + cc % (CPR / 2) / 2;
+                gcol = 128 * (q / 4) + 16 * (q % 4) + 8 * (cc % 2) + (cc < CPR / 2 ? 0 : 64);
+            }
+            const int grow = m0 + row;
             const size_t at = (size_t)grow * N + gcol;
             if constexpr (kEpi == kEpiRope) {
                 if (gcol < p.rope_cols) {
-                    const int hd = p.rope_hd, half = hd >> 1;
+                    const int hd = p.rope_hd, half = hd >> 1, apart = halves ? TN / 2 : half;
                     const int i = gcol & (hd - 1);
                     const bool low = i < half;
-                    const u32x4 w2 = *reinterpret_cast<const u32x4 *>(&ct[row * LDC + 8 * cc + (low ? half : -half)]);
+                    const u32x4 w2 = *reinterpret_cast<const u32x4 *>(&ct[row * LDC + 8 * cc + (low ? apart : -apart)]);
                     const uint16_t *lut = p.aux + (size_t)(p.rope_pos0 + grow) * hd + (low ? i : i - half);
                     const u32x4 cs = *reinterpret_cast<const u32x4 *>(lut), sn = *reinterpret_cast<const u32x4 *>(lut + half);
 #pragma unroll
@@ -599,13 +613,13 @@ __device__ __forceinline__ void pf_tile(const PfArgs &p, unsigned char *lds, int
         }
     };
     if (pair) {
-        if constexpr (NCB % 2 == 0) {
-            constexpr int HW = WN / 2, OCPR = TN / 16;   // output columns per wave, 16-byte output chunks per row
+        if constexpr (NCB > 1) {
+            constexpr int HW = NCB % 2 == 0 ? WN / 2 : TN / 2, WW = NCB % 2 == 0 ? WN : TN, OCPR = TN / 16;   // output columns per wave, 16-byte output chunks per row
             const int Nout = N, ocol0 = col0 / 2;
             for (int chunk = threadIdx.x; chunk < TM * OCPR; chunk += kPfThreads) {
                 const int row = chunk / OCPR, oc = 8 * (chunk % OCPR);
                 if (m0 + row >= M) continue;
-                const uint16_t *src = &ct[row * LDC + (oc / HW) * WN + oc % HW];
+                const uint16_t *src = &ct[row * LDC + (oc / HW) * WW + oc % HW];
                 const u32x4 gv = *reinterpret_cast<const u32x4 *>(src), uv = *reinterpret_cast<const u32x4 *>(src + HW);
                 u32x4 v;
 #pragma unroll
@@ -666,7 +680,7 @@ __global__ void __launch_bounds__(kPfThreads, 1) gemm_wsp_kernel(const PfArgs p)
 struct Widths {
     int ncb;            // columns / 64 of the "wide" tiles: 4, or 2 / 1 for the narrow uniform tilings
     int wide, narrow;   // number of column tiles of ncb * 64 columns and of the narrow width
-    int ncb_narrow = 3; // columns / 64 of the narrow tiles of a mixed launch: 3, or 2 where tiles must be halves or whole heads
+    int ncb_narrow = 3; // columns / 64 of the narrow tiles of a mixed launch: 3, or 2 where columns come in pairs
 };
 
 double split_cost(long n_wide_tiles, long n_narrow_tiles, int cus, double narrow_cost) {
@@ -684,8 +698,10 @@ double split_cost(long n_wide_tiles, long n_narrow_tiles, int cus, double narrow
     return *std::max_element(load.begin(), load.end());
 }
 
-// `heads128`: every tile must hold whole heads of 128 columns (RoPE epilogue) or halve into whole 16-column tiles
-// (gate and up in one tile): no 192- or 64-column tiles; the wide tiles are then mixed with 128-column ones.
+// `heads128`: a tile's columns come in pairs, of RoPE heads of 128 or of gate and up: no 64-column tiles, and 192 columns as two halves (pf_tile); 128-column ones may
+// stand beside the wide ones too, at 2.8 for 3.  (Those alone before there were halves: gate and up of 2048 x 14336 x 4096 four tiles a CU either way, 410 -> 389 us, Q | K | V of
+// 2048 x 6144 x 4096 122 -> 105 in one round of 192 instead of three quarters of one of 256.  Prompts of four layers, same bits: width 4096 and 14336, 2048 tokens, where the clock gives way,
+// 3184 -> 3163 us, 1500 2619 -> 2566, 1000 1974 -> 1891, 700 1634 -> 1540; width 2048 and 8192, 2048 tokens 1338 -> 1300.)
 Widths pick_widths(int tiles_m, int U, int cus, bool heads128) {
     struct Entry {
         int tiles_m, U, cus;
@@ -700,18 +716,16 @@ Widths pick_widths(int tiles_m, int U, int cus, bool heads128) {
         if (e.U == U && e.tiles_m == tiles_m && e.cus == cus && e.heads128 == heads128) return e.w;
     Widths best{4, -1, -1};
     double best_cost = -1;
-    const int nn = heads128 ? 2 : 3;
-    const double narrow_cost = heads128 ? 2 * kPfSlowdown128 : 3.0;
-    for (int a = U / 4; a >= 0; --a) {   // ties go to the split with more wide tiles
-        if ((U - 4 * a) % nn) continue;
-        const int b = (U - 4 * a) / nn;
-        if (a == 0 && heads128) continue;   // (the uniform 128-column tiling is priced below)
-        const double cost = split_cost((long)tiles_m * a, (long)tiles_m * b, cus, narrow_cost);
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = Widths{4, a, b, nn};
+    for (int nn = 3; nn >= (heads128 ? 2 : 3); --nn)
+        for (int a = U / 4; a >= (nn == 2 ? 1 : 0); --a) {   // ties go to the split with more wide tiles (the uniform 128-column tiling is priced below)
+            if ((U - 4 * a) % nn) continue;
+            const int b = (U - 4 * a) / nn;
+            const double cost = split_cost((long)tiles_m * a, (long)tiles_m * b, cus, nn == 2 ? 2 * kPfSlowdown128 : 3.0);
+            if (best_cost < 0 || cost < best_cost) {
+                best_cost = cost;
+                best = Widths{4, a, b, nn};
+            }
         }
-    }
     // uniform narrow tilings: rounds x width x (measured) slowdown of the narrower tile's inner loop
     const struct { int ncb; double slowdown; } narrow[2] = {{2, kPfSlowdown128}, {1, kPfSlowdown64}};
     for (const auto &nv : narrow) {
@@ -811,7 +825,7 @@ double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes) { 
 double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
     const Widths wd = pick_widths(tiles_m, 2 * H / 64, 256, true);
-    return wsp_us(K, (long)tiles_m * (wd.wide + (wd.ncb == 4 ? wd.narrow : 0)), wd.ncb, q4);
+    return wsp_us(K, (long)tiles_m * (wd.wide + (wd.ncb == 4 ? wd.narrow : 0)), wd.wide ? wd.ncb : 3, q4);
 }
 size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most) {
     const int s = wsp_slices(M, K, N, q4, most).slices;
@@ -852,7 +866,7 @@ hipError_t launch_gemm_prefill_ws(const uint16_t *x, const void *w, uint16_t *y,
     // where the launch takes that mix (RoPE heads of 128, gate and up in one tile)
     const int force = g_gemv_ws_tune.prefill_tile;
     if (force == 1 && U % 4 == 0) wd = Widths{4, U / 4, 0};
-    if (force == 2 && U % 3 == 0 && !heads128) wd = Widths{4, 0, U / 3};
+    if (force == 2 && U % 3 == 0) wd = Widths{4, 0, U / 3};
     if (force == 3 && U % 2 == 0) wd = Widths{2, U / 2, 0};
     if (force == 4 && !heads128) wd = Widths{1, U, 0};
     if (force == 5 && heads128 && U % 2 == 0 && U >= 6) wd = Widths{4, (U - 2) / 4, U % 4 == 0 ? 2 : 1, 2};
@@ -882,15 +896,21 @@ hipError_t launch_gemm_prefill_ws_swiglu(const uint16_t *x, const void *w_gate, 
     p.M = M, p.K = K, p.N = H, p.G = K / kGroup, p.NB = ws_blocks(K);
     p.tiles_m = (M + kPfRows - 1) / kPfRows;
     p.band = pf_band(p.tiles_m);
-    const int U = 2 * H / 64;   // the tile grid runs over 2 H columns; 192- and 64-column tiles cannot be halved
+    const int U = 2 * H / 64;   // the tile grid runs over 2 H columns
     Widths wd = pick_widths(p.tiles_m, U, 256, true);
     const int force = g_gemv_ws_tune.prefill_tile;
     if (force == 1 && U % 4 == 0) wd = Widths{4, U / 4, 0};
+    if (force == 2 && U % 3 == 0) wd = Widths{4, 0, U / 3};
     if (force == 3) wd = Widths{2, U / 2, 0};
     if (force == 5 && U >= 6) wd = Widths{4, (U - 2) / 4, U % 4 == 0 ? 2 : 1, 2};
     p.n_wide = wd.wide, p.n_narrow = wd.ncb == 4 ? wd.narrow : 0;
     if (wd.ncb == 2) return launch_wsp<2, 0>(p, stream);
-    return p.n_narrow ? launch_wsp<4, 2>(p, stream) : launch_wsp<4, 0>(p, stream);
+    if (wd.wide == 0) {
+        p.n_wide = wd.narrow, p.n_narrow = 0;
+        return launch_wsp<3, 0>(p, stream);
+    }
+    if (wd.narrow == 0) return launch_wsp<4, 0>(p, stream);
+    return wd.ncb_narrow == 2 ? launch_wsp<4, 2>(p, stream) : launch_wsp<4, 3>(p, stream);
 }
 
 }  // namespace w4a16

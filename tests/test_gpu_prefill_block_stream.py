@@ -279,6 +279,17 @@ def test_prefill_rms_qkv_rope_stream(ops, tiled_gemm, M, E, nh, nkv, hd, pos0, t
     assert np.mean(got != ref_r) < 0.1, np.mean(got != ref_r)
 
 
+# 192-column tiles of heads of 128 (a head and half of one) and of gate and up: one of them, several, beside wide ones, ragged rows
+@pytest.mark.parametrize("M,E,nh,nkv,pos0,tile", [(100, 256, 1, 1, 4, 2), (270, 512, 4, 1, 0, 2), (2048, 256, 9, 3, 9, 0), (1000, 256, 32, 8, 2, 0)])
+def test_prefill_rms_qkv_rope_stream_in_192_columns(ops, tiled_gemm, M, E, nh, nkv, pos0, tile):
+    test_prefill_rms_qkv_rope_stream(ops, tiled_gemm, M, E, nh, nkv, 128, pos0, tile)
+
+
+@pytest.mark.parametrize("M,E,H,tile", [(130, 256, 768, 2), (300, 512, 1536, 2), (2048, 256, 14336, 0), (700, 256, 9728, 0)])
+def test_prefill_block_stream_gate_up_in_192_columns(ops, M, E, H, tile):
+    test_prefill_block_stream_paired_gate_up_launch_equals_two_launches(ops, M, E, H, tile)
+
+
 def test_prefill_rms_qkv_rope_stream_position_zero_is_the_identity(ops, tiled_gemm):
     """Every row at position 0 (a one-row table, cos = 1, sin = 0) leaves Q and K unrotated: the fused call equals
     RMSNorm + plain GEMM bit for bit; and shifting pos0 equals shifting the table."""
