@@ -18,6 +18,11 @@
 //
 // Head sizes that are common have kernels of their own (EXACT: everything unrolled); any other size runs on the next
 // larger register allotment with uniform bounds.
+//
+// What bounds it: the chain of a block of keys.  In the kernels of their own four operands are on their way from LDS while one is multiplied (five to six spill), and
+// no load of the queries can be in flight when the loop begins.  (Before, every block waited for the next one to arrive from memory and for most of its LDS reads one
+// by one.  us, 2048 tokens: 16 heads of 128 + 64 / 128 62.6 -> 56.1, 8 heads 53.0 -> 43.2; 16 windowed heads of 128 over 4, window 1024 32.9 -> 29.7, window 2048 50.2 -> 43.6; of 64,
+// window 2048 32.9 -> 26.9.  Taken back on top: the keys stored beside the softmax and the values beside the scores, the two sets half a block apart: 2 to 40 % slower.)
 #include <algorithm>
 
 #include "dense.h"
@@ -109,6 +114,10 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
         m[b] = kNoMax;
     }
 
+    // the queries have arrived before the first block is asked for: with these loads possibly in flight the compiler waits for everything asked for since,
+    // the next block included, in front of the first product of every block
+    if constexpr (EXACT) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+
     // a chunk is 8 elements of a row; the first dim of a K row come from the expanded matrix, the rest from the cache
     const T *k_base = p.kv + kvh * p.head_k, *v_base = p.kv + p.v_off + kvh * p.head_v + vcol0, *r_base = p.cache + p.rot_off;
     auto row_of = [&](int kb, int i) {   // row of key kb + i of a block (a ring holds whole blocks)
@@ -166,17 +175,37 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
         if (it + SETS < blocks) fetch(it + SETS);
         if (it < blocks && kb <= wave_last && (!WINDOW || kb + KB > wave_first)) {
             floatx4 s[NKK][QB];
+            if constexpr (EXACT) {   // kAhead operands are on their way from LDS (left to itself the compiler asks for one, waits, multiplies)
+                constexpr int N = NKK * NQ, kAhead = 4;
+                Vec8<T> a[kAhead];
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) {
+                for (int kk = 0; kk < NKK; ++kk)
 #pragma unroll
-                for (int b = 0; b < QB; ++b) s[kk][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    for (int b = 0; b < QB; ++b) s[kk][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+                auto ask = [&](int n) { a[n % kAhead] = load8(kt + (16 * (n / NQ) + ql) * kp + 32 * (n % NQ) + 8 * g); };
 #pragma unroll
-                for (int ks = 0; ks < NQ; ++ks)
-                    if (EXACT || ks < nq) {
-                        const Vec8<T> a = load8(kt + (16 * kk + ql) * kp + 32 * ks + 8 * g);
+                for (int n = 0; n < kAhead; ++n) ask(n);
 #pragma unroll
-                        for (int b = 0; b < QB; ++b) s[kk][b] = mma32(a, qf[b][ks], s[kk][b]);
-                    }
+                for (int n = 0; n < N; ++n) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b) s[n / NQ][b] = mma32(a[n % kAhead], qf[b][n % NQ], s[n / NQ][b]);
+                    if (n + kAhead < N) ask(n + kAhead);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < NKK; ++kk) {
+#pragma unroll
+                    for (int b = 0; b < QB; ++b) s[kk][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int ks = 0; ks < NQ; ++ks)
+                        if (ks < nq) {
+                            const Vec8<T> a = load8(kt + (16 * kk + ql) * kp + 32 * ks + 8 * g);
+#pragma unroll
+                            for (int b = 0; b < QB; ++b) s[kk][b] = mma32(a, qf[b][ks], s[kk][b]);
+                        }
+                }
             }
             // s[kk][b][r]: key kb + 16 kk + 4 g + r against query qpos[b]
             const bool masked = kb + KB - 1 > pos0 + q0;
@@ -185,18 +214,22 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
 #pragma unroll
             for (int b = 0; b < QB; ++b) {
                 if (masked) {
+                    int last = qpos[b] - kb - 4 * g;   // (in here: in front of the products it would take registers)
+                    if constexpr (EXACT) asm volatile("" : "+v"(last));
 #pragma unroll
                     for (int kk = 0; kk < NKK; ++kk)
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            if (kb + 16 * kk + 4 * g + r > qpos[b]) s[kk][b][r] = kMasked;
+                            if (16 * kk + r > last) s[kk][b][r] = kMasked;
                 }
                 if (WINDOW && kb <= wave_last - p.window) {
+                    int hidden = qpos[b] - p.window - kb - 4 * g;
+                    if constexpr (EXACT) asm volatile("" : "+v"(hidden));
 #pragma unroll
                     for (int kk = 0; kk < NKK; ++kk)
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            if (kb + 16 * kk + 4 * g + r <= qpos[b] - p.window) s[kk][b][r] = kMasked;
+                            if (16 * kk + r <= hidden) s[kk][b][r] = kMasked;
                 }
                 float v = kMasked;
 #pragma unroll
@@ -232,11 +265,26 @@ __global__ void __launch_bounds__(SETS * kSetThreads, SETS) latent_prefill_kerne
                     l[b] = mma32(ones8<T>(), pb[b][t], l[b]);
                 }
             }
+            if constexpr (EXACT) {
+                constexpr int N = NT * NV, kAhead = 4;
+                Vec8<T> a[kAhead];
+                auto ask = [&](int n) { a[n % kAhead] = column8(vt + 32 * (n / NV) * vp, vp, 16 * (n % NV)); };
+#pragma unroll
+                for (int n = 0; n < kAhead; ++n) ask(n);
+#pragma unroll
+                for (int n = 0; n < N; ++n) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b) o[b][n % NV] = mma32(a[n % kAhead], pb[b][n / NV], o[b][n % NV]);
+                    if (n + kAhead < N) ask(n + kAhead);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            } else
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int d = 0; d < NV; ++d)
-                    if (EXACT || d < nv) {
+                    if (d < nv) {
                         const Vec8<T> a = column8(vt + 32 * t * vp, vp, 16 * d);
 #pragma unroll
                         for (int b = 0; b < QB; ++b) o[b][d] = mma32(a, pb[b][t], o[b][d]);
@@ -398,11 +446,11 @@ PrefillArgs<T> args_of(const HeadShape &s, const HeadRows &r, const void *q, voi
     return p;
 }
 
-// Whether a workgroup takes 64 queries, 16 to a wave, instead of 128, for heads of 128 + 64 / 128 and of 128 / 128 behind long windows.  A block of 64 keys takes a wave set 2.75 us
-// with 16 queries to a wave and 3.3 with 32 (staging, scores, softmax and outputs are a chain between two barriers, a workgroup has its CU to itself): the longest item is done
-// sooner, all of them together take 1.7 times as long.  So where they are no more than 256 CUs have room for beside the longest.  us, 128 / 64 queries, 16 heads of 128 + 64 / 128:
-// 128 tokens 12.3 / 8.4, 1024 33.0 / 26.3, 1500 45.5 / 36.9, 3000 81.1 / 112.8, 500 behind 500 31.6 / 24.1, 1000 behind 3000 104.1 / 94.0, 2048 behind 2048 107.9 / 145.9; 64 heads: 300
-// 16.1 / 13.5, 1024 47.7 / 61.6.  (On the line, 16 heads and 2048 tokens, 58.9 / 54.1 alone, but 3 us more between a model's products.)
+// Whether a workgroup takes 64 queries, 16 to a wave, instead of 128, for heads of 128 + 64 / 128 and of 128 / 128 behind long windows.  A block of 64 keys takes a wave set 2.3 us
+// with 16 queries to a wave and 3.0 with 32 (staging, scores, softmax and outputs are a chain between two barriers, a workgroup has its CU to itself): the longest item is done
+// sooner, all of them together take 1.5 times as long.  So where they are no more than 256 CUs have room for beside the longest.  us, 128 / 64 queries, 16 heads of 128 + 64 / 128:
+// 128 tokens 13.3 / 9.2, 1000 31.6 / 24.9, 1500 43.2 / 35.2, 1800 50.2 / 45.6, 3000 80.2 / 108.8; 8 heads 3000 73.6 / 62.6; 32 heads 700 25.1 / 20.7, 1000 33.8 / 32.6, 2048 74.0 / 99.4.
+// (On the line, 16 heads and 2048 tokens, 56.0 / 52.8.)
 template <class T>
 long item_blocks(const PrefillArgs<T> &p, long first, long queries = 64) {   // blocks of 64 keys of the item of so many queries from position `first` on
     const long end = std::min<long>(first + queries, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
@@ -421,10 +469,8 @@ bool few_queries(const PrefillArgs<T> &p) {
 
 // Whether windowed heads that otherwise take 64 queries to a workgroup take 128 after all: 512 items of 64 or fewer, two to a CU, of which more than 256 are nearly as long as the
 // longest.  Two long ones on a CU take 1.02 us a block of keys together, one alone 0.76, an item of 128 queries 0.93 (heads of 64); where lengths differ a long one shares with short ones.
-// us, 128 / 64 queries, heads of 64: 8, window 2048, 4096 tokens 31.4 / 33.4 (512 items, 280 of them long), 16, window 4096, 2048 tokens behind 4096 56.0 / 62.9, 1500 55.0 / 61.3;
-// but 6, window 2048, 4096 tokens 31.0 / 27.6 (384 and 210), 16, window 1024, 3000 tokens 32.2 / 24.4 (752 items); below 17 blocks 0.95 to 1.01 times.  Heads of 128 (windows up to 768): 16
-// of them, 2048 tokens, windows of 640 22.1 / 22.9, 768 24.5 / 25.7, but 576 22.1 / 21.6, 704 24.6 / 23.2: the two wave sets of 128 queries take blocks in turn, so an odd number costs
-// them one more.
+// us, 128 / 64 queries, heads of 64: 8, window 2048, 4096 tokens 32.0 / 35.0, window 1024 19.8 / 21.4; heads of 128 (windows up to 768): 16 of them, 2048 tokens, window 640 23.2 / 25.1,
+// but 4096 tokens 46.8 / 45.6.  The two wave sets of 128 queries take blocks in turn, so an odd number costs them one more.
 template <class T>
 bool even_round(const PrefillArgs<T> &p, bool wide) {
     const long items = (p.M + 63) / 64 * (long)p.heads, start = p.total - p.M;
@@ -456,6 +502,7 @@ hipError_t launch_latent_prefill(int dtype, const LatentShape &s, const LatentRo
     if ((double)p.total * ldkv * sizeof(bf16) < 4e9) {
         if (nq == 6 && nv == 8) return few_queries(p) ? launch<bf16, 6, 8, 1, 32, 2, true>(p, stream) : launch<bf16, 6, 8, 2, 64, 2, true>(p, stream);
         // (two workgroups to a CU: 4 to 64 heads, 128 to 4096 tokens 1.0 to 1.4 times as fast as with 128 queries)
+        if (nq == 4 && nv == 4) return launch<bf16, 4, 4, 1, 64, 2, true>(p, stream);
         if (nq == 3 && nv == 4) return launch<bf16, 3, 4, 1, 64, 2, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false>(p, stream);
@@ -478,10 +525,13 @@ hipError_t launch_head_prefill(int dtype, const HeadShape &s, const HeadRows &r,
     }
     const PrefillArgs<bf16> p = args_of<bf16>(s, r, q, out, ldo);
     if ((double)s.ring * (s.dim + s.vdim) * sizeof(bf16) < 4e9) {
+        // (128 / 64, also behind 96 + 32 / 64 above: bounds were asked at every operand.  16 heads, 2048 tokens, window 1024 74 -> 25.5 us, 300 30 -> 13.8; 96 + 32 / 64, 16 heads, 2048
+        // tokens 141 -> 34.2, 1000 71.5 -> 16.6.  By 128 queries 24.6, 14.6, 39.0, 22.0; blocks of 32 keys 0 to 4 % slower.)
         // (windows of few blocks are mostly start and end, which the smaller items share a CU for: 16 to 64 heads, 1024 to 4096 tokens, windows of 64 to 256 1.03 to 1.4 times
         // as fast, of 384 to 700 0.99 to 1.3)
         if (nq == 4 && nv == 8)
             return (p.window <= 768 && !even_round(p, true)) || few_queries(p) ? launch<bf16, 4, 8, 1, 32, 2, true, true>(p, stream) : launch<bf16, 4, 8, 2, 64, 2, true, true>(p, stream);
+        if (nq == 4 && nv == 4) return launch<bf16, 4, 4, 1, 64, 2, true, true>(p, stream);
         if (nq == 2 && nv == 4) return even_round(p, false) ? launch<bf16, 2, 4, 2, 64, 2, true, true>(p, stream) : launch<bf16, 2, 4, 1, 32, 2, true, true>(p, stream);
     }
     if (nq <= 4 && nv <= 4) return launch<bf16, 4, 4, 1, 64, 1, false, true>(p, stream);

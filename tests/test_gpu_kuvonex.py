@@ -393,6 +393,17 @@ def test_latent_attention_of_many_heads_whole_and_in_portions(dense, T, cut):
     assert bool(whole.isfinite().all()) and bool(((whole - parts).norm(dim=1) <= 2.0 ** -7 * whole.norm(dim=1)).all())
 
 
+@pytest.mark.parametrize("sizes,T", [((3, 96, 32, 64, 128), 150), ((2, 64, 64, 64, 64), 65), ((5, 96, 32, 64, 256), 700)])
+def test_latent_attention_of_keys_of_128_and_values_of_64(dense, sizes, T):
+    """The kernel of their own, whole and in portions, against the plain result (bounds as below)."""
+    say("latent attention, 128 / 64", sizes, T)
+    far = [p for p in [(40, 0), (64, 31), (63, 32), (127, 64), (128, 63), (129, 65), (255, 128), (256, 193), (699, 1), (640, 639)] if p[0] < T]
+    x = Latents(dense, sizes, T, BF16, seed=T, far=far)
+    want = x.want()
+    for cut in (T, 70):
+        each_head_close(torch.cat([x.run("rows", a, min(a + cut, T)) for a in range(0, T, cut)]), want, sizes[0], 2.0 ** -5, cut)
+
+
 @pytest.mark.parametrize("heads,T", [(128, 330), (64, 1000)])
 def test_latent_attention_by_items_of_128_and_of_64_queries(dense, heads, T):
     """Both kernels of heads of 128 + 64 / 128 against the plain result, far keys around the edges of blocks of 64 keys and of items.  2^-5 a head: queries, keys and

@@ -215,6 +215,11 @@ def test_windowed_attention(dense, dtype, sizes, form):
         close(parts[i], want[i], dtype, i, **tol)
 
 
+@pytest.mark.parametrize("sizes", [(4, 2, 128, 64, 33), (3, 3, 128, 64, 64), (8, 2, 128, 64, 190)])
+def test_windowed_attention_of_keys_of_128_and_values_of_64(dense, sizes):
+    test_windowed_attention(dense, BF16, sizes, "rows")
+
+
 @pytest.mark.parametrize("sizes", [(64, 8, 128, 128, 1000), (64, 8, 128, 128, 768), (64, 16, 64, 64, 1000)])
 @pytest.mark.parametrize("T,cut", [(1100, 256), (1025, 65)])
 def test_windowed_attention_of_many_heads_whole_and_in_portions(dense, sizes, T, cut):
