@@ -5,17 +5,17 @@
 // Input is the [M, (n_heads + 2 n_kv) * HD] tensor of w4a16_prefill_rms_qkv_rope_bf16 (roped Q | roped K | V per
 // row); output attn_out bf16 [M, n_heads * HD].
 //
-// A workgroup is two sets of four waves on one KV head.  A wave owns 32 queries of one query head; the four waves of a
+// A workgroup is two sets of four waves on one KV head.  A wave owns 32 queries of one query head (16 where there are few items, kFewItems); the four waves of a
 // set are HPW heads of the KV head's group times 4 / HPW query blocks (HPW = 4 for the 32 / 8 head models: the four
 // heads of a group meet the same keys at the same time, so no wave idles at the diagonal) and share the K and V rows
-// that go through LDS: an "item" of 32 * 4 / HPW queries.  Causal items differ in length by the number of items, so
+// that go through LDS: an "item" of 32 (16) * 4 / HPW queries.  Causal items differ in length by the number of items, so
 // the workgroup takes a pair, the j-th longest with the j-th shortest (nA + nB key blocks, the same for every pair):
 // set 0 runs the first half of that many blocks of the long item, set 1 the short item and then the long item's
 // remaining blocks, and the two partial results of the long item are merged through LDS at the end.  Every wave of
 // the chip then has the same number of blocks to do, whichever CU its workgroup lands on.  Keys go by in
 // blocks of 64 through LDS, double buffered, one barrier per block; the rows travel global -> registers during the
 // block before and registers -> LDS at the head of the block.  The online softmax keeps one running maximum and sum
-// per query.  Everything is computed transposed so that a lane owns one query (of each of its two 16-query blocks)
+// per query.  Everything is computed transposed so that a lane owns one query (of each of its one or two 16-query blocks)
 // throughout (MFMA 16x16x32 bf16):
 //   S^T[key, q] = K . Q^T      A = K rows from LDS (16-byte reads), B = Q^T held in registers
 //   O^T[d, q]  += V^T . P^T    A = V^T, B = P^T built from the lane's own S^T registers
@@ -50,6 +50,10 @@ struct PrefillAttnParams {
 
 constexpr float kMasked = -1.0e30f;
 constexpr float kLazy = 8.0f;   // the reference maximum of the softmax may lag the true one by this much (log2 domain)
+// Queries of a wave: 16 where their items, two to a workgroup, are no more than a round of workgroups, else 32.  A step is a chain, of 3.4 us with 32 queries and heads of 128 and 2.3 with 16, and
+// most of the CUs had nothing to do.  us, 32 / 16 queries: 32 heads of 128 over 8, 64 tokens 12.6 / 8.0, 300 17.0 / 11.7, 1000 (256 workgroups) 33.4 / 25.3, 1500 (376) 43.8 / 56.9; of 64,
+// 1000 tokens 21.3 / 16.1, 1500 27.7 / 28.5; 8 heads of 128 over 8, 300 tokens 20.8 / 14.8, 2048 59.8 / 42.0.
+constexpr int kFewItems = 256;
 constexpr int kAttnKeys = 64;   // keys per block (heads of 128: 54 us at 64 keys, 60 us at 32, M = 2048, 32 / 8 heads)
 
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -65,13 +69,13 @@ constexpr size_t attn_lds_bytes() {
 // (This file is compiled with -fno-honor-nans: otherwise every MFMA result is canonicalised before it enters a
 // maximum, one more instruction per score.  A NaN in the inputs gives unspecified output values.)
 
-template <int HD, int HPW>
+template <int HD, int HPW, int QB>
 __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnParams p) {
     constexpr int KB = kAttnKeys, NKK = KB / 16, NT = KB / 32;   // 16-key blocks of S^T, K-steps of the second product
     constexpr int KP = HD + 8;     // K tile row pitch (elements): 144 / 272 B, conflict-free 16-byte reads over 16 rows
     constexpr int VP = HD + 16;    // V tile row pitch: 160 / 288 B = 32 B mod 256, conflict-free transposing reads
-    constexpr int QS = 4 / HPW;    // 32-query blocks per wave set
-    constexpr int QW = 32 * QS;    // queries of an item
+    constexpr int QS = 4 / HPW;    // blocks of 16 QB queries per wave set
+    constexpr int QW = 16 * QB * QS;   // queries of an item
     constexpr int kTile = KB * (KP + VP);   // elements of one K + V tile
     extern __shared__ __attribute__((aligned(16))) uint16_t attn_lds[];
 
@@ -104,15 +108,15 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
         return it < nA ? it : -1;
     };
 
-    int q0, qi[2];
-    bf16x8 qf[2][HD / 32];
-    floatx4 o[2][HD / 16];
-    float m[2];         // reference maximum of the raw scores (may lag the true maximum by kLazy in the log2 domain)
-    floatx4 l[2];       // sum of the bf16 probabilities: the product of a row of ones with P^T, every register the same
+    int q0, qi[QB];
+    bf16x8 qf[QB][HD / 32];
+    floatx4 o[QB][HD / 16];
+    float m[QB];        // reference maximum of the raw scores (may lag the true maximum by kLazy in the log2 domain)
+    floatx4 l[QB];      // sum of the bf16 probabilities: the product of a row of ones with P^T, every register the same
     auto begin_item = [&](int x) {
-        q0 = x * QW + 32 * (w4 / HPW);
+        q0 = x * QW + 16 * QB * (w4 / HPW);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
             qi[b] = q0 + 16 * b + ql;                                      // this lane's queries (may be >= M in the last item)
             const int qrow = qi[b] < p.M ? qi[b] : p.M - 1;                // load in range, never stored
 #pragma unroll
@@ -129,7 +133,7 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
     };
     auto store_item = [&]() {
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
             if (qi[b] >= p.M) continue;
             const float inv = 1.0f / l[b][0];
             uint16_t *dst = p.out + (size_t)qi[b] * p.n_heads * HD + head * HD + 4 * g;
@@ -177,23 +181,43 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
     auto block = [&](int it, int buf, bool masked) {
         const uint16_t *tile = kt + buf * kTile;
         const int kb = it * KB;
-        floatx4 s[NKK][2];
+        floatx4 s[NKK][QB];
+        constexpr int NS = NKK * (HD / 32), NO = NT * (HD / 16), kAhead = 4;
+        // operands on their way from LDS at a time (16 queries: 42.2 -> 40.3 us, 16 heads of 128 over 4, 2048 tokens; with 32, which use an operand twice, nothing)
+        constexpr bool kRing = QB == 1;
+        if constexpr (kRing) {
 #pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) {
-            s[kk][0] = s[kk][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int kk = 0; kk < NKK; ++kk) s[kk][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+            bf16x8 a[kAhead];
+            auto ask = [&](int n) { a[n % kAhead] = *reinterpret_cast<const bf16x8 *>(&tile[k_lane + 16 * (n / (HD / 32)) * KP + 32 * (n % (HD / 32))]); };
 #pragma unroll
-            for (int ks = 0; ks < HD / 32; ++ks) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&tile[k_lane + 16 * kk * KP + 32 * ks]);
-                s[kk][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[0][ks], s[kk][0], 0, 0, 0);
-                s[kk][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[1][ks], s[kk][1], 0, 0, 0);
+            for (int n = 0; n < kAhead; ++n) ask(n);
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+                __builtin_amdgcn_sched_barrier(0);
+                s[n / (HD / 32)][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n % kAhead], qf[0][n % (HD / 32)], s[n / (HD / 32)][0], 0, 0, 0);
+                if (n + kAhead < NS) ask(n + kAhead);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) {
+#pragma unroll
+                for (int b = 0; b < QB; ++b) s[kk][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < HD / 32; ++ks) {
+                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&tile[k_lane + 16 * kk * KP + 32 * ks]);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b) s[kk][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[b][ks], s[kk][b], 0, 0, 0);
+                }
             }
         }
         // s[kk][b][r] is the raw score of key kb + 16 kk + 4 g + r against query qi[b]
-        bf16x8 pb[2][NT];   // [query block][K-step of 32 keys]
-        float bm[2];
+        bf16x8 pb[QB][NT];   // [query block][K-step of 32 keys]
+        float bm[QB];
         bool lag = false;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
             if (masked) {   // (wave-uniform; one copy of the products for both cases keeps the output registers in place)
 #pragma unroll
                 for (int kk = 0; kk < NKK; ++kk)
@@ -213,11 +237,11 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
         }
         // The reference maximum follows the true one only when that has moved by more than 2^kLazy (probabilities up to
         // 2^kLazy instead of 1: harmless in fp32 and bf16, and the final division takes the factor out again), so the
-        // rescaling of the 2 (HD / 16 + 1) accumulators is rare after the first blocks.  (The first block always
+        // rescaling of the QB (HD / 16 + 1) accumulators is rare after the first blocks.  (The first block always
         // rescales: finite against -1e30; key 0 is visible to every query.)
         if (__builtin_amdgcn_ballot_w64(lag) != 0) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
+            for (int b = 0; b < QB; ++b) {
                 const float m_new = fmaxf(m[b], bm[b]);
                 const float alpha = __builtin_amdgcn_exp2f((m[b] - m_new) * p.scale_log2);
                 m[b] = m_new;
@@ -227,7 +251,7 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
             }
         }
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
             const float msc = m[b] * p.scale_log2;
             // v_exp_f32 directly: results that would be denormal may flush to zero, and a masked score (-1e30 against a
             // finite maximum) gives exactly 0
@@ -246,19 +270,29 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
                 l[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[b][t], l[b], 0, 0, 0);
             }
         }
+        auto column = [&](int n) {
+            const uint16_t *src = &tile[v_lane + 32 * (n / (HD / 16)) * VP + 16 * (n % (HD / 16))];
+            const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)src);
+            const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)(src + 16 * VP));
+            const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
+            return __builtin_bit_cast(bf16x8, (u32x4{lo2.x, lo2.y, hi2.x, hi2.y}));
+        };
+        bf16x8 a[kRing ? kAhead : 1];
+        if constexpr (kRing) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+            for (int n = 0; n < kAhead; ++n) a[n] = column(n);
+        }
 #pragma unroll
-            for (int d = 0; d < HD / 16; ++d) {
-                const uint16_t *src = &tile[v_lane + 32 * t * VP + 16 * d];
-                const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)src);
-                const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4 *)(src + 16 * VP));
-                const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
-                const u32x4 aw = {lo2.x, lo2.y, hi2.x, hi2.y};
-                const bf16x8 a = __builtin_bit_cast(bf16x8, aw);
-                o[0][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[0][t], o[0][d], 0, 0, 0);
-                o[1][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[1][t], o[1][d], 0, 0, 0);
-            }
+        for (int n = 0; n < NO; ++n) {
+            const int d = n % (HD / 16);
+            if constexpr (kRing) __builtin_amdgcn_sched_barrier(0);
+            else a[0] = column(n);
+#pragma unroll
+            for (int b = 0; b < QB; ++b) o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kRing ? n % kAhead : 0], pb[b][n / (HD / 16)], o[b][d], 0, 0, 0);
+            if constexpr (kRing)
+                if (n + kAhead < NO) a[n % kAhead] = column(n + kAhead);
+        }
+        if constexpr (kRing) __builtin_amdgcn_sched_barrier(0);
     };
 
     // Every wave of the workgroup runs hA steps with one barrier each (set 1 may have one step less to do).  Step s
@@ -275,7 +309,7 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
             }
             const int it = block_of_step(s);
             const int kb = it * KB;
-            if (it >= 0 && kb <= q0 + 31) block(it, buf, kb + KB - 1 > q0);   // else every key is after this wave's queries
+            if (it >= 0 && kb <= q0 + 16 * QB - 1) block(it, buf, kb + KB - 1 > q0);   // else every key is after this wave's queries
             __syncthreads();
         }
     };
@@ -297,17 +331,17 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
 
     // Set 1's partial result for the heavy item (neutral if it had no block of it) goes through LDS, lane to lane: the
     // same wave and lane of set 0 owns the same queries and output elements.
-    constexpr int NREG = 2 * (HD / 16) * 4 + 4;
+    constexpr int NREG = QB * (HD / 16) * 4 + 2 * QB;
     float *xch = reinterpret_cast<float *>(attn_lds) + w4 * NREG * 64 + lane;
     if (set == 1) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
 #pragma unroll
             for (int d = 0; d < HD / 16; ++d)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) xch[((b * (HD / 16) + d) * 4 + r) * 64] = o[b][d][r];
-            xch[(NREG - 4 + b) * 64] = m[b];
-            xch[(NREG - 2 + b) * 64] = l[b][0];
+            xch[(NREG - 2 * QB + b) * 64] = m[b];
+            xch[(NREG - QB + b) * 64] = l[b][0];
         }
     }
     __syncthreads();
@@ -339,8 +373,8 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
         return;
     }
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const float m1 = xch[(NREG - 4 + b) * 64], l1 = xch[(NREG - 2 + b) * 64];
+    for (int b = 0; b < QB; ++b) {
+        const float m1 = xch[(NREG - 2 * QB + b) * 64], l1 = xch[(NREG - QB + b) * 64];
         const float mm = fmaxf(m[b], m1);
         const float f0 = __builtin_amdgcn_exp2f((m[b] - mm) * p.scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mm) * p.scale_log2);
         l[b][0] = l[b][0] * f0 + l1 * f1;
@@ -352,17 +386,24 @@ __global__ void __launch_bounds__(512) prefill_attn_kernel(const PrefillAttnPara
     store_item();
 }
 
-template <int HD, int HPW>
-hipError_t launch_attn(const PrefillAttnParams &p, hipStream_t stream) {
+template <int HD, int HPW, int QB>
+hipError_t launch_items(const PrefillAttnParams &p, hipStream_t stream) {
     constexpr size_t lds = attn_lds_bytes<HD>();
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&prefill_attn_kernel<HD, HPW>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&prefill_attn_kernel<HD, HPW, QB>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    constexpr int QW = 32 * (4 / HPW);
+    constexpr int QW = 16 * QB * (4 / HPW);
     const int nx = (p.M + QW - 1) / QW;
     const dim3 grid((nx + 1) / 2, p.n_kv * (p.n_heads / p.n_kv / HPW));
-    hipLaunchKernelGGL((prefill_attn_kernel<HD, HPW>), grid, dim3(512), lds, stream, p);
+    hipLaunchKernelGGL((prefill_attn_kernel<HD, HPW, QB>), grid, dim3(512), lds, stream, p);
     return hipGetLastError();
+}
+
+template <int HD, int HPW>
+hipError_t launch_attn(const PrefillAttnParams &p, hipStream_t stream) {
+    constexpr int QW = 16 * (4 / HPW);
+    const long items = (long)((p.M + QW - 1) / QW + 1) / 2 * (p.n_heads / HPW);
+    return items <= kFewItems ? launch_items<HD, HPW, 1>(p, stream) : launch_items<HD, HPW, 2>(p, stream);
 }
 
 }  // namespace

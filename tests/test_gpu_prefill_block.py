@@ -288,6 +288,13 @@ def test_prefill_attention_fills_the_caches(ops, M, nh, nkv, hd):
             ops.prefill_attention(qkv, nh, nkv, hd, new(M - 1), new(M - 1))
 
 
+# 16 queries to a wave up to 256 workgroups, 32 past them: both sides of the line, ragged items, every number of heads to a workgroup
+@pytest.mark.parametrize("M,nh,nkv,hd", [(1024, 32, 8, 64), (1025, 32, 8, 64), (1009, 32, 8, 128), (15, 4, 4, 128), (17, 8, 4, 64), (129, 8, 8, 64), (65, 6, 3, 128), (511, 16, 4, 128)])
+def test_prefill_attention_by_16_and_by_32_queries(ops, M, nh, nkv, hd):
+    test_prefill_attention(ops, M, nh, nkv, hd)
+    test_prefill_attention_fills_the_caches(ops, M, nh, nkv, hd)
+
+
 def test_prefill_attention_scores_of_wide_range(ops):
     """Scores spread over hundreds of log2 units: the kernel's reference maximum, which follows the true one in steps,
     must not lose the small terms or overflow; and a second call returns the same bits."""
