@@ -50,7 +50,7 @@ struct PrefillAttnParams {
 
 constexpr float kMasked = -1.0e30f;
 constexpr float kLazy = 8.0f;   // the reference maximum of the softmax may lag the true one by this much (log2 domain)
-// Queries of a wave: 16 where their items, two to a workgroup, are no more than a round of workgroups, else 32.  A step is a chain, of 3.4 us with 32 queries and heads of 128 and 2.3 with 16, and
+// Queries of a wave: 16 where their items, two to a workgroup, are no more than a round of workgroups, else 32.  A step is a chain, of 2.6 us with 32 queries and heads of 128 and 1.9 with 16, and
 // most of the CUs had nothing to do.  us, 32 / 16 queries: 32 heads of 128 over 8, 64 tokens 12.6 / 8.0, 300 17.0 / 11.7, 1000 (256 workgroups) 33.4 / 25.3, 1500 (376) 43.8 / 56.9; of 64,
 // 1000 tokens 21.3 / 16.1, 1500 27.7 / 28.5; 8 heads of 128 over 8, 300 tokens 20.8 / 14.8, 2048 59.8 / 42.0.
 constexpr int kFewItems = 256;
