@@ -418,6 +418,8 @@ int w4a16_decode_attention_bf16(const uint16_t *qkv, const uint16_t *rope_lut_ro
  * prefill ELFs): out[m, :] = bf16((x[m, :] / sqrt(mean(x[m, :]^2) + eps)) * norm_weight), K % 8 == 0, K <= 8192.
  */
 size_t w4a16_prefill_block_workspace_bytes(int M, int E, int H);
+/* What the same on stream-order weights can use: few rows run in slices of K as far as their parts fit behind the bytes above. */
+size_t w4a16_prefill_block_workspace_most(int M, int E, int H);
 int rms_norm_rows_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps, uint16_t *out, int M, int K,
                        void *stream);
 int w4a16_prefill_o_ffn_bf16(const uint16_t *attn_out, const uint16_t *x_residual,
@@ -459,6 +461,7 @@ int w4a16_prefill_o_ffn_stream_bf16(const uint16_t *attn_out, const uint16_t *x_
  * E % 128 == 0, E <= 8192.  The workspace is plain scratch, w4a16_prefill_qkv_workspace_bytes(M, E) = 2 M E bytes.
  */
 size_t w4a16_prefill_qkv_workspace_bytes(int M, int E);
+size_t w4a16_prefill_qkv_workspace_most(int M, int E);   /* (stream order: with the parts of few rows, as above) */
 int w4a16_prefill_rms_qkv_rope_bf16(const uint16_t *x, const uint16_t *attn_norm_weight, float eps,
                                     const int32_t *qkv_qweight, const int32_t *qkv_qzeros, const uint16_t *qkv_scales,
                                     const uint16_t *rope_lut, int rope_lut_rows, int pos0, uint16_t *qkv_out,

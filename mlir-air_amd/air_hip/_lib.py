@@ -40,9 +40,11 @@ SYMBOLS = {
     "w4a16_attention_workspace_bytes": (_sz, [_ci, _ci]),
     "w4a16_decode_attention_bf16": (_ci, [_vp] * 5 + [_ci] * 5 + [_vp, _sz, _vp]),
     "w4a16_prefill_block_workspace_bytes": (_sz, [_ci, _ci, _ci]),
+    "w4a16_prefill_block_workspace_most": (_sz, [_ci, _ci, _ci]),
     "rms_norm_rows_bf16": (_ci, [_vp, _vp, _cf, _vp, _ci, _ci, _vp]),
     "w4a16_prefill_o_ffn_bf16": (_ci, [_vp, _vp, _vp, _cf] + [_vp] * 15 + [_ci, _ci, _ci, _ci, _vp, _sz, _vp]),
     "w4a16_prefill_qkv_workspace_bytes": (_sz, [_ci, _ci]),
+    "w4a16_prefill_qkv_workspace_most": (_sz, [_ci, _ci]),
     "w4a16_prefill_rms_qkv_rope_bf16": (_ci, [_vp, _vp, _cf, _vp, _vp, _vp, _vp, _ci, _ci, _vp] + [_ci] * 6 + [_vp, _sz, _vp]),
     "w4a16_prefill_rms_qkv_rope_stream_bf16": (_ci, [_vp, _vp, _cf, _vp, _vp, _ci, _ci, _vp] + [_ci] * 6 + [_vp, _sz, _vp]),
     "w4a16_prefill_o_ffn_stream_bf16": (_ci, [_vp, _vp, _vp, _cf] + [_vp] * 7 + [_ci, _ci, _ci, _ci, _vp, _sz, _vp]),

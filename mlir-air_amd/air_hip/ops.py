@@ -693,7 +693,7 @@ def prefill_rms_qkv_rope_stream(x, attn_norm_weight, wqkv, rope_lut, pos0, n_hea
     key = (x.device.index, _stream(), "prefill_qkv", M, E)
     ws = _attn_ws.get(key)
     if ws is None:
-        ws = torch.empty(int(lib.w4a16_prefill_qkv_workspace_bytes(M, E)), dtype=torch.uint8, device=x.device)
+        ws = torch.empty(int(lib.w4a16_prefill_qkv_workspace_most(M, E)), dtype=torch.uint8, device=x.device)
         _attn_ws[key] = ws
     if codec == "q4nx":
         _lib.check(lib.w4a16_q4nx_prefill_rms_qkv_rope_stream_bf16(_ptr(_bits(x)), _ptr(_bits(attn_norm_weight)), float(eps),
@@ -724,7 +724,7 @@ def prefill_o_ffn_stream(attn_out, x_residual, ffn_norm_weight, wo, gate, up, do
     key = (attn_out.device.index, _stream(), "prefill_block", M, E, H)
     ws = _attn_ws.get(key)
     if ws is None:
-        ws = torch.empty(int(lib.w4a16_prefill_block_workspace_bytes(M, E, H)), dtype=torch.uint8, device=attn_out.device)
+        ws = torch.empty(int(lib.w4a16_prefill_block_workspace_most(M, E, H)), dtype=torch.uint8, device=attn_out.device)
         _attn_ws[key] = ws
     args = (_ptr(_bits(attn_out)), _ptr(_bits(x_residual)), _ptr(_bits(ffn_norm_weight)), float(eps), _ptr(wo.buf), _ptr(gate.buf),
             _ptr(up.buf), _ptr(down.buf), _ptr(y), _ptr(res1) if res1 is not None else None, _ptr(h) if h is not None else None,

@@ -732,6 +732,8 @@ size_t w4a16_prefill_block_workspace_bytes(int M, int E, int H) {
     return prefill_block_supported(M, E, H) ? prefill_block_scratch_bytes(M, E, H) : 0;
 }
 
+size_t w4a16_prefill_block_workspace_most(int M, int E, int H) { return prefill_block_supported(M, E, H) ? prefill_block_scratch_most(M, E, H) : 0; }
+
 int rms_norm_rows_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps, uint16_t *out, int M, int K,
                        void *stream) {
     if (!x || !norm_weight || !out) return W4A16_ERR_NULL;
@@ -744,6 +746,8 @@ int rms_norm_rows_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps
 size_t w4a16_prefill_qkv_workspace_bytes(int M, int E) {
     return prefill_block_supported(M, E, 8) ? prefill_qkv_scratch_bytes(M, E) : 0;
 }
+
+size_t w4a16_prefill_qkv_workspace_most(int M, int E) { return prefill_block_supported(M, E, 8) ? prefill_qkv_scratch_most(M, E) : 0; }
 
 int w4a16_prefill_rms_qkv_rope_bf16(const uint16_t *x, const uint16_t *attn_norm_weight, float eps,
                                     const int32_t *qkv_qweight, const int32_t *qkv_qzeros, const uint16_t *qkv_scales,
@@ -833,7 +837,7 @@ int prefill_qkv_stream_call(const uint16_t *x, const uint16_t *attn_norm_weight,
     if (!workspace || workspace_bytes < w4a16_prefill_qkv_workspace_bytes(M, E)) return W4A16_ERR_WORKSPACE;
     if (misaligned(workspace)) return W4A16_ERR_ALIGN;
     hipError_t e = launch_prefill_rms_qkv_rope_stream(x, attn_norm_weight, eps, qkv_wstream, rope_lut, pos0, qkv_out, M, E, n_heads,
-                                                      n_kv_heads, head_dim, workspace, static_cast<hipStream_t>(stream), q4);
+                                                      n_kv_heads, head_dim, workspace, workspace_bytes, static_cast<hipStream_t>(stream), q4);
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
 
@@ -851,7 +855,7 @@ int prefill_o_ffn_stream_call(const uint16_t *attn_out, const uint16_t *x_residu
     if (!workspace || workspace_bytes < w4a16_prefill_block_workspace_bytes(M, E, H)) return W4A16_ERR_WORKSPACE;
     if (misaligned(workspace)) return W4A16_ERR_ALIGN;
     hipError_t e = launch_prefill_o_ffn_stream(attn_out, x_residual, ffn_norm_weight, eps, o_wstream, gate_wstream, up_wstream,
-                                               down_wstream, y, res1_out, h_out, M, E, H, workspace, static_cast<hipStream_t>(stream), q4);
+                                               down_wstream, y, res1_out, h_out, M, E, H, workspace, workspace_bytes, static_cast<hipStream_t>(stream), q4);
     return e == hipSuccess ? W4A16_OK : hip_fail(e);
 }
 }  // namespace

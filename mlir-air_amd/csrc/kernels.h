@@ -179,6 +179,9 @@ struct PrefillLinear {
 bool prefill_block_supported(int M, int E, int H);
 size_t prefill_block_scratch_bytes(int M, int E, int H);   // sized for split-K on a 256-CU device
 size_t prefill_qkv_scratch_bytes(int M, int E);
+// with room for the parts of the stream-order products of few rows, which run in as many slices as fit
+size_t prefill_block_scratch_most(int M, int E, int H);
+size_t prefill_qkv_scratch_most(int M, int E);
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream);
 // Causal GQA attention over the M rows of a prefill (prefill_attention.hip); qkv is [M, (n_heads + 2 n_kv) * head_dim].
 // With caches [n_kv, max_seq, head_dim] their rows 0 .. M - 1 become the K and V of qkv.
@@ -193,14 +196,14 @@ hipError_t launch_prefill_o_ffn(const uint16_t *attn_out, const uint16_t *x_resi
                                 const PrefillLinear &wd, uint16_t *y, uint16_t *res1_out, uint16_t *h_out, int M, int E,
                                 int H, void *workspace, int cus, hipStream_t stream);
 // The same blocks on stream-order weights (every matrix re-packed with launch_repack_ws; `q4`: with launch_repack_ws_q4); workspaces of prefill_qkv_scratch_bytes
-// and prefill_block_scratch_bytes.
+// and prefill_block_scratch_bytes or more.
 bool prefill_block_stream_supported(int M, int E, int H);
 hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t *norm_w, float eps, const void *wqkv,
                                               const uint16_t *rope_lut, int pos0, uint16_t *qkv_out, int M, int E, int n_heads,
-                                              int n_kv, int head_dim, void *workspace, hipStream_t stream, bool q4 = false);
+                                              int n_kv, int head_dim, void *workspace, size_t workspace_bytes, hipStream_t stream, bool q4 = false);
 hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t *x_residual, const uint16_t *ffn_norm_w, float eps,
                                        const void *wo, const void *wg, const void *wu, const void *wd, uint16_t *y,
-                                       uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace,
+                                       uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace, size_t workspace_bytes,
                                        hipStream_t stream, bool q4 = false);
 
 // Q4NX / Q4_0 block codec (q4nx.hip).  mode: 0 w = s q + m, 1 w = s (q - m), 2 signed q, w = s q.

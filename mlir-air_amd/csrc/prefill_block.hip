@@ -89,15 +89,18 @@ static size_t splitk_bytes(int M, int E, int H, int cus) {
 static size_t tail_bytes(int M, int E, int H) { return std::max(splitk_bytes(M, E, H, kPlanCus), gemm_wsm_parts_bytes(M, std::max(E, 2 * H))); }
 static size_t block_rows_bytes(int M, int E, int H) { return 2 * round256((size_t)M * E * sizeof(uint16_t)) + 2 * round256((size_t)M * H * sizeof(uint16_t)); }
 
+size_t prefill_block_scratch_bytes(int M, int E, int H) { return block_rows_bytes(M, E, H) + round256(splitk_bytes(M, E, H, kPlanCus)); }
+size_t prefill_qkv_scratch_bytes(int M, int E) { return round256((size_t)M * E * sizeof(uint16_t)); }
+
 // (a workspace for many rows also serves fewer of them, whose products run in slices)
-size_t prefill_block_scratch_bytes(int M, int E, int H) {
+size_t prefill_block_scratch_most(int M, int E, int H) {
     const int few = std::min(M, kWsmSliceRows);
     return std::max(block_rows_bytes(M, E, H) + round256(tail_bytes(M, E, H)), block_rows_bytes(few, E, H) + round256(gemm_wsm_parts_bytes(few, std::max(E, 2 * H))));
 }
 
 // Behind the normed rows: parts of the projections of few rows (how wide those are the call says; three times E where every head has keys of its own)
 static size_t qkv_parts_bytes(int M, int E) { return round256(gemm_wsm_parts_bytes(M, 3 * E)); }
-size_t prefill_qkv_scratch_bytes(int M, int E) {
+size_t prefill_qkv_scratch_most(int M, int E) {
     const int few = std::min(M, kWsmSliceRows);
     return std::max(round256((size_t)M * E * sizeof(uint16_t)) + qkv_parts_bytes(M, E), round256((size_t)few * E * sizeof(uint16_t)) + qkv_parts_bytes(few, E));
 }
@@ -168,7 +171,7 @@ static bool by_wsm(const WsmPlan &plan, double elements, double tiled_us) {
 
 hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t *norm_w, float eps, const void *wqkv,
                                               const uint16_t *rope_lut, int pos0, uint16_t *qkv_out, int M, int E, int n_heads,
-                                              int n_kv, int head_dim, void *workspace, hipStream_t stream, bool q4) {
+                                              int n_kv, int head_dim, void *workspace, size_t workspace_bytes, hipStream_t stream, bool q4) {
     uint16_t *normed = static_cast<uint16_t *>(workspace);
     const size_t own_e = round256((size_t)M * E * sizeof(uint16_t));
     hipError_t e = launch_rmsnorm_rows(x, norm_w, normed, M, E, eps, stream);
@@ -176,7 +179,7 @@ hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t 
     const GemmRope rope = {(n_heads + n_kv) * head_dim, head_dim, pos0};
     const int N = (n_heads + 2 * n_kv) * head_dim;
     if (gemm_wsm_supported(17, E, N)) {
-        const WsmPlan plan = plan_wsm_rounded(M, E, N, 1, q4, qkv_parts_bytes(M, E));
+        const WsmPlan plan = plan_wsm_rounded(M, E, N, 1, q4, std::min(qkv_parts_bytes(M, E), workspace_bytes - std::min(workspace_bytes, own_e)));
         if (by_wsm(plan, (double)M * rope.cols, gemm_prefill_ws_us(M, E, N, q4, 0)))
             return launch_gemm_wsm_rope(plan, normed, wqkv, qkv_out, rope_lut, rope, reinterpret_cast<float *>(static_cast<char *>(workspace) + own_e), M, E, N, q4, stream);
     }
@@ -196,7 +199,7 @@ static hipError_t product_add(const uint16_t *x, const void *w, uint16_t *y, int
 
 hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t *x_residual, const uint16_t *ffn_norm_w, float eps,
                                        const void *wo, const void *wg, const void *wu, const void *wd, uint16_t *y,
-                                       uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace,
+                                       uint16_t *res1_out, uint16_t *h_out, int M, int E, int H, void *workspace, size_t workspace_bytes,
                                        hipStream_t stream, bool q4) {
     char *base = static_cast<char *>(workspace);
     uint16_t *res1 = reinterpret_cast<uint16_t *>(base);
@@ -208,7 +211,7 @@ hipError_t launch_prefill_o_ffn_stream(const uint16_t *attn_out, const uint16_t 
     uint16_t *h = reinterpret_cast<uint16_t *>(base);
     base += round256((size_t)M * H * sizeof(uint16_t));
     float *tail = reinterpret_cast<float *>(base);
-    const size_t most = tail_bytes(M, E, H);
+    const size_t most = std::min(tail_bytes(M, E, H), workspace_bytes - std::min(workspace_bytes, block_rows_bytes(M, E, H)));
     // scratch of the two products with a residual: what is not in use yet (gate, h) or any more (normed, gate)
     const size_t own_h = round256((size_t)M * H * sizeof(uint16_t)), own_e = round256((size_t)M * E * sizeof(uint16_t));
     if (res1_out) res1 = res1_out;

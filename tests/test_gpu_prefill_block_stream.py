@@ -279,6 +279,42 @@ def test_prefill_rms_qkv_rope_stream(ops, tiled_gemm, M, E, nh, nkv, hd, pos0, t
     assert np.mean(got != ref_r) < 0.1, np.mean(got != ref_r)
 
 
+@pytest.mark.parametrize("M", [1, 17, 40, 100, 300])
+def test_prefill_blocks_stream_in_the_least_workspace(ops, M):
+    """2 M E bytes for the projections, the block's rows and split parts for the rest: what callers had to bring before few rows ran in slices, and nothing behind it is written.
+    Slices only change the order of the fp32 sums: a bf16 step here and there, which the FFN carries on (2^-7 of a row's norm)."""
+    from air_hip import _lib
+    from oracle import decode as odec
+    lib = _lib.load_library()
+    E, H, nh, nkv, hd = 1024, 2048, 8, 4, 128
+    _, fused = _qkv_weights(E, nh, nkv, hd, seed=M)
+    ws = [_sw(ops, w) for w in _weights(E, H, seed=M)]
+    sw, lut = _sw(ops, fused), dev(odec.generate_rope_lut(hd, 500000.0, M))
+    x, attn, nw = dev(make_x((M, E), seed=M)), dev(make_x((M, E), seed=M + 1)), dev(_norm_w(E, 3))
+    guard = 4096
+    def least(n):
+        buf = torch.full((n + guard,), 77, dtype=torch.uint8, device="cuda")
+        return buf, buf[:n]
+    print("prompt blocks, least workspace", M, flush=True)
+    stream = torch.cuda.current_stream().cuda_stream
+    b1, w1 = least(lib.w4a16_prefill_qkv_workspace_bytes(M, E))
+    assert w1.numel() == -(-2 * M * E // 256) * 256
+    q1 = torch.empty((M, (nh + 2 * nkv) * hd), dtype=torch.bfloat16, device="cuda")
+    _lib.check(lib.w4a16_prefill_rms_qkv_rope_stream_bf16(x.data_ptr(), nw.data_ptr(), 1e-5, sw.buf.data_ptr(), lut.data_ptr(), M, 0, q1.data_ptr(), M, E, nh, nkv, hd, 128,
+                                                          w1.data_ptr(), w1.numel(), stream))
+    b2, w2 = least(lib.w4a16_prefill_block_workspace_bytes(M, E, H))
+    y1 = torch.empty((M, E), dtype=torch.bfloat16, device="cuda")
+    _lib.check(lib.w4a16_prefill_o_ffn_stream_bf16(attn.data_ptr(), x.data_ptr(), nw.data_ptr(), 1e-5, *(w.buf.data_ptr() for w in ws), y1.data_ptr(), None, None, M, E, H, 128,
+                                                   w2.data_ptr(), w2.numel(), stream))
+    q2 = ops.prefill_rms_qkv_rope_stream(x, nw, sw, lut, 0, nh, nkv, hd)
+    y2 = ops.prefill_o_ffn_stream(attn, x, nw, *ws)
+    torch.cuda.synchronize()
+    assert bool((b1[w1.numel():] == 77).all()) and bool((b2[w2.numel():] == 77).all())
+    for got, want in ((q1, q2), (y1, y2)):
+        got, want = got.double(), want.double()
+        assert bool(((got - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1)).all())
+
+
 # 192-column tiles of heads of 128 (a head and half of one) and of gate and up: one of them, several, beside wide ones, ragged rows
 @pytest.mark.parametrize("M,E,nh,nkv,pos0,tile", [(100, 256, 1, 1, 4, 2), (270, 512, 4, 1, 0, 2), (2048, 256, 9, 3, 9, 0), (1000, 256, 32, 8, 2, 0)])
 def test_prefill_rms_qkv_rope_stream_in_192_columns(ops, tiled_gemm, M, E, nh, nkv, pos0, tile):
