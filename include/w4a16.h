@@ -621,7 +621,7 @@ int w4a16_decode_run_bf16(const w4a16_decode_model_t *model, const uint16_t *fir
  * "gemv_spin_limit" (reducer poll bound), "gemv_skip_publish" (fault injection for the
  * timeout test: split-K producers do not publish), "gemv_ws_ct", "gemv_ws_waves",
  * "gemm_ws_cb", "gemm_ws_rows" (stream-order GEMV / small-batch shapes; rows: most rows per batched launch, 16, 32 or 64), "prefill_tile" (one tile width only, 1: 256 columns, 2: 192, 3: 128,
- * 4: 64; 5: 256 mixed with 128 in the launches that take that mix; 0: by shape), "prefill_min_m" (smallest M given to the tiled prefill kernel), "prefill_band" (row panels per band of its tile order), "gemm_splitk" (exact products of 17 rows and more: 0 by shape, 1 always tiles of rows and columns, in two slices of K where the scratch holds them, 2 always whole-K launches), "gemm_wsm_rt", "gemm_wsm_nt", "gemm_wsm_slices" (those tiles: 2 .. 7 rows of 16, 1 .. 3 times 64 columns, 1 .. 16 slices, where a kernel has them; 0: by time), "prefill_wsm" (products of rounded weights: 0 by time, 1 always in those tiles, 2 never) and "prefill_swiglu_split" (1: the
+ * 4: 64; 5: 256 mixed with 128 in the launches that take that mix; 0: by shape), "prefill_min_m" (smallest M given to the tiled prefill kernel), "prefill_band" (row panels per band of its tile order), "gemm_splitk" (exact products of 17 rows and more: 0 by shape, 1 always tiles of rows and columns, in two slices of K where the scratch holds them, 2 always whole-K launches), "gemm_wsm_rt", "gemm_wsm_nt", "gemm_wsm_slices" (those tiles: rows of 16, 2 .. 7 (of rounded weights also 8 and 10; sizes that a width has no kernel for go to the next taller one), 1 .. 3 times 64 columns, 1 .. 16 slices; 0: by time), "gemm_wsm_two" (of two kernels of a size the one of two workgroups to a CU, 1, or of one, 2; 0: by time), "prefill_wsm" (products of rounded weights: 0 by time, 1 always in those tiles, 2 never) and "prefill_swiglu_split" (1: the
  * stream-order prompt-pass FFN runs its gate and up projections as two launches instead of one; same bits).  Process-wide.
  */
 int w4a16_tune(const char *key, int value);

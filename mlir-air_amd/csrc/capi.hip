@@ -547,7 +547,7 @@ int w4a16_gemv_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, 
 // the kernels of each kind by their estimated times (us, 64 and 300 rows of K = 14336, N = 4096: whole-K launches 55, tiled 150;
 // gemm_wsm 18 with slices and 32 without, 73; 2048 rows of K = 4096, N = 14336: tiled 172, gemm_wsm 275).
 static bool gemm_stream_rounded(int M, int K, int N, bool q4, bool residual) {
-    const int least = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : q4 ? 65 : kGemmWsMaxM + 1;
+    const int least = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : gemm_rounded_rows(q4);
     return M >= least && !(q4 && residual) && gemm_prefill_ws_supported(M, K, N);
 }
 
@@ -561,7 +561,7 @@ static WsmPlan gemm_stream_plan(int M, int K, int N, bool q4, bool residual, siz
     p = plan_gemm_wsm(M, K, N, q4, rounded, scratch_bytes);
     const bool always = rounded ? tune.prefill_wsm == 1 : tune.splitk == 1;
     // (rougher estimates have to differ by 5 %)
-    if (!always && p.us > (rounded ? 0.95 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : (q4 || residual ? 0.95 : 1.0) * gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
+    if (!always && p.us > (rounded ? 0.97 * gemm_prefill_ws_us(M, K, N, q4, scratch_bytes) : (q4 || residual ? 0.95 : 1.0) * gemm_ws_us(M, K, N, q4, residual))) p.us = -1;
     return p;
 }
 
@@ -588,17 +588,16 @@ size_t w4a16_gemm_stream_scratch_bytes(int M, int K, int N) {
 
 // Slices of K run by the GPU's time alone.  For the advice a second launch and its scratch count as what they take a host that issues calls one
 // after the other, 12.5 us with the first launch (30 rows of K = 3328, N = 1472: 12.4 us a call in slices that the GPU does in 8.5, 8.4 in one
-// launch): no scratch where the call without any is done by then, give or take the 5 % that its estimate is off.
+// launch): no scratch where the call without any is done by then, give or take what its estimate is off.
 static size_t gemm_stream_best_scratch(int M, int K, int N, bool q4, bool residual) {
     constexpr size_t kMost = (size_t)1 << 30;
-    constexpr double kTwoLaunchesUs = 12.5;
     const WsmPlan p = gemm_stream_plan(M, K, N, q4, residual, kMost);
     if (p.us < 0) return gemm_stream_rounded(M, K, N, q4, residual) ? gemm_prefill_ws_scratch_bytes(M, K, N, q4, kMost) : 0;
     if (p.slices == 1) return 0;
     if (g_gemv_ws_tune.splitk != 1) {
         const WsmPlan none = gemm_stream_plan(M, K, N, q4, residual, 0);
         const double whole = gemm_stream_rounded(M, K, N, q4, residual) ? gemm_prefill_ws_us(M, K, N, q4, 0) : gemm_ws_us(M, K, N, q4, residual);
-        if (0.95 * (none.us >= 0 ? none.us : whole) <= std::max(p.us, kTwoLaunchesUs)) return 0;
+        if (0.98 * (none.us >= 0 ? none.us : whole) <= std::max(p.us, kTwoLaunchesUs)) return 0;
     }
     return gemm_wsm_scratch_bytes(p, M, N);
 }
@@ -1188,6 +1187,9 @@ int w4a16_tune(const char *key, int value) {
     } else if (!strcmp(key, "gemm_wsm_rt")) {
         if (value == 1 || value > 10) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.wsm_rt = value;
+    } else if (!strcmp(key, "gemm_wsm_two")) {
+        if (value < 0 || value > 2) return W4A16_ERR_TUNE;
+        g_gemv_ws_tune.wsm_two = value;
     } else if (!strcmp(key, "gemm_wsm_nt")) {
         if (value > 3) return W4A16_ERR_TUNE;
         g_gemv_ws_tune.wsm_nt = value;

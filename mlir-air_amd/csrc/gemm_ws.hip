@@ -681,6 +681,7 @@ struct Widths {
     int ncb;            // columns / 64 of the "wide" tiles: 4, or 2 / 1 for the narrow uniform tilings
     int wide, narrow;   // number of column tiles of ncb * 64 columns and of the narrow width
     int ncb_narrow = 3; // columns / 64 of the narrow tiles of a mixed launch: 3, or 2 where columns come in pairs
+    double rounds = 0;  // the longest CU's tiles, in tiles of ncb (no wide ones: ncb_narrow)
 };
 
 double split_cost(long n_wide_tiles, long n_narrow_tiles, int cus, double narrow_cost) {
@@ -723,7 +724,7 @@ Widths pick_widths(int tiles_m, int U, int cus, bool heads128) {
             const double cost = split_cost((long)tiles_m * a, (long)tiles_m * b, cus, nn == 2 ? 2 * kPfSlowdown128 : 3.0);
             if (best_cost < 0 || cost < best_cost) {
                 best_cost = cost;
-                best = Widths{4, a, b, nn};
+                best = Widths{4, a, b, nn, cost / (a ? 4.0 : 3.0)};
             }
         }
     // uniform narrow tilings: rounds x width x (measured) slowdown of the narrower tile's inner loop
@@ -734,7 +735,7 @@ Widths pick_widths(int tiles_m, int U, int cus, bool heads128) {
         const double cost = (double)((tiles + cus - 1) / cus) * nv.ncb * nv.slowdown;
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
-            best = Widths{nv.ncb, U / nv.ncb, 0, 3};
+            best = Widths{nv.ncb, U / nv.ncb, 0, 3, (double)((tiles + cus - 1) / cus)};
         }
     }
     cache[next] = Entry{tiles_m, U, cus, heads128, best};
@@ -792,14 +793,14 @@ __global__ void __launch_bounds__(256) gemm_wsp_sum_kernel(const float *__restri
 
 bool gemm_prefill_ws_supported(int M, int K, int N) { return M > 0 && K > 0 && K % (2 * kGroup) == 0 && N > 0 && N % 64 == 0; }
 
-// Rounds of tiles over the chip, each a start and K steps of a cost linear in the tile's width and growing a little with the share of the CUs that are busy (fitted to 1044
-// timings in a graph, 40 .. 1500 rows of 36 matrices from 512 x 512 to 14336 x 14336 in tiles of 64, 128 and 256 columns; rms error 6 %, Q4NX 4.5 %)
-static double wsp_us(int K, long tiles, int ncb, bool q4) {
-    const long rounds = (tiles + 255) / 256;
-    const double share = (double)tiles / (256.0 * rounds);
-    return q4 ? 2.1 + rounds * (0.8 + 2.05 * ncb + 1e-3 * K * (0.88 + 0.12 * share) * (8.15 + 3.2 * ncb))
-              : 1.8 + rounds * (0.9 + 2.0 * ncb + 1e-3 * K * (0.85 + 0.15 * share) * (7.45 + 2.6 * ncb));
+// Rounds of tiles over the chip, each a start and K steps of a cost linear in the tile's width and growing a little with the share of the CUs that are busy (fitted to 800 products
+// on weights from memory, 17 .. 1600 rows, K and N 1024 .. 14336; rms error 5 %, Q4NX 3.5 %; on weights in the last-level cache they take 10 % less)
+static double wsp_us(int K, double rounds, long tiles, int ncb, bool q4) {
+    const double share = std::min(1.0, (double)tiles / (256.0 * rounds));
+    return q4 ? 2.0 + rounds * (2.27 * ncb - 0.63 + 1e-3 * K * (0.93 + 0.07 * share) * (9.21 + 2.88 * ncb))
+              : 2.0 + rounds * (2.68 * ncb - 1.64 + 1e-3 * K * (0.91 + 0.09 * share) * (8.98 + 2.10 * ncb));
 }
+static double wsp_us(int K, const Widths &wd, int tiles_m, bool q4) { return wsp_us(K, wd.rounds, (long)tiles_m * (wd.wide + wd.narrow), wd.wide ? wd.ncb : wd.ncb_narrow, q4); }
 
 // Slices of K (1: none) in tiles of 256 columns for products of many rows that have too few of them for the chip, where the whole-K
 // launch takes narrow ones: they cost 1.4 to 2 times as much per column.  The fp32 sums are written and read once, at 5 TB/s.
@@ -812,11 +813,12 @@ struct WspSlices {
 static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
     const Widths wd = pick_widths(tiles_m, N / 64, 256, false);
-    WspSlices best{1, wsp_us(K, (long)tiles_m * (wd.wide + wd.narrow), wd.ncb, q4)};
+    WspSlices best{1, wsp_us(K, wd, tiles_m, q4)};
     if (M < 512 || N % 256 || g_gemv_ws_tune.prefill_tile) return best;
     const double whole = best.us;
     for (int s = 2; s <= 8 && s <= K / (4 * kGroup) && 2L * s * N <= (long)K + N && (size_t)s * M * N * sizeof(float) <= scratch_bytes; ++s) {
-        const double us = wsp_us((K + s - 1) / s, (long)tiles_m * (N / 256) * s, 4, q4) + 3.0 + s * ((double)M * N * 8e-6 / 5.0);
+        const long tiles = (long)tiles_m * (N / 256) * s;
+        const double us = wsp_us((K + s - 1) / s, (double)((tiles + 255) / 256), tiles, 4, q4) + 3.0 + s * ((double)M * N * 8e-6 / 5.0);
         if (us < 0.92 * whole && us < best.us) best = {s, us};
     }
     return best;
@@ -824,8 +826,7 @@ static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) 
 double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes) { return wsp_slices(M, K, N, q4, scratch_bytes).us; }
 double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
-    const Widths wd = pick_widths(tiles_m, 2 * H / 64, 256, true);
-    return wsp_us(K, (long)tiles_m * (wd.wide + (wd.ncb == 4 ? wd.narrow : 0)), wd.wide ? wd.ncb : 3, q4);
+    return wsp_us(K, pick_widths(tiles_m, 2 * H / 64, 256, true), tiles_m, q4);
 }
 size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most) {
     const int s = wsp_slices(M, K, N, q4, most).slices;

@@ -17,14 +17,21 @@
 //   Q4NX       : a scale and a minimum per K-step would make that flush four times as dear: s q, which has 12 significant bits, is cut
 //                into two bf16, and the minimum is an operand of its own: three MFMAs per K-step with every product exact, as s sum q x +
 //                min sum x has them.  (s q + min in two operands keeps 16 bits of it, which loses minima small against the scale.)
-//   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, in its order of sums: the same bits, and a residual is
+//   rounded    : bf16 weights as the tiled kernel of gemm_ws.hip multiplies them, on whole K in its order of sums: the same bits, and a residual is
 //                added to the rounded product as its epilogue does.  KW = 1, and an accumulator's products follow each other, so what hides a wave's LDS reads and
 //                dequantisation are its own products: those of a K-step run beside the reads and the dequantisation of the next one (sm_interleave), across
-//                groups too, for which a group has landed one group ahead.  What bounds it then is issue, 4 cycles an instruction: a group of 5 x 3 tiles has 240
-//                vector, 60 matrix and 110 other ones.  Tall and wide forms (up to 10 x 2 and 7 x 3 tiles, one workgroup to a CU, rings of 160 KB) need the fewest.
-//                us before / with: 300 rows of 4096 x 11008 40.7 / 36.4 (5 x 3 tiles instead of 4 x 2), 256 of 4096 x 14336 41.0 / 35.4 (8 x 2), 160 of 4096 x 11008 28.4 / 27.1,
-//                300 of 14336 x 4096 68.0 / 62.9; 120 random products of 66 to 1400 rows 1.049 times as fast.  (Every instruction in its place by volatile asm, none behind one that it
-//                depends on: 38.3, 34.6, 27.3, 72: not taken.)
+//                groups too.  What bounds it then is issue, 4 cycles an instruction: a group of 5 x 3 tiles has 240 vector, 60 matrix and 110 other ones.  Tall and wide
+//                forms (up to 10 x 2 and 7 x 3 tiles, one workgroup to a CU, rings of 160 KB) need the fewest; two workgroups to a CU, each with half of LDS, hide each
+//                other's latencies and fill the chip with twice as many tiles.  Reading a group ahead takes a stage of the ring: with four it is asked for two groups
+//                before it is needed, with three one group, with two it could not be.  So with fewer than four all of a group's x is read in its first half (kEarly: 2 RT more
+//                registers of operands) and its own stage is filled again: three stages are two groups, two stages one.
+//                Weights from memory, us, K-steps one after the other / read ahead without kEarly, where two stages leave one workgroup to a CU / now: 349 rows of 4352 x 13760
+//                54.9 / 64.5 / 52.5, 386 of 6656 x 12800 82.2 / 95.4 / 82.9, 652 of 1280 x 8896 22.6 / 27.8 / 22.2, 170 of 2048 x 5120 11.5 / 12.4 / 11.5, 1519 of 1536 x 5568 31.6 /
+//                40.2 / 32.6, 300 of 4096 x 11008 43.0 / 39.1 / 38.4, Q4NX 486 of 2560 x 12480 45.1 / 60.0 / 42.3, 282 of 10240 x 6336 69.4 / 77.3 / 67.5.  400 random products of 129 to
+//                2000 rows against the loop of K-steps one after the other: 1.14 times as fast (from memory 0.90 at worst, five below 0.95: 1000 to 1300 rows of wide short matrices,
+//                where the tiled kernel and the tallest forms are close, and eight groups of K; from the last-level cache 0.92, one); 17 to 128 rows, exact ones mostly, 1.06 and 1.07
+//                (0.94 and 0.96 at worst).  (Every instruction in its place by
+//                volatile asm, none behind one that it depends on, 300 of 4096 x 11008 36.4 -> 38.3: not taken.)
 //   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
 #include <algorithm>
 #include <utility>
@@ -52,15 +59,13 @@ struct SmArgs {
     int own_sets;                  // column sets of one matrix
 };
 
-// (rounded: two workgroups to a CU where three stages of each fit LDS, else one with all of it)
 // A step in LDS: the x tiles of its groups, then per wave its cells and its scale words ([64]: tile lane / 16, column lane % 16; Q4NX:
 // [NT][64], K-step lane / 16)
 constexpr int sm_wave_bytes(int nt, bool q4) { return nt * (int)kWsCellBytes + (q4 ? nt : 1) * 256; }
 constexpr int sm_stage(int rt, int nt, int kw, bool q4) { return kw * (16 * rt * 256 + 4 * sm_wave_bytes(nt, q4)); }
 constexpr int sm_sums(int rt, int kw, bool q4) { return q4 ? 0 : 2 * kw * 16 * rt * 4; }   // bytes of the sums of x of two steps
-constexpr bool sm_together(int rt, int nt, bool q4) { return 3 * sm_stage(rt, nt, 1, q4) <= kSmLds / 2; }
-constexpr int sm_ring(int rt, int nt, int kw, bool q4) {
-    const int n = ((kw == 1 && sm_together(rt, nt, q4) ? kSmLds / 2 : kSmLds) - sm_sums(rt, kw, q4)) / sm_stage(rt, nt, kw, q4);
+constexpr int sm_ring(int rt, int nt, int kw, bool q4, bool two) {
+    const int n = ((two ? kSmLds / 2 : kSmLds) - sm_sums(rt, kw, q4)) / sm_stage(rt, nt, kw, q4);
     return n < 4 ? n : 4;
 }
 
@@ -87,13 +92,13 @@ __device__ __forceinline__ floatx4 widen4(uint2 v) {
 __device__ __forceinline__ uint2 narrow4(floatx4 v) { return uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}; }
 __device__ __forceinline__ floatx4 rounded4(floatx4 v) { return widen4(narrow4(v)); }
 
-template <int RT, int NT, int KW, int MODE>
+template <int RT, int NT, int KW, int MODE, bool TWO>
 __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(const SmArgs p) {
     constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded, kExact = MODE == kSmAwq;
     constexpr int ROWS = 16 * RT, XT = ROWS * 256;                     // rows and bytes of an x tile (a group: 128 bf16 a row)
     constexpr int MC = Q4 ? NT : 1;                                    // copies (256 bytes) of a wave's scale words
     constexpr int V = RT + NT + MC;                                    // requests of a wave and step: x, cells, scale words
-    constexpr int kWave = sm_wave_bytes(NT, Q4), kStage = sm_stage(RT, NT, KW, Q4), R = sm_ring(RT, NT, KW, Q4);
+    constexpr int kWave = sm_wave_bytes(NT, Q4), kStage = sm_stage(RT, NT, KW, Q4), R = sm_ring(RT, NT, KW, Q4, TWO);
     // Exact AWQ by two waves a SIMD: pipelined.  (Four waves hide each other's latencies, and there are few registers: 2 x 2 tiles 16.0 us without, 17.0 with, 64 rows of 4096 x 14336.)
     constexpr bool kAhead = kExact && KW == 2 && RT * NT <= 12;
     constexpr bool kSums = kExact && !kAhead && R > 2 && RT <= 4;      // sums of x handed round, taken a step ahead; else a wave takes its own
@@ -225,7 +230,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 
     // The first steps are requested; past the slice's end its last group once more (into a stage that nobody reads again).
     const int g_wave = g_lo + kq, g_last = g_hi - 1;
-    constexpr int kFirst = kAhead ? R : R - 1;
+    constexpr bool kEarly = MODE >= kSmAwqRounded && R < 4 && TWO;   // (2 x 1 and 3 x 1 tiles have four stages: 1 to 4 % slower with it)
+    constexpr int kFirst = kAhead || kEarly ? R : R - 1;
 #pragma unroll
     for (int i = 0; i < kFirst; ++i) request(min(g_wave + i * KW, g_last), i * kStage);
     // VALU instructions, LDS reads and copies of a K-step
@@ -366,9 +372,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
             flush(own);
         }
     } else if constexpr (MODE >= kSmAwqRounded) {
+        static_assert(kEarly || R >= 3, "a group lands while another is multiplied");
         // Products of K-step t from one side of a and b, while the other one is made.  Between K-steps 1 and 2 the next group has landed for everybody, and nobody
-        // reads the one before this any more: its stage is filled from there on.
-        bf16x8 a[2][RT], b[2][NT];
+        // reads the one before this any more (kEarly: this one), whose stage is filled from there on.
+        bf16x8 a[kEarly ? 4 : 2][RT], b[2][NT];
         u32x4 cell[NT];
         uint32_t word[NT][Q4 ? 4 : 1];
         AwqScale d[NT];
@@ -415,15 +422,15 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
                 }
             }
         };
-        auto products = [&](int side) {
+        auto products = [&](int t) {
 #pragma unroll
             for (int c = 0; c < NT; ++c)
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[side][rt], b[side][c], Y[rt][c], 0, 0, 0);
+                for (int rt = 0; rt < RT; ++rt) Y[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kEarly ? t : t & 1][rt], b[t & 1][c], Y[rt][c], 0, 0, 0);
         };
         constexpr int kDq = NT * (Q4 ? 25 : 17);
         constexpr std::integral_constant<int, RT * NT> P;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * V) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kFirst - 1) * V) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         read_w(0);
@@ -433,35 +440,37 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         for (int g = g_lo; g < g_hi; ++g) {
 #pragma unroll
             for (int j = 0; j < RT; ++j) asm volatile("" : "+v"(xoff[j]));
-            const int fill = stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
-            const int gn = min(g + R - 1, g_last);
+            const int fill = kEarly ? stage : stage == 0 ? (R - 1) * kStage : stage - kStage, next = stage == (R - 1) * kStage ? 0 : stage + kStage;
+            const int gn = min(g + kFirst, g_last);
             __builtin_amdgcn_sched_barrier(0);
             read_a(stage, 1, 1);
+            if constexpr (kEarly) read_a(stage, 2, 2);
             dequant(1, 1);
             products(0);
-            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
+            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, kEarly ? 2 * RT : RT>(), std::integral_constant<int, 0>());
             __builtin_amdgcn_sched_barrier(0);
-            read_a(stage, 2, 0);
+            if constexpr (kEarly) read_a(stage, 3, 3);
+            else read_a(stage, 2, 0);
             dequant(2, 0);
             keep_last();
             products(1);
             interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT>(), std::integral_constant<int, 0>());
             __builtin_amdgcn_sched_barrier(0);
-            // the next group has landed for everybody, and nobody reads the one before this any more
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 3) * V) : "memory");
+            // the next group has landed for everybody, and nobody reads the stage to fill any more
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kFirst - 2) * V) : "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            read_a(stage, 3, 1);
+            if constexpr (!kEarly) read_a(stage, 3, 1);
             read_w(next);
             dequant(3, 1);
-            products(0);
+            products(2);
             request_x(gn, fill, 0, RT);
-            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, RT + NT * (Q4 ? 5 : 2)>(), std::integral_constant<int, RT>());
+            interleave(P, std::integral_constant<int, kDq>(), std::integral_constant<int, (kEarly ? 0 : RT) + NT * (Q4 ? 5 : 2)>(), std::integral_constant<int, RT>());
             __builtin_amdgcn_sched_barrier(0);
             read_a(next, 0, 0);
             scales();
             dequant(0, 0);
-            products(1);
+            products(3);
             request_w(gn, fill);
             interleave(P, std::integral_constant<int, kDq + (Q4 ? 0 : 4 * NT)>(), std::integral_constant<int, RT>(), std::integral_constant<int, NT + MC>());
             __builtin_amdgcn_sched_barrier(0);
@@ -752,53 +761,71 @@ void parts_at_a_time(int slices, F f) {
     else f(std::integral_constant<int, 8>());
 }
 
-template <int RT, int NT, int KW, int MODE>
+template <int RT, int NT, int KW, int MODE, bool TWO>
 hipError_t launch_wsm(const SmArgs &p, hipStream_t stream) {
     constexpr bool Q4 = MODE == kSmQ4 || MODE == kSmQ4Rounded;
-    constexpr size_t ring = (size_t)sm_ring(RT, NT, KW, Q4) * sm_stage(RT, NT, KW, Q4) + sm_sums(RT, KW, Q4);
+    constexpr size_t ring = (size_t)sm_ring(RT, NT, KW, Q4, TWO) * sm_stage(RT, NT, KW, Q4) + sm_sums(RT, KW, Q4);
     constexpr size_t out = (size_t)16 * RT * (64 * NT + 4) * sizeof(float), parts = (size_t)(KW - 1) * 4 * RT * NT * 1024;
     constexpr size_t lds = ring > out ? (ring > parts ? ring : parts) : out > parts ? out : parts;
     static_assert(lds <= kSmLds, "fits LDS");
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wsm_kernel<RT, NT, KW, MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wsm_kernel<RT, NT, KW, MODE, TWO>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     if ((p.blocks - 1) * 16 * RT >= p.M || p.blocks * 16 * RT < p.M) return hipErrorInvalidValue;   // every block has rows, every row a block
     const int total = p.sets * p.slices * p.blocks;
-    hipLaunchKernelGGL((gemm_wsm_kernel<RT, NT, KW, MODE>), dim3((total + 7) / 8 * 8), dim3(256 * KW), lds, stream, p);
+    hipLaunchKernelGGL((gemm_wsm_kernel<RT, NT, KW, MODE, TWO>), dim3((total + 7) / 8 * 8), dim3(256 * KW), lds, stream, p);
     return hipGetLastError();
 }
 
 // Four groups to a step for the smallest row tiles, whose waves have least to do in one.
 template <int NT, int MODE>
-hipError_t launch_wsm_rt(int rt, const SmArgs &p, hipStream_t stream) {
-    constexpr int KW = MODE >= kSmAwqRounded ? 1 : 2;   // (rounded: the sums in one order)
+hipError_t launch_wsm_exact(int rt, const SmArgs &p, hipStream_t stream) {
     switch (rt) {
-        case 1:
-        case 2: return launch_wsm<2, NT, KW == 1 ? 1 : 4, MODE>(p, stream);
-        case 3: return launch_wsm<3, NT, KW, MODE>(p, stream);
-        case 4: return launch_wsm<4, NT, KW, MODE>(p, stream);
-        case 5: return launch_wsm<5, NT, KW, MODE>(p, stream);
-        case 6: return launch_wsm<6, NT, KW, MODE>(p, stream);
-        case 7: return launch_wsm<7, NT, KW, MODE>(p, stream);
-        default:
-            if constexpr (MODE >= kSmAwqRounded && NT == 2) return rt == 8 ? launch_wsm<8, NT, KW, MODE>(p, stream) : launch_wsm<10, NT, KW, MODE>(p, stream);
-            else return hipErrorInvalidValue;
+        case 2: return launch_wsm<2, NT, 4, MODE, false>(p, stream);
+        case 3: return launch_wsm<3, NT, 2, MODE, false>(p, stream);
+        case 4: return launch_wsm<4, NT, 2, MODE, false>(p, stream);
+        case 5: return launch_wsm<5, NT, 2, MODE, false>(p, stream);
+        case 6: return launch_wsm<6, NT, 2, MODE, false>(p, stream);
+        case 7: return launch_wsm<7, NT, 2, MODE, false>(p, stream);
+        default: return hipErrorInvalidValue;
     }
+}
+
+// Forms of products of rounded weights (KW = 1: the sums in one order).  `two`: two workgroups to a CU.  For AWQ and Q4NX the microseconds that a workgroup takes besides its groups,
+// that a group takes one that is alone, what is added with every CU full, and with just more workgroups than CUs.  Fitted to 1200 products in a graph with every form (17 .. 1600
+// rows, K and N 1024 .. 14336; half of them on weights from memory, which takes the forms of few tiles up to a tenth longer): rms error 4 to 5 %, the form it picks takes 0.2 to 0.7 % more
+// than the best of them on average.  (3 x 3 tiles, and 4 x 3 by two workgroups, are never more than 1 % faster than all others.)
+struct SmForm {
+    int rt, nt;
+    bool two;
+    float each[2], alone[2], more[2], half[2];
+};
+constexpr SmForm kSmForms[] = {{4, 3, false, {3.93f, 3.87f}, {0.856f, 0.974f}, {0.079f, 0.067f}}, {5, 3, false, {4.49f, 4.59f}, {0.880f, 1.031f}, {0.106f, 0.082f}},
+                               {6, 1, false, {2.47f, 2.32f}, {0.497f, 0.542f}, {0.049f, 0.050f}}, {7, 1, false, {2.81f, 2.62f}, {0.521f, 0.563f}, {0.072f, 0.065f}},
+                               {5, 2, false, {3.26f, 3.36f}, {0.682f, 0.777f}, {0.077f, 0.065f}}, {6, 2, false, {3.87f, 3.78f}, {0.729f, 0.810f}, {0.090f, 0.074f}},
+                               {7, 2, false, {4.22f, 4.21f}, {0.777f, 0.956f}, {0.109f, 0.078f}}, {8, 2, false, {3.72f, 3.38f}, {0.936f, 1.112f}, {0.084f, 0.024f}},
+                               {10, 2, false, {4.61f, 4.49f}, {1.019f, 1.163f}, {0.128f, 0.103f}}, {6, 3, false, {4.97f, 4.98f}, {0.916f, 1.125f}, {0.149f, 0.100f}},
+                               {7, 3, false, {4.98f, 4.73f}, {1.028f, 1.275f}, {0.154f, 0.077f}}, {2, 1, true, {1.18f, 1.11f}, {0.415f, 0.441f}, {0.021f, 0.034f}, {0.157f, 0.196f}},
+                               {3, 1, true, {1.72f, 1.44f}, {0.407f, 0.456f}, {0.200f, 0.206f}, {0.193f, 0.223f}}, {4, 1, true, {1.96f, 1.79f}, {0.437f, 0.484f}, {0.265f, 0.263f}, {0.239f, 0.254f}},
+                               {5, 1, true, {2.28f, 2.19f}, {0.479f, 0.500f}, {0.333f, 0.338f}, {0.294f, 0.308f}}, {6, 1, true, {1.93f, 1.36f}, {0.686f, 0.727f}, {0.260f, 0.245f}, {0.180f, 0.224f}},
+                               {3, 2, true, {2.46f, 2.44f}, {0.592f, 0.690f}, {0.360f, 0.351f}, {0.355f, 0.406f}}, {4, 2, true, {2.97f, 3.05f}, {0.645f, 0.737f}, {0.414f, 0.445f}, {0.394f, 0.463f}},
+                               {6, 2, true, {2.96f, 2.69f}, {0.841f, 0.935f}, {0.514f, 0.504f}, {0.469f, 0.512f}}, {7, 2, true, {3.29f, 3.21f}, {0.927f, 1.017f}, {0.593f, 0.534f}, {0.551f, 0.559f}},
+                               {5, 3, true, {3.81f, 3.59f}, {0.942f, 1.191f}, {0.679f, 0.564f}, {0.646f, 0.686f}}};
+
+template <int MODE, size_t... I>
+hipError_t launch_wsm_rounded(const WsmPlan &plan, const SmArgs &p, hipStream_t stream, std::index_sequence<I...>) {
+    hipError_t e = hipErrorInvalidValue;
+    auto one = [&](auto i) {
+        constexpr SmForm f = kSmForms[decltype(i)::value];
+        if (plan.rt == f.rt && plan.nt == f.nt && plan.two == f.two) e = launch_wsm<f.rt, f.nt, 1, MODE, f.two>(p, stream);
+    };
+    (one(std::integral_constant<size_t, I>()), ...);
+    return e;
 }
 
 template <int MODE>
 hipError_t launch_wsm_mode(const WsmPlan &plan, const SmArgs &p, hipStream_t stream) {
-    if constexpr (MODE >= kSmAwqRounded) {
-        if (plan.nt == 3) {
-            switch (plan.rt) {
-                case 3: return launch_wsm<3, 3, 1, MODE>(p, stream);
-                case 4: return launch_wsm<4, 3, 1, MODE>(p, stream);
-                case 5: return launch_wsm<5, 3, 1, MODE>(p, stream);
-                case 6: return launch_wsm<6, 3, 1, MODE>(p, stream);
-                default: return launch_wsm<7, 3, 1, MODE>(p, stream);
-            }
-        }
-    }
-    return plan.nt == 1 ? launch_wsm_rt<1, MODE>(plan.rt, p, stream) : launch_wsm_rt<2, MODE>(plan.rt, p, stream);
+    if constexpr (MODE >= kSmAwqRounded) return launch_wsm_rounded<MODE>(plan, p, stream, std::make_index_sequence<sizeof(kSmForms) / sizeof(SmForm)>());
+    else return plan.nt == 1 ? launch_wsm_exact<1, MODE>(plan.rt, p, stream) : launch_wsm_exact<2, MODE>(plan.rt, p, stream);
 }
 
 // The time of a launch on the GPU in microseconds.
@@ -817,30 +844,14 @@ struct SmExactForm {
 };
 constexpr SmExactForm kSmExact[2][6] = {{{0.874f, 0.172f}, {0.690f, 0.044f}, {0.827f, 0.023f}, {1.013f, 0.067f}, {1.072f, 0.082f}, {1.256f, 0.116f}},
                                         {{1.208f, 0.206f}, {0.866f, 0.057f}, {1.077f, 0.066f}, {1.336f, 0.085f}, {1.620f, 0.102f}, {2.023f, 0.f}}};   // [nt - 1][rt - 2]
-// Rounded weights: what a group takes a workgroup that is alone, and what is added with every CU full, for each form there is (AWQ, Q4NX).  Fitted to 1600 timings a codec
-// in a graph (14 matrices from 1024 x 4096 to 10240 x 8192, 66 .. 1600 rows, every form; rms error 5 to 6 %; the form it picks takes 1.2 % more than the best of them on
-// average, 15 % at worst: few columns and much K).
-struct SmForm {
-    int rt, nt;
-    float alone[2], more[2];
-};
-constexpr SmForm kSmForms[] = {{2, 1, {0.248f, 0.281f}, {0.184f, 0.187f}}, {3, 1, {0.340f, 0.363f}, {0.251f, 0.267f}}, {4, 1, {0.421f, 0.461f}, {0.266f, 0.274f}},
-                               {5, 1, {0.488f, 0.496f}, {0.280f, 0.326f}}, {6, 1, {0.456f, 0.488f}, {0.095f, 0.095f}}, {7, 1, {0.491f, 0.531f}, {0.094f, 0.086f}},
-                               {2, 2, {0.484f, 0.555f}, {0.332f, 0.367f}}, {3, 2, {0.559f, 0.655f}, {0.389f, 0.407f}}, {4, 2, {0.613f, 0.685f}, {0.476f, 0.502f}},
-                               {5, 2, {0.679f, 0.794f}, {0.100f, 0.075f}}, {6, 2, {0.741f, 0.847f}, {0.104f, 0.097f}}, {7, 2, {0.805f, 0.991f}, {0.123f, 0.086f}},
-                               {8, 2, {0.866f, 0.951f}, {0.146f, 0.135f}}, {10, 2, {0.974f, 1.166f}, {0.196f, 0.160f}}, {3, 3, {0.745f, 0.966f}, {0.593f, 0.053f}},
-                               {4, 3, {0.861f, 0.969f}, {0.102f, 0.100f}}, {5, 3, {0.912f, 1.058f}, {0.115f, 0.112f}}, {6, 3, {0.951f, 1.157f}, {0.174f, 0.148f}},
-                               {7, 3, {1.006f, 1.268f}, {0.212f, 0.149f}}};
-
 double wsm_rounded_us(const SmForm &f, int blocks, int K, int N, bool q4) {
-    const bool two = sm_together(f.rt, f.nt, q4);   // workgroups to a CU
-    const int chip = two ? 512 : 256, groups = K / kGroup;
+    const int chip = f.two ? 512 : 256, groups = K / kGroup;
     const long wgs = (long)((N + 64 * f.nt - 1) / (64 * f.nt)) * blocks, full = wgs / chip;
-    const double rest = (double)(wgs % chip) / chip, start = q4 ? 3.75 : 3.5, each = q4 ? 2.02 : 2.13;
-    double us = start + full * (each + groups * (f.alone[q4] + f.more[q4]));
-    // (from half of them on some CUs have two, which take most of `more`)
-    const double share = !two ? rest : rest <= 0.5 ? 0.45 * rest : 0.95 + 0.1 * (rest - 0.5);
-    if (rest > 0) us += each + groups * (f.alone[q4] + f.more[q4] * share);
+    const double rest = (double)(wgs % chip) / chip;
+    double us = (q4 ? 2.01 : 1.80) + full * (f.each[q4] + groups * (f.alone[q4] + f.more[q4]));
+    // (two to a CU: from half a round on some CUs have both)
+    const double more = !f.two ? f.more[q4] * rest : rest <= 0.5 ? 0.37 * f.more[q4] * rest : f.half[q4] + (q4 ? 0.72 : 0.79) * f.more[q4] * (rest - 0.5);
+    if (rest > 0) us += f.each[q4] + groups * (f.alone[q4] + more);
     return us;
 }
 
@@ -872,15 +883,15 @@ size_t gemm_wsm_scratch_bytes(const WsmPlan &p, int M, int N) { return p.slices 
 // Parts of products of rounded weights: within 12 MB, as they are where there are fewer workgroups than the chip takes (512 of 64 x 64 results are 8 MB)
 size_t gemm_wsm_parts_bytes(int M, int N) { return M > kWsmSliceRows ? 0 : std::min((size_t)16 * M * N * sizeof(float), (size_t)12 << 20); }
 
-// Slices where few rows leave the chip idle: at least eight groups each, and no more parts than the workspace of a prompt pass always has (gemm_wsm_parts_bytes),
-// so that a plain product and the same one inside such a pass run the same slices.  Whole K / slices: 297 x 8704 x 1280 36.8 / 19.5 us, 369 x 13568 x 1088 53.7 / 23.5,
-// Q4NX 108 x 8448 x 1664 38.8 / 14.0.
+// Slices where few rows leave the chip idle: at least eight groups each, and no more parts than the workspace of a prompt pass has at most (gemm_wsm_parts_bytes); of one
+// matrix, from the rows on from which its plain product has rounded weights, only where whole K would take longer than two launches take the host.  So a plain product and the same
+// one inside such a pass run the same slices, if the pass has that workspace (with less of it fewer).  Whole K / slices: 297 x 8704 x 1280 36.8 / 19.5 us, 369 x 13568 x 1088 53.7 / 23.5, Q4NX 108 x 8448 x 1664 38.8 / 14.0.
 WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scratch_bytes) {
     const auto &tune = g_gemv_ws_tune;
     const int tiles = (M + 15) / 16;
-    WsmPlan best;
-    best.us = -1;
-    double best_rank = 0;   // slices have to be 4 % faster: the estimate is no better than that
+    WsmPlan best, whole;
+    best.us = whole.us = -1;
+    double best_rank = 0;   // slices have to be 2 % faster: a second launch and its scratch for nothing
     // a tune key's form, or the tallest of its width where there is none so tall
     int only_rt = tune.wsm_rt, only_nt = tune.wsm_nt;
     if (only_rt || only_nt) {
@@ -894,8 +905,9 @@ WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scra
     }
     for (const SmForm &f : kSmForms) {
         if ((only_rt && f.rt != only_rt) || (only_nt && f.nt != only_nt) || (f.rt > 8 && K >= 1 << 23)) continue;   // (the copies' 32-bit offsets)
+        if (tune.wsm_two && f.two != (tune.wsm_two == 1) && std::any_of(std::begin(kSmForms), std::end(kSmForms), [&](const SmForm &o) { return o.rt == f.rt && o.nt == f.nt && o.two != f.two; })) continue;
         WsmPlan p;
-        p.rt = f.rt, p.nt = f.nt, p.blocks = (tiles + f.rt - 1) / f.rt;
+        p.rt = f.rt, p.nt = f.nt, p.two = f.two, p.blocks = (tiles + f.rt - 1) / f.rt;
         auto fits = [&](int slices) {
             p.slices = slices;
             return slices <= 1 || (K / kGroup / slices >= 8 && M <= kWsmSliceRows &&
@@ -907,11 +919,13 @@ WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scra
             if (!fits(slices)) break;
             p.us = wsm_rounded_us(f, p.blocks * slices * matrices, (K / kGroup + slices - 1) / slices * kGroup, N, q4);
             if (slices > 1) p.us += 0.98 + 0.21 * ((slices + 7) / 8) + slices * matrices * ((double)M * N * 8e-6 / 3.52);
-            const double rank = slices > 1 ? 1.04 * p.us : p.us;
+            const double rank = slices > 1 ? 1.02 * p.us : p.us;
             if (best.us < 0 || rank < best_rank) best = p, best_rank = rank;
+            if (slices == 1 && (whole.us < 0 || p.us < whole.us)) whole = p;
             if (only) break;
         }
     }
+    if (matrices == 1 && M >= gemm_rounded_rows(q4) && best.slices > 1 && whole.us >= 0 && 0.98 * whole.us <= std::max(best.us, kTwoLaunchesUs)) return whole;
     return best;
 }
 
@@ -922,7 +936,7 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
     const int only_nt = tune.wsm_nt <= 2 ? tune.wsm_nt : 0, only_slices = std::min(tune.wsm_slices ? tune.wsm_slices : tune.splitk == 1 ? 2 : 0, G);
     WsmPlan best;
     best.us = -1;
-    double best_rank = 0;   // slices have to be 4 % faster: the estimate is no better than that
+    double best_rank = 0;   // slices have to be 2 % faster: a second launch and its scratch for nothing
     for (int nt = 1; nt <= 2; ++nt) {
         if (only_nt && nt != only_nt) continue;
         const int options[3] = {few, few + 1, (tiles + 3) / 4};   // blocks of rows
@@ -936,7 +950,7 @@ WsmPlan plan_gemm_wsm(int M, int K, int N, bool q4, bool rounded, size_t scratch
                 p.slices = slices;
                 if (slices > 1 && gemm_wsm_scratch_bytes(p, M, N) > scratch_bytes) return false;
                 p.us = wsm_us(p, M, K, N, q4);
-                const double rank = slices > 1 ? 1.04 * p.us : p.us;
+                const double rank = slices > 1 ? 1.02 * p.us : p.us;
                 if (best.us < 0 || rank < best_rank) best = p, best_rank = rank;
                 return true;
             };

@@ -841,10 +841,11 @@ static int gemm_ws_cb(int tiles) {
 }
 
 // Each launch rounds of workgroups over the chip, a group of K a cost by rows and tile columns.  Launches of up to 64 rows: fitted to 360 timings (60 matrices of K = 1024 ..
-// 14336, 17 .. 128 rows; rms error 6 %); of 16 (Q4NX, or with a residual): to 13 matrices (Q4NX, 32 rows of K = 4096, N = 14336 26.1 estimated / 24.1 measured)
+// 14336, 17 .. 128 rows; rms error 6 %; a second round of single columns runs beside the first one's end); of 16 (Q4NX, or with a residual): to 13 matrices (Q4NX, 32 rows of K = 4096, N = 14336 26.1 estimated / 24.1 measured)
 double gemm_ws_us(int M, int K, int N, bool q4, bool residual) {
     const int tiles = N / kWsTileCols, cb = gemm_ws_cb(tiles), most = q4 || residual ? 16 : 64, G = K / kGroup;
-    const double rounds = (tiles / cb + 255) / 256, wide = cb == 4 ? 0.136 : cb == 2 ? 0.076 : 0.042, step16 = cb == 4 ? 0.33 : cb == 2 ? 0.20 : 0.15;
+    const int whole = (tiles / cb + 255) / 256;
+    const double rounds = most == 64 && cb == 1 ? 0.2 + 0.8 * whole : whole, wide = cb == 4 ? 0.136 : cb == 2 ? 0.076 : 0.042, step16 = cb == 4 ? 0.33 : cb == 2 ? 0.20 : 0.15;
     auto launch = [&](int rows) { return most == 16 ? 2.5 + G * rounds * step16 * (0.5 + rows / 32.0) : 3.3 + G * rounds * (wide + 0.007 * rows); };
     return (M / most) * launch(most) + (M % most ? launch(M % most) : 0);
 }

@@ -110,6 +110,7 @@ struct GemvWsTune {
     int prefill_band = 0;    // prefill kernel: row panels per band of the tile order (0 = default)
     int splitk = 0;          // exact products of 17 rows and more: 0 by shape, 1 always gemm_wsm.hip, in two slices of K where the scratch holds them, 2 always whole-K launches
     int wsm_rt = 0, wsm_nt = 0, wsm_slices = 0;   // gemm_wsm.hip: row tiles, 64-column sets and slices where a kernel has them (0: by time)
+    int wsm_two = 0;   // of two forms of a size the one of two workgroups to a CU (1) or of one (2)
     int prefill_wsm = 0;     // products of rounded weights: 0 by time, 1 always gemm_wsm.hip, 2 never
     int prefill_swiglu_split = 0;   // 1: the prompt-pass FFN runs gate and up as two launches instead of one
 };
@@ -133,6 +134,7 @@ double gemm_ws_us(int M, int K, int N, bool q4, bool residual);   // its time, a
 // `rounded`: bf16-rounded weights, the bits of launch_gemm_prefill_ws; a residual is added to the rounded product.
 struct WsmPlan {
     int rt, blocks, nt, slices;
+    bool two = false;   // two workgroups to a CU (rounded weights)
     double us;   // the estimate by which it was chosen
 };
 bool gemm_wsm_supported(int M, int K, int N);
@@ -144,6 +146,8 @@ hipError_t launch_gemm_wsm(const WsmPlan &p, const uint16_t *x, const void *w, u
 // epilogues on this product); `gate` [M, H] is scratch.
 WsmPlan plan_wsm_rounded(int M, int K, int N, int matrices, bool q4, size_t scratch_bytes);
 constexpr int kWsmSliceRows = 512;           // more rows run whole K
+constexpr int gemm_rounded_rows(bool q4) { return q4 ? 65 : 129; }   // rows from which a plain product has rounded weights
+constexpr double kTwoLaunchesUs = 12.5;      // what two launches and their scratch take a host that issues calls one after the other
 size_t gemm_wsm_parts_bytes(int M, int N);   // the most scratch that such a plan asks for
 hipError_t launch_gemm_wsm_rope(const WsmPlan &p, const uint16_t *x, const void *w, uint16_t *y, const uint16_t *lut, const GemmRope &rope, float *scratch, int M, int K, int N,
                                 bool q4, hipStream_t stream);

@@ -166,7 +166,7 @@ static bool by_wsm(const WsmPlan &plan, double elements, double tiled_us) {
     const auto &tune = g_gemv_ws_tune;
     double more = plan.slices == 1 && elements > 0 ? 1.2 + elements * 4e-6 / 3.5 : 0.0;   // (the sum of slices is part of the plan's time)
     if ((plan.slices > 1 || elements > 0) && plan.us < 12) more += 2.8;
-    return plan.us >= 0 && !tune.prefill_tile && tune.prefill_wsm != 2 && (tune.prefill_wsm == 1 || plan.us + more < 0.95 * tiled_us);
+    return plan.us >= 0 && !tune.prefill_tile && tune.prefill_wsm != 2 && (tune.prefill_wsm == 1 || plan.us + more < 0.97 * tiled_us);
 }
 
 hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t *norm_w, float eps, const void *wqkv,

@@ -308,6 +308,36 @@ def test_rounded_tiles_of_every_ring(codec, rt, nt):
                     ops.tune(key, 0)
 
 
+@pytest.mark.parametrize("codec", ["awq", "q4nx"])
+@pytest.mark.parametrize("rt,nt,two", [(2, 1, 1), (4, 1, 1), (5, 1, 1), (6, 1, 1), (6, 1, 2), (3, 2, 1), (4, 2, 1), (6, 2, 1), (7, 2, 1), (7, 2, 2), (5, 3, 1), (5, 3, 2)])
+def test_rounded_tiles_of_one_and_two_workgroups_to_a_cu(codec, rt, nt, two):
+    """Rings of two, three and four stages of half of LDS, from as many groups as stages on, whole and in slices: on whole K the tiled kernel's bits, a grid that leaves no CU
+    with one workgroup included; in slices one more rounding of fp32 sums."""
+    from air_hip import ops
+    keys = ("prefill_min_m", "prefill_wsm", "gemm_wsm_rt", "gemm_wsm_nt", "gemm_wsm_two", "gemm_wsm_slices")
+    for M, K, N in ((16 * rt * max(1, 80 // (16 * rt)) + 1, 256, 64 * nt + 64), (16 * rt * 2 - 7, 512, 64 * nt), (16 * rt * 4 - 1, 768, 64 * 3 * nt), (200, 2048 + 256, 1024),
+                    (16 * rt * 24, 1024, 64 * nt * 24)):
+        print("rounded tiles, workgroups to a CU", codec, rt, nt, two, M, K, N, flush=True)
+        if codec == "awq":
+            w, product = ops.repack_stream(*map(dev, make_awq(K, N, seed=rt))), ops.w4a16_gemm_stream
+        else:
+            q, s, m = make(N, K, seed=rt)
+            w, product = ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T)), ops.q4nx_gemm_stream
+        x = dev(make_x((M, K), seed=K))
+        try:
+            results = []
+            for values in ((17, 1, rt, nt, two, 1), (17, 2, 0, 0, 0, 0), (17, 1, rt, nt, two, 2)):
+                for key, value in zip(keys, values):
+                    ops.tune(key, value)
+                results.append(product(x, w))
+            assert torch.equal(*(r.view(torch.int16) for r in results[:2])), (codec, rt, nt, two, M, K)
+            whole, cut = results[0].double(), results[2].double()
+            assert bool(((whole - cut).abs() <= 2.0 ** -7 * whole.abs() + 2.0 ** -14 * whole.abs().amax()).all()), (codec, rt, nt, two, M, K)
+        finally:
+            for key in keys:
+                ops.tune(key, 0)
+
+
 @pytest.mark.parametrize("rt,nt", [(3, 1), (4, 1), (7, 1), (3, 2), (4, 2), (6, 2)])
 def test_exact_tiles_of_few_groups(rt, nt):
     """Pipelined exact tiles with fewer groups than sets of waves, than stages, and one more than whole steps: one bf16 rounding of an fp32 sum; a row of infinities stays
