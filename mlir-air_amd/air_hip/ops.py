@@ -690,7 +690,7 @@ def prefill_rms_qkv_rope_stream(x, attn_norm_weight, wqkv, rope_lut, pos0, n_hea
     if (wqkv.K, wqkv.N) != (E, N):
         raise ValueError(f"wqkv is [{wqkv.K}, {wqkv.N}], the block needs [{E}, {N}]")
     out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    key = (x.device.index, _stream(), "prefill_qkv", M, E)
+    key = (x.device.index, _stream(), "prefill_qkv_stream", M, E)
     ws = _attn_ws.get(key)
     if ws is None:
         ws = torch.empty(int(lib.w4a16_prefill_qkv_workspace_most(M, E)), dtype=torch.uint8, device=x.device)
@@ -721,7 +721,7 @@ def prefill_o_ffn_stream(attn_out, x_residual, ffn_norm_weight, wo, gate, up, do
     y = torch.empty((M, E), dtype=torch.bfloat16, device=attn_out.device)
     res1 = torch.empty((M, E), dtype=torch.bfloat16, device=attn_out.device) if return_intermediates else None
     h = torch.empty((M, H), dtype=torch.bfloat16, device=attn_out.device) if return_intermediates else None
-    key = (attn_out.device.index, _stream(), "prefill_block", M, E, H)
+    key = (attn_out.device.index, _stream(), "prefill_block_stream", M, E, H)
     ws = _attn_ws.get(key)
     if ws is None:
         ws = torch.empty(int(lib.w4a16_prefill_block_workspace_most(M, E, H)), dtype=torch.uint8, device=attn_out.device)

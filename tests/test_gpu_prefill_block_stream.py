@@ -315,6 +315,31 @@ def test_prefill_blocks_stream_in_the_least_workspace(ops, M):
         assert bool(((got - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1)).all())
 
 
+@pytest.mark.parametrize("M", [33, 100])
+def test_prefill_blocks_stream_after_those_on_the_checkpoint_layout(ops, monkeypatch, M):
+    """The same sizes in both layouts in one process: the stream blocks run in as many slices, and so with the same bits, as where they come first."""
+    from oracle import decode as odec
+    E, H, nh, nkv, hd = 2048, 4096, 24, 4, 64
+    parts, fused = _qkv_weights(E, nh, nkv, hd, seed=M)
+    layer = _weights(E, H, seed=M)
+    sw, ws = _sw(ops, fused), [_sw(ops, w) for w in layer]
+    lut = dev(odec.generate_rope_lut(hd, 500000.0, M))
+    x, attn, nw = dev(make_x((M, E), seed=M)), dev(make_x((M, E), seed=M + 1)), dev(_norm_w(E, 3))
+    on_gpu = lambda w: tuple(map(dev, w))
+    print("prompt blocks of both layouts", M, flush=True)
+
+    def stream():
+        return ops.prefill_rms_qkv_rope_stream(x, nw, sw, lut, 0, nh, nkv, hd), ops.prefill_o_ffn_stream(attn, x, nw, *ws)
+
+    monkeypatch.setattr(ops, "_attn_ws", {})
+    first = stream()
+    monkeypatch.setattr(ops, "_attn_ws", {})
+    ops.prefill_rms_qkv_rope(x, nw, on_gpu(fused), lut, 0, nh, nkv, hd)
+    ops.prefill_o_ffn(attn, x, nw, *map(on_gpu, layer))
+    for got, want in zip(stream(), first):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 # 192-column tiles of heads of 128 (a head and half of one) and of gate and up: one of them, several, beside wide ones, ragged rows
 @pytest.mark.parametrize("M,E,nh,nkv,pos0,tile", [(100, 256, 1, 1, 4, 2), (270, 512, 4, 1, 0, 2), (2048, 256, 9, 3, 9, 0), (1000, 256, 32, 8, 2, 0)])
 def test_prefill_rms_qkv_rope_stream_in_192_columns(ops, tiled_gemm, M, E, nh, nkv, pos0, tile):
