@@ -418,7 +418,8 @@ int w4a16_decode_attention_bf16(const uint16_t *qkv, const uint16_t *rope_lut_ro
  * prefill ELFs): out[m, :] = bf16((x[m, :] / sqrt(mean(x[m, :]^2) + eps)) * norm_weight), K % 8 == 0, K <= 8192.
  */
 size_t w4a16_prefill_block_workspace_bytes(int M, int E, int H);
-/* What the same on stream-order weights can use: few rows run in slices of K as far as their parts fit behind the bytes above. */
+/* What the same on stream-order weights can use: products of up to 512 rows run in slices of K as far as their parts fit behind the bytes above (at most 12 MB more).  So the
+ * order of their fp32 sums, and with it some roundings of the result, depend on workspace_bytes. */
 size_t w4a16_prefill_block_workspace_most(int M, int E, int H);
 int rms_norm_rows_bf16(const uint16_t *x, const uint16_t *norm_weight, float eps, uint16_t *out, int M, int K,
                        void *stream);
@@ -433,11 +434,12 @@ int w4a16_prefill_o_ffn_bf16(const uint16_t *attn_out, const uint16_t *x_residua
 
 /*
  * The two prompt-pass blocks on stream-order weights (w4a16_repack_stream of the same matrices; the Q|K|V matrices
- * concatenated along N before the re-pack): w4a16_prefill_rms_qkv_rope_bf16 and w4a16_prefill_o_ffn_bf16 with the tiled
- * stream-order GEMM (w4a16_gemm_stream_bf16's kernel for M >= 129) and its fused epilogues in place of the
- * checkpoint-layout GEMM.  Same references (rms_gemms_rope_int4_multi.py:4-17, 414-436, 543-561;
+ * concatenated along N before the re-pack): w4a16_prefill_rms_qkv_rope_bf16 and w4a16_prefill_o_ffn_bf16 with the products of
+ * w4a16_gemm_stream_bf16 on bf16-rounded weights in place of the checkpoint-layout GEMM: for many rows the tiled kernel with RoPE,
+ * residual and SwiGLU in its epilogues, for fewer tiles of fewer rows and columns, by time, in slices of K too, with RoPE, SwiGLU and the sums of slices as launches of
+ * their own.  Same references (rms_gemms_rope_int4_multi.py:4-17, 414-436, 543-561;
  * o_ffn_int4_multi.py:4-17, 644-665), same rounding points, same workspaces (w4a16_prefill_qkv_workspace_bytes,
- * w4a16_prefill_block_workspace_bytes; plain scratch).  E % 256 == 0, H % 256 == 0, every N % 64 == 0.
+ * w4a16_prefill_block_workspace_bytes; plain scratch; .._most for slices).  E % 256 == 0, H % 256 == 0, every N % 64 == 0.
  */
 int w4a16_prefill_rms_qkv_rope_stream_bf16(const uint16_t *x, const uint16_t *attn_norm_weight, float eps, const void *qkv_wstream,
                                            const uint16_t *rope_lut, int rope_lut_rows, int pos0, uint16_t *qkv_out, int M, int E,

@@ -183,7 +183,7 @@ struct PrefillLinear {
 bool prefill_block_supported(int M, int E, int H);
 size_t prefill_block_scratch_bytes(int M, int E, int H);   // sized for split-K on a 256-CU device
 size_t prefill_qkv_scratch_bytes(int M, int E);
-// with room for the parts of the stream-order products of few rows, which run in as many slices as fit
+// with room for the parts of stream-order products of up to kWsmSliceRows rows, which run in as many slices as fit
 size_t prefill_block_scratch_most(int M, int E, int H);
 size_t prefill_qkv_scratch_most(int M, int E);
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream);

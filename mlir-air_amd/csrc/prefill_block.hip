@@ -92,18 +92,12 @@ static size_t block_rows_bytes(int M, int E, int H) { return 2 * round256((size_
 size_t prefill_block_scratch_bytes(int M, int E, int H) { return block_rows_bytes(M, E, H) + round256(splitk_bytes(M, E, H, kPlanCus)); }
 size_t prefill_qkv_scratch_bytes(int M, int E) { return round256((size_t)M * E * sizeof(uint16_t)); }
 
-// (a workspace for many rows also serves fewer of them, whose products run in slices)
-size_t prefill_block_scratch_most(int M, int E, int H) {
-    const int few = std::min(M, kWsmSliceRows);
-    return std::max(block_rows_bytes(M, E, H) + round256(tail_bytes(M, E, H)), block_rows_bytes(few, E, H) + round256(gemm_wsm_parts_bytes(few, std::max(E, 2 * H))));
-}
+// (more rows than run in slices take no more than the least)
+size_t prefill_block_scratch_most(int M, int E, int H) { return block_rows_bytes(M, E, H) + round256(tail_bytes(M, E, H)); }
 
 // Behind the normed rows: parts of the projections of few rows (how wide those are the call says; three times E where every head has keys of its own)
 static size_t qkv_parts_bytes(int M, int E) { return round256(gemm_wsm_parts_bytes(M, 3 * E)); }
-size_t prefill_qkv_scratch_most(int M, int E) {
-    const int few = std::min(M, kWsmSliceRows);
-    return std::max(round256((size_t)M * E * sizeof(uint16_t)) + qkv_parts_bytes(M, E), round256((size_t)few * E * sizeof(uint16_t)) + qkv_parts_bytes(few, E));
-}
+size_t prefill_qkv_scratch_most(int M, int E) { return prefill_qkv_scratch_bytes(M, E) + qkv_parts_bytes(M, E); }
 
 hipError_t launch_rmsnorm_rows(const uint16_t *x, const uint16_t *w, uint16_t *out, int M, int K, float eps, hipStream_t stream) {
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, K, eps);

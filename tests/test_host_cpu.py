@@ -184,6 +184,16 @@ def test_library_exports_every_declared_symbol():
     assert lib.w4a16_strerror(0) == b"ok" and b"128" in lib.w4a16_strerror(_lib.ERR_GROUP)
 
 
+@pytest.mark.parametrize("E,H", [(256, 512), (2048, 8192), (4096, 14336)])
+def test_prompt_workspaces_ask_for_no_more_than_is_used(E, H):
+    """Parts of K slices, at most 12 MB, up to 512 rows; nothing for them past that."""
+    lib = _lib.load_library()
+    for M in (1, 40, 300, 512, 513, 600, 700, 3600, 8192):
+        for least, most in ((lib.w4a16_prefill_qkv_workspace_bytes(M, E), lib.w4a16_prefill_qkv_workspace_most(M, E)),
+                            (lib.w4a16_prefill_block_workspace_bytes(M, E, H), lib.w4a16_prefill_block_workspace_most(M, E, H))):
+            assert least <= most <= least + ((12 << 20) if M <= 512 else 0), (M, E, H)
+
+
 def test_c_abi_rejects_bad_arguments_before_touching_the_gpu():
     lib = _lib.load_library()
     P = 0x10000   # fake, aligned, never dereferenced: validation fails first
