@@ -677,6 +677,18 @@ def prefill_o_ffn(attn_out, x_residual, ffn_norm_weight, wo, gate, up, down, eps
     return (y, res1, h) if return_intermediates else y
 
 
+def _prompt_workspace(use, most, device, M, *widths):
+    """Plain scratch of a prompt block on stream-order weights, kept for the stream.  Up to 512 rows, where parts of K slices are most of it, 64 lengths share one (what a length
+    runs does not depend on what lies behind its own bytes)."""
+    last = (M + 63) // 64 * 64 if M <= 512 else M
+    key = (device.index, _stream(), use, last, *widths)
+    ws = _attn_ws.get(key)
+    if ws is None:
+        ws = torch.empty(max(int(most(m, *widths)) for m in range(last - 63 if M <= 512 else M, last + 1)), dtype=torch.uint8, device=device)
+        _attn_ws[key] = ws
+    return ws
+
+
 def prefill_rms_qkv_rope_stream(x, attn_norm_weight, wqkv, rope_lut, pos0, n_heads, n_kv_heads, head_dim, eps=1e-5, group=GROUP,
                                 codec="awq"):
     """prefill_rms_qkv_rope on a StreamWeight (the re-pack of the concatenated Q|K|V matrix): the tiled stream-order
@@ -690,11 +702,7 @@ def prefill_rms_qkv_rope_stream(x, attn_norm_weight, wqkv, rope_lut, pos0, n_hea
     if (wqkv.K, wqkv.N) != (E, N):
         raise ValueError(f"wqkv is [{wqkv.K}, {wqkv.N}], the block needs [{E}, {N}]")
     out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    key = (x.device.index, _stream(), "prefill_qkv_stream", M, E)
-    ws = _attn_ws.get(key)
-    if ws is None:
-        ws = torch.empty(int(lib.w4a16_prefill_qkv_workspace_most(M, E)), dtype=torch.uint8, device=x.device)
-        _attn_ws[key] = ws
+    ws = _prompt_workspace("prefill_qkv_stream", lib.w4a16_prefill_qkv_workspace_most, x.device, M, E)
     if codec == "q4nx":
         _lib.check(lib.w4a16_q4nx_prefill_rms_qkv_rope_stream_bf16(_ptr(_bits(x)), _ptr(_bits(attn_norm_weight)), float(eps),
                                                                    _ptr(wqkv.buf), _ptr(_bits(rope_lut)), rope_lut.shape[0], int(pos0),
@@ -721,11 +729,7 @@ def prefill_o_ffn_stream(attn_out, x_residual, ffn_norm_weight, wo, gate, up, do
     y = torch.empty((M, E), dtype=torch.bfloat16, device=attn_out.device)
     res1 = torch.empty((M, E), dtype=torch.bfloat16, device=attn_out.device) if return_intermediates else None
     h = torch.empty((M, H), dtype=torch.bfloat16, device=attn_out.device) if return_intermediates else None
-    key = (attn_out.device.index, _stream(), "prefill_block_stream", M, E, H)
-    ws = _attn_ws.get(key)
-    if ws is None:
-        ws = torch.empty(int(lib.w4a16_prefill_block_workspace_most(M, E, H)), dtype=torch.uint8, device=attn_out.device)
-        _attn_ws[key] = ws
+    ws = _prompt_workspace("prefill_block_stream", lib.w4a16_prefill_block_workspace_most, attn_out.device, M, E, H)
     args = (_ptr(_bits(attn_out)), _ptr(_bits(x_residual)), _ptr(_bits(ffn_norm_weight)), float(eps), _ptr(wo.buf), _ptr(gate.buf),
             _ptr(up.buf), _ptr(down.buf), _ptr(y), _ptr(res1) if res1 is not None else None, _ptr(h) if h is not None else None,
             M, E, H)

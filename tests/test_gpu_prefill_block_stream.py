@@ -340,6 +340,30 @@ def test_prefill_blocks_stream_after_those_on_the_checkpoint_layout(ops, monkeyp
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+def test_prompt_lengths_share_their_workspaces(ops, monkeypatch):
+    """64 lengths take the memory of one, and each runs what it runs in a workspace of its own: the same bits after a shorter, after a longer one and alone."""
+    from oracle import decode as odec
+    E, H, nh, nkv, hd = 2048, 1024, 24, 4, 64
+    sw, ws = _sw(ops, _qkv_weights(E, nh, nkv, hd, seed=1)[1]), [_sw(ops, w) for w in _weights(E, H, seed=1)]
+    lut, nw = dev(odec.generate_rope_lut(hd, 500000.0, 200)), dev(_norm_w(E, 3))
+    x, attn = dev(make_x((200, E), seed=1)), dev(make_x((200, E), seed=2))
+    monkeypatch.setattr(ops, "_attn_ws", {})
+
+    def run(M):
+        print("prompt lengths", M, flush=True)
+        return ops.prefill_rms_qkv_rope_stream(x[:M].contiguous(), nw, sw, lut, 0, nh, nkv, hd), ops.prefill_o_ffn_stream(attn[:M].contiguous(), x[:M].contiguous(), nw, *ws)
+
+    lengths = (65, 128, 66, 100, 127)
+    shared = [run(M) for M in lengths]
+    kept = sum(t.numel() for t in ops._attn_ws.values())
+    assert kept <= max(sum(int(f(M, *w)) for f, w in ((ops._lib.load_library().w4a16_prefill_qkv_workspace_most, (E,)),
+                                                      (ops._lib.load_library().w4a16_prefill_block_workspace_most, (E, H)))) for M in range(65, 129)) * 1.1
+    for M, outs in zip(lengths, shared):
+        monkeypatch.setattr(ops, "_attn_ws", {})
+        for got, want in zip(outs, run(M)):
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), M
+
+
 # 192-column tiles of heads of 128 (a head and half of one) and of gate and up: one of them, several, beside wide ones, ragged rows
 @pytest.mark.parametrize("M,E,nh,nkv,pos0,tile", [(100, 256, 1, 1, 4, 2), (270, 512, 4, 1, 0, 2), (2048, 256, 9, 3, 9, 0), (1000, 256, 32, 8, 2, 0)])
 def test_prefill_rms_qkv_rope_stream_in_192_columns(ops, tiled_gemm, M, E, nh, nkv, pos0, tile):
