@@ -810,9 +810,9 @@ struct WspSlices {
     int slices;
     double us;
 };
-static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) {
+static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes, bool heads128 = false) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
-    const Widths wd = pick_widths(tiles_m, N / 64, 256, false);
+    const Widths wd = pick_widths(tiles_m, N / 64, 256, heads128);
     WspSlices best{1, wsp_us(K, wd, tiles_m, q4)};
     if (M < 512 || N % 256 || g_gemv_ws_tune.prefill_tile) return best;
     const double whole = best.us;
@@ -824,6 +824,7 @@ static WspSlices wsp_slices(int M, int K, int N, bool q4, size_t scratch_bytes) 
     return best;
 }
 double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes) { return wsp_slices(M, K, N, q4, scratch_bytes).us; }
+double gemm_prefill_ws_rope_us(int M, int K, int N, int head_dim, bool q4) { return wsp_slices(M, K, N, q4, 0, head_dim == 128).us; }
 double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4) {
     const int tiles_m = (M + kPfRows - 1) / kPfRows;
     return wsp_us(K, pick_widths(tiles_m, 2 * H / 64, 256, true), tiles_m, q4);

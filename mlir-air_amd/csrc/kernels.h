@@ -156,6 +156,7 @@ hipError_t launch_gemm_wsm_swiglu(const WsmPlan &p, const uint16_t *x, const voi
 // Prefill GEMM on stream-order weights (gemm_ws.hip): bf16-rounded weights dequantised in registers, x through LDS.
 bool gemm_prefill_ws_supported(int M, int K, int N);   // K % 256 == 0, N % 64 == 0
 double gemm_prefill_ws_swiglu_us(int M, int K, int H, bool q4);
+double gemm_prefill_ws_rope_us(int M, int K, int N, int head_dim, bool q4);
 double gemm_prefill_ws_us(int M, int K, int N, bool q4, size_t scratch_bytes);   // its time without an epilogue, an estimate for choosing between the kernels
 size_t gemm_prefill_ws_scratch_bytes(int M, int K, int N, bool q4, size_t most);   // plain scratch that makes it faster (0: none)
 // Epilogues as for launch_gemm_prefill (kEpi*); kEpiRope with heads of 128 needs N % 128 == 0.

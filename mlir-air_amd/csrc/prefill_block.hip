@@ -174,7 +174,7 @@ hipError_t launch_prefill_rms_qkv_rope_stream(const uint16_t *x, const uint16_t 
     const int N = (n_heads + 2 * n_kv) * head_dim;
     if (gemm_wsm_supported(17, E, N)) {
         const WsmPlan plan = plan_wsm_rounded(M, E, N, 1, q4, std::min(qkv_parts_bytes(M, E), workspace_bytes - std::min(workspace_bytes, own_e)));
-        if (by_wsm(plan, (double)M * rope.cols, gemm_prefill_ws_us(M, E, N, q4, 0)))
+        if (by_wsm(plan, (double)M * rope.cols, gemm_prefill_ws_rope_us(M, E, N, head_dim, q4)))
             return launch_gemm_wsm_rope(plan, normed, wqkv, qkv_out, rope_lut, rope, reinterpret_cast<float *>(static_cast<char *>(workspace) + own_e), M, E, N, q4, stream);
     }
     return launch_gemm_prefill_ws(normed, wqkv, qkv_out, M, E, N, stream, kEpiRope, rope_lut, &rope, q4);
