@@ -588,9 +588,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         }
     }
 
-    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, a tile at a time in the same order, operand by operand from memory.  Where that stands decides
-    // how the compiler schedules the loop above: here for two tiles side by side, at the stores for one and three (15 forms and 6 sizes, against the kernel without: 0.98 to 1.04, 1.01
-    // for what the sizes take; all tiles at once behind the loop in every form 0.98 to 1.05 and 1.006).
+    // Scales from 2^117 on (wsdequant.h): the wave's columns once more, a tile at a time in the same order, operand by operand from memory, in place of what it stores.  (21 forms and
+    // 5 sizes against the kernel without: 0.96 to 1.05, 1.002 on average; with two tiles side by side in registers, behind the loop, 6 x 2 and 7 x 2 tiles 1.04 to 1.10.)
     bool over = false;
     auto again = [&](int rt, int c) {
         typedef const __attribute__((address_space(1))) uint32_t *Word;
@@ -612,12 +611,6 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
         static_assert(KW == 1, "a wave has all of K");
 #pragma unroll
         for (int c = 0; c < NT; ++c) over |= awq_overflowed(Y[0][c][0], Y[RT - 1][c][0]);
-        if (NT == 2 && __ballot(over)) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int c = 0; c < NT; ++c) Y[rt][c] = again(rt, c);
-        }
     }
 
     // The parts of K meet, then the sums leave through LDS, so that a store is whole rows of the workgroup's columns.  (No copy of
@@ -650,7 +643,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : KW) gemm_wsm_kernel(co
 #pragma unroll
                 for (int i = 0; i < 4; ++i) yt[(16 * rt + 4 * lg + i) * LDP + (NT * wq + c) * kWsTileCols + ln] = Y[rt][c][i];
     }
-    if constexpr (MODE == kSmAwqRounded && NT != 2) {
+    if constexpr (MODE == kSmAwqRounded) {
         if (__ballot(over)) {
 #pragma unroll 1
             for (int n = 0; n < RT * NT; ++n) {
@@ -801,14 +794,14 @@ struct SmForm {
 };
 constexpr SmForm kSmForms[] = {{4, 3, false, {3.93f, 3.87f}, {0.856f, 0.974f}, {0.079f, 0.067f}}, {5, 3, false, {4.49f, 4.59f}, {0.880f, 1.031f}, {0.106f, 0.082f}},
                                {6, 1, false, {2.47f, 2.32f}, {0.497f, 0.542f}, {0.049f, 0.050f}}, {7, 1, false, {2.81f, 2.62f}, {0.521f, 0.563f}, {0.072f, 0.065f}},
-                               {5, 2, false, {3.26f, 3.36f}, {0.682f, 0.777f}, {0.077f, 0.065f}}, {6, 2, false, {3.87f, 3.78f}, {0.729f, 0.810f}, {0.090f, 0.074f}},
-                               {7, 2, false, {4.22f, 4.21f}, {0.777f, 0.956f}, {0.109f, 0.078f}}, {8, 2, false, {3.72f, 3.38f}, {0.936f, 1.112f}, {0.084f, 0.024f}},
+                               {5, 2, false, {3.26f, 3.36f}, {0.682f, 0.777f}, {0.077f, 0.065f}}, {6, 2, false, {3.87f, 3.78f}, {0.703f, 0.810f}, {0.090f, 0.074f}},
+                               {7, 2, false, {4.22f, 4.21f}, {0.748f, 0.956f}, {0.109f, 0.078f}}, {8, 2, false, {3.72f, 3.38f}, {0.936f, 1.112f}, {0.084f, 0.024f}},
                                {10, 2, false, {4.61f, 4.49f}, {1.019f, 1.163f}, {0.128f, 0.103f}}, {6, 3, false, {4.97f, 4.98f}, {0.916f, 1.125f}, {0.149f, 0.100f}},
                                {7, 3, false, {4.98f, 4.73f}, {1.028f, 1.275f}, {0.154f, 0.077f}}, {2, 1, true, {1.18f, 1.11f}, {0.415f, 0.441f}, {0.021f, 0.034f}, {0.157f, 0.196f}},
                                {3, 1, true, {1.72f, 1.44f}, {0.407f, 0.456f}, {0.200f, 0.206f}, {0.193f, 0.223f}}, {4, 1, true, {1.96f, 1.79f}, {0.437f, 0.484f}, {0.265f, 0.263f}, {0.239f, 0.254f}},
                                {5, 1, true, {2.28f, 2.19f}, {0.479f, 0.500f}, {0.333f, 0.338f}, {0.294f, 0.308f}}, {6, 1, true, {1.93f, 1.36f}, {0.686f, 0.727f}, {0.260f, 0.245f}, {0.180f, 0.224f}},
                                {3, 2, true, {2.46f, 2.44f}, {0.592f, 0.690f}, {0.360f, 0.351f}, {0.355f, 0.406f}}, {4, 2, true, {2.97f, 3.05f}, {0.645f, 0.737f}, {0.414f, 0.445f}, {0.394f, 0.463f}},
-                               {6, 2, true, {2.96f, 2.69f}, {0.841f, 0.935f}, {0.514f, 0.504f}, {0.469f, 0.512f}}, {7, 2, true, {3.29f, 3.21f}, {0.927f, 1.017f}, {0.593f, 0.534f}, {0.551f, 0.559f}},
+                               {6, 2, true, {2.96f, 2.69f}, {0.816f, 0.935f}, {0.499f, 0.504f}, {0.455f, 0.512f}}, {7, 2, true, {3.29f, 3.21f}, {0.876f, 1.017f}, {0.560f, 0.534f}, {0.521f, 0.559f}},
                                {5, 3, true, {3.81f, 3.59f}, {0.942f, 1.191f}, {0.679f, 0.564f}, {0.646f, 0.686f}}};
 
 template <int MODE, size_t... I>
