@@ -254,6 +254,45 @@ def test_scales_up_to_the_largest(M, K, N, forms):
             ops.tune(key, 0)
 
 
+@pytest.mark.parametrize("nt,rt", [(1, 2), (2, 6), (3, 5)])
+def test_scales_up_to_the_largest_in_slices(nt, rt):
+    """Scales of 2^118 to 2^124 in some groups of K, and so in some slices and not in others, which decide alone what they take again: the powers of two cancel against x, so every
+    product and sum has the bits of moderate scales."""
+    from air_hip import ops
+    print("largest scales in slices", nt, rt, flush=True)
+    M, K, N = 200, 4096, 256
+    rng = np.random.default_rng(rt)
+    q, z = rng.integers(0, 16, (K, N), dtype=np.uint8), rng.integers(0, 16, (K // 128, N), dtype=np.uint8)
+    s = np.exp2(rng.uniform(8, 14, (K // 128, N))).astype(np.float32) * rng.choice([-1, 1], (K // 128, N))
+    x = (rng.uniform(0.125, 4, (M, K)) * rng.choice([-1, 1], (M, K))).astype(np.float32)
+    exact = lambda b, by: f32_to_bf16_bits(bf16_bits_to_f32(b) * by)
+    s, x = (f32_to_bf16_bits(np.ascontiguousarray(t.astype(np.float32))) for t in (s, x))
+    qz = dev(oawq.pack_awq_int32(q)), dev(oawq.pack_awq_int32(z))
+    w = ops.repack_stream(*qz, dev(s))
+    keys = ("prefill_wsm", "gemm_wsm_nt", "gemm_wsm_rt", "gemm_wsm_slices")
+    lib, parts = ops._lib.load_library(), torch.empty(4 * M * N, dtype=torch.float32, device="cuda")
+
+    def product(xb, w, slices):
+        for key, value in zip(keys, (1, nt, rt, slices)):
+            ops.tune(key, value)
+        y, xd = torch.empty((M, N), dtype=torch.bfloat16, device="cuda"), dev(xb)
+        parts.fill_(float("nan"))
+        ops._lib.check(lib.w4a16_gemm_stream_scratch_bf16(xd.data_ptr(), w.buf.data_ptr(), y.data_ptr(), M, K, N, 128, parts.data_ptr(), parts.numel() * 4,
+                                                          torch.cuda.current_stream().cuda_stream))
+        assert int(parts.isfinite().sum()) == (slices * M * N if slices > 1 else 0), "parts in the scratch"
+        return bits(y)
+
+    try:
+        for large in (np.arange(K // 128) < 8, np.arange(K // 128) == 20, np.arange(K // 128) % 16 == 15):
+            by = np.where(large, 2.0**110, 1.0).astype(np.float32)
+            w_large, small_x = ops.repack_stream(*qz, dev(exact(s, by[:, None]))), exact(x, np.repeat(1 / by, 128)[None, :])
+            for slices in (1, 2, 4):
+                assert np.array_equal(product(small_x, w_large, slices), product(x, w, slices)), (slices, np.flatnonzero(large))
+    finally:
+        for key in keys:
+            ops.tune(key, 0)
+
+
 @pytest.mark.parametrize("form", [(1, 1, 2, 0), (1, 3, 4, 0), (2, 0, 0, 1), (2, 0, 0, 3)])
 def test_every_weight_under_the_largest_scales(form):
     """One-hot rows of x, small and largest scales in one column: the dequantised weights bit for bit."""

@@ -517,3 +517,109 @@ def test_prompt_blocks_of_few_rows(ops, codec, M, E, H, nh, nkv, hd):
         assert np.all(np.abs(f(h) - want) <= 2 * bf16_ulp(want) + 1.2 * bf16_ulp(g) * np.abs(u) + bf16_ulp(u) * np.abs(g) + 1e-3)
         want = f(d) + f(res1)
         assert np.all(np.abs(f(y) - want) <= bf16_ulp(want) + bf16_ulp(f(d)) + 2e-3)
+
+
+@pytest.mark.parametrize("codec", ["awq", "q4nx"])
+@pytest.mark.parametrize("M,E,H,nh,nkv,hd,slices", [(17, 1024, 14336, 8, 4, 128, 12), (33, 1024, 12288, 4, 2, 64, 8), (1, 1024, 6144, 1, 1, 128, 6), (33, 6144, 256, 3, 1, 128, 6),
+                                                    (17, 8192, 256, 2, 1, 64, 8)])
+def test_prompt_blocks_in_many_slices(ops, monkeypatch, codec, M, E, H, nh, nkv, hd, slices):
+    """Six parts and more, of which some are asked for beside others and some alone: the projections with RoPE, O and down with the residual, gate and up with SwiGLU, where K holds so
+    many (eight groups each).  Bounds as for few rows."""
+    from oracle import decode as odec
+    print(f"prompt blocks in many slices {codec} M={M} E={E} H={H} heads {nh}/{nkv} of {hd}, {slices}", flush=True)
+    N = (nh + 2 * nkv) * hd
+
+    def weight(K, n, seed):
+        if codec == "awq":
+            return _sw(ops, _scaled(K, n, seed, 0.1))
+        from test_gpu_q4nx import make
+        q, s, m = make(n, K, seed=seed)
+        return ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+
+    monkeypatch.setattr(ops, "_attn_ws", {})
+    many = E // 128 >= 8 * slices   # else down alone
+    wg, wu, wd = weight(E, H, 3), weight(E, H, 4), weight(H, E, 5)
+    wo = weight(E, E, 2)
+    attn, xres, nw, lut = dev(make_x((M, E), seed=6)), dev(make_x((M, E), seed=7)), dev(_norm_w(E, 8)), dev(odec.generate_rope_lut(hd, 500000.0, M + 3))
+    wqkv = weight(E, N, 1) if many else None
+
+    def blocks(wsm, slices):
+        ops.tune("prefill_wsm", wsm)
+        ops.tune("gemm_wsm_slices", slices)
+        try:
+            qkv = ops.prefill_rms_qkv_rope_stream(xres, nw, wqkv, lut, 3, nh, nkv, hd, codec=codec) if many else None
+            return [qkv, *ops.prefill_o_ffn_stream(attn, xres, nw, wo, wg, wu, wd, return_intermediates=True, codec=codec)]
+        finally:
+            ops.tune("prefill_wsm", 0)
+            ops.tune("gemm_wsm_slices", 0)
+
+    tiled = blocks(2, 0)
+    for ws in ops._attn_ws.values():
+        ws.fill_(0xFF)
+    cut = blocks(1, slices)
+    # so many parts were written behind the rows of each workspace
+    round256 = lambda n: (n + 255) // 256 * 256
+    rows = {"prefill_qkv_stream": round256(2 * M * E), "prefill_block_stream": 2 * round256(2 * M * E) + 2 * round256(2 * M * H)}
+    parts = {"prefill_qkv_stream": slices * M * N, "prefill_block_stream": slices * M * (max(E, 2 * H) if many else E)}
+    for key, ws in ops._attn_ws.items():
+        behind = ws[rows[key[2]]:].view(torch.int32) != -1
+        assert bool(behind[:parts[key[2]]].all()) and not bool(behind[parts[key[2]]:].any()), key
+    for got, want in [(cut[0], tiled[0]), (cut[2], tiled[2])] if many else []:
+        bound = 2.0**-7 * want.float().abs().amax(1, keepdim=True)
+        assert bool(((got.float() - want.float()).abs() <= bound).all())
+    _, y, res1, h = cut
+    normed = ops.rms_norm_rows(res1, nw)
+    plain = ops.q4nx_gemm_stream if codec == "q4nx" else ops.w4a16_gemm_stream
+    f = lambda t: t.double().cpu().numpy()
+    ops.tune("prefill_min_m", 17)
+    ops.tune("prefill_wsm", 2)
+    try:
+        pad = lambda t: torch.cat([t, torch.zeros((max(0, 17 - M), t.shape[1]), dtype=t.dtype, device="cuda")])   # (fewer rows have another kernel)
+        g, u, d = (plain(pad(t), w)[:M] for t, w in ((normed, wg), (normed, wu), (h, wd)))
+    finally:
+        ops.tune("prefill_min_m", 0)
+        ops.tune("prefill_wsm", 0)
+    g, u = f(g), f(u)
+    want = g / (1.0 + np.exp(-g)) * u
+    assert np.all(np.abs(f(h) - want) <= 2 * bf16_ulp(want) + 1.2 * bf16_ulp(g) * np.abs(u) + bf16_ulp(u) * np.abs(g) + 1e-3)
+    want = f(d) + f(res1)
+    assert np.all(np.abs(f(y) - want) <= bf16_ulp(want) + bf16_ulp(f(d)) + 2e-3)
+
+
+@pytest.mark.parametrize("codec", ["awq", "q4nx"])
+@pytest.mark.parametrize("wsm,slices", [(1, 1), (1, 2), (2, 0)])
+def test_rows_that_are_not_finite_stay_alone(ops, codec, wsm, slices):
+    """Infinities and NaN in one row of x or of the attention's output, through the sums, RoPE, the residual and SwiGLU: the other rows keep their bits, and nothing finite comes of these."""
+    from oracle import decode as odec
+    M, E, H, nh, nkv, hd = 40, 2048, 2048, 4, 2, 64
+    print("rows that are not finite", codec, wsm, slices, flush=True)
+
+    def weight(K, n, seed):
+        if codec == "awq":
+            return _sw(ops, _scaled(K, n, seed, 0.1))
+        from test_gpu_q4nx import make
+        q, s, m = make(n, K, seed=seed)
+        return ops.q4nx_repack_stream(dev(oawq.pack_awq_int32(q.T)), dev(s.T), dev(m.T))
+
+    wqkv, wo, wg, wu, wd = (weight(*a) for a in ((E, (nh + 2 * nkv) * hd, 1), (E, E, 2), (E, H, 3), (E, H, 4), (H, E, 5)))
+    x, attn, nw, lut = make_x((M, E), seed=6), make_x((M, E), seed=7), dev(_norm_w(E, 8)), dev(odec.generate_rope_lut(hd, 500000.0, M))
+
+    def run(x, attn):
+        ops.tune("prefill_wsm", wsm)
+        ops.tune("gemm_wsm_slices", slices)
+        try:
+            return [ops.prefill_rms_qkv_rope_stream(dev(x), nw, wqkv, lut, 0, nh, nkv, hd, codec=codec),
+                    *ops.prefill_o_ffn_stream(dev(attn), dev(make_x((M, E), seed=9)), nw, wo, wg, wu, wd, return_intermediates=True, codec=codec)]
+        finally:
+            ops.tune("prefill_wsm", 0)
+            ops.tune("gemm_wsm_slices", 0)
+
+    plain = run(x, attn)
+    rows = {2: 0x7F80, 17: 0xFF80, 39: 0x7FC0}
+    for row, value in rows.items():
+        x[row, 100 + row] = attn[row, 1500 + row] = value
+    others = torch.tensor([m for m in range(M) if m not in rows], device="cuda")
+    for name, got, want in zip(("qkv", "y", "res1", "h"), run(x, attn), plain):
+        assert bool(want.isfinite().all()), name
+        assert torch.equal(got[others].view(torch.int16), want[others].view(torch.int16)), name
+        assert not bool(got[list(rows)].isfinite().any()), name
