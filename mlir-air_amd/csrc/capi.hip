@@ -544,8 +544,8 @@ int w4a16_gemv_stream_bf16(const uint16_t *x, const void *wstream, uint16_t *y, 
 
 // Products of 2 rows and more, whose arguments have been checked.  By precision: bf16-rounded weights from 129 rows on (Q4NX: 65, and
 // not with a residual, which is added in fp32 before the one rounding) where the tiled kernel takes the shape, else exact ones.  Between
-// the kernels of each kind by their estimated times (us, 64 and 300 rows of K = 14336, N = 4096: whole-K launches 55, tiled 150;
-// gemm_wsm 18 with slices and 32 without, 73; 2048 rows of K = 4096, N = 14336: tiled 172, gemm_wsm 275).
+// the kernels of each kind by their estimated times (us, weights from memory, 64 and 300 rows of K = 14336, N = 4096: whole-K launches
+// 55, tiled 157; gemm_wsm 20 with slices and 35 without, 52; 2048 rows of K = 4096, N = 14336: tiled 176, gemm_wsm 251).
 static bool gemm_stream_rounded(int M, int K, int N, bool q4, bool residual) {
     const int least = g_gemv_ws_tune.prefill_min_m > 16 ? g_gemv_ws_tune.prefill_min_m : gemm_rounded_rows(q4);
     return M >= least && !(q4 && residual) && gemm_prefill_ws_supported(M, K, N);

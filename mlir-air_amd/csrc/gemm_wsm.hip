@@ -23,14 +23,14 @@
 //                groups too.  What bounds it then is issue, 4 cycles an instruction: a group of 5 x 3 tiles has 240 vector, 60 matrix and 110 other ones.  Tall and wide
 //                forms (up to 10 x 2 and 7 x 3 tiles, one workgroup to a CU, rings of 160 KB) need the fewest; two workgroups to a CU, each with half of LDS, hide each
 //                other's latencies and fill the chip with twice as many tiles.  Reading a group ahead takes a stage of the ring: with four it is asked for two groups
-//                before it is needed, with three one group, with two it could not be.  So with fewer than four all of a group's x is read in its first half (kEarly: 2 RT more
-//                registers of operands) and its own stage is filled again: three stages are two groups, two stages one.
+//                before it is needed, with three one group, with two it could not be.  So with fewer than four all of a group's x is read in its first half (kEarly: 8 RT more
+//                registers) and its own stage is filled again: three stages are two groups, two stages one.
 //                Weights from memory, us, K-steps one after the other / read ahead without kEarly, where two stages leave one workgroup to a CU / now: 349 rows of 4352 x 13760
 //                54.9 / 64.5 / 52.5, 386 of 6656 x 12800 82.2 / 95.4 / 82.9, 652 of 1280 x 8896 22.6 / 27.8 / 22.2, 170 of 2048 x 5120 11.5 / 12.4 / 11.5, 1519 of 1536 x 5568 31.6 /
 //                40.2 / 32.6, 300 of 4096 x 11008 43.0 / 39.1 / 38.4, Q4NX 486 of 2560 x 12480 45.1 / 60.0 / 42.3, 282 of 10240 x 6336 69.4 / 77.3 / 67.5.  400 random products of 129 to
-//                2000 rows against the loop of K-steps one after the other: 1.14 times as fast (from memory 0.90 at worst, five below 0.95: 1000 to 1300 rows of wide short matrices,
-//                where the tiled kernel and the tallest forms are close, and eight groups of K; from the last-level cache 0.92, one); 17 to 128 rows, exact ones mostly, 1.06 and 1.07
-//                (0.94 and 0.96 at worst).  (Every instruction in its place by
+//                2000 rows against the loop of K-steps one after the other: 1.14 times as fast (from memory 0.88 at worst, seven below 0.95: 1000 to 1300 rows of wide short matrices,
+//                where the tiled kernel and the tallest forms are close, and eight to ten groups of K; from the last-level cache 0.95, one); 17 to 128 rows, exact ones mostly, 1.06 and
+//                1.07 (0.94 and 0.96 at worst).  (Every instruction in its place by
 //                volatile asm, none behind one that it depends on, 300 of 4096 x 11008 36.4 -> 38.3: not taken.)
 //   slices > 1 : fp32 sums to plain scratch, added in slice order by a second launch (deterministic)
 #include <algorithm>

@@ -447,10 +447,10 @@ PrefillArgs<T> args_of(const HeadShape &s, const HeadRows &r, const void *q, voi
 }
 
 // Whether a workgroup takes 64 queries, 16 to a wave, instead of 128, for heads of 128 + 64 / 128 and of 128 / 128 behind long windows.  A block of 64 keys takes a wave set 2.6 us
-// with 16 queries to a wave and 2.8 with 32 (staging, scores, softmax and outputs are a chain between two barriers, a workgroup has its CU to itself): the longest item is done
-// sooner, all of them together take 1.5 times as long.  So where they are no more than 256 CUs have room for beside the longest.  us, 128 / 64 queries, 16 heads of 128 + 64 / 128:
-// 128 tokens 13.3 / 9.2, 1000 31.6 / 24.9, 1500 43.2 / 35.2, 1800 50.2 / 45.6, 3000 80.2 / 108.8; 8 heads 3000 73.6 / 62.6; 32 heads 700 25.1 / 20.7, 1000 33.8 / 32.6, 2048 74.0 / 99.4.
-// (On the line, 16 heads and 2048 tokens, 56.0 / 52.8.)
+// with 16 queries to a wave and 2.8 with 32 (staging, scores, softmax and outputs are a chain between two barriers, a workgroup has its CU to itself), so of 64 queries the longest
+// item is done sooner, and launches of several items to a CU take 1.35 times as long.  The line: 256 CUs get all items done in the time of the longest.  us, 128 / 64 queries, 16 heads of
+// 128 + 64 / 128: 128 tokens 13.3 / 9.2, 1000 31.6 / 24.9, 1500 43.2 / 35.2, 1800 50.2 / 45.6, 3000 80.2 / 108.8; 8 heads 3000 73.6 / 62.6; 32 heads 700 25.1 / 20.7, 1000 33.8 / 32.6, 2048
+// 74.0 / 99.4.  Just past it 64 would still be faster alone (16 heads and 2048 tokens, 3 % more blocks than that, 56.0 / 52.8): the line is not fitted there.
 template <class T>
 long item_blocks(const PrefillArgs<T> &p, long first, long queries = 64) {   // blocks of 64 keys of the item of so many queries from position `first` on
     const long end = std::min<long>(first + queries, p.total), unseen = p.window > 0 && first >= p.window ? (first - p.window + 1) / 64 : 0;
