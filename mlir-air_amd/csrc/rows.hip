@@ -38,8 +38,19 @@ __global__ void __launch_bounds__(kRowThreads) embed_rows_kernel(const int32_t *
 // 1024 rows of 2048, eight experts 10.2 / 8.9; 2048 rows of 2048, eight experts 16.1 / 16.2.
 
 // y[m] of a row's four elements: the sum of `parts` matrices [M][width] (a product's slices along K), in their order
+// (in turn: a loop with no bounds to look at; 520 rows of 6144, two parts 11.3 -> 10.2 us)
 template <int AT>
 __device__ __forceinline__ void load_parts(const float *y, int parts, size_t size, float (&v)[4]) {
+    if constexpr (AT == 1) {
+        load4(y, v);
+        for (int s = 1; s < parts; ++s) {
+            float u[4];
+            load4(y + s * size, u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] += u[j];
+        }
+        return;
+    }
     for (int s0 = 0; s0 < parts; s0 += AT) {
         float u[AT][4];
 #pragma unroll
@@ -56,6 +67,16 @@ template <int AT, class Y>
 __device__ __forceinline__ void load_weighted(const Y *y, const float *weights, int top, int width, float (&v)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = 0.f;
+    if constexpr (AT == 1) {
+        for (int s = 0; s < top; ++s) {
+            float u[4];
+            load4(y + (size_t)s * width, u);
+            const float wt = weights[s];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = fmaf(wt, u[j], v[j]);
+        }
+        return;
+    }
     for (int s0 = 0; s0 < top; s0 += AT) {
         float u[AT][4], wt[AT];
 #pragma unroll
@@ -217,7 +238,9 @@ __global__ void __launch_bounds__(kRowThreads) add_norm_rows_kernel(float *res, 
 
 // f(quads a thread, parts at a time) with the kernel's constants for M rows of `parts`.  Over `few` rows the other workgroups of a CU cover the round trips, and fewer registers keep
 // more of them there: loads in turn again, and by way of LDS where a row has more quads than `quads_few` of few rows, `quads_many` of many.  (2048 rows of 2048, eight parts at a time
-// 27.2 us, in turn 25.9; 1024 rows, two parts 5.4 / 4.9; eight experts 8.9 / 10.2, at 2048 rows 16.6 / 16.2.)
+// 27.2 us, in turn 25.9; 1024 rows, two parts 5.4 / 4.9; eight experts 8.9 / 10.2, at 2048 rows 16.6 / 16.2.)  By way of LDS also where half a workgroup or more has no quad and would
+// ask for many operands of one all the same (registers / LDS, 2048 rows, eight experts of 512 5.6 / 4.7, of 256 5.1 / 4.2, four 4.1 / 3.7; but one or two of 512 3.0 / 3.2, eight of 768 4.0 / 4.3,
+// 520 rows of eight of 512 3.3 / 3.5).
 template <class F>
 void row_form(int M, int few, int width, int quads_few, int quads_many, int parts, F f) {
     auto with_parts = [&](auto quads) {
@@ -227,7 +250,8 @@ void row_form(int M, int few, int width, int quads_few, int quads_many, int part
         else f(quads, std::integral_constant<int, 8>());
     };
     const int quads = (width + 4 * kRowThreads - 1) / (4 * kRowThreads), most = M > few ? quads_many : quads_few;
-    if (quads > most) with_parts(std::integral_constant<int, 0>());
+    const bool narrow = M > 1024 && width <= 512 && width <= 128 * parts;
+    if (quads > most || narrow) with_parts(std::integral_constant<int, 0>());
     else if (quads == 1) with_parts(std::integral_constant<int, 1>());
     else if (quads == 2) with_parts(std::integral_constant<int, 2>());
     else with_parts(std::integral_constant<int, 4>());
