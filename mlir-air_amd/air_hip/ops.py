@@ -679,7 +679,9 @@ def prefill_o_ffn(attn_out, x_residual, ffn_norm_weight, wo, gate, up, down, eps
 
 def _prompt_workspace(use, most, device, M, *widths):
     """Plain scratch of a prompt block on stream-order weights, kept for the stream.  Up to 512 rows, where parts of K slices are most of it, 64 lengths share one (what a length
-    runs does not depend on what lies behind its own bytes)."""
+    runs does not depend on what lies behind its own bytes).  In a capture it is the graph's own: graphs of two lengths may be replayed on two streams."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(int(most(M, *widths)), dtype=torch.uint8, device=device)
     last = (M + 63) // 64 * 64 if M <= 512 else M
     key = (device.index, _stream(), use, last, *widths)
     ws = _attn_ws.get(key)

@@ -364,6 +364,40 @@ def test_prompt_lengths_share_their_workspaces(ops, monkeypatch):
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), M
 
 
+def test_graphs_of_two_lengths_have_workspaces_of_their_own(ops, monkeypatch):
+    """Lengths that share a workspace otherwise, captured on one stream and replayed on two at a time: each replay has the eager bits."""
+    from oracle import decode as odec
+    E, H, nh, nkv, hd = 2048, 1024, 24, 4, 64
+    sw, ws = _sw(ops, _qkv_weights(E, nh, nkv, hd, seed=1)[1]), [_sw(ops, w) for w in _weights(E, H, seed=1)]
+    lut, nw = dev(odec.generate_rope_lut(hd, 500000.0, 200)), dev(_norm_w(E, 3))
+    monkeypatch.setattr(ops, "_attn_ws", {})
+    runs = []
+    for M in (70, 100):
+        x, attn = dev(make_x((M, E), seed=M)), dev(make_x((M, E), seed=M + 1))
+        run = lambda x=x, attn=attn: [t for _ in range(4) for t in (ops.prefill_rms_qkv_rope_stream(x, nw, sw, lut, 0, nh, nkv, hd), ops.prefill_o_ffn_stream(attn, x, nw, *ws))]
+        want = run()
+        torch.cuda.synchronize()
+        kept = set(ops._attn_ws)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = run()
+        assert set(ops._attn_ws) == kept
+        runs.append((graph, outs, want, torch.cuda.Stream(), x, attn))
+    for turn in range(3):
+        print("two lengths on two streams", turn, flush=True)
+        for _, outs, *_ in runs:
+            for t in outs:
+                t.zero_()
+        torch.cuda.synchronize()
+        for graph, _, _, stream, *_ in runs:
+            with torch.cuda.stream(stream):
+                graph.replay()
+        torch.cuda.synchronize()
+        for _, outs, want, *_ in runs:
+            for got, w in zip(outs, want):
+                assert torch.equal(got.view(torch.int16), w.view(torch.int16))
+
+
 # 192-column tiles of heads of 128 (a head and half of one) and of gate and up: one of them, several, beside wide ones, ragged rows
 @pytest.mark.parametrize("M,E,nh,nkv,pos0,tile", [(100, 256, 1, 1, 4, 2), (270, 512, 4, 1, 0, 2), (2048, 256, 9, 3, 9, 0), (1000, 256, 32, 8, 2, 0)])
 def test_prefill_rms_qkv_rope_stream_in_192_columns(ops, tiled_gemm, M, E, nh, nkv, pos0, tile):
