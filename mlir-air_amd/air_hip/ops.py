@@ -682,11 +682,11 @@ def _prompt_workspace(use, most, device, M, *widths):
     runs does not depend on what lies behind its own bytes).  In a capture it is the graph's own: graphs of two lengths may be replayed on two streams."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(int(most(M, *widths)), dtype=torch.uint8, device=device)
-    last = (M + 63) // 64 * 64 if M <= 512 else M
+    last = (M + 63) // 64 * 64 if M <= 512 else M   # takes the most of the 64: slices are by tiles of 256 rows or by bytes
     key = (device.index, _stream(), use, last, *widths)
     ws = _attn_ws.get(key)
     if ws is None:
-        ws = torch.empty(max(int(most(m, *widths)) for m in range(last - 63 if M <= 512 else M, last + 1)), dtype=torch.uint8, device=device)
+        ws = torch.empty(int(most(last, *widths)), dtype=torch.uint8, device=device)
         _attn_ws[key] = ws
     return ws
 

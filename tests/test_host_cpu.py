@@ -194,6 +194,15 @@ def test_prompt_workspaces_ask_for_no_more_than_is_used(E, H):
             assert least <= most <= least + ((12 << 20) if M <= 512 else 0), (M, E, H)
 
 
+@pytest.mark.parametrize("E,H", [(64, 128), (1096, 2056), (2048, 8192), (4096, 14336), (8192, 28672)])
+def test_prompt_workspaces_of_64_lengths_are_the_last_ones(E, H):
+    """The longest of 64 lengths takes the most of them: its workspace is enough for all."""
+    lib = _lib.load_library()
+    for last in range(64, 513, 64):
+        for f, widths in ((lib.w4a16_prefill_qkv_workspace_most, (E,)), (lib.w4a16_prefill_block_workspace_most, (E, H))):
+            assert max(f(M, *widths) for M in range(last - 63, last + 1)) == f(last, *widths) > 0, (last, widths)
+
+
 def test_c_abi_rejects_bad_arguments_before_touching_the_gpu():
     lib = _lib.load_library()
     P = 0x10000   # fake, aligned, never dereferenced: validation fails first
